@@ -47,7 +47,14 @@ extern "C" {
  *   skyrl_conv_save stores the last `taps` rows of every sequence's columns [0, channels) of x T [T, stride]
  *                   in ring T [rows, taps, channels], the row of position p at p % taps. Sequences: tokens
  *                   [cu[s], cu[s+1]) of row rows[s] (< 0: skipped), positions consecutive from positions[cu[s]].
- *   skyrl_softcap   out f32 = cap * tanh(x / cap) over count elements of x T (cap <= 0: a copy). */
+ *   skyrl_softcap   out f32 = cap * tanh(x / cap) over count elements of x T (cap <= 0: a copy).
+ *   skyrl_rows_product  few rows: y = x bf16 [n, K] (row stride ldx) w bf16 [N, K]^T (row stride ldw), summed in f32, rows
+ *                   16-byte aligned. act < 0: y + bias bf16 [N] (may be NULL), as bf16 [n, N] (splits 0, row stride ldo),
+ *                   or as f32 [splits, n, ldo] whose sum over the first index is the product, the bias in the first. act
+ *                   of skyrl_gate_mul: w holds N gate rows, then N up rows; the gated product bf16 [n, N], splits 0.
+ *                   skyrl_rows_product_fits: whether it takes the sizes; skyrl_rows_product_splits: the splits.
+ *   skyrl_add_norm_parts, skyrl_gate_norm_add_parts  of a model in bf16, the sublayer's output being such a sum of
+ *                   `parts` f32 [n, H]. */
 #define SKYRL_NORM_LAYER 0
 #define SKYRL_NORM_RMS 1
 #define SKYRL_ACT_SILU 0
@@ -70,6 +77,16 @@ int skyrl_gate_mul(const void* gate_up, int64_t gu_stride, int64_t n, int32_t I,
 int skyrl_gate_norm_add(const void* a, const int64_t* rows, int32_t parts, const void* gate, int64_t gate_stride,
                         const float* gate_bias, const void* weight, int32_t groups, float eps, float mult, float* hidden,
                         int32_t fresh, const void* next, int32_t n, int32_t H, void* out, int32_t dtype, void* stream);
+int32_t skyrl_rows_product_fits(int32_t n, int32_t K, int32_t N, int32_t gated);
+int32_t skyrl_rows_product_splits(int32_t n, int32_t K, int32_t N);
+int skyrl_rows_product(const void* x, int64_t ldx, int32_t n, int32_t K, const void* w, int64_t ldw, int32_t N,
+                       const void* bias, int32_t act, float alpha, float limit, int32_t splits, void* out, int64_t ldo,
+                       void* stream);
+int skyrl_add_norm_parts(const float* delta, int32_t parts, float* hidden, const void* step, const void* weight, float w_base,
+                         int32_t n, int32_t H, float eps, int32_t kind, void* out, void* stream);
+int skyrl_gate_norm_add_parts(const float* a, int32_t parts, const void* gate, int64_t gate_stride, const float* gate_bias,
+                              const void* weight, int32_t groups, float eps, float mult, float* hidden, const void* next,
+                              int32_t n, int32_t H, void* out, void* stream);
 int skyrl_tanh(const void* x, int64_t stride, int64_t n, int32_t I, void* out, int32_t dtype, void* stream);
 int skyrl_conv_save(const void* x, int64_t stride, int32_t channels, int32_t taps, const int32_t* cu,
                     const int32_t* rows, const int64_t* positions, int32_t nseq, void* ring, int32_t dtype,

@@ -2,17 +2,19 @@
 // (include/skyrl_layers.h). The residual stream stays f32 in HBM: the add, the norm and the optional
 // per-pass step vector of a looped layer stack are one pass over a row.
 #include "conv.h"
+#include "gate.h"
 
 namespace skyrl {
 namespace {
 
 constexpr int kNT = 256;
 
-// One block per row, the row in registers: kMaxV groups of VEC elements per thread.
-template <typename T, int VEC, int kMaxV>
-__global__ __launch_bounds__(kNT) void add_norm_kernel(const T* __restrict__ delta, float* __restrict__ h,
-                                                       const T* __restrict__ step, const T* __restrict__ w,
-                                                       float w_base, int H, float eps, int kind,
+// One block per row, the row in registers: kMaxV groups of VEC elements per thread. D: type of delta, the sum of `parts`
+// rows part_stride apart (a product's shares of the depth).
+template <typename T, typename D, int VEC, int kMaxV>
+__global__ __launch_bounds__(kNT) void add_norm_kernel(const D* __restrict__ delta, int parts, int64_t part_stride,
+                                                       float* __restrict__ h, const T* __restrict__ step,
+                                                       const T* __restrict__ w, float w_base, int H, float eps, int kind,
                                                        T* __restrict__ out) {
     __shared__ float s_red[kNT / kWave];
     const int64_t base = (int64_t)blockIdx.x * H;
@@ -26,7 +28,14 @@ __global__ __launch_bounds__(kNT) void add_norm_kernel(const T* __restrict__ del
             if constexpr (VEC == 4) {
                 float4 a = ld4(h + base + 4 * v);
                 if (delta) {
-                    const float4 d = ld4(delta + base + 4 * v);
+                    float4 d = ld4(delta + base + 4 * v);
+                    if constexpr (sizeof(D) > sizeof(T)) {
+#pragma unroll 4
+                        for (int i = 1; i < parts; ++i) {
+                            const float4 e = ld4(delta + i * part_stride + base + 4 * v);
+                            d.x += e.x; d.y += e.y; d.z += e.z; d.w += e.w;
+                        }
+                    }
                     a.x += d.x; a.y += d.y; a.z += d.z; a.w += d.w;
                 }
                 if (step) {
@@ -37,7 +46,12 @@ __global__ __launch_bounds__(kNT) void add_norm_kernel(const T* __restrict__ del
                 x[k][0] = a.x; x[k][1] = a.y; x[k][2] = a.z; x[k][3] = a.w;
             } else {
                 float a = h[base + v];
-                if (delta) a += ld(delta + base + v);
+                if (delta) {
+                    float d = ld(delta + base + v);
+                    if constexpr (sizeof(D) > sizeof(T))
+                        for (int i = 1; i < parts; ++i) d += ld(delta + i * part_stride + base + v);
+                    a += d;
+                }
                 if (step) a += ld(step + v);
                 if (delta || step) h[base + v] = a;
                 x[k][0] = a;
@@ -192,22 +206,6 @@ __global__ __launch_bounds__(kNT) void norm_add_kernel(NormAdd<T> p) {
             stw<T, VEC>(p.out + base + VEC * v, h[k]);
         }
     }
-}
-
-struct Gate {
-    int act;
-    float alpha, limit;  // of the clamped form
-};
-
-// The gated product of one pair.
-__device__ __forceinline__ float gated(float g, float u, const Gate& f) {
-    if (f.act == SKYRL_ACT_SILU) return siluf_(g) * u;
-    if (f.act == SKYRL_ACT_CLAMPED) {
-        g = fminf(g, f.limit);
-        u = fminf(fmaxf(u, -f.limit), f.limit);
-        return g / (1.f + expf(-f.alpha * g)) * (u + 1.f);
-    }
-    return 0.5f * g * (1.f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g))) * u;
 }
 
 template <typename T, int VEC>
@@ -390,11 +388,12 @@ __global__ __launch_bounds__(NT) void gated_norm_kernel(const T* __restrict__ y,
 }
 
 // ---- a sublayer's result between two norms in equal parts: gated, normed, added to the residual, normed again ----
-template <typename T>
+template <typename T, typename A>
 struct GateNormAdd {
-    const T* a;
+    const A* a;
     const int64_t* rows;  // row of a (NULL: the output's own)
-    int parts;            // consecutive rows of a that are summed
+    int parts;            // rows of a that are summed, part_stride apart
+    int64_t row_stride, part_stride;
     const T* z;           // gate logits (NULL: no gate) and their bias
     int64_t z_stride;
     const float* zb;
@@ -411,8 +410,8 @@ struct GateNormAdd {
 // One block per row, the row in registers: chunks of VEC elements, chunk threadIdx + k NT, each in one group of `per`
 // chunks. A group's sum: within L lanes (the power of two in per, at most a wave) by shuffles, then over per / L numbers
 // in LDS. PARTS: rows that are summed (0: any number).
-template <typename T, int NT, int VEC, int kMaxV, int PARTS>
-__global__ __launch_bounds__(NT) void gate_norm_add_kernel(GateNormAdd<T> p, int L) {
+template <typename T, typename A, int NT, int VEC, int kMaxV, int PARTS>
+__global__ __launch_bounds__(NT) void gate_norm_add_kernel(GateNormAdd<T, A> p, int L) {
     extern __shared__ float s_p[];
     __shared__ float s_red[NT / kWave];
     const int nv = p.H / VEC, per = nv / p.groups, sums = per / L;
@@ -463,12 +462,12 @@ __global__ __launch_bounds__(NT) void gate_norm_add_kernel(GateNormAdd<T> p, int
 #pragma unroll
         for (int j = 0; j < VEC; ++j) y[k][j] = h[k][j] = 0.f;
         if (v < nv) {
-            const T* src = p.a + row * parts * p.H + VEC * v;
-            ldv<T, VEC>(src, y[k]);
+            const A* src = p.a + row * p.row_stride + VEC * v;
+            ldv<A, VEC>(src, y[k]);
             if (!p.fresh) ldv<float, VEC>(p.h + base + VEC * v, h[k]);
             auto add = [&](int i) {
                 float x[VEC];
-                ldv<T, VEC>(src + (int64_t)i * p.H, x);
+                ldv<A, VEC>(src + i * p.part_stride, x);
 #pragma unroll
                 for (int j = 0; j < VEC; ++j) y[k][j] += x[j];
             };
@@ -546,9 +545,26 @@ unsigned grid_for(int64_t items) {
 
 using namespace skyrl;
 
-#define LAUNCH_NORM(V, K) \
-    hipLaunchKernelGGL((add_norm_kernel<T, V, K>), dim3(n), dim3(kNT), 0, s, d, hidden, st_, w, w_base, H, eps, \
-                       kind, o)
+namespace {
+
+template <typename T, typename D>
+void launch_add_norm(const D* delta, int parts, float* hidden, const T* step, const T* w, float w_base, int n, int H, float eps,
+                     int kind, T* out, hipStream_t s) {
+#define LAUNCH_NORM(V, K)                                                                                                  \
+    hipLaunchKernelGGL((add_norm_kernel<T, D, V, K>), dim3(n), dim3(kNT), 0, s, delta, parts, (int64_t)n * H, hidden, step, w, \
+                       w_base, H, eps, kind, out)
+    if (H % 4 == 0) {
+        if (H <= 4 * kNT) LAUNCH_NORM(4, 1);
+        else if (H <= 8 * kNT) LAUNCH_NORM(4, 2);
+        else if (H <= 16 * kNT) LAUNCH_NORM(4, 4);
+        else LAUNCH_NORM(4, 8);
+    } else {
+        if (H <= 4 * kNT) LAUNCH_NORM(1, 4);
+        else LAUNCH_NORM(1, 32);
+    }
+}
+
+}  // namespace
 
 extern "C" int skyrl_add_norm(const void* delta, float* hidden, const void* step, const void* weight, float w_base,
                               int32_t n, int32_t H, float eps, int32_t kind, void* out, int32_t dtype, void* stream) {
@@ -557,22 +573,23 @@ extern "C" int skyrl_add_norm(const void* delta, float* hidden, const void* step
     SKYRL_REQUIRE(kind == SKYRL_NORM_LAYER || kind == SKYRL_NORM_RMS, "add_norm: unknown norm kind");
     if (n == 0) return SKYRL_OK;
     SKYRL_REQUIRE(hidden && weight && out, "add_norm: null pointer");
-    hipStream_t s = as_stream(stream);
     SKYRL_DISPATCH_T(dtype, {
-        const T* d = reinterpret_cast<const T*>(delta);
-        const T* st_ = reinterpret_cast<const T*>(step);
-        const T* w = reinterpret_cast<const T*>(weight);
-        T* o = reinterpret_cast<T*>(out);
-        if (H % 4 == 0) {
-            if (H <= 4 * kNT) LAUNCH_NORM(4, 1);
-            else if (H <= 8 * kNT) LAUNCH_NORM(4, 2);
-            else if (H <= 16 * kNT) LAUNCH_NORM(4, 4);
-            else LAUNCH_NORM(4, 8);
-        } else {
-            if (H <= 4 * kNT) LAUNCH_NORM(1, 4);
-            else LAUNCH_NORM(1, 32);
-        }
+        launch_add_norm<T, T>(reinterpret_cast<const T*>(delta), 1, hidden, reinterpret_cast<const T*>(step),
+                              reinterpret_cast<const T*>(weight), w_base, n, H, eps, kind, reinterpret_cast<T*>(out),
+                              as_stream(stream));
     })
+    return check_launch("add_norm_kernel");
+}
+
+extern "C" int skyrl_add_norm_parts(const float* delta, int32_t parts, float* hidden, const void* step, const void* weight,
+                                    float w_base, int32_t n, int32_t H, float eps, int32_t kind, void* out, void* stream) {
+    SKYRL_REQUIRE(n >= 0 && H > 0 && H <= 8192 && parts > 0, "add_norm_parts: H must be in [1, 8192], parts positive");
+    SKYRL_REQUIRE(kind == SKYRL_NORM_LAYER || kind == SKYRL_NORM_RMS, "add_norm_parts: unknown norm kind");
+    if (n == 0) return SKYRL_OK;
+    SKYRL_REQUIRE(delta && hidden && weight && out, "add_norm_parts: null pointer");
+    launch_add_norm<uint16_t, float>(delta, parts, hidden, reinterpret_cast<const uint16_t*>(step),
+                                     reinterpret_cast<const uint16_t*>(weight), w_base, n, H, eps, kind,
+                                     reinterpret_cast<uint16_t*>(out), as_stream(stream));
     return check_launch("add_norm_kernel");
 }
 
@@ -667,8 +684,24 @@ extern "C" int skyrl_xielu(const void* x, int64_t stride, int64_t n, int32_t I, 
     return check_launch("xielu_kernel");
 }
 
-#define LAUNCH_GNA_(NT, V, K, P) \
-    hipLaunchKernelGGL((gate_norm_add_kernel<T, NT, V, K, P>), dim3(n), dim3(NT), lds, as_stream(stream), p, L)
+namespace {
+
+// The rows of a: `parts` of a token one after another, or (SHARES) a product's shares of the depth, n rows each.
+template <typename T, typename A>
+int launch_gate_norm_add(const void* a, bool shares, const int64_t* rows, int parts, const void* gate, int64_t gate_stride,
+                         const float* gate_bias, const void* weight, int groups, float eps, float mult, float* hidden,
+                         int fresh, const void* next, int n, int H, void* out, hipStream_t s) {
+    auto t = [](const void* q) { return reinterpret_cast<const T*>(q); };
+    const GateNormAdd<T, A> p{reinterpret_cast<const A*>(a), rows, parts, shares ? H : (int64_t)parts * H,
+                              shares ? (int64_t)n * H : H, t(gate), gate_stride, gate_bias, t(weight), groups, eps, mult,
+                              hidden, fresh, t(next), reinterpret_cast<T*>(out), H};
+    const bool wide = H / groups % 8 == 0 && (!gate || (gate_stride % 8 == 0 && aligned16(gate))) && aligned16(a) &&
+                      aligned16(hidden) && aligned16(weight) && aligned16(next) && aligned16(out);
+    const int V = wide ? 8 : 1;
+    int L = 1;
+    while (L < kWave && H / V / groups % (2 * L) == 0) L <<= 1;
+    const size_t lds = groups > 1 ? (size_t)(H / V / L) * sizeof(float) : 0;
+#define LAUNCH_GNA_(NT, V, K, P) hipLaunchKernelGGL((gate_norm_add_kernel<T, A, NT, V, K, P>), dim3(n), dim3(NT), lds, s, p, L)
 #define LAUNCH_GNA(NT)                              \
     do {                                            \
         if (parts == 1) LAUNCH_GNA_(NT, 8, 1, 1);   \
@@ -677,6 +710,18 @@ extern "C" int skyrl_xielu(const void* x, int64_t stride, int64_t n, int32_t I, 
         else if (parts == 8) LAUNCH_GNA_(NT, 8, 1, 8); \
         else LAUNCH_GNA_(NT, 8, 1, 0);              \
     } while (0)
+    if (wide) {
+        if (H <= 8 * 256) LAUNCH_GNA(256);
+        else if (H <= 8 * 512) LAUNCH_GNA(512);
+        else LAUNCH_GNA(1024);
+    } else {
+        if (H <= 4 * kNT) LAUNCH_GNA_(kNT, 1, 4, 0);
+        else LAUNCH_GNA_(kNT, 1, 32, 0);
+    }
+    return check_launch("gate_norm_add_kernel");
+}
+
+}  // namespace
 
 extern "C" int skyrl_gate_norm_add(const void* a, const int64_t* rows, int32_t parts, const void* gate,
                                    int64_t gate_stride, const float* gate_bias, const void* weight, int32_t groups,
@@ -689,25 +734,21 @@ extern "C" int skyrl_gate_norm_add(const void* a, const int64_t* rows, int32_t p
     if (n == 0) return SKYRL_OK;
     SKYRL_REQUIRE(a && weight && hidden && next && out, "gate_norm_add: null pointer");
     SKYRL_DISPATCH_T(dtype, {
-        auto t = [](const void* q) { return reinterpret_cast<const T*>(q); };
-        const GateNormAdd<T> p{t(a), rows, parts, t(gate), gate_stride, gate_bias, t(weight), groups, eps, mult, hidden,
-                               fresh, t(next), reinterpret_cast<T*>(out), H};
-        const bool wide = H / groups % 8 == 0 && (!gate || (gate_stride % 8 == 0 && aligned16(gate))) && aligned16(a) &&
-                          aligned16(hidden) && aligned16(weight) && aligned16(next) && aligned16(out);
-        const int V = wide ? 8 : 1;
-        int L = 1;
-        while (L < kWave && H / V / groups % (2 * L) == 0) L <<= 1;
-        const size_t lds = groups > 1 ? (size_t)(H / V / L) * sizeof(float) : 0;
-        if (wide) {
-            if (H <= 8 * 256) LAUNCH_GNA(256);
-            else if (H <= 8 * 512) LAUNCH_GNA(512);
-            else LAUNCH_GNA(1024);
-        } else {
-            if (H <= 4 * kNT) LAUNCH_GNA_(kNT, 1, 4, 0);
-            else LAUNCH_GNA_(kNT, 1, 32, 0);
-        }
+        return launch_gate_norm_add<T, T>(a, false, rows, parts, gate, gate_stride, gate_bias, weight, groups, eps, mult,
+                                          hidden, fresh, next, n, H, out, as_stream(stream));
     })
-    return check_launch("gate_norm_add_kernel");
+}
+
+extern "C" int skyrl_gate_norm_add_parts(const float* a, int32_t parts, const void* gate, int64_t gate_stride,
+                                         const float* gate_bias, const void* weight, int32_t groups, float eps, float mult,
+                                         float* hidden, const void* next, int32_t n, int32_t H, void* out, void* stream) {
+    SKYRL_REQUIRE(n >= 0 && H > 0 && H <= 8192 && parts > 0, "gate_norm_add_parts: H must be in [1, 8192], parts positive");
+    SKYRL_REQUIRE(groups > 0 && H % groups == 0, "gate_norm_add_parts: H must be a multiple of groups");
+    SKYRL_REQUIRE(!gate || (gate_bias && gate_stride >= H), "gate_norm_add_parts: gate needs a bias and a stride >= H");
+    if (n == 0) return SKYRL_OK;
+    SKYRL_REQUIRE(a && weight && hidden && next && out, "gate_norm_add_parts: null pointer");
+    return launch_gate_norm_add<uint16_t, float>(a, true, nullptr, parts, gate, gate_stride, gate_bias, weight, groups, eps,
+                                                 mult, hidden, 0, next, n, H, out, as_stream(stream));
 }
 
 extern "C" int skyrl_tanh(const void* x, int64_t stride, int64_t n, int32_t I, void* out, int32_t dtype, void* stream) {

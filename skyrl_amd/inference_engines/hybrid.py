@@ -31,7 +31,6 @@ from dataclasses import dataclass, field
 from typing import Any, Dict, Iterable, Iterator, List, Optional, Tuple
 
 import torch
-import torch.nn.functional as F
 
 from . import kernels
 from . import layer_kernels as lk
@@ -337,12 +336,12 @@ class HybridDecoder:
             step = None if r.step is None else self.loop_step[r.step]
             for weight, sub in self.layers[r.layer]["subs"]:
                 lk.add_norm(delta, h, weight, step=step, out=x, **norm)
-                delta, step = sub.forward(x, inp, state, ws), None
+                delta, step = sub.forward(x, inp, state, ws, parts=True), None
             if trail is not None:
-                trail.append(h + delta.float())
+                trail.append(h + lk.joined(delta).float())
         if want is None:
             return lk.add_norm(delta, h, self.norm, out=x, **norm)
-        return lk.add_norm(None if delta is None else delta[want], h[want], self.norm, **norm)
+        return lk.add_norm(None if delta is None else delta.index_select(-2, want), h[want], self.norm, **norm)
 
     def _run_output_normed(self, inp: StepInputs, cache: HybridCache, want: Optional[torch.Tensor], trail=None):
         s = self.spec
@@ -387,7 +386,10 @@ class HybridDecoder:
                 lk.gate_norm_add(y, (full := h.clone()), after, self.norm, gate=gate, **args)
                 trail.append(full)
             if last and want is not None:
-                y = y.view(-1, sub.rows_per_token, s.hidden_size)[want].view(-1, s.hidden_size)
+                if y.dim() == 3:  # a product's parts
+                    y = y.index_select(1, want)
+                else:
+                    y = y.view(-1, sub.rows_per_token, s.hidden_size)[want].view(-1, s.hidden_size)
                 h, gate, x = h[want], gate[want], None
             x = lk.gate_norm_add(y, h, after, before[k + 1], gate=gate, out=x, **args)
             if trail is not None and k in ends and not last:
@@ -404,4 +406,4 @@ class HybridDecoder:
 
     def logits(self, hidden: torch.Tensor) -> torch.Tensor:
         """f32 [n, V]."""
-        return lk.softcap(F.linear(hidden, self.lm_head), self.spec.logit_softcap)
+        return lk.softcap(lk.linear(hidden, self.lm_head), self.spec.logit_softcap)

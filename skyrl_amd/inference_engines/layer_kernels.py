@@ -9,6 +9,7 @@ import ctypes
 from typing import Optional
 
 import torch
+import torch.nn.functional as F
 
 from .. import _ffi
 from ..ops import _ptr, _require_gpu, _stream
@@ -61,20 +62,79 @@ def embed(tokens: torch.Tensor, table: torch.Tensor, scale: float, positions: Op
     return out
 
 
+# ---------------------------------------------------------------- products of few rows
+MAX_ROWS = 128  # that skyrl_rows_product takes at most
+
+
+def _rows_fit(x: torch.Tensor, w: torch.Tensor, gated: bool = False) -> bool:
+    """Whether skyrl_rows_product takes x [n, K] (a column range) and w [N, K] of these sizes, types and alignments."""
+    n, K = x.shape
+    if n > MAX_ROWS:
+        return False
+    N = w.shape[0] // 2 if gated else w.shape[0]
+    return (x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.is_cuda
+            and bool(_ffi.query("skyrl_rows_product_fits", n, K, N, int(gated)))
+            and x.stride(1) == 1 and w.stride(1) == 1 and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0
+            and (n == 1 or x.stride(0) >= K) and w.stride(0) >= K and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+
+
+def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, parts: bool = False) -> torch.Tensor:
+    """x w^T + bias. Few bf16 rows take skyrl_rows_product, everything else the library. With `parts` the result of
+    few rows may be f32 [splits, n, N], to be summed over the first index where it is read (add_norm, gate_norm_add,
+    joined)."""
+    if not _rows_fit(x, w):
+        return F.linear(x, w, bias)
+    dev = _require_gpu(x, w, bias)
+    (n, K), N = x.shape, w.shape[0]
+    if w.shape[1] != K:
+        raise ValueError(f"w must be [N, {K}], got {tuple(w.shape)}")
+    _check(bias, "bias", torch.bfloat16, (N,))
+    splits = int(_ffi.query("skyrl_rows_product_splits", n, K, N)) if parts else 0
+    out = (torch.empty((splits, n, N), dtype=torch.float32, device=dev) if splits
+           else torch.empty((n, N), dtype=torch.bfloat16, device=dev))
+    _ffi.call("skyrl_rows_product", _ptr(x), x.stride(0), n, K, _ptr(w), w.stride(0), N, _ptr(bias), -1, 0.0, 0.0, splits,
+              _ptr(out), N, _stream(dev))
+    return out
+
+
+def joined(y: torch.Tensor) -> torch.Tensor:
+    """A product's rows [n, N] from what linear returned."""
+    return y if y.dim() == 2 else y.sum(0)
+
+
+def gated_linear(x: torch.Tensor, w: torch.Tensor, act: str, alpha: float = 1.0, limit: float = 0.0) -> Optional[torch.Tensor]:
+    """gate_mul of x w^T, w the gate rows and then the up rows, in one launch for few bf16 rows; None otherwise."""
+    if w.shape[0] % 2 or not _rows_fit(x, w, True):
+        return None
+    dev = _require_gpu(x, w)
+    (n, K), N = x.shape, w.shape[0] // 2
+    if w.shape[1] != K:
+        raise ValueError(f"w must be [2 N, {K}], got {tuple(w.shape)}")
+    out = torch.empty((n, N), dtype=torch.bfloat16, device=dev)
+    _ffi.call("skyrl_rows_product", _ptr(x), x.stride(0), n, K, _ptr(w), w.stride(0), N, None, ACTIVATIONS[act], float(alpha),
+              float(limit), 0, _ptr(out), N, _stream(dev))
+    return out
+
+
 def add_norm(delta: Optional[torch.Tensor], hidden: torch.Tensor, weight: torch.Tensor, eps: float,
              kind: str = "layer", step: Optional[torch.Tensor] = None,
              out: Optional[torch.Tensor] = None, base: float = 0.0) -> torch.Tensor:
     """hidden (f32, in place) += delta and += step (one vector for every row), then the norm, times
-    base + weight (base 1: the weight is stored as its distance from 1)."""
+    base + weight (base 1: the weight is stored as its distance from 1). delta: rows, or linear's f32 parts."""
     dev = _require_gpu(hidden, weight, delta, step, out)
     n, H = hidden.shape
+    parts = delta.shape[0] if delta is not None and delta.dim() == 3 else 0
     _check(hidden, "hidden", torch.float32)
-    _check(weight, "weight", weight.dtype, (H,))
-    _check(delta, "delta", weight.dtype, (n, H))
+    _check(weight, "weight", torch.bfloat16 if parts else weight.dtype, (H,))
+    _check(delta, "delta", torch.float32 if parts else weight.dtype, (parts, n, H) if parts else (n, H))
     _check(step, "step", weight.dtype, (H,))
     if out is None:
         out = torch.empty((n, H), dtype=weight.dtype, device=dev)
     _check(out, "out", weight.dtype, (n, H))
+    if parts:
+        _ffi.call("skyrl_add_norm_parts", _ptr(delta), parts, _ptr(hidden), _ptr(step), _ptr(weight), float(base), n, H,
+                  float(eps), NORMS[kind], _ptr(out), _stream(dev))
+        return out
     _ffi.call("skyrl_add_norm", _ptr(delta), _ptr(hidden), _ptr(step), _ptr(weight), float(base), n, H, float(eps),
               NORMS[kind], _ptr(out), _code(weight), _stream(dev))
     return out
@@ -113,13 +173,19 @@ def gate_norm_add(a: torch.Tensor, hidden: torch.Tensor, weight: torch.Tensor, n
                   out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """hidden (f32 [n, H], in place; fresh: from 0) += mult norm(y) weight, y the sum of `parts` consecutive rows of a,
     times sigmoid(gate + gate_bias) with a gate; returns norm(hidden) next_weight. A norm is an RMS norm in `groups`
-    equal parts of the row. `rows` int64 [n]: which rows of a (parts 1)."""
+    equal parts of the row. `rows` int64 [n]: which rows of a (parts 1). a may be linear's f32 parts (`parts` 1)."""
     dev = _require_gpu(a, hidden, weight, next_weight, gate, gate_bias, rows, out)
     n, H = hidden.shape
     _check(hidden, "hidden", torch.float32)
-    if a.dim() != 2 or a.shape[1] != H or (rows is None and a.shape[0] != n * parts) or (rows is not None and parts != 1):
+    shares = a.shape[0] if a.dim() == 3 else 0
+    if shares:
+        if rows is not None or parts != 1 or fresh or weight.dtype != torch.bfloat16:
+            raise ValueError("a product's parts are of a model in bfloat16, one row per token, added to the residual")
+        _check(a, "a", torch.float32, (shares, n, H))
+    elif a.dim() != 2 or a.shape[1] != H or (rows is None and a.shape[0] != n * parts) or (rows is not None and parts != 1):
         raise ValueError(f"a must be [{n} * parts, {H}], with rows [any, {H}] and one part")
-    _check(a, "a", weight.dtype)
+    if not shares:
+        _check(a, "a", weight.dtype)
     _check(weight, "weight", weight.dtype, (H,))
     _check(next_weight, "next_weight", weight.dtype, (H,))
     _check(rows, "rows", torch.int64, (n,))
@@ -131,6 +197,11 @@ def gate_norm_add(a: torch.Tensor, hidden: torch.Tensor, weight: torch.Tensor, n
     if out is None:
         out = torch.empty((n, H), dtype=weight.dtype, device=dev)
     _check(out, "out", weight.dtype, (n, H))
+    if shares:
+        _ffi.call("skyrl_gate_norm_add_parts", _ptr(a), shares, _ptr(gate), 0 if gate is None else max(gate.stride(0), H),
+                  _ptr(gate_bias), _ptr(weight), groups, float(eps), float(mult), _ptr(hidden), _ptr(next_weight), n, H,
+                  _ptr(out), _stream(dev))
+        return out
     _ffi.call("skyrl_gate_norm_add", _ptr(a), _ptr(rows), parts, _ptr(gate), 0 if gate is None else max(gate.stride(0), H),
               _ptr(gate_bias), _ptr(weight), groups, float(eps), float(mult), _ptr(hidden), int(fresh), _ptr(next_weight), n, H,
               _ptr(out), _code(weight), _stream(dev))

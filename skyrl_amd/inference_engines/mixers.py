@@ -204,6 +204,7 @@ class Products:
 
     def __init__(self, parts: List[Any], width: int, w: Weights, apart: bool = False, beside: int = 0):
         self.parts, self.ranges, self.apart, self.beside = parts, [], apart, None
+        self.fused = None  # of a single part: input product and `inner` in one launch, for few rows
         a = c = 0
         for p in parts:
             self.ranges.append((a, c))
@@ -224,6 +225,8 @@ class Products:
         self.w_out = w.matrix(width, c)
         self.b_out = w.zeros(width) if any(p.out_bias for p in parts) else None
         self.padded = any(p.out_cols % 8 for p in parts)
+        if len(parts) == 1 and not beside and not self.padded:
+            self.fused = getattr(parts[0], "fused", None)
         for p, (a, c) in zip(parts, self.ranges):
             p.bind(self.w_in[a:a + p.in_rows], self.b_in[a:a + p.in_rows] if p.in_bias else None,
                    self.w_out[:, c:c + p.out_cols], self.b_out if p.out_bias else None)
@@ -232,20 +235,25 @@ class Products:
     def biased(self) -> bool:
         return self.b_in is not None or any(p.out_bias for p in self.parts)
 
-    def forward(self, x: torch.Tensor, inp, state, workspace):
-        proj = F.linear(x, self.w_in, self.b_in)
+    def forward(self, x: torch.Tensor, inp, state, workspace, parts: bool = False):
+        """parts: the output may be layer_kernels.linear's parts (not with `apart`)."""
+        if self.fused is not None:
+            cat = self.fused(x)
+            if cat is not None:
+                return lk.linear(cat, self.w_out, self.b_out, parts)
+        proj = lk.linear(x, self.w_in, self.b_in)
         if self.apart:
             outs = []
             for p, (a, _), (wo, bo), st in zip(self.parts, self.ranges, self.outs, state):
                 o = torch.empty((x.shape[0], p.out_cols), dtype=x.dtype, device=x.device)
                 p.inner(proj[:, a:a + p.in_rows], o, inp, st, workspace)
-                outs.append(F.linear(o, wo, bo))
+                outs.append(lk.linear(o, wo, bo))
             return tuple(outs)
         make = torch.zeros if self.padded else torch.empty  # padding columns meet weights: they must be finite
         cat = make((x.shape[0], self.w_out.shape[1]), dtype=x.dtype, device=x.device)
         for p, (a, c) in zip(self.parts, self.ranges):
             p.inner(proj[:, a:a + p.in_rows], cat[:, c:c + p.out_cols], inp, state, workspace)
-        y = F.linear(cat, self.w_out, self.b_out)
+        y = lk.linear(cat, self.w_out, self.b_out, parts)
         return y if self.beside is None else (y, proj[:, self.beside[0]:self.beside[1]])
 
 
@@ -265,8 +273,8 @@ class Gated:
 
     def forward(self, x: torch.Tensor, inp, state, workspace):
         if isinstance(self.sub, Products):
-            return self.sub.forward(x, inp, state, workspace)
-        return self.sub.forward(x, inp, state, workspace), F.linear(x, self.weight)
+            return self.sub.forward(x, inp, state, workspace, parts=True)
+        return self.sub.forward(x, inp, state, workspace), lk.linear(x, self.weight)
 
 
 class LatentAttention:
@@ -382,7 +390,7 @@ class LatentAttention:
         lk.latent_write(proj, *where, halves=self.halves, **first, **own)
         q = proj[:, :self.q_rows]
         if qr:
-            q = F.linear(q, self.wuq)
+            q = lk.linear(q, self.wuq)
             lk.latent_write(q, *where, heads=H, dim=self.dim, halves=self.halves)
         gate = None if self.gate_at is None else proj[:, self.gate_at:]
         prompt = inp.plan is not None and self.window in inp.plan and lk.prefill_fits(self.dim, self.rot_dim, self.vdim, self.dtype)
@@ -457,9 +465,9 @@ class GatedDelta:
         yield "chunks", lambda: chunk_plan(seq_lens, first_seq, first_token)
 
     # ---- step
-    def forward(self, x: torch.Tensor, inp, state, workspace) -> torch.Tensor:
+    def forward(self, x: torch.Tensor, inp, state, workspace, parts: bool = False) -> torch.Tensor:
         S, ring = state
-        proj = F.linear(x, self.wproj)
+        proj = lk.linear(x, self.wproj)
         out = torch.empty((x.shape[0], self.heads * self.vdim), dtype=self.dtype, device=x.device)
         args = (self.conv, self.a_log, self.dt_bias, self.norm)
         n = inp.rows.shape[0]
@@ -474,7 +482,7 @@ class GatedDelta:
                             inp.short_tokens, out)
         if not inp.one_token:
             lk.conv_save(proj, lk.delta_channels(self.shape), inp.cu, inp.rows, inp.positions, ring)
-        return F.linear(out, self.wo)
+        return lk.linear(out, self.wo, parts=parts)
 
 
 class GeneralDelta:
@@ -538,7 +546,7 @@ class GeneralDelta:
 
     # ---- step
     def inner(self, proj: torch.Tensor, out: torch.Tensor, inp, state: torch.Tensor, workspace) -> None:
-        wl = F.linear(lk.tanh(proj[:, 5 * self.out_cols:]), self.w2)
+        wl = lk.linear(lk.tanh(proj[:, 5 * self.out_cols:]), self.w2)
         args = (proj, wl, self.w0, self.a_bias, self.norm)
         n = inp.rows.shape[0]
         prompt = inp.plan is not None and "chunks" in inp.plan
@@ -992,6 +1000,9 @@ class GatedMLP:
         if self.in_bias:
             yield from split_rows(self.bgu, (("gate.b", self.ff), ("up.b", self.ff)))
             yield "down.b", self.bd
+
+    def fused(self, x: torch.Tensor) -> Optional[torch.Tensor]:
+        return None if self.in_bias else lk.gated_linear(x, self.wgu, self.act, self.alpha, self.limit)
 
     def inner(self, proj: torch.Tensor, out: torch.Tensor, inp, state, workspace) -> None:
         lk.gate_mul(proj, self.act, self.alpha, self.limit, out=out)

@@ -1,0 +1,104 @@
+"""Products of few rows (csrc/rows_product.hip) against f64: every kernel form at the edges of its tiles, remainders of the
+depth and of the columns, strided rows, biases, f32 parts and the norms that read them, gated products."""
+
+import pytest
+import torch
+
+from skyrl_amd.inference_engines import layer_kernels as lk
+
+pytestmark = pytest.mark.gpu
+
+# rows on both sides of every form's limit; columns: scalar tail, one tile, wide tiles with a remainder; depths below a
+# piece, with a remainder, with unequal shares
+SHAPES = [(1, 17, 8), (1, 203, 2072), (1, 8200, 520), (2, 16, 64), (3, 203, 72), (16, 40, 1000), (16, 8200, 136),
+          (17, 50, 328), (32, 8192, 64), (33, 24, 712), (48, 96, 2048), (64, 8216, 200), (64, 1000, 1544), (65, 64, 264),
+          (128, 4096, 72), (100, 136, 1088)]
+
+
+def _data(dev, n, N, K, seed, pad=0):
+    g = torch.Generator(device=dev).manual_seed(seed)
+    x = torch.randn(n, K + pad, device=dev, generator=g).bfloat16()[:, :K]
+    w = torch.randn(N, K + pad, device=dev, generator=g).bfloat16()[:, :K]
+    b = torch.randn(N, device=dev, generator=g).bfloat16()
+    return x, w, b
+
+
+def _bounds(x, w):
+    """The exact product and what f32 sums of its exact terms, in any order, may be off by."""
+    y = x.double() @ w.double().t()
+    return y, x.shape[1] * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t()) + 1e-30
+
+
+@pytest.mark.parametrize("n,N,K", SHAPES)
+@pytest.mark.parametrize("pad", (0, 24))
+def test_products(dev, n, N, K, pad):
+    x, w, b = _data(dev, n, N, K, n + N, pad)
+    assert lk._rows_fit(x, w)
+    ref, off = _bounds(x, w)
+    for bias in (None, b):
+        want = ref if bias is None else ref + bias.double()
+        y = lk.linear(x, w, bias)
+        assert y.dtype == torch.bfloat16 and bool(((y.double() - want).abs() <= 2.0 ** -8 * want.abs() + 2 * off).all())
+        parts = lk.linear(x, w, bias, parts=True)
+        assert parts.dtype == torch.float32 and parts.shape[1:] == (n, N)
+        assert bool(((lk.joined(parts).double() - want).abs() <= 2 * off + 2.0 ** -21 * want.abs()).all())
+
+
+@pytest.mark.parametrize("act", ("silu", "gelu_tanh", "clamped"))
+@pytest.mark.parametrize("n,N,K", [(1, 100, 264), (2, 8, 64), (16, 4100, 136), (17, 36, 200), (32, 72, 1032), (33, 132, 520),
+                                   (64, 6144, 72)])
+def test_gated(dev, n, N, K, act):
+    x, w, _ = _data(dev, n, 2 * N, K, 5 * n)
+    y = lk.gated_linear(x, w, act, 1.702, 7.0)
+    z, off = _bounds(x, w)
+    g, u = z[:, :N], z[:, N:]
+    if act == "silu":
+        ref = g * torch.sigmoid(g) * u
+    elif act == "gelu_tanh":
+        ref = torch.nn.functional.gelu(g, approximate="tanh") * u
+    else:
+        g, u = g.clamp(max=7.0), u.clamp(-7.0, 7.0)
+        ref = g * torch.sigmoid(1.702 * g) * (u + 1)
+    slack = 1.2 * off[:, :N] * (u.abs() + 1) + (g.abs() + 1) * off[:, N:]  # the gates' slopes are at most 1.2
+    assert bool(((y.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2 * slack + 1e-5 * (g * u).abs() + 1e-6).all())
+
+
+def test_what_the_library_takes(dev):
+    x, w, _ = _data(dev, 129, 64, 64, 0)
+    assert not lk._rows_fit(x, w)                                  # too many rows
+    assert not lk._rows_fit(*_data(dev, 65, 4104, 64, 0)[:2])
+    assert not lk._rows_fit(*_data(dev, 4, 64, 60, 0)[:2])         # depth no multiple of 8
+    big = torch.randn(4, 132, device=dev).bfloat16()
+    assert not lk._rows_fit(big[:, 1:65], w)                       # misaligned rows
+    assert not lk._rows_fit(big[:, :64], w)                        # and row strides
+    assert not lk._rows_fit(x[:4].float(), w.float())
+    assert lk.gated_linear(x[:65], w, "silu") is None
+    for a, b in ((big[:, 1:65], w), (x, w), (x[:4].float(), w.float())):
+        torch.testing.assert_close(lk.linear(a, b, parts=True), torch.nn.functional.linear(a, b))
+    with pytest.raises(ValueError):
+        lk.linear(x[:4], torch.zeros(8, 72, device=dev, dtype=torch.bfloat16))
+
+
+@pytest.mark.parametrize("n,H", [(1, 40), (3, 203), (16, 2048), (64, 1536), (70, 4096)])
+@pytest.mark.parametrize("parts", (1, 2, 3, 4, 8))
+def test_norms_of_parts(dev, n, H, parts):
+    g = torch.Generator(device=dev).manual_seed(parts)
+    r = lambda *s: torch.randn(*s, device=dev, generator=g)  # noqa: E731
+    d, h = r(parts, n, H), r(n, H)
+    w, step, nxt, b = r(H).bfloat16(), r(H).bfloat16(), r(H).bfloat16(), r(H)
+    full = h.double() + d.double().sum(0) + step.double()
+    got = h.clone()
+    y = lk.add_norm(d, got, w, 1e-6, "layer", step=step)
+    c = full - full.mean(1, keepdim=True)
+    torch.testing.assert_close(got.double(), full, atol=4e-6, rtol=1e-6)
+    torch.testing.assert_close(y.double(), c / c.square().mean(1, keepdim=True).add(1e-6).sqrt() * w.double(), atol=1e-4, rtol=2 ** -8)
+    for groups in (1, 4):
+        if H % groups:
+            continue
+        norm = lambda v: (v.view(n, groups, -1) / v.view(n, groups, -1).square().mean(-1, keepdim=True).add(1e-6).sqrt()).view(n, H)  # noqa: E731
+        z = r(n, H).bfloat16()
+        full = h.double() + 0.5 * norm(d.double().sum(0) * torch.sigmoid(z.double() + b.double())) * w.double()
+        got = h.clone()
+        y = lk.gate_norm_add(d, got, w, nxt, 1e-6, groups=groups, mult=0.5, gate=z, gate_bias=b)
+        torch.testing.assert_close(got.double(), full, atol=2e-5, rtol=1e-5)
+        torch.testing.assert_close(y.double(), norm(full) * nxt.double(), atol=1e-4, rtol=2 ** -8)
