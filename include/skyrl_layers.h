@@ -54,7 +54,8 @@ extern "C" {
  *                   of skyrl_gate_mul: w holds N gate rows, then N up rows; the gated product bf16 [n, N], splits 0.
  *                   skyrl_rows_product_fits: whether it takes the sizes; skyrl_rows_product_splits: the splits.
  *   skyrl_add_norm_parts, skyrl_gate_norm_add_parts  of a model in bf16, the sublayer's output being such a sum of
- *                   `parts` f32 [n, H]. */
+ *                   `parts` (a_shares > 0) f32 [n, H], or (gate_shares > 0) the gate's logits being one of f32
+ *                   [n, gate_stride]. */
 #define SKYRL_NORM_LAYER 0
 #define SKYRL_NORM_RMS 1
 #define SKYRL_ACT_SILU 0
@@ -84,9 +85,9 @@ int skyrl_rows_product(const void* x, int64_t ldx, int32_t n, int32_t K, const v
                        void* stream);
 int skyrl_add_norm_parts(const float* delta, int32_t parts, float* hidden, const void* step, const void* weight, float w_base,
                          int32_t n, int32_t H, float eps, int32_t kind, void* out, void* stream);
-int skyrl_gate_norm_add_parts(const float* a, int32_t parts, const void* gate, int64_t gate_stride, const float* gate_bias,
-                              const void* weight, int32_t groups, float eps, float mult, float* hidden, const void* next,
-                              int32_t n, int32_t H, void* out, void* stream);
+int skyrl_gate_norm_add_parts(const void* a, int32_t a_shares, int32_t parts, const void* gate, int32_t gate_shares,
+                              int64_t gate_stride, const float* gate_bias, const void* weight, int32_t groups, float eps,
+                              float mult, float* hidden, const void* next, int32_t n, int32_t H, void* out, void* stream);
 int skyrl_tanh(const void* x, int64_t stride, int64_t n, int32_t I, void* out, int32_t dtype, void* stream);
 int skyrl_conv_save(const void* x, int64_t stride, int32_t channels, int32_t taps, const int32_t* cu,
                     const int32_t* rows, const int64_t* positions, int32_t nseq, void* ring, int32_t dtype,
@@ -387,6 +388,8 @@ int skyrl_gdelta_out(const skyrl_gdelta_shape* shape, const int32_t* chunk, int3
  * correction f32 [experts]; of `groups` equal groups of neighbours the `keep` with the largest sum of their two largest
  * choice scores may be chosen from; the `top` largest of those are, ties to the lower index. Pair p = token * top + i.
  *   skyrl_moe_route    idx i32 [n, top], weight f32 [n, top] (the scores s of the chosen).
+ *   skyrl_moe_choose   the same from logits f32 that are the sum of `shares` rows share_stride apart, row_stride between
+ *                      tokens (at most 64 experts), and, with order, skyrl_moe_sort of them (at most 128 pairs).
  *   skyrl_moe_tiles    the most tiles of tm rows that npairs pairs can fill.
  *   skyrl_moe_sort     pairs by expert: order i32 [ntiles, tm] (pair, or -1), tile_expert i32 [ntiles + 1] (-1: unused; the
  *                      last: tiles in use). counts: scratch of skyrl_moe_counts(experts, npairs) i32 (0: NULL).
@@ -398,6 +401,9 @@ typedef struct {
 } skyrl_moe_shape;
 int skyrl_moe_route(const skyrl_moe_shape* shape, const void* x, int32_t n, const void* router, const float* correction,
                     int32_t* idx, float* weight, int32_t dtype, void* stream);
+int skyrl_moe_choose(const skyrl_moe_shape* shape, const float* logits, int32_t shares, int64_t share_stride,
+                     int64_t row_stride, int32_t n, const float* correction, int32_t* idx, float* weight, int32_t tm,
+                     int32_t ntiles, int32_t* order, int32_t* tile_expert, void* stream);
 int32_t skyrl_moe_tiles(int32_t experts, int32_t npairs, int32_t tm);
 int32_t skyrl_moe_counts(int32_t experts, int32_t npairs);
 int skyrl_moe_sort(const int32_t* idx, int32_t npairs, int32_t experts, int32_t tm, int32_t ntiles, int32_t* counts,

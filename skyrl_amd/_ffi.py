@@ -291,7 +291,7 @@ LAYERS_SIGNATURES = {
     "skyrl_rows_product_splits": (_I32, [_I32, _I32, _I32]),
     "skyrl_rows_product": (_INT, [_P, _I64, _I32, _I32, _P, _I64, _I32, _P, _I32, _F, _F, _I32, _P, _I64, _P]),
     "skyrl_add_norm_parts": (_INT, [_P, _I32, _P, _P, _P, _F, _I32, _I32, _F, _I32, _P, _P]),
-    "skyrl_gate_norm_add_parts": (_INT, [_P, _I32, _P, _I64, _P, _P, _I32, _F, _F, _P, _P, _I32, _I32, _P, _P]),
+    "skyrl_gate_norm_add_parts": (_INT, [_P, _I32, _I32, _P, _I32, _I64, _P, _P, _I32, _F, _F, _P, _P, _I32, _I32, _P, _P]),
     "skyrl_tanh": (_INT, [_P, _I64, _I64, _I32, _P, _I32, _P]),
     "skyrl_latent_write": (_INT, [_P, _I64, _I32, _I32, _I32, _I32, _I32, _I32, _P, _I32, _I32, _P, _F, _P, _P, _P, _P, _I32,
                                   _I32, _P]),
@@ -334,6 +334,7 @@ LAYERS_SIGNATURES = {
     "skyrl_gdelta_chain": (_INT, [_GS, _P, _P, _I32, _I32, _P, _P, _P, _P, _P, _P, _P, _P]),
     "skyrl_gdelta_out": (_INT, [_GS, _P, _I32, _P, _P, _P, _P, _I64, _P, _P, _I64, _I32, _P]),
     "skyrl_moe_route": (_INT, [_MS, _P, _I32, _P, _P, _P, _P, _I32, _P]),
+    "skyrl_moe_choose": (_INT, [_MS, _P, _I32, _I64, _I64, _I32, _P, _P, _P, _I32, _I32, _P, _P, _P]),
     "skyrl_moe_tiles": (_I32, [_I32, _I32, _I32]),
     "skyrl_moe_counts": (_I32, [_I32, _I32]),
     "skyrl_moe_sort": (_INT, [_P, _I32, _I32, _I32, _I32, _P, _P, _P, _P]),

@@ -388,14 +388,15 @@ __global__ __launch_bounds__(NT) void gated_norm_kernel(const T* __restrict__ y,
 }
 
 // ---- a sublayer's result between two norms in equal parts: gated, normed, added to the residual, normed again ----
-template <typename T, typename A>
+template <typename T, typename A, typename Z>
 struct GateNormAdd {
     const A* a;
     const int64_t* rows;  // row of a (NULL: the output's own)
     int parts;            // rows of a that are summed, part_stride apart
     int64_t row_stride, part_stride;
-    const T* z;           // gate logits (NULL: no gate) and their bias
-    int64_t z_stride;
+    const Z* z;           // gate logits (NULL: no gate), the sum of z_parts rows, and their bias
+    int z_parts;
+    int64_t z_stride, z_part_stride;
     const float* zb;
     const T* w;
     int groups;
@@ -410,8 +411,8 @@ struct GateNormAdd {
 // One block per row, the row in registers: chunks of VEC elements, chunk threadIdx + k NT, each in one group of `per`
 // chunks. A group's sum: within L lanes (the power of two in per, at most a wave) by shuffles, then over per / L numbers
 // in LDS. PARTS: rows that are summed (0: any number).
-template <typename T, typename A, int NT, int VEC, int kMaxV, int PARTS>
-__global__ __launch_bounds__(NT) void gate_norm_add_kernel(GateNormAdd<T, A> p, int L) {
+template <typename T, typename A, typename Z, int NT, int VEC, int kMaxV, int PARTS>
+__global__ __launch_bounds__(NT) void gate_norm_add_kernel(GateNormAdd<T, A, Z> p, int L) {
     extern __shared__ float s_p[];
     __shared__ float s_red[NT / kWave];
     const int nv = p.H / VEC, per = nv / p.groups, sums = per / L;
@@ -479,7 +480,17 @@ __global__ __launch_bounds__(NT) void gate_norm_add_kernel(GateNormAdd<T, A> p, 
             }
             if (p.z) {
                 float z[VEC], b[VEC];
-                ldv<T, VEC>(p.z + blockIdx.x * p.z_stride + VEC * v, z);
+                const Z* zp = p.z + blockIdx.x * p.z_stride + VEC * v;
+                ldv<Z, VEC>(zp, z);
+                if constexpr (sizeof(Z) > sizeof(T)) {
+#pragma unroll 4
+                    for (int i = 1; i < p.z_parts; ++i) {
+                        float x[VEC];
+                        ldv<Z, VEC>(zp + i * p.z_part_stride, x);
+#pragma unroll
+                        for (int j = 0; j < VEC; ++j) z[j] += x[j];
+                    }
+                }
                 ldv<float, VEC>(p.zb + VEC * v, b);
 #pragma unroll
                 for (int j = 0; j < VEC; ++j) y[k][j] *= sigmoid_<T>(z[j] + b[j]);
@@ -687,21 +698,22 @@ extern "C" int skyrl_xielu(const void* x, int64_t stride, int64_t n, int32_t I, 
 namespace {
 
 // The rows of a: `parts` of a token one after another, or (SHARES) a product's shares of the depth, n rows each.
-template <typename T, typename A>
-int launch_gate_norm_add(const void* a, bool shares, const int64_t* rows, int parts, const void* gate, int64_t gate_stride,
-                         const float* gate_bias, const void* weight, int groups, float eps, float mult, float* hidden,
-                         int fresh, const void* next, int n, int H, void* out, hipStream_t s) {
+template <typename T, typename A, typename Z>
+int launch_gate_norm_add(const void* a, bool shares, const int64_t* rows, int parts, const void* gate, int gate_shares,
+                         int64_t gate_stride, const float* gate_bias, const void* weight, int groups, float eps, float mult,
+                         float* hidden, int fresh, const void* next, int n, int H, void* out, hipStream_t s) {
     auto t = [](const void* q) { return reinterpret_cast<const T*>(q); };
-    const GateNormAdd<T, A> p{reinterpret_cast<const A*>(a), rows, parts, shares ? H : (int64_t)parts * H,
-                              shares ? (int64_t)n * H : H, t(gate), gate_stride, gate_bias, t(weight), groups, eps, mult,
-                              hidden, fresh, t(next), reinterpret_cast<T*>(out), H};
+    const GateNormAdd<T, A, Z> p{reinterpret_cast<const A*>(a), rows, parts, shares ? H : (int64_t)parts * H,
+                                 shares ? (int64_t)n * H : H, reinterpret_cast<const Z*>(gate), gate_shares, gate_stride,
+                                 n * gate_stride, gate_bias, t(weight), groups, eps, mult, hidden, fresh, t(next),
+                                 reinterpret_cast<T*>(out), H};
     const bool wide = H / groups % 8 == 0 && (!gate || (gate_stride % 8 == 0 && aligned16(gate))) && aligned16(a) &&
                       aligned16(hidden) && aligned16(weight) && aligned16(next) && aligned16(out);
     const int V = wide ? 8 : 1;
     int L = 1;
     while (L < kWave && H / V / groups % (2 * L) == 0) L <<= 1;
     const size_t lds = groups > 1 ? (size_t)(H / V / L) * sizeof(float) : 0;
-#define LAUNCH_GNA_(NT, V, K, P) hipLaunchKernelGGL((gate_norm_add_kernel<T, A, NT, V, K, P>), dim3(n), dim3(NT), lds, s, p, L)
+#define LAUNCH_GNA_(NT, V, K, P) hipLaunchKernelGGL((gate_norm_add_kernel<T, A, Z, NT, V, K, P>), dim3(n), dim3(NT), lds, s, p, L)
 #define LAUNCH_GNA(NT)                              \
     do {                                            \
         if (parts == 1) LAUNCH_GNA_(NT, 8, 1, 1);   \
@@ -734,21 +746,29 @@ extern "C" int skyrl_gate_norm_add(const void* a, const int64_t* rows, int32_t p
     if (n == 0) return SKYRL_OK;
     SKYRL_REQUIRE(a && weight && hidden && next && out, "gate_norm_add: null pointer");
     SKYRL_DISPATCH_T(dtype, {
-        return launch_gate_norm_add<T, T>(a, false, rows, parts, gate, gate_stride, gate_bias, weight, groups, eps, mult,
+        return launch_gate_norm_add<T, T, T>(a, false, rows, parts, gate, 1, gate_stride, gate_bias, weight, groups, eps, mult,
                                           hidden, fresh, next, n, H, out, as_stream(stream));
     })
 }
 
-extern "C" int skyrl_gate_norm_add_parts(const float* a, int32_t parts, const void* gate, int64_t gate_stride,
-                                         const float* gate_bias, const void* weight, int32_t groups, float eps, float mult,
-                                         float* hidden, const void* next, int32_t n, int32_t H, void* out, void* stream) {
-    SKYRL_REQUIRE(n >= 0 && H > 0 && H <= 8192 && parts > 0, "gate_norm_add_parts: H must be in [1, 8192], parts positive");
+extern "C" int skyrl_gate_norm_add_parts(const void* a, int32_t a_shares, int32_t parts, const void* gate, int32_t gate_shares,
+                                         int64_t gate_stride, const float* gate_bias, const void* weight, int32_t groups,
+                                         float eps, float mult, float* hidden, const void* next, int32_t n, int32_t H, void* out,
+                                         void* stream) {
+    SKYRL_REQUIRE(n >= 0 && H > 0 && H <= 8192 && parts > 0 && a_shares >= 0 && gate_shares >= 0,
+                  "gate_norm_add_parts: H must be in [1, 8192], parts positive");
     SKYRL_REQUIRE(groups > 0 && H % groups == 0, "gate_norm_add_parts: H must be a multiple of groups");
     SKYRL_REQUIRE(!gate || (gate_bias && gate_stride >= H), "gate_norm_add_parts: gate needs a bias and a stride >= H");
+    SKYRL_REQUIRE((a_shares > 0) != (gate_shares > 0) && (!a_shares || parts == 1),
+                  "gate_norm_add_parts: shares of the output or of the gate");
     if (n == 0) return SKYRL_OK;
-    SKYRL_REQUIRE(a && weight && hidden && next && out, "gate_norm_add_parts: null pointer");
-    return launch_gate_norm_add<uint16_t, float>(a, true, nullptr, parts, gate, gate_stride, gate_bias, weight, groups, eps,
-                                                 mult, hidden, 0, next, n, H, out, as_stream(stream));
+    SKYRL_REQUIRE(a && weight && hidden && next && out && (gate || !gate_shares), "gate_norm_add_parts: null pointer");
+    if (a_shares)
+        return launch_gate_norm_add<uint16_t, float, uint16_t>(a, true, nullptr, a_shares, gate, 1, gate_stride, gate_bias, weight,
+                                                               groups, eps, mult, hidden, 0, next, n, H, out, as_stream(stream));
+    return launch_gate_norm_add<uint16_t, uint16_t, float>(a, false, nullptr, parts, gate, gate_shares, gate_stride, gate_bias,
+                                                           weight, groups, eps, mult, hidden, 0, next, n, H, out,
+                                                           as_stream(stream));
 }
 
 extern "C" int skyrl_tanh(const void* x, int64_t stride, int64_t n, int32_t I, void* out, int32_t dtype, void* stream) {

@@ -216,9 +216,10 @@ __global__ __launch_bounds__(1024) void moe_count_kernel(const int32_t* __restri
     __syncthreads();
     for (int e = threadIdx.x; e < experts; e += 1024) counts[blockIdx.x * experts + e] = s_n[e];
 }
-__global__ __launch_bounds__(1024) void moe_sort_kernel(const int32_t* __restrict__ idx, int npairs, int experts, int tm,
-                                                        int ntiles, int span, const int32_t* __restrict__ counts,
-                                                        int32_t* __restrict__ order, int32_t* __restrict__ tile_expert) {
+// The sort of a workgroup of 1024 threads.
+__device__ __forceinline__ void sort_pairs(const int32_t* idx, int npairs, int experts, int tm, int ntiles, int span,
+                                           const int32_t* __restrict__ counts, int32_t* __restrict__ order,
+                                           int32_t* __restrict__ tile_expert) {
     __shared__ int s_n[kMaxExperts], s_at[kMaxExperts], s_sum[16];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int p0 = blockIdx.x * span, p1 = min(npairs, p0 + span);
@@ -266,6 +267,39 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(const int32_t* __restric
     }
     __syncthreads();
     for (int p = p0 + tid; p < p1; p += 1024) order[atomicAdd(&s_at[idx[p]], 1)] = p;
+}
+__global__ __launch_bounds__(1024) void moe_sort_kernel(const int32_t* __restrict__ idx, int npairs, int experts, int tm,
+                                                        int ntiles, int span, const int32_t* __restrict__ counts,
+                                                        int32_t* __restrict__ order, int32_t* __restrict__ tile_expert) {
+    sort_pairs(idx, npairs, experts, tm, ntiles, span, counts, order, tile_expert);
+}
+
+// Choice from logits that another product formed (up to 64 experts): the sum of `shares` f32 rows, share_stride apart. A
+// wave per token: a choice is some 200 dependent instructions, so few waves share a CU. SORT: one workgroup has all pairs,
+// at most kChosen, and lists them too; with more tokens its CU would be what is waited for (64 tokens: 24 us in one
+// workgroup, 8 in two launches). The router's own product took 14 to 16 us: one workgroup per 16 tokens read the whole router.
+constexpr int kChosen = 128;
+template <bool SORT>
+__global__ __launch_bounds__(SORT ? 1024 : kNT) void moe_choose_kernel(
+    Router ro, const float* __restrict__ z, int shares, int64_t share_stride, int64_t ld_, int n,
+    const float* __restrict__ correction, int32_t* __restrict__ idx, float* __restrict__ weight, int tm, int ntiles,
+    int32_t* __restrict__ order, int32_t* __restrict__ tile_expert) {
+    constexpr int NWV = (SORT ? 1024 : kNT) / kWave;
+    __shared__ float s_own[NWV][4 * kWave];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, e = min(lane, ro.experts - 1);
+    float* own = s_own[wave];
+    for (int t = blockIdx.x * NWV + wave; t < n; t += gridDim.x * NWV) {
+        float v = 0.f;
+#pragma unroll 4
+        for (int i = 0; i < shares; ++i) v += z[i * share_stride + t * ld_ + e];
+        own[lane] = v;  // pick reads its own lane's
+        pick<1>(ro, own, correction, own + kWave, own + 2 * kWave, own + 3 * kWave, lane, idx + (int64_t)t * ro.top,
+                weight + (int64_t)t * ro.top);
+    }
+    if constexpr (SORT) {
+        __syncthreads();  // the choices, written by this workgroup
+        sort_pairs(idx, n * ro.top, ro.experts, tm, ntiles, n * ro.top, nullptr, order, tile_expert);
+    }
 }
 
 // ---- products, any size and type: 16 rows x 64 columns per workgroup ---------------------------------
@@ -589,6 +623,31 @@ extern "C" int skyrl_moe_route(const skyrl_moe_shape* shape, const void* x, int3
                            reinterpret_cast<const T*>(router), correction, idx, weight);
     })
     return check_launch("moe_route_plain_kernel");
+}
+
+extern "C" int skyrl_moe_choose(const skyrl_moe_shape* shape, const float* logits, int32_t shares, int64_t share_stride,
+                                int64_t row_stride, int32_t n, const float* correction, int32_t* idx, float* weight, int32_t tm,
+                                int32_t ntiles, int32_t* order, int32_t* tile_expert, void* stream) {
+    const char* bad = bad_router(shape);
+    SKYRL_REQUIRE(!bad, bad);
+    SKYRL_REQUIRE(shape->experts <= kWave, "moe_choose: at most 64 experts");
+    SKYRL_REQUIRE(n >= 0 && shares > 0 && row_stride >= shape->experts && share_stride >= 0, "moe_choose: bad sizes");
+    SKYRL_REQUIRE(!order == !tile_expert, "moe_choose: order and tile_expert go together");
+    if (n == 0) return SKYRL_OK;
+    SKYRL_REQUIRE(logits && correction && idx && weight, "moe_choose: null pointer");
+    const int64_t pairs = (int64_t)n * shape->top;
+    SKYRL_REQUIRE(!order || (pairs <= kChosen && tm > 0 && tm % 16 == 0 &&
+                             ntiles >= skyrl_moe_tiles(shape->experts, (int32_t)pairs, tm)),
+                  "moe_choose: more pairs than it sorts, or too few tiles");
+    const Router ro{shape->experts, shape->top, shape->groups, shape->keep};
+    hipStream_t s = as_stream(stream);
+    if (order)
+        hipLaunchKernelGGL((moe_choose_kernel<true>), dim3(1), dim3(1024), 0, s, ro, logits, shares, share_stride, row_stride, n,
+                           correction, idx, weight, tm, ntiles, order, tile_expert);
+    else
+        hipLaunchKernelGGL((moe_choose_kernel<false>), dim3((n + 3) / 4), dim3(kNT), 0, s, ro, logits, shares, share_stride,
+                           row_stride, n, correction, idx, weight, tm, ntiles, order, tile_expert);
+    return check_launch("moe_choose_kernel");
 }
 
 extern "C" int32_t skyrl_moe_tiles(int32_t experts, int32_t npairs, int32_t tm) {

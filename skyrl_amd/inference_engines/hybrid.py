@@ -390,7 +390,7 @@ class HybridDecoder:
                     y = y.index_select(1, want)
                 else:
                     y = y.view(-1, sub.rows_per_token, s.hidden_size)[want].view(-1, s.hidden_size)
-                h, gate, x = h[want], gate[want], None
+                h, gate, x = h[want], gate.index_select(-2, want), None
             x = lk.gate_norm_add(y, h, after, before[k + 1], gate=gate, out=x, **args)
             if trail is not None and k in ends and not last:
                 trail.append(h.clone())

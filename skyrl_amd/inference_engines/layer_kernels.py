@@ -173,7 +173,8 @@ def gate_norm_add(a: torch.Tensor, hidden: torch.Tensor, weight: torch.Tensor, n
                   out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """hidden (f32 [n, H], in place; fresh: from 0) += mult norm(y) weight, y the sum of `parts` consecutive rows of a,
     times sigmoid(gate + gate_bias) with a gate; returns norm(hidden) next_weight. A norm is an RMS norm in `groups`
-    equal parts of the row. `rows` int64 [n]: which rows of a (parts 1). a may be linear's f32 parts (`parts` 1)."""
+    equal parts of the row. `rows` int64 [n]: which rows of a (parts 1). a (`parts` 1) or the gate may be linear's f32
+    parts, of the gate's the first H columns."""
     dev = _require_gpu(a, hidden, weight, next_weight, gate, gate_bias, rows, out)
     n, H = hidden.shape
     _check(hidden, "hidden", torch.float32)
@@ -191,18 +192,24 @@ def gate_norm_add(a: torch.Tensor, hidden: torch.Tensor, weight: torch.Tensor, n
     _check(rows, "rows", torch.int64, (n,))
     if (gate is None) != (gate_bias is None):
         raise ValueError("gate and gate_bias go together")
+    gate_shares = gate.shape[0] if gate is not None and gate.dim() == 3 else 0
     if gate is not None:
-        _check_view(gate, "gate", weight.dtype, (n, H))
+        if gate_shares:
+            if shares or rows is not None or fresh or weight.dtype != torch.bfloat16 or gate.shape[2] < H:
+                raise ValueError("a gate's parts are of a model in bfloat16, beside rows that are added to the residual")
+            _check(gate, "gate", torch.float32, (gate_shares, n, gate.shape[2]))
+        else:
+            _check_view(gate, "gate", weight.dtype, (n, H))
         _check(gate_bias, "gate_bias", torch.float32, (H,))
     if out is None:
         out = torch.empty((n, H), dtype=weight.dtype, device=dev)
     _check(out, "out", weight.dtype, (n, H))
-    if shares:
-        _ffi.call("skyrl_gate_norm_add_parts", _ptr(a), shares, _ptr(gate), 0 if gate is None else max(gate.stride(0), H),
-                  _ptr(gate_bias), _ptr(weight), groups, float(eps), float(mult), _ptr(hidden), _ptr(next_weight), n, H,
-                  _ptr(out), _stream(dev))
+    gs = 0 if gate is None else gate.shape[2] if gate_shares else max(gate.stride(0), H)
+    if shares or gate_shares:
+        _ffi.call("skyrl_gate_norm_add_parts", _ptr(a), shares, parts, _ptr(gate), gate_shares, gs, _ptr(gate_bias), _ptr(weight),
+                  groups, float(eps), float(mult), _ptr(hidden), _ptr(next_weight), n, H, _ptr(out), _stream(dev))
         return out
-    _ffi.call("skyrl_gate_norm_add", _ptr(a), _ptr(rows), parts, _ptr(gate), 0 if gate is None else max(gate.stride(0), H),
+    _ffi.call("skyrl_gate_norm_add", _ptr(a), _ptr(rows), parts, _ptr(gate), gs,
               _ptr(gate_bias), _ptr(weight), groups, float(eps), float(mult), _ptr(hidden), int(fresh), _ptr(next_weight), n, H,
               _ptr(out), _code(weight), _stream(dev))
     return out
@@ -1006,6 +1013,33 @@ def moe_route(sh, x, router, correction):
     return idx, weight
 
 
+CHOOSE_EXPERTS, CHOOSE_SORTS = 64, 128  # experts that skyrl_moe_choose takes, pairs that it sorts too
+
+
+def moe_choose(sh, logits, column: int, correction, tm: int):
+    """moe_route and moe_sort from router logits that another product formed: columns [column, column + experts) of
+    linear's parts f32 [shares, n, N]. Returns (idx, weight, order, tile_expert)."""
+    dev = _require_gpu(logits, correction)
+    shares, n, N = logits.shape
+    _check(logits, "logits", torch.float32)
+    _check(correction, "correction", torch.float32, (sh.experts,))
+    if sh.experts > CHOOSE_EXPERTS or not 0 <= column <= N - sh.experts:
+        raise ValueError("moe_choose: at most 64 experts, within the product's columns")
+    idx = torch.empty((n, sh.top), dtype=torch.int32, device=dev)
+    weight = torch.empty((n, sh.top), dtype=torch.float32, device=dev)
+    order = tile_expert = None
+    pairs = n * sh.top
+    tiles = int(_ffi.query("skyrl_moe_tiles", sh.experts, pairs, tm))
+    if 0 < pairs <= CHOOSE_SORTS:
+        order = torch.empty((tiles, tm), dtype=torch.int32, device=dev)
+        tile_expert = torch.empty((tiles + 1,), dtype=torch.int32, device=dev)
+    _ffi.call("skyrl_moe_choose", ctypes.byref(sh), ctypes.c_void_p(logits.data_ptr() + 4 * column), shares, n * N, N, n,
+              _ptr(correction), _ptr(idx), _ptr(weight), tm, tiles, _ptr(order), _ptr(tile_expert), _stream(dev))
+    if order is None:
+        order, tile_expert = moe_sort(sh, idx, tm)
+    return idx, weight, order, tile_expert
+
+
 def moe_tile(sh, n: int) -> int:
     """Rows per tile of the experts' products for n tokens."""
     mean = n * sh.top / sh.experts
@@ -1027,9 +1061,9 @@ def moe_sort(sh, idx, tm: int):
     return order, tile_expert
 
 
-def moe_experts(sh, x, idx, weight, gate_up, down, tm: Optional[int] = None) -> torch.Tensor:
+def moe_experts(sh, x, idx, weight, gate_up, down, tm: Optional[int] = None, tiles_of=None) -> torch.Tensor:
     """Rows [n * top, width]: every pair's expert output times its weight. gate_up [experts, 2, ff, width], down
-    [experts, width, ff]."""
+    [experts, width, ff]. tiles_of: (order, tile_expert) of moe_sort for tiles of tm rows, formed here otherwise."""
     dev = _require_gpu(x, idx, weight, gate_up, down)
     n = x.shape[0]
     _check(x, "x", x.dtype, (n, sh.width))
@@ -1041,7 +1075,7 @@ def moe_experts(sh, x, idx, weight, gate_up, down, tm: Optional[int] = None) -> 
     out = torch.empty((n * sh.top, sh.width), dtype=x.dtype, device=dev)
     if n == 0:
         return out
-    order, tile_expert = moe_sort(sh, idx, tm)
+    order, tile_expert = moe_sort(sh, idx, tm) if tiles_of is None else tiles_of
     tiles = order.shape[0]
     act = torch.empty((tiles * tm, sh.ff), dtype=x.dtype, device=dev)
     ref, st = ctypes.byref(sh), _stream(dev)

@@ -270,10 +270,20 @@ class Gated:
             self.weight = self.sub.w_beside
         else:
             self.sub, self.weight = sub, w.matrix(width, width)
+            router = getattr(sub, "router", None)
+            self.joint = None
+            if router is not None:  # one product for the gate's logits and the router's
+                self.joint = torch.empty((width + router.shape[0], width), dtype=w.dtype, device=w.device)
+                self.joint[:width], self.joint[width:] = self.weight, router
+                self.weight, sub.router = self.joint[:width], self.joint[width:]
 
     def forward(self, x: torch.Tensor, inp, state, workspace):
         if isinstance(self.sub, Products):
             return self.sub.forward(x, inp, state, workspace, parts=True)
+        if self.joint is not None and self.sub.chooses(x):
+            logits = lk.linear(x, self.joint, parts=True)
+            if logits.dim() == 3:  # few rows
+                return self.sub.forward(x, inp, state, workspace, logits=(logits, self.weight.shape[0])), logits
         return self.sub.forward(x, inp, state, workspace), lk.linear(x, self.weight)
 
 
@@ -1050,7 +1060,16 @@ class RoutedExperts:
             yield from ((f"e{e}.gate", self.gate_up[e, 0]), (f"e{e}.up", self.gate_up[e, 1]), (f"e{e}.down", self.down[e]))
         yield from (("router", self.router), ("correction", self.correction))
 
-    def forward(self, x: torch.Tensor, inp, state, workspace) -> torch.Tensor:
+    def chooses(self, x: torch.Tensor) -> bool:
+        """Whether few rows may come with their router logits."""
+        return x.dtype == torch.bfloat16 and x.shape[0] <= lk.MAX_ROWS and self.experts <= lk.CHOOSE_EXPERTS
+
+    def forward(self, x: torch.Tensor, inp, state, workspace, logits=None) -> torch.Tensor:
+        """logits: (layer_kernels.linear's parts that hold the router's, their first column)."""
+        if logits is not None:
+            tm = lk.moe_tile(self.shape, x.shape[0])
+            idx, weight, *tiles = lk.moe_choose(self.shape, *logits, self.correction, tm)
+            return lk.moe_experts(self.shape, x, idx, weight, self.gate_up, self.down, tm, tiles)
         idx, weight = lk.moe_route(self.shape, x, self.router, self.correction)
         return lk.moe_experts(self.shape, x, idx, weight, self.gate_up, self.down)
 
