@@ -433,13 +433,23 @@ def layer_lib_of(name: str) -> str:
 
 def load_layers(lib: str = "layers") -> ctypes.CDLL:
     """One of LAYER_LIBS, likewise."""
-    out = _open(layer_lib_path(lib), {n: s for n, s in LAYERS_SIGNATURES.items() if layer_lib_of(n) == lib})
-    out.skyrl_last_error.restype = ctypes.c_char_p
-    return out
+    path = layer_lib_path(lib)
+    if path in _libs:
+        return _libs[path]
+    own = {n: s for n, s in LAYERS_SIGNATURES.items() if layer_lib_of(n) == lib}
+    return _open(path, dict(own, skyrl_last_error=(ctypes.c_char_p, [])))
+
+
+_LAYER_LIB_BY_NAME = {n: layer_lib_of(n) for n in LAYERS_SIGNATURES}
+_lib_by_name: dict = {}  # the opened library of every entry point that has been called
 
 
 def _lib_of(name: str) -> ctypes.CDLL:
-    return load_layers(layer_lib_of(name)) if name in LAYERS_SIGNATURES else load()
+    lib = _lib_by_name.get(name)
+    if lib is None:
+        word = _LAYER_LIB_BY_NAME.get(name)
+        lib = _lib_by_name[name] = load() if word is None else load_layers(word)
+    return lib
 
 
 def call(name: str, *args) -> int:

@@ -22,31 +22,32 @@ LOSS_REDUCTIONS = {"token_mean": 0, "sequence_mean": 1, "seq_mean_token_sum_norm
 
 
 # ---------------------------------------------------------------------------- plumbing
-def _ptr(t: Optional[torch.Tensor]):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
+    return None if t is None else t.data_ptr()
 
 
-def _stream(device: torch.device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+def _stream(device: torch.device) -> int:
+    """The device's current stream, without a torch.cuda.Stream object for every launch."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)
 
 
 def _require_gpu(*tensors: Optional[torch.Tensor]) -> torch.device:
-    dev = None
+    first = None
     for t in tensors:
         if t is None:
             continue
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise RuntimeError(
                 "skyrl_amd HIP path requires device tensors (got a tensor on "
                 f"{t.device}); there is no CPU fallback"
             )
-        if dev is None:
-            dev = t.device
-        elif t.device != dev:
-            raise RuntimeError(f"tensors on different devices: {dev} vs {t.device}")
-    if dev is None:
+        if first is None:
+            first, index = t, t.get_device()
+        elif t.get_device() != index:
+            raise RuntimeError(f"tensors on different devices: {first.device} vs {t.device}")
+    if first is None:
         raise RuntimeError("no device tensor given")
-    return dev
+    return first.device
 
 
 def _f32c(t: Optional[torch.Tensor], name: str) -> Optional[torch.Tensor]:
@@ -68,7 +69,7 @@ class _Workspaces:
         self._bufs: Dict[Tuple, torch.Tensor] = {}
 
     def get(self, device: torch.device, kind: str, nbytes: int) -> torch.Tensor:
-        stream = torch.cuda.current_stream(device).cuda_stream
+        stream = _stream(device)
         key = (device.index, stream, kind)
         buf = self._bufs.get(key)
         if buf is None or buf.numel() < nbytes:
