@@ -17,6 +17,8 @@
 //   U = U0 - W S,   O = diag(e^G) Q S + P U,   S <- e^{G_n} S + K^T diag(e^{G_n - G}) U.
 // Everything is f32, the products on the f32 matrix instructions (v_mfma_f32_16x16x4_f32): a lane's
 // four consecutive k values of a 16-step feed four instructions, the same permutation of k on both sides.
+#include <type_traits>
+
 #include "conv.h"
 
 namespace skyrl {
@@ -206,23 +208,34 @@ struct SeqRef {
     const int64_t* positions;
 };
 
+// Operand order: a 16 x 16 tile of a matrix that is read as an operand of the matrix instructions is 256 consecutive numbers,
+// lane (c, g)'s four first: row c, columns 4 g .. 4 g + 3. A wave's load is then 1 KB in a piece (64 bytes a cycle); the
+// same tile in rows cost four times as long, a cache line per lane. Tokens past a chunk's end are zero.
+//   q, k   qk [chunk][key head][q | k][token tile][dim tile]      k transposed   kt [chunk][key head][dim tile][token tile]
+//   v transposed  vt [chunk][head][vdim tile][token tile]         W  [chunk][head][token tile][dim tile]
+//   P      [chunk][head][token tile][token tile]                  U  as its product leaves it: row 4 g + i, column c, tiles as vt
+constexpr int kTile = 256;
+
 // Convolution, silu, unit norms and gates. grid (nchunks, K + ceil(H V / 256)): the first K groups are the
-// key heads (q and k), the others 256 value channels each; gates with group 0.
-template <typename T>
+// key heads (q and k), the others 256 value channels each; gates with group 0. A channel's 64 inputs and the TAPS - 1 before
+// are all in flight at once (TAPS 0: any number of taps, loaded where they are used). Bound: 470 MB for 8192 tokens of 8192
+// channels (100 us at a large copy's rate).
+template <typename T, int TAPS>
 __global__ __launch_bounds__(kNT) void delta_conv_kernel(Dims d, SeqRef sq, const T* __restrict__ proj, int64_t stride,
                                                          const T* __restrict__ conv_w, const float* __restrict__ a_log,
                                                          const float* __restrict__ dt_bias,
                                                          const T* __restrict__ conv_state, float* __restrict__ qk,
-                                                         float* __restrict__ kt, float* __restrict__ vout, float* __restrict__ lg,
+                                                         float* __restrict__ kt, float* __restrict__ vt, float* __restrict__ lg,
                                                          float* __restrict__ beta) {
-    extern __shared__ float smem[];  // [16][2 D] of the key heads
+    extern __shared__ __attribute__((aligned(16))) float smem[];  // [16][2 D + 4] of the key heads
+    __shared__ float s_r[32];                                     // their scales
     const int32_t* ck = sq.chunk + 4 * blockIdx.x;
     const int t0 = ck[0], n = ck[1], seq = ck[2];
     const int sfirst = sq.cu[seq];
     const int pos0 = (int)sq.positions[sfirst] + (t0 - sfirst);
-    const int ch_all = d.channels(), D = d.D, D16 = d.d16();
+    const int ch_all = d.channels(), D = d.D, V = d.V, nd = d.d16() / 16, nv = d.v16() / 16, LK = 2 * D + 4;
     const T* ring = conv_state + (int64_t)sq.rows[seq] * d.taps * ch_all;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x;
     const bool keys = (int)blockIdx.y < d.K;
     const int kh = blockIdx.y;
     if (blockIdx.y == 0) {
@@ -239,78 +252,80 @@ __global__ __launch_bounds__(kNT) void delta_conv_kernel(Dims d, SeqRef sq, cons
         if (t0 + i >= sfirst) return ld(proj + (int64_t)(t0 + i) * stride + ch);
         return ld(ring + (int64_t)((pos0 + i) % d.taps) * ch_all + ch);
     };
-    const int nch = keys ? 2 * D : min(kNT, d.H * d.V - ((int)blockIdx.y - d.K) * kNT);
-    const bool held = d.taps <= kConvWindow, carry = nch <= kNT;  // carry: one channel per thread, inputs stay in registers
-    constexpr int kSub = 16, kBack = kConvWindow - 1;
-    float x[kBack + kSub];
-    for (int i0 = 0; i0 < n; i0 += kSub) {
-        const int m = min(kSub, n - i0);
+    const int nch = keys ? 2 * D : min(kNT, d.H * V - ((int)blockIdx.y - d.K) * kNT);
+    constexpr int kSub = 16, kBack = TAPS > 0 ? TAPS - 1 : 0;
+    const bool once = nch <= kNT;  // one channel per thread: its inputs stay in registers
+    float x[kBack + kC], w[TAPS > 0 ? TAPS : 1];
+    auto channel = [&](int e) {
+        return !keys ? 2 * d.K * D + ((int)blockIdx.y - d.K) * kNT + e : e < D ? kh * D + e : (d.K + kh) * D + (e - D);
+    };
+    auto fetch = [&](int ch) {
+#pragma unroll
+        for (int j = 0; j < TAPS; ++j)
+            w[j] = j >= TAPS - d.taps ? ld(conv_w + (int64_t)ch * d.taps + j - (TAPS - d.taps)) : 0.f;
+#pragma unroll
+        for (int i = 0; i < kC; ++i) x[kBack + i] = ld(proj + (int64_t)(t0 + min(i, n - 1)) * stride + ch);
+#pragma unroll
+        for (int j = 0; j < kBack; ++j) x[j] = j > kBack - d.taps ? input(ch, j - kBack) : 0.f;
+    };
+    if constexpr (TAPS > 0)
+        if (once && tid < nch) fetch(channel(tid));
+#pragma unroll
+    for (int sub = 0; sub < kC / kSub; ++sub) {
+        const int i0 = sub * kSub;
         for (int e = tid; e < nch; e += kNT) {
-            const int ch = !keys ? 2 * d.K * D + ((int)blockIdx.y - d.K) * kNT + e
-                                 : e < D ? kh * D + e : (d.K + kh) * D + (e - D);
-            float w[kConvWindow];
-            if (held) {
-                if (carry && i0 > 0) {
-#pragma unroll
-                    for (int j = 0; j < kBack; ++j) x[j] = x[j + kSub];
-                } else {
-#pragma unroll
-                    for (int j = 0; j < kBack; ++j) x[j] = j >= kConvWindow - d.taps ? input(ch, i0 - kBack + j) : 0.f;
-                }
-#pragma unroll
-                for (int j = 0; j < kSub; ++j)
-                    x[kBack + j] = ld(proj + (int64_t)(t0 + min(i0 + j, n - 1)) * stride + ch);
-#pragma unroll
-                for (int j = 0; j < kConvWindow; ++j)
-                    w[j] = j >= kConvWindow - d.taps ? ld(conv_w + (int64_t)ch * d.taps + j - (kConvWindow - d.taps)) : 0.f;
-            }
+            const int ch = channel(e);
+            if constexpr (TAPS > 0)
+                if (!once) fetch(ch);
+            float y[kSub];
 #pragma unroll
             for (int i = 0; i < kSub; ++i) {
-                float y = 0.f;
-                if (held) {
+                y[i] = 0.f;
+                if constexpr (TAPS > 0) {
 #pragma unroll
-                    for (int j = 0; j < kConvWindow; ++j) y += x[i + j] * w[j];
-                } else if (i < m) {
+                    for (int j = 0; j < TAPS; ++j) y[i] += x[i0 + i + j] * w[j];
+                } else if (i0 + i < n) {
                     for (int j = 0; j < d.taps; ++j)
-                        y += input(ch, i0 + i - (d.taps - 1) + j) * ld(conv_w + (int64_t)ch * d.taps + j);
+                        y[i] += input(ch, i0 + i - (d.taps - 1) + j) * ld(conv_w + (int64_t)ch * d.taps + j);
                 }
-                y = siluf_(y);
-                if (keys) smem[i * 2 * D + e] = y;
-                else if (i < m) vout[(int64_t)(t0 + i0 + i) * d.H * d.V + ((int)blockIdx.y - d.K) * kNT + e] = y;
+                y[i] = i0 + i < n ? y[i] * sigmoid_<T>(y[i]) : 0.f;
+                if (keys) smem[i * LK + e] = y[i];
             }
+            if (keys) continue;
+            const int col = ((int)blockIdx.y - d.K) * kNT + e, h = col / V, c = col - h * V;
+            float* dst = vt + ((((int64_t)blockIdx.x * d.H + h) * nv + c / 16) * 4 + sub) * kTile + c % 16 * 4;
+#pragma unroll
+            for (int g = 0; g < 4; ++g) st4(dst + g * 64, make_float4(y[4 * g], y[4 * g + 1], y[4 * g + 2], y[4 * g + 3]));
         }
         if (!keys) continue;
         __syncthreads();
-        for (int e = wave; e < 2 * m; e += kNT / kWave) {
-            const int i = e >> 1, which = e & 1;
-            float* src = smem + i * 2 * D + which * D;
+        {  // eight threads per (token, q or k)
+            const int i = tid >> 4, which = (tid >> 3) & 1, part = tid & 7;
+            const float* src = smem + i * LK + which * D;
             float ss = 0.f;
-            for (int k = lane; k < D; k += kWave) ss += src[k] * src[k];
-            float r = 1.f / sqrtf(wave_sum(ss) + 1e-6f);
+            for (int k = part; k < D; k += 8) ss += src[k] * src[k];
+#pragma unroll
+            for (int o = 1; o < 8; o <<= 1) ss += __shfl_xor(ss, o, kWave);
+            float r = 1.f / sqrtf(ss + 1e-6f);
             if (which == 0) r *= 1.f / sqrtf((float)D);
-            float* dst = qk + (((int64_t)(t0 + i0 + i) * 2 + which) * d.K + kh) * D16;
-            for (int k = lane; k < D16; k += kWave) {
-                const float y = k < D ? src[k] * r : 0.f;
-                dst[k] = y;
-                if (which && k < D) src[k] = y;
-            }
+            if (part == 0) s_r[2 * i + which] = r;
         }
         __syncthreads();
-        float* tr = kt + (((int64_t)blockIdx.x * d.K + kh) * D16) * kC + i0;  // K^T, zero past the chunk's end
-        for (int e = tid; e < D16 * 4; e += kNT) {
-            const int k = e >> 2, i = (e & 3) * 4;
+        const int64_t head = (int64_t)blockIdx.x * d.K + kh;
+        for (int e = tid; e < nd * 3 * kWave; e += kNT) {
+            const int l = e & 63, tile = (e >> 6) % nd, form = (e >> 6) / nd, c = l & 15, g = l >> 4;
             float y[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) y[j] = (k < D && i + j < m) ? smem[(i + j) * 2 * D + D + k] : 0.f;
-            st4(tr + (int64_t)k * kC + i, make_float4(y[0], y[1], y[2], y[3]));
+            for (int j = 0; j < 4; ++j) {
+                const int i = form < 2 ? c : 4 * g + j, k = 16 * tile + (form < 2 ? 4 * g + j : c);
+                y[j] = k < D ? smem[i * LK + (form > 0 ? D : 0) + k] * s_r[2 * i + (form > 0)] : 0.f;
+            }
+            float* dst = form < 2 ? qk + (((head * 2 + form) * 4 + sub) * nd + tile) * kTile
+                                  : kt + ((head * nd + tile) * 4 + sub) * kTile;
+            st4(dst + l * 4, make_float4(y[0], y[1], y[2], y[3]));
         }
         __syncthreads();
     }
-    if (keys)
-        for (int i0 = (n + kSub - 1) / kSub * kSub; i0 < kC; i0 += kSub)
-            for (int e = tid; e < D16 * 4; e += kNT)
-                st4(kt + (((int64_t)blockIdx.x * d.K + kh) * D16 + (e >> 2)) * kC + i0 + (e & 3) * 4,
-                    make_float4(0.f, 0.f, 0.f, 0.f));
 }
 
 __device__ __forceinline__ f32x4 mma4(const float4& a, const float4& b, f32x4 acc) {
@@ -324,10 +339,10 @@ __device__ __forceinline__ float4 as_float4(const f32x4& v) { return make_float4
 // One workgroup per (chunk, head). The 64 x 64 system is solved in 16 x 16 blocks: each wave inverts one
 // diagonal block by substitution, the blocks below follow diagonal by diagonal from
 // T_rb = -T_rr sum_k A_rk T_kb, and T then multiplies both right-hand sides. A 16 x 16 result's registers
-// (rows 4 g + i, column c) are the next product's right operand as they are.
+// (rows 4 g + i, column c) are the next product's right operand as they are, and a transposed product's are its operand order.
 __global__ __launch_bounds__(kNT) void delta_chunk_kernel(Dims d, const int32_t* __restrict__ chunk,
-                                                          const float* __restrict__ qk, const float* __restrict__ v,
-                                                          const float* __restrict__ lg, const float* __restrict__ beta,
+                                                          const float* __restrict__ qk, const float* __restrict__ kt,
+                                                          const float* __restrict__ vt, const float* __restrict__ lg, const float* __restrict__ beta,
                                                           float* __restrict__ W, float* __restrict__ U,
                                                           float* __restrict__ P, float* __restrict__ G) {
     constexpr int LD = kC + 4;
@@ -352,7 +367,9 @@ __global__ __launch_bounds__(kNT) void delta_chunk_kernel(Dims d, const int32_t*
         s_g[lane] = x;
         s_b[lane] = be;
         s_w[lane] = be * expf(x);
-        G[ch * kC + lane] = x;
+        const float last = __shfl(x, kWave - 1, kWave);
+        G[ch * 2 * kC + lane] = expf(x);
+        G[ch * 2 * kC + kC + lane] = expf(last - x);
     }
     // K K^T and Q K^T on the ten blocks at and below the diagonal: 20 block products, five per wave
     f32x4 acc[5];
@@ -364,23 +381,26 @@ __global__ __launch_bounds__(kNT) void delta_chunk_kernel(Dims d, const int32_t*
         br[k] = item >= 6 ? 3 : item >= 3 ? 2 : item >= 1 ? 1 : 0;
         bc[k] = item - br[k] * (br[k] + 1) / 2;
     }
-    for (int d0 = 0; d0 < D16; d0 += kC) {
-        const int w4 = min(kC, D16 - d0) / 4;
+    const int nd = D16 / 16;
+    const float* qp = qk + ((int64_t)ci * d.K + kh) * 2 * 4 * nd * kTile;
+    for (int d0 = 0; d0 < nd; d0 += 4) {
+        const int w = min(4, nd - d0);
         __syncthreads();
-        for (int e = tid; e < kC * w4; e += kNT) {
-            const int i = e / w4, x = (e - i * w4) * 4;
-            const float* src = qk + ((int64_t)(t0 + min(i, n - 1)) * 2 * d.K + kh) * D16 + d0 + x;
-            float4 qv = ld4(src), kv = ld4(src + (int64_t)d.K * D16);
-            st4(&s_k[i * LD + x], kv);
-            st4(&s_q[i * LD + x], qv);
+        for (int e = tid; e < 4 * 4 * kWave; e += kNT) {  // four dim tiles of every token tile
+            const int i = e >> 8, x = e & 255;
+            if (x >> 6 >= w) continue;
+            const float* src = qp + (i * nd + d0) * kTile + x * 4;
+            st4(&s_q[e * 4], ld4(src));
+            st4(&s_k[e * 4], ld4(src + 4 * nd * kTile));
         }
         __syncthreads();
-        for (int s = 0; s < w4 / 4; ++s) {
+        for (int s = 0; s < w; ++s) {
 #pragma unroll
             for (int k = 0; k < 5; ++k) {
-                const float* left = wave + 4 * k < 10 ? s_k : s_q;
-                acc[k] = mma4(ld4(&left[(16 * br[k] + c) * LD + 16 * s + 4 * g]),
-                              ld4(&s_k[(16 * bc[k] + c) * LD + 16 * s + 4 * g]), acc[k]);
+                const bool own = wave + 4 * k < 10;  // K K^T; otherwise (Q K^T)^T
+                const float* right = own ? s_k : s_q;
+                acc[k] = mma4(ld4(&s_k[((own ? br[k] : bc[k]) * 4 + s) * kTile + lane * 4]),
+                              ld4(&right[((own ? bc[k] : br[k]) * 4 + s) * kTile + lane * 4]), acc[k]);
             }
         }
     }
@@ -388,12 +408,21 @@ __global__ __launch_bounds__(kNT) void delta_chunk_kernel(Dims d, const int32_t*
     float *s_a = s_k, *s_t = s_q;
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
+        if (wave + 4 * k < 10) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int r = 16 * br[k] + 4 * g + i, cc = 16 * bc[k] + c;
-            const float dec = cc <= r ? expf(s_g[r] - s_g[cc]) : 0.f;
-            if (wave + 4 * k < 10) s_a[r * LD + cc] = cc < r ? s_b[r] * dec * acc[k][i] : 0.f;
-            else P[(ch * kC + r) * kC + cc] = dec * acc[k][i];
+            for (int i = 0; i < 4; ++i) {
+                const int r = 16 * br[k] + 4 * g + i, cc = 16 * bc[k] + c;
+                s_a[r * LD + cc] = cc < r ? s_b[r] * expf(s_g[r] - s_g[cc]) * acc[k][i] : 0.f;
+            }
+        } else {
+            const int r = 16 * br[k] + c;
+            float y[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int cc = 16 * bc[k] + 4 * g + i;
+                y[i] = cc <= r ? expf(s_g[r] - s_g[cc]) * acc[k][i] : 0.f;
+            }
+            st4(P + ((ch * 4 + br[k]) * 4 + bc[k]) * kTile + lane * 4, make_float4(y[0], y[1], y[2], y[3]));
         }
     }
     __syncthreads();
@@ -434,52 +463,49 @@ __global__ __launch_bounds__(kNT) void delta_chunk_kernel(Dims d, const int32_t*
         }
     }
     __syncthreads();
-    // T times [diag(beta e^G) K | diag(beta) V], 16 columns at a time
-    const int nw = D16 / 16, ntile = nw + V16 / 16;
-    for (int tile = wave; tile < ntile; tile += 4) {
-        const bool isw = tile < nw;
-        const int cc = 16 * (isw ? tile : tile - nw) + c;
-        const float* src = isw ? qk + ((int64_t)t0 * 2 + 1) * d.K * D16 + (int64_t)kh * D16 + cc
-                               : v + ((int64_t)t0 * d.H + h) * d.V + min(cc, d.V - 1);
-        const int64_t step = isw ? (int64_t)2 * d.K * D16 : (int64_t)d.H * d.V;
-        float x[16];
+    // T times [diag(beta e^G) K | diag(beta) V], 16 columns at a time; the first transposed
+    const int nv = V16 / 16;
+    for (int tile = wave; tile < nd + nv; tile += 4) {
+        const bool isw = tile < nd;
+        const int vtile = tile - nd;
+        const float* src = (isw ? kt + (((int64_t)ci * d.K + kh) * nd + tile) * 4 * kTile : vt + (ch * nv + vtile) * 4 * kTile) + lane * 4;
+        const bool on = isw || 16 * vtile + c < d.V;  // columns past vdim hold nothing
+        float4 x[4];
 #pragma unroll
-        for (int j = 0; j < 16; ++j) x[j] = src[min(16 * (j >> 2) + 4 * g + (j & 3), n - 1) * step];
+        for (int s = 0; s < 4; ++s) x[s] = on ? ld4(src + s * kTile) : make_float4(0.f, 0.f, 0.f, 0.f);
         f32x4 o[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) o[r] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
             const float4 sc = ld4((isw ? s_w : s_b) + 16 * s + 4 * g);
-            const float4 bv = make_float4(x[4 * s] * sc.x, x[4 * s + 1] * sc.y, x[4 * s + 2] * sc.z, x[4 * s + 3] * sc.w);
+            const float4 bv = make_float4(x[s].x * sc.x, x[s].y * sc.y, x[s].z * sc.z, x[s].w * sc.w);
 #pragma unroll
-            for (int r = s; r < 4; ++r) o[r] = mma4(ld4(&s_t[(16 * r + c) * LD + 16 * s + 4 * g]), bv, o[r]);
+            for (int r = s; r < 4; ++r) {
+                const float4 t = ld4(&s_t[(16 * r + c) * LD + 16 * s + 4 * g]);
+                o[r] = isw ? mma4(bv, t, o[r]) : mma4(t, bv, o[r]);
+            }
         }
-        if (isw) {
-            float* dst = W + ch * kC * D16 + cc;
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) dst[(16 * r + 4 * g + i) * D16] = o[r][i];
-        } else {  // U^T
-            float* dst = U + (ch * V16 + cc) * kC + 4 * g;
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                st4(dst + 16 * r, cc < d.V ? as_float4(o[r]) : make_float4(0.f, 0.f, 0.f, 0.f));
-        }
+        for (int r = 0; r < 4; ++r)
+            st4((isw ? W + ((ch * 4 + r) * nd + tile) * kTile : U + ((ch * nv + vtile) * 4 + r) * kTile) + lane * 4, as_float4(o[r]));
     }
 }
 
 // One workgroup per (sequence, head, 16 columns of S). NS: 16-wide steps of dim (EXACT: dim = 16 NS); DT
-// 16-row tiles of S per wave. What a phase has consumed is loaded for the next chunk at once, into the
-// same registers: W and Q during the second phase, K^T and P during the next chunk's first.
-template <int NS, bool EXACT>
-__global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(NS <= 8 ? 2 : 1))) void delta_chain_kernel(
+// 16-row tiles of S per wave; SETS: register sets of operands. With two (dim up to 128) a chunk's operands are under way for
+// the whole chunk before: they come from HBM, and a chunk's f32 products take 1.7 us. Only U = U0 - W S and the update of S
+// are a chain; the products that end in the output stand where the others' results go through LDS. Bound: the f32 matrix
+// rate (178 us for 8192 tokens of 32 heads of 128 x 128). Measured there: 712 us with operands in rows, loaded half a chunk
+// ahead, and products in the order of the equations; 412 us this way, of which 300 with operands that are in L2 (three
+// sets spill, and a touch of the lines two chunks ahead is waited for itself: loads return in order).
+template <int NS, bool EXACT, int SETS>
+__global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(1))) void delta_chain_kernel(
     Dims d, SeqRef sq, const int32_t* __restrict__ seq_chunks, int seq0, int nseq, const float* __restrict__ qk,
     const float* __restrict__ kt, const float* __restrict__ W, const float* __restrict__ U, const float* __restrict__ P,
     const float* __restrict__ G, float* __restrict__ state, float* __restrict__ o) {
     constexpr int LS = NS * 16 + 4, LU = kC + 4, DT = (NS + 3) / 4;
-    __shared__ __attribute__((aligned(16))) float s_s[16 * LS];      // S^T slice
+    __shared__ __attribute__((aligned(16))) float s_s[2][16 * LS];   // S^T slice, by turns
     __shared__ __attribute__((aligned(16))) float s_u[2][16 * LU];   // U^T and its decayed copy
     const int V16 = d.v16(), D16 = EXACT ? NS * 16 : d.d16(), VP = d.vpad(), nt = V16 / 16;
     // the slices of one (sequence, head) read the same W, Q, K and P: consecutive on one XCD
@@ -506,95 +532,117 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(NS <= 8 ? 2
             const int dd = 16 * tile + 4 * g + i;
             S[k][i] = (pos0 > 0 && dd < d.D && vcol < VP) ? st_[(int64_t)dd * VP + vcol] : 0.f;
         }
-        if (EXACT || tile < ns) *reinterpret_cast<f32x4*>(&s_s[c * LS + 16 * tile + 4 * g]) = S[k];
+        if (EXACT || tile < ns) *reinterpret_cast<f32x4*>(&s_s[0][c * LS + 16 * tile + 4 * g]) = S[k];
     }
     const int c0 = seq_chunks[si], c1 = seq_chunks[si + 1];
-    const int woff = (16 * wave + c) * D16 + 4 * g, poff = (16 * wave + c) * kC + 4 * g;
-    const int koff = (16 * wave + c) * kC + 4 * g, goff = 16 * wave + 4 * g, uoff = vcol * kC + goff;
-    const int qstep = 2 * d.K * D16, ostep = d.H * d.V;
-    float4 w[NS], q[NS], p[4], kk[DT][4], u0, gr;
-    float gl;
-    auto load_first = [&](int ci, int t0, int n) {
-        const float* wp = W + ((int64_t)ci * d.H + h) * kC * D16;
-        const float* qp = qk + ((int64_t)t0 * 2 * d.K + kh) * D16;
-        const int qoff = min(16 * wave + c, n - 1) * qstep + 4 * g;
-#pragma unroll
-        for (int s = 0; s < NS; ++s) {
-            if (EXACT || s < ns) {
-                w[s] = ld4(wp + woff + 16 * s);
-                q[s] = ld4(qp + qoff + 16 * s);
-            }
-        }
-        const float* gp = G + ((int64_t)ci * d.H + h) * kC;
-        u0 = ld4(U + ((int64_t)ci * d.H + h) * V16 * kC + uoff);
-        gr = ld4(gp + goff);
-        gl = gp[kC - 1];
+    if (c0 >= c1) return;
+    const int first = sq.chunk[4 * c0], last = sq.chunk[4 * c1 - 3];  // first token, tokens of the last chunk
+    const int goff = 16 * wave + 4 * g, ostep = d.H * d.V, woff = wave * ns * kTile + 4 * lane;
+    struct Operands {
+        float4 w[NS], q[NS], p[4], kk[DT][4], u0, eg, er;
+        float decay;
+    } in[SETS];
+    // the parts of a chunk's operands that a step of 16 dims, or of 16 tokens, needs
+    auto load_ends = [&](Operands& x, int ci) {
+        const int64_t ch = (int64_t)ci * d.H + h;
+        x.u0 = ld4(U + ((ch * nt + vt) * 4 + wave) * kTile + 4 * lane);
+        x.eg = ld4(G + ch * 2 * kC + goff);
+        x.er = ld4(G + ch * 2 * kC + kC + goff);
+        x.decay = G[ch * 2 * kC + kC - 1];
     };
-    auto load_second = [&](int ci) {
-        const float* pp = P + ((int64_t)ci * d.H + h) * kC * kC;
-        const float* kp = kt + ((int64_t)ci * d.K + kh) * D16 * kC;
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            if (s <= wave) p[s] = ld4(pp + poff + 16 * s);  // P is lower triangular
-#pragma unroll
-            for (int k = 0; k < DT; ++k)
-                if (EXACT || wave + 4 * k < ns) kk[k][s] = ld4(kp + koff + 64 * k * kC + 16 * s);
-        }
+    auto load_dims = [&](Operands& x, int ci, int s) {
+        if (!EXACT && s >= ns) return;
+        x.w[s] = ld4(W + ((int64_t)ci * d.H + h) * 4 * ns * kTile + woff + s * kTile);
+        x.q[s] = ld4(qk + ((int64_t)ci * d.K + kh) * 8 * ns * kTile + woff + s * kTile);
     };
-    int t0 = 0, n = 0;
-    if (c0 < c1) {
-        t0 = sq.chunk[4 * c0];
-        n = sq.chunk[4 * c0 + 1];
-        load_first(c0, t0, n);
-    }
-    for (int ci = c0; ci < c1; ++ci) {
-        load_second(ci);
+    auto load_tokens = [&](Operands& x, int ci, int s) {
+#pragma unroll
+        for (int k = 0; k < DT; ++k)
+            if (EXACT || wave + 4 * k < ns)
+                x.kk[k][s] = ld4(kt + (((int64_t)ci * d.K + kh) * ns + wave + 4 * k) * 4 * kTile + s * kTile + 4 * lane);
+        if (SETS > 1 || s <= wave)  // P is lower triangular: the blocks above are loaded, not used
+            x.p[s] = ld4(P + ((((int64_t)ci * d.H + h) * 4 + wave) * 4 + s) * kTile + 4 * lane);
+    };
+    auto step = [&](auto turn, int ci) {
+        constexpr int B = decltype(turn)::value;
+        Operands &x = in[B % SETS], &next = in[(B + 1) % SETS];
+        const int cn = min(ci + 1, c1 - 1);  // the last chunk's again: loads without a branch are waited for one by one
+        if constexpr (SETS == 1) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) load_tokens(x, ci, s);
+        }
         __syncthreads();  // S^T of the previous chunk is in LDS
+        float4 b[NS];
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+            if (EXACT || s < ns) b[s] = ld4(&s_s[B][c * LS + 16 * s + 4 * g]);
+        const float4 eg = x.eg;  // with one set the next chunk's take their place
+        const float decay = x.decay;
         f32x4 aw = {0.f, 0.f, 0.f, 0.f}, ao = aw;
+        // A load a product or two: a burst of them would hold the products up.
+        if constexpr (SETS > 1) load_ends(next, cn);
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
-            if (EXACT || s < ns) {
-                const float4 b = ld4(&s_s[c * LS + 16 * s + 4 * g]);
-                aw = mma4(w[s], b, aw);
-                ao = mma4(q[s], b, ao);
-            }
+            if (EXACT || s < ns) aw = mma4(x.w[s], b[s], aw);
+            if (SETS > 1) load_dims(next, cn, s);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        const float4 u = make_float4(u0.x - aw[0], u0.y - aw[1], u0.z - aw[2], u0.w - aw[3]);
-        const float4 ud = make_float4(u.x * expf(gl - gr.x), u.y * expf(gl - gr.y), u.z * expf(gl - gr.z),
-                                      u.w * expf(gl - gr.w));
-        ao[0] *= expf(gr.x);
-        ao[1] *= expf(gr.y);
-        ao[2] *= expf(gr.z);
-        ao[3] *= expf(gr.w);
-        const float decay = expf(gl);
+        const float4 u = make_float4(x.u0.x - aw[0], x.u0.y - aw[1], x.u0.z - aw[2], x.u0.w - aw[3]);
         st4(&s_u[0][c * LU + goff], u);
-        st4(&s_u[1][c * LU + goff], ud);
-        __syncthreads();
-        const int tc = t0, nc = n;
-        if (ci + 1 < c1) {
-            t0 = sq.chunk[4 * ci + 4];
-            n = sq.chunk[4 * ci + 5];
-            load_first(ci + 1, t0, n);
+        st4(&s_u[1][c * LU + goff], make_float4(u.x * x.er.x, u.y * x.er.y, u.z * x.er.z, u.w * x.er.w));
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            if (EXACT || s < ns) ao = mma4(x.q[s], b[s], ao);
+            if (SETS > 1 && s < 4) load_tokens(next, cn, s);
+            __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
         for (int k = 0; k < DT; ++k) S[k] = S[k] * decay;
+        __syncthreads();
+        float4 ud[4], ul[4];
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const float4 b = ld4(&s_u[1][c * LU + 16 * s + 4 * g]);
-            if (s <= wave) ao = mma4(p[s], ld4(&s_u[0][c * LU + 16 * s + 4 * g]), ao);
+        for (int s = 0; s < 4; ++s) ud[s] = ld4(&s_u[1][c * LU + 16 * s + 4 * g]);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) ul[s] = ld4(&s_u[0][c * LU + 16 * s + 4 * g]);
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
 #pragma unroll
             for (int k = 0; k < DT; ++k)
-                if (EXACT || wave + 4 * k < ns) S[k] = mma4(kk[k][s], b, S[k]);
+                if (EXACT || wave + 4 * k < ns) S[k] = mma4(x.kk[k][s], ud[s], S[k]);
+        if constexpr (SETS == 1) {
+            load_ends(next, cn);
+#pragma unroll
+            for (int s = 0; s < NS; ++s) load_dims(next, cn, s);
         }
 #pragma unroll
         for (int k = 0; k < DT; ++k)
-            if (EXACT || wave + 4 * k < ns) *reinterpret_cast<f32x4*>(&s_s[c * LS + 16 * (wave + 4 * k) + 4 * g]) = S[k];
-        float* op = o + ((int64_t)tc * d.H + h) * d.V;
+            if (EXACT || wave + 4 * k < ns)
+                *reinterpret_cast<f32x4*>(&s_s[1 - B][c * LS + 16 * (wave + 4 * k) + 4 * g]) = S[k];
+        ao[0] *= eg.x;
+        ao[1] *= eg.y;
+        ao[2] *= eg.z;
+        ao[3] *= eg.w;
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+            if (s <= wave) ao = mma4(x.p[s], ul[s], ao);
+        float* op = o + ((int64_t)(first + (ci - c0) * kC) * d.H + h) * d.V;
+        const int n = ci + 1 < c1 ? kC : last;
         if (vcol < d.V) {
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                if (goff + i < nc) op[(goff + i) * ostep + vcol] = ao[i];
+                if (goff + i < n) op[(goff + i) * ostep + vcol] = ao[i];
         }
+    };
+    load_ends(in[0], c0);
+#pragma unroll
+    for (int s = 0; s < NS; ++s) load_dims(in[0], c0, s);
+    if constexpr (SETS > 1) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) load_tokens(in[0], c0, s);
+    }
+    for (int ci = c0; ci < c1; ci += 2) {
+        step(std::integral_constant<int, 0>{}, ci);
+        if (ci + 1 < c1) step(std::integral_constant<int, 1>{}, ci + 1);
     }
 #pragma unroll
     for (int k = 0; k < DT; ++k)
@@ -716,7 +764,7 @@ extern "C" int skyrl_delta_scan(const skyrl_delta_shape* shape, const void* proj
 extern "C" int skyrl_delta_conv(const skyrl_delta_shape* shape, const void* proj, int64_t proj_stride,
                                 const void* conv_w, const float* a_log, const float* dt_bias, const int32_t* chunk,
                                 int32_t nchunks, const int32_t* cu, const int32_t* rows, const int64_t* positions,
-                                const void* conv_state, float* qk, float* kt, float* v, float* lg, float* beta,
+                                const void* conv_state, float* qk, float* kt, float* vt, float* lg, float* beta,
                                 int32_t dtype, void* stream) {
     SKYRL_REQUIRE_T(dtype, "delta_conv");
     const char* bad = bad_shape(shape);
@@ -724,34 +772,38 @@ extern "C" int skyrl_delta_conv(const skyrl_delta_shape* shape, const void* proj
     const Dims d = dims_of(shape);
     SKYRL_REQUIRE(nchunks >= 0 && proj_stride >= proj_width(d), "delta_conv: bad sizes");
     if (nchunks == 0) return SKYRL_OK;
-    SKYRL_REQUIRE(proj && conv_w && a_log && dt_bias && chunk && cu && rows && positions && conv_state && qk && kt && v &&
+    SKYRL_REQUIRE(proj && conv_w && a_log && dt_bias && chunk && cu && rows && positions && conv_state && qk && kt && vt &&
                       lg && beta,
                   "delta_conv: null pointer");
     SKYRL_DISPATCH_T(dtype, {
-        hipLaunchKernelGGL((delta_conv_kernel<T>), dim3(nchunks, d.K + (d.H * d.V + kNT - 1) / kNT), dim3(kNT),
-                           16 * 2 * d.D * sizeof(float), as_stream(stream), d, SeqRef{chunk, cu, rows, positions},
-                           reinterpret_cast<const T*>(proj), proj_stride, reinterpret_cast<const T*>(conv_w), a_log,
-                           dt_bias, reinterpret_cast<const T*>(conv_state), qk, kt, v, lg, beta);
+#define LAUNCH_CONV(TAPS)                                                                                                 \
+    hipLaunchKernelGGL((delta_conv_kernel<T, TAPS>), dim3(nchunks, d.K + (d.H * d.V + kNT - 1) / kNT), dim3(kNT),          \
+                       16 * (2 * d.D + 4) * sizeof(float), as_stream(stream), d, SeqRef{chunk, cu, rows, positions},       \
+                       reinterpret_cast<const T*>(proj), proj_stride, reinterpret_cast<const T*>(conv_w), a_log, dt_bias,  \
+                       reinterpret_cast<const T*>(conv_state), qk, kt, vt, lg, beta)
+        if (d.taps <= 4) LAUNCH_CONV(4);
+        else if (d.taps <= kConvWindow) LAUNCH_CONV(kConvWindow);
+        else LAUNCH_CONV(0);
     })
     return check_launch("delta_conv_kernel");
 }
 
 extern "C" int skyrl_delta_chunk(const skyrl_delta_shape* shape, const int32_t* chunk, int32_t nchunks,
-                                 const float* qk, const float* v, const float* lg, const float* beta, float* W,
-                                 float* U, float* P, float* G, void* stream) {
+                                 const float* qk, const float* kt, const float* vt, const float* lg, const float* beta,
+                                 float* W, float* U, float* P, float* G, void* stream) {
     const char* bad = bad_shape(shape);
     SKYRL_REQUIRE(!bad, bad);
     const Dims d = dims_of(shape);
     SKYRL_REQUIRE(nchunks >= 0 && (int64_t)nchunks * d.H < (1 << 30), "delta_chunk: bad sizes");
     if (nchunks == 0) return SKYRL_OK;
-    SKYRL_REQUIRE(chunk && qk && v && lg && beta && W && U && P && G, "delta_chunk: null pointer");
-    hipLaunchKernelGGL(delta_chunk_kernel, dim3(nchunks * d.H), dim3(kNT), 0, as_stream(stream), d, chunk, qk, v, lg,
-                       beta, W, U, P, G);
+    SKYRL_REQUIRE(chunk && qk && kt && vt && lg && beta && W && U && P && G, "delta_chunk: null pointer");
+    hipLaunchKernelGGL(delta_chunk_kernel, dim3(nchunks * d.H), dim3(kNT), 0, as_stream(stream), d, chunk, qk, kt, vt,
+                       lg, beta, W, U, P, G);
     return check_launch("delta_chunk_kernel");
 }
 
-#define LAUNCH_CHAIN(NS, EXACT)                                                                                 \
-    hipLaunchKernelGGL((delta_chain_kernel<NS, EXACT>),                                                           \
+#define LAUNCH_CHAIN(NS, EXACT, SETS)                                                                           \
+    hipLaunchKernelGGL((delta_chain_kernel<NS, EXACT, SETS>),                                                           \
                        dim3((unsigned)(nseq * d.H + 7) / 8 * 8 * (d.v16() / 16)), dim3(kNT), 0, as_stream(stream), \
                        d, SeqRef{chunk, cu, rows, positions}, seq_chunks, seq0, nseq, qk, kt, W, U, P, G, state, o)
 
@@ -767,11 +819,11 @@ extern "C" int skyrl_delta_chain(const skyrl_delta_shape* shape, const int32_t* 
     if (nseq == 0) return SKYRL_OK;
     SKYRL_REQUIRE(chunk && seq_chunks && cu && rows && positions && qk && kt && W && U && P && G && state && o,
                   "delta_chain: null pointer");
-    if (d.D == 64) LAUNCH_CHAIN(4, true);
-    else if (d.D < 64) LAUNCH_CHAIN(4, false);
-    else if (d.D == 128) LAUNCH_CHAIN(8, true);
-    else if (d.D < 128) LAUNCH_CHAIN(8, false);
-    else LAUNCH_CHAIN(16, false);
+    if (d.D == 64) LAUNCH_CHAIN(4, true, 2);
+    else if (d.D < 64) LAUNCH_CHAIN(4, false, 2);
+    else if (d.D == 128) LAUNCH_CHAIN(8, true, 2);
+    else if (d.D < 128) LAUNCH_CHAIN(8, false, 2);
+    else LAUNCH_CHAIN(16, false, 1);
     return check_launch("delta_chain_kernel");
 }
 
