@@ -53,6 +53,7 @@ extern "C" {
  *                   or as f32 [splits, n, ldo] whose sum over the first index is the product, the bias in the first. act
  *                   of skyrl_gate_mul: w holds N gate rows, then N up rows; the gated product bf16 [n, N], splits 0.
  *                   skyrl_rows_product_fits: whether it takes the sizes; skyrl_rows_product_splits: the splits.
+ *   skyrl_rows_batch  `batch` such products without bias, x, w and out bf16 x_batch, w_batch and out_batch apart.
  *   skyrl_add_norm_parts, skyrl_gate_norm_add_parts  of a model in bf16, the sublayer's output being such a sum of
  *                   `parts` (a_shares > 0) f32 [n, H], or (gate_shares > 0) the gate's logits being one of f32
  *                   [n, gate_stride]. */
@@ -83,6 +84,8 @@ int32_t skyrl_rows_product_splits(int32_t n, int32_t K, int32_t N);
 int skyrl_rows_product(const void* x, int64_t ldx, int32_t n, int32_t K, const void* w, int64_t ldw, int32_t N,
                        const void* bias, int32_t act, float alpha, float limit, int32_t splits, void* out, int64_t ldo,
                        void* stream);
+int skyrl_rows_batch(const void* x, int64_t ldx, int64_t x_batch, int32_t n, int32_t K, const void* w, int64_t ldw,
+                     int64_t w_batch, int32_t N, int32_t batch, void* out, int64_t ldo, int64_t out_batch, void* stream);
 int skyrl_add_norm_parts(const float* delta, int32_t parts, float* hidden, const void* step, const void* weight, float w_base,
                          int32_t n, int32_t H, float eps, int32_t kind, void* out, void* stream);
 int skyrl_gate_norm_add_parts(const void* a, int32_t a_shares, int32_t parts, const void* gate, int32_t gate_shares,

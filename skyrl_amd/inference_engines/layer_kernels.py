@@ -97,6 +97,27 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
     return out
 
 
+# Rows up to which the products of a batch are faster here: 16 / 32 heads' two products and the copy between layouts took the library
+# 24.1 / 27.1 us for 256 rows, 11.3 / 22.7 us here, and 21.4 / 27.0 us for 512, 22.2 / 36.6 us here.
+BATCH_ROWS = 256
+
+
+def rows_batch(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> bool:
+    """out [B, n, N] = x [B, n, K] w [B, N, K]^T for every B, each with unit column stride and any other strides; False
+    (nothing done) for sizes, types and alignments that are the library's."""
+    B, n, K = x.shape
+    N = w.shape[1]
+    if w.shape != (B, N, K) or out.shape != (B, n, N):
+        raise ValueError(f"w and out must be [{B}, N, {K}] and [{B}, {n}, N], got {tuple(w.shape)} and {tuple(out.shape)}")
+    if (not 0 < n <= BATCH_ROWS or K % 8 or any(t.dtype != torch.bfloat16 or not t.is_cuda or t.stride(2) != 1 for t in (x, w, out))
+            or any(s % 8 for t in (x, w) for s in t.stride()[:2]) or w.stride(1) < K or x.data_ptr() % 16 or w.data_ptr() % 16):
+        return False
+    dev = _require_gpu(x, w, out)
+    _ffi.call("skyrl_rows_batch", _ptr(x), x.stride(1), x.stride(0), n, K, _ptr(w), w.stride(1), w.stride(0), N, B, _ptr(out),
+              out.stride(1), out.stride(0), _stream(dev))
+    return True
+
+
 def joined(y: torch.Tensor) -> torch.Tensor:
     """A product's rows [n, N] from what linear returned."""
     return y if y.dim() == 2 else y.sum(0)

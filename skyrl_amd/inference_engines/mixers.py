@@ -330,7 +330,8 @@ class LatentAttention:
         self.dkv_norm = w.ones(self.rank) if own else None
         self.wuk = w.matrix(H * self.dim, self.rank)
         self.wuv = w.matrix(H * self.vdim, self.rank)
-        self.wuv_t = w.zeros(H, self.rank, self.vdim)  # per head transposed: the decode form's right operand
+        # per head transposed: the decode form's right operands, of the library's products and of rows_batch
+        self.wuv_t, self.wuk_t = w.zeros(H, self.rank, self.vdim), w.zeros(H, self.rank, self.dim)
         self.sinks = w.zeros(H, dtype=torch.float32) if sink else None
         self.refresh()
 
@@ -347,6 +348,7 @@ class LatentAttention:
     def refresh(self) -> None:
         """Recompute derived tensors, in place, after the weights changed."""
         self.wuv_t.copy_(self.wuv.view(self.heads, self.vdim, self.rank).transpose(1, 2))
+        self.wuk_t.copy_(self.wuk.view(self.heads, self.dim, self.rank).transpose(1, 2))
 
     # ---- cache
     def block_bytes(self) -> int:
@@ -385,12 +387,16 @@ class LatentAttention:
         H, D, R = self.heads, self.dim, self.rank
         n = b - a
         q3 = q[a:b].view(n, H, D + self.rot_dim)
-        qa = torch.bmm(q3[:, :, :D].transpose(0, 1), self.wuk.view(H, D, R))
+        qa = torch.empty((H, n, R), dtype=q.dtype, device=q.device)
+        if not lk.rows_batch(q3[:, :, :D].transpose(0, 1), self.wuk_t, qa):
+            qa = torch.bmm(q3[:, :, :D].transpose(0, 1), self.wuk.view(H, D, R))
         o = lk.latent_attend(qa, q3[:, :, D:], cache, R, self.rot_dim, inp.block_tables, inp.bt_row[a:b],
                              inp.positions[a:b], self.scale, self.window, nparts=self.nparts(n, inp.max_ctx),
                              part_min=kernels.MIN_PARTITION, workspace=workspace, sinks=self.sinks,
                              gate=None if gate is None else gate[a:b])
-        out[a:b].view(n, H, self.vdim).copy_(torch.bmm(o, self.wuv_t).transpose(0, 1))
+        to = out[a:b].view(n, H, self.vdim).transpose(0, 1)
+        if not lk.rows_batch(o, self.wuv.view(H, self.vdim, R), to):
+            to.copy_(torch.bmm(o, self.wuv_t))
 
     def inner(self, proj: torch.Tensor, out: torch.Tensor, inp, cache: torch.Tensor, workspace) -> None:
         H, T, qr = self.heads, proj.shape[0], self.q_rank

@@ -102,3 +102,18 @@ def test_norms_of_parts(dev, n, H, parts):
         y = lk.gate_norm_add(d, got, w, nxt, 1e-6, groups=groups, mult=0.5, gate=z, gate_bias=b)
         torch.testing.assert_close(got.double(), full, atol=2e-5, rtol=1e-5)
         torch.testing.assert_close(y.double(), norm(full) * nxt.double(), atol=1e-4, rtol=2 ** -8)
+
+
+@pytest.mark.parametrize("B,n,N,K", [(16, 1, 512, 128), (3, 2, 40, 24), (5, 17, 130, 264), (2, 33, 24, 136), (4, 64, 128, 512),
+                                     (3, 65, 50, 200), (2, 200, 72, 328), (1, 256, 16, 64)])
+def test_batch(dev, B, n, N, K):
+    g = torch.Generator(device=dev).manual_seed(B + n)
+    x = torch.randn(n, B, K + 8, device=dev, generator=g).bfloat16()[:, :, :K].transpose(0, 1)  # heads side by side in a row
+    w = torch.randn(B, N, K, device=dev, generator=g).bfloat16()
+    out = torch.full((n, B, N), float("nan"), device=dev, dtype=torch.bfloat16).transpose(0, 1)
+    assert lk.rows_batch(x, w, out)
+    for b in range(B):
+        ref, off = _bounds(x[b], w[b])
+        assert bool(((out[b].double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2 * off).all())
+    assert not lk.rows_batch(x[:, :, 1:], w[:, :, 1:].contiguous(), out)  # a depth and rows that are not 16-byte pieces
+    assert not lk.rows_batch(x.float(), w.float(), out.float())
