@@ -397,8 +397,8 @@ int skyrl_gdelta_out(const skyrl_gdelta_shape* shape, const int32_t* chunk, int3
  *   skyrl_moe_tiles    the most tiles of tm rows that npairs pairs can fill.
  *   skyrl_moe_sort     pairs by expert: order i32 [ntiles, tm] (pair, or -1), tile_expert i32 [ntiles + 1] (-1: unused; the
  *                      last: tiles in use). counts: scratch of skyrl_moe_counts(experts, npairs) i32 (0: NULL).
- *   skyrl_moe_gate_up  act T [ntiles tm, ff], by sorted place = silu(gate x) * up x. tm a multiple of 16; 16, 64, 128 and
- *                      256 have a matrix form (bf16, width and ff multiples of 8).
+ *   skyrl_moe_gate_up  act T [ntiles tm, ff], by sorted place = silu(gate x) * up x. tm a multiple of 16; 16, 32, 64, 128
+ *                      and 256 have a matrix form (bf16, width and ff multiples of 8).
  *   skyrl_moe_down     out T [n top, width], by pair = weight * down act. */
 typedef struct {
     int32_t width, ff, experts, top, groups, keep;

@@ -13,15 +13,10 @@
 // The products stage pieces of the rows and of the weight rows through LDS (16-byte direct loads, chunk index
 // xor-swizzled by the row so that the reads of 16 rows do not conflict), weights as the left operand: a lane holds
 // four consecutive columns of a token. Small tiles (decode) keep several stages in flight: they stream weights.
-#include "elem.h"
+#include "stream.h"
 
 namespace skyrl {
 namespace {
-
-typedef short s16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) void lds_void;
-typedef __attribute__((address_space(1))) void gbl_void;
 
 constexpr int kNT = 256;
 constexpr int kMaxExperts = 1024;
@@ -373,7 +368,50 @@ __device__ __forceinline__ void wait_loads() {
 __device__ __forceinline__ void lds_read(s16x8& v, uint32_t at, int offset) {
     asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(at), "n"(offset));
 }
-__device__ const uint4 kZero16 = {0u, 0u, 0u, 0u};
+
+// A tile of 16 MT rows (a few pairs per expert, decode steps): 16 NT weight rows (GATED: half of each matrix) per workgroup, whose
+// waves stream a share of the depth each (stream.h). Bound: the experts' weights, each read once. Measured, 64 experts of 768 x
+// 2048, 8 per token, gate_up / down, us (TB/s of weights) against moe_gemm_kernel's, whose stages hold two workgroups a CU, in
+// step: 4 tokens 32.1 / 16.9 (5.3 / 5.0) against 41.5 / 17.7, 64 tokens 69.8 / 38.8 (5.8 / 5.2) against 83.0 / 39.4,
+// 128 tokens in tiles of 32 72.8 / 42.3 against 86.8 / 41.3, 256 in tiles of 64 79.9 / - against 86.8 / 42.5.
+template <int NT, int MT, int WK, int S, bool GATED>
+__global__ __launch_bounds__(WK* kWave) void moe_stream_kernel(Product p, const uint16_t* __restrict__ x,
+                                                               const uint16_t* __restrict__ w, uint16_t* __restrict__ out,
+                                                               int ncols) {
+    using St = Stream<NT, MT, WK, S>;
+    constexpr int OC = GATED ? St::BN / 2 : St::BN;
+    __shared__ __attribute__((aligned(16))) uint16_t smem[St::kLds];
+    const int tile = blockIdx.x / ncols, n0 = blockIdx.x % ncols * OC;
+    const int e = p.tile_expert[tile];
+    if (e < 0) return;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t place0 = (int64_t)tile * St::BM;
+    const uint16_t* we = w + (int64_t)e * (GATED ? 2 : 1) * p.N * p.K;
+    const int steps = (p.K + 63) / 64, s0 = steps * wave / WK, nk = steps * (wave + 1) / WK - s0;
+    f32x4 acc[MT][NT];
+    St::run(
+        smem, p.K, s0, nk,
+        [&](int r) { return we + (int64_t)((GATED && r >= OC ? p.N : 0) + min(n0 + (GATED ? r % OC : r), p.N - 1)) * p.K; },
+        [&](int r) {  // places without a pair: row 0, not stored
+            const int pair = p.order[place0 + r];
+            return x + (pair < 0 ? 0 : p.row_div ? pair / p.row_div : place0 + r) * p.K;
+        },
+        acc);
+    St::store(smem, acc);
+    for (int i = tid; i < St::BM * (OC / 4); i += WK * kWave) {
+        const int r = i / (OC / 4), n = i % (OC / 4) * 4, col = n0 + n, pair = p.order[place0 + r];
+        if (pair < 0 || col >= p.N) continue;  // N is a multiple of 8
+        f32x4 y = St::total(smem, r, n);
+        if constexpr (GATED) {
+            const f32x4 u = St::total(smem, r, OC + n);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) y[j] = y[j] * sigmoid_<uint16_t>(y[j]) * u[j];
+        } else {
+            y = y * (p.weight ? p.weight[pair] : 1.f);
+        }
+        st4(out + (p.out_pairs ? (int64_t)pair : place0 + r) * p.N + col, make_float4(y[0], y[1], y[2], y[3]));
+    }
+}
 
 // A workgroup: one tile of TM rows and TN weight rows (GATED: half of each matrix, the same columns), WM x WN waves. S
 // stages of 64-deep pieces. Tiles of one expert share its weights and a tile's columns its rows: with several tiles per
@@ -544,12 +582,12 @@ __global__ __launch_bounds__(WM* WN* kWave) void moe_gemm_kernel(Product p, cons
 }
 
 bool fast_form(int K, int N, int tm, int dtype, const void* x, const void* w, const void* out) {
-    return dtype == SKYRL_BF16 && K % 8 == 0 && N % 8 == 0 && (tm == 16 || tm == 64 || tm == 128 || tm == 256) && aligned16(x) &&
+    return dtype == SKYRL_BF16 && K % 8 == 0 && N % 8 == 0 && (tm == 16 || tm == 32 || tm == 64 || tm == 128 || tm == 256) && aligned16(x) &&
            aligned16(w) && aligned16(out);
 }
 
 template <bool GATED>
-int launch_product(const Product& p, const void* x, const void* w, void* out, int ntiles, int dtype, hipStream_t s) {
+int launch_product(const Product& p, const void* x, const void* w, void* out, int ntiles, int experts, int dtype, hipStream_t s) {
     if (fast_form(p.K, p.N, p.tm, dtype, x, w, out)) {
         const uint16_t* x_ = reinterpret_cast<const uint16_t*>(x);
         const uint16_t* w_ = reinterpret_cast<const uint16_t*>(w);
@@ -563,9 +601,25 @@ int launch_product(const Product& p, const void* x, const void* w, void* out, in
         hipLaunchKernelGGL((moe_gemm_kernel<TM, TN, WM, WN, S, GATED>), dim3((unsigned)(TM > 16 ? grid : (int64_t)ncols * ntiles)), \
                            dim3(WM * WN * kWave), 0, s, p, x_, w_, o_, ncols, ntiles);                                \
     } while (0)
+#define LAUNCH_STREAM(NT, MT, WK, S)                                                                                  \
+    do {                                                                                                              \
+        constexpr int kCols = GATED ? 8 * NT : 16 * NT;                                                               \
+        const int64_t ncols = (p.N + kCols - 1) / kCols;                                                              \
+        SKYRL_REQUIRE(ncols * ntiles < (1ll << 31), "moe: grid too large");                                           \
+        hipLaunchKernelGGL((moe_stream_kernel<NT, MT, WK, S, GATED>), dim3((unsigned)(ncols * ntiles)), dim3(WK * kWave), 0, s, \
+                           p, x_, w_, o_, (int)ncols);                                                                \
+    } while (0)
+        // Streamed where an expert has about one tile, so that its weights are read once: tiles of 16 below 16 pairs per
+        // expert (ntiles is npairs / tm + experts), of 32, and, for the wider of the two products, of 64 from 24 pairs on. Tiles
+        // of 16 and 64 that are asked for at other loads sum a row in the order that larger ones do.
+        const bool once = ntiles <= 2 * experts;
         if (p.tm == 256) LAUNCH_GEMM(256, 256, 2, 4, 2);
         else if (p.tm == 128) LAUNCH_GEMM(128, 128, 2, 2, 2);
-        else if (p.tm == 64) LAUNCH_GEMM(64, 128, 2, 2, 3);
+        else if (p.tm == 64) {
+            if (GATED && once && (int64_t)(ntiles - experts) * 64 >= 24ll * experts) LAUNCH_STREAM(4, 4, 2, 2);
+            else LAUNCH_GEMM(64, 128, 2, 2, 3);
+        } else if (p.tm == 32) LAUNCH_STREAM(4, 2, 4, 1);
+        else if (once) LAUNCH_STREAM(4, 1, 4, 2);
         else LAUNCH_GEMM(16, 128, 1, 4, 4);
         return check_launch("moe_gemm_kernel");
     }
@@ -687,7 +741,7 @@ extern "C" int skyrl_moe_gate_up(const skyrl_moe_shape* shape, const void* x, co
     if (ntiles == 0) return SKYRL_OK;
     SKYRL_REQUIRE(x && w && order && tile_expert && act, "moe_gate_up: null pointer");
     const Product p{shape->width, shape->ff, order, tile_expert, tm, shape->top, nullptr, 0};
-    return launch_product<true>(p, x, w, act, ntiles, dtype, as_stream(stream));
+    return launch_product<true>(p, x, w, act, ntiles, shape->experts, dtype, as_stream(stream));
 }
 
 extern "C" int skyrl_moe_down(const skyrl_moe_shape* shape, const void* act, const void* w, const int32_t* order,
@@ -700,5 +754,5 @@ extern "C" int skyrl_moe_down(const skyrl_moe_shape* shape, const void* act, con
     if (ntiles == 0) return SKYRL_OK;
     SKYRL_REQUIRE(act && w && order && tile_expert && weight && out, "moe_down: null pointer");
     const Product p{shape->ff, shape->width, order, tile_expert, tm, 0, weight, 1};
-    return launch_product<false>(p, act, w, out, ntiles, dtype, as_stream(stream));
+    return launch_product<false>(p, act, w, out, ntiles, shape->experts, dtype, as_stream(stream));
 }

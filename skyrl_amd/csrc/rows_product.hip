@@ -3,10 +3,8 @@
 // Bound: the weights' bytes. At 1 to 128 rows a weight matrix is read once and used little, and what the time went on
 // before was how it was read: the library's tiles for these shapes leave most CUs idle or few loads in flight. Here:
 //   one row   a wave per weight row (or gate and up row), lanes along the depth, so that every load is 1 KB of one row.
-//   more      a wave owns 16 NT weight rows and a share of the depth alone: it fetches its pieces (64 deep, whole 128-byte
-//             lines, chunks xor-swizzled by the row) with direct loads into LDS of its own, S of them in flight, and
-//             never meets the other waves until the sums of the shares are joined. Few weight rows are cut into
-//             `splits` shares of the depth across workgroups too, each with f32 sums of its own that the next norm adds.
+//   more      a wave has a share of the depth to itself (stream.h). Few weight rows are cut into `splits` shares of the
+//             depth across workgroups too, each with f32 sums of its own that the next norm adds.
 // Measured on one MI355X, weights from HBM, us (GB/s of weights) against the library's:
 //   N, K            1 row            16 rows          32 rows          64 rows
 //   2048, 2048      3.8 / 11.0       4.1 / 11.1       4.4 / 11.3       5.3 / 11.8
@@ -17,14 +15,10 @@
 // Batches (a head's up-projections of latent attention, 512 x 128 and 128 x 512): 16 heads, 1 / 64 rows, both products with the
 // copy that the library's needed: 15.4 / 17.1 us, here 5.9 / 7.6 us.
 #include "gate.h"
+#include "stream.h"
 
 namespace skyrl {
 namespace {
-
-typedef short s16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) void lds_void;
-typedef __attribute__((address_space(1))) void gbl_void;
 
 enum Mode { kRound, kParts, kGated };
 
@@ -42,15 +36,6 @@ struct RowsProduct {
     int row_blocks;  // gridDim.z = batch row_blocks
     int64_t x_batch, w_batch, out_batch;
 };
-
-template <int N>
-__device__ __forceinline__ void wait_loads() {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-__device__ __forceinline__ void lds_read(s16x8& v, uint32_t at, int offset) {
-    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(at), "n"(offset));
-}
-__device__ const uint4 kZero16 = {0u, 0u, 0u, 0u};
 
 // One row: R consecutive outputs per wave (kGated: R pairs), C loads of every weight row in flight.
 template <int MODE, int C, int NWV>
@@ -102,110 +87,30 @@ __global__ __launch_bounds__(NWV* kWave) void one_row_kernel(RowsProduct p) {
 // blocks of MT tiles and products of a batch along z.
 template <int MODE, int NT, int MT, int WK, int S>
 __global__ __launch_bounds__(WK* kWave) void rows_product_kernel(RowsProduct p) {
-    constexpr int BN = 16 * NT, BM = 16 * MT, WP = 2 * NT, XP = 2 * MT, L = WP + XP;  // 1 KB pieces: 8 rows, 64 deep
-    constexpr int OC = MODE == kGated ? BN / 2 : BN;  // output columns
-    constexpr int kStage = (BN + BM) * 64;            // elements
-    constexpr int LR = BN + 4;                        // a row of a share's sums
-    constexpr int kSums = WK * BM * LR * 2, kPieces = WK * S * kStage;
+    using St = Stream<NT, MT, WK, S>;
+    constexpr int BM = St::BM, OC = MODE == kGated ? St::BN / 2 : St::BN;  // output columns
     static_assert(MODE != kGated || NT % 2 == 0, "gate and up rows");
-    static_assert(S <= 4, "the waits below");
-    __shared__ __attribute__((aligned(16))) uint16_t smem[kPieces > kSums ? kPieces : kSums];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int c = lane & 15, g = lane >> 4;
+    __shared__ __attribute__((aligned(16))) uint16_t smem[St::kLds];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n0 = blockIdx.x * OC, batch = blockIdx.z / p.row_blocks, m0 = blockIdx.z % p.row_blocks * BM;
     const int steps = (p.K + 63) / 64, shares = gridDim.y * WK, share = blockIdx.y * WK + wave;
     const int s0 = (int)((int64_t)steps * share / shares), nk = (int)((int64_t)steps * (share + 1) / shares) - s0;
-    uint16_t* own = smem + wave * (S * kStage);
-    // this lane's 16 bytes of every piece: row lane / 8, chunk (lane % 8) ^ row, so that 16 rows read at a time lie in
-    // different banks; rows past the last are the last again and are not stored
-    const int r8 = lane >> 3, ch = ((lane & 7) ^ r8) * 8;
-    const uint16_t *ws[WP], *xs[XP];
-#pragma unroll
-    for (int i = 0; i < WP; ++i) {
-        const int r = i * 8 + r8;
-        const int row = MODE == kGated && r >= OC ? p.N + min(n0 + r - OC, p.N - 1) : min(n0 + r, p.N - 1);
-        ws[i] = p.w + batch * p.w_batch + row * p.ldw + s0 * 64 + ch;
-    }
-#pragma unroll
-    for (int i = 0; i < XP; ++i) xs[i] = p.x + batch * p.x_batch + min(m0 + i * 8 + r8, p.n - 1) * p.ldx + s0 * 64 + ch;
-    auto fetch = [&](int t) {
-        uint16_t* dst = own + (t % S) * kStage;
-        const bool in = (s0 + t) * 64 + ch < p.K;  // K is a multiple of 8
-#pragma unroll
-        for (int i = 0; i < WP; ++i) {
-            const void* src = in ? (const void*)(ws[i] + t * 64) : (const void*)&kZero16;
-            __builtin_amdgcn_global_load_lds((gbl_void*)src, (lds_void*)(dst + i * 512), 16, 0, 0);
-        }
-#pragma unroll
-        for (int i = 0; i < XP; ++i) {
-            const void* src = in ? (const void*)(xs[i] + t * 64) : (const void*)&kZero16;
-            __builtin_amdgcn_global_load_lds((gbl_void*)src, (lds_void*)(dst + (WP + i) * 512), 16, 0, 0);
-        }
-    };
     f32x4 acc[MT][NT];
-#pragma unroll
-    for (int m = 0; m < MT; ++m)
-#pragma unroll
-        for (int n = 0; n < NT; ++n) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int t = 0; t < S; ++t)
-        if (t < nk) fetch(t);
-    const uint32_t base = (uint32_t)(uintptr_t)(lds_void*)own + c * 128;
-    for (int t = 0; t < nk; ++t) {
-        const int left = nk - 1 - t;  // pieces after this one; at most S - 1 of them are under way
-        if (left >= S - 1) wait_loads<(S - 1) * L>();
-        else if (S > 3 && left == 2) wait_loads<2 * L>();
-        else if (S > 2 && left == 1) wait_loads<L>();
-        else wait_loads<0>();
-        // The reads are not the compiler's: it would wait for every load into LDS under way before one. They are waited
-        // for at once, and their registers tied past the wait.
-        s16x8 wf[2][NT], xf[2][MT];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const uint32_t at = base + (t % S) * kStage * 2 + ((h * 4 + g) ^ (c & 7)) * 16;
-#pragma unroll
-            for (int n = 0; n < NT; ++n) lds_read(wf[h][n], at, n * 2048);
-#pragma unroll
-            for (int m = 0; m < MT; ++m) lds_read(xf[h][m], at, (NT + m) * 2048);
-        }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-#pragma unroll
-            for (int n = 0; n < NT; ++n) asm volatile("" : "+v"(wf[h][n]));
-#pragma unroll
-            for (int m = 0; m < MT; ++m) asm volatile("" : "+v"(xf[h][m]));
-        }
-        if (t + S < nk) fetch(t + S);  // over the piece that has been read
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int m = 0; m < MT; ++m)
-#pragma unroll
-                for (int n = 0; n < NT; ++n)
-                    acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[h][n], xf[h][m], acc[m][n], 0, 0, 0);
-    }
-    __syncthreads();  // nothing is under way any more: the sums take the pieces' place
-    float* sums = reinterpret_cast<float*>(smem);
-#pragma unroll
-    for (int m = 0; m < MT; ++m)
-#pragma unroll
-        for (int n = 0; n < NT; ++n)
-            *reinterpret_cast<f32x4*>(sums + (wave * BM + m * 16 + c) * LR + n * 16 + 4 * g) = acc[m][n];
-    __syncthreads();
-    auto total = [&](int m, int n) {
-        f32x4 s = *reinterpret_cast<f32x4*>(sums + m * LR + n);
-#pragma unroll
-        for (int k = 1; k < WK; ++k) s += *reinterpret_cast<f32x4*>(sums + (k * BM + m) * LR + n);
-        return s;
-    };
+    St::run(
+        smem, p.K, s0, nk,
+        [&](int r) {  // rows past the last: the last
+            const int row = MODE == kGated && r >= OC ? p.N + min(n0 + r - OC, p.N - 1) : min(n0 + r, p.N - 1);
+            return p.w + batch * p.w_batch + row * p.ldw;
+        },
+        [&](int r) { return p.x + batch * p.x_batch + min(m0 + r, p.n - 1) * p.ldx; }, acc);
+    St::store(smem, acc);
     const bool four = p.N % 4 == 0 && p.ldo % 4 == 0 && p.out_batch % 4 == 0 && (reinterpret_cast<uintptr_t>(p.out) & 7) == 0;
     for (int i = tid; i < BM * (OC / 4); i += WK * kWave) {
         const int m = i / (OC / 4), n = i % (OC / 4) * 4, col = n0 + n;
         if (m0 + m >= p.n || col >= p.N) continue;
-        f32x4 y = total(m, n);
+        f32x4 y = St::total(smem, m, n);
         if constexpr (MODE == kGated) {
-            const f32x4 u = total(m, OC + n);
+            const f32x4 u = St::total(smem, m, OC + n);
 #pragma unroll
             for (int j = 0; j < 4; ++j) y[j] = gated(y[j], u[j], p.gate);
         } else if (p.bias && blockIdx.y == 0) {

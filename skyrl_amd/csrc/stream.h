@@ -1,0 +1,129 @@
+// Products of few bf16 rows with streamed weight rows on the matrix instructions (rows_product.hip, moe.hip). A wave fetches its
+// own share of the depth, in pieces of 64, with direct loads into LDS of its own: whole 128-byte lines, 16-byte chunks
+// xor-swizzled by the row, S pieces under way. Waves meet when the shares' sums are joined, not before.
+#pragma once
+#include "elem.h"
+
+namespace skyrl {
+
+typedef short s16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) void lds_void;
+typedef __attribute__((address_space(1))) void gbl_void;
+
+__device__ const uint4 kZero16 = {0u, 0u, 0u, 0u};
+
+// NT 16-row weight tiles, MT 16-row tiles of x, WK waves.
+template <int NT, int MT, int WK, int S>
+struct Stream {
+    static constexpr int BN = 16 * NT, BM = 16 * MT, WP = 2 * NT, XP = 2 * MT, L = WP + XP;  // 1 KB pieces: 8 rows, 64 deep
+    static constexpr int kStage = (BN + BM) * 64;  // elements
+    static constexpr int LR = BN + 4;              // a row of a share's sums
+    static constexpr int kSums = WK * BM * LR * 2, kPieces = WK * S * kStage;
+    static constexpr int kLds = kPieces > kSums ? kPieces : kSums;  // elements
+    static_assert(S <= 4, "the waits below");
+
+    template <int N>
+    static __device__ __forceinline__ void wait_loads() {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+    }
+    static __device__ __forceinline__ void lds_read(s16x8& v, uint32_t at, int offset) {
+        asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(at), "n"(offset));
+    }
+
+    // acc[m][n]: lane (c, g) has x row 16 m + c, weight rows 16 n + 4 g .. + 3. wrow(r), xrow(r): start of the tile's row r, valid
+    // for every r (rows past the last: any row, not stored). K a multiple of 8, the wave's pieces s0 .. s0 + nk - 1 of 64.
+    template <class WRow, class XRow>
+    static __device__ __forceinline__ void run(uint16_t* smem, int K, int s0, int nk, WRow wrow, XRow xrow, f32x4 (&acc)[MT][NT]) {
+        const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        const int c = lane & 15, g = lane >> 4;
+        uint16_t* own = smem + wave * (S * kStage);
+        // this lane's 16 bytes of every piece: row lane / 8, chunk (lane % 8) ^ row, so that 16 rows read at a time lie in
+        // different banks
+        const int r8 = lane >> 3, ch = ((lane & 7) ^ r8) * 8;
+        const uint16_t *ws[WP], *xs[XP];
+#pragma unroll
+        for (int i = 0; i < WP; ++i) ws[i] = wrow(i * 8 + r8) + s0 * 64 + ch;
+#pragma unroll
+        for (int i = 0; i < XP; ++i) xs[i] = xrow(i * 8 + r8) + s0 * 64 + ch;
+        auto fetch = [&](int t) {
+            uint16_t* dst = own + (t % S) * kStage;
+            const bool in = (s0 + t) * 64 + ch < K;
+#pragma unroll
+            for (int i = 0; i < WP; ++i) {
+                const void* src = in ? (const void*)(ws[i] + t * 64) : (const void*)&kZero16;
+                __builtin_amdgcn_global_load_lds((gbl_void*)src, (lds_void*)(dst + i * 512), 16, 0, 0);
+            }
+#pragma unroll
+            for (int i = 0; i < XP; ++i) {
+                const void* src = in ? (const void*)(xs[i] + t * 64) : (const void*)&kZero16;
+                __builtin_amdgcn_global_load_lds((gbl_void*)src, (lds_void*)(dst + (WP + i) * 512), 16, 0, 0);
+            }
+        };
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int n = 0; n < NT; ++n) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < S; ++t)
+            if (t < nk) fetch(t);
+        const uint32_t base = (uint32_t)(uintptr_t)(lds_void*)own + c * 128;
+        for (int t = 0; t < nk; ++t) {
+            const int left = nk - 1 - t;  // pieces after this one; at most S - 1 of them are under way
+            if (left >= S - 1) wait_loads<(S - 1) * L>();
+            else if (S > 3 && left == 2) wait_loads<2 * L>();
+            else if (S > 2 && left == 1) wait_loads<L>();
+            else wait_loads<0>();
+            // The reads are not the compiler's: it would wait for every load into LDS under way before one. They are waited
+            // for at once, and their registers tied past the wait.
+            s16x8 wf[2][NT], xf[2][MT];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const uint32_t at = base + (t % S) * kStage * 2 + ((h * 4 + g) ^ (c & 7)) * 16;
+#pragma unroll
+                for (int n = 0; n < NT; ++n) lds_read(wf[h][n], at, n * 2048);
+#pragma unroll
+                for (int m = 0; m < MT; ++m) lds_read(xf[h][m], at, (NT + m) * 2048);
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+#pragma unroll
+                for (int n = 0; n < NT; ++n) asm volatile("" : "+v"(wf[h][n]));
+#pragma unroll
+                for (int m = 0; m < MT; ++m) asm volatile("" : "+v"(xf[h][m]));
+            }
+            if (t + S < nk) fetch(t + S);  // over the piece that has been read
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int m = 0; m < MT; ++m)
+#pragma unroll
+                    for (int n = 0; n < NT; ++n)
+                        acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[h][n], xf[h][m], acc[m][n], 0, 0, 0);
+        }
+    }
+
+    // The waves' sums side by side in LDS, in the pieces' place; total() then adds them.
+    static __device__ __forceinline__ void store(uint16_t* smem, const f32x4 (&acc)[MT][NT]) {
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;
+        float* sums = reinterpret_cast<float*>(smem);
+        __syncthreads();  // nothing is under way any more
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+                *reinterpret_cast<f32x4*>(sums + (wave * BM + m * 16 + c) * LR + n * 16 + 4 * g) = acc[m][n];
+        __syncthreads();
+    }
+    // x row m, weight rows n .. n + 3
+    static __device__ __forceinline__ f32x4 total(const uint16_t* smem, int m, int n) {
+        const float* sums = reinterpret_cast<const float*>(smem);
+        f32x4 s = *reinterpret_cast<const f32x4*>(sums + m * LR + n);
+#pragma unroll
+        for (int k = 1; k < WK; ++k) s += *reinterpret_cast<const f32x4*>(sums + (k * BM + m) * LR + n);
+        return s;
+    }
+};
+
+}  // namespace skyrl

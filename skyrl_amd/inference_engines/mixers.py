@@ -1073,7 +1073,7 @@ class RoutedExperts:
     def forward(self, x: torch.Tensor, inp, state, workspace, logits=None) -> torch.Tensor:
         """logits: (layer_kernels.linear's parts that hold the router's, their first column)."""
         if logits is not None:
-            tm = lk.moe_tile(self.shape, x.shape[0])
+            tm = lk.moe_rows(self.shape, x.shape[0])
             idx, weight, *tiles = lk.moe_choose(self.shape, *logits, self.correction, tm)
             return lk.moe_experts(self.shape, x, idx, weight, self.gate_up, self.down, tm, tiles)
         idx, weight = lk.moe_route(self.shape, x, self.router, self.correction)

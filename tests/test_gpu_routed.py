@@ -359,6 +359,27 @@ def test_experts(width, ff, experts, top, n, dtype):
         close(lk.moe_experts(sh, dev(x), dev(idx), dev(weight), dev(wgu), dev(wd), tm=tm), want, dtype, f32=5e-6, bf16=8e-3)
 
 
+@pytest.mark.parametrize("width,ff,experts,top,n,tm", [(128, 64, 16, 2, 1, 16), (200, 72, 16, 2, 100, 16), (136, 40, 8, 2, 70, 32),
+                                                       (2048, 768, 64, 8, 95, 16), (1096, 200, 8, 4, 90, 32), (72, 136, 4, 2, 60, 64),
+                                                       (1024, 264, 16, 4, 128, 64)])
+def test_streamed_products(width, ff, experts, top, n, tm):
+    """Few pairs per expert: weights streamed by waves with a share of the depth each, at the edges of tiles and pieces."""
+    g = torch.Generator(device=DEV).manual_seed(width + n)
+    sh = lk.moe_shape(width, ff, experts, top)
+    mk = lambda *s, scale=1.0: (torch.randn(s, generator=g, device=DEV) * scale).to(BF16)  # noqa: E731
+    x, wgu, wd = mk(n, width), mk(experts, 2, ff, width, scale=width ** -0.5), mk(experts, width, ff, scale=ff ** -0.5)
+    idx = torch.stack([torch.randperm(experts, generator=g, device=DEV)[:top] for _ in range(n)]).int()
+    weight = torch.rand(n, top, generator=g, device=DEV)
+    y = lk.moe_experts(sh, x, idx, weight, wgu, wd, tm=tm).view(n, top, width)
+    want = torch.empty(n, top, width, dtype=torch.float64, device=DEV)
+    for t in range(n):
+        for k, e in enumerate(idx[t].tolist()):
+            h = x[t].double()
+            a = ref.silu(wgu[e, 0].double() @ h) * (wgu[e, 1].double() @ h)
+            want[t, k] = weight[t, k].double() * (wd[e].double() @ a)
+    close(y, want.cpu(), BF16, bf16=8e-3)
+
+
 @pytest.mark.parametrize("width,ff,experts,top,n", [(2048, 768, 32, 8, 1500), (1024, 512, 64, 4, 300), (4096, 320, 8, 2, 90)])
 def test_tile_sizes_agree_bit_for_bit(width, ff, experts, top, n):
     """A row's sums are formed in the same order whatever its tile: products of a real layer's size, over and over."""
