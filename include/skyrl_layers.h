@@ -362,11 +362,13 @@ int skyrl_ssd_prompt(const skyrl_ssd_shape* shape, const void* xt, const void* b
  * State per row: f32 [rows, heads, dim, vpad], vpad = dim up to a multiple of 4. Sequences, rows and chunks as for the
  * gated delta rule. dim <= 256.
  *   skyrl_gdelta_scan   token by token, the state in registers: decode steps and short portions.
- *   Prompt form, chunks of 64, d16 = dim up to a multiple of 16, all f32:
- *   skyrl_gdelta_chunk  1: what a chunk does to the state, S <- M S + N, and its outputs O + R S: M [nchunks, heads, d16,
- *                       d16], N [.., d16 values, d16 keys], R and O [.., 64, d16].
+ *   Prompt form, chunks of 64, d16 = dim up to a multiple of 16, all f32, in tiles of 16 x 16 (256 numbers, lane l the four
+ *   at 4 l; "operand": row l % 16, columns 4 (l / 16) ..; "result": rows 4 (l / 16) .., column l % 16):
+ *   skyrl_gdelta_chunk  1: what a chunk does to the state, S <- M S + N, and its outputs O + R S: M [nchunks, heads, key
+ *                       tiles, key tiles] operand, N [.., value tiles, key tiles] result, R [.., 4, key tiles] operand, O
+ *                       [.., 4, value tiles] result.
  *   skyrl_gdelta_chain  2: sequences seq0.. of nseq: the states along each sequence's chunks [seq_chunks[i], seq_chunks[i
- *                       + 1]), updated in `state`, every chunk's first one in first [nchunks, heads, d16 values, d16 keys].
+ *                       + 1]), updated in `state`, every chunk's first one in first, as N.
  *   skyrl_gdelta_out    3: outputs, head norm, weight and gate (gate T [T, gate_stride]: proj's output gate columns). */
 typedef struct {
     int32_t heads, dim;

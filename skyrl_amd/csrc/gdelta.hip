@@ -17,6 +17,8 @@
 // with a 16-column slice of S per workgroup and leaves every chunk's first state, gdelta_out forms O with the head
 // norms and the output gate. Everything is f32, the products on v_mfma_f32_16x16x4_f32: a lane's four consecutive k
 // values of a 16-step feed four instructions, the same permutation of k on both sides.
+#include <type_traits>
+
 #include "elem.h"
 
 namespace skyrl {
@@ -26,6 +28,8 @@ constexpr int kC = 64;   // tokens per chunk
 constexpr int LD = kC + 4;
 constexpr float kRate = 0.6065306597126334f;  // e^(-1/2)
 constexpr float kUnitEps = 1e-6f;
+constexpr float kLog2eLow = 1.9259629911e-8f;  // log2(e) less its f32 value
+constexpr float kLn2 = 0.6931471805599453f;
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -215,14 +219,367 @@ __device__ __forceinline__ f32x4 zero4() { return f32x4{0.f, 0.f, 0.f, 0.f}; }
 // exp of a summed log decay: the bare base-2 instruction (its argument is rounded once more than expf's)
 __device__ __forceinline__ float exp_sum(float x) { return fast_exp2(x * kLog2e); }
 
-// What gdelta_chunk leaves, all f32: M [chunk][head][d16][d16], N transposed [..][value][key], R and O0 [..][64][d16].
+// What gdelta_chunk leaves, all f32 per (chunk, head), in tiles of 16 x 16 as the next kernel's matrix instructions read
+// them, 256 numbers each, lane (g, c) = (lane / 16, lane % 16) the four at 4 lane: a wave's load is 1 KB in one piece
+// (row by row, 16 rows of 64 bytes, it comes at a quarter of the rate).
+//   left operands:   M [key out / 16][key in / 16]: rows c, columns 4 g + i;  R [token / 16][key / 16] alike.
+//   accumulators:    N [value / 16][key / 16]: rows (keys) 4 g + i, column (value) c;  O0 [token / 16][value / 16]: rows
+//                    (tokens) 4 g + i, column (value) c. `first` (gdelta_chain) as N: a result is a right operand.
 struct ChunkOut {
     float *M, *N, *R, *O;
 };
 
+__device__ __forceinline__ void put_tile(float* at, const f32x4& v) { *reinterpret_cast<f32x4*>(at) = v; }
+
+// 1 / (1 + e^-x) by the base-2 exponential, what its argument's rounding lost multiplied back, and a reciprocal with
+// one Newton step: as exact as sigmoidf_ in two thirds of its instructions. Past 88 either way the result is 1 or
+// below 1e-38; a NaN passes the comparisons.
+__device__ __forceinline__ float sigmoid_rcp(float x) {
+    x = x > 88.f ? 88.f : x;
+    x = x < -88.f ? -88.f : x;
+    const float hi = -x * kLog2e, lo = fmaf(-x, kLog2eLow, fmaf(-x, kLog2e, -hi));
+    float e = fast_exp2(hi);
+    e = fmaf(e, lo * kLn2, e) + 1.f;
+    const float r = __builtin_amdgcn_rcpf(e);
+    return fmaf(r, fmaf(-e, r, 1.f), r);
+}
+
+// Sums of squares over the wave's lanes, of k[lane / 8]: each exchange halves what a lane still adds up (10 of them, 48
+// for eight sums one by one).
+template <int N>
+__device__ __forceinline__ void fold_sums(float (&x)[8], int lane) {
+    const bool up = lane & (8 * N);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const float give = up ? x[i] : x[i + N], keep = up ? x[i + N] : x[i];
+        x[i] = keep + __shfl_xor(give, 8 * N, kWave);
+    }
+}
+__device__ __forceinline__ float sums8(const float (&k)[8], int lane) {
+    float x[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = k[i] * k[i];
+    fold_sums<4>(x, lane);
+    fold_sums<2>(x, lane);
+    fold_sums<1>(x, lane);
+#pragma unroll
+    for (int o = 4; o > 0; o >>= 1) x[0] += __shfl_xor(x[0], o, kWave);
+    return x[0];
+}
+__device__ __forceinline__ float masked(float x, int mask) { return __int_as_float(__float_as_int(x) & mask); }
+__device__ __forceinline__ float lane_value(float x, int lane) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane));
+}
+
+// dim <= 64: one workgroup of eight waves per (chunk, head), two workgroups on a CU (79 KB of LDS, 128 registers): one's
+// loads, exponentials and triangular solve run under the other's products. With X = T B the two products with V become
+// one each: O0 = (Q - P X) V and N = diag(e^{G_n}) (ka - X^T be)^T V.
+//   slabs  al, be, ka and rh as tiles [token / 16][channel / 16], four tokens of a channel side by side: a right operand
+//          (token by channel) in one 16-byte read, a left one (channels as k) in four 4-byte reads; 68 floats from one
+//          quad of tokens to the next keep both without bank conflicts.
+//   blocks the ten 16 x 16 blocks at and below the diagonal of A, B, P and Q, five a wave, then over the slabs of al and
+//          rh, whose columns the waves hold by then. A and P as left operands, B and Q as results.
+//   solve  wave b inverts diagonal block b by substitution and forms column b of T in A's place.
+//   then   waves 0..3: 16 channels each of W = T al, of R and of M, 16 values of O0; waves 4..7: a column each of X (in
+//          B's place, negated) and of Q - P X (in Q's place, a left operand), 16 channels of ka - X^T be and of N.
+// What the next kernel reads as a left operand is formed transposed, by the operands' exchange. f32 products bound it: 32
+// heads of 64, 91 chunks: 2016 instructions of 32 cycles a workgroup, 86 us, and 310 MB in and out, 67 us; it takes 168 us
+// (329 us with 142 KB and one workgroup on a CU, results by rows, expf and divisions for the gates; 177 us with four waves a
+// workgroup; loads and stores are 25 us of it, the rest the exponentials and the solve where both workgroups are in them).
+template <typename T>
+__global__ __launch_bounds__(512, 4) void gdelta_chunk64_kernel(Dims d, In<T> in, const int32_t* __restrict__ chunk,
+                                                                ChunkOut co) {
+    constexpr int QS = 68, TS = 4 * QS, SLAB = 16 * TS, LOW = 10 * 256, TW = 8;
+    __shared__ __attribute__((aligned(16))) float s_mem[2 * SLAB + 4 * LOW];
+    __shared__ __attribute__((aligned(16))) float s_seg[8 * kC], s_eg[kC];
+    float *s_be = s_mem, *s_ka = s_be + SLAB, *s_al = s_ka + SLAB, *s_rh = s_al + SLAB;
+    // after the blocks' products; V at last over A and P
+    float *s_A = s_al, *s_P = s_A + LOW, *s_B = s_P + LOW, *s_Q = s_B + LOW, *s_V = s_A;
+    const int h = blockIdx.x % d.H, ci = blockIdx.x / d.H;
+    const int32_t* ck = chunk + 4 * ci;
+    const int t0 = ck[0], n = ck[1];
+    const int D = d.D, D16 = d.d16(), HD = d.width(), nt = D16 / 16;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c = lane & 15, g = lane >> 4;
+    const int64_t rec = (int64_t)ci * d.H + h;
+    auto tri = [](int r, int b) { return (r * (r + 1) / 2 + b) * 256; };
+    auto right = [&](const float* slab, int s, int t) { return ld4(slab + (s * 4 + t) * TS + g * QS + 4 * c); };
+    auto left = [&](const float* slab, int s, int t) {
+        const float* p = slab + (s * 4 + t) * TS + (c >> 2) * QS + (c & 3) + 16 * g;
+        return make_float4(p[0], p[4], p[8], p[12]);
+    };
+    auto tile = [&](const float* at) { return ld4(at + 4 * lane); };
+    auto transposed = [&](float* at, const f32x4& x) {  // a result as a left operand
+#pragma unroll
+        for (int i = 0; i < 4; ++i) at[((c >> 2) * 16 + 4 * g + i) * 4 + (c & 3)] = x[i];
+    };
+
+    const int tw = TW * wave;  // the wave's first token of the slabs
+    float v[TW];               // value column `lane`
+    {                          // channel `lane`
+        const bool on = lane < D;
+        const int col = on ? lane : 0;
+        const float w0 = in.w0[h * D + col], ab = in.ab[h * D + col];
+        float r[TW], k[TW], a[TW], G[TW];
+        const T* p = in.proj + (int64_t)(t0 + min(tw, n - 1)) * in.stride + h * D;
+        const T* pl = in.wl + (int64_t)(t0 + min(tw, n - 1)) * in.wl_stride + h * D;
+#pragma unroll
+        for (int i = 0; i < TW; ++i) {
+            r[i] = ld(p + col);
+            k[i] = ld(p + HD + col);
+            v[i] = ld(p + 2 * HD + col);
+            a[i] = ld(p + 4 * HD + col);
+            G[i] = ld(pl + col);
+            if (tw + i < n - 1) p += in.stride, pl += in.wl_stride;
+        }
+        float sum = 0.f;
+#pragma unroll
+        for (int i = 0; i < TW; ++i) {
+            const int use = on && tw + i < n ? -1 : 0;  // by bits: a select's branch would be around the exponentials
+            G[i] = masked(-kRate * sigmoid_rcp(G[i] + w0), use);
+            a[i] = sigmoid_rcp(a[i] + ab);
+            r[i] = masked(r[i], use);
+            k[i] = masked(k[i], use);
+            v[i] = masked(v[i], use);
+            sum += G[i];
+        }
+        s_seg[wave * kC + lane] = sum;
+        const float norm = 1.f / sqrtf(sums8(k, lane) + kUnitEps);  // of token tw + lane / 8
+        __syncthreads();
+        float base = 0.f, all = 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float x = s_seg[j * kC + lane];
+            if (j < wave) base += x;
+            all += x;
+        }
+        if (wave == 0) s_eg[lane] = exp_sum(all);
+        float ep = exp_sum(base);
+        const int at = ((wave >> 1) * 4 + g) * TS + (wave & 1) * 2 * QS + 4 * c;
+#pragma unroll
+        for (int q = 0; q < TW / 4; ++q) {
+            float al[4], be[4], ka[4], rh[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int i = 4 * q + j;
+                base += G[i];
+                const float ec = exp_sum(base), en = exp_sum(-base), u = k[i] * lane_value(norm, 8 * i);
+                al[j] = ep * u;
+                be[j] = en * a[i] * u;
+                ka[j] = en * k[i];
+                rh[j] = ec * r[i];
+                ep = ec;
+            }
+            st4(s_al + at + q * QS, make_float4(al[0], al[1], al[2], al[3]));
+            st4(s_be + at + q * QS, make_float4(be[0], be[1], be[2], be[3]));
+            st4(s_ka + at + q * QS, make_float4(ka[0], ka[1], ka[2], ka[3]));
+            st4(s_rh + at + q * QS, make_float4(rh[0], rh[1], rh[2], rh[3]));
+        }
+        __syncthreads();
+    }
+    const int w = wave & 3;     // the wave's column
+    const bool mine = w < nt;   // channels and values 16 w ..
+    const bool lower = wave < 4;
+    float4 alc[4], rhc[4];      // waves 0..3: al as a right operand, rh as a transposed result
+    {
+        // blocks of matrix wave / 2 (A, B, P, Q): rows 0 and 3, or 1 and 2
+        const bool result = wave & 2, inner = wave & 1;
+        f32x4 acc[5];
+        const float* ls = wave < 4 ? s_al : s_rh;
+        const float* rs = result ? s_ka : s_be;
+        const int r0 = inner ? 1 : 0, r1 = inner ? 2 : 3, n0 = inner ? 2 : 1;
+        auto blocks = [&](auto result_, auto inner_) {
+#pragma unroll
+            for (int k = 0; k < 5; ++k) acc[k] = zero4();
+#pragma unroll 2
+            for (int t = 0; t < nt; ++t) {
+                constexpr int R0 = inner_ ? 1 : 0, R1 = inner_ ? 2 : 3;
+                const float4 x[2] = {left(ls, R0, t), left(ls, R1, t)};
+                float4 y[R1 + 1];
+#pragma unroll
+                for (int s = 0; s <= R1; ++s) y[s] = left(rs, s, t);
+#pragma unroll
+                for (int k = 0; k < 5; ++k) {
+                    const int q = k <= R0 ? 0 : 1, b = k - q * (R0 + 1);
+                    acc[k] = result_ ? mma4(x[q], y[b], acc[k]) : mma4(y[b], x[q], acc[k]);
+                }
+            }
+        };
+        using Yes = std::true_type;
+        using No = std::false_type;
+        if (result) {
+            if (inner) blocks(Yes{}, Yes{});
+            else blocks(Yes{}, No{});
+        } else {
+            if (inner) blocks(No{}, Yes{});
+            else blocks(No{}, No{});
+        }
+        if (lower) {
+            const int own = mine ? w : 0;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) alc[s] = right(s_al, s, own), rhc[s] = left(s_rh, s, own);
+        }
+        // a diagonal block's upper half, with the diagonal in A and B
+        auto cut = [&](f32x4& m) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int row = result ? 4 * g + i : c, colm = result ? c : 4 * g + i;
+                if (colm > row || (wave < 4 && colm == row)) m[i] = 0.f;
+            }
+        };
+        cut(acc[4]);
+        if (inner) cut(acc[1]);
+        else cut(acc[0]);
+        __syncthreads();  // al and rh are read
+        float* dst = wave < 4 ? (wave & 2 ? s_B : s_A) : (wave & 2 ? s_Q : s_P);
+#pragma unroll
+        for (int k = 0; k < 5; ++k) put_tile(dst + (k < n0 ? tri(r0, k) : tri(r1, k - n0)) + 4 * lane, acc[k]);
+    }
+    __syncthreads();
+    f32x4 Tc[4];  // column w of T
+    if (lower) {
+        const float* blk = s_A + tri(w, w);
+        float x[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            float r = i == c ? 1.f : 0.f;
+#pragma unroll
+            for (int j4 = 0; j4 < (i + 3) / 4; ++j4) {
+                const float4 a = ld4(blk + (j4 * 16 + i) * 4);
+                r -= a.x * x[4 * j4];
+                if (4 * j4 + 1 < i) r -= a.y * x[4 * j4 + 1];
+                if (4 * j4 + 2 < i) r -= a.z * x[4 * j4 + 2];
+                if (4 * j4 + 3 < i) r -= a.w * x[4 * j4 + 3];
+            }
+            x[i] = r;
+        }
+        f32x4 own;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) own[i] = g == 0 ? x[i] : g == 1 ? x[4 + i] : g == 2 ? x[8 + i] : x[12 + i];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) Tc[r] = r == w ? own : zero4();
+        transposed(s_A + tri(w, w), own);
+    }
+    __syncthreads();
+    if (lower)
+#pragma unroll
+        for (int r = 1; r < 4; ++r)
+            if (r > w) {
+                f32x4 m = zero4();
+#pragma unroll
+                for (int k = 0; k < r; ++k)
+                    if (k >= w) m = mma4(tile(s_A + tri(r, k)), as_float4(Tc[k]), m);
+                Tc[r] = -mma4(tile(s_A + tri(r, r)), as_float4(m), zero4());
+            }
+    __syncthreads();  // A is read
+    if (lower)
+#pragma unroll
+        for (int r = 1; r < 4; ++r)
+            if (r > w) transposed(s_A + tri(r, w), Tc[r]);
+    __syncthreads();
+    f32x4 W[4];  // - T al, channels 16 w ..
+    if (!lower) {
+        const int b = 3 - w;  // the longer columns to the SIMDs that had T's shorter ones
+        f32x4 X[4];           // column b of - T B
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (k >= b) {
+                const float4 x = tile(s_B + tri(k, b));
+                X[k] = f32x4{x.x, x.y, x.z, x.w};
+            }
+#pragma unroll
+        for (int r = 3; r >= 0; --r)  // upwards: row r of the product needs rows up to r of B
+            if (r >= b) {
+                f32x4 m = zero4();
+#pragma unroll
+                for (int k = 0; k <= r; ++k)
+                    if (k >= b) m = mma4(tile(s_A + tri(r, k)), as_float4(X[k]), m);
+                X[r] = -m;
+                put_tile(s_B + tri(r, b) + 4 * lane, X[r]);
+            }
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (r >= b) {
+                f32x4 m = zero4();
+#pragma unroll
+                for (int k = 0; k <= r; ++k)
+                    if (k >= b) m = mma4(tile(s_P + tri(r, k)), as_float4(X[k]), m);
+                const float4 q = tile(s_Q + tri(r, b));
+                transposed(s_Q + tri(r, b), f32x4{q.x, q.y, q.z, q.w} + m);
+            }
+    } else if (mine) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            f32x4 m = zero4();
+#pragma unroll
+            for (int s = 0; s <= r; ++s) m = mma4(tile(s_A + tri(r, s)), alc[s], m);
+            W[r] = -m;
+        }
+        float* dst = co.R + rec * kC * D16 + 4 * lane;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            f32x4 m = zero4();
+#pragma unroll
+            for (int s = 0; s <= r; ++s) m = mma4(as_float4(W[s]), tile(s_P + tri(r, s)), m);
+            put_tile(dst + (r * nt + w) * 256, f32x4{rhc[r].x, rhc[r].y, rhc[r].z, rhc[r].w} + m);
+        }
+    }
+    __syncthreads();  // A and P are read: V, tiles [value / 16][token / 16]
+#pragma unroll
+    for (int q = 0; q < TW / 4; ++q)
+        st4(s_V + (g * 4 + (wave >> 1)) * 256 + (((wave & 1) * 2 + q) * 16 + c) * 4,
+            make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]));
+    __syncthreads();
+    if (!mine) return;
+    if (lower) {
+        float* dst = co.M + rec * D16 * D16 + 4 * lane;
+        for (int t = 0; t < nt; ++t) {
+            f32x4 m = zero4();
+#pragma unroll
+            for (int s = 0; s < 4; ++s) m = mma4(as_float4(W[s]), right(s_be, s, t), m);
+            const float eg = s_eg[16 * t + c];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) m[i] = eg * ((t == w && c == 4 * g + i ? 1.f : 0.f) + m[i]);
+            put_tile(dst + (t * nt + w) * 256, m);
+        }
+        float4 V[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) V[s] = tile(s_V + (w * 4 + s) * 256);
+        dst = co.O + rec * kC * D16 + 4 * lane;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            f32x4 m = zero4();
+#pragma unroll
+            for (int s = 0; s <= r; ++s) m = mma4(tile(s_Q + tri(r, s)), V[s], m);
+            put_tile(dst + (r * nt + w) * 256, m);
+        }
+    } else {
+        f32x4 K[4];  // ka - X^T be, channels 16 w ..
+        float4 be[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) be[s] = right(s_be, s, w);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            f32x4 m = zero4();
+#pragma unroll
+            for (int r = s; r < 4; ++r) m = mma4(tile(s_B + tri(r, s)), be[r], m);
+            const float4 ka = right(s_ka, s, w);
+            K[s] = f32x4{ka.x, ka.y, ka.z, ka.w} + m;
+        }
+        const float4 eg = ld4(s_eg + 16 * w + 4 * g);
+        float* dst = co.N + rec * D16 * D16 + 4 * lane;
+        for (int t = 0; t < nt; ++t) {
+            f32x4 m = zero4();
+#pragma unroll
+            for (int s = 0; s < 4; ++s) m = mma4(as_float4(K[s]), tile(s_V + (t * 4 + s) * 256), m);
+            put_tile(dst + (t * nt + w) * 256, f32x4{eg.x * m[0], eg.y * m[1], eg.z * m[2], eg.w * m[3]});
+        }
+    }
+}
+
 constexpr int kNW = 8;  // waves
 
-// One workgroup per (chunk, head). Channels come in slabs of 64: al, be, ka and rh of a slab are formed in LDS (token by
+// dim > 64: one workgroup per (chunk, head). Channels come in slabs of 64: al, be, ka and rh of a slab are formed in LDS (token by
 // channel), and the four 64 x 64 products sum over slabs. The triangular system is solved in 16 x 16 blocks: a wave
 // inverts a diagonal block by substitution, the blocks of T = (I + A)^-1 below follow diagonal by diagonal and are kept
 // in the unused blocks above A's diagonal (block (r, b) at (b, r)). Then every wave takes 16 columns of W or of V: a
@@ -420,13 +777,10 @@ __global__ __launch_bounds__(kNW * kWave) void gdelta_chunk_kernel(Dims d, In<T>
 #pragma unroll
             for (int r = 0; r < 4; ++r) bv[r] = lower(s_B, r, V[q], zero4());
             times_t(bv, U[q]);
-            float* dst = co.O + rec * kC * D16 + cc;
+            float* dst = co.O + rec * kC * D16 + 4 * lane;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const f32x4 a = lower(s_Q, r, V[q], zero4()), b = lower(s_P, r, U[q], zero4());
-#pragma unroll
-                for (int i = 0; i < 4; ++i) dst[(int64_t)(16 * r + 4 * g + i) * D16] = a[i] - b[i];
-            }
+            for (int r = 0; r < 4; ++r)
+                put_tile(dst + (r * nt + vt[q]) * 256, lower(s_Q, r, V[q], zero4()) - lower(s_P, r, U[q], zero4()));
         }
     }
     const bool again = D16 > kC;
@@ -445,15 +799,14 @@ __global__ __launch_bounds__(kNW * kWave) void gdelta_chunk_kernel(Dims d, In<T>
 #pragma unroll
                 for (int j = 0; j < 4; ++j) x[s][j] = s_al[(16 * s + 4 * g + j) * LD + col];
             times_t(x, W[q]);
-            float* dst = co.R + rec * kC * D16 + d0 + col;
+            float* dst = co.R + rec * kC * D16 + 4 * lane;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const f32x4 pw = lower(s_P, r, W[q], zero4());
+            for (int r = 0; r < 4; ++r) {  // transposed
+                f32x4 pw = zero4();
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int t = 16 * r + 4 * g + i;
-                    dst[(int64_t)t * D16] = s_rh[t * LD + col] - pw[i];
-                }
+                for (int s = 0; s <= r; ++s) pw = mma4(as_float4(W[q][s]), ld4(&s_P[(16 * r + c) * LD + 16 * s + 4 * g]), pw);
+                const float4 rh = ld4(&s_rh[(16 * r + c) * LD + 16 * wt[q] - d0 + 4 * g]);
+                put_tile(dst + (r * nt + wt[q]) * 256, f32x4{rh.x, rh.y, rh.z, rh.w} - pw);
             }
         }
     }
@@ -465,37 +818,35 @@ __global__ __launch_bounds__(kNW * kWave) void gdelta_chunk_kernel(Dims d, In<T>
         const int nb = min(kC, D16 - d0) / 16;
         for (int rb = 0; rb < nb; ++rb) {  // rows d0 + 16 rb .. of M and N
             // transposed left operands: channel 16 rb + c of tokens 16 s + 4 g ..
-            float4 bt[4], kt[4];
+            float4 bt[4], kat[4];
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
                 const int at = (16 * s + 4 * g) * LD + 16 * rb + c;
                 bt[s] = make_float4(s_be[at], s_be[at + LD], s_be[at + 2 * LD], s_be[at + 3 * LD]);
-                kt[s] = make_float4(s_ka[at], s_ka[at + LD], s_ka[at + 2 * LD], s_ka[at + 3 * LD]);
+                kat[s] = make_float4(s_ka[at], s_ka[at + LD], s_ka[at + 2 * LD], s_ka[at + 3 * LD]);
             }
             const float4 eg = make_float4(s_eg[16 * rb + 4 * g], s_eg[16 * rb + 4 * g + 1], s_eg[16 * rb + 4 * g + 2],
                                           s_eg[16 * rb + 4 * g + 3]);
-            const int dr = d0 + 16 * rb + 4 * g;
+            const float egc = s_eg[16 * rb + c];
+            const int kt = d0 / 16 + rb;
 #pragma unroll
             for (int q = 0; q < TPW; ++q) {
                 if (wt[q] < nt) {
                     f32x4 m = zero4();
 #pragma unroll
-                    for (int s = 0; s < 4; ++s) m = mma4(bt[s], as_float4(W[q][s]), m);
-                    const int cc = 16 * wt[q] + c;
-                    float* dst = co.M + (rec * D16 + dr) * D16 + cc;
-                    dst[0] = eg.x * ((cc == dr ? 1.f : 0.f) - m[0]);
-                    dst[D16] = eg.y * ((cc == dr + 1 ? 1.f : 0.f) - m[1]);
-                    dst[2 * D16] = eg.z * ((cc == dr + 2 ? 1.f : 0.f) - m[2]);
-                    dst[3 * D16] = eg.w * ((cc == dr + 3 ? 1.f : 0.f) - m[3]);
+                    for (int s = 0; s < 4; ++s) m = mma4(as_float4(W[q][s]), bt[s], m);  // transposed
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) m[i] = egc * ((kt == wt[q] && c == 4 * g + i ? 1.f : 0.f) - m[i]);
+                    put_tile(co.M + rec * D16 * D16 + (kt * nt + wt[q]) * 256 + 4 * lane, m);
                 }
                 if (vt[q] < nt) {
                     f32x4 a = zero4(), b = a;
 #pragma unroll
                     for (int s = 0; s < 4; ++s) {
-                        a = mma4(kt[s], as_float4(V[q][s]), a);
+                        a = mma4(kat[s], as_float4(V[q][s]), a);
                         b = mma4(bt[s], as_float4(U[q][s]), b);
                     }
-                    st4(co.N + (rec * D16 + 16 * vt[q] + c) * D16 + dr,
+                    st4(co.N + rec * D16 * D16 + (vt[q] * nt + kt) * 256 + 4 * lane,
                         make_float4(eg.x * (a[0] - b[0]), eg.y * (a[1] - b[1]), eg.z * (a[2] - b[2]), eg.w * (a[3] - b[3])));
                 }
             }
@@ -511,13 +862,13 @@ struct SeqRef {
 };
 
 // One workgroup per (sequence, head, 16 columns of S), four waves. NS: 16-wide steps of dim at most; DT 16-row tiles of
-// S per wave; PF chunks of M and N in flight. `first` holds every chunk's first state, transposed [value][key].
+// S per wave; PF chunks of M and N in flight. `first` holds every chunk's first state.
 template <int NS, int PF>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void gdelta_chain_kernel(
     Dims d, SeqRef sq, const int32_t* __restrict__ seq_chunks, int seq0, int nseq, const float* __restrict__ M,
     const float* __restrict__ N, float* __restrict__ state, float* __restrict__ first) {
-    constexpr int LS = NS * 16 + 4, DT = (NS + 3) / 4;
-    __shared__ __attribute__((aligned(16))) float s_s[2][16 * LS];  // S^T slice
+    constexpr int DT = (NS + 3) / 4;
+    __shared__ __attribute__((aligned(16))) float s_s[2][NS * 256];  // the slice's tiles
     const int D16 = d.d16(), VP = d.vpad(), nt = D16 / 16, ns = nt;
     // the slices of one (sequence, head) read the same M: consecutive on one XCD
     const int xcd = blockIdx.x % 8, slot = blockIdx.x / 8, grp = slot / nt * 8 + xcd;
@@ -544,9 +895,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
 #pragma unroll
         for (int k = 0; k < DT; ++k) {
             const int tile = min(wave + 4 * k, ns - 1);
-            nv[k] = ld4(N + at + (int64_t)vcol * D16 + 16 * tile + 4 * g);
+            nv[k] = ld4(N + at + (vt * nt + tile) * 256 + 4 * lane);
 #pragma unroll
-            for (int s = 0; s < NS; ++s) mm[k][s] = ld4(M + at + (int64_t)(16 * tile + c) * D16 + 16 * min(s, ns - 1) + 4 * g);
+            for (int s = 0; s < NS; ++s) mm[k][s] = ld4(M + at + (tile * nt + min(s, ns - 1)) * 256 + 4 * lane);
         }
     };
     if (c0 < c1)
@@ -558,20 +909,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
             const int ci = cb + p;
             if (ci >= c1) continue;
             float* buf = s_s[(ci - c0) & 1];
-            float* fp = first + (((int64_t)ci * d.H + h) * D16 + vcol) * D16;
+            float* fp = first + ((int64_t)ci * d.H + h) * D16 * D16 + vt * nt * 256;
 #pragma unroll
             for (int k = 0; k < DT; ++k) {
                 const int tile = wave + 4 * k;
                 if (tile < ns) {
-                    *reinterpret_cast<f32x4*>(&buf[c * LS + 16 * tile + 4 * g]) = S[k];
-                    *reinterpret_cast<f32x4*>(fp + 16 * tile + 4 * g) = S[k];
+                    put_tile(buf + tile * 256 + 4 * lane, S[k]);
+                    put_tile(fp + tile * 256 + 4 * lane, S[k]);
                 }
             }
             __syncthreads();  // the other half is still read by waves that lag: it is written after the next barrier
             float4 b[NS];
 #pragma unroll
             for (int s = 0; s < NS; ++s)
-                if (s < ns) b[s] = ld4(&buf[c * LS + 16 * s + 4 * g]);
+                if (s < ns) b[s] = ld4(buf + s * 256 + 4 * lane);
 #pragma unroll
             for (int k = 0; k < DT; ++k) {
                 f32x4 lo = {nn[p][k].x, nn[p][k].y, nn[p][k].z, nn[p][k].w}, hi = zero4();
@@ -614,19 +965,20 @@ __global__ __launch_bounds__(256) void gdelta_out_kernel(Dims d, const int32_t* 
 #pragma unroll
     for (int v = 0; v < NS; ++v) {
         o[v] = zero4();
-        if (v < ns)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) o[v][i] = O0[(rec * kC + 16 * wave + 4 * g + i) * D16 + 16 * v + c];
+        if (v < ns) {
+            const float4 x = ld4(O0 + rec * kC * D16 + (wave * ns + v) * 256 + 4 * lane);
+            o[v] = f32x4{x.x, x.y, x.z, x.w};
+        }
     }
-    const float* rp = R + (rec * kC + 16 * wave + c) * D16 + 4 * g;
-    const float* sp = first + (rec * D16 + c) * D16 + 4 * g;
+    const float* rp = R + rec * kC * D16 + wave * ns * 256 + 4 * lane;
+    const float* sp = first + rec * D16 * D16 + 4 * lane;
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
         if (s >= ns) continue;
-        const float4 r = ld4(rp + 16 * s);
+        const float4 r = ld4(rp + s * 256);
 #pragma unroll
         for (int v = 0; v < NS; ++v)
-            if (v < ns) o[v] = mma4(r, ld4(sp + (int64_t)16 * v * D16 + 16 * s), o[v]);
+            if (v < ns) o[v] = mma4(r, ld4(sp + (v * ns + s) * 256), o[v]);
     }
     float ss[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -717,7 +1069,10 @@ extern "C" int skyrl_gdelta_chunk(const skyrl_gdelta_shape* shape, const void* p
     SKYRL_DISPATCH_T(dtype, {
         const In<T> in{reinterpret_cast<const T*>(proj), proj_stride, reinterpret_cast<const T*>(wl), wl_stride, w0, a_bias};
         const ChunkOut co{M, N, R, O};
-        if (d.D <= 128)
+        if (d.D <= kC)  // one slab of channels
+            hipLaunchKernelGGL((gdelta_chunk64_kernel<T>), dim3(nchunks * d.H), dim3(512), 0, as_stream(stream), d, in,
+                               chunk, co);
+        else if (d.D <= 128)
             hipLaunchKernelGGL((gdelta_chunk_kernel<T, 1>), dim3(nchunks * d.H), dim3(kNW * kWave), 0, as_stream(stream), d,
                                in, chunk, co);
         else

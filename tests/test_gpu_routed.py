@@ -246,6 +246,26 @@ def test_general_delta_fast_decay_and_strong_removal(dim):
     r.check(r.run([(61, 150)]))
 
 
+@pytest.mark.parametrize("heads,dim", [(2, 64), (1, 48), (3, 17), (1, 65)])
+def test_general_delta_gates_out_of_range(heads, dim):
+    """Gate logits far past where the exponentials saturate, up to infinity, through whole and ragged chunks; a NaN among
+    them shows in its own head's channels and in no other sequence."""
+    r = Rule(heads, dim, torch.float32, seed=dim, lens=(64, 147))
+    HD = heads * dim
+    for p, wl in zip(r.proj, r.wl):
+        wl[::3, ::2] = 200.0
+        wl[1::3, 1::2] = -200.0
+        p[::4, 4 * HD:5 * HD:3] = 95.0
+        p[1::4, 4 * HD + 1:5 * HD:3] = -300.0
+        p[2::4, 4 * HD:5 * HD:5] = math.inf
+        wl[3::7, ::3] = -math.inf
+    r.check(r.run([(64, 147)]))
+    r.wl[1][100, 0] = math.nan
+    a, b = r.run([(64, 147)])
+    assert bool(a.isfinite().all()) and bool(b[:64].isfinite().all()) and bool(b[128:, 0].isnan().all())
+    assert bool(b[:, dim:].isfinite().all())
+
+
 def test_general_delta_long_and_far():
     """One loud write, heard 700 tokens later through chunks, short portions and single steps."""
     n, D = 760, 32
