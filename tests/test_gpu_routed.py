@@ -400,6 +400,29 @@ def test_streamed_products(width, ff, experts, top, n, tm):
     close(y, want.cpu(), BF16, bf16=8e-3)
 
 
+@pytest.mark.parametrize("width,ff,loads", [
+    (64, 128, (1, 300)), (256, 128, (0, 1, 63, 64, 65, 128, 129, 192, 193, 255, 256, 257, 0)), (512, 384, (700, 0, 31, 513)),
+    (320, 128, (90, 257)), (256, 192, (90, 257)), (1024, 1024, (0, 20001, 1000, 5, 3000, 2050))])
+def test_wide_tiles(width, ff, loads):
+    """Tiles of 256 at the edges of their sixty-fours, depths of one step, one and several items per workgroup; the general
+    form where the depth or the columns are no multiples (320, 192)."""
+    g = torch.Generator(device=DEV).manual_seed(width + ff)
+    n, E = sum(loads), len(loads)
+    sh = lk.moe_shape(width, ff, E, 1)
+    mk = lambda *s, scale=1.0: (torch.randn(s, generator=g, device=DEV) * scale).to(BF16)  # noqa: E731
+    x, wgu, wd = mk(n, width), mk(E, 2, ff, width, scale=width ** -0.5), mk(E, width, ff, scale=ff ** -0.5)
+    idx = torch.repeat_interleave(torch.arange(E, device=DEV), torch.tensor(loads, device=DEV))[torch.randperm(n, generator=g, device=DEV)]
+    weight = torch.rand(n, 1, generator=g, device=DEV) + 0.2
+    y = lk.moe_experts(sh, x, idx.int().view(n, 1), weight, wgu, wd, tm=256).view(n, width)
+    for e in (e for e in range(E) if loads[e]):
+        at = (idx == e).nonzero().flatten()
+        at = at[torch.cat([torch.arange(min(len(at), 300)), torch.arange(max(len(at) - 300, 0), len(at))])]
+        h = x[at].float()
+        a = ref.silu(h @ wgu[e, 0].float().t()) * (h @ wgu[e, 1].float().t())
+        close(y[at], (weight[at] * (a @ wd[e].float().t())).double().cpu(), BF16, bf16=8e-3)
+    assert torch.equal(y, lk.moe_experts(sh, x, idx.int().view(n, 1), weight, wgu, wd, tm=128).view(n, width))
+
+
 @pytest.mark.parametrize("width,ff,experts,top,n", [(2048, 768, 32, 8, 1500), (1024, 512, 64, 4, 300), (4096, 320, 8, 2, 90)])
 def test_tile_sizes_agree_bit_for_bit(width, ff, experts, top, n):
     """A row's sums are formed in the same order whatever its tile: products of a real layer's size, over and over."""
