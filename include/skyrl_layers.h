@@ -53,6 +53,10 @@ extern "C" {
  *                   or as f32 [splits, n, ldo] whose sum over the first index is the product, the bias in the first. act
  *                   of skyrl_gate_mul: w holds N gate rows, then N up rows; the gated product bf16 [n, N], splits 0.
  *                   skyrl_rows_product_fits: whether it takes the sizes; skyrl_rows_product_splits: the splits.
+ *   skyrl_gated_product  many rows: the gated product (act of skyrl_gate_mul) of x bf16 [n, K] (row stride ldx) and w bf16
+ *                   [N gate rows, N up rows] (row stride ldw), rows 16-byte aligned, as bf16 [n, N] contiguous: summed and
+ *                   gated in f32, rounded once. K a multiple of 64, N of 128. skyrl_gated_product_fits: whether it takes the
+ *                   sizes and is the faster form.
  *   skyrl_rows_batch  `batch` such products without bias, x, w and out bf16 x_batch, w_batch and out_batch apart.
  *   skyrl_add_norm_parts, skyrl_gate_norm_add_parts  of a model in bf16, the sublayer's output being such a sum of
  *                   `parts` (a_shares > 0) f32 [n, H], or (gate_shares > 0) the gate's logits being one of f32
@@ -79,6 +83,9 @@ int skyrl_gate_mul(const void* gate_up, int64_t gu_stride, int64_t n, int32_t I,
 int skyrl_gate_norm_add(const void* a, const int64_t* rows, int32_t parts, const void* gate, int64_t gate_stride,
                         const float* gate_bias, const void* weight, int32_t groups, float eps, float mult, float* hidden,
                         int32_t fresh, const void* next, int32_t n, int32_t H, void* out, int32_t dtype, void* stream);
+int32_t skyrl_gated_product_fits(int32_t n, int32_t K, int32_t N);
+int skyrl_gated_product(const void* x, int64_t ldx, int32_t n, int32_t K, const void* w, int64_t ldw, int32_t N, int32_t act,
+                        float alpha, float limit, void* out, void* stream);
 int32_t skyrl_rows_product_fits(int32_t n, int32_t K, int32_t N, int32_t gated);
 int32_t skyrl_rows_product_splits(int32_t n, int32_t K, int32_t N);
 int skyrl_rows_product(const void* x, int64_t ldx, int32_t n, int32_t K, const void* w, int64_t ldw, int32_t N,

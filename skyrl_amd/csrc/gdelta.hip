@@ -391,7 +391,6 @@ __global__ __launch_bounds__(512, 4) void gdelta_chunk64_kernel(Dims d, In<T> in
         auto blocks = [&](auto result_, auto inner_) {
 #pragma unroll
             for (int k = 0; k < 5; ++k) acc[k] = zero4();
-#pragma unroll 2
             for (int t = 0; t < nt; ++t) {
                 constexpr int R0 = inner_ ? 1 : 0, R1 = inner_ ? 2 : 3;
                 const float4 x[2] = {left(ls, R0, t), left(ls, R1, t)};

@@ -13,16 +13,14 @@
 // The products stage pieces of the rows and of the weight rows through LDS (16-byte direct loads, chunk index
 // xor-swizzled by the row so that the reads of 16 rows do not conflict), weights as the left operand: a lane holds
 // four consecutive columns of a token. Small tiles (decode) keep several stages in flight: they stream weights.
-#include <type_traits>
-
 #include "stream.h"
+#include "wide.h"
 
 namespace skyrl {
 namespace {
 
 constexpr int kNT = 256;
 constexpr int kMaxExperts = 1024;
-constexpr int kCUs = 256;  // a multiple of the 8 XCDs
 
 struct Router {
     int experts, top, groups, keep;
@@ -363,15 +361,6 @@ __global__ __launch_bounds__(kNT) void moe_plain_kernel(Product p, const T* __re
 }
 
 // ---- products, bf16, depth and columns multiples of 8 ------------------------------------------------
-// All but the N latest loads have landed, all LDS reads have returned.
-template <int N>
-__device__ __forceinline__ void wait_loads() {
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
-}
-__device__ __forceinline__ void lds_read(s16x8& v, uint32_t at, int offset) {
-    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(at), "n"(offset));
-}
-
 // A tile of 16 MT rows (a few pairs per expert, decode steps): 16 NT weight rows (GATED: half of each matrix) per workgroup, whose
 // waves stream a share of the depth each (stream.h). Bound: the experts' weights, each read once. Measured, 64 experts of 768 x
 // 2048, 8 per token, gate_up / down, us (TB/s of weights) against moe_gemm_kernel's, whose stages hold two workgroups a CU, in
@@ -413,240 +402,6 @@ __global__ __launch_bounds__(WK* kWave) void moe_stream_kernel(Product p, const 
             y = y * (p.weight ? p.weight[pair] : 1.f);
         }
         st4(out + (p.out_pairs ? (int64_t)pair : place0 + r) * p.N + col, make_float4(y[0], y[1], y[2], y[3]));
-    }
-}
-
-// a += w x on 16 x 16 x 32, in the accumulator's own registers (the compiler's form may take others and copy them back on
-// every turn of a loop). Before anything but a product reads them, the caller lets 16 cycles pass.
-__device__ __forceinline__ void product(f32x4& a, const s16x8& w, const s16x8& x) {
-    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(a) : "v"(w), "v"(x));
-}
-
-// Tiles of 256 (prompts): 256 weight rows per workgroup of four waves, 128 x 128 results and a SIMD each, 128 KB of LDS in two
-// stages of 64. A wave has nobody to hide behind, so its reads of the next operands and the loads of the next stage are
-// placed between the products, one every few, and are waited for a quarter of a step later. With 128 x 64 a wave (eight of
-// them) the operands' reads alone took as many LDS cycles as the products took matrix cycles.
-// A workgroup per CU goes through its XCD's run of (tile, columns): the next one's first two stages are loaded while the
-// results leave, 16 rows at a time through a piece of LDS of the wave's own.
-// A tile's rows are spread over the two rows of waves by sixteens, and products past its last 64 used rows are left out: with
-// 700 pairs per expert the padding is a sixth of the rows. The depth is a multiple of 64, the columns of the tile's. GATED: x has
-// a row per token, the output one per place; else x one per place, the output one per pair.
-// Bound: the products (2048 cycles of a step's 2800, the rest waits for the direct loads, 64 bytes a cycle and CU, or for a
-// stage) and, down, the rows that leave. Measured, 64 experts of 768 x 2048, 8 per token, gate_up / down, us (before: eight
-// waves, a workgroup per tile and columns): 2048 tokens 161 / 95 (182 / 96), 5637 tokens 268 / 181 (300 / 184), 8192 tokens
-// 380 / 277 (439 / 276).
-template <bool GATED>
-__global__ __launch_bounds__(256) void moe_wide_kernel(Product p, const uint16_t* __restrict__ x,
-                                                       const uint16_t* __restrict__ w, uint16_t* __restrict__ out,
-                                                       int ncols, int ntiles) {
-    constexpr int TM = 256, TN = 256, BK = 64, NT = 8, L = 8;  // results: NT 16-wide tiles of columns a wave; L pieces each
-    constexpr int kStage = (TM + TN) * BK;                     // elements
-    constexpr int OC = GATED ? TN / 2 : TN, WC = OC / 2;       // output columns, a wave's
-    constexpr int LR = WC / 8, SI = LR / 4, LO = WC + 8;       // lanes per row as it leaves, stores of 16 rows, row in LDS
-    constexpr int F3 = 8, F0 = 8;  // a piece's loads in the groups of products from its stage's release on
-    __shared__ __attribute__((aligned(16))) uint16_t smem[2 * kStage], s_out[4][16 * LO];
-    __shared__ int s_row[2][TM], s_rows[2][4];  // of the output, or -1; the last in use
-    __shared__ float s_wt[2][TM];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int c = lane & 15, g = lane >> 4, wm = wave >> 1, wn = wave & 1;
-    const int64_t items = (int64_t)p.tile_expert[ntiles] * ncols;
-    const int xcd = blockIdx.x % 8, stride = gridDim.x / 8;
-    const int end = (int)(items * (xcd + 1) / 8);
-    int item = (int)(items * xcd / 8) + blockIdx.x / 8;
-    if (item >= end) return;
-    const int nk = p.K / BK;
-
-    // the item after this one: its rows' pairs are read an item ahead
-    int next_e, next_pair, next_rows[L];
-    auto peek = [&](int it) {
-        const int tile = it / ncols;
-        const int32_t* order = p.order + (int64_t)tile * TM;
-        next_e = p.tile_expert[tile];
-        next_pair = order[tid];
-        if constexpr (GATED)
-#pragma unroll
-            for (int i = 0; i < L; ++i) next_rows[i] = order[(wave * L + i) * 8 + lane / 8];
-    };
-    // global sources of this lane's 16 bytes per piece: row 8 piece + lane / 8, chunk (lane % 8) ^ (row / 2 % 8), so that the
-    // 16 rows a matrix operand reads at a time lie in different banks. Weight rows follow each other, and so do places.
-    const int chunk[2] = {(lane % 8 ^ lane / 16) * 8, (lane % 8 ^ (lane / 16 + 4)) * 8};  // even, odd piece
-    const uint16_t *xs[GATED ? L : 2], *ws[2];
-    auto fetch = [&](int t, int i) {  // load i of piece t (the last again past the end) into stage t % 2
-        uint16_t* dst = smem + (t & 1) * kStage + (i < L ? 0 : TM * BK) + (wave * L + i % L) * 512;
-        const int64_t k0 = min(t, nk - 1) * BK, down = (int64_t)(i % L) * 8 * p.K;
-        const uint16_t* src = i >= L ? ws[i % 2] + (k0 + down) : GATED ? xs[i % L] + k0 : xs[i % 2] + (k0 + down);
-        __builtin_amdgcn_global_load_lds((gbl_void*)src, (lds_void*)dst, 16, 0, 0);
-    };
-    int n0, q = 0;
-    const float per_row = GATED ? 1.f / p.row_div : 0.f;
-    auto open = [&](int it) {  // start on the item that was peeked at
-        const int tile = it / ncols, r0 = wave * L * 8;
-        n0 = it % ncols * OC;
-        const uint16_t* we = w + (int64_t)max(next_e, 0) * (GATED ? 2 : 1) * p.N * p.K;
-        we += (int64_t)(GATED ? n0 + r0 % OC + r0 / OC * p.N : n0 + r0) * p.K + lane / 8 * p.K;
-        ws[0] = we + chunk[0], ws[1] = we + chunk[1];
-        if constexpr (GATED) {
-#pragma unroll
-            for (int i = 0; i < L; ++i) {
-                const int pair = max(next_rows[i], 0);  // places without a pair: row 0, not stored
-                const int d = (int)((float)pair * per_row), rest = pair - d * p.row_div;  // pair / row_div, one off at most
-                xs[i] = x + (int64_t)(d + (rest >= p.row_div) - (rest < 0)) * p.K + chunk[i % 2];
-            }
-        } else {
-            const uint16_t* xt = x + ((int64_t)tile * TM + r0 + lane / 8) * p.K;
-            xs[0] = xt + chunk[0], xs[1] = xt + chunk[1];
-        }
-#pragma unroll
-        for (int i = 0; i < 2 * L; ++i) fetch(0, i);
-#pragma unroll
-        for (int i = 0; i < F3; ++i) fetch(1, i);
-        s_row[q][tid] = GATED && next_pair >= 0 ? tile * TM + tid : next_pair;
-        if constexpr (!GATED) s_wt[q][tid] = p.weight && next_pair >= 0 ? p.weight[next_pair] : 1.f;
-        const uint64_t in = __ballot(next_pair >= 0);
-        if (lane == 0) s_rows[q][wave] = in ? 64 * wave + 64 - __builtin_clzll(in) : 0;
-    };
-    const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_void*)smem;
-    const uint32_t xat = lds0 + (wm * 16 + c) * BK * 2;
-    const uint32_t wat = lds0 + (TM + wn * (GATED ? NT / 2 : NT) * 16 + c) * BK * 2;
-    const uint32_t oat = (uint32_t)(uintptr_t)(lds_void*)s_out[wave];
-
-    // A step's products in four groups: half of the depth ks, half h of the 2 MH tiles of rows that are in use.
-    auto run = [&](auto mh_, bool more) {
-        constexpr int MH = mh_, M = MH * NT;
-        f32x4 acc[2 * MH][NT];
-#pragma unroll
-        for (int m = 0; m < 2 * MH; ++m)
-#pragma unroll
-            for (int n = 0; n < NT; ++n) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
-        s16x8 wf[2][NT], xf[2][MH];
-        // The operands' reads are not the compiler's: it would wait for every load into LDS under way before one. Their
-        // registers are tied past the wait that ends the group they are in.
-        auto chunk_at = [&](int t, int ks) { return (uint32_t)((t & 1) * kStage * 2) + ((ks * 4 + g) ^ (c / 2)) * 16; };
-        auto read_w = [&](int t, int ks, int n) {
-            lds_read(wf[ks][n], wat + chunk_at(t, ks), (n < NT / 2 || !GATED ? n * 16 : OC + (n - NT / 2) * 16) * BK * 2);
-        };
-        auto read_x = [&](int t, int ks, int h, int i) { lds_read(xf[h][i], xat + chunk_at(t, ks), (h * MH + i) * 32 * BK * 2); };
-        auto landed = [&]() {
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-            for (int ks = 0; ks < 2; ++ks) {
-#pragma unroll
-                for (int n = 0; n < NT; ++n) asm volatile("" : "+v"(wf[ks][n]));
-#pragma unroll
-                for (int i = 0; i < MH; ++i) asm volatile("" : "+v"(xf[ks][i]));
-            }
-        };
-        // the products of (ks, h) with `jobs` calls of job spread between them
-        auto group = [&](auto ks_, auto h_, auto jobs_, auto job) {
-            constexpr int ks = ks_, h = h_, J = jobs_;
-#pragma unroll
-            for (int i = 0; i < M; ++i) {
-                const int m = i / NT, n = i % NT;
-                product(acc[h * MH + m][n], wf[ks][n], xf[h][m]);
-#pragma unroll
-                for (int j = 0; j < J; ++j)
-                    if (j * M / J == i) job(j);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            landed();
-        };
-        using I0 = std::integral_constant<int, 0>;
-        using I1 = std::integral_constant<int, 1>;
-#pragma unroll
-        for (int n = 0; n < NT; ++n) read_w(0, 0, n), read_w(0, 1, n);
-#pragma unroll
-        for (int i = 0; i < MH; ++i) read_x(0, 0, 0, i), read_x(0, 0, 1, i);
-        landed();
-        for (int t = 0; t < nk; ++t) {
-            group(I0{}, I0{}, std::integral_constant<int, MH + F0>{}, [&](int j) {
-                if (j < MH) read_x(t, 0, 1, j);
-                else fetch(t + 1, F3 + j - MH);
-            });
-            group(I0{}, I1{}, std::integral_constant<int, NT + MH>{}, [&](int j) {
-                if (j < NT) read_w(t, 1, j);
-                else read_x(t, 1, 0, j - NT);
-            });
-            group(I1{}, I0{}, std::integral_constant<int, MH>{}, [&](int j) { read_x(t, 1, 1, j); });
-            wait_loads<0>();               // this wave's loads of piece t + 1 have landed, its reads of piece t too
-            __builtin_amdgcn_s_barrier();  // and everyone's
-            asm volatile("" ::: "memory");
-            group(I1{}, I1{}, std::integral_constant<int, NT + MH + F3>{}, [&](int j) {
-                if (j < NT) read_w(t + 1, 0, j);
-                else if (j < NT + MH) read_x(t + 1, 0, 0, j - NT);
-                else fetch(t + 2, j - NT - MH);
-            });
-        }
-        wait_loads<0>();
-        asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last products are in their registers
-        __syncthreads();
-        const int o = q;
-        uint16_t* to = out + n0 + wn * WC + lane % LR * 8;
-        float scale[2 * MH];
-        if constexpr (!GATED)
-#pragma unroll
-            for (int m = 0; m < 2 * MH; ++m) scale[m] = s_wt[o][(2 * m + wm) * 16 + c];
-        if (more) {
-            q ^= 1;
-            open(item + stride);
-        }
-        uint4 v[2][SI];
-        auto gather = [&](int m, uint4 (&y)[SI]) {
-#pragma unroll
-            for (int n = 0; n < NT; ++n) asm volatile("" : "+a"(acc[m][n]));  // in the accumulators' registers until here
-#pragma unroll
-            for (int n = 0; n < (GATED ? NT / 2 : NT); ++n) {
-                float z[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    if constexpr (GATED) z[i] = acc[m][n][i] * sigmoid_<uint16_t>(acc[m][n][i]) * acc[m][n + NT / 2][i];
-                    else z[i] = acc[m][n][i] * scale[m];
-                }
-                *reinterpret_cast<uint2*>(&s_out[wave][c * LO + n * 16 + 4 * g]) =
-                    make_uint2(pack_bf16x2(z[0], z[1]), pack_bf16x2(z[2], z[3]));
-            }
-            asm volatile("" ::: "memory");
-            s16x8 b[SI];
-#pragma unroll
-            for (int k = 0; k < SI; ++k) lds_read(b[k], oat + (lane / LR * LO + lane % LR * 8) * 2, k * (64 / LR) * LO * 2);
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-            for (int k = 0; k < SI; ++k) {
-                asm volatile("" : "+v"(b[k]));
-                y[k] = *reinterpret_cast<const uint4*>(&b[k]);
-            }
-        };
-        auto leave = [&](int m, const uint4 (&y)[SI]) {
-            int row[SI];
-#pragma unroll
-            for (int k = 0; k < SI; ++k) row[k] = s_row[o][(2 * m + wm) * 16 + k * (64 / LR) + lane / LR];
-#pragma unroll
-            for (int k = 0; k < SI; ++k)
-                if (row[k] >= 0) *reinterpret_cast<uint4*>(to + (int64_t)row[k] * p.N) = y[k];
-        };
-        gather(0, v[0]);
-        gather(1, v[1]);
-        wait_loads<0>();  // the next item's first stages, before stores are under way too
-        leave(0, v[0]);
-        leave(1, v[1]);
-#pragma unroll
-        for (int m = 2; m < 2 * MH; ++m) {
-            gather(m, v[m & 1]);
-            leave(m, v[m & 1]);
-        }
-    };
-    peek(item);
-    open(item);
-    wait_loads<0>();
-    for (; item < end; item += stride) {
-        __syncthreads();
-        const int* sr = s_rows[q];
-        const int rows = max(max(sr[0], sr[1]), max(sr[2], sr[3]));
-        const bool more = item + stride < end;
-        if (more) peek(item + stride);
-        if (rows > 192) run(std::integral_constant<int, 4>{}, more);
-        else if (rows > 128) run(std::integral_constant<int, 3>{}, more);
-        else if (rows > 64) run(std::integral_constant<int, 2>{}, more);
-        else run(std::integral_constant<int, 1>{}, more);
     }
 }
 
@@ -838,15 +593,6 @@ int launch_product(const Product& p, const void* x, const void* w, void* out, in
         hipLaunchKernelGGL((moe_gemm_kernel<TM, TN, WM, WN, S, GATED>), dim3((unsigned)(TM > 16 ? grid : (int64_t)ncols * ntiles)), \
                            dim3(WM * WN * kWave), 0, s, p, x_, w_, o_, ncols, ntiles);                                \
     } while (0)
-#define LAUNCH_WIDE()                                                                                                 \
-    do {                                                                                                              \
-        constexpr int kCols = GATED ? 128 : 256;                                                                      \
-        const int ncols = p.N / kCols;                                                                                \
-        const int64_t items = (int64_t)ncols * ntiles;                                                                \
-        SKYRL_REQUIRE(items < (1ll << 31), "moe: grid too large");                                                    \
-        hipLaunchKernelGGL((moe_wide_kernel<GATED>), dim3((unsigned)(items > 3 * kCUs ? kCUs : (items + 7) / 8 * 8)), \
-                           dim3(256), 0, s, p, x_, w_, o_, ncols, ntiles);                                            \
-    } while (0)
 #define LAUNCH_STREAM(NT, MT, WK, S)                                                                                  \
     do {                                                                                                              \
         constexpr int kCols = GATED ? 8 * NT : 16 * NT;                                                               \
@@ -855,16 +601,15 @@ int launch_product(const Product& p, const void* x, const void* w, void* out, in
         hipLaunchKernelGGL((moe_stream_kernel<NT, MT, WK, S, GATED>), dim3((unsigned)(ncols * ntiles)), dim3(WK * kWave), 0, s, \
                            p, x_, w_, o_, (int)ncols);                                                                \
     } while (0)
-        // Of tiles of 256 an item each for up to three rounds of workgroups, which then go to the CUs as these get free; with
-        // more, a workgroup per CU (gate_up as above, 2048 tokens: 161 us against 171; 8192: 395 against 380).
         // Streamed where an expert has about one tile, so that its weights are read once: tiles of 16 below 16 pairs per
         // expert (ntiles is npairs / tm + experts), of 32, and, for the wider of the two products, of 64 from 24 pairs on. Tiles
         // of 16 and 64 that are asked for at other loads sum a row in the order that larger ones do.
         const bool once = ntiles <= 2 * experts;
-        if (p.tm == 256) {
-            if (p.K % 64 == 0 && p.N % (GATED ? 128 : 256) == 0) LAUNCH_WIDE();
-            else LAUNCH_GEMM(256, 256, 2, 4, 2);
+        if (p.tm == 256 && wide_fits(p.K, p.N, GATED)) {
+            return launch_wide<GATED ? kGateUp : kDown>(Wide{x_, w_, o_, p.K, p.N, p.K, p.K, ntiles, p.order, p.tile_expert,
+                                                             p.row_div, p.weight, 0, Gate{}}, s);
         }
+        if (p.tm == 256) LAUNCH_GEMM(256, 256, 2, 4, 2);
         else if (p.tm == 128) LAUNCH_GEMM(128, 128, 2, 2, 2);
         else if (p.tm == 64) {
             if (GATED && once && (int64_t)(ntiles - experts) * 64 >= 24ll * experts) LAUNCH_STREAM(4, 4, 2, 2);

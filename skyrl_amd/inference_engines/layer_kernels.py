@@ -73,8 +73,12 @@ def _rows_fit(x: torch.Tensor, w: torch.Tensor, gated: bool = False) -> bool:
         return False
     N = w.shape[0] // 2 if gated else w.shape[0]
     return (x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.is_cuda
-            and bool(_ffi.query("skyrl_rows_product_fits", n, K, N, int(gated)))
-            and x.stride(1) == 1 and w.stride(1) == 1 and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0
+            and bool(_ffi.query("skyrl_rows_product_fits", n, K, N, int(gated))) and _rows_aligned(x, w))
+
+
+def _rows_aligned(x: torch.Tensor, w: torch.Tensor) -> bool:
+    n, K = x.shape
+    return (x.stride(1) == 1 and w.stride(1) == 1 and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0
             and (n == 1 or x.stride(0) >= K) and w.stride(0) >= K and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
@@ -124,14 +128,20 @@ def joined(y: torch.Tensor) -> torch.Tensor:
 
 
 def gated_linear(x: torch.Tensor, w: torch.Tensor, act: str, alpha: float = 1.0, limit: float = 0.0) -> Optional[torch.Tensor]:
-    """gate_mul of x w^T, w the gate rows and then the up rows, in one launch for few bf16 rows; None otherwise."""
-    if w.shape[0] % 2 or not _rows_fit(x, w, True):
+    """gate_mul of x w^T, w the gate rows and then the up rows, in one launch for few or many bf16 rows; None otherwise."""
+    (n, K), N = x.shape, w.shape[0] // 2
+    many = (n > MAX_ROWS and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.is_cuda
+            and bool(_ffi.query("skyrl_gated_product_fits", n, K, N)) and _rows_aligned(x, w))
+    if w.shape[0] % 2 or not (many or _rows_fit(x, w, True)):
         return None
     dev = _require_gpu(x, w)
-    (n, K), N = x.shape, w.shape[0] // 2
     if w.shape[1] != K:
         raise ValueError(f"w must be [2 N, {K}], got {tuple(w.shape)}")
     out = torch.empty((n, N), dtype=torch.bfloat16, device=dev)
+    if many:
+        _ffi.call("skyrl_gated_product", _ptr(x), x.stride(0), n, K, _ptr(w), w.stride(0), N, ACTIVATIONS[act], float(alpha),
+                  float(limit), _ptr(out), _stream(dev))
+        return out
     _ffi.call("skyrl_rows_product", _ptr(x), x.stride(0), n, K, _ptr(w), w.stride(0), N, None, ACTIVATIONS[act], float(alpha),
               float(limit), 0, _ptr(out), N, _stream(dev))
     return out

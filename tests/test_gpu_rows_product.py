@@ -1,5 +1,6 @@
 """Products of few rows (csrc/rows_product.hip) against f64: every kernel form at the edges of its tiles, remainders of the
-depth and of the columns, strided rows, biases, f32 parts and the norms that read them, gated products."""
+depth and of the columns, strided rows, biases, f32 parts and the norms that read them, gated products, also of many rows
+(csrc/gated_product.hip)."""
 
 import pytest
 import torch
@@ -46,7 +47,7 @@ def test_products(dev, n, N, K, pad):
 
 @pytest.mark.parametrize("act", ("silu", "gelu_tanh", "clamped"))
 @pytest.mark.parametrize("n,N,K", [(1, 100, 264), (2, 8, 64), (16, 4100, 136), (17, 36, 200), (32, 72, 1032), (33, 132, 520),
-                                   (64, 6144, 72)])
+                                   (64, 6144, 72), (513, 12288, 64), (1030, 6144, 192), (8200, 896, 128), (5000, 5120, 64)])
 def test_gated(dev, n, N, K, act):
     x, w, _ = _data(dev, n, 2 * N, K, 5 * n)
     y = lk.gated_linear(x, w, act, 1.702, 7.0)
@@ -73,6 +74,8 @@ def test_what_the_library_takes(dev):
     assert not lk._rows_fit(big[:, :64], w)                        # and row strides
     assert not lk._rows_fit(x[:4].float(), w.float())
     assert lk.gated_linear(x[:65], w, "silu") is None
+    for n, N, K in ((511, 12288, 64), (1024, 5888, 64), (1024, 6208, 64), (1024, 6144, 72)):  # few rows, few items, remainders
+        assert lk.gated_linear(*_data(dev, n, 2 * N, K, 0)[:2], "silu") is None
     for a, b in ((big[:, 1:65], w), (x, w), (x[:4].float(), w.float())):
         torch.testing.assert_close(lk.linear(a, b, parts=True), torch.nn.functional.linear(a, b))
     with pytest.raises(ValueError):
