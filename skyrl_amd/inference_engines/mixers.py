@@ -34,7 +34,9 @@ BLOCK_SIZE = kernels.BLOCK_SIZE
 # From this many tokens on a portion takes the prompt forms (keys expanded once per key, chunked
 # recurrence) instead of one query row or one recurrence step per token.
 PROMPT_MIN = 32
-ATTEND_WORKGROUPS = 256  # of the decode attention: one per CU (more split finer than they overlap)
+# Of the decode attention, at most: one per CU. One more round costs more than the shares save (context 1024, us with the merge:
+# 48 rows in 4 shares 27, in 6 43; 96 in 2 37, in 3 55).
+ATTEND_WORKGROUPS = 256
 PREFILL_TILE = 128  # queries per workgroup of the prompt attention
 
 
@@ -373,7 +375,8 @@ class LatentAttention:
     # ---- decode split
     def nparts(self, tokens: int, max_ctx: int) -> int:
         ctx = min(max_ctx, self.window + BLOCK_SIZE) if self.window else max_ctx
-        return kernels.choose_nparts(tokens, (self.heads + 31) // 32, ctx, target_waves=ATTEND_WORKGROUPS)
+        groups = tokens * ((self.heads + 31) // 32)
+        return kernels.choose_nparts(1, 1, ctx, target_waves=max(1, ATTEND_WORKGROUPS // max(1, groups)))
 
     def workspace_bytes(self, tokens: int, max_ctx: int) -> int:
         from .. import _ffi
