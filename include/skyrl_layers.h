@@ -52,7 +52,8 @@ extern "C" {
  *                   16-byte aligned. act < 0: y + bias bf16 [N] (may be NULL), as bf16 [n, N] (splits 0, row stride ldo),
  *                   or as f32 [splits, n, ldo] whose sum over the first index is the product, the bias in the first. act
  *                   of skyrl_gate_mul: w holds N gate rows, then N up rows; the gated product bf16 [n, N], splits 0.
- *                   skyrl_rows_product_fits: whether it takes the sizes; skyrl_rows_product_splits: the splits.
+ *                   skyrl_rows_product_fits: whether it takes the sizes and is the faster form of them (form 0:
+ *                   rounded, 1: gated, 2: in splits); skyrl_rows_product_splits: the splits.
  *   skyrl_gated_product  many rows: the gated product (act of skyrl_gate_mul) of x bf16 [n, K] (row stride ldx) and w bf16
  *                   [N gate rows, N up rows] (row stride ldw), rows 16-byte aligned, as bf16 [n, N] contiguous: summed and
  *                   gated in f32, rounded once. K a multiple of 64, N of 128. skyrl_gated_product_fits: whether it takes the
@@ -86,7 +87,7 @@ int skyrl_gate_norm_add(const void* a, const int64_t* rows, int32_t parts, const
 int32_t skyrl_gated_product_fits(int32_t n, int32_t K, int32_t N);
 int skyrl_gated_product(const void* x, int64_t ldx, int32_t n, int32_t K, const void* w, int64_t ldw, int32_t N, int32_t act,
                         float alpha, float limit, void* out, void* stream);
-int32_t skyrl_rows_product_fits(int32_t n, int32_t K, int32_t N, int32_t gated);
+int32_t skyrl_rows_product_fits(int32_t n, int32_t K, int32_t N, int32_t form);
 int32_t skyrl_rows_product_splits(int32_t n, int32_t K, int32_t N);
 int skyrl_rows_product(const void* x, int64_t ldx, int32_t n, int32_t K, const void* w, int64_t ldw, int32_t N,
                        const void* bias, int32_t act, float alpha, float limit, int32_t splits, void* out, int64_t ldo,

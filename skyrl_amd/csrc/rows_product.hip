@@ -135,10 +135,31 @@ constexpr int kWide = 8192;       // output columns from which wider tiles still
 constexpr int kFill = 256;        // workgroups that a split product is cut into
 constexpr int kManyRowsCols = 4096;
 
-bool rows_fit(int n, int K, int N, bool gated) {
-    // Above 64 rows the library's tiles are as fast on wide matrices (128 rows, 12288 x 2048: 21.0 against 20.7 us) and
-    // slower on narrow ones (2048 x 2048: 6.9 against 11.5 us, 2048 x 6144: 13.6 against 18.2 us, in parts).
-    return n > 0 && K > 0 && N > 0 && K % 8 == 0 && (n <= 64 || (n <= 128 && N <= kManyRowsCols && !gated));
+enum Form { kFormRound, kFormGated, kFormParts };
+
+// What the kernels compute.
+bool rows_take(int n, int K, int N, int form) {
+    return n > 0 && K > 0 && N > 0 && K % 8 == 0 && (n <= 64 || (n <= 128 && N <= kManyRowsCols && form == kFormParts));
+}
+
+// Where they are the faster form; us, here / the library's. Above 64 rows its tiles are as fast on wide matrices (128 rows, 12288
+// x 2048: 21.0 / 20.7) and slower on narrow ones only against parts (2048 x 2048 6.9 / 11.5, 2048 x 6144 14.2 / 17.8; rounded
+// 29.3). Depths above 2048 give them more to pipeline:
+//   up to 16 rows  until a matrix is both deep and large: 4096 x 4096 10.2 / 15.9, 30720 x 4096 44.7 / 59.8, 2048 x 6144 in parts
+//                  8.2 / 12.2, but 4096 x 8192 16.8 / 16.4, and one row of 2048 x 8192 14.6 / 13.6, of 4096 x 12288 24.5 / 21.7.
+//   more rows      in parts, up to 8192 columns (32 rows: 4096 x 12288 24.1 / 27.2, 8192 x 4096 16.0 / 17.1; 64 rows: 27.3 /
+//                  36.0, 18.2 / 18.9); rounded or gated, narrow ones (64 rows, 4096 x 4096 14.3 / 15.6, but 6144 x 4096 23.4 /
+//                  17.8) and up to 32 rows of wide ones 4096 deep (32768 x 4096 53.5 / 65.6, gated 24576 x 4096 43.8 / 49.8;
+//                  64 rows: 67.8 / 61.8, 55.0 / 50.7).
+//   past 16384     at any number of rows (4096 x 18432: 38.0 / 50.7, 42.4 / 122.3, 54.9 / 130.8 at 1, 32, 64 rows).
+bool rows_fit(int n, int K, int N, int form) {
+    if (!rows_take(n, K, N, form)) return false;
+    if (n > 64 || K <= 2048 || K > (1 << 14)) return true;
+    const bool parts = form == kFormParts;
+    const int64_t rows = form == kFormGated ? 2ll * N : N;
+    if (n <= 16) return K <= 4096 || rows * K < (n > 1 && parts ? 1 << 25 : 1 << 24);
+    if (rows <= kWide) return parts || (K <= 4096 && rows <= kManyRowsCols);
+    return n <= 32 && K >= 4096;
 }
 
 int splits_for(int n, int K, int N) {
@@ -162,8 +183,8 @@ void launch_rows(RowsProduct p, int splits, hipStream_t s, int batch = 1) {
 
 using namespace skyrl;
 
-extern "C" int32_t skyrl_rows_product_fits(int32_t n, int32_t K, int32_t N, int32_t gated) {
-    return rows_fit(n, K, N, gated != 0);
+extern "C" int32_t skyrl_rows_product_fits(int32_t n, int32_t K, int32_t N, int32_t form) {
+    return rows_fit(n, K, N, form);
 }
 
 extern "C" int32_t skyrl_rows_product_splits(int32_t n, int32_t K, int32_t N) { return splits_for(n, K, N); }
@@ -172,7 +193,7 @@ extern "C" int skyrl_rows_product(const void* x, int64_t ldx, int32_t n, int32_t
                                   const void* bias, int32_t act, float alpha, float limit, int32_t splits, void* out,
                                   int64_t ldo, void* stream) {
     const bool gate = act >= 0;
-    SKYRL_REQUIRE(rows_fit(n, K, N, gate), "rows_product: sizes that the library takes");
+    SKYRL_REQUIRE(rows_take(n, K, N, gate ? kFormGated : splits ? kFormParts : kFormRound), "rows_product: sizes that the library takes");
     SKYRL_REQUIRE(x && w && out, "rows_product: null pointer");
     SKYRL_REQUIRE(aligned16(x) && aligned16(w) && ldx % 8 == 0 && ldw % 8 == 0 && ldw >= K && (n == 1 || ldx >= K),
                   "rows_product: rows must be 16-byte aligned");
@@ -208,8 +229,7 @@ extern "C" int skyrl_rows_product(const void* x, int64_t ldx, int32_t n, int32_t
     } else {
         if (n <= 16) launch_rows<kRound, 1, 1, 4, 4>(p, 1, s);
         else if (n <= 32) launch_rows<kRound, 1, 2, 4, 3>(p, 1, s);
-        else if (n <= 64) launch_rows<kRound, 1, 4, 4, 2>(p, 1, s);
-        else launch_rows<kRound, 1, 8, 4, 2>(p, 1, s);
+        else launch_rows<kRound, 1, 4, 4, 2>(p, 1, s);
     }
     return check_launch("rows_product_kernel");
 }

@@ -66,14 +66,15 @@ def embed(tokens: torch.Tensor, table: torch.Tensor, scale: float, positions: Op
 MAX_ROWS = 128  # that skyrl_rows_product takes at most
 
 
-def _rows_fit(x: torch.Tensor, w: torch.Tensor, gated: bool = False) -> bool:
-    """Whether skyrl_rows_product takes x [n, K] (a column range) and w [N, K] of these sizes, types and alignments."""
+def _rows_fit(x: torch.Tensor, w: torch.Tensor, gated: bool = False, parts: bool = False) -> bool:
+    """Whether skyrl_rows_product takes x [n, K] (a column range) and w [N, K] of these sizes, types and alignments, and is
+    the faster form."""
     n, K = x.shape
     if n > MAX_ROWS:
         return False
     N = w.shape[0] // 2 if gated else w.shape[0]
     return (x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.is_cuda
-            and bool(_ffi.query("skyrl_rows_product_fits", n, K, N, int(gated))) and _rows_aligned(x, w))
+            and bool(_ffi.query("skyrl_rows_product_fits", n, K, N, 1 if gated else 2 if parts else 0)) and _rows_aligned(x, w))
 
 
 def _rows_aligned(x: torch.Tensor, w: torch.Tensor) -> bool:
@@ -86,7 +87,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
     """x w^T + bias. Few bf16 rows take skyrl_rows_product, everything else the library. With `parts` the result of
     few rows may be f32 [splits, n, N], to be summed over the first index where it is read (add_norm, gate_norm_add,
     joined)."""
-    if not _rows_fit(x, w):
+    if not _rows_fit(x, w, parts=parts):
         return F.linear(x, w, bias)
     dev = _require_gpu(x, w, bias)
     (n, K), N = x.shape, w.shape[0]

@@ -34,7 +34,7 @@ def _bounds(x, w):
 @pytest.mark.parametrize("pad", (0, 24))
 def test_products(dev, n, N, K, pad):
     x, w, b = _data(dev, n, N, K, n + N, pad)
-    assert lk._rows_fit(x, w)
+    assert lk._rows_fit(x, w, parts=True) and lk._rows_fit(x, w) == (n <= 64)
     ref, off = _bounds(x, w)
     for bias in (None, b):
         want = ref if bias is None else ref + bias.double()
@@ -76,6 +76,14 @@ def test_what_the_library_takes(dev):
     assert lk.gated_linear(x[:65], w, "silu") is None
     for n, N, K in ((511, 12288, 64), (1024, 5888, 64), (1024, 6208, 64), (1024, 6144, 72)):  # few rows, few items, remainders
         assert lk.gated_linear(*_data(dev, n, 2 * N, K, 0)[:2], "silu") is None
+    # depths above 2048 where the library is the faster one: (rows, N, K, rounded, parts, gated of N / 2)
+    for n, N, K, rounded, parts, gated in ((1, 4096, 4096, 1, 1, 1), (1, 4096, 8192, 0, 0, 0), (16, 2048, 6144, 1, 1, 1),
+                                           (16, 2048, 8192, 0, 1, 0), (32, 8192, 4096, 0, 1, 0), (33, 4096, 4096, 1, 1, 1),
+                                           (33, 4096, 12288, 0, 1, 0), (32, 8208, 4096, 1, 1, 1), (33, 8208, 4096, 0, 0, 0),
+                                           (32, 8208, 3072, 0, 0, 0), (64, 32768, 2048, 1, 1, 1), (128, 2048, 2048, 0, 1, 0),
+                                           (1, 4096, 16384, 0, 0, 0), (64, 4096, 18432, 1, 1, 1)):
+        got = [bool(lk._ffi.query("skyrl_rows_product_fits", n, K, m, f)) for m, f in ((N, 0), (N, 2), (N // 2, 1))]
+        assert got == [bool(rounded), bool(parts), bool(gated)], (n, N, K)
     for a, b in ((big[:, 1:65], w), (x, w), (x[:4].float(), w.float())):
         torch.testing.assert_close(lk.linear(a, b, parts=True), torch.nn.functional.linear(a, b))
     with pytest.raises(ValueError):
