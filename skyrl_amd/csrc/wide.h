@@ -131,7 +131,7 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
         __builtin_amdgcn_global_load_lds((gbl_void*)src, (lds_void*)dst, 16, 0, 0);
     };
     int n0, q = 0;
-    const float per_row = KIND == kGateUp ? 1.f / p.row_div : 0.f;
+    const double per_row = KIND == kGateUp ? 1.0 / p.row_div : 0.0;
     auto open = [&](int it) {  // start on the item that was peeked at
         const int r0 = wave * 16 + lane / 8;
         int tile, nb;
@@ -148,7 +148,7 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
 #pragma unroll
             for (int i = 0; i < L; ++i) {
                 const int pair = max(next_rows[i], 0);  // places without a pair: row 0, not stored
-                const int d = (int)((float)pair * per_row), rest = pair - d * p.row_div;  // pair / row_div, one off at most
+                const int d = (int)(pair * per_row), rest = pair - d * p.row_div;  // pair / row_div, one off at most
                 xs[i] = p.x + (d + (rest >= p.row_div) - (rest < 0)) * p.ldx + chunk[i % 2];
             }
         } else {

@@ -423,6 +423,21 @@ def test_wide_tiles(width, ff, loads):
     assert torch.equal(y, lk.moe_experts(sh, x, idx.int().view(n, 1), weight, wgu, wd, tm=128).view(n, width))
 
 
+def test_wide_tiles_of_more_pairs_than_a_float_counts():
+    """A pair's token is exact past 2^24 pairs: the last tokens of 2.2 million that run all of eight experts."""
+    g = torch.Generator(device=DEV).manual_seed(1)
+    n, width, ff, E = 2_200_000, 64, 128, 8
+    sh = lk.moe_shape(width, ff, E, E)
+    mk = lambda *s, scale=1.0: (torch.randn(s, generator=g, device=DEV) * scale).to(BF16)  # noqa: E731
+    x, wgu, wd = mk(n, width), mk(E, 2, ff, width, scale=width ** -0.5), mk(E, width, ff, scale=ff ** -0.5)
+    idx = torch.arange(E, dtype=torch.int32, device=DEV).expand(n, E).contiguous()
+    y = lk.moe_experts(sh, x, idx, torch.ones(n, E, device=DEV), wgu, wd, tm=256).view(n, E, width)
+    h = x[-400:].float()
+    for e in range(E):
+        a = ref.silu(h @ wgu[e, 0].float().t()) * (h @ wgu[e, 1].float().t())
+        close(y[-400:, e], (a @ wd[e].float().t()).double().cpu(), BF16, bf16=8e-3)
+
+
 @pytest.mark.parametrize("width,ff,experts,top,n", [(2048, 768, 32, 8, 1500), (1024, 512, 64, 4, 300), (4096, 320, 8, 2, 90)])
 def test_tile_sizes_agree_bit_for_bit(width, ff, experts, top, n):
     """A row's sums are formed in the same order whatever its tile: products of a real layer's size, over and over."""
