@@ -365,7 +365,7 @@ __global__ __launch_bounds__(kNT) void moe_plain_kernel(Product p, const T* __re
 // waves stream a share of the depth each (stream.h). Bound: the experts' weights, each read once. Measured, 64 experts of 768 x
 // 2048, 8 per token, gate_up / down, us (TB/s of weights) against moe_gemm_kernel's, whose stages hold two workgroups a CU, in
 // step: 4 tokens 32.1 / 16.9 (5.3 / 5.0) against 41.5 / 17.7, 64 tokens 69.8 / 38.8 (5.8 / 5.2) against 83.0 / 39.4,
-// 128 tokens in tiles of 32 72.8 / 42.3 against 86.8 / 41.3, 256 in tiles of 64 79.9 / - against 86.8 / 42.5.
+// 128 tokens in tiles of 32 72.8 / 42.3 against 86.8 / 41.3.
 template <int NT, int MT, int WK, int S, bool GATED>
 __global__ __launch_bounds__(WK* kWave) void moe_stream_kernel(Product p, const uint16_t* __restrict__ x,
                                                                const uint16_t* __restrict__ w, uint16_t* __restrict__ out,
@@ -602,9 +602,9 @@ int launch_product(const Product& p, const void* x, const void* w, void* out, in
                            p, x_, w_, o_, (int)ncols);                                                                \
     } while (0)
         // Streamed where an expert has about one tile, so that its weights are read once: tiles of 16 below 16 pairs per
-        // expert (ntiles is npairs / tm + experts), of 32, and, for the wider of the two products, of 64 from 24 pairs on
-        // up to 2048 deep (256 tokens, 64 experts of 768 x 2048: 79.9 us against 86.8, of 1536 x 4096: 348 against 284). Tiles
-        // of 16 and 64 that are asked for at other loads sum a row in the order that larger ones do.
+        // expert (ntiles is npairs / tm + experts), and of 32. A streamed row is the sum of its waves' shares of the depth. Tiles
+        // of 64 and more, and of 16 at other loads, sum a row in one order, so that a step's rows do not depend on which of
+        // them its load takes (tiles of 64 streamed: 79.9 us against 86.8 for 256 tokens of 64 experts of 768 x 2048).
         const bool once = ntiles <= 2 * experts;
         if (p.tm == 256 && wide_fits(p.K, p.N, GATED)) {
             return launch_wide<GATED ? kGateUp : kDown>(Wide{x_, w_, o_, p.K, p.N, p.K, p.K, ntiles, p.order, p.tile_expert,
@@ -612,10 +612,8 @@ int launch_product(const Product& p, const void* x, const void* w, void* out, in
         }
         if (p.tm == 256) LAUNCH_GEMM(256, 256, 2, 4, 2);
         else if (p.tm == 128) LAUNCH_GEMM(128, 128, 2, 2, 2);
-        else if (p.tm == 64) {
-            if (GATED && once && p.K <= 2048 && (int64_t)(ntiles - experts) * 64 >= 24ll * experts) LAUNCH_STREAM(4, 4, 2, 2);
-            else LAUNCH_GEMM(64, 128, 2, 2, 3);
-        } else if (p.tm == 32) LAUNCH_STREAM(4, 2, 4, 1);
+        else if (p.tm == 64) LAUNCH_GEMM(64, 128, 2, 2, 3);
+        else if (p.tm == 32) LAUNCH_STREAM(4, 2, 4, 1);
         else if (once) LAUNCH_STREAM(4, 1, 4, 2);
         else LAUNCH_GEMM(16, 128, 1, 4, 4);
         return check_launch("moe_gemm_kernel");

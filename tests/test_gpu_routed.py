@@ -456,6 +456,20 @@ def test_tile_sizes_agree_bit_for_bit(width, ff, experts, top, n):
     assert all(torch.equal(outs[0], o) for o in outs[1:])
 
 
+@pytest.mark.parametrize("n", [192, 256, 383])
+def test_a_steps_own_tiles_agree_with_larger_ones(n):
+    """Tiles of 64 at the loads that a step of up to 383 tokens has them for: bit for bit those of 128 and 256."""
+    g = torch.Generator(device=DEV).manual_seed(n)
+    width, ff, experts, top = 2048, 768, 64, 8
+    sh = lk.moe_shape(width, ff, experts, top, 8, 4)
+    assert lk.moe_rows(sh, n) == 64
+    mk = lambda *s: (torch.randn(s, generator=g, device=DEV) * 0.03).to(BF16)  # noqa: E731
+    x, wgu, wd = mk(n, width) * 30, mk(experts, 2, ff, width), mk(experts, width, ff)
+    idx, weight = lk.moe_route(sh, x, mk(experts, width), torch.zeros(experts, device=DEV))
+    own, *larger = (lk.moe_experts(sh, x, idx, weight, wgu, wd, tm=tm) for tm in (None, 128, 256))
+    assert bool(own.isfinite().all()) and all(torch.equal(own, o) for o in larger)
+
+
 # ---------------------------------------------------------------- the model through the engine's steps
 def shaped(cfg, dtype, seed=0, max_len=512):
     """f32: routing by the tokens; bf16: a choice that rounding does not change."""
