@@ -6,6 +6,7 @@ import asyncio
 import io
 import json
 import math
+from types import SimpleNamespace
 
 import numpy as np
 import pytest
@@ -166,6 +167,40 @@ def test_prefill_with_sinks_and_gates(heads, dim, rot, vdim, rank, window, segs)
             else:
                 assert float(got[:, h].abs().max()) < 1e-12
         tok += n
+
+
+@pytest.mark.parametrize("heads", [3, 16])
+@pytest.mark.parametrize("T,n,alone", [(256, 256, True), (129, 129, True), (300, 48, False), (129, 100, False), (128, 48, False), (48, 48, True)])
+def test_decode_rows_of_many_tokens_take_the_librarys_products(heads, T, n, alone):
+    """Steps of more than 128 tokens: a row's up-projections bit for bit the library's, its shares beside portions as many
+    as fill a round; fewer tokens: the few-row products and shares that fit."""
+    D, R, V, C, ctx = 128, 64, 128, 512, 400
+    cfg = sandwich_config([low_rank(heads=heads, dim=D, rot_dim=R, vdim=V, kv_rank=C, q_rank=128, window=None)], [None], width=256, groups=1)
+    mix = build(cfg, BF16)[0].layers[0]["mixer"]
+    g = torch.Generator(device=DEV).manual_seed(T + n)
+    mk = lambda *s: torch.randn(s, generator=g, device=DEV).to(BF16)  # noqa: E731
+    blocks = -(-ctx // BS)
+    cache = mk(8 * blocks, BS, lk.latent_row(C, R))
+    inp = SimpleNamespace(block_tables=torch.arange(8 * blocks, dtype=torch.int32, device=DEV).view(8, blocks),
+                          bt_row=(torch.arange(T, device=DEV) % 8).int(), positions=(torch.arange(T, device=DEV) * 37 + 300) % ctx,
+                          max_ctx=ctx, one_token=alone)
+    q, out = mk(T, heads * (D + R)), torch.zeros(T, heads * V, dtype=BF16, device=DEV)
+    mix._attend_rows(q, None, out, inp, 0, n, cache, None)
+    q3 = q[:n].view(n, heads, D + R)
+    qa, o = torch.empty(heads, n, C, dtype=BF16, device=DEV), torch.empty(n, heads, V, dtype=BF16, device=DEV)
+    few = T <= 128
+    if few:
+        assert lk.rows_batch(q3[:, :, :D].transpose(0, 1), mix.wuk_t, qa)
+    else:
+        qa = torch.bmm(q3[:, :, :D].transpose(0, 1), mix.wuk.view(heads, D, C))
+    shares = min(256 // n if few or alone else -(-256 // n), -(-ctx // 64)) or 1
+    mid = lk.latent_attend(qa, q3[:, :, D:], cache, C, R, inp.block_tables, inp.bt_row[:n], inp.positions[:n], mix.scale, None, nparts=shares, sinks=mix.sinks)
+    if few:
+        assert lk.rows_batch(mid, mix.wuv.view(heads, V, C), o.transpose(0, 1))
+    else:
+        o.copy_(torch.bmm(mid, mix.wuv_t).transpose(0, 1))
+    assert bool(o.isfinite().all()) and torch.equal(out[:n].view(n, heads, V), o)
+
 
 
 # ---------------------------------------------------------------- generalized delta rule
