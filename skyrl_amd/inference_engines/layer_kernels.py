@@ -77,6 +77,11 @@ def _rows_fit(x: torch.Tensor, w: torch.Tensor, gated: bool = False, parts: bool
             and bool(_ffi.query("skyrl_rows_product_fits", n, K, N, 1 if gated else 2 if parts else 0)) and _rows_aligned(x, w))
 
 
+def gives_parts(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether linear(x, w, parts=True) returns parts."""
+    return _rows_fit(x, w, parts=True)
+
+
 def _rows_aligned(x: torch.Tensor, w: torch.Tensor) -> bool:
     n, K = x.shape
     return (x.stride(1) == 1 and w.stride(1) == 1 and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0

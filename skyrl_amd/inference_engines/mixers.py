@@ -282,10 +282,9 @@ class Gated:
     def forward(self, x: torch.Tensor, inp, state, workspace):
         if isinstance(self.sub, Products):
             return self.sub.forward(x, inp, state, workspace, parts=True)
-        if self.joint is not None and self.sub.chooses(x):
+        if self.joint is not None and self.sub.chooses(x, self.joint):
             logits = lk.linear(x, self.joint, parts=True)
-            if logits.dim() == 3:  # few rows
-                return self.sub.forward(x, inp, state, workspace, logits=(logits, self.weight.shape[0])), logits
+            return self.sub.forward(x, inp, state, workspace, logits=(logits, self.weight.shape[0])), logits
         return self.sub.forward(x, inp, state, workspace), lk.linear(x, self.weight)
 
 
@@ -1075,9 +1074,11 @@ class RoutedExperts:
             yield from ((f"e{e}.gate", self.gate_up[e, 0]), (f"e{e}.up", self.gate_up[e, 1]), (f"e{e}.down", self.down[e]))
         yield from (("router", self.router), ("correction", self.correction))
 
-    def chooses(self, x: torch.Tensor) -> bool:
-        """Whether few rows may come with their router logits."""
-        return x.dtype == torch.bfloat16 and x.shape[0] <= lk.MAX_ROWS and self.experts <= lk.CHOOSE_EXPERTS
+    def chooses(self, x: torch.Tensor, joint: torch.Tensor) -> bool:
+        """Whether rows come with their router logits, the product with `joint` that holds them giving parts. Asked ahead of that
+        product: at 65 to 128 rows it takes at most 4096 columns, the gate's and the router's together, and what the library
+        formed instead would be of no use."""
+        return self.experts <= lk.CHOOSE_EXPERTS and lk.gives_parts(x, joint)
 
     def forward(self, x: torch.Tensor, inp, state, workspace, logits=None) -> torch.Tensor:
         """logits: (layer_kernels.linear's parts that hold the router's, their first column)."""

@@ -11,6 +11,8 @@ from hybrid_cases import (CONFIGS, NORMED, PARALLEL, SANDWICH, attend, config, d
                           make_normed_weights, make_parallel_weights, make_sandwich_weights, make_weights, normed_config,
                           parallel_config, rglru, routed, sandwich_config, side, ssd)
 from oracle import hybrid_ref as ref
+from skyrl_amd import _ffi
+from skyrl_amd.inference_engines import layer_kernels as lk
 from skyrl_amd.inference_engines import mixers
 from skyrl_amd.inference_engines.engine import BLOCK_SIZE, EngineCore, ModelRunner, RequestParams
 from skyrl_amd.inference_engines.hybrid import HybridCache, HybridDecoder, HybridSpec
@@ -604,3 +606,27 @@ def test_normed_plans_and_window_tiles():
     keys = [t[1] + min(t[2], 128) for t in tiles.tolist()]
     assert keys == sorted(keys, reverse=True)
     assert ModelRunner(m, 4, 6).buckets == [2, 4, 6]
+
+
+@pytest.mark.parametrize("width,n,fits", [(256, 1, True), (256, 65, True), (256, 128, True), (256, 129, False), (4096, 64, True), (4096, 65, False),
+                                          (4096, 128, False), (8192, 1, False), (8192, 33, False)])
+def test_gated_experts_form_one_product_for_gate_and_router(width, n, fits, monkeypatch):
+    """The joint product runs where its parts are read, and the gate's own elsewhere: never both."""
+    w = mixers.Weights(torch.device("cpu"), torch.bfloat16, None, 0.02)
+    sub = mixers.RoutedExperts(routed(ff=8, experts=64, top=2), width, w)
+    gated = mixers.Gated(sub, width, w)
+    formed, given = [], []
+
+    def few(x, w_, gated=False, parts=False):
+        return bool(_ffi.query("skyrl_rows_product_fits", x.shape[0], x.shape[1], w_.shape[0], 2 if parts else 0)) and x.shape[0] <= lk.MAX_ROWS
+
+    def linear(x, w_, bias=None, parts=False):
+        formed.append(w_.shape[0])
+        return torch.empty((1, 1, 1) if parts and few(x, w_, parts=True) else (1, 1))
+
+    monkeypatch.setattr(lk, "_rows_fit", few)
+    monkeypatch.setattr(lk, "linear", linear)
+    monkeypatch.setattr(sub, "forward", lambda x, inp, state, ws, logits=None: given.append(logits))
+    gated.forward(torch.empty(n, width, dtype=torch.bfloat16), None, None, None)
+    assert formed == [width + 64 if fits else width]
+    assert (given[0] is not None) == fits and (not fits or given[0][1] == width)
