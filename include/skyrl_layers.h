@@ -171,8 +171,8 @@ int skyrl_latent_prefill(const void* q, int64_t q_stride, const void* k_nope, in
  *                          save_conv 1 also stores the convolution inputs and needs every sequence to
  *                          have one token; otherwise skyrl_conv_save of the channels follows.
  *   Prompt form, for portions of many tokens, in chunks of 64: chunk i32 [nchunks, 4] (first token,
- *   tokens <= 64, sequence, 0), chunks of one sequence consecutive and in order, cut from its first
- *   token on; d16, v16 = dim, vdim up to a multiple of 16. dim <= 256.
+ *   tokens <= 64, any of them short, sequence, 0), chunks of one sequence consecutive and in order, cut
+ *   from its first token on; d16, v16 = dim, vdim up to a multiple of 16. dim <= 256.
  *   In operand order a matrix is its 16 x 16 tiles, 256 numbers each: number 4 l + i is row l % 16, column 4 (l / 16) + i.
  *   skyrl_delta_conv       1: qk f32 [nchunks, kv_heads, 2, 64, d16] (unit vectors, q scaled), kt f32 [nchunks, kv_heads,
  *                          d16, 64] (k transposed), vt f32 [nchunks, heads, v16, 64] (v transposed), in operand order,

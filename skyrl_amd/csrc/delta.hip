@@ -573,11 +573,11 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(1))) void d
     }
     const int c0 = seq_chunks[si], c1 = seq_chunks[si + 1];
     if (c0 >= c1) return;
-    const int first = sq.chunk[4 * c0], last = sq.chunk[4 * c1 - 3];  // first token, tokens of the last chunk
     const int goff = 16 * wave + 4 * g, ostep = d.H * d.V, woff = wave * ns * kTile + 4 * lane;
     struct Operands {
         float4 w[NS], q[NS], p[4], kk[DT][4], u0, eg, er;
         float decay;
+        int t0, n;  // first token, tokens: any chunk may be short
     } in[SETS];
     // the parts of a chunk's operands that a step of 16 dims, or of 16 tokens, needs
     auto load_ends = [&](Operands& x, int ci) {
@@ -586,6 +586,8 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(1))) void d
         x.eg = ld4(G + ch * 2 * kC + goff);
         x.er = ld4(G + ch * 2 * kC + kC + goff);
         x.decay = G[ch * 2 * kC + kC - 1];
+        x.t0 = sq.chunk[4 * ci];
+        x.n = sq.chunk[4 * ci + 1];
     };
     auto load_dims = [&](Operands& x, int ci, int s) {
         if (!EXACT && s >= ns) return;
@@ -615,6 +617,7 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(1))) void d
             if (EXACT || s < ns) b[s] = ld4(&s_s[B][c * LS + 16 * s + 4 * g]);
         const float4 eg = x.eg;  // with one set the next chunk's take their place
         const float decay = x.decay;
+        const int t0 = x.t0, n = x.n;
         f32x4 aw = {0.f, 0.f, 0.f, 0.f}, ao = aw;
         // A load a product or two: a burst of them would hold the products up.
         if constexpr (SETS > 1) load_ends(next, cn);
@@ -662,8 +665,7 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(1))) void d
 #pragma unroll
         for (int s = 0; s < 4; ++s)
             if (s <= wave) ao = mma4(x.p[s], ul[s], ao);
-        float* op = o + ((int64_t)(first + (ci - c0) * kC) * d.H + h) * d.V;
-        const int n = ci + 1 < c1 ? kC : last;
+        float* op = o + ((int64_t)t0 * d.H + h) * d.V;
         if (vcol < d.V) {
 #pragma unroll
             for (int i = 0; i < 4; ++i)

@@ -8,6 +8,7 @@ the root mean square of the difference over that of the reference."""
 import asyncio
 import math
 
+import numpy as np
 import pytest
 import torch
 
@@ -303,6 +304,32 @@ def test_delta_recalls_one_far_write():
     c.step([(1, 300, x[300:398])])
     c.step([(1, 398, x[398:399])])
     close(c.step([(1, 399, x[399:])])[0], want[399:], torch.float32)
+
+
+@pytest.mark.parametrize("shape", [(2, 1, 64, 48, 3), (2, 2, 128, 128, 4), (3, 3, 18, 10, 1), (1, 1, 200, 130, 2)])
+def test_delta_chunks_of_any_length(shape, monkeypatch):
+    """A plan may cut a sequence into short chunks anywhere, not at its end alone."""
+    cuts = {0: (1, 64, 17, 64, 4), 1: (40, 3, 64)}
+
+    def plan(lens, first_seq, first_token):
+        chunk, ends, tok = [], [0], first_token
+        for i in range(first_seq, len(lens)):
+            assert sum(cuts[i]) == lens[i]
+            for n in cuts[i]:
+                chunk.append((tok, n, i, 0))
+                tok += n
+            ends.append(len(chunk))
+        return np.asarray(chunk, dtype=np.int32), np.asarray(ends, dtype=np.int32)
+
+    monkeypatch.setattr(mixers, "chunk_plan", plan)
+    c = DeltaCase(*shape, torch.float32, seed=2)
+    a, b = c.inputs(150), c.inputs(107)
+    (wa, Sa), (wb, Sb) = c.oracle(a), c.oracle(b)
+    oa, ob = c.step([(3, 0, a), (1, 0, b)], 0)
+    close(oa, wa, torch.float32)
+    close(ob, wb, torch.float32)
+    close(c.S[3][..., :c.sh.vdim], Sa, torch.float32)
+    close(c.S[1][..., :c.sh.vdim], Sb, torch.float32)
 
 
 # ---------------------------------------------------------------- the model through the engine's steps
