@@ -325,7 +325,7 @@ __global__ __launch_bounds__(kNT) void delta_conv_kernel(Dims d, SeqRef sq, cons
                     for (int j = 0; j < d.taps; ++j)
                         y[i] += input(ch, i0 + i - (d.taps - 1) + j) * ld(conv_w + (int64_t)ch * d.taps + j);
                 }
-                y[i] = i0 + i < n ? y[i] * sigmoid_<T>(y[i]) : 0.f;
+                y[i] = i0 + i < n ? siluf_(y[i]) : 0.f;
                 if (keys) smem[i * LK + e] = y[i];
             }
             if (keys) continue;

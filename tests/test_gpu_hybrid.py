@@ -6,6 +6,7 @@ scale); bf16 ones by one rounding of inputs and weights each (2e-2). Model logit
 the root mean square of the difference over that of the reference."""
 
 import asyncio
+import ctypes
 import math
 
 import numpy as np
@@ -304,6 +305,27 @@ def test_delta_recalls_one_far_write():
     c.step([(1, 300, x[300:398])])
     c.step([(1, 398, x[398:399])])
     close(c.step([(1, 399, x[399:])])[0], want[399:], torch.float32)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_delta_conv_leaves_f32(dtype):
+    """What the prompt form keeps of a convolution in f32 is exact to f32 for both types: of one tap of 1, whose sum is the
+    input, silu's exponential (1 ulp, 2^-23), sum and quotient (half an ulp each), half as much again."""
+    c = DeltaCase(2, 1, 16, 48, 1, dtype)
+    c.dev[0].fill_(1.0)
+    T, V, sh = 64, 48, c.sh
+    proj = torch.zeros(T, lk.delta_width(sh), dtype=dtype)
+    x = (torch.linspace(-60.0, 60.0, T * 2 * V).view(T, 2 * V)).to(dtype)
+    proj[:, 32:32 + 2 * V] = x
+    f32 = lambda *s: torch.empty(s, device=DEV)  # noqa: E731
+    i32 = lambda *v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
+    vt, proj, pos = f32(1, 2, 3, 4, 4, 16, 4), proj.to(DEV), torch.arange(T, device=DEV)
+    lk._ffi.call("skyrl_delta_conv", ctypes.byref(sh), lk._ptr(proj), proj.stride(0), *map(lk._ptr, c.dev[:3]), lk._ptr(i32(0, T, 0, 0)), 1,
+                 lk._ptr(i32(0, T)), lk._ptr(i32(0)), lk._ptr(pos), lk._ptr(c.ring), lk._ptr(f32(1, 1, 2, T, 16)), lk._ptr(f32(1, 1, 16, T)),
+                 lk._ptr(vt), lk._ptr(f32(T, 2)), lk._ptr(f32(T, 2)), lk._DTYPES[dtype], lk._stream(DEV))
+    got = vt[0].permute(2, 3, 5, 0, 1, 4).reshape(T, 2 * V).double().cpu()  # (token / 16, / 4 % 4, % 4), head, (value / 16, % 16)
+    want = ref.silu(x.double())
+    assert float(((got - want).abs() / want.abs().clamp(min=1e-30)).max()) < 1.5 * 2 ** -22
 
 
 @pytest.mark.parametrize("shape", [(2, 1, 64, 48, 3), (2, 2, 128, 128, 4), (3, 3, 18, 10, 1), (1, 1, 200, 130, 2)])
