@@ -255,9 +255,10 @@ constexpr int kTile = 256;
 
 // Convolution, silu, unit norms and gates. grid (nchunks, K + ceil(H V / 256)): the first K groups are the
 // key heads (q and k), the others 256 value channels each; gates with group 0. A channel's 64 inputs and the TAPS - 1 before
-// are all in flight at once (TAPS 0: any number of taps, loaded where they are used). Bound: 470 MB for 8192 tokens of 8192
-// channels (100 us at a large copy's rate).
-template <typename T, int TAPS>
+// are all in flight at once (TAPS 0: any number of taps, loaded where they are used; ONCE: a channel per thread in every group,
+// otherwise a key head's threads take sixteen inputs of each of their channels at a time). Bound: 470 MB for 8192 tokens of 8192
+// channels (100 us at a large copy's rate); 120 us, 190 with both forms in one kernel, whose registers leave half the waves.
+template <typename T, int TAPS, bool ONCE>
 __global__ __launch_bounds__(kNT) void delta_conv_kernel(Dims d, SeqRef sq, const T* __restrict__ proj, int64_t stride,
                                                          const T* __restrict__ conv_w, const float* __restrict__ a_log,
                                                          const float* __restrict__ dt_bias,
@@ -291,29 +292,31 @@ __global__ __launch_bounds__(kNT) void delta_conv_kernel(Dims d, SeqRef sq, cons
     };
     const int nch = keys ? 2 * D : min(kNT, d.H * V - ((int)blockIdx.y - d.K) * kNT);
     constexpr int kSub = 16, kBack = TAPS > 0 ? TAPS - 1 : 0;
-    const bool once = nch <= kNT;  // one channel per thread: its inputs stay in registers
+    const bool once = ONCE || nch <= kNT;  // one channel per thread: its inputs stay in registers
     float x[kBack + kC], w[TAPS > 0 ? TAPS : 1];
     auto channel = [&](int e) {
         return !keys ? 2 * d.K * D + ((int)blockIdx.y - d.K) * kNT + e : e < D ? kh * D + e : (d.K + kh) * D + (e - D);
     };
-    auto fetch = [&](int ch) {
+    auto fetch = [&](int ch, int from, int to) {  // inputs [from, to) of the channel's, in the unrolled loops
 #pragma unroll
         for (int j = 0; j < TAPS; ++j)
             w[j] = j >= TAPS - d.taps ? ld(conv_w + (int64_t)ch * d.taps + j - (TAPS - d.taps)) : 0.f;
 #pragma unroll
-        for (int i = 0; i < kC; ++i) x[kBack + i] = ld(proj + (int64_t)(t0 + min(i, n - 1)) * stride + ch);
+        for (int i = 0; i < kC; ++i)
+            if (kBack + i >= from && kBack + i < to) x[kBack + i] = ld(proj + (int64_t)(t0 + min(i, n - 1)) * stride + ch);
 #pragma unroll
-        for (int j = 0; j < kBack; ++j) x[j] = j > kBack - d.taps ? input(ch, j - kBack) : 0.f;
+        for (int j = 0; j < kBack; ++j)
+            if (j >= from) x[j] = j > kBack - d.taps ? input(ch, j - kBack) : 0.f;
     };
     if constexpr (TAPS > 0)
-        if (once && tid < nch) fetch(channel(tid));
+        if (once && tid < nch) fetch(channel(tid), 0, kBack + kC);
 #pragma unroll
     for (int sub = 0; sub < kC / kSub; ++sub) {
         const int i0 = sub * kSub;
         for (int e = tid; e < nch; e += kNT) {
             const int ch = channel(e);
             if constexpr (TAPS > 0)
-                if (!once) fetch(ch);
+                if (!once) fetch(ch, i0, i0 + kBack + kSub);
             float y[kSub];
 #pragma unroll
             for (int i = 0; i < kSub; ++i) {
@@ -818,9 +821,10 @@ extern "C" int skyrl_delta_conv(const skyrl_delta_shape* shape, const void* proj
                   "delta_conv: null pointer");
     SKYRL_DISPATCH_T(dtype, {
 #define LAUNCH_CONV(TAPS)                                                                                                 \
-    hipLaunchKernelGGL((delta_conv_kernel<T, TAPS>), dim3(nchunks, d.K + (d.H * d.V + kNT - 1) / kNT), dim3(kNT),          \
-                       16 * (2 * d.D + 4) * sizeof(float), as_stream(stream), d, SeqRef{chunk, cu, rows, positions},       \
-                       reinterpret_cast<const T*>(proj), proj_stride, reinterpret_cast<const T*>(conv_w), a_log, dt_bias,  \
+    hipLaunchKernelGGL((2 * d.D <= kNT ? delta_conv_kernel<T, TAPS, true> : delta_conv_kernel<T, TAPS, false>),            \
+                       dim3(nchunks, d.K + (d.H * d.V + kNT - 1) / kNT), dim3(kNT), 16 * (2 * d.D + 4) * sizeof(float),       \
+                       as_stream(stream), d, SeqRef{chunk, cu, rows, positions}, reinterpret_cast<const T*>(proj),         \
+                       proj_stride, reinterpret_cast<const T*>(conv_w), a_log, dt_bias,                                    \
                        reinterpret_cast<const T*>(conv_state), qk, kt, vt, lg, beta)
         if (d.taps <= 4) LAUNCH_CONV(4);
         else if (d.taps <= kConvWindow) LAUNCH_CONV(kConvWindow);
