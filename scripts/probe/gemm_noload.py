@@ -47,8 +47,8 @@ def run():
     print(json.dumps({"lib": "product"}), flush=True)
     lsb.gemm_sweep(shapes)
     for name in VARIANTS:
-        _ffi._libs.clear()
         _ffi.LIB_PATH = os.path.join(HERE, f"libgemm_{name}.so")
+        _ffi.forget()
         print(json.dumps({"lib": name}), flush=True)
         lsb.gemm_sweep(shapes)
 

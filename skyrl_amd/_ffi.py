@@ -455,6 +455,13 @@ def _lib_of(name: str) -> ctypes.CDLL:
     return lib
 
 
+def forget() -> None:
+    """Look every library up again at its next call: for a LIB_PATH that has changed."""
+    with _lock:
+        _libs.clear()
+        _lib_by_name.clear()
+
+
 def call(name: str, *args) -> int:
     """Invoke a status-returning entry point; raise SkyrlHipError on a non-zero status. Under an
     active ``variant(...)`` an entry point with an _ex form runs that form with the variant."""

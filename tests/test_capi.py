@@ -28,6 +28,24 @@ def test_library_exports_every_declared_symbol():
     assert not missing, f"declared in skyrl_hip.h but not exported: {missing}"
 
 
+def test_a_changed_library_is_what_is_called(monkeypatch):
+    """Entry points are looked up once, until the tables are dropped."""
+    class Lib:
+        def __init__(self, path):
+            self.skyrl_sample_workspace_bytes = lambda n, v: path
+
+    monkeypatch.setattr(_ffi, "_libs", {})
+    monkeypatch.setattr(_ffi, "_lib_by_name", {})
+    monkeypatch.setattr(_ffi, "_open", lambda path, signatures: _ffi._libs.setdefault(path, Lib(path)))
+    ask = lambda: _ffi.query("skyrl_sample_workspace_bytes", 1, 1)  # noqa: E731
+    monkeypatch.setattr(_ffi, "LIB_PATH", "one")
+    assert ask() == "one"
+    monkeypatch.setattr(_ffi, "LIB_PATH", "two")
+    assert ask() == "one"
+    _ffi.forget()
+    assert ask() == "two" and list(_ffi._libs) == ["two"]
+
+
 def test_ffi_signatures_cover_header():
     assert sorted(_ffi.SIGNATURES) == header_functions()
 
