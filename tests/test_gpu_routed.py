@@ -418,7 +418,8 @@ def test_experts(width, ff, experts, top, n, dtype):
                                                        (2048, 768, 64, 8, 95, 16), (1096, 200, 8, 4, 90, 32), (72, 136, 4, 2, 60, 64),
                                                        (1024, 264, 16, 4, 128, 64)])
 def test_streamed_products(width, ff, experts, top, n, tm):
-    """Few pairs per expert: weights streamed by waves with a share of the depth each, at the edges of tiles and pieces."""
+    """Few pairs per expert: weights streamed by waves with a share of the depth each (tiles of 16 and 32), at the edges of
+    tiles and pieces."""
     g = torch.Generator(device=DEV).manual_seed(width + n)
     sh = lk.moe_shape(width, ff, experts, top)
     mk = lambda *s, scale=1.0: (torch.randn(s, generator=g, device=DEV) * scale).to(BF16)  # noqa: E731
@@ -475,7 +476,8 @@ def test_wide_tiles_of_more_pairs_than_a_float_counts():
 
 @pytest.mark.parametrize("width,ff,experts,top,n", [(2048, 768, 32, 8, 1500), (1024, 512, 64, 4, 300), (4096, 320, 8, 2, 90)])
 def test_tile_sizes_agree_bit_for_bit(width, ff, experts, top, n):
-    """A row's sums are formed in the same order whatever its tile: products of a real layer's size, over and over."""
+    """A row's sums are formed in the same order whatever its tile, from 64 rows on and in tiles of 16 at loads that are not
+    streamed (more than one tile per expert): products of a real layer's size, over and over."""
     g = torch.Generator(device=DEV).manual_seed(width)
     sh = lk.moe_shape(width, ff, experts, top)
     mk = lambda *s, scale=1.0: (torch.randn(s, generator=g, device=DEV) * scale).to(BF16)  # noqa: E731
@@ -489,6 +491,26 @@ def test_tile_sizes_agree_bit_for_bit(width, ff, experts, top, n):
         a = ref.silu(wgu[e, 0].double().cpu() @ h) * (wgu[e, 1].double().cpu() @ h)
         close(outs[0][r], float(weight[t, r % top]) * (wd[e].double().cpu() @ a), BF16, bf16=8e-3)
     assert all(torch.equal(outs[0], o) for o in outs[1:])
+
+
+@pytest.mark.parametrize("experts,top,n,tm", [(64, 8, 4, 16), (64, 8, 95, 16), (64, 8, 128, 32), (16, 4, 60, 32)])
+def test_streamed_tiles_repeat_bit_for_bit(experts, top, n, tm):
+    """The tiles that decode steps take, products of a real layer's size over and over: an operand that is overwritten while it
+    is read would show."""
+    g = torch.Generator(device=DEV).manual_seed(n)
+    width, ff = 2048, 768
+    sh = lk.moe_shape(width, ff, experts, top)
+    assert lk.moe_rows(sh, n) == tm and lk._ffi.query("skyrl_moe_tiles", experts, n * top, tm) <= 2 * experts
+    mk = lambda *s, scale=1.0: (torch.randn(s, generator=g, device=DEV) * scale).to(BF16)  # noqa: E731
+    x, wgu, wd = mk(n, width), mk(experts, 2, ff, width, scale=0.03), mk(experts, width, ff, scale=0.03)
+    idx, weight = lk.moe_route(sh, x, mk(experts, width, scale=0.03), torch.zeros(experts, device=DEV))
+    outs = [lk.moe_experts(sh, x, idx, weight, wgu, wd) for _ in range(8)]
+    assert all(torch.equal(outs[0], o) for o in outs[1:])
+    for r in torch.randint(0, n * top, (8,), generator=torch.Generator().manual_seed(1)).tolist():
+        t, e = r // top, int(idx[r // top, r % top])
+        h = x[t].double().cpu()
+        a = ref.silu(wgu[e, 0].double().cpu() @ h) * (wgu[e, 1].double().cpu() @ h)
+        close(outs[0][r], float(weight[t, r % top]) * (wd[e].double().cpu() @ a), BF16, bf16=8e-3)
 
 
 @pytest.mark.parametrize("n", [192, 256, 383])

@@ -128,3 +128,41 @@ def test_batch(dev, B, n, N, K):
         assert bool(((out[b].double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2 * off).all())
     assert not lk.rows_batch(x[:, :, 1:], w[:, :, 1:].contiguous(), out)  # a depth and rows that are not 16-byte pieces
     assert not lk.rows_batch(x.float(), w.float(), out.float())
+
+
+# n, columns, depth; what the form has: waves along the depth, slots of each wave's ring
+DEEP = {"rounded": [(16, 3650, 2056, 4, 4), (20, 3650, 2056, 4, 3), (64, 3650, 2056, 4, 2),
+                    (16, 8200, 2056, 4, 2), (32, 8200, 2040, 4, 2), (50, 8200, 2040, 2, 2)],
+        "parts": [(16, 4104, 2056, 4, 4), (11, 2048, 6152, 4, 4), (32, 2050, 6152, 4, 2), (64, 2056, 6152, 4, 2), (100, 2056, 6152, 4, 1)],
+        "gated": [(16, 2056, 2040, 4, 2), (32, 2056, 2040, 4, 2), (64, 2056, 2040, 2, 2)],
+        "batch": [(16, 40, 1096, 4, 2), (32, 72, 1096, 4, 2), (100, 24, 1096, 4, 2)]}
+
+
+@pytest.mark.parametrize("form,n,N,K,waves,slots", [(f, *s) for f, shapes in DEEP.items() for s in shapes])
+def test_rings_are_refilled(dev, form, n, N, K, waves, slots):
+    """Every wave's share goes round its ring of slots, with a remainder at the end; over and over, since a slot that is
+    overwritten while it is read need not show at once."""
+    x, w, _ = _data(dev, n, 2 * N if form == "gated" else N, K, n + K)
+    shares = waves * (int(lk._ffi.query("skyrl_rows_product_splits", n, K, N)) if form == "parts" else 1)
+    assert -(-K // 64) // shares >= slots + 2 and K % 64
+    z, off = _bounds(x, w)
+    if form == "batch":
+        out = torch.empty(3, n, N, device=dev, dtype=torch.bfloat16)
+        run = lambda: (lk.rows_batch(x.expand(3, n, K).contiguous(), w.expand(3, N, K).contiguous(), out.zero_()), out.clone())  # noqa: E731
+        outs = [run() for _ in range(4)]
+        assert all(took for took, _ in outs)
+        outs = [y for _, y in outs]
+    else:
+        run = {"rounded": lambda: lk.linear(x, w), "parts": lambda: lk.linear(x, w, parts=True),
+               "gated": lambda: lk.gated_linear(x, w, "silu")}[form]
+        assert lk._rows_fit(x, w, gated=form == "gated", parts=form == "parts")
+        outs = [run() for _ in range(4)]
+    assert all(torch.equal(outs[0], y) for y in outs[1:])
+    y = outs[0].double()
+    if form == "gated":
+        g, u = z[:, :N], z[:, N:]
+        z, off = g * torch.sigmoid(g) * u, 1.2 * off[:, :N] * (u.abs() + 1) + (g.abs() + 1) * off[:, N:]
+    if form == "parts":
+        assert bool(((y.sum(0) - z).abs() <= 2 * off + 2.0 ** -21 * z.abs()).all())
+    else:
+        assert bool(((y - z).abs() <= 2.0 ** -8 * z.abs() + 2 * off + 1e-5).all())
