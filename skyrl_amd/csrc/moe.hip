@@ -604,7 +604,9 @@ int launch_product(const Product& p, const void* x, const void* w, void* out, in
         // Streamed where an expert has about one tile, so that its weights are read once: tiles of 16 below 16 pairs per
         // expert (ntiles is npairs / tm + experts), and of 32. A streamed row is the sum of its waves' shares of the depth. Tiles
         // of 64 and more, and of 16 at other loads, sum a row in one order, so that a step's rows do not depend on which of
-        // them its load takes (tiles of 64 streamed: 79.9 us against 86.8 for 256 tokens of 64 experts of 768 x 2048).
+        // them its load takes (tiles of 64 streamed: 79.9 us against 86.8 for 256 tokens of 64 experts of 768 x 2048). The
+        // package itself asks for 16 below 12 pairs per expert, streamed; a caller who asks for them at larger loads has the
+        // bits of larger tiles (both products, 300 tokens: 202 us, streamed 183, in tiles of 64 146).
         const bool once = ntiles <= 2 * experts;
         if (p.tm == 256 && wide_fits(p.K, p.N, GATED)) {
             return launch_wide<GATED ? kGateUp : kDown>(Wide{x_, w_, o_, p.K, p.N, p.K, p.K, ntiles, p.order, p.tile_expert,
