@@ -604,9 +604,11 @@ int launch_product(const Product& p, const void* x, const void* w, void* out, in
         // Streamed where an expert has about one tile, so that its weights are read once: tiles of 16 below 16 pairs per
         // expert (ntiles is npairs / tm + experts), and of 32. A streamed row is the sum of its waves' shares of the depth. Tiles
         // of 64 and more, and of 16 at other loads, sum a row in one order, so that a step's rows do not depend on which of
-        // them its load takes (tiles of 64 streamed: 79.9 us against 86.8 for 256 tokens of 64 experts of 768 x 2048). The
-        // package itself asks for 16 below 12 pairs per expert, streamed; a caller who asks for them at larger loads has the
-        // bits of larger tiles (both products, 300 tokens: 202 us, streamed 183, in tiles of 64 146).
+        // them its load takes. The package itself asks for 16 below 12 pairs per expert, streamed; a caller who asks for them at
+        // larger loads has the bits of larger tiles (both products, 300 tokens: 202 us, streamed 183, in tiles of 64 146).
+        // Tiles of 64, gated: up to 2048 deep 64 weight rows in four stages, two workgroups of either form on a CU but twice as
+        // many of this one (64 experts of 768 x 2048, both products, 256 tokens: 139.6 us against 143.5, streamed in shares 137;
+        // 1536 x 4096: 469 against 459).
         const bool once = ntiles <= 2 * experts;
         if (p.tm == 256 && wide_fits(p.K, p.N, GATED)) {
             return launch_wide<GATED ? kGateUp : kDown>(Wide{x_, w_, o_, p.K, p.N, p.K, p.K, ntiles, p.order, p.tile_expert,
@@ -614,8 +616,10 @@ int launch_product(const Product& p, const void* x, const void* w, void* out, in
         }
         if (p.tm == 256) LAUNCH_GEMM(256, 256, 2, 4, 2);
         else if (p.tm == 128) LAUNCH_GEMM(128, 128, 2, 2, 2);
-        else if (p.tm == 64) LAUNCH_GEMM(64, 128, 2, 2, 3);
-        else if (p.tm == 32) LAUNCH_STREAM(4, 2, 4, 1);
+        else if (p.tm == 64) {
+            if (GATED && p.K <= 2048) LAUNCH_GEMM(64, 64, 2, 2, 4);
+            else LAUNCH_GEMM(64, 128, 2, 2, 3);
+        } else if (p.tm == 32) LAUNCH_STREAM(4, 2, 4, 1);
         else if (once) LAUNCH_STREAM(4, 1, 4, 2);
         else LAUNCH_GEMM(16, 128, 1, 4, 4);
         return check_launch("moe_gemm_kernel");
