@@ -59,6 +59,7 @@ extern "C" {
  *                   gated in f32, rounded once. K a multiple of 64, N of 128. skyrl_gated_product_fits: whether it takes the
  *                   sizes and is the faster form.
  *   skyrl_rows_batch  `batch` such products without bias, x, w and out bf16 x_batch, w_batch and out_batch apart.
+ *                   skyrl_rows_batch_in_order: each sum in the order of the depth, not in shares of it.
  *   skyrl_add_norm_parts, skyrl_gate_norm_add_parts  of a model in bf16, the sublayer's output being such a sum of
  *                   `parts` (a_shares > 0) f32 [n, H], or (gate_shares > 0) the gate's logits being one of f32
  *                   [n, gate_stride]. */
@@ -94,6 +95,9 @@ int skyrl_rows_product(const void* x, int64_t ldx, int32_t n, int32_t K, const v
                        void* stream);
 int skyrl_rows_batch(const void* x, int64_t ldx, int64_t x_batch, int32_t n, int32_t K, const void* w, int64_t ldw,
                      int64_t w_batch, int32_t N, int32_t batch, void* out, int64_t ldo, int64_t out_batch, void* stream);
+int skyrl_rows_batch_in_order(const void* x, int64_t ldx, int64_t x_batch, int32_t n, int32_t K, const void* w, int64_t ldw,
+                              int64_t w_batch, int32_t N, int32_t batch, void* out, int64_t ldo, int64_t out_batch,
+                              void* stream);
 int skyrl_add_norm_parts(const float* delta, int32_t parts, float* hidden, const void* step, const void* weight, float w_base,
                          int32_t n, int32_t H, float eps, int32_t kind, void* out, void* stream);
 int skyrl_gate_norm_add_parts(const void* a, int32_t a_shares, int32_t parts, const void* gate, int32_t gate_shares,

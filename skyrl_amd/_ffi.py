@@ -293,6 +293,7 @@ LAYERS_SIGNATURES = {
     "skyrl_rows_product_splits": (_I32, [_I32, _I32, _I32]),
     "skyrl_rows_product": (_INT, [_P, _I64, _I32, _I32, _P, _I64, _I32, _P, _I32, _F, _F, _I32, _P, _I64, _P]),
     "skyrl_rows_batch": (_INT, [_P, _I64, _I64, _I32, _I32, _P, _I64, _I64, _I32, _I32, _P, _I64, _I64, _P]),
+    "skyrl_rows_batch_in_order": (_INT, [_P, _I64, _I64, _I32, _I32, _P, _I64, _I64, _I32, _I32, _P, _I64, _I64, _P]),
     "skyrl_add_norm_parts": (_INT, [_P, _I32, _P, _P, _P, _F, _I32, _I32, _F, _I32, _P, _P]),
     "skyrl_gate_norm_add_parts": (_INT, [_P, _I32, _I32, _P, _I32, _I64, _P, _P, _I32, _F, _F, _P, _P, _I32, _I32, _P, _P]),
     "skyrl_tanh": (_INT, [_P, _I64, _I64, _I32, _P, _I32, _P]),

@@ -110,11 +110,15 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
 # Rows up to which the products of a batch are faster here: 16 / 32 heads' two products and the copy between layouts took the library
 # 24.1 / 27.1 us for 256 rows, 11.3 / 22.7 us here, and 21.4 / 27.0 us for 512, 22.2 / 36.6 us here.
 BATCH_ROWS = 256
+# Sums along the depth are the library's bit for bit past 32 rows and up to a depth of 512 (8 to 32 heads, up-projections of 64
+# to 512); below and above its forms cut the depth.
+ORDERED_ROWS, ORDERED_DEPTH = 32, 512
 
 
-def rows_batch(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> bool:
+def rows_batch(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, in_order: bool = False) -> bool:
     """out [B, n, N] = x [B, n, K] w [B, N, K]^T for every B, each with unit column stride and any other strides; False
-    (nothing done) for sizes, types and alignments that are the library's."""
+    (nothing done) for sizes, types and alignments that are the library's. `in_order`: every sum goes along the depth, for results
+    that are the library's."""
     B, n, K = x.shape
     N = w.shape[1]
     if w.shape != (B, N, K) or out.shape != (B, n, N):
@@ -122,9 +126,11 @@ def rows_batch(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> bool:
     if (not 0 < n <= BATCH_ROWS or K % 8 or any(t.dtype != torch.bfloat16 or not t.is_cuda or t.stride(2) != 1 for t in (x, w, out))
             or any(s % 8 for t in (x, w) for s in t.stride()[:2]) or w.stride(1) < K or x.data_ptr() % 16 or w.data_ptr() % 16):
         return False
+    if in_order and (n <= ORDERED_ROWS or K > ORDERED_DEPTH):
+        return False
     dev = _require_gpu(x, w, out)
-    _ffi.call("skyrl_rows_batch", _ptr(x), x.stride(1), x.stride(0), n, K, _ptr(w), w.stride(1), w.stride(0), N, B, _ptr(out),
-              out.stride(1), out.stride(0), _stream(dev))
+    _ffi.call("skyrl_rows_batch_in_order" if in_order else "skyrl_rows_batch", _ptr(x), x.stride(1), x.stride(0), n, K, _ptr(w),
+              w.stride(1), w.stride(0), N, B, _ptr(out), out.stride(1), out.stride(0), _stream(dev))
     return True
 
 

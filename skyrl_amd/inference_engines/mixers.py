@@ -386,24 +386,23 @@ class LatentAttention:
 
     # ---- step
     def _attend_rows(self, q, gate, out, inp, a: int, b: int, cache, workspace):
-        """Tokens [a, b) in the decode form. In a step of more than lk.MAX_ROWS tokens every product is the library's, the
-        up-projections too, and the rows beside portions keep shares that fill a round: a row there has the same bits whatever
-        is the faster form of fewer rows (rows_batch: 13 us less a layer for 256 rows; shares that fit: 19 us for 48 beside
-        prompts, of steps of 1300 and 2100 us)."""
+        """Tokens [a, b) in the decode form. In a step of more than lk.MAX_ROWS tokens every product has the library's bits, the
+        up-projections too, and rows beside portions keep shares that fill a round: a row there is what it was whatever is the
+        faster form of fewer rows (shares that fit: 19 us less a layer for 48 rows beside prompts, of a step of 2100 us)."""
         H, D, R = self.heads, self.dim, self.rank
         n = b - a
-        few = q.shape[0] <= lk.MAX_ROWS
+        many = q.shape[0] > lk.MAX_ROWS
         q3 = q[a:b].view(n, H, D + self.rot_dim)
-        qa = torch.empty((H, n, R), dtype=q.dtype, device=q.device) if few else None
-        if qa is None or not lk.rows_batch(q3[:, :, :D].transpose(0, 1), self.wuk_t, qa):
+        qa = torch.empty((H, n, R), dtype=q.dtype, device=q.device)
+        if not lk.rows_batch(q3[:, :, :D].transpose(0, 1), self.wuk_t, qa, in_order=many):
             qa = torch.bmm(q3[:, :, :D].transpose(0, 1), self.wuk.view(H, D, R))
         o = lk.latent_attend(qa, q3[:, :, D:], cache, R, self.rot_dim, inp.block_tables, inp.bt_row[a:b],
                              inp.positions[a:b], self.scale, self.window,
-                             nparts=self.nparts(n, inp.max_ctx, up=not (few or inp.one_token)),
+                             nparts=self.nparts(n, inp.max_ctx, up=many and not inp.one_token),
                              part_min=kernels.MIN_PARTITION, workspace=workspace, sinks=self.sinks,
                              gate=None if gate is None else gate[a:b])
         to = out[a:b].view(n, H, self.vdim).transpose(0, 1)
-        if not (few and lk.rows_batch(o, self.wuv.view(H, self.vdim, R), to)):
+        if not lk.rows_batch(o, self.wuv.view(H, self.vdim, R), to, in_order=many):
             to.copy_(torch.bmm(o, self.wuv_t))
 
     def inner(self, proj: torch.Tensor, out: torch.Tensor, inp, cache: torch.Tensor, workspace) -> None:

@@ -130,6 +130,34 @@ def test_batch(dev, B, n, N, K):
     assert not lk.rows_batch(x.float(), w.float(), out.float())
 
 
+@pytest.mark.parametrize("B,D,C", [(16, 128, 512), (12, 128, 512), (32, 128, 512), (8, 64, 256), (16, 96, 384)])
+@pytest.mark.parametrize("n", [33, 48, 64, 65, 100, 191, 256])
+def test_batch_in_order_is_the_librarys(dev, B, n, D, C):
+    """Both up-projections of latent attention, from and to heads side by side in a row, bit for bit torch.bmm's."""
+    g = torch.Generator(device=dev).manual_seed(B + n)
+    q = torch.randn(n, B, D + 64, device=dev, generator=g).bfloat16()[:, :, :D].transpose(0, 1)
+    for x, K, N in ((q, D, C), (torch.randn(B, n, C, device=dev, generator=g).bfloat16(), C, D)):
+        w = (torch.randn(B, K, N, device=dev, generator=g) * 0.05).bfloat16()
+        out = torch.full((n, B, N), float("nan"), device=dev, dtype=torch.bfloat16).transpose(0, 1)
+        assert lk.rows_batch(x, w.transpose(1, 2).contiguous(), out, in_order=True)
+        assert torch.equal(out, torch.bmm(x, w))
+
+
+@pytest.mark.parametrize("n,N,K", [(33, 72, 328), (64, 130, 264), (200, 50, 72), (256, 24, 136), (100, 40, 512), (40, 16, 8)])
+def test_batch_in_order(dev, n, N, K):
+    g = torch.Generator(device=dev).manual_seed(n)
+    x = torch.randn(n, 3, K + 8, device=dev, generator=g).bfloat16()[:, :, :K].transpose(0, 1)
+    w = torch.randn(3, N, K, device=dev, generator=g).bfloat16()
+    out = torch.full((n, 3, N), float("nan"), device=dev, dtype=torch.bfloat16).transpose(0, 1)
+    assert lk.rows_batch(x, w, out, in_order=True)
+    for b in range(3):
+        ref, off = _bounds(x[b], w[b])
+        assert bool(((out[b].double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2 * off).all())
+    assert not lk.rows_batch(x[:, :32], w, out[:, :32], in_order=True)
+    big = torch.zeros(3, n, 520, device=dev, dtype=torch.bfloat16)
+    assert not lk.rows_batch(big, torch.zeros(3, N, 520, device=dev, dtype=torch.bfloat16), out, in_order=True)
+
+
 # n, columns, depth; what the form has: waves along the depth, slots of each wave's ring
 DEEP = {"rounded": [(16, 3650, 2056, 4, 4), (20, 3650, 2056, 4, 3), (64, 3650, 2056, 4, 2),
                     (16, 8200, 2056, 4, 2), (32, 8200, 2040, 4, 2), (50, 8200, 2040, 2, 2)],
