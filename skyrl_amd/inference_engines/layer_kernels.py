@@ -111,7 +111,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
 # 24.1 / 27.1 us for 256 rows, 11.3 / 22.7 us here, and 21.4 / 27.0 us for 512, 22.2 / 36.6 us here.
 BATCH_ROWS = 256
 # Sums along the depth are the library's bit for bit past 32 rows and up to a depth of 512 (8 to 32 heads, up-projections of 64
-# to 512); below and above its forms cut the depth.
+# to 512); below and above, its forms cut the depth.
 ORDERED_ROWS, ORDERED_DEPTH = 32, 512
 
 

@@ -386,12 +386,13 @@ class LatentAttention:
 
     # ---- step
     def _attend_rows(self, q, gate, out, inp, a: int, b: int, cache, workspace):
-        """Tokens [a, b) in the decode form. In a step of more than lk.MAX_ROWS tokens every product has the library's bits, the
-        up-projections too, and rows beside portions keep shares that fill a round: a row there is what it was whatever is the
-        faster form of fewer rows (shares that fit: 19 us less a layer for 48 rows beside prompts, of a step of 2100 us)."""
+        """Tokens [a, b) in the decode form. More than lk.ORDERED_ROWS of them in a step of more than lk.MAX_ROWS tokens, whose
+        products are all the library's, have its bits in their up-projections too, and beside portions the shares that fill a
+        round: such a row is what it was whatever is the faster form of fewer rows (shares that fit: 19 us less a layer for 48
+        rows beside prompts, of a step of 2100 us)."""
         H, D, R = self.heads, self.dim, self.rank
         n = b - a
-        many = q.shape[0] > lk.MAX_ROWS
+        many = q.shape[0] > lk.MAX_ROWS and n > lk.ORDERED_ROWS
         q3 = q[a:b].view(n, H, D + self.rot_dim)
         qa = torch.empty((H, n, R), dtype=q.dtype, device=q.device)
         if not lk.rows_batch(q3[:, :, :D].transpose(0, 1), self.wuk_t, qa, in_order=many):

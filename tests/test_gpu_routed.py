@@ -170,10 +170,11 @@ def test_prefill_with_sinks_and_gates(heads, dim, rot, vdim, rank, window, segs)
 
 
 @pytest.mark.parametrize("heads", [3, 16])
-@pytest.mark.parametrize("T,n,alone", [(256, 256, True), (129, 129, True), (300, 48, False), (129, 100, False), (128, 48, False), (48, 48, True)])
+@pytest.mark.parametrize("T,n,alone", [(256, 256, True), (129, 129, True), (300, 48, False), (300, 33, False), (300, 32, False), (129, 100, False),
+                                       (128, 48, False), (48, 48, True)])
 def test_decode_rows_of_many_tokens_take_the_librarys_products(heads, T, n, alone):
-    """Steps of more than 128 tokens: a row's up-projections bit for bit the library's, its shares beside portions as many
-    as fill a round; fewer tokens: the few-row products and shares that fit."""
+    """More than 32 rows in steps of more than 128 tokens: a row's up-projections bit for bit the library's, its shares beside
+    portions as many as fill a round; otherwise the few-row products and shares that fit."""
     D, R, V, C, ctx = 128, 64, 128, 512, 400
     cfg = sandwich_config([low_rank(heads=heads, dim=D, rot_dim=R, vdim=V, kv_rank=C, q_rank=128, window=None)], [None], width=256, groups=1)
     mix = build(cfg, BF16)[0].layers[0]["mixer"]
@@ -188,7 +189,7 @@ def test_decode_rows_of_many_tokens_take_the_librarys_products(heads, T, n, alon
     mix._attend_rows(q, None, out, inp, 0, n, cache, None)
     q3 = q[:n].view(n, heads, D + R)
     qa, o = torch.empty(heads, n, C, dtype=BF16, device=DEV), torch.empty(n, heads, V, dtype=BF16, device=DEV)
-    few = T <= 128
+    few = T <= 128 or n <= 32
     if few:
         assert lk.rows_batch(q3[:, :, :D].transpose(0, 1), mix.wuk_t, qa)
     else:
