@@ -252,7 +252,8 @@ __global__ __launch_bounds__(kNT * HG) __attribute__((amdgpu_waves_per_eu(1, 2))
     // The query rows of this head group, [latent | rotated | 0], through LDS into MFMA operands. Loads return in order: those of
     // whole 16-byte pieces go ahead of the pages', all at once, and land while the block table is read (16 heads, 512 + 64,
     // context 1024, us with the merge, against a loop of loads behind the first pages': 1 row 12.3 against 18.0, 64 rows 23.7
-    // against 28.8, 256 rows 60.5 against 67.1, the cache's 302 MB at 5.0 TB/s).
+    // against 28.8, 256 rows 60.5 against 67.1, over and over on one cache, part of which stays on chip; in engine passes 64 rows
+    // take 30 to 35, 256 rows 68, the cache's 302 MB at 4.4 TB/s).
     constexpr int QP = HG * 16 * NK * 4, QL = (QP + NT - 1) / NT;
     const bool pieces = rank % 8 == 0 && rot % 8 == 0 && q_stride % 8 == 0 && q_head % 8 == 0 &&
                         (reinterpret_cast<uintptr_t>(q_rot) & 15) == 0;
