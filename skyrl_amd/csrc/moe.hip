@@ -606,9 +606,9 @@ int launch_product(const Product& p, const void* x, const void* w, void* out, in
         // of 64 and more, and of 16 at other loads, sum a row in one order, so that a step's rows do not depend on which of
         // them its load takes. The package itself asks for 16 below 12 pairs per expert, streamed; a caller who asks for them at
         // larger loads has the bits of larger tiles (both products, 300 tokens: 202 us, streamed 183, in tiles of 64 146).
-        // Tiles of 64, gated: up to 2048 deep 64 weight rows in four stages, two workgroups of either form on a CU but twice as
-        // many of this one (64 experts of 768 x 2048, both products, 256 tokens: 139.6 us against 143.5, streamed in shares 137;
-        // 1536 x 4096: 469 against 459).
+        // Tiles of 64, gated: up to 2048 deep 64 weight rows in four stages in place of 128 in three. Two workgroups of either fit
+        // a CU, and 64 tiles of 768 columns are three rounds of the narrow ones, one and a half of the others (64 experts of 768
+        // x 2048, both products, 256 tokens: 139.6 us against 143.5, streamed in shares 137; 1536 x 4096: 469 against 459).
         const bool once = ntiles <= 2 * experts;
         if (p.tm == 256 && wide_fits(p.K, p.N, GATED)) {
             return launch_wide<GATED ? kGateUp : kDown>(Wide{x_, w_, o_, p.K, p.N, p.K, p.K, ntiles, p.order, p.tile_expert,
