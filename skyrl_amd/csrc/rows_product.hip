@@ -1,17 +1,21 @@
 // Products of a few activation rows with a weight matrix, y[n, N] = x[n, K] w[N, K]^T (decode steps; include/skyrl_layers.h).
 //
 // Bound: the weights' bytes. At 1 to 128 rows a weight matrix is read once and used little, and what the time went on
-// before was how it was read: the library's tiles for these shapes leave most CUs idle or few loads in flight. Here:
-//   one row   a wave per weight row (or gate and up row), lanes along the depth, so that every load is 1 KB of one row.
-//   more      a wave has a share of the depth to itself (stream.h). Few weight rows are cut into `splits` shares of the
-//             depth across workgroups too, each with f32 sums of its own that the next norm adds.
+// before was how it was read: the library's tiles for these shapes leave most CUs idle or few loads in flight. Here a wave has a
+// share of the depth to itself (stream.h). Few weight rows are cut into `splits` shares of the depth across workgroups too, each
+// with f32 sums of its own that the next norm adds. One row takes the same form, with that row in all 16 places: a wave per
+// weight row, lanes along the depth, took 5.6, 11.6, 6.2, 12.8 and 27.0 us for the five matrices below (its sums start when the
+// whole row is there).
 // Measured on one MI355X, weights from HBM, us (GB/s of weights) against the library's:
 //   N, K            1 row            16 rows          32 rows          64 rows
-//   2048, 2048      3.8 / 11.0       4.1 / 11.1       4.4 / 11.3       5.3 / 11.8
-//   2048, 6144      6.5 / 12.0       7.4 / 12.2       7.8 / 16.8       9.7 / 19.7
-//   3648, 2048      4.9 / 12.1       5.5 / 12.0       6.5 / 11.8       8.5 / 12.2   (no splits)
-//   12288, 2048     10.6 / 16.7      12.7 / 16.6      13.1 / 16.8      16.3 / 18.3  (no splits; 4.8 TB/s at one row)
-//   32768, 2048     23.6 / 35.0      26.3 / 34.5      29.5 / 36.8      30.3 / 37.1  (no splits; 5.7 TB/s at one row)
+//   2048, 2048      4.1 / 11.0       4.3 / 11.1       4.6 / 11.3       5.6 / 11.8
+//   2048, 6144      6.8 / 11.0       7.5 / 11.2       8.0 / 16.8       9.9 / 19.7
+//   3648, 2048      5.1 / 11.8       5.6 / 11.8       6.6 / 11.8       8.5 / 12.2   (no splits)
+//   12288, 2048     11.5 / 14.9      11.9 / 14.9      13.4 / 16.8      16.8 / 18.3  (no splits; 4.4 TB/s at one row)
+//   12288, 2048     11.6             11.8             13.4             16.4         (gated)
+//   32768, 2048     25.5 / 31.8      26.0 / 31.9      28.3 / 36.8      28.7 / 37.1  (no splits; 5.3 TB/s at one row)
+// At 64 rows a workgroup's x is as many bytes as its weights, over the same 64 bytes a clock into LDS: 12288 x 2048 gated takes
+// 16.4 us, 13.4 without x, 7.3 without the weights, 5.3 without either; leaving out the products changes it by 0.4.
 // Batches (a head's up-projections of latent attention, 512 x 128 and 128 x 512): 16 heads, 1 / 64 rows, both products with the
 // copy that the library's needed: 15.4 / 17.1 us, here 5.9 / 7.6 us.
 #include "gate.h"
@@ -36,52 +40,6 @@ struct RowsProduct {
     int row_blocks;  // gridDim.z = batch row_blocks
     int64_t x_batch, w_batch, out_batch;
 };
-
-// One row: R consecutive outputs per wave (kGated: R pairs), C loads of every weight row in flight.
-template <int MODE, int C, int NWV>
-__global__ __launch_bounds__(NWV* kWave) void one_row_kernel(RowsProduct p) {
-    constexpr int R = MODE == kGated ? 2 : 1;
-    const int lane = threadIdx.x & 63, n = blockIdx.x * NWV + (threadIdx.x >> 6);
-    if (n >= p.N) return;
-    const uint16_t* w[R];
-    float acc[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        w[r] = p.w + (int64_t)(n + r * p.N) * p.ldw;
-        acc[r] = 0.f;
-    }
-    for (int k = lane * 8; k < p.K; k += 512 * C) {
-        uint4 wv[R][C], xv[C];
-#pragma unroll
-        for (int j = 0; j < C; ++j) {
-            const int at = min(k + j * 512, p.K - 8);
-#pragma unroll
-            for (int r = 0; r < R; ++r) wv[r][j] = *reinterpret_cast<const uint4*>(w[r] + at);
-            xv[j] = *reinterpret_cast<const uint4*>(p.x + at);
-        }
-#pragma unroll
-        for (int j = 0; j < C; ++j) {
-            if (k + j * 512 >= p.K) break;
-            float x[8];
-            unpack8(xv[j], x);
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                float v[8];
-                unpack8(wv[r][j], v);
-#pragma unroll
-                for (int i = 0; i < 8; ++i) acc[r] = fmaf(v[i], x[i], acc[r]);
-            }
-        }
-    }
-#pragma unroll
-    for (int r = 0; r < R; ++r) acc[r] = wave_sum(acc[r]);
-    if (lane) return;
-    float y = acc[0];
-    if constexpr (MODE == kGated) y = gated(y, acc[1], p.gate);
-    else if (p.bias) y += ld(p.bias + n);
-    if constexpr (MODE == kParts) st(reinterpret_cast<float*>(p.out) + n, y);
-    else st(reinterpret_cast<uint16_t*>(p.out) + n, y);
-}
 
 // NT 16-row weight tiles (kGated: half of each matrix) and MT 16-row tiles of x per workgroup, the depth in gridDim.y * WK shares;
 // blocks of MT tiles and products of a batch along z.
@@ -145,25 +103,24 @@ bool rows_take(int n, int K, int N, int form) {
 // Where they are the faster form; us, here / the library's. Above 64 rows its tiles are as fast on wide matrices (128 rows, 12288
 // x 2048: 21.0 / 20.7) and slower on narrow ones only against parts (2048 x 2048 6.9 / 11.5, 2048 x 6144 14.2 / 17.8; rounded
 // 29.3). Depths above 2048 give them more to pipeline:
-//   up to 16 rows  until a matrix is both deep and large: 4096 x 4096 10.2 / 15.9, 30720 x 4096 44.7 / 59.8, 2048 x 6144 in parts
-//                  8.2 / 12.2, but 4096 x 8192 16.8 / 16.4, and one row of 2048 x 8192 14.6 / 13.6, of 4096 x 12288 24.5 / 21.7.
+//   up to 16 rows  until a matrix is both deep and large: 4096 x 4096 8.5 / 15.5, 30720 x 4096 44.7 / 59.8, 4096 x 6144 in parts
+//                  12.4 / 22.6 (one row: 11.0 / 22.5), 2048 x 8192 8.7 / 13.2 (8.1 / 12.6), but 4096 x 8192 16.7 / 15.9 (16.6 / 15.5).
 //   more rows      in parts, up to 8192 columns (32 rows: 4096 x 12288 24.1 / 27.2, 8192 x 4096 16.0 / 17.1; 64 rows: 27.3 /
 //                  36.0, 18.2 / 18.9); rounded or gated, narrow ones (64 rows, 4096 x 4096 14.3 / 15.6, but 6144 x 4096 23.4 /
 //                  17.8) and up to 32 rows of wide ones 4096 deep (32768 x 4096 53.5 / 65.6, gated 24576 x 4096 43.8 / 49.8;
 //                  64 rows: 67.8 / 61.8, 55.0 / 50.7).
-//   past 16384     at any number of rows (4096 x 18432: 38.0 / 50.7, 42.4 / 122.3, 54.9 / 130.8 at 1, 32, 64 rows).
+//   past 16384     at any number of rows (4096 x 18432: 26.9 / 46.7, 42.4 / 122.3, 54.9 / 130.8 at 1, 32, 64 rows).
 bool rows_fit(int n, int K, int N, int form) {
     if (!rows_take(n, K, N, form)) return false;
     if (n > 64 || K <= 2048 || K > (1 << 14)) return true;
     const bool parts = form == kFormParts;
     const int64_t rows = form == kFormGated ? 2ll * N : N;
-    if (n <= 16) return K <= 4096 || rows * K < (n > 1 && parts ? 1 << 25 : 1 << 24);
+    if (n <= 16) return K <= 4096 || rows * K < (parts ? 1 << 25 : 1 << 24);
     if (rows <= kWide) return parts || (K <= 4096 && rows <= kManyRowsCols);
     return n <= 32 && K >= 4096;
 }
 
 int splits_for(int n, int K, int N) {
-    if (n == 1) return 1;
     const int bn = n <= 16 ? 16 : 32, tiles = (N + bn - 1) / bn, most = K / 64 / 4;  // a piece per wave at least
     int s = (kFill + tiles / 2) / tiles;
     if (s > most) s = most;
@@ -204,26 +161,21 @@ extern "C" int skyrl_rows_product(const void* x, int64_t ldx, int32_t n, int32_t
     const RowsProduct p{reinterpret_cast<const uint16_t*>(x), ldx, n, K, reinterpret_cast<const uint16_t*>(w), ldw, N,
                         reinterpret_cast<const uint16_t*>(bias), Gate{act, alpha, limit}, out, ldo, (int64_t)n * ldo, 1, 0, 0, 0};
     hipStream_t s = as_stream(stream);
-    if (n == 1) {  // 4 loads of a row: 2048 deep at a time
-        const dim3 grid((N + 3) / 4), block(4 * kWave);
-        if (gate) hipLaunchKernelGGL((one_row_kernel<kGated, 4, 4>), grid, block, 0, s, p);
-        else if (splits) hipLaunchKernelGGL((one_row_kernel<kParts, 4, 4>), grid, block, 0, s, p);
-        else hipLaunchKernelGGL((one_row_kernel<kRound, 4, 4>), grid, block, 0, s, p);
-        return check_launch("one_row_kernel");
-    }
     // Wide tiles where there are columns enough, since every workgroup reads x again; else 16 rows of weights, so that
-    // the chip is full (3648 x 2048 at 64 rows: 8.5 us with 16, 9.4 with 32).
+    // the chip is full (3648 x 2048 at 64 rows: 8.5 us with 16, 9.4 with 32). Up to 16 rows 64 rows of weights for the wide ones
+    // (12352 x 2048: 12.0 us, with 32 13.8; gated 11.8 with two waves of four slots, 12.4 with four of two). Gated, 64 rows: four
+    // waves 16.4 us, two 18.3.
     if (gate) {
-        if (n <= 16) launch_rows<kGated, 2, 1, 4, 2>(p, 1, s);
+        if (n <= 16) launch_rows<kGated, 4, 1, 2, 4>(p, 1, s);
         else if (n <= 32) launch_rows<kGated, 4, 2, 4, 2>(p, 1, s);
-        else launch_rows<kGated, 4, 4, 2, 2>(p, 1, s);
+        else launch_rows<kGated, 4, 4, 4, 2>(p, 1, s);
     } else if (splits) {
         if (n <= 16) launch_rows<kParts, 1, 1, 4, 4>(p, splits, s);
         else if (n <= 32) launch_rows<kParts, 2, 2, 4, 2>(p, splits, s);
         else if (n <= 64) launch_rows<kParts, 2, 4, 4, 2>(p, splits, s);
         else launch_rows<kParts, 2, 8, 4, 1>(p, splits, s);
     } else if (N >= kWide) {
-        if (n <= 16) launch_rows<kRound, 2, 1, 4, 2>(p, 1, s);
+        if (n <= 16) launch_rows<kRound, 4, 1, 4, 2>(p, 1, s);
         else if (n <= 32) launch_rows<kRound, 4, 2, 4, 2>(p, 1, s);
         else launch_rows<kRound, 4, 4, 2, 2>(p, 1, s);
     } else {
