@@ -573,8 +573,8 @@ class ModelRunner:
 
     Decode runs over the persistent batch rows [0, nb) (nb = the smallest bucket >= 1 + the
     highest running row): per-row inputs (token, position, slot, context length, block-table
-    row) are staged in pinned host buffers and copied with two H2D copies into static device
-    buffers, and the forward + lm_head of bucket nb is a captured HIP graph replayed per step
+    row) are staged in a pinned host buffer and copied with one H2D copy into a static device
+    buffer, and the forward + lm_head of bucket nb is a captured HIP graph replayed per step
     (one launch instead of ~10 per layer from Python). Idle rows feed token 0 at position 0
     with slot -1 (no cache write) and context 1. Prefill runs eagerly (ragged shapes)."""
 
@@ -620,19 +620,22 @@ class ModelRunner:
         self.cache = None
         R = max_num_seqs
         pin = torch.cuda.is_available()
-        self.h_i64 = torch.zeros((3, R), dtype=torch.int64, pin_memory=pin)       # token | position | slot
-        self.h_i32 = torch.zeros((R, self.max_blocks), dtype=torch.int32, pin_memory=pin)  # block tables
-        self.h_ctx = torch.zeros(R, dtype=torch.int32, pin_memory=pin)
+        # A step's inputs in one buffer, so that one copy stages them: i64 token | position | slot [3, R], i32 contexts [R] and
+        # state rows [R], block tables [R, max_blocks], whose rows past the step's stay out. (Four copies of their own and the
+        # index of the wanted rows took 3.4 us each, of a step of 290 us for one row.)
+        self._head = 32 * R
+        size = self._head + 4 * R * self.max_blocks
+        self.h_in = torch.zeros(size, dtype=torch.uint8, pin_memory=pin)
+        self.d_in = torch.zeros(size, dtype=torch.uint8, device=self.device)
+        self.h_i64, self.h_ctx, self.h_rows, self.h_i32 = self._staging(self.h_in)
+        self.d_i64, self.d_ctx, self.d_rows, self.d_i32 = self._staging(self.d_in)
         self.h_keys = torch.zeros(R, dtype=torch.int64, pin_memory=pin)
         self.n_i64, self.n_i32, self.n_keys = self.h_i64.numpy(), self.h_i32.numpy(), self.h_keys.numpy()
-        self.n_ctx = self.h_ctx.numpy()
-        self.d_i64 = torch.zeros((3, R), dtype=torch.int64, device=self.device)
-        self.d_i32 = torch.zeros((R, self.max_blocks), dtype=torch.int32, device=self.device)
-        self.d_ctx = torch.ones(R, dtype=torch.int32, device=self.device)
-        if model.portions:  # decode steps also name each row's state row (-1: idle)
-            self.h_rows = torch.full((R,), -1, dtype=torch.int32, pin_memory=pin)
-            self.n_rows = self.h_rows.numpy()
-            self.d_rows = torch.full((R,), -1, dtype=torch.int32, device=self.device)
+        self.n_ctx, self.n_rows = self.h_ctx.numpy(), self.h_rows.numpy()
+        for ctx, rows in ((self.h_ctx, self.h_rows), (self.d_ctx, self.d_rows)):  # state rows: -1 is idle
+            ctx.fill_(1)
+            rows.fill_(-1)
+        if model.portions:
             self.d_iota = torch.arange(R + 1, dtype=torch.int32, device=self.device)
         self.d_keys = torch.zeros(R, dtype=torch.int64, device=self.device)
         self.tokens = torch.empty(R, dtype=torch.int32, device=self.device)
@@ -660,6 +663,12 @@ class ModelRunner:
         """Weights were re-allocated (sleep level 2 / wake_up): captured graphs point at the old storage."""
         self._graphs.clear()
         self._pool = None
+
+    def _staging(self, flat):
+        """Views of a staging buffer: token | position | slot, contexts, state rows, block tables."""
+        torch, R = self.torch, self.max_num_seqs
+        i32 = flat[24 * R:].view(torch.int32)
+        return flat[:24 * R].view(torch.int64).view(3, R), i32[:R], i32[R:2 * R], i32[2 * R:].view(R, self.max_blocks)
 
     def _h2d(self, arr: np.ndarray):
         return self.torch.from_numpy(arr).pin_memory().to(self.device, non_blocking=True)
@@ -742,13 +751,11 @@ class ModelRunner:
         n_i64[1, rows] = pos
         n_i64[2, rows] = n_i32[rows, pos // BLOCK_SIZE].astype(np.int64) * BLOCK_SIZE + pos % BLOCK_SIZE
         n_ctx[rows] = L
-        self.d_i64[:, :nb].copy_(self.h_i64[:, :nb], non_blocking=True)
-        self.d_i32[:nb].copy_(self.h_i32[:nb], non_blocking=True)
-        self.d_ctx[:nb].copy_(self.h_ctx[:nb], non_blocking=True)
         if self.model.portions:
             self.n_rows[:nb] = -1
             self.n_rows[rows] = rows
-            self.d_rows[:nb].copy_(self.h_rows[:nb], non_blocking=True)
+        n = self._head + 4 * nb * self.max_blocks
+        self.d_in[:n].copy_(self.h_in[:n], non_blocking=True)
         if self._staged is not None:
             self._staged.record(self.torch.cuda.current_stream(self.device))
 
@@ -811,6 +818,8 @@ class ModelRunner:
             if not want:
                 return None
             idx = np.fromiter((batch.requests[i].row for i, _ in want), dtype=np.int64, count=len(want))
+            if np.array_equal(idx, np.arange(len(want))):  # the first rows in order: nothing to gather
+                return self.model.logits(hidden[:len(want)])
             return self.model.logits(hidden.index_select(0, self._h2d(idx)))
         hidden = self._run_portions(batch, want)
         return self.model.logits(hidden) if want else None
