@@ -118,6 +118,44 @@ __device__ __forceinline__ Part wave_reduce_part(Part p) {
     return r0;
 }
 
+// Wave-wide sums and bests on DPP, as above: the cut of a filtered row is a chain of them. Require all 64 lanes active.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint64_t dpp64(uint64_t v) {  // a lane without a source (or of a row that ROWS leaves out): 0
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, CTRL, ROWS, 0xF, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), CTRL, ROWS, 0xF, false);
+    return ((uint64_t)hi << 32) | lo;
+}
+template <typename F>
+__device__ __forceinline__ F dpp_scan(F v) {  // inclusive sums over the lanes, of 64-bit integers or doubles
+    auto step = [&](uint64_t o) { v += __builtin_bit_cast(F, o); };
+    step(dpp64<0x111, 0xF>(__builtin_bit_cast(uint64_t, v)));  // row_shr 1, 2, 4, 8
+    step(dpp64<0x112, 0xF>(__builtin_bit_cast(uint64_t, v)));
+    step(dpp64<0x114, 0xF>(__builtin_bit_cast(uint64_t, v)));
+    step(dpp64<0x118, 0xF>(__builtin_bit_cast(uint64_t, v)));
+    step(dpp64<0x142, 0xA>(__builtin_bit_cast(uint64_t, v)));  // row_bcast 15, 31
+    step(dpp64<0x143, 0xC>(__builtin_bit_cast(uint64_t, v)));
+    return v;
+}
+template <int CTRL>
+__device__ __forceinline__ void best_dpp_step(Best& b) {
+    const Best o{__int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(b.score), CTRL, 0xF, 0xF, false)),
+                 __builtin_amdgcn_update_dpp(0, b.idx, CTRL, 0xF, 0xF, false)};
+    if (better(o.score, o.idx, b)) b = o;
+}
+__device__ __forceinline__ Best wave_best(Best b) {
+    best_dpp_step<0xB1>(b);
+    best_dpp_step<0x4E>(b);
+    best_dpp_step<0x124>(b);
+    best_dpp_step<0x128>(b);
+    Best r = b;
+#pragma unroll
+    for (int l = 0; l < kWave; l += 16) {
+        const Best o{__int_as_float(__builtin_amdgcn_readlane(__float_as_int(b.score), l)), __builtin_amdgcn_readlane(b.idx, l)};
+        if (l == 0 || better(o.score, o.idx, r)) r = o;
+    }
+    return r;
+}
+
 template <typename T>
 __device__ __forceinline__ float to_f(T v);
 template <> __device__ __forceinline__ float to_f<uint16_t>(uint16_t v) { return bf16_to_f32(v); }
@@ -1599,7 +1637,8 @@ constexpr int kPTieCap = 1024;  // elements at a split cut key
 constexpr int kPTieRes = 64;    // pass 1 ranks at most this many cut-key records (else pass 2)
 constexpr int kPCandCap = 2048; // pass 1's exactly scored elements (seeds + bound survivors)
 constexpr int32_t kRowPending = -4;  // RowFilter.ik between the two top_p kernels: pass 2 to run
-constexpr int kP2Splits = 8;         // workgroups per left row in sample_topp_pass2_kernel
+constexpr int kP2Splits = 8;         // pieces per left row in sample_topp_pass2_kernel
+constexpr int kP2Rows = 32;          // rows side by side in its grid: a workgroup per CU
 struct ToppPending {  // a row pass 1 did not decide, for sample_topp_pass2_kernel
     float xlo, xc, lse, mx;  // admissibility bound, the cut key's value, the raw lse, the raw max
     float e_s;               // e*: pass 1's best admissible record (score, index)
@@ -1621,7 +1660,7 @@ __global__ __launch_bounds__(kPNT) __attribute__((amdgpu_waves_per_eu(4))) void 
     static_assert(sizeof(T) == 2, "bf16 rows");
     constexpr int NT = kPNT, NW = NT / kWave, VEC = 8;
     constexpr int kDummy = 2 * kPHalf;  // 64 words taking the out-of-window elements' increments (no branch)
-    __shared__ uint32_t s_hist[2 * kPHalf + kWave];
+    __shared__ __attribute__((aligned(16))) uint32_t s_hist[2 * kPHalf + kWave];
     __shared__ uint16_t s_slow[kPSlowCap];
     __shared__ uint32_t s_nslow, s_bad, s_nt, s_zero[2];
     __shared__ float s_vmax[NW], s_bar;
@@ -1633,7 +1672,7 @@ __global__ __launch_bounds__(kPNT) __attribute__((amdgpu_waves_per_eu(4))) void 
     __shared__ float s_cs[kPCandCap];     // pass 1's exactly scored elements: score, index, key
     __shared__ int32_t s_ci[kPCandCap];
     __shared__ uint16_t s_ck[kPCandCap];
-    __shared__ uint32_t s_nc, s_ntie, s_trn;
+    __shared__ uint32_t s_nc, s_ntie;
 #ifdef SKYRL_TP_COUNT
     __shared__ uint32_t s_cnt[2];
     if (threadIdx.x < 2) s_cnt[threadIdx.x] = 0u;
@@ -1643,8 +1682,8 @@ __global__ __launch_bounds__(kPNT) __attribute__((amdgpu_waves_per_eu(4))) void 
     __shared__ float s_bar1, s_runmax;
     __shared__ __attribute__((aligned(16))) float s_wbest[NW];  // R > 1: each wave's best exact score
     constexpr int kRBar = TOPP ? SKYRL_TP_RBAR : 1;
-    __shared__ float s_bs[NW];
-    __shared__ int32_t s_bi[NW];
+    __shared__ float s_bs[NW], s_ts[NW];
+    __shared__ int32_t s_bi[NW], s_ti[NW];
     __shared__ int s_icut;
     __shared__ RowFilter s_rf;
     const int row_i = blockIdx.x;
@@ -2003,79 +2042,79 @@ __global__ __launch_bounds__(kPNT) __attribute__((amdgpu_waves_per_eu(4))) void 
     const uint64_t t_p1 = __builtin_amdgcn_s_memrealtime();  // (probe 11: the cut's time per row)
 
     bool fb = s_bad != 0u || s_nslow > (uint32_t)kPSlowCap;  // block-uniform
-    // the raw logits' sum-exp for the logprob, from the counts (another summation order than a
-    // streaming lse: equal to float rounding)
+    // On chip: the raw logits' sum-exp for the logprob, from the counts (another summation order than a streaming lse: equal to
+    // float rounding), and with top_p the bins' masses, their sum Z, the cut key and its tie count. With two rows a CU every
+    // row gets here at about the same time, so this is a chain of latencies behind the stream: bins are read once, as 16-byte
+    // pieces, values whose mass is 0 form none, sums and scans go over DPP and meet at one barrier (512 x 151,936, top_p 0.95:
+    // 4.7 us at T = 0.6, 6.3 at T = 1; with shuffles, two reads of the bins and a barrier for each sum 7.1 and 7.4).
     float lse = 0.f;
+    uint32_t kc = 0u;
+    bool split = false;
+    long long c = 0;
+    long long cut_cnt = 0;  // the cut key's element count (top_p)
+    int ic = 0x7fffffff;
     if (!fb) {
+        // thread t: the positive bins at descending positions p = 8t .. 8t+7 (value offset 4095 - p),
+        // the negative bins at ascending |x| (offset p), the list entries t, t + NT, ...
+        const int t8 = 8 * (int)threadIdx.x;
+        auto bins = [&](int end, uint32_t (&n)[8]) {  // end - 1, end - 2, ..
+            const uint4* h = reinterpret_cast<const uint4*>(s_hist + end - 8);
+            const uint4 lo = h[0], hi = h[1];
+            n[0] = hi.w; n[1] = hi.z; n[2] = hi.y; n[3] = hi.x;
+            n[4] = lo.w; n[5] = lo.z; n[6] = lo.y; n[7] = lo.x;
+        };
+        uint32_t pc[8], nn[8];
+        bins(2 * kPHalf - t8, pc);
+        bins(kPHalf - t8, nn);
+        auto pbits = [&](int q) { return (uint32_t)((kPE0 << 7) + kPHalf - 1 - (t8 + q)); };
+        auto nbits = [&](int q) { return 0x8000u | (uint32_t)((kPE0 << 7) + t8 + q); };
         double se = 0.0;
         auto sexp = [&](uint32_t bits, uint32_t n) {
             if (n) se += (double)n * (double)fast_exp2((bf16_to_f32((uint16_t)bits) - mx) * kLog2e);
         };
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
-            const int p8 = 8 * (int)threadIdx.x + q;
-            sexp((uint32_t)((kPE0 << 7) + p8), s_hist[kPHalf + p8]);
-            sexp(0x8000u | (uint32_t)((kPE0 << 7) + p8), s_hist[kPHalf - 1 - p8]);
+            sexp(pbits(q), pc[q]);
+            sexp(nbits(q), nn[q]);
         }
         for (int i = threadIdx.x; i < (int)s_nslow; i += NT) sexp(s_slow[i], 1u);
         if (threadIdx.x < 2) sexp(threadIdx.x ? 0x8000u : 0u, s_zero[threadIdx.x]);
-        se = wave_sum(se);
-        if (lane == 0) s_wexp[w] = se;
-        __syncthreads();
-        double S = 0.0;
-        for (int j = 0; j < NW; ++j) S += s_wexp[j];
-        lse = mx + fast_log2((float)S) * kLn2;
-    }
-
-    // ---- on chip (top_p): bin masses (once per bin, kept in registers), Z, the raw lse, the cut
-    //      key and its tie count
-    uint32_t kc = 0u;
-    bool split = false;
-    long long c = 0;
-    long long cut_cnt = 0;  // the cut key's element count (top_p)
-    int ic = 0x7fffffff;
-    if constexpr (TOPP) {
-        if (!fb) {
-            // thread t: the positive bins at descending positions p = 8t .. 8t+7 (value offset 4095 - p),
-            // the negative bins at ascending |x| (offset p), the list entries t, t + NT, ...
+        se = dpp_scan(se);
+        if (lane == kWave - 1) s_wexp[w] = se;
+        auto lse_of = [&]() {  // (behind a barrier)
+            double S = 0.0;
+            for (int j = 0; j < NW; ++j) S += s_wexp[j];
+            return mx + fast_log2((float)S) * kLn2;
+        };
+        if constexpr (!TOPP) {
+            __syncthreads();
+            lse = lse_of();
+        } else {
             auto mass_of = [&](uint32_t bits, uint32_t n) -> unsigned long long {
                 const float x = bf16_to_f32((uint16_t)bits);
-                if (n == 0u || (use_minp && !(x * inv_t >= mthr))) return 0ull;
+                // below 2^-32 of the max's: mass_q is 0
+                if (n == 0u || ((x - mx) * inv_t) * 1.4426950408889634f < -32.f || (use_minp && !(x * inv_t >= mthr))) return 0ull;
                 return (unsigned long long)n * (unsigned long long)mass_q(x, mx, inv_t);
             };
             unsigned long long pm[8], nm[8];
             unsigned long long pos = 0ull, neg = 0ull, mid = 0ull;
 #pragma unroll
             for (int q = 0; q < 8; ++q) {
-                const int p8 = 8 * (int)threadIdx.x + q;
-                const uint32_t pb = (uint32_t)((kPE0 << 7) + kPHalf - 1 - p8), nb = 0x8000u | (uint32_t)((kPE0 << 7) + p8);
-                const uint32_t pc = s_hist[2 * kPHalf - 1 - p8], nc = s_hist[kPHalf - 1 - p8];
-                pm[q] = mass_of(pb, pc);
-                nm[q] = mass_of(nb, nc);
+                pm[q] = mass_of(pbits(q), pc[q]);
+                nm[q] = mass_of(nbits(q), nn[q]);
                 pos += pm[q];
                 neg += nm[q];
             }
             for (int i = threadIdx.x; i < (int)s_nslow; i += NT) mid += mass_of(s_slow[i], 1u);
             if (threadIdx.x < 2) mid += mass_of(threadIdx.x ? 0x8000u : 0u, s_zero[threadIdx.x]);
-            unsigned long long ip = pos, in = neg;
-#pragma unroll
-            for (int off = 1; off < kWave; off <<= 1) {
-                const unsigned long long op = (unsigned long long)__shfl_up((long long)ip, off, kWave);
-                const unsigned long long on = (unsigned long long)__shfl_up((long long)in, off, kWave);
-                if (lane >= off) {
-                    ip += op;
-                    in += on;
-                }
-            }
-            unsigned long long wm = mid;
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) wm += (unsigned long long)__shfl_xor((long long)wm, off, kWave);
+            const unsigned long long ip = dpp_scan(pos), in = dpp_scan(neg), wm = dpp_scan(mid);
             if (lane == kWave - 1) {
                 s_wpos[w] = ip;
                 s_wneg[w] = in;
+                s_woth[w] = wm;
             }
-            if (lane == 0) s_woth[w] = wm;
             __syncthreads();
+            lse = lse_of();
             unsigned long long offp = 0ull, offn = 0ull, Zp = 0ull, Zn = 0ull, Zm = 0ull;
             for (int j = 0; j < NW; ++j) {
                 if (j < w) {
@@ -2237,33 +2276,38 @@ __global__ __launch_bounds__(kPNT) __attribute__((amdgpu_waves_per_eu(4))) void 
                 return bf16_to_f32(s_ck[i]) >= xlo ? 1 : 0;
             }
         };
-        Best e{-INFINITY, 0x7fffffff};
-        for (int i = threadIdx.x; i < nc; i += NT)
-            if (cls(i) == 1 && better(s_cs[i], s_ci[i], e)) e = Best{s_cs[i], s_ci[i]};
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            const float os = __shfl_xor(e.score, off, kWave);
-            const int oi = __shfl_xor(e.idx, off, kWave);
-            if (better(os, oi, e)) e = Best{os, oi};
+        // the best record that is kept and the best of the split cut key's; the lane that holds the first keeps its bits
+        Best e{-INFINITY, 0x7fffffff}, t{-INFINITY, 0x7fffffff};
+        uint16_t eb = 0;
+        for (int i = threadIdx.x; i < nc; i += NT) {
+            const int cl = cls(i);
+            if (cl == 1 && better(s_cs[i], s_ci[i], e)) {
+                e = Best{s_cs[i], s_ci[i]};
+                eb = s_ck[i];
+            }
+            if (TOPP && cl == 2 && better(s_cs[i], s_ci[i], t)) t = Best{s_cs[i], s_ci[i]};
         }
+        const int own = e.idx;
+        e = wave_best(e);
+        if (TOPP && split) t = wave_best(t);
         if (lane == 0) {
             s_bs[w] = e.score;
             s_bi[w] = e.idx;
+            s_ts[w] = t.score;
+            s_ti[w] = t.idx;
         }
         __syncthreads();
-        Best es{s_bs[0], s_bi[0]};
-        for (int j = 1; j < NW; ++j)
+        Best es{s_bs[0], s_bi[0]}, ts{s_ts[0], s_ti[0]};
+        for (int j = 1; j < NW; ++j) {
             if (better(s_bs[j], s_bi[j], es)) es = Best{s_bs[j], s_bi[j]};
+            if (better(s_ts[j], s_ti[j], ts)) ts = Best{s_ts[j], s_ti[j]};
+        }
         e0 = es;
-        uint32_t ntie = 0u;
-        if (TOPP && split)
-            for (int i = threadIdx.x; i < nc; i += NT) ntie += (better(s_cs[i], s_ci[i], es) && cls(i) == 2) ? 1u : 0u;
-        if (ntie) atomicAdd(&s_ntie, ntie);
-        __syncthreads();
         const float bar_end = kRBar > 1 ? rbar() : s_bar1;  // (after the barriers above: final)
-        bool ties_ok = s_ntie == 0u;
+        bool ties_ok = !(TOPP && split) || ts.idx == 0x7fffffff || !better(ts.score, ts.idx, es);
+        bool tie = false;  // the row goes to an element of the split cut key
 #ifdef SKYRL_TP_REASON
-        why |= (complete ? 0u : 1u) | (es.idx == 0x7fffffff ? 2u : 0u) | (s_ntie ? 4u : 0u) | (es.score < bar_end ? 8u : 0u);
+        why |= (complete ? 0u : 1u) | (es.idx == 0x7fffffff ? 2u : 0u) | (ties_ok ? 0u : 4u) | (es.score < bar_end ? 8u : 0u);
 #endif
 #if SKYRL_TP_TIERES
         // recorded elements of the split cut key that beat e*: kept iff fewer than c elements of that
@@ -2271,18 +2315,20 @@ __global__ __launch_bounds__(kPNT) __attribute__((amdgpu_waves_per_eu(4))) void 
         // (cached: the row was just read) for the key's indices, instead of leaving the row to pass 2.
         // The unrecorded ones scored below the bar, so below e*: the decision is the best of e* and the
         // kept listed records.
-        if (TOPP && split && !ties_ok && s_ntie <= (uint32_t)kPTieRes && probe != 5 && complete &&
-            es.idx != 0x7fffffff && es.score >= bar_end) {
-            if (threadIdx.x == 0) s_trn = 0u;
-            __syncthreads();
+        const bool rank = TOPP && split && !ties_ok && probe != 5 && complete && es.idx != 0x7fffffff && es.score >= bar_end;
+        if (rank) {  // (block-uniform)
             for (int i = threadIdx.x; i < nc; i += NT)
                 if (cls(i) == 2 && better(s_cs[i], s_ci[i], es)) {
-                    const uint32_t p = atomicAdd(&s_trn, 1u);  // < kPTieRes (s_ntie counted the same set)
-                    s_tri[p] = s_ci[i];
-                    s_trs[p] = s_cs[i];
+                    const uint32_t p = atomicAdd(&s_ntie, 1u);
+                    if (p < (uint32_t)kPTieRes) {
+                        s_tri[p] = s_ci[i];
+                        s_trs[p] = s_cs[i];
+                    }
                 }
             __syncthreads();
-            const int nr = (int)s_trn;
+        }
+        if (rank && s_ntie <= (uint32_t)kPTieRes) {
+            const int nr = (int)s_ntie;
             int imin = 0x7fffffff, imax = 0;
             for (int j = 0; j < nr; ++j) {
                 imin = min(imin, s_tri[j]);
@@ -2350,15 +2396,19 @@ __global__ __launch_bounds__(kPNT) __attribute__((amdgpu_waves_per_eu(4))) void 
             }
             __syncthreads();
             for (int j = 0; j < NW; ++j)
-                if (better(s_bs[j], s_bi[j], es)) es = Best{s_bs[j], s_bi[j]};
+                if (better(s_bs[j], s_bi[j], es)) {
+                    es = Best{s_bs[j], s_bi[j]};
+                    tie = true;
+                }
             ties_ok = true;
         }
 #endif
         const bool certified = probe != 5 && complete && es.idx != 0x7fffffff && ties_ok && es.score >= bar_end;
         if (certified) {
-            if (threadIdx.x == 0) {
+            // the lane that holds the winner, whose logit it has (a load of it here takes a microsecond)
+            if (tie ? threadIdx.x == 0 : own == es.idx) {
                 tokens[row_i] = es.idx;
-                if (logp_out) logp_out[row_i] = to_f<T>(row[es.idx]) - lse;
+                if (logp_out) logp_out[row_i] = (tie ? xc : bf16_to_f32(eb)) - lse;
                 // (tk = 1: decided in pass 1; ic unresolved: not needed)
                 filt[row_i] = RowFilter{mx, 1u, kRowDone, kc, split ? -1 : ic};
             }
@@ -2704,30 +2754,39 @@ __global__ __launch_bounds__(kPNT) __attribute__((amdgpu_waves_per_eu(4))) void 
 }
 
 // Pass 2 of the rows sample_topp_kernel left pending (RowFilter.ik = kRowPending), each row cut into
-// kP2Splits workgroups of contiguous vectors (a fixed partition: the split-mode sampler's pattern).
-// (Measured and dropped in r05: a (slots x 8) grid over the left rows only, 25.6 vs 24 us; pass 2
+// kP2Splits pieces of contiguous vectors (a fixed partition: the split-mode sampler's pattern). Mostly no row is left, so a
+// workgroup looks at every kP2Rows-th row: 512 rows take 2.9 us to find that there are none, with a workgroup for each row and
+// piece 3.7 (64 rows 2.1 and 1.9, one row 2.3 and 3.6; the next launch's own minimum is 1.7).
+// (Measured and dropped: a (slots x 8) grid over the left rows only, 25.6 vs 24 us; pass 2
 // inside pass 1's launch with the left rows' pieces claimed by the workgroups that finished -- a
 // CAS-claimed queue head ~1.4 ms, a row-by-row walk ~120 us, tickets ~88-91 vs 80-82 us a launch:
 // a piece claimed after the row's cut waits out the same latency chain as a launch, plus the claim.)
 // MODE 2 over the admissible elements x >= xlo of the piece, bar and best starting from e*; the
 // split cut key's indices appended to the row's tie list (one agent-scope add per lane). The last
 // arriving piece (arrive_last) merges the pieces' bests, ranks the ties by index (the first c are
-// admissible, scored exactly) and writes token, logprob and cut. The other rows' workgroups exit.
+// admissible, scored exactly) and writes token, logprob and cut.
 template <typename T, bool TOPP>
 __global__ __launch_bounds__(kPNT) void sample_topp_pass2_kernel(
     const T* __restrict__ logits, int64_t ld, int V, float inv_t, uint64_t seed, const int64_t* __restrict__ seq_ids,
     int64_t step, int32_t* __restrict__ tokens, float* __restrict__ logp_out, RowFilter* __restrict__ filt,
     const ToppPending* __restrict__ pend, unsigned* __restrict__ pend_nt, int32_t* __restrict__ ties,
-    Best* __restrict__ parts) {
+    Best* __restrict__ parts, int nseq) {
     constexpr int NT = kPNT, NW = NT / kWave, VEC = 8, kPer = 8;  // up to kPer vectors per lane
-    const int row_i = blockIdx.x, piece = blockIdx.y;
-    if (filt[row_i].ik != kRowPending) return;  // (workgroup-uniform)
     __shared__ float s_bar, s_bs[NW];
     __shared__ int32_t s_bi[NW];
     __shared__ int s_last, s_icut;
     __shared__ int32_t s_tidx[kPTieCap];
-    const ToppPending st = pend[row_i];
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+    // of the rows r0, r0 + gridDim.x, .. the left ones (no row of them is done before this workgroup's piece is: every wave reads
+    // the same)
+    auto left = [&](int r0) {
+        const int r = r0 + lane * (int)gridDim.x;
+        return __builtin_amdgcn_ballot_w64(r < nseq && filt[r].ik == kRowPending);
+    };
+    unsigned long long m = left(blockIdx.x);
+    if (m == 0 && nseq <= kWave * (int)gridDim.x) return;
+    auto run = [&](int row_i, int piece) {
+    const ToppPending st = pend[row_i];
     const T* row = logits + (int64_t)row_i * ld;
     const uint4* rv = reinterpret_cast<const uint4*>(row);
     const int nvec = V / VEC;
@@ -2944,6 +3003,16 @@ __global__ __launch_bounds__(kPNT) void sample_topp_pass2_kernel(
         filt[row_i] = RowFilter{st.mx, 0u, kRowDone, st.kc, icut};
 #endif
     }
+    };
+    for (int r0 = blockIdx.x;;) {
+        for (; m; m &= m - 1) {
+            run(r0 + (__ffsll((long long)m) - 1) * (int)gridDim.x, blockIdx.y);
+            __syncthreads();  // the shared words are the next row's
+        }
+        r0 += kWave * gridDim.x;
+        if (r0 >= nseq) return;
+        m = left(r0);
+    }
 }
 
 constexpr int kMaxSplits = 64;
@@ -3049,8 +3118,8 @@ int launch_sample(const void* logits, int64_t ld, int nseq, int V, float tempera
                                    probe);
             int rc = check_launch("sample_topp_kernel");
             if (rc || !use_topp || (probe >= 1 && probe <= 4) || probe == 11) return rc;  // (probes 1-4, 11)
-            hipLaunchKernelGGL((sample_topp_pass2_kernel<T, true>), dim3(nseq, kP2Splits), dim3(kPNT), 0, stream, lg, ld,
-                               V, inv_t, seed, seq_ids, step, tokens, logp, filt, pend, pend_nt, pties, pparts);
+            hipLaunchKernelGGL((sample_topp_pass2_kernel<T, true>), dim3(nseq < kP2Rows ? nseq : kP2Rows, kP2Splits), dim3(kPNT), 0, stream, lg, ld,
+                               V, inv_t, seed, seq_ids, step, tokens, logp, filt, pend, pend_nt, pties, pparts, nseq);
             return check_launch("sample_topp_pass2_kernel");
         }
     }

@@ -124,6 +124,22 @@ def test_topp_fast_ranks_cut_key_ties_in_pass1(dev):
         _ab(x.to(dev), 0, temperature=temp, top_p=p, seed=9, seq_ids=ids.to(dev), step=step)
 
 
+@pytest.mark.parametrize("n", [31, 32, 33, 100, 2100])
+@pytest.mark.parametrize("temp,p", [(1.0, 0.9), (0.05, 0.95), (8.0, 0.5)])
+def test_pass2_workgroups_take_several_rows(dev, n, temp, p):
+    """Pass 2's grid has 32 rows side by side, whose workgroups take every 32nd, 64 of them at a look: all rows through pass 2
+    and the ordinary run, at temperatures whose masses end far above and far below the row's values."""
+    V = 2056
+    g = torch.Generator().manual_seed(n)
+    x = (torch.randn(n, V, generator=g) * 3).to(torch.bfloat16).to(dev)
+    ids = torch.arange(n, dtype=torch.int64, device=dev)
+    kw = dict(temperature=temp, top_p=p, seed=3, seq_ids=ids, step=n)
+    tok, lp, done = _ab(x, 1, **kw)
+    with ops.variant(sampler_topp_fast=2, topp_probe=5):
+        t2, l2 = ops.sample(x, **kw)
+    assert torch.equal(t2.cpu(), tok) and torch.allclose(l2.cpu(), lp, atol=2e-5, rtol=1e-5)
+
+
 def test_minp_list_mode_overflow_and_ordinary_rows(dev):
     """min_p alone: pass 1 lists the elements within T |ln min_p| of the running max and decides
     from the list (sampler.hip SKYRL_MP_LIST). Rows with thousands of elements at the max overflow
