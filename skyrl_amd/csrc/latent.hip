@@ -15,6 +15,8 @@
 // up-projection once per key instead of once per query, and the scores cost dim + rot_dim instead of
 // rank + rot_dim per pair. latent_prefill is a windowed flash-style kernel: four waves share a K and
 // a V^T tile of 64 keys in LDS, each wave owns 32 queries of one head.
+#include <type_traits>
+
 #include "elem.h"
 
 namespace skyrl {
@@ -538,19 +540,47 @@ __device__ __forceinline__ s16x8 key_chunk(const uint16_t* nope, const uint16_t*
     return f;
 }
 
+// LDS reads that the compiler does not know as such: it would have them wait for every direct load under way. They are waited for
+// by count, and their registers tied past the wait.
+__device__ __forceinline__ void lds_read(s16x8& v, uint32_t at, int offset) {
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(at), "n"(offset));
+}
+__device__ __forceinline__ void lds_wait(s16x8& v, int left) {  // left: of the reads behind it that may be under way
+    asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(v) : "n"(left) : "memory");
+}
+// the largest of the lanes c, c + 16, c + 32, c + 48
+__device__ __forceinline__ float rows_max(float v) {
+    const uint32_t u = __float_as_uint(v);
+    const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    const uint32_t t = __float_as_uint(fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1])));
+    const auto b = __builtin_amdgcn_permlane32_swap(t, t, false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+typedef __attribute__((address_space(3))) void lds_void;
+typedef __attribute__((address_space(1))) void gbl_void;
+__device__ const uint4 kNoKey = {0u, 0u, 0u, 0u};
+
 // QT: 16-query tiles per wave, 128 queries per workgroup. VEC: every row piece is 16-byte aligned.
+// A tile of 64 keys is in pieces of 1 KB: 8 key rows of 64 columns or 8 value rows (of V^T) of 64 keys, whole 128-byte lines, by
+// direct loads into one of two buffers while the other is worked on: one barrier a tile, and at dk = 192, vdim = 128 two workgroups
+// fill a CU's LDS. In the scores' product row r of 16-row tile t is key 32 (t / 2) + 8 (r / 4) + 4 (t % 2) + r % 4, so that a lane's
+// weights are of 8 keys in a row, which one 16-byte read of V^T gives; 16-byte chunks are swizzled for both reads. Bound: the
+// matrix cores', the LDS reads' and the vector units' time, of which two waves a SIMD overlap a part. 16 heads, dk 192, vdim 128,
+// window 1024, us: one prompt of 8192 109, eight of 341 to 1024 51, three of 300 to 700 25.5; dk 256, vdim 256, one of 1500 49.5. (Tiles
+// staged through 40 registers a lane in lines cut in two, two barriers a tile, operands read where they were used, masks formed for
+// every tile: 150, 70, 35.5, 84. Without exponentials 98, with all tiles in L2 99, without the scores' products 85.)
 template <int NK, int NV, int QT, bool VEC>
 __global__ __launch_bounds__(512 / QT) __attribute__((amdgpu_waves_per_eu(2))) void latent_prefill_kernel(
     const uint16_t* __restrict__ q, int64_t q_stride, const uint16_t* __restrict__ k_nope, int64_t k_stride,
     const uint16_t* __restrict__ k_rot, const uint16_t* __restrict__ v_t, int64_t vt_stride,
     const int32_t* __restrict__ tiles, int heads, int dim, int rot, int vdim, float scale_log2, int window,
     HeadEnd<uint16_t> end, uint16_t* __restrict__ out, int64_t out_stride) {
-    constexpr int NT = 512 / QT, QW = 16 * QT;
-    constexpr int LDK = NK * 32 + 8, LDV = kKT + 8;
-    constexpr int TPK = NT / kKT, KPT = NK * 4 / TPK;     // threads per key row, 16-byte chunks per thread
-    constexpr int VPT = NV * 16 * (kKT / 8) / NT, VROWS = NT / 8;
-    __shared__ __attribute__((aligned(16))) uint16_t s_k[kKT * LDK];
-    __shared__ __attribute__((aligned(16))) uint16_t s_v[NV * 16 * LDV];
+    constexpr int NT = 512 / QT, NW = NT / kWave, QW = 16 * QT;
+    constexpr int KG = NK / 2, KB = KG * kKT * 128, VB = NV * 16 * 128, BUF = KB + VB;  // 64-column groups; bytes
+    constexpr int KPW = KG * 8 / NW, VPW = NV * 2 / NW;                                  // pieces per wave
+    static_assert(NK % 2 == 0 && KG * 8 % NW == 0 && NV * 2 % NW == 0 && kKT == 64, "whole pieces");
+    static_assert(2 * BUF <= 160 * 1024 && BUF <= 65536, "LDS; offsets of the reads");
+    __shared__ __attribute__((aligned(16))) char smem[2 * BUF];
     const int h = blockIdx.x % heads;  // one head's tiles stay on one XCD when heads is a multiple of 8
     const int32_t* tl = tiles + 8 * (blockIdx.x / heads);
     const int tok0 = tl[0], ntok = tl[1], pos0 = tl[2], seg_row = tl[3], seg_pos = tl[4];
@@ -571,9 +601,14 @@ __global__ __launch_bounds__(512 / QT) __attribute__((amdgpu_waves_per_eu(2))) v
         for (int s = 0; s < NK; ++s) {
             s16x8 f = {0, 0, 0, 0, 0, 0, 0, 0};
             if (ok) f = key_chunk<VEC>(qr, qr + dim, 32 * s + 8 * g, dim, rot);
+            if (!(scale_log2 > 0.f)) {  // the largest score is the largest product's: a scale below 0 turns the queries instead
+#pragma unroll
+                for (int i = 0; i < 8; ++i) f[i] = scale_log2 < 0.f ? f[i] ^ (short)0x8000 : scale_log2 == 0.f ? (short)0 : f[i];
+            }
             qf[qq][s] = f;
         }
     }
+    scale_log2 = scale_log2 == 0.f ? 1.f : fabsf(scale_log2);
     f32x4 o[NV][QT];
 #pragma unroll
     for (int n = 0; n < NV; ++n)
@@ -590,102 +625,144 @@ __global__ __launch_bounds__(512 / QT) __attribute__((amdgpu_waves_per_eu(2))) v
     const int j0 = (lo - seg_pos) / kKT, j1 = (pos0 + ntok - 1 - seg_pos) / kKT;
     const int wq0 = pos0 + QW * wave;                                // the wave's first query
     const int wq1 = min(wq0 + QW - 1, pos0 + ntok - 1);                  // and its last
-    s16x8 kr[KPT], vr[VPT];
-    const int ktok = threadIdx.x / TPK, kd = (threadIdx.x % TPK) * 8;   // key row and first column of this thread
-    const int vd = threadIdx.x >> 3, vtok = (threadIdx.x & 7) * 8;      // value row and first key
+
+    // Pieces: this lane's 16 bytes of row lane / 8. Key row r has its chunk x at x ^ key_swizzle(r), value row d at x ^ d % 8.
+    const int r8 = lane >> 3;
+    auto key_swizzle = [](int r) { return ((r & 3) >> 1) | ((r >> 3 & 3) << 1); };
+    auto piece = [&](int i) { return wave + NW * i; };  // the wave's i-th: of keys 8-row group % 8, column group / 8
+    auto kcol = [&](int i) { return 64 * (piece(i) / 8) + 8 * ((lane & 7) ^ key_swizzle(piece(i) % 8 * 8 + r8)); };
+    s16x8 kr[VEC ? 1 : KPW];
     auto fetch = [&](int j) {
+        char* dst = smem + (j - j0 & 1) * BUF;
         const int64_t r0 = seg_row + (int64_t)j * kKT;
-        const uint16_t* kp = k_nope + (r0 + ktok) * k_stride + (int64_t)h * dim;
-        const uint16_t* rp = k_rot + (r0 + ktok) * rot;
 #pragma unroll
-        for (int i = 0; i < KPT; ++i) kr[i] = key_chunk<VEC>(kp, rp, kd + 8 * TPK * i, dim, rot);
-        const uint16_t* vp = v_t + ((int64_t)h * vdim + vd) * vt_stride + r0 + vtok;
+        for (int i = 0; i < KPW; ++i) {
+            const int64_t row = r0 + piece(i) % 8 * 8 + r8;
+            const int d = kcol(i);
+            const uint16_t *kp = k_nope + row * k_stride + (int64_t)h * dim, *rp = k_rot + row * rot;
+            if constexpr (VEC) {
+                const void* src = d < dim ? (const void*)(kp + d) : d < dk ? (const void*)(rp + (d - dim)) : (const void*)&kNoKey;
+                __builtin_amdgcn_global_load_lds((gbl_void*)src, (lds_void*)(dst + piece(i) * 1024), 16, 0, 0);
+            } else {
+                kr[i] = key_chunk<false>(kp, rp, d, dim, rot);
+            }
+        }
+        const uint16_t* vp = v_t + (int64_t)h * vdim * vt_stride + r0 + 8 * ((lane & 7) ^ r8);
 #pragma unroll
-        for (int i = 0; i < VPT; ++i) {
-            vr[i] = s16x8{0, 0, 0, 0, 0, 0, 0, 0};
-            if (vd + VROWS * i < vdim) vr[i] = *reinterpret_cast<const s16x8*>(vp + (int64_t)VROWS * i * vt_stride);
+        for (int i = 0; i < VPW; ++i) {  // rows past the last: the last, whose sums nothing reads
+            const int d = min(piece(i) * 8 + r8, vdim - 1);
+            __builtin_amdgcn_global_load_lds((gbl_void*)(vp + d * vt_stride), (lds_void*)(dst + KB + piece(i) * 1024), 16, 0, 0);
         }
     };
+    const uint32_t lds = (uint32_t)(uintptr_t)(lds_void*)smem;
+    const int krow = 8 * (c >> 2) + (c & 3);  // of tile t: + 32 (t / 2) + 4 (t % 2)
+    const uint32_t ka[2] = {lds + krow * 128 + ((g ^ key_swizzle(krow)) * 16), lds + krow * 128 + (((4 + g) ^ key_swizzle(krow)) * 16)};
+    const uint32_t va[2] = {lds + KB + c * 128 + ((g ^ (c & 7)) * 16), lds + KB + c * 128 + (((4 + g) ^ (c & 7)) * 16)};
     fetch(j0);
     for (int j = j0; j <= j1; ++j) {
-        __syncthreads();  // the previous tile is consumed
+        const uint32_t buf = (j - j0 & 1) * BUF;
+        if constexpr (!VEC) {
 #pragma unroll
-        for (int i = 0; i < KPT; ++i) *reinterpret_cast<s16x8*>(&s_k[ktok * LDK + kd + 8 * TPK * i]) = kr[i];
-#pragma unroll
-        for (int i = 0; i < VPT; ++i) *reinterpret_cast<s16x8*>(&s_v[(vd + VROWS * i) * LDV + vtok]) = vr[i];
-        __syncthreads();
+            for (int i = 0; i < KPW; ++i) *reinterpret_cast<s16x8*>(smem + buf + piece(i) * 1024 + lane * 16) = kr[i];
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();  // this tile is there, the one before consumed
         if (j < j1) fetch(j + 1);
         const int kp0 = seg_pos + j * kKT, kp1 = kp0 + kKT - 1;
         if (kp0 > wq1 || kp1 < wq0 - w + 1 || wq0 > wq1) continue;  // no key of this tile for this wave
         const bool edge = kp1 > wq0 || kp0 < wq1 - w + 1 || wq1 != wq0 + QW - 1;
+        // key rows are read AHEAD products ahead, the first value rows while the scores become weights
+        constexpr int AHEAD = QT == 1 ? 8 : 5, VAHEAD = 3;
         f32x4 sc[4][QT];
 #pragma unroll
         for (int tt = 0; tt < 4; ++tt)
 #pragma unroll
             for (int qq = 0; qq < QT; ++qq) sc[tt][qq] = f32x4{0.f, 0.f, 0.f, 0.f};
+        s16x8 kf[AHEAD + 1], vf[VAHEAD + 1][2];
+        auto key = [&](int f) {  // step f / 4, tile f % 4
+            lds_read(kf[f % (AHEAD + 1)], ka[f / 4 & 1] + buf, (f / 8) * (kKT * 128) + (f % 4 / 2) * 4096 + (f & 1) * 512);
+        };
+        auto values = [&](int n) {
+            lds_read(vf[n % (VAHEAD + 1)][0], va[0] + buf, n * 2048);
+            lds_read(vf[n % (VAHEAD + 1)][1], va[1] + buf, n * 2048);
+        };
 #pragma unroll
-        for (int s = 0; s < NK; ++s) {
+        for (int f = 0; f < AHEAD; ++f) key(f);
 #pragma unroll
-            for (int tt = 0; tt < 4; ++tt) {
-                const s16x8 kf = *reinterpret_cast<const s16x8*>(&s_k[(16 * tt + c) * LDK + 32 * s + 8 * g]);
-#pragma unroll
-                for (int qq = 0; qq < QT; ++qq)
-                    sc[tt][qq] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[qq][s], sc[tt][qq], 0, 0, 0);
+        for (int f = 0; f < 4 * NK; ++f) {
+            s16x8& k = kf[f % (AHEAD + 1)];
+            if (f + AHEAD < 4 * NK) {
+                key(f + AHEAD);
+                lds_wait(k, AHEAD);
+            } else {
+                lds_wait(k, 4 * NK - 1 - f);
             }
+#pragma unroll
+            for (int qq = 0; qq < QT; ++qq)
+                sc[f % 4][qq] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k, qf[qq][f / 4], sc[f % 4][qq], 0, 0, 0);
         }
+#pragma unroll
+        for (int n = 0; n < VAHEAD; ++n) values(n);
         s16x8 pf[QT][2];  // [query tile][32-key step]
         float alpha[QT];
+        auto weights = [&](auto masked) {  // masked: some key of the tile is after a query or too far back
 #pragma unroll
-        for (int qq = 0; qq < QT; ++qq) {
-            float bm = -INFINITY;
-            const unsigned dist = qpos[qq] - kp0 - 4 * g;  // to the lane's first key
+            for (int qq = 0; qq < QT; ++qq) {
+                float bm = -INFINITY;
+                const unsigned dist = qpos[qq] - kp0 - 8 * g;  // to the lane's first key
 #pragma unroll
-            for (int tt = 0; tt < 4; ++tt)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    float v = sc[tt][qq][i] * scale_log2;
-                    if (edge && dist - (16 * tt + i) >= (unsigned)w) v = -INFINITY;  // after the query, or too far back
-                    sc[tt][qq][i] = v;
-                    bm = fmaxf(bm, v);
-                }
-            bm = fmaxf(bm, __shfl_xor(bm, 16, kWave));
-            bm = fmaxf(bm, __shfl_xor(bm, 32, kWave));
-            const float mn = fmaxf(m[qq], bm);
-            const float base = mn == -INFINITY ? 0.f : mn;  // no key seen yet: every weight is 0
-            alpha[qq] = fast_exp2(m[qq] - base);
-            float sum = 0.f;
-#pragma unroll
-            for (int kk = 0; kk < 2; ++kk) {
-                uint32_t pk[4];
-#pragma unroll
-                for (int b = 0; b < 2; ++b) {
-                    float p[4];
+                for (int tt = 0; tt < 4; ++tt)
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        p[i] = fast_exp2(sc[2 * kk + b][qq][i] - base);
-                        sum += p[i];
+                        if (decltype(masked)::value && dist - (32 * (tt / 2) + 4 * (tt % 2) + i) >= (unsigned)w) sc[tt][qq][i] = -INFINITY;
+                        bm = fmaxf(bm, sc[tt][qq][i]);
                     }
-                    pk[2 * b] = pack_bf16x2(p[0], p[1]);
-                    pk[2 * b + 1] = pack_bf16x2(p[2], p[3]);
+                bm = rows_max(bm) * scale_log2;
+                const float mn = fmaxf(m[qq], bm);
+                const float base = mn == -INFINITY ? 0.f : mn;  // no key seen yet: every weight is 0
+                alpha[qq] = fast_exp2(m[qq] - base);
+                float sum = 0.f;
+#pragma unroll
+                for (int kk = 0; kk < 2; ++kk) {
+                    uint32_t pk[4];
+#pragma unroll
+                    for (int b = 0; b < 2; ++b) {
+                        float p[4];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            p[i] = fast_exp2(fmaf(sc[2 * kk + b][qq][i], scale_log2, -base));
+                            sum += p[i];
+                        }
+                        pk[2 * b] = pack_bf16x2(p[0], p[1]);
+                        pk[2 * b + 1] = pack_bf16x2(p[2], p[3]);
+                    }
+                    pf[qq][kk] = __builtin_bit_cast(s16x8, make_uint4(pk[0], pk[1], pk[2], pk[3]));
                 }
-                pf[qq][kk] = __builtin_bit_cast(s16x8, make_uint4(pk[0], pk[1], pk[2], pk[3]));
+                l[qq] = l[qq] * alpha[qq] + sum;
+                m[qq] = mn;
             }
-            l[qq] = l[qq] * alpha[qq] + sum;
-            m[qq] = mn;
+        };
+        if (edge) weights(std::true_type{});
+        else weights(std::false_type{});
+        bool same = true;  // no maximum has moved: factors of 1
+#pragma unroll
+        for (int qq = 0; qq < QT; ++qq) same &= alpha[qq] == 1.f;
+        if (!__all(same)) {
+#pragma unroll
+            for (int n = 0; n < NV; ++n)
+#pragma unroll
+                for (int qq = 0; qq < QT; ++qq) o[n][qq] = o[n][qq] * alpha[qq];
         }
 #pragma unroll
         for (int n = 0; n < NV; ++n) {
-#pragma unroll
-            for (int qq = 0; qq < QT; ++qq) o[n][qq] = o[n][qq] * alpha[qq];
+            s16x8(&v)[2] = vf[n % (VAHEAD + 1)];
+            if (n + VAHEAD < NV) values(n + VAHEAD);
 #pragma unroll
             for (int kk = 0; kk < 2; ++kk) {
-                const uint16_t* vp = &s_v[(16 * n + c) * LDV + 32 * kk + 4 * g];
-                const s16x4 v0 = *reinterpret_cast<const s16x4*>(vp);
-                const s16x4 v1 = *reinterpret_cast<const s16x4*>(vp + 16);
-                const s16x8 vf = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
+                lds_wait(v[kk], 2 * (min(n + VAHEAD, NV - 1) - n) + 1 - kk);
 #pragma unroll
                 for (int qq = 0; qq < QT; ++qq)
-                    o[n][qq] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[qq][kk], o[n][qq], 0, 0, 0);
+                    o[n][qq] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[kk], pf[qq][kk], o[n][qq], 0, 0, 0);
             }
         }
     }

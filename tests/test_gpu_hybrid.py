@@ -192,6 +192,27 @@ def test_latent_prefill(heads, dim, rot, vdim, rank, window, segs):
         tok += n
 
 
+@pytest.mark.parametrize("dim,rot,vdim", [(40, 24, 72), (64, 64, 64), (128, 64, 128), (128, 64, 100), (200, 56, 250), (20, 12, 28)])
+def test_latent_prefill_over_many_tiles(dim, rot, vdim):
+    """Both tile buffers again and again: the same bits every time, also after another head count has used the LDS; a scale below
+    0 is that of the negated queries, one of 0 gives the mean of the keys in sight."""
+    g = torch.Generator().manual_seed(dim)
+    heads, T, window = 3, 900, 333
+    seg, tiles, rows, _ = mixers.prompt_plan([T], [0], 0, 0, window)
+    q, kn, kr, vt = (rnd(g, *s, dtype=torch.bfloat16).to(DEV) for s in ((T, heads * (dim + rot)), (rows, heads * dim), (rows, rot),
+                                                                       (heads * vdim, rows)))
+    t = torch.from_numpy(tiles).to(DEV)
+    run = lambda qq, s: lk.latent_prefill(qq, kn, kr, vt, t, heads, dim, rot, vdim, s, window,  # noqa: E731
+                                          torch.zeros(T, heads * vdim, dtype=torch.bfloat16, device=DEV))
+    first = run(q, 0.1)
+    for _ in range(3):
+        assert torch.equal(run(q, 0.1), first)
+    assert torch.equal(run(-q, -0.1), first)
+    d = torch.arange(T)[:, None] - torch.arange(T)[None]
+    sight = ((d >= 0) & (d < window)).double()
+    close(run(q, 0.0), (sight / sight.sum(1, keepdim=True)) @ vt[:, :T].double().cpu().t(), torch.bfloat16)
+
+
 # ---------------------------------------------------------------- gated delta rule
 DELTA = [  # heads, kv_heads, dim, vdim, taps
     (4, 2, 24, 36, 3), (3, 1, 64, 48, 3), (2, 2, 128, 128, 4), (3, 3, 18, 10, 1), (2, 1, 200, 130, 9), (1, 1, 16, 200, 2),
