@@ -141,46 +141,29 @@ __global__ __launch_bounds__(kNT) void moe_route_plain_kernel(Router ro, const T
 }
 
 // bf16, width a multiple of 8, at most 16 NE experts (rows past the last: the last again): 16 tokens per workgroup, the
-// width in shares of NWV waves, U steps of 32 in flight.
-template <int NE, int NWV, int U>
+// width in shares of NWV waves, each summed in order and then in turn. Bound: what a CU reads of the router (256 KB at 64 experts
+// of 2048), so whole lines through LDS (stream.h): as operands from memory, 16 half lines an instruction, they came at a quarter
+// of the rate. 64 experts, us (and so): width 2048, 256 tokens 8.0 (14.0), 1563 8.3 (14.4), 5637 16.8 (24.1); width 4096, 1563 11.8 (23.2).
+template <int NE, int NWV, int S>
 __global__ __launch_bounds__(NWV * kWave) void moe_route_kernel(Router ro, const uint16_t* __restrict__ x, int n,
                                                                 int width, const uint16_t* __restrict__ w,
                                                                 const float* __restrict__ correction,
                                                                 int32_t* __restrict__ idx, float* __restrict__ weight) {
-    constexpr int E16 = NE * 16, LZ = E16 + 4, EP = (E16 + kWave - 1) / kWave;
-    __shared__ __attribute__((aligned(16))) float s_z[NWV][16 * LZ];
+    using St = Stream<NE, 1, NWV, S>;
+    constexpr int E16 = NE * 16, LZ = St::LR, EP = (E16 + kWave - 1) / kWave;
+    __shared__ __attribute__((aligned(16))) uint16_t smem[St::kLds];
+    float(*s_z)[16 * LZ] = reinterpret_cast<float(*)[16 * LZ]>(smem);  // the shares' sums, where the pieces were
     float* own = s_z[1] + (threadIdx.x >> 6) * 3 * E16;  // a wave's scores, once the shares are summed
     static_assert((NWV - 1) * 16 * LZ >= NWV * 3 * E16, "room for the scores");
     const int t0 = blockIdx.x * 16;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int c = lane & 15, g = lane >> 4;
-    f32x4 acc[NE];
-#pragma unroll
-    for (int k = 0; k < NE; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const uint16_t* xr = x + (int64_t)min(t0 + c, n - 1) * width;
-    const uint16_t* wr[NE];
-#pragma unroll
-    for (int k = 0; k < NE; ++k) wr[k] = w + (int64_t)min(16 * k + c, ro.experts - 1) * width;
     const int steps = (width + 31) / 32, share = (steps + NWV - 1) / NWV;
-    const int s1 = min(steps, (wave + 1) * share);
-    for (int s = wave * share; s < s1; s += U) {
-        s16x8 xf[U], wf[U][NE];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int k0 = 32 * (s + u) + 8 * g, at = min(k0, width - 8);
-            xf[u] = *reinterpret_cast<const s16x8*>(xr + at);
-#pragma unroll
-            for (int k = 0; k < NE; ++k) wf[u][k] = *reinterpret_cast<const s16x8*>(wr[k] + at);
-            if (k0 >= width || s + u >= s1) xf[u] = s16x8{0, 0, 0, 0, 0, 0, 0, 0};  // the router's weights are finite
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-            for (int k = 0; k < NE; ++k) acc[k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u][k], xf[u], acc[k], 0, 0, 0);
-    }
-#pragma unroll
-    for (int k = 0; k < NE; ++k) *reinterpret_cast<f32x4*>(&s_z[wave][c * LZ + 16 * k + 4 * g]) = acc[k];
-    __syncthreads();
+    const int k0 = min(width, 32 * wave * share), k1 = min(width, 32 * (wave + 1) * share);
+    f32x4 acc[1][NE];
+    St::run(
+        smem, k1 - k0, 0, (k1 - k0 + 63) / 64, [&](int r) { return w + (int64_t)min(r, ro.experts - 1) * width + k0; },
+        [&](int r) { return x + (int64_t)min(t0 + r, n - 1) * width + k0; }, acc);
+    St::store(smem, acc);
     for (int e = threadIdx.x; e < 16 * E16; e += NWV * kWave) {
         const int at = e / E16 * LZ + e % E16;
         float z = 0.f;
@@ -663,14 +646,14 @@ extern "C" int skyrl_moe_route(const skyrl_moe_shape* shape, const void* x, int3
         const uint16_t* x_ = reinterpret_cast<const uint16_t*>(x);
         const uint16_t* w_ = reinterpret_cast<const uint16_t*>(router);
         const dim3 grid((n + 15) / 16);
-#define LAUNCH_ROUTE(NE, NWV, U)                                                                                     \
-    hipLaunchKernelGGL((moe_route_kernel<NE, NWV, U>), grid, dim3(NWV * kWave), 0, s, ro, x_, n, W, w_, correction, idx, \
+#define LAUNCH_ROUTE(NE, NWV, S)                                                                                     \
+    hipLaunchKernelGGL((moe_route_kernel<NE, NWV, S>), grid, dim3(NWV * kWave), 0, s, ro, x_, n, W, w_, correction, idx, \
                        weight)
-        if (ro.experts <= 16) LAUNCH_ROUTE(1, 16, 4);
-        else if (ro.experts <= 32) LAUNCH_ROUTE(2, 16, 4);
-        else if (ro.experts <= 64) LAUNCH_ROUTE(4, 16, 4);
-        else if (ro.experts <= 128) LAUNCH_ROUTE(8, 8, 4);
-        else LAUNCH_ROUTE(16, 4, 4);
+        if (ro.experts <= 16) LAUNCH_ROUTE(1, 16, 2);
+        else if (ro.experts <= 32) LAUNCH_ROUTE(2, 16, 1);
+        else if (ro.experts <= 64) LAUNCH_ROUTE(4, 16, 1);
+        else if (ro.experts <= 128) LAUNCH_ROUTE(8, 8, 1);
+        else LAUNCH_ROUTE(16, 4, 1);
         return check_launch("moe_route_kernel");
     }
     SKYRL_DISPATCH_T(dtype, {
