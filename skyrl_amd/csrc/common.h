@@ -138,6 +138,84 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
+// Exchanges between lanes l and l ^ O without LDS (a shuffle is an LDS round trip, some 130 cycles; these are one or two vector
+// instructions). All 64 lanes active. lane_add<O>(v) is v + __shfl_xor(v, O) bit for bit, wave_total(v) wave_sum(v).
+template <int O>
+__device__ __forceinline__ float lane_other(float v) {  // the value of lane l ^ O
+    const int x = __float_as_int(v);
+    if constexpr (O == 1) return __int_as_float(__builtin_amdgcn_update_dpp(0, x, 0xB1, 0xF, 0xF, false));
+    else if constexpr (O == 2) return __int_as_float(__builtin_amdgcn_update_dpp(0, x, 0x4E, 0xF, 0xF, false));
+    else if constexpr (O == 4) {  // banks of four lanes: 0 and 2 from the right, 1 and 3 from the left
+        const int y = __builtin_amdgcn_update_dpp(0, x, 0x104, 0xF, 0x5, false);
+        return __int_as_float(__builtin_amdgcn_update_dpp(y, x, 0x114, 0xF, 0xA, false));
+    } else if constexpr (O == 8) return __int_as_float(__builtin_amdgcn_update_dpp(0, x, 0x128, 0xF, 0xF, false));
+    else if constexpr (O == 16) {
+        const auto p = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)x, false, false);
+        return __uint_as_float(threadIdx.x & 16 ? p[0] : p[1]);
+    } else {
+        static_assert(O == 32, "a power of two below 64");
+        const auto p = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)x, false, false);
+        return __uint_as_float(threadIdx.x & 32 ? p[0] : p[1]);
+    }
+}
+template <int O, class F>
+__device__ __forceinline__ float lane_pair(float v, F f) {  // f of both values, commutative
+    if constexpr (O == 16) {
+        const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        return f(__uint_as_float(p[0]), __uint_as_float(p[1]));
+    } else if constexpr (O == 32) {
+        const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        return f(__uint_as_float(p[0]), __uint_as_float(p[1]));
+    } else {
+        return f(v, lane_other<O>(v));
+    }
+}
+template <int O>
+__device__ __forceinline__ float lane_add(float v) {
+    return lane_pair<O>(v, [](float a, float b) { return a + b; });
+}
+template <int O>
+__device__ __forceinline__ float lane_max(float v) {
+    return lane_pair<O>(v, [](float a, float b) { return fmaxf(a, b); });
+}
+// sums over the lanes first, 2 first, .. 32 apart (first: a power of two), in that order
+__device__ __forceinline__ float lanes_add_from(float v, int first) {
+    if (first <= 1) v = lane_add<1>(v);
+    if (first <= 2) v = lane_add<2>(v);
+    if (first <= 4) v = lane_add<4>(v);
+    if (first <= 8) v = lane_add<8>(v);
+    if (first <= 16) v = lane_add<16>(v);
+    if (first <= 32) v = lane_add<32>(v);
+    return v;
+}
+template <class F>
+__device__ __forceinline__ float half_fold(float v, F f) {  // pairs 16, 8, .. 1 apart
+    v = lane_pair<16>(v, f);
+    v = lane_pair<8>(v, f);
+    // the halves of a row of 16 are equal by now: a rotation by 4 meets what lane l ^ 4 holds
+    v = f(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124, 0xF, 0xF, false)));
+    v = lane_pair<2>(v, f);
+    return lane_pair<1>(v, f);
+}
+__device__ __forceinline__ float wave_total(float v) {
+    return half_fold(lane_add<32>(v), [](float a, float b) { return a + b; });
+}
+__device__ __forceinline__ float wave_largest(float v) {
+    return half_fold(lane_max<32>(v), [](float a, float b) { return fmaxf(a, b); });
+}
+__device__ __forceinline__ float wave_dot(float a, float b) {  // of a b, the lane's own product unrounded in the first sum
+    return half_fold(fmaf(a, b, lane_other<32>(a * b)), [](float x, float y) { return x + y; });
+}
+__device__ __forceinline__ int wave_scan(int v) {  // inclusive sums over the lanes
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);  // row_shr 1, 2, 4, 8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // row_bcast 15, 31
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);
+    return v;
+}
+
 // Wave-wide max broadcast as a wave-uniform value, without LDS: DPP quad_perm xor1/xor2 and
 // row_ror 4/8 give every lane its 16-lane row max (out-of-row sources keep -inf), then the
 // four row maxima are read with v_readlane. Requires all 64 lanes active.

@@ -143,7 +143,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void de
             const float* b = wave == 0 ? s_q : s_k;
             float x = 0.f;
             for (int i = lane; i < D; i += kWave) x += a[i] * b[i];
-            x = wave_sum(x);
+            x = wave_total(x);
             if (lane == 0) s_n[wave] = x;
         }
         __syncthreads();
@@ -169,12 +169,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void de
                 }
             }
             if (fold)  // the wave's own row groups first
-                for (int o = NC; o < kWave; o <<= 1) {
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        a[j] += __shfl_xor(a[j], o, kWave);
-                        b[j] += __shfl_xor(b[j], o, kWave);
-                    }
+                for (int j = 0; j < 4; ++j) {
+                    a[j] = lanes_add_from(a[j], NC);
+                    b[j] = lanes_add_from(b[j], NC);
                 }
             if (!fold || lane < NC) {
                 const int rec = fold ? wave : rg;
@@ -210,7 +208,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void de
         if (wave * kWave < V) {
             float x = 0.f;
             for (int i = lane; i < V; i += kWave) x += s_o[i] * s_o[i];
-            x = wave_sum(x);
+            x = wave_total(x);
             const float r = 1.f / sqrtf(x / (float)V + d.eps);
             T* dst = out + (int64_t)t * out_stride + h * V;
             if (tid < V) st(dst + tid, s_o[tid] * r * nw * siluf_(gate));

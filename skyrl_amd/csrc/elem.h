@@ -85,7 +85,7 @@ __device__ __forceinline__ float softplusf_(float x) { return fmaxf(x, 0.f) + lo
 // Sum over a block of NT threads, in every thread; lds holds NT / 64 floats and is free again on return.
 template <int NT>
 __device__ __forceinline__ float block_total(float v, float* lds) {
-    v = wave_sum(v);
+    v = wave_total(v);
     if ((threadIdx.x & (kWave - 1)) == 0) lds[threadIdx.x / kWave] = v;
     __syncthreads();
     float s = 0.f;

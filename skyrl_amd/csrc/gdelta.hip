@@ -118,7 +118,7 @@ __global__ __launch_bounds__(NT) void gdelta_scan_kernel(Dims d, In<T> in, const
             s_a[tid] = a * k;
             s_v[tid] = ch ? v_ : 0.f;
         }
-        const float kk = wave_sum(k * k), ra = wave_sum(r * a * k), rk = wave_sum(r * k);
+        const float kk = wave_dot(k, k), ra = wave_dot(r * a, k), rk = wave_dot(r, k);
         if (lane == 0) {
             s_n[4 * wave] = kk;
             s_n[4 * wave + 1] = ra;
@@ -149,12 +149,10 @@ __global__ __launch_bounds__(NT) void gdelta_scan_kernel(Dims d, In<T> in, const
                 }
             }
             if (fold)  // the wave's own row groups first
-                for (int o = NC; o < kWave; o <<= 1) {
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        z[j] += __shfl_xor(z[j], o, kWave);
-                        y[j] += __shfl_xor(y[j], o, kWave);
-                    }
+                for (int j = 0; j < 4; ++j) {
+                    z[j] = lanes_add_from(z[j], NC);
+                    y[j] = lanes_add_from(y[j], NC);
                 }
             if (!fold || lane < NC) {
                 const int rec = fold ? wave : rg;
@@ -190,7 +188,7 @@ __global__ __launch_bounds__(NT) void gdelta_scan_kernel(Dims d, In<T> in, const
             }
             o = Y - dra * un * un * Z + drk * s_v[tid];
         }
-        const float ss = wave_sum(o * o);
+        const float ss = wave_dot(o, o);
         if (lane == 0) s_n[4 * wave + 3] = ss;
         __syncthreads();
         float tot = 0.f;

@@ -362,8 +362,7 @@ __global__ __launch_bounds__(kNT * HG) __attribute__((amdgpu_waves_per_eu(1, 2))
         float bm = -INFINITY;
 #pragma unroll
         for (int w = 0; w < 4; ++w) bm = fmaxf(bm, fmaxf(fmaxf(x[w][0], x[w][1]), fmaxf(x[w][2], x[w][3])));
-        bm = fmaxf(bm, __shfl_xor(bm, 16, kWave));
-        bm = fmaxf(bm, __shfl_xor(bm, 32, kWave));
+        bm = lane_max<32>(lane_max<16>(bm));
         const float mn = fmaxf(m, bm);
         const float alpha = fast_exp2(m - mn);  // first tile: m = -inf, 0; every share starts with a visible key
         float sum = 0.f;
@@ -408,8 +407,7 @@ __global__ __launch_bounds__(kNT * HG) __attribute__((amdgpu_waves_per_eu(1, 2))
         }
         for (int j0 = 0; j0 < npw; j0 += 4) tile(w0, j0);
     }
-    l += __shfl_xor(l, 16, kWave);  // the sum over all keys, the same in every wave
-    l += __shfl_xor(l, 32, kWave);
+    l = lane_add<32>(lane_add<16>(l));  // the sum over all keys, the same in every wave
     const int h = h0 + 16 * hg + c;
     if (h >= heads) return;
     if (sp.parts == 1) {
@@ -456,10 +454,10 @@ __global__ __launch_bounds__(kWave * 2) void latent_merge_kernel(const float* __
     const int rp = ((rank + 15) / 16) * 16;
     float M = -INFINITY;
     for (int p = lane; p < sp.parts; p += kWave) M = fmaxf(M, ws_ml[(rec + p) * 2]);
-    M = wave_max(M);
+    M = wave_largest(M);
     float L = 0.f;
     for (int p = lane; p < sp.parts; p += kWave) L += fast_exp2(ws_ml[(rec + p) * 2] - M) * ws_ml[(rec + p) * 2 + 1];
-    const float inv = sum_factor(M, wave_sum(L), end.sink(h) * kLog2e) * end.gated(t, h);
+    const float inv = sum_factor(M, wave_total(L), end.sink(h) * kLog2e) * end.gated(t, h);
     uint16_t* orow = out + ((int64_t)h * ntok + t) * rank;
     for (int d = threadIdx.x * 4; d < rp; d += kWave * 8) {
         float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -547,14 +545,6 @@ __device__ __forceinline__ void lds_read(s16x8& v, uint32_t at, int offset) {
 }
 __device__ __forceinline__ void lds_wait(s16x8& v, int left) {  // left: of the reads behind it that may be under way
     asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(v) : "n"(left) : "memory");
-}
-// the largest of the lanes c, c + 16, c + 32, c + 48
-__device__ __forceinline__ float rows_max(float v) {
-    const uint32_t u = __float_as_uint(v);
-    const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-    const uint32_t t = __float_as_uint(fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1])));
-    const auto b = __builtin_amdgcn_permlane32_swap(t, t, false, false);
-    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
 typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((address_space(1))) void gbl_void;
@@ -717,7 +707,7 @@ __global__ __launch_bounds__(512 / QT) __attribute__((amdgpu_waves_per_eu(2))) v
                         if (decltype(masked)::value && dist - (32 * (tt / 2) + 4 * (tt % 2) + i) >= (unsigned)w) sc[tt][qq][i] = -INFINITY;
                         bm = fmaxf(bm, sc[tt][qq][i]);
                     }
-                bm = rows_max(bm) * scale_log2;
+                bm = lane_max<32>(lane_max<16>(bm)) * scale_log2;
                 const float mn = fmaxf(m[qq], bm);
                 const float base = mn == -INFINITY ? 0.f : mn;  // no key seen yet: every weight is 0
                 alpha[qq] = fast_exp2(m[qq] - base);
@@ -769,8 +759,7 @@ __global__ __launch_bounds__(512 / QT) __attribute__((amdgpu_waves_per_eu(2))) v
 #pragma unroll
     for (int qq = 0; qq < QT; ++qq) {
         float s = l[qq];
-        s += __shfl_xor(s, 16, kWave);
-        s += __shfl_xor(s, 32, kWave);
+        s = lane_add<32>(lane_add<16>(s));
         const int qi = QW * wave + 16 * qq + c;
         if (qi >= ntok) continue;
         const float inv = sum_factor(m[qq], s, end.sink(h) * kLog2e) * end.gated(tok0 + qi, h);

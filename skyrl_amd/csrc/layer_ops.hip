@@ -433,8 +433,14 @@ __global__ __launch_bounds__(NT) void gate_norm_add_kernel(GateNormAdd<T, A, Z> 
             return;
         }
 #pragma unroll
-        for (int k = 0; k < kMaxV; ++k)
-            for (int o = 1; o < L; o <<= 1) r[k] += __shfl_xor(r[k], o, kWave);
+        for (int k = 0; k < kMaxV; ++k) {
+            if (L > 1) r[k] = lane_add<1>(r[k]);
+            if (L > 2) r[k] = lane_add<2>(r[k]);
+            if (L > 4) r[k] = lane_add<4>(r[k]);
+            if (L > 8) r[k] = lane_add<8>(r[k]);
+            if (L > 16) r[k] = lane_add<16>(r[k]);
+            if (L > 32) r[k] = lane_add<32>(r[k]);
+        }
         if (sums > 1) {
             __syncthreads();  // the sums before these are read
 #pragma unroll

@@ -13,6 +13,8 @@
 // The products stage pieces of the rows and of the weight rows through LDS (16-byte direct loads, chunk index
 // xor-swizzled by the row so that the reads of 16 rows do not conflict), weights as the left operand: a lane holds
 // four consecutive columns of a token. Small tiles (decode) keep several stages in flight: they stream weights.
+#include <type_traits>
+
 #include "stream.h"
 #include "wide.h"
 
@@ -53,16 +55,22 @@ __device__ __forceinline__ void pick(const Router& ro, const float* z, const flo
     wave_lds_sync();
     if (EP == 1 && ro.keep < ro.groups && (per & (per - 1)) == 0) {  // an expert per lane, a group in neighbouring lanes
         float a = ch[0], b = -INFINITY;  // the two largest
-        for (int o = 1; o < per; o <<= 1) {
-            const float x = __shfl_xor(a, o, kWave), y = __shfl_xor(b, o, kWave);
+        auto join = [&](auto o) {
+            const float x = lane_other<o.value>(a), y = lane_other<o.value>(b);
             b = fmaxf(fminf(a, x), fmaxf(b, y));
             a = fmaxf(a, x);
-        }
+        };
+        if (per > 1) join(std::integral_constant<int, 1>{});
+        if (per > 2) join(std::integral_constant<int, 2>{});
+        if (per > 4) join(std::integral_constant<int, 4>{});
+        if (per > 8) join(std::integral_constant<int, 8>{});
+        if (per > 16) join(std::integral_constant<int, 16>{});
+        if (per > 32) join(std::integral_constant<int, 32>{});
         const float score = per > 1 ? a + b : a;
         const int q = lane / per;
         int better = 0;
         for (int i = 0; i < ro.groups; ++i) {
-            const float x = __shfl(score, i * per, kWave);
+            const float x = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(score), i * per));
             better += x > score || (x == score && i < q);
         }
         if (better >= ro.keep) ch[0] = -INFINITY;
@@ -220,12 +228,7 @@ __device__ __forceinline__ void sort_pairs(const int32_t* idx, int npairs, int e
     }
     // tiles before each expert: a scan over at most 1024 experts
     const int tiles = (cnt + tm - 1) / tm;
-    int x = tiles;
-#pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-        const int y = __shfl_up(x, o, kWave);
-        if (lane >= o) x += y;
-    }
+    const int x = wave_scan(tiles);
     if (lane == kWave - 1) s_sum[wave] = x;
     __syncthreads();
     int before = x - tiles, total = 0;

@@ -25,7 +25,8 @@ def _pairs(idx, order, tile_expert, tm):
 
 # groups of powers of two and others, one group, one expert per group, all kept, all experts chosen; rows on both sides of
 # what one launch sorts
-@pytest.mark.parametrize("experts,groups,keep,top", [(64, 8, 4, 8), (64, 1, 1, 6), (60, 12, 5, 7), (16, 16, 3, 3), (33, 3, 2, 22),
+@pytest.mark.parametrize("experts,groups,keep,top", [(64, 8, 4, 8), (64, 1, 1, 6), (60, 12, 5, 7), (64, 32, 9, 8), (64, 16, 5, 8),
+                                                     (64, 4, 2, 8), (64, 2, 1, 8), (64, 64, 20, 8), (16, 16, 3, 3), (33, 3, 2, 22),
                                                      (8, 2, 2, 8), (1, 1, 1, 1)])
 @pytest.mark.parametrize("n,shares", [(1, 1), (5, 3), (16, 2), (46, 8), (129, 2)])
 def test_choice(dev, experts, groups, keep, top, n, shares):

@@ -115,6 +115,21 @@ def test_norms_of_parts(dev, n, H, parts):
         torch.testing.assert_close(y.double(), norm(full) * nxt.double(), atol=1e-4, rtol=2 ** -8)
 
 
+@pytest.mark.parametrize("H,groups", [(2048, 256), (2048, 128), (2048, 64), (2048, 32), (2048, 16), (2048, 8), (2048, 4), (1536, 4), (4096, 2)])
+def test_norms_in_parts_of_any_size(dev, H, groups):
+    """Sums over 1, 2, 4, .. 64 neighbouring lanes, and over several such."""
+    g = torch.Generator(device=dev).manual_seed(groups)
+    r = lambda *s: torch.randn(*s, device=dev, generator=g)  # noqa: E731
+    n = 5
+    a, z, h, w, nxt, b = r(2 * n, H).bfloat16(), r(n, H).bfloat16(), r(n, H), r(H).bfloat16(), r(H).bfloat16(), r(H)
+    norm = lambda v: (v.view(n, groups, -1) / v.view(n, groups, -1).square().mean(-1, keepdim=True).add(1e-6).sqrt()).view(n, H)  # noqa: E731
+    full = h.double() + 0.5 * norm(a.double().view(n, 2, H).sum(1) * torch.sigmoid(z.double() + b.double())) * w.double()
+    got = h.clone()
+    y = lk.gate_norm_add(a, got, w, nxt, 1e-6, groups=groups, mult=0.5, parts=2, gate=z, gate_bias=b)
+    torch.testing.assert_close(got.double(), full, atol=2e-5, rtol=1e-5)
+    torch.testing.assert_close(y.double(), norm(full) * nxt.double(), atol=1e-4, rtol=2 ** -8)
+
+
 @pytest.mark.parametrize("B,n,N,K", [(16, 1, 512, 128), (3, 2, 40, 24), (5, 17, 130, 264), (2, 33, 24, 136), (4, 64, 128, 512),
                                      (3, 65, 50, 200), (2, 200, 72, 328), (1, 256, 16, 64)])
 def test_batch(dev, B, n, N, K):
