@@ -54,6 +54,13 @@ extern "C" {
  *                   of skyrl_gate_mul: w holds N gate rows, then N up rows; the gated product bf16 [n, N], splits 0.
  *                   skyrl_rows_product_fits: whether it takes the sizes and is the faster form of them (form 0:
  *                   rounded, 1: gated, 2: in splits); skyrl_rows_product_splits: the splits.
+ *                   skyrl_rows_product_tanh: columns [first, last) of the bf16 result through tanh. skyrl_rows_product_capped: no
+ *                   bias, the bf16 result as skyrl_softcap makes it, f32 [n, N] of row stride ldo.
+ *   skyrl_add_norm_product, skyrl_gate_norm_product  one row of a model in bf16: the norm of skyrl_add_norm_parts (parts 0: no
+ *                   sum) or skyrl_gate_norm_add_parts and skyrl_rows_product of the normed row, in one launch. The residual is
+ *                   read from h and leaves in h_out, another buffer; x_out (may be NULL): the normed row. turn0, turn1 as
+ *                   skyrl_rows_product_tanh's columns (equal: none; not with splits or act). skyrl_normed_product_fits: whether a
+ *                   row of K with that many shares (of the sum or of the gate's logits) and rows to be summed is taken.
  *   skyrl_gated_product  many rows: the gated product (act of skyrl_gate_mul) of x bf16 [n, K] (row stride ldx) and w bf16
  *                   [N gate rows, N up rows] (row stride ldw), rows 16-byte aligned, as bf16 [n, N] contiguous: summed and
  *                   gated in f32, rounded once. K a multiple of 64, N of 128. skyrl_gated_product_fits: whether it takes the
@@ -93,6 +100,27 @@ int32_t skyrl_rows_product_splits(int32_t n, int32_t K, int32_t N);
 int skyrl_rows_product(const void* x, int64_t ldx, int32_t n, int32_t K, const void* w, int64_t ldw, int32_t N,
                        const void* bias, int32_t act, float alpha, float limit, int32_t splits, void* out, int64_t ldo,
                        void* stream);
+int skyrl_rows_product_tanh(const void* x, int64_t ldx, int32_t n, int32_t K, const void* w, int64_t ldw, int32_t N,
+                            const void* bias, int32_t first, int32_t last, void* out, int64_t ldo, void* stream);
+int skyrl_rows_product_capped(const void* x, int64_t ldx, int32_t n, int32_t K, const void* w, int64_t ldw, int32_t N, float cap,
+                              float* out, int64_t ldo, void* stream);
+typedef struct {
+    const float* h;
+    float* h_out;
+    void* x_out;
+    const void* w;
+    int64_t ldw;
+    const void* bias;
+    void* out;
+    int32_t K, N, act, splits, turn0, turn1;
+    float alpha, limit;
+} skyrl_normed_product;
+int32_t skyrl_normed_product_fits(int32_t K, int32_t shares, int32_t rows);
+int skyrl_add_norm_product(const skyrl_normed_product* product, const float* delta, int32_t parts, const void* step,
+                           const void* weight, float w_base, float eps, int32_t kind, void* stream);
+int skyrl_gate_norm_product(const skyrl_normed_product* product, const void* a, int32_t a_shares, int32_t parts, const void* gate,
+                            int32_t gate_shares, int64_t gate_stride, const float* gate_bias, const void* weight, int32_t groups,
+                            float eps, float mult, const void* next, void* stream);
 int skyrl_rows_batch(const void* x, int64_t ldx, int64_t x_batch, int32_t n, int32_t K, const void* w, int64_t ldw,
                      int64_t w_batch, int32_t N, int32_t batch, void* out, int64_t ldo, int64_t out_batch, void* stream);
 int skyrl_rows_batch_in_order(const void* x, int64_t ldx, int64_t x_batch, int32_t n, int32_t K, const void* w, int64_t ldw,

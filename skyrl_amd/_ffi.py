@@ -271,6 +271,14 @@ class MoeShape(ctypes.Structure):
     _fields_ = [(n, ctypes.c_int32) for n in ("width", "ff", "experts", "top", "groups", "keep")]
 
 
+class NormedProduct(ctypes.Structure):
+    """Mirror of ``skyrl_normed_product`` (include/skyrl_layers.h)."""
+
+    _fields_ = [("h", _P), ("h_out", _P), ("x_out", _P), ("w", _P), ("ldw", _I64), ("bias", _P), ("out", _P)] + [
+        (n, ctypes.c_int32) for n in ("K", "N", "act", "splits", "turn0", "turn1")] + [
+        (n, ctypes.c_float) for n in ("alpha", "limit")]
+
+
 # the exported surface of include/skyrl_layers.h, in libraries of its own (LAYER_LIBS)
 _DS = ctypes.POINTER(DeltaShape)
 _FS = ctypes.POINTER(DiffShape)
@@ -278,6 +286,7 @@ _AS = ctypes.POINTER(AttnShape)
 _SS = ctypes.POINTER(SSDShape)
 _GS = ctypes.POINTER(GeneralDeltaShape)
 _MS = ctypes.POINTER(MoeShape)
+_NP = ctypes.POINTER(NormedProduct)
 LAYERS_SIGNATURES = {
     "skyrl_embed": (_INT, [_P, _P, _I64, _I32, _F, _P, _P, _P, _P, _I32, _P]),
     "skyrl_norm_add": (_INT, [_P, _P, _P, _P, _F, _P, _P, _I32, _P, _I32, _I32, _I32, _F, _P, _I32, _P]),
@@ -292,6 +301,11 @@ LAYERS_SIGNATURES = {
     "skyrl_rows_product_fits": (_I32, [_I32, _I32, _I32, _I32]),
     "skyrl_rows_product_splits": (_I32, [_I32, _I32, _I32]),
     "skyrl_rows_product": (_INT, [_P, _I64, _I32, _I32, _P, _I64, _I32, _P, _I32, _F, _F, _I32, _P, _I64, _P]),
+    "skyrl_rows_product_tanh": (_INT, [_P, _I64, _I32, _I32, _P, _I64, _I32, _P, _I32, _I32, _P, _I64, _P]),
+    "skyrl_rows_product_capped": (_INT, [_P, _I64, _I32, _I32, _P, _I64, _I32, _F, _P, _I64, _P]),
+    "skyrl_normed_product_fits": (_I32, [_I32, _I32, _I32]),
+    "skyrl_add_norm_product": (_INT, [_NP, _P, _I32, _P, _P, _F, _F, _I32, _P]),
+    "skyrl_gate_norm_product": (_INT, [_NP, _P, _I32, _I32, _P, _I32, _I64, _P, _P, _I32, _F, _F, _P, _P]),
     "skyrl_rows_batch": (_INT, [_P, _I64, _I64, _I32, _I32, _P, _I64, _I64, _I32, _I32, _P, _I64, _I64, _P]),
     "skyrl_rows_batch_in_order": (_INT, [_P, _I64, _I64, _I32, _I32, _P, _I64, _I64, _I32, _I32, _P, _I64, _I64, _P]),
     "skyrl_add_norm_parts": (_INT, [_P, _I32, _P, _P, _P, _F, _I32, _I32, _F, _I32, _P, _P]),

@@ -1,0 +1,80 @@
+// What the products of a few rows (rows_product.hip, normed_product.hip) share: their operands and what becomes of the sums.
+#pragma once
+#include "gate.h"
+#include "stream.h"
+
+namespace skyrl {
+
+enum Mode { kRound, kParts, kGated, kCapped };
+
+struct RowsProduct {
+    const uint16_t* x;
+    int64_t ldx;
+    int n, K;
+    const uint16_t* w;
+    int64_t ldw;
+    int N;  // output columns; kGated: gate rows, the up rows follow
+    const uint16_t* bias;
+    Gate gate;
+    int turn0, turn1;  // kRound: columns whose rounded values go through tanh
+    float cap;         // kCapped: the rounded values between -cap and cap by tanh, f32 (0: as they are)
+    void* out;
+    int64_t ldo, ldsplit;
+    int row_blocks;  // gridDim.z = batch row_blocks
+    int64_t x_batch, w_batch, out_batch;
+};
+
+template <int MODE, int NT>
+constexpr int out_cols() {  // of a workgroup
+    static_assert(MODE != kGated || NT % 2 == 0, "gate and up rows");
+    return MODE == kGated ? 8 * NT : 16 * NT;
+}
+
+// What follows a product and moves little stands here instead of in a launch of its own (3 to 6 us of a decode step each): the
+// logits' cap and the tanh of a low-rank product's inputs, on the rounded values as those launches had them.
+template <int MODE, class St, int WK>
+__device__ __forceinline__ void put_rows(const uint16_t* smem, const RowsProduct& p, int n0, int m0, int batch) {
+    constexpr int BM = St::BM, OC = MODE == kGated ? St::BN / 2 : St::BN;
+    const int tid = threadIdx.x;
+    const bool four = p.N % 4 == 0 && p.ldo % 4 == 0 && p.out_batch % 4 == 0 && (reinterpret_cast<uintptr_t>(p.out) & 7) == 0;
+    for (int i = tid; i < BM * (OC / 4); i += WK * kWave) {
+        const int m = i / (OC / 4), n = i % (OC / 4) * 4, col = n0 + n;
+        if (m0 + m >= p.n || col >= p.N) continue;
+        f32x4 y = St::total(smem, m, n);
+        if constexpr (MODE == kGated) {
+            const f32x4 u = St::total(smem, m, OC + n);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) y[j] = gated(y[j], u[j], p.gate);
+        } else if (p.bias && blockIdx.y == 0) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) y[j] += ld(p.bias + min(col + j, p.N - 1));
+        }
+        if constexpr (MODE == kRound) {
+            if (col + 3 >= p.turn0 && col < p.turn1) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (col + j >= p.turn0 && col + j < p.turn1) y[j] = tanhf(bf16_to_f32(f32_to_bf16(y[j])));
+            }
+        }
+        if constexpr (MODE == kCapped) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float v = bf16_to_f32(f32_to_bf16(y[j]));
+                y[j] = p.cap > 0.f ? p.cap * tanhf(v / p.cap) : v;
+            }
+        }
+        if constexpr (MODE == kParts || MODE == kCapped) {
+            float* o = reinterpret_cast<float*>(p.out) + (MODE == kParts ? blockIdx.y * p.ldsplit : 0) + (m0 + m) * p.ldo + col;
+            if (four) st4(o, make_float4(y[0], y[1], y[2], y[3]));
+            else
+                for (int j = 0; j < 4 && col + j < p.N; ++j) st(o + j, y[j]);
+        } else {
+            uint16_t* o = reinterpret_cast<uint16_t*>(p.out) + batch * p.out_batch + (m0 + m) * p.ldo + col;
+            if (four) st4(o, make_float4(y[0], y[1], y[2], y[3]));
+            else
+                for (int j = 0; j < 4 && col + j < p.N; ++j) st(o + j, y[j]);
+        }
+    }
+}
+
+}  // namespace skyrl

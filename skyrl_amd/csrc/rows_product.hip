@@ -18,36 +18,17 @@
 // 16.4 us, 13.4 without x, 7.3 without the weights, 5.3 without either; leaving out the products changes it by 0.4.
 // Batches (a head's up-projections of latent attention, 512 x 128 and 128 x 512): 16 heads, 1 / 64 rows, both products with the
 // copy that the library's needed: 15.4 / 17.1 us, here 5.9 / 7.6 us.
-#include "gate.h"
-#include "stream.h"
+#include "rows.h"
 
 namespace skyrl {
 namespace {
-
-enum Mode { kRound, kParts, kGated };
-
-struct RowsProduct {
-    const uint16_t* x;
-    int64_t ldx;
-    int n, K;
-    const uint16_t* w;
-    int64_t ldw;
-    int N;  // output columns; kGated: gate rows, the up rows follow
-    const uint16_t* bias;
-    Gate gate;
-    void* out;
-    int64_t ldo, ldsplit;
-    int row_blocks;  // gridDim.z = batch row_blocks
-    int64_t x_batch, w_batch, out_batch;
-};
 
 // NT 16-row weight tiles (kGated: half of each matrix) and MT 16-row tiles of x per workgroup, the depth in gridDim.y * WK shares;
 // blocks of MT tiles and products of a batch along z.
 template <int MODE, int NT, int MT, int WK, int S>
 __global__ __launch_bounds__(WK* kWave) void rows_product_kernel(RowsProduct p) {
     using St = Stream<NT, MT, WK, S>;
-    constexpr int BM = St::BM, OC = MODE == kGated ? St::BN / 2 : St::BN;  // output columns
-    static_assert(MODE != kGated || NT % 2 == 0, "gate and up rows");
+    constexpr int BM = St::BM, OC = out_cols<MODE, NT>();
     __shared__ __attribute__((aligned(16))) uint16_t smem[St::kLds];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n0 = blockIdx.x * OC, batch = blockIdx.z / p.row_blocks, m0 = blockIdx.z % p.row_blocks * BM;
@@ -62,31 +43,7 @@ __global__ __launch_bounds__(WK* kWave) void rows_product_kernel(RowsProduct p) 
         },
         [&](int r) { return p.x + batch * p.x_batch + min(m0 + r, p.n - 1) * p.ldx; }, acc);
     St::store(smem, acc);
-    const bool four = p.N % 4 == 0 && p.ldo % 4 == 0 && p.out_batch % 4 == 0 && (reinterpret_cast<uintptr_t>(p.out) & 7) == 0;
-    for (int i = tid; i < BM * (OC / 4); i += WK * kWave) {
-        const int m = i / (OC / 4), n = i % (OC / 4) * 4, col = n0 + n;
-        if (m0 + m >= p.n || col >= p.N) continue;
-        f32x4 y = St::total(smem, m, n);
-        if constexpr (MODE == kGated) {
-            const f32x4 u = St::total(smem, m, OC + n);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) y[j] = gated(y[j], u[j], p.gate);
-        } else if (p.bias && blockIdx.y == 0) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) y[j] += ld(p.bias + min(col + j, p.N - 1));
-        }
-        if constexpr (MODE == kParts) {
-            float* o = reinterpret_cast<float*>(p.out) + blockIdx.y * p.ldsplit + (m0 + m) * p.ldo + col;
-            if (four) st4(o, make_float4(y[0], y[1], y[2], y[3]));
-            else
-                for (int j = 0; j < 4 && col + j < p.N; ++j) st(o + j, y[j]);
-        } else {
-            uint16_t* o = reinterpret_cast<uint16_t*>(p.out) + batch * p.out_batch + (m0 + m) * p.ldo + col;
-            if (four) st4(o, make_float4(y[0], y[1], y[2], y[3]));
-            else
-                for (int j = 0; j < 4 && col + j < p.N; ++j) st(o + j, y[j]);
-        }
-    }
+    put_rows<MODE, St, WK>(smem, p, n0, m0, batch);
 }
 
 constexpr int kWide = 8192;       // output columns from which wider tiles still fill the chip and read x less often
@@ -135,6 +92,19 @@ void launch_rows(RowsProduct p, int splits, hipStream_t s, int batch = 1) {
                        dim3(WK * kWave), 0, s, p);
 }
 
+template <int MODE>
+void launch_rounded(const RowsProduct& p, hipStream_t s) {
+    if (p.N >= kWide) {
+        if (p.n <= 16) launch_rows<MODE, 4, 1, 4, 2>(p, 1, s);
+        else if (p.n <= 32) launch_rows<MODE, 4, 2, 4, 2>(p, 1, s);
+        else launch_rows<MODE, 4, 4, 2, 2>(p, 1, s);
+    } else {
+        if (p.n <= 16) launch_rows<MODE, 1, 1, 4, 4>(p, 1, s);
+        else if (p.n <= 32) launch_rows<MODE, 1, 2, 4, 3>(p, 1, s);
+        else launch_rows<MODE, 1, 4, 4, 2>(p, 1, s);
+    }
+}
+
 }  // namespace
 }  // namespace skyrl
 
@@ -146,20 +116,23 @@ extern "C" int32_t skyrl_rows_product_fits(int32_t n, int32_t K, int32_t N, int3
 
 extern "C" int32_t skyrl_rows_product_splits(int32_t n, int32_t K, int32_t N) { return splits_for(n, K, N); }
 
-extern "C" int skyrl_rows_product(const void* x, int64_t ldx, int32_t n, int32_t K, const void* w, int64_t ldw, int32_t N,
-                                  const void* bias, int32_t act, float alpha, float limit, int32_t splits, void* out,
-                                  int64_t ldo, void* stream) {
+namespace {
+
+// capped: f32 [n, N], the rounded product between -cap and cap; turn0, turn1: columns of a rounded one that go through tanh.
+int rows_product(const void* x, int64_t ldx, int32_t n, int32_t K, const void* w, int64_t ldw, int32_t N, const void* bias,
+                 int32_t act, float alpha, float limit, int32_t splits, void* out, int64_t ldo, bool capped, float cap, int32_t turn0,
+                 int32_t turn1, void* stream) {
     const bool gate = act >= 0;
     SKYRL_REQUIRE(rows_take(n, K, N, gate ? kFormGated : splits ? kFormParts : kFormRound), "rows_product: sizes that the library takes");
     SKYRL_REQUIRE(x && w && out, "rows_product: null pointer");
     SKYRL_REQUIRE(aligned16(x) && aligned16(w) && ldx % 8 == 0 && ldw % 8 == 0 && ldw >= K && (n == 1 || ldx >= K),
                   "rows_product: rows must be 16-byte aligned");
-    SKYRL_REQUIRE((reinterpret_cast<uintptr_t>(out) & (splits ? 3 : 1)) == 0 && (n == 1 || ldo >= N), "rows_product: bad output");
+    SKYRL_REQUIRE((reinterpret_cast<uintptr_t>(out) & (splits || capped ? 3 : 1)) == 0 && (n == 1 || ldo >= N), "rows_product: bad output");
     SKYRL_REQUIRE(!gate || (!bias && splits == 0 && (act == SKYRL_ACT_SILU || act == SKYRL_ACT_GELU_TANH || act == SKYRL_ACT_CLAMPED)),
                   "rows_product: a gated product has an activation, no bias and no splits");
     SKYRL_REQUIRE(splits == 0 || splits == splits_for(n, K, N), "rows_product: splits are skyrl_rows_product_splits'");
     const RowsProduct p{reinterpret_cast<const uint16_t*>(x), ldx, n, K, reinterpret_cast<const uint16_t*>(w), ldw, N,
-                        reinterpret_cast<const uint16_t*>(bias), Gate{act, alpha, limit}, out, ldo, (int64_t)n * ldo, 1, 0, 0, 0};
+                        reinterpret_cast<const uint16_t*>(bias), Gate{act, alpha, limit}, turn0, turn1, cap, out, ldo, (int64_t)n * ldo, 1, 0, 0, 0};
     hipStream_t s = as_stream(stream);
     // Wide tiles where there are columns enough, since every workgroup reads x again; else 16 rows of weights, so that
     // the chip is full (3648 x 2048 at 64 rows: 8.5 us with 16, 9.4 with 32). Up to 16 rows 64 rows of weights for the wide ones
@@ -174,16 +147,31 @@ extern "C" int skyrl_rows_product(const void* x, int64_t ldx, int32_t n, int32_t
         else if (n <= 32) launch_rows<kParts, 2, 2, 4, 2>(p, splits, s);
         else if (n <= 64) launch_rows<kParts, 2, 4, 4, 2>(p, splits, s);
         else launch_rows<kParts, 2, 8, 4, 1>(p, splits, s);
-    } else if (N >= kWide) {
-        if (n <= 16) launch_rows<kRound, 4, 1, 4, 2>(p, 1, s);
-        else if (n <= 32) launch_rows<kRound, 4, 2, 4, 2>(p, 1, s);
-        else launch_rows<kRound, 4, 4, 2, 2>(p, 1, s);
+    } else if (capped) {
+        launch_rounded<kCapped>(p, s);
     } else {
-        if (n <= 16) launch_rows<kRound, 1, 1, 4, 4>(p, 1, s);
-        else if (n <= 32) launch_rows<kRound, 1, 2, 4, 3>(p, 1, s);
-        else launch_rows<kRound, 1, 4, 4, 2>(p, 1, s);
+        launch_rounded<kRound>(p, s);
     }
     return check_launch("rows_product_kernel");
+}
+
+}  // namespace
+
+extern "C" int skyrl_rows_product(const void* x, int64_t ldx, int32_t n, int32_t K, const void* w, int64_t ldw, int32_t N,
+                                  const void* bias, int32_t act, float alpha, float limit, int32_t splits, void* out,
+                                  int64_t ldo, void* stream) {
+    return rows_product(x, ldx, n, K, w, ldw, N, bias, act, alpha, limit, splits, out, ldo, false, 0.f, 0, 0, stream);
+}
+
+extern "C" int skyrl_rows_product_tanh(const void* x, int64_t ldx, int32_t n, int32_t K, const void* w, int64_t ldw, int32_t N,
+                                       const void* bias, int32_t first, int32_t last, void* out, int64_t ldo, void* stream) {
+    SKYRL_REQUIRE(first >= 0 && first <= last && last <= N, "rows_product_tanh: bad columns");
+    return rows_product(x, ldx, n, K, w, ldw, N, bias, -1, 0.f, 0.f, 0, out, ldo, false, 0.f, first, last, stream);
+}
+
+extern "C" int skyrl_rows_product_capped(const void* x, int64_t ldx, int32_t n, int32_t K, const void* w, int64_t ldw, int32_t N,
+                                         float cap, float* out, int64_t ldo, void* stream) {
+    return rows_product(x, ldx, n, K, w, ldw, N, nullptr, -1, 0.f, 0.f, 0, out, ldo, true, cap, 0, 0, stream);
 }
 
 namespace {
@@ -198,7 +186,7 @@ int rows_batch(const void* x, int64_t ldx, int64_t x_batch, int32_t n, int32_t K
                       ldw >= K && (reinterpret_cast<uintptr_t>(out) & 1) == 0,
                   "rows_batch: rows must be 16-byte aligned");
     const RowsProduct p{reinterpret_cast<const uint16_t*>(x), ldx, n, K, reinterpret_cast<const uint16_t*>(w), ldw, N, nullptr,
-                        Gate{-1, 0.f, 0.f}, out, ldo, 0, 1, x_batch, w_batch, out_batch};
+                        Gate{-1, 0.f, 0.f}, 0, 0, 0.f, out, ldo, 0, 1, x_batch, w_batch, out_batch};
     hipStream_t s = as_stream(stream);
     // A head's matrix is small: all its pieces are under way at once. Shallow ones (the queries' up-projection) take two
     // waves a workgroup and 32 columns, deep ones (the outputs') four waves and 16 columns. In order: one wave, which has the

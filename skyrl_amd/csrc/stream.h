@@ -13,15 +13,15 @@ typedef __attribute__((address_space(1))) void gbl_void;
 
 __device__ const uint4 kZero16 = {0u, 0u, 0u, 0u};
 
-// NT 16-row weight tiles, MT 16-row tiles of x, WK waves.
-template <int NT, int MT, int WK, int S>
+// NT 16-row weight tiles, MT 16-row tiles of x, WK waves. HELD: the rows of x lie in LDS whole and are not streamed.
+template <int NT, int MT, int WK, int S, bool HELD = false>
 struct Stream {
-    static constexpr int BN = 16 * NT, BM = 16 * MT, WP = 2 * NT, XP = 2 * MT, L = WP + XP;  // 1 KB pieces: 8 rows, 64 deep
-    static constexpr int kStage = (BN + BM) * 64;  // elements
+    static constexpr int BN = 16 * NT, BM = 16 * MT, WP = 2 * NT, XP = HELD ? 0 : 2 * MT, L = WP + XP;  // 1 KB pieces: 8 rows, 64 deep
+    static constexpr int kStage = (BN + (HELD ? 0 : BM)) * 64;  // elements
     static constexpr int LR = BN + 4;              // a row of a share's sums
     static constexpr int kSums = WK * BM * LR * 2, kPieces = WK * S * kStage;
     static constexpr int kLds = kPieces > kSums ? kPieces : kSums;  // elements
-    static_assert(S <= 4, "the waits below");
+    static_assert(S <= 8 && (S - 1) * L < 64, "the waits below");
 
     template <int N>
     static __device__ __forceinline__ void wait_loads() {
@@ -33,15 +33,22 @@ struct Stream {
 
     // acc[m][n]: lane (c, g) has x row 16 m + c, weight rows 16 n + 4 g .. + 3. wrow(r), xrow(r): start of the tile's row r, valid
     // for every r (rows past the last: any row, not stored). K a multiple of 8, the wave's pieces s0 .. s0 + nk - 1 of 64.
-    template <class WRow, class XRow>
-    static __device__ __forceinline__ void run(uint16_t* smem, int K, int s0, int nk, WRow wrow, XRow xrow, f32x4 (&acc)[MT][NT]) {
+    // HELD: between(), called when the first pieces are under way, returns the LDS address of the one row there is, readable up to
+    // a multiple of 64 with numbers in it; xrow is not called.
+    struct Streamed {
+        __device__ uint32_t operator()() const { return 0; }
+    };
+    template <class WRow, class XRow, class Between = Streamed>
+    static __device__ __forceinline__ void run(uint16_t* smem, int K, int s0, int nk, WRow wrow, XRow xrow, f32x4 (&acc)[MT][NT],
+                                               Between between = Between{}) {
         const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
         const int c = lane & 15, g = lane >> 4;
         uint16_t* own = smem + wave * (S * kStage);
         // this lane's 16 bytes of every piece: row lane / 8, chunk (lane % 8) ^ row, so that 16 rows read at a time lie in
         // different banks
         const int r8 = lane >> 3, ch = ((lane & 7) ^ r8) * 8;
-        const uint16_t *ws[WP], *xs[XP];
+        static_assert(!HELD || MT == 1, "one tile of held rows");
+        const uint16_t *ws[WP], *xs[XP ? XP : 1];
 #pragma unroll
         for (int i = 0; i < WP; ++i) ws[i] = wrow(i * 8 + r8) + s0 * 64 + ch;
 #pragma unroll
@@ -68,10 +75,15 @@ struct Stream {
         for (int t = 0; t < S; ++t)
             if (t < nk) fetch(t);
         const uint32_t base = (uint32_t)(uintptr_t)(lds_void*)own + c * 128;
+        const uint32_t held = HELD ? between() + s0 * 128 + g * 16 : 0;
         for (int t = 0; t < nk; ++t) {
             const int left = nk - 1 - t;  // pieces after this one; at most S - 1 of them are under way
             if (left >= S - 1) wait_loads<(S - 1) * L>();
-            else if (S > 3 && left == 2) wait_loads<2 * L>();
+            else if (S > 7 && left == 6) wait_loads<(S > 7 ? 6 * L : 0)>();
+            else if (S > 6 && left == 5) wait_loads<(S > 6 ? 5 * L : 0)>();
+            else if (S > 5 && left == 4) wait_loads<(S > 5 ? 4 * L : 0)>();
+            else if (S > 4 && left == 3) wait_loads<(S > 4 ? 3 * L : 0)>();
+            else if (S > 3 && left == 2) wait_loads<(S > 3 ? 2 * L : 0)>();
             else if (S > 2 && left == 1) wait_loads<L>();
             else wait_loads<0>();
             // The reads are not the compiler's: it would wait for every load into LDS under way before one. They are waited
@@ -83,7 +95,10 @@ struct Stream {
 #pragma unroll
                 for (int n = 0; n < NT; ++n) lds_read(wf[h][n], at, n * 2048);
 #pragma unroll
-                for (int m = 0; m < MT; ++m) lds_read(xf[h][m], at, (NT + m) * 2048);
+                for (int m = 0; m < MT; ++m) {
+                    if constexpr (HELD) lds_read(xf[h][m], held + t * 128, h * 64);
+                    else lds_read(xf[h][m], at, (NT + m) * 2048);
+                }
             }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll

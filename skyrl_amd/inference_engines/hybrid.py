@@ -331,12 +331,14 @@ class HybridDecoder:
         h = lk.embed(inp.tokens, self.embed, s.embed_scale)
         x = torch.empty(h.shape, dtype=self.dtype, device=self.device)
         delta = None
+        form = lk.normed if trail is None else lk.add_norm
         ws = self.workspace if inp.one_token else self.portion_workspace
         for r, state in zip(s.runs, cache.runs):
             step = None if r.step is None else self.loop_step[r.step]
             for weight, sub in self.layers[r.layer]["subs"]:
-                lk.add_norm(delta, h, weight, step=step, out=x, **norm)
-                delta, step = sub.forward(x, inp, state, ws, parts=True), None
+                rows = form(delta, h, weight, step=step, out=x, **norm)
+                delta, step = sub.forward(rows, inp, state, ws, parts=True), None
+                h = lk.residual(rows, h)
             if trail is not None:
                 trail.append(h + lk.joined(delta).float())
         if want is None:
@@ -380,6 +382,7 @@ class HybridDecoder:
         ws = self.workspace if inp.one_token else self.portion_workspace
         for k, (state, _, sub, after) in enumerate(steps):
             y, gate = sub.forward(x, inp, state, ws)
+            h, x = lk.residual(x, h), lk.rows_of(x)
             args = dict(norm, mult=s.residual_mult, parts=sub.rows_per_token, gate_bias=sub.bias)
             last = k == len(steps) - 1
             if last and trail is not None:
@@ -391,7 +394,8 @@ class HybridDecoder:
                 else:
                     y = y.view(-1, sub.rows_per_token, s.hidden_size)[want].view(-1, s.hidden_size)
                 h, gate, x = h[want], gate.index_select(-2, want), None
-            x = lk.gate_norm_add(y, h, after, before[k + 1], gate=gate, out=x, **args)
+            form = lk.gate_norm_add if last or trail is not None else lk.gate_normed
+            x = form(y, h, after, before[k + 1], gate=gate, out=x, **args)
             if trail is not None and k in ends and not last:
                 trail.append(h.clone())
         return x
@@ -406,4 +410,4 @@ class HybridDecoder:
 
     def logits(self, hidden: torch.Tensor) -> torch.Tensor:
         """f32 [n, V]."""
-        return lk.softcap(lk.linear(hidden, self.lm_head), self.spec.logit_softcap)
+        return lk.capped_linear(hidden, self.lm_head, self.spec.logit_softcap)

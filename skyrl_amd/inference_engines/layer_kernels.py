@@ -62,6 +62,137 @@ def embed(tokens: torch.Tensor, table: torch.Tensor, scale: float, positions: Op
     return out
 
 
+# ---------------------------------------------------------------- the norm ahead of a product
+class NormedRow:
+    """A row [1, H] whose norm is formed by the first product of it (skyrl_add_norm_product, skyrl_gate_norm_product), or by a
+    launch of its own when something else asks for the rows. `hidden` is the residual, of before or, afterwards, of behind the
+    norm."""
+
+    def __init__(self, hidden: torch.Tensor, out: torch.Tensor, fused, alone):
+        self.hidden, self.out, self.fused, self.alone = hidden, out, fused, alone
+        self.shape, self.dtype, self.device = out.shape, out.dtype, out.device
+
+    def rows(self) -> torch.Tensor:
+        if self.alone is not None:
+            self.alone(self.out)
+            self.fused = self.alone = None
+        return self.out
+
+    def product(self, w: torch.Tensor, bias=None, parts: bool = False, turn=None, act: Optional[str] = None, alpha: float = 1.0,
+                limit: float = 0.0) -> Optional[torch.Tensor]:
+        """linear's or gated_linear's; None: not as one launch."""
+        gated = act is not None
+        if self.fused is None or not _rows_fit(self.out, w, gated, parts) or w.shape[1] != self.out.shape[1] or (gated and w.shape[0] % 2):
+            return None
+        dev = _require_gpu(self.out, w, bias)
+        H, N = self.out.shape[1], w.shape[0] // 2 if gated else w.shape[0]
+        _check(bias, "bias", torch.bfloat16, (N,))
+        if turn is not None and (parts or gated):
+            raise ValueError("parts and gated products turn no columns")
+        splits = int(_ffi.query("skyrl_rows_product_splits", 1, H, N)) if parts else 0
+        y = (torch.empty((splits, 1, N), dtype=torch.float32, device=dev) if splits
+             else torch.empty((1, N), dtype=torch.bfloat16, device=dev))
+        h = torch.empty_like(self.hidden)
+        q = _ffi.NormedProduct(self.hidden.data_ptr(), h.data_ptr(), self.out.data_ptr(), w.data_ptr(), w.stride(0),
+                               None if bias is None else bias.data_ptr(), y.data_ptr(), H, N, ACTIVATIONS[act] if gated else -1,
+                               splits, *(turn or (0, 0)), alpha, limit)
+        if not self.fused(q, gated, splits):
+            return None
+        self.hidden, self.fused, self.alone = h, None, None
+        return y
+
+
+def _as_rows(x) -> torch.Tensor:
+    """Shape, type and place of rows; a NormedRow's may not be formed yet."""
+    return x.out if isinstance(x, NormedRow) else x
+
+
+def rows_of(x) -> torch.Tensor:
+    return x.rows() if isinstance(x, NormedRow) else x
+
+
+def residual(x, hidden: torch.Tensor) -> torch.Tensor:
+    """The residual behind the norm that x is from."""
+    if not isinstance(x, NormedRow):
+        return hidden
+    x.rows()
+    return x.hidden
+
+
+def _row_fits(hidden: torch.Tensor, weight: torch.Tensor, shares: int, rows: int, *others) -> bool:
+    return (hidden.shape[0] == 1 and weight.dtype == torch.bfloat16 and hidden.is_cuda and hidden.is_contiguous()
+            and bool(_ffi.query("skyrl_normed_product_fits", hidden.shape[1], shares, rows))
+            and all(t is None or t.data_ptr() % 16 == 0 for t in (hidden, weight, *others)))
+
+
+def normed(delta: Optional[torch.Tensor], hidden: torch.Tensor, weight: torch.Tensor, eps: float, kind: str = "layer",
+           step: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None, base: float = 0.0):
+    """add_norm, or for one row of a model in bf16 a NormedRow."""
+    n, H = hidden.shape
+    parts = delta.shape[0] if delta is not None and delta.dim() == 3 else 0
+
+    def alone(to):
+        return add_norm(delta, hidden, weight, eps, kind, step, to, base)
+
+    if (delta is not None and not parts) or not _row_fits(hidden, weight, parts, 1, delta, step, out):
+        return alone(out)
+    _check(hidden, "hidden", torch.float32)
+    _check(weight, "weight", torch.bfloat16, (H,))
+    _check(delta, "delta", torch.float32, (parts, 1, H))
+    _check(step, "step", torch.bfloat16, (H,))
+    _check(out, "out", torch.bfloat16, (1, H))
+    dev = _require_gpu(hidden, weight, delta, step, out)
+
+    def fused(q, gated, splits):
+        if splits:
+            return False
+        _ffi.call("skyrl_add_norm_product", ctypes.byref(q), _ptr(delta), parts, _ptr(step), _ptr(weight), float(base), float(eps),
+                  NORMS[kind], _stream(dev))
+        return True
+
+    return NormedRow(hidden, torch.empty((1, H), dtype=torch.bfloat16, device=dev) if out is None else out, fused, alone)
+
+
+def gate_normed(a: torch.Tensor, hidden: torch.Tensor, weight: torch.Tensor, next_weight: torch.Tensor, eps: float, groups: int = 1,
+                mult: float = 1.0, parts: int = 1, gate: Optional[torch.Tensor] = None, gate_bias: Optional[torch.Tensor] = None,
+                out: Optional[torch.Tensor] = None):
+    """gate_norm_add, or for one row of a model in bf16, with either its sum or the gate's logits in parts, a NormedRow."""
+    n, H = hidden.shape
+    shares = a.shape[0] if a.dim() == 3 else 0
+    gate_shares = gate.shape[0] if gate is not None and gate.dim() == 3 else 0
+
+    def alone(to):
+        return gate_norm_add(a, hidden, weight, next_weight, eps, groups, mult, parts, gate, gate_bias, out=to)
+
+    if (gate is None or gate_bias is None or bool(shares) == bool(gate_shares) or groups < 1 or H % groups or H // groups % 8
+            or (shares and parts != 1) or (gate_shares and gate.shape[2] % 4)
+            or not _row_fits(hidden, weight, max(shares, gate_shares), parts, a, next_weight, gate, gate_bias, out)):
+        return alone(out)
+    _check(hidden, "hidden", torch.float32)
+    _check(a, "a", torch.float32 if shares else torch.bfloat16, (shares, 1, H) if shares else (parts, H))
+    _check(weight, "weight", torch.bfloat16, (H,))
+    _check(next_weight, "next_weight", torch.bfloat16, (H,))
+    _check(gate_bias, "gate_bias", torch.float32, (H,))
+    _check(out, "out", torch.bfloat16, (1, H))
+    if gate_shares:
+        _check(gate, "gate", torch.float32)
+        if gate.shape[1] != 1 or gate.shape[2] < H:
+            raise ValueError(f"a gate's parts must be [shares, 1, {H} or more]")
+    else:
+        _check_view(gate, "gate", torch.bfloat16, (1, H))
+    dev = _require_gpu(a, hidden, weight, next_weight, gate, gate_bias, out)
+
+    def fused(q, gated, splits):
+        if gated or (splits and not shares):
+            return False
+        _ffi.call("skyrl_gate_norm_product", ctypes.byref(q), _ptr(a), shares, parts, _ptr(gate), gate_shares,
+                  gate.shape[2] if gate_shares else H, _ptr(gate_bias), _ptr(weight), groups, float(eps), float(mult),
+                  _ptr(next_weight), _stream(dev))
+        return True
+
+    return NormedRow(hidden, torch.empty((1, H), dtype=torch.bfloat16, device=dev) if out is None else out, fused, alone)
+
+
 # ---------------------------------------------------------------- products of few rows
 MAX_ROWS = 128  # that skyrl_rows_product takes at most
 
@@ -79,7 +210,12 @@ def _rows_fit(x: torch.Tensor, w: torch.Tensor, gated: bool = False, parts: bool
 
 def gives_parts(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether linear(x, w, parts=True) returns parts."""
-    return _rows_fit(x, w, parts=True)
+    return _rows_fit(_as_rows(x), w, parts=True)
+
+
+def turns(x, w: torch.Tensor) -> bool:
+    """Whether linear(x, w, turn=...) is taken: the product is no library's."""
+    return _rows_fit(_as_rows(x), w)
 
 
 def _rows_aligned(x: torch.Tensor, w: torch.Tensor) -> bool:
@@ -88,11 +224,18 @@ def _rows_aligned(x: torch.Tensor, w: torch.Tensor) -> bool:
             and (n == 1 or x.stride(0) >= K) and w.stride(0) >= K and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
-def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, parts: bool = False) -> torch.Tensor:
+def linear(x, w: torch.Tensor, bias: Optional[torch.Tensor] = None, parts: bool = False, turn=None) -> torch.Tensor:
     """x w^T + bias. Few bf16 rows take skyrl_rows_product, everything else the library. With `parts` the result of
     few rows may be f32 [splits, n, N], to be summed over the first index where it is read (add_norm, gate_norm_add,
-    joined)."""
+    joined). turn (first, last): these columns go through tanh, where `turns` says so. x: rows, or a NormedRow."""
+    if isinstance(x, NormedRow):
+        y = x.product(w, bias, parts=parts, turn=turn)
+        if y is not None:
+            return y
+        x = x.rows()
     if not _rows_fit(x, w, parts=parts):
+        if turn is not None:
+            raise ValueError("a library's product turns no columns")
         return F.linear(x, w, bias)
     dev = _require_gpu(x, w, bias)
     (n, K), N = x.shape, w.shape[0]
@@ -102,6 +245,12 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
     splits = int(_ffi.query("skyrl_rows_product_splits", n, K, N)) if parts else 0
     out = (torch.empty((splits, n, N), dtype=torch.float32, device=dev) if splits
            else torch.empty((n, N), dtype=torch.bfloat16, device=dev))
+    if turn is not None:
+        if splits:
+            raise ValueError("parts turn no columns")
+        _ffi.call("skyrl_rows_product_tanh", _ptr(x), x.stride(0), n, K, _ptr(w), w.stride(0), N, _ptr(bias), *turn, _ptr(out), N,
+                  _stream(dev))
+        return out
     _ffi.call("skyrl_rows_product", _ptr(x), x.stride(0), n, K, _ptr(w), w.stride(0), N, _ptr(bias), -1, 0.0, 0.0, splits,
               _ptr(out), N, _stream(dev))
     return out
@@ -140,7 +289,13 @@ def joined(y: torch.Tensor) -> torch.Tensor:
 
 
 def gated_linear(x: torch.Tensor, w: torch.Tensor, act: str, alpha: float = 1.0, limit: float = 0.0) -> Optional[torch.Tensor]:
-    """gate_mul of x w^T, w the gate rows and then the up rows, in one launch for few or many bf16 rows; None otherwise."""
+    """gate_mul of x w^T, w the gate rows and then the up rows, in one launch for few or many bf16 rows; None otherwise. x: rows,
+    or a NormedRow."""
+    if isinstance(x, NormedRow):
+        y = x.product(w, act=act, alpha=alpha, limit=limit)
+        if y is not None:
+            return y
+        x = x.rows()
     (n, K), N = x.shape, w.shape[0] // 2
     many = (n > MAX_ROWS and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.is_cuda
             and bool(_ffi.query("skyrl_gated_product_fits", n, K, N)) and _rows_aligned(x, w))
@@ -317,6 +472,20 @@ def softcap(x: torch.Tensor, cap: Optional[float]) -> torch.Tensor:
     _check(x, "x", x.dtype)
     out = torch.empty(x.shape, dtype=torch.float32, device=dev)
     _ffi.call("skyrl_softcap", _ptr(x), _ptr(out), x.numel(), float(cap or 0.0), _code(x), _stream(dev))
+    return out
+
+
+def capped_linear(x: torch.Tensor, w: torch.Tensor, cap: Optional[float]) -> torch.Tensor:
+    """softcap of linear(x, w), for few rows in one launch."""
+    if not _rows_fit(x, w):
+        return softcap(linear(x, w), cap)
+    dev = _require_gpu(x, w)
+    (n, K), N = x.shape, w.shape[0]
+    if w.shape[1] != K:
+        raise ValueError(f"w must be [N, {K}], got {tuple(w.shape)}")
+    out = torch.empty((n, N), dtype=torch.float32, device=dev)
+    _ffi.call("skyrl_rows_product_capped", _ptr(x), x.stride(0), n, K, _ptr(w), w.stride(0), N, float(cap or 0.0), _ptr(out), N,
+              _stream(dev))
     return out
 
 

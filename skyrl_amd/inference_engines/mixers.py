@@ -206,6 +206,8 @@ class Products:
 
     def __init__(self, parts: List[Any], width: int, w: Weights, apart: bool = False, beside: int = 0):
         self.parts, self.ranges, self.apart, self.beside = parts, [], apart, None
+        # of a single part: its columns that go through tanh next, in the input product for few rows (`inner`'s `turned`)
+        self.turn = getattr(parts[0], "turn", None) if len(parts) == 1 and not apart else None
         self.fused = None  # of a single part: input product and `inner` in one launch, for few rows
         a = c = 0
         for p in parts:
@@ -243,7 +245,10 @@ class Products:
             cat = self.fused(x)
             if cat is not None:
                 return lk.linear(cat, self.w_out, self.b_out, parts)
-        proj = lk.linear(x, self.w_in, self.b_in)
+        turn, turned = None, {}
+        if self.turn is not None and lk.turns(x, self.w_in):
+            turn, turned = self.turn, {"turned": True}
+        proj = lk.linear(x, self.w_in, self.b_in, turn=turn)
         if self.apart:
             outs = []
             for p, (a, _), (wo, bo), st in zip(self.parts, self.ranges, self.outs, state):
@@ -254,7 +259,7 @@ class Products:
         make = torch.zeros if self.padded else torch.empty  # padding columns meet weights: they must be finite
         cat = make((x.shape[0], self.w_out.shape[1]), dtype=x.dtype, device=x.device)
         for p, (a, c) in zip(self.parts, self.ranges):
-            p.inner(proj[:, a:a + p.in_rows], cat[:, c:c + p.out_cols], inp, state, workspace)
+            p.inner(proj[:, a:a + p.in_rows], cat[:, c:c + p.out_cols], inp, state, workspace, **turned)
         y = lk.linear(cat, self.w_out, self.b_out, parts)
         return y if self.beside is None else (y, proj[:, self.beside[0]:self.beside[1]])
 
@@ -284,7 +289,8 @@ class Gated:
             return self.sub.forward(x, inp, state, workspace, parts=True)
         if self.joint is not None and self.sub.chooses(x, self.joint):
             logits = lk.linear(x, self.joint, parts=True)
-            return self.sub.forward(x, inp, state, workspace, logits=(logits, self.weight.shape[0])), logits
+            return self.sub.forward(lk.rows_of(x), inp, state, workspace, logits=(logits, self.weight.shape[0])), logits
+        x = lk.rows_of(x)
         return self.sub.forward(x, inp, state, workspace), lk.linear(x, self.weight)
 
 
@@ -569,8 +575,13 @@ class GeneralDelta:
         yield "chunks", lambda: chunk_plan(seq_lens, first_seq, first_token)
 
     # ---- step
-    def inner(self, proj: torch.Tensor, out: torch.Tensor, inp, state: torch.Tensor, workspace) -> None:
-        wl = lk.linear(lk.tanh(proj[:, 5 * self.out_cols:]), self.w2)
+    @property
+    def turn(self):
+        return 5 * self.out_cols, self.in_rows
+
+    def inner(self, proj: torch.Tensor, out: torch.Tensor, inp, state: torch.Tensor, workspace, turned: bool = False) -> None:
+        wl = proj[:, 5 * self.out_cols:]
+        wl = lk.linear(wl if turned else lk.tanh(wl), self.w2)
         args = (proj, wl, self.w0, self.a_bias, self.norm)
         n = inp.rows.shape[0]
         prompt = inp.plan is not None and "chunks" in inp.plan

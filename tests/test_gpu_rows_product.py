@@ -209,3 +209,101 @@ def test_rings_are_refilled(dev, form, n, N, K, waves, slots):
         assert bool(((y.sum(0) - z).abs() <= 2 * off + 2.0 ** -21 * z.abs()).all())
     else:
         assert bool(((y - z).abs() <= 2.0 ** -8 * z.abs() + 2 * off + 1e-5).all())
+
+
+def _close(y, x, w, want=None):
+    ref, off = _bounds(x, w)
+    want = ref if want is None else want
+    y = lk.joined(y).double()
+    return bool(((y - want).abs() <= 2.0 ** -8 * want.abs() + 2 * off).all())
+
+
+# rows of one group of four, of a remainder of the last piece, of both register forms; wide and narrow products
+@pytest.mark.parametrize("H,N", [(8, 16), (72, 203), (264, 8200), (1536, 96), (2048, 8192), (2056, 40), (4096, 12296), (4096, 24)])
+@pytest.mark.parametrize("parts", (0, 1, 2, 4))
+def test_norm_ahead_of_a_product(dev, H, N, parts):
+    g = torch.Generator(device=dev).manual_seed(H + N + parts)
+    _, w, b = _data(dev, 1, N, H, H)
+    delta = torch.randn(parts, 1, H, device=dev, generator=g) if parts else None
+    step = torch.randn(H, device=dev, generator=g).bfloat16() if parts % 2 == 0 else None
+    weight = torch.randn(H, device=dev, generator=g).bfloat16()
+    for kind, base in (("layer", 0.0), ("rms", 1.0)):
+        h = torch.randn(1, H, device=dev, generator=g) + 3
+        want_h = h.clone()
+        want = lk.add_norm(delta, want_h, weight, 1e-3, kind, step, base=base)
+        for gated in (False, True):
+            before = h.clone()
+            row = lk.normed(delta, before, weight, 1e-3, kind, step, base=base)
+            assert isinstance(row, lk.NormedRow)
+            y = lk.gated_linear(row, w, "silu") if gated and N % 2 == 0 else lk.linear(row, w, b)
+            assert row.fused is None and torch.equal(before, h)  # the old residual is read by every workgroup
+            assert torch.equal(lk.residual(row, before), want_h) and torch.equal(lk.rows_of(row), want)
+            assert torch.equal(lk.linear(row, w, b), lk.linear(want, w, b))  # a second product: of the rows
+            if gated and N % 2 == 0:
+                z = want.double() @ w.double().t()
+                ref = torch.nn.functional.silu(z[:, :N // 2]) * z[:, N // 2:]
+                assert float((y.double() - ref).norm()) <= 2.0 ** -8 * float(ref.norm()) + 1e-6
+            else:
+                assert _close(y, want, w, want.double() @ w.double().t() + b.double())
+    alone = lk.normed(delta, h, weight, 1e-3, "layer", step)
+    want = lk.add_norm(delta, h.clone(), weight, 1e-3, "layer", step)
+    assert torch.equal(lk.rows_of(alone), want)
+
+
+@pytest.mark.parametrize("H,groups", [(64, 4), (1536, 4), (2048, 4), (2048, 1), (4096, 4), (4096, 2), (1048, 1), (2080, 4)])
+@pytest.mark.parametrize("experts", (False, True))
+def test_gate_and_norms_ahead_of_a_product(dev, H, groups, experts):
+    g = torch.Generator(device=dev).manual_seed(H + groups)
+    rand = lambda *s: torch.randn(*s, device=dev, generator=g)  # noqa: E731
+    _, w, b = _data(dev, 1, 136, H, H)
+    weight, nxt = rand(H).bfloat16(), rand(H).bfloat16()
+    for parts in (1, 3) if not experts else (2, 8):
+        a = rand(parts, H).bfloat16() if experts else rand(parts, 1, H)
+        gate = rand(2, 1, H + 64) if experts else rand(1, H).bfloat16()
+        args = dict(groups=groups, mult=0.5, parts=parts if experts else 1, gate=gate, gate_bias=rand(H))
+        h = rand(1, H)
+        want_h = h.clone()
+        want = lk.gate_norm_add(a, want_h, weight, nxt, 1e-6, **args)
+        row = lk.gate_normed(a, h, weight, nxt, 1e-6, **args)
+        assert isinstance(row, lk.NormedRow)
+        turn = (40, 103) if experts else None
+        y = lk.linear(row, w, b, parts=not experts, turn=turn)
+        assert row.fused is None
+        # some of the sums round their products on one side and not on the other
+        assert float((lk.residual(row, h) - want_h).norm()) <= 1e-6 * float(want_h.norm())
+        assert float((lk.rows_of(row) - want).float().norm()) <= 2.0 ** -9 * float(want.float().norm())
+        ref = lk.rows_of(row).double() @ w.double().t() + b.double()
+        if experts:
+            plain = lk.linear(lk.rows_of(row), w, b)
+            assert torch.equal(y[:, :40], plain[:, :40]) and torch.equal(y[:, 103:], plain[:, 103:])
+            assert torch.equal(y[:, 40:103], torch.tanh(plain[:, 40:103].float()).bfloat16())
+        else:
+            assert y.dim() == 3 and _close(y, lk.rows_of(row), w, ref)
+
+
+def test_rows_that_are_normed_alone(dev):
+    """More than one row, f32 models, longer rows and more shares than the joint launch takes."""
+    for n, H, parts, dtype in ((2, 64, 2, torch.bfloat16), (1, 64, 0, torch.float32), (1, 4104, 1, torch.bfloat16), (1, 64, 5, torch.bfloat16)):
+        h, w = torch.randn(n, H, device=dev), torch.randn(H, device=dev).to(dtype)
+        delta = torch.randn(parts, n, H, device=dev) if parts else None
+        want_h = h.clone()
+        want = lk.add_norm(delta, want_h, w, 1e-6)
+        x = lk.normed(delta, h, w, 1e-6)
+        assert not isinstance(x, lk.NormedRow) and torch.equal(x, want) and torch.equal(h, want_h)
+
+
+@pytest.mark.parametrize("n,N,K", [(1, 17, 8), (1, 8200, 136), (16, 203, 72), (17, 8192, 64), (33, 24, 712), (64, 8216, 200), (65, 40, 64)])
+def test_what_follows_a_product(dev, n, N, K):
+    """The cap of logits and the tanh of some columns are those of their own launches, bit for bit."""
+    x, w, b = _data(dev, n, N, K, n + N)
+    y = lk.linear(x, w)
+    for cap in (30.0, None):
+        assert torch.equal(lk.capped_linear(x, w, cap), lk.softcap(y, cap))
+    for first, last in ((0, N), (5, 14), (N - 3, N), (7, 7)):
+        if not lk.turns(x, w):
+            assert n > 64
+            continue
+        t, plain = lk.linear(x, w, b, turn=(first, last)), lk.linear(x, w, b)
+        assert torch.equal(t[:, :first], plain[:, :first]) and torch.equal(t[:, last:], plain[:, last:])
+        if last > first:
+            assert torch.equal(t[:, first:last], lk.tanh(plain[:, first:last]))
