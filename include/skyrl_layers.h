@@ -157,6 +157,13 @@ int skyrl_softcap(const void* x, float* out, int64_t count, float cap, int32_t d
  *                        multiple of 16, per workgroup; nparts > 1 needs skyrl_latent_attend_workspace_bytes. f32, and
  *                        shapes outside the MFMA form (skyrl_latent_attend_mfma == 0), take a plain
  *                        kernel and ignore nparts.
+ *   skyrl_latent_lift    up to 64 tokens in bf16: skyrl_latent_write with queries, and the up-projection of their unrotated
+ *                        parts, in one launch: qa bf16 [heads, T, up_rank] = q_n up^T, up bf16 [heads, up_rank, dim].
+ *   skyrl_latent_query   one token in bf16: skyrl_latent_write with a query latent, which is not stored, and the product
+ *                        behind it: q bf16 [N] = normed wuq^T, wuq bf16 [N, q_rank], q_rank a multiple of 8 up to 2048.
+ *   skyrl_latent_attend_up  skyrl_latent_attend in bf16 with the outputs' up-projection behind its merge: y[t y_token + h y_head
+ *                        + i] = out[h][t] . up[h][i], up bf16 [heads, vdim, rank]; of out only rows that needed no merge
+ *                        are written. skyrl_latent_attend_up_fits: whether it takes the sizes (up to 4 tokens).
  *   skyrl_latent_gather  prompt form, step 1: copies for each of nseg segments the cached rows of
  *                        positions [seg_first, seg_first + seg_count) (seg i32 [nseg, 4]: block-table
  *                        row, first position, count, first packed row) to latent T [rows, rank] and
@@ -179,6 +186,18 @@ int skyrl_latent_attend(const void* qa, const void* q_rot, int64_t q_stride, int
                         const int64_t* positions, int32_t T, int32_t heads, int32_t rank, int32_t rot_dim,
                         float scale, int32_t window, int32_t part_min, int32_t nparts, const float* sinks,
                         const void* gate, int64_t gate_stride, void* out, void* workspace, int32_t dtype, void* stream);
+int skyrl_latent_lift(void* proj, int64_t proj_stride, int32_t T, int32_t heads, int32_t dim, int32_t rot_dim, int32_t halves,
+                      int32_t rank, const void* norm_weight, float eps, const int64_t* positions, const int64_t* slots,
+                      const float* cos_sin, void* cache, int32_t row, const void* up, int32_t up_rank, void* qa, void* stream);
+int skyrl_latent_query(void* proj, int64_t proj_stride, int32_t rot_dim, int32_t halves, int32_t q_rank, const void* q_norm,
+                       int32_t rank, const void* norm_weight, float eps, const int64_t* positions, const int64_t* slots,
+                       const float* cos_sin, void* cache, int32_t row, const void* wuq, int32_t N, void* q, void* stream);
+int32_t skyrl_latent_attend_up_fits(int32_t T, int32_t rank, int32_t rot_dim, int32_t row, int32_t nparts);
+int skyrl_latent_attend_up(const void* qa, const void* q_rot, int64_t q_stride, int64_t q_head, const void* cache, int32_t row,
+                           const int32_t* block_tables, int64_t bt_stride, const int32_t* bt_row, const int64_t* positions,
+                           int32_t T, int32_t heads, int32_t rank, int32_t rot_dim, float scale, int32_t window,
+                           int32_t part_min, int32_t nparts, const float* sinks, const void* gate, int64_t gate_stride, void* out,
+                           void* workspace, const void* up, int32_t vdim, void* y, int64_t y_token, int64_t y_head, void* stream);
 int skyrl_latent_gather(const void* cache, int32_t row, const int32_t* block_tables, int64_t bt_stride,
                         const int32_t* seg, int32_t nseg, int32_t max_count, int32_t rank, int32_t rot_dim,
                         void* latent, void* k_rot, int32_t dtype, void* stream);

@@ -317,6 +317,11 @@ LAYERS_SIGNATURES = {
     "skyrl_latent_attend_workspace_bytes": (_SZ, [_I32, _I32, _I32, _I32]),
     "skyrl_latent_attend": (_INT, [_P, _P, _I64, _I64, _P, _I32, _P, _I64, _P, _P, _I32, _I32, _I32, _I32, _F, _I32,
                                    _I32, _I32, _P, _P, _I64, _P, _P, _I32, _P]),
+    "skyrl_latent_lift": (_INT, [_P, _I64, _I32, _I32, _I32, _I32, _I32, _I32, _P, _F, _P, _P, _P, _P, _I32, _P, _I32, _P, _P]),
+    "skyrl_latent_query": (_INT, [_P, _I64, _I32, _I32, _I32, _P, _I32, _P, _F, _P, _P, _P, _P, _I32, _P, _I32, _P, _P]),
+    "skyrl_latent_attend_up_fits": (_I32, [_I32, _I32, _I32, _I32, _I32]),
+    "skyrl_latent_attend_up": (_INT, [_P, _P, _I64, _I64, _P, _I32, _P, _I64, _P, _P, _I32, _I32, _I32, _I32, _F, _I32, _I32, _I32,
+                                      _P, _P, _I64, _P, _P, _P, _I32, _P, _I64, _I64, _P]),
     "skyrl_latent_gather": (_INT, [_P, _I32, _P, _I64, _P, _I32, _I32, _I32, _I32, _P, _P, _I32, _P]),
     "skyrl_latent_prefill": (_INT, [_P, _I64, _P, _I64, _P, _P, _I64, _P, _I32, _I32, _I32, _I32, _I32, _F, _I32, _P,
                                     _P, _I64, _P, _I64, _P]),

@@ -17,14 +17,12 @@
 // a V^T tile of 64 keys in LDS, each wave owns 32 queries of one head.
 #include <type_traits>
 
-#include "elem.h"
+#include "normed.h"
 
 namespace skyrl {
 namespace {
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef short s16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kBS = 16;  // tokens per cache block
 constexpr int kNT = 256;
@@ -36,58 +34,114 @@ struct Pairs {
     __device__ __forceinline__ int second(int i) const { return halves ? i + rot / 2 : 2 * i + 1; }
 };
 
-// One workgroup per token. Parts of the row p that are there: the rotated parts of `heads` queries at its start, or
-// (q_rank > 0) a query latent that is normed in place; the key latent and its rotated part at lat_at (rank > 0).
+// Parts of a token's row that are there: the rotated parts of `heads` queries at its start, or (q_rank > 0) a query latent that is
+// normed in place; the key latent and its rotated part at lat_at (rank > 0).
 template <typename T>
-__global__ __launch_bounds__(kNT) void latent_write_kernel(T* __restrict__ proj, int64_t stride, int heads, int dim,
-                                                           Pairs pr, int q_rank, const T* __restrict__ q_norm,
-                                                           int rank, int lat_at, const T* __restrict__ norm_w,
-                                                           float eps, const int64_t* __restrict__ positions,
-                                                           const int64_t* __restrict__ slots,
-                                                           const float* __restrict__ cos_sin, T* __restrict__ cache,
-                                                           int row) {
-    __shared__ float s_red[kNT / kWave];
-    const int t = blockIdx.x;
-    T* p = proj + (int64_t)t * stride;
-    const int rot = pr.rot, qd = dim + rot, h2 = rot / 2;
-    const float* cs = cos_sin + positions[t] * rot;
-    if (q_rank > 0) {
+struct Write {
+    T* proj;
+    int64_t stride;
+    int heads, dim;
+    Pairs pr;
+    int q_rank;
+    const T* q_norm;
+    int rank, lat_at;
+    const T* norm_w;
+    float eps;
+    const int64_t *positions, *slots;
+    const float* cos_sin;
+    T* cache;
+    int row;
+};
+// A workgroup of NT threads, token t. A row is little and its time is latencies, so what a thread handles first of each part is
+// loaded ahead of everything else.
+constexpr int kHeld = 4, kPairs = 2;
+template <typename T, int NT>
+__device__ __forceinline__ void write_row(const Write<T>& w, int t) {
+    __shared__ float s_red[NT / kWave];
+    struct Held {
+        T x[kHeld], w[kHeld];
+    };
+    const int tid = threadIdx.x;
+    T* p = w.proj + (int64_t)t * w.stride;
+    const Pairs pr = w.pr;
+    const int rot = pr.rot, qd = w.dim + rot, h2 = rot / 2, turns = w.heads * h2;
+    const T* lat = p + w.lat_at;
+    Held q, k;
+    auto load = [&](Held& h, const T* x, const T* weight, int n) {
+#pragma unroll
+        for (int j = 0; j < kHeld; ++j) {
+            const int i = min(tid + j * NT, n - 1);
+            h.x[j] = x[i];
+            h.w[j] = weight[i];
+        }
+    };
+    auto factor = [&](const Held& h, const T* x, int n) {
         float ss = 0.f;
-        for (int i = threadIdx.x; i < q_rank; i += kNT) {
-            const float v = ld(p + i);
+#pragma unroll
+        for (int j = 0; j < kHeld; ++j) {
+            const float v = tid + j * NT < n ? ld(&h.x[j]) : 0.f;
             ss += v * v;
         }
-        const float r = 1.f / sqrtf(block_total<kNT>(ss, s_red) / (float)q_rank + eps);
-        for (int i = threadIdx.x; i < q_rank; i += kNT) st(p + i, ld(p + i) * r * ld(q_norm + i));
+        for (int i = tid + kHeld * NT; i < n; i += NT) {
+            const float v = ld(x + i);
+            ss += v * v;
+        }
+        return 1.f / sqrtf(block_total<NT>(ss, s_red) / (float)n + w.eps);
+    };
+    auto put = [&](const Held& h, const T* x, const T* weight, T* to, int n, float r) {
+#pragma unroll
+        for (int j = 0; j < kHeld; ++j)
+            if (tid + j * NT < n) st(to + tid + j * NT, ld(&h.x[j]) * r * ld(&h.w[j]));
+        for (int i = tid + kHeld * NT; i < n; i += NT) st(to + i, ld(x + i) * r * ld(weight + i));
+    };
+    struct Turned {
+        T u, v;
+        float c, s;
+    };
+    const float* cs = w.cos_sin + w.positions[t] * rot;
+    auto pair = [&](const T* x, int i) { return Turned{x[pr.first(i)], x[pr.second(i)], cs[i], cs[h2 + i]}; };
+    auto turn = [&](const Turned& e, T* to, int i) {
+        const float u = ld(&e.u), v = ld(&e.v);
+        st(to + pr.first(i), u * e.c - v * e.s);
+        st(to + pr.second(i), v * e.c + u * e.s);
+    };
+    auto head = [&](int e) { return p + (int64_t)(e / h2) * qd + w.dim; };
+    if (w.q_rank > 0) load(q, p, w.q_norm, w.q_rank);
+    int64_t slot = -1;
+    if (w.rank > 0) {
+        slot = w.slots[t];
+        load(k, lat, w.norm_w, w.rank);
     }
-    if (rank > 0) {
-        const T* lat = p + lat_at;
-        float ss = 0.f;
-        for (int i = threadIdx.x; i < rank; i += kNT) {
-            const float v = ld(lat + i);
-            ss += v * v;
+    Turned key{}, qs[kPairs] = {};
+    if (w.rank > 0 && h2 > 0) key = pair(lat + w.rank, min(tid, h2 - 1));
+    if (turns > 0) {
+#pragma unroll
+        for (int j = 0; j < kPairs; ++j) {
+            const int e = min(tid + j * NT, turns - 1);
+            qs[j] = pair(head(e), e % h2);
         }
-        const float r = 1.f / sqrtf(block_total<kNT>(ss, s_red) / (float)rank + eps);
-        const int64_t slot = slots[t];
+    }
+    if (w.q_rank > 0) put(q, p, w.q_norm, p, w.q_rank, factor(q, p, w.q_rank));
+    if (w.rank > 0) {
+        const float r = factor(k, lat, w.rank);
         if (slot >= 0) {
-            T* c = cache + slot * row;
-            for (int i = threadIdx.x; i < rank; i += kNT) st(c + i, ld(lat + i) * r * ld(norm_w + i));
-            for (int i = threadIdx.x; i < h2; i += kNT) {
-                const int a = pr.first(i), b = pr.second(i);
-                const float u = ld(lat + rank + a), v = ld(lat + rank + b);
-                st(c + rank + a, u * cs[i] - v * cs[h2 + i]);
-                st(c + rank + b, v * cs[i] + u * cs[h2 + i]);
-            }
+            T* c = w.cache + slot * w.row;
+            put(k, lat, w.norm_w, c, w.rank, r);
+            if (tid < h2) turn(key, c + w.rank, tid);
+            for (int i = tid + NT; i < h2; i += NT) turn(pair(lat + w.rank, i), c + w.rank, i);
         }
     }
-    for (int e = threadIdx.x; e < heads * h2; e += kNT) {
-        const int h = e / h2, i = e - h * h2;
-        T* q = p + (int64_t)h * qd + dim;
-        const int a = pr.first(i), b = pr.second(i);
-        const float u = ld(q + a), v = ld(q + b);
-        st(q + a, u * cs[i] - v * cs[h2 + i]);
-        st(q + b, v * cs[i] + u * cs[h2 + i]);
+    if (turns > 0) {
+#pragma unroll
+        for (int j = 0; j < kPairs; ++j)
+            if (tid + j * NT < turns) turn(qs[j], head(tid + j * NT), (tid + j * NT) % h2);
+        for (int e = tid + kPairs * NT; e < turns; e += NT) turn(pair(head(e), e % h2), head(e), e % h2);
     }
+}
+
+template <typename T>
+__global__ __launch_bounds__(kNT) void latent_write_kernel(Write<T> w) {
+    write_row<T, kNT>(w, blockIdx.x);
 }
 
 // What ends a head's softmax: a learned sink in the denominator and a sigmoid gate on the output, each optional.
@@ -477,6 +531,170 @@ __global__ __launch_bounds__(kWave * 2) void latent_merge_kernel(const float* __
     }
 }
 
+// ---- steps of few rows: what stands between the large products and the attention -----------------
+// Each of these is a launch of a few us that waits for the one before; what does not depend on each other shares one.
+
+// A row's write, and the up-projection of its queries' unrotated parts, which the write leaves alone: the first workgroups write a
+// token each, the others take the product (rows_batch's form of up to 256 deep). 16 heads, us: one row 4.2 + 3.7 before, now
+// 4.9; 64 rows 5.6 + 5.5, a step of two such layers 11 less.
+template <int MT>
+__global__ __launch_bounds__(kNT) void latent_lift_kernel(Write<uint16_t> w, int ntok, RowsProduct p, int cols) {
+    __shared__ __attribute__((aligned(16))) uint16_t smem[Stream<2, MT, kNT / kWave, 1>::kLds];
+    int b = blockIdx.x;
+    if (b < ntok) return write_row<uint16_t, kNT>(w, b);
+    b -= ntok;
+    rows_block<kRound, 2, MT, kNT / kWave, 1>(p, smem, b % cols, 0, b / cols, 1);
+}
+
+// The row of one query latent, normed (write_row).
+struct LatentNorm {
+    const uint16_t *x, *w;
+    int n;
+    float eps;
+    template <int MAXK>
+    struct Row {
+        uint16_t x[MAXK], w[MAXK];
+        __device__ __forceinline__ void load(const LatentNorm& p) {
+#pragma unroll
+            for (int k = 0; k < MAXK; ++k) {
+                const int i = min((int)threadIdx.x % kFormers + k * kFormers, p.n - 1);
+                x[k] = p.x[i];
+                w[k] = p.w[i];
+            }
+        }
+        static __device__ __forceinline__ int barriers(const LatentNorm&) { return 1; }
+        __device__ __forceinline__ void form(const LatentNorm& p, uint32_t to, int, uint32_t red) {
+            float ss = 0.f;
+#pragma unroll
+            for (int k = 0; k < MAXK; ++k) {
+                const float v = bf16_to_f32(x[k]);
+                if ((int)threadIdx.x % kFormers + k * kFormers < p.n) ss += v * v;
+            }
+            const float r = 1.f / sqrtf(total(ss, red) / (float)p.n + p.eps);
+#pragma unroll
+            for (int k = 0; k < MAXK; ++k) {
+                const int i = threadIdx.x % kFormers + k * kFormers;
+                if (i < p.n) lds_put16(to + 2 * i, f32_to_bf16(bf16_to_f32(x[k]) * r * bf16_to_f32(w[k])));
+            }
+        }
+        __device__ __forceinline__ void leave(const LatentNorm&) const {}
+    };
+    template <int LONG>
+    using RowOf = Row<LONG / kFormers>;
+};
+
+// One token's query latent, normed, and the product behind it; the last workgroup writes the key latent. Rank 768, 16 heads of 192:
+// 5.6 + 3.8 us before, now 5.0.
+constexpr int kQueryRank = 2048;
+__global__ __launch_bounds__(2 * kFormers) void latent_query_kernel(Write<uint16_t> w, RowsProduct p, LatentNorm pre) {
+    __shared__ __attribute__((aligned(16))) uint16_t smem[formed_lds<1, 4, kQueryRank, 1, 8>()];
+    if (blockIdx.x == gridDim.x - 1) return write_row<uint16_t, 2 * kFormers>(w, 0);
+    formed_product<kRound, 1, 4, kQueryRank, 1, 8>(p, pre, smem, 0, false);
+}
+
+// The shares of up to kMergeRows tokens' contexts, merged (latent_merge_kernel) for a head, blockIdx.z.
+constexpr int kMergeRows = 4, kMergeRank = 512, kMergeParts = 256;
+struct Merge {
+    const float *ws_o, *ws_ml;
+    const int64_t* positions;
+    int ntok, heads, rank, window, part_min, nparts;
+    HeadEnd<uint16_t> end;
+    const uint16_t* out;  // of a token whose context is one share
+    // Everything is loaded at once, ahead of the number of shares (those past it hold anything and are left out).
+    struct Row {
+        static constexpr int kAhead = 24;
+        float2 v[kAhead];  // of the thread's first two dimensions
+        float2 ml;         // of the wave's first token
+        int pos, mine;     // positions of the tokens of these
+        float sink, gate;
+        static __device__ __forceinline__ int parts(const Merge& m, int pos) {
+            return page_split(m.window > 0 ? max(0, pos - m.window + 1) : 0, pos, m.part_min, m.nparts).parts;
+        }
+        static __device__ __forceinline__ int64_t record(const Merge& m, int t) {
+            return ((int64_t)t * m.heads + blockIdx.z) * m.nparts;
+        }
+        __device__ __forceinline__ void load(const Merge& m) {
+            const int tid = threadIdx.x % kFormers, half = m.rank / 2, e = min(tid, m.ntok * half - 1), t = e / half;
+            const int own = min(tid >> 6, m.ntok - 1), rp = (m.rank + 15) / 16 * 16;
+            mine = (int)m.positions[own];
+            pos = (int)m.positions[t];
+            ml = reinterpret_cast<const float2*>(m.ws_ml)[record(m, own) + min(tid & 63, m.nparts - 1)];
+            sink = m.end.sink(blockIdx.z) * kLog2e;
+            gate = m.end.gated(own, blockIdx.z);
+            const float* src = m.ws_o + record(m, t) * rp + (e - t * half) * 2;
+#pragma unroll
+            for (int p = 0; p < kAhead; ++p) v[p] = *reinterpret_cast<const float2*>(src + min(p, m.nparts - 1) * rp);
+        }
+        static __device__ __forceinline__ int barriers(const Merge&) { return 1; }
+        __device__ __forceinline__ void form(const Merge& m, uint32_t x, int pitch, uint32_t red) {
+            typedef __attribute__((address_space(3))) const float lds_float;
+            const int tid = threadIdx.x % kFormers, lane = tid & 63, rp = (m.rank + 15) / 16 * 16, half = m.rank / 2;
+            const int own = tid >> 6;
+            static_assert(kMergeRows <= kFormers / kWave, "a wave per token");
+            if (own < m.ntok) {  // its shares' weights
+                const int n = parts(m, mine);
+                const float2* rest = reinterpret_cast<const float2*>(m.ws_ml) + record(m, own);
+                float M = lane < n ? ml.x : -INFINITY, L = 0.f;
+                for (int p = lane + kWave; p < n; p += kWave) M = fmaxf(M, rest[p].x);
+                M = wave_largest(M);
+                if (lane < n) L = fast_exp2(ml.x - M) * ml.y;
+                for (int p = lane + kWave; p < n; p += kWave) L += fast_exp2(rest[p].x - M) * rest[p].y;
+                const float inv = sum_factor(M, wave_total(L), sink) * gate;
+                if (lane < n) lds_put(red + (own * kMergeParts + lane) * 4, fast_exp2(ml.x - M) * inv);
+                for (int p = lane + kWave; p < n; p += kWave)
+                    lds_put(red + (own * kMergeParts + p) * 4, fast_exp2(rest[p].x - M) * inv);
+            }
+            lds_barrier();
+            auto place = [&](int e, int& t, int& d) {
+                t = e / half;
+                d = (e - t * half) * 2;
+            };
+            auto merged = [&](int t, int d, int n, int from, float2 acc) {
+                lds_float* wt = (lds_float*)(uintptr_t)(red + t * kMergeParts * 4);
+                const float* src = m.ws_o + record(m, t) * rp + d;
+#pragma unroll 8
+                for (int p = from; p < n; ++p) {
+                    const float w = wt[p];
+                    const float2 u = *reinterpret_cast<const float2*>(src + (int64_t)p * rp);
+                    acc.x += w * u.x;
+                    acc.y += w * u.y;
+                }
+                // one share: the row is there
+                const uint32_t y = n == 1 ? *reinterpret_cast<const uint32_t*>(m.out + ((int64_t)blockIdx.z * m.ntok + t) * m.rank + d)
+                                          : pack_bf16x2(acc.x, acc.y);
+                lds_put32(x + t * pitch + d * 2, y);
+            };
+            int t, d;
+            place(min(tid, m.ntok * half - 1), t, d);  // threads past the last do the last one's again
+            const int n = parts(m, pos);
+            lds_float* wt = (lds_float*)(uintptr_t)(red + t * kMergeParts * 4);
+            float2 acc = make_float2(0.f, 0.f);
+#pragma unroll
+            for (int p = 0; p < kAhead; ++p) {
+                const float w = wt[p];
+                acc.x = p < n ? acc.x + w * v[p].x : acc.x;
+                acc.y = p < n ? acc.y + w * v[p].y : acc.y;
+            }
+            merged(t, d, n, kAhead, acc);
+            for (int e = tid + kFormers; e < m.ntok * half; e += kFormers) {
+                place(e, t, d);
+                merged(t, d, parts(m, (int)m.positions[t]), 0, make_float2(0.f, 0.f));
+            }
+        }
+        __device__ __forceinline__ void leave(const Merge&) const {}
+    };
+    template <int>
+    using RowOf = Row;
+};
+
+// The merge and the outputs' up-projection: grid (columns / 16, 1, heads), each workgroup merges its head's rows. 16 heads, one row
+// of 17 shares: 4.5 + 3.7 us before, now 5.5.
+__global__ __launch_bounds__(2 * kFormers) void latent_merge_up_kernel(RowsProduct p, Merge pre) {
+    constexpr int kRed = kMergeRows * kMergeParts;
+    __shared__ __attribute__((aligned(16))) uint16_t smem[formed_lds<1, 2, kMergeRank, kMergeRows, kRed>()];
+    formed_product<kRound, 1, 2, kMergeRank, kMergeRows, kRed>(p, pre, smem, blockIdx.z, false);
+}
+
 // ---- prompt form --------------------------------------------------------------------------------
 // grid (ceil(max rows / 16), nseg): 16 packed rows per workgroup; rows past the segment's count up to the next
 // multiple of 64 are zeroed.
@@ -786,30 +1004,113 @@ __global__ __launch_bounds__(512 / QT) __attribute__((amdgpu_waves_per_eu(2))) v
 
 using namespace skyrl;
 
+namespace {
+
+const char* bad_write(const void* proj, int64_t proj_stride, int32_t T_, int32_t heads, int32_t dim, int32_t rot_dim, int32_t q_rank,
+                      const void* q_norm, int32_t rank, int32_t latent_at, const void* norm_weight, const int64_t* positions,
+                      const int64_t* slots, const float* cos_sin, const void* cache, int32_t row) {
+    if (!(T_ >= 0 && heads >= 0 && dim >= 0 && rot_dim >= 0 && rot_dim % 2 == 0 && rank >= 0 && q_rank >= 0))
+        return "latent_write: bad sizes";
+    if (!(heads == 0 || q_rank == 0)) return "latent_write: queries or their latent, not both";
+    if (!(rank == 0 || (row % 32 == 0 && row >= rank + rot_dim)))
+        return "latent_write: row must be a multiple of 32 >= rank + rot_dim";
+    const int64_t qw = q_rank > 0 ? q_rank : (int64_t)heads * (dim + rot_dim);
+    if (!(proj_stride >= qw && (rank == 0 || (latent_at >= qw && proj_stride >= (int64_t)latent_at + rank + rot_dim))))
+        return "latent_write: proj_stride";
+    if (T_ > 0 && !(proj && positions && cos_sin && (q_rank == 0 || q_norm) && (rank == 0 || (norm_weight && slots && cache))))
+        return "latent_write: null pointer";
+    return nullptr;
+}
+
+template <typename T>
+Write<T> write_of(void* proj, int64_t proj_stride, int32_t heads, int32_t dim, int32_t rot_dim, int32_t halves, int32_t q_rank,
+                  const void* q_norm, int32_t rank, int32_t latent_at, const void* norm_weight, float eps,
+                  const int64_t* positions, const int64_t* slots, const float* cos_sin, void* cache, int32_t row) {
+    return Write<T>{reinterpret_cast<T*>(proj), proj_stride, heads, dim, Pairs{rot_dim, halves}, q_rank,
+                    reinterpret_cast<const T*>(q_norm), rank, latent_at, reinterpret_cast<const T*>(norm_weight), eps, positions,
+                    slots, cos_sin, reinterpret_cast<T*>(cache), row};
+}
+
+}  // namespace
+
 extern "C" int skyrl_latent_write(void* proj, int64_t proj_stride, int32_t T_, int32_t heads, int32_t dim,
                                   int32_t rot_dim, int32_t halves, int32_t q_rank, const void* q_norm, int32_t rank,
                                   int32_t latent_at, const void* norm_weight, float eps, const int64_t* positions,
                                   const int64_t* slots, const float* cos_sin, void* cache, int32_t row, int32_t dtype,
                                   void* stream) {
     SKYRL_REQUIRE_T(dtype, "latent_write");
-    SKYRL_REQUIRE(T_ >= 0 && heads >= 0 && dim >= 0 && rot_dim >= 0 && rot_dim % 2 == 0 && rank >= 0 && q_rank >= 0,
-                  "latent_write: bad sizes");
-    SKYRL_REQUIRE(heads == 0 || q_rank == 0, "latent_write: queries or their latent, not both");
-    SKYRL_REQUIRE(rank == 0 || (row % 32 == 0 && row >= rank + rot_dim),
-                  "latent_write: row must be a multiple of 32 >= rank + rot_dim");
-    const int64_t qw = q_rank > 0 ? q_rank : (int64_t)heads * (dim + rot_dim);
-    SKYRL_REQUIRE(proj_stride >= qw && (rank == 0 || (latent_at >= qw && proj_stride >= (int64_t)latent_at + rank + rot_dim)),
-                  "latent_write: proj_stride");
+    const char* bad = bad_write(proj, proj_stride, T_, heads, dim, rot_dim, q_rank, q_norm, rank, latent_at, norm_weight, positions,
+                                slots, cos_sin, cache, row);
+    SKYRL_REQUIRE(!bad, bad);
     if (T_ == 0) return SKYRL_OK;
-    SKYRL_REQUIRE(proj && positions && cos_sin && (q_rank == 0 || q_norm) && (rank == 0 || (norm_weight && slots && cache)),
-                  "latent_write: null pointer");
     SKYRL_DISPATCH_T(dtype, {
         hipLaunchKernelGGL((latent_write_kernel<T>), dim3(T_), dim3(kNT), 0, as_stream(stream),
-                           reinterpret_cast<T*>(proj), proj_stride, heads, dim, Pairs{rot_dim, halves}, q_rank,
-                           reinterpret_cast<const T*>(q_norm), rank, latent_at, reinterpret_cast<const T*>(norm_weight),
-                           eps, positions, slots, cos_sin, reinterpret_cast<T*>(cache), row);
+                           write_of<T>(proj, proj_stride, heads, dim, rot_dim, halves, q_rank, q_norm, rank, latent_at, norm_weight,
+                                       eps, positions, slots, cos_sin, cache, row));
     })
     return check_launch("latent_write_kernel");
+}
+
+extern "C" int skyrl_latent_lift(void* proj, int64_t proj_stride, int32_t T_, int32_t heads, int32_t dim, int32_t rot_dim,
+                                 int32_t halves, int32_t rank, const void* norm_weight, float eps, const int64_t* positions,
+                                 const int64_t* slots, const float* cos_sin, void* cache, int32_t row, const void* up,
+                                 int32_t up_rank, void* qa, void* stream) {
+    const int latent_at = heads * (dim + rot_dim);
+    const char* bad = bad_write(proj, proj_stride, T_, heads, dim, rot_dim, 0, nullptr, rank, latent_at, norm_weight, positions, slots,
+                                cos_sin, cache, row);
+    SKYRL_REQUIRE(!bad, bad);
+    SKYRL_REQUIRE(T_ <= 64 && heads > 0 && dim > 0 && dim <= 256 && dim % 8 == 0 && up_rank > 0, "latent_lift: bad sizes");
+    if (T_ == 0) return SKYRL_OK;
+    SKYRL_REQUIRE(up && qa && aligned16(proj) && aligned16(up) && aligned16(qa) && proj_stride % 8 == 0 && (dim + rot_dim) % 8 == 0,
+                  "latent_lift: rows must be 16-byte aligned");
+    const auto w = write_of<uint16_t>(proj, proj_stride, heads, dim, rot_dim, halves, 0, nullptr, rank, latent_at, norm_weight, eps,
+                                      positions, slots, cos_sin, cache, row);
+    RowsProduct p{};
+    p.x = reinterpret_cast<const uint16_t*>(proj);
+    p.ldx = proj_stride;
+    p.n = T_;
+    p.K = dim;
+    p.w = reinterpret_cast<const uint16_t*>(up);
+    p.ldw = dim;
+    p.N = up_rank;
+    p.out = qa;
+    p.ldo = up_rank;
+    p.row_blocks = 1;
+    p.x_batch = dim + rot_dim;
+    p.w_batch = (int64_t)up_rank * dim;
+    p.out_batch = (int64_t)T_ * up_rank;
+    const int cols = (up_rank + 31) / 32;
+    const dim3 grid(T_ + cols * heads), block(kNT);
+    hipStream_t s = as_stream(stream);
+    if (T_ <= 16) hipLaunchKernelGGL(latent_lift_kernel<1>, grid, block, 0, s, w, T_, p, cols);
+    else if (T_ <= 32) hipLaunchKernelGGL(latent_lift_kernel<2>, grid, block, 0, s, w, T_, p, cols);
+    else hipLaunchKernelGGL(latent_lift_kernel<4>, grid, block, 0, s, w, T_, p, cols);
+    return check_launch("latent_lift_kernel");
+}
+
+extern "C" int skyrl_latent_query(void* proj, int64_t proj_stride, int32_t rot_dim, int32_t halves, int32_t q_rank, const void* q_norm,
+                                  int32_t rank, const void* norm_weight, float eps, const int64_t* positions,
+                                  const int64_t* slots, const float* cos_sin, void* cache, int32_t row, const void* wuq, int32_t N,
+                                  void* q, void* stream) {
+    const char* bad = bad_write(proj, proj_stride, 1, 0, 0, rot_dim, q_rank, q_norm, rank, q_rank, norm_weight, positions, slots, cos_sin,
+                                cache, row);
+    SKYRL_REQUIRE(!bad, bad);
+    SKYRL_REQUIRE(q_rank > 0 && q_rank <= kQueryRank && q_rank % 8 == 0 && N > 0, "latent_query: bad sizes");
+    SKYRL_REQUIRE(wuq && q && aligned16(wuq) && (reinterpret_cast<uintptr_t>(q) & 1) == 0, "latent_query: rows must be 16-byte aligned");
+    const auto w = write_of<uint16_t>(proj, proj_stride, 0, 0, rot_dim, halves, 0, nullptr, rank, q_rank, norm_weight, eps, positions,
+                                      slots, cos_sin, cache, row);
+    RowsProduct p{};
+    p.n = 1;
+    p.K = q_rank;
+    p.w = reinterpret_cast<const uint16_t*>(wuq);
+    p.ldw = q_rank;
+    p.N = N;
+    p.out = q;
+    p.ldo = N;
+    p.row_blocks = 1;
+    hipLaunchKernelGGL(latent_query_kernel, dim3((N + 15) / 16 + 1), dim3(2 * kFormers), 0, as_stream(stream), w, p,
+                       LatentNorm{reinterpret_cast<const uint16_t*>(proj), reinterpret_cast<const uint16_t*>(q_norm), q_rank, eps});
+    return check_launch("latent_query_kernel");
 }
 
 extern "C" int skyrl_latent_attend_mfma(int32_t rank, int32_t rot_dim, int32_t row, int32_t dtype) {
@@ -831,12 +1132,13 @@ extern "C" size_t skyrl_latent_attend_workspace_bytes(int32_t T_, int32_t heads,
     if (heads > 16) LAUNCH_ATTEND_(NV, NK, EX, 2);   \
     else LAUNCH_ATTEND_(NV, NK, EX, 1)
 
-extern "C" int skyrl_latent_attend(const void* qa, const void* q_rot, int64_t q_stride, int64_t q_head,
-                                   const void* cache, int32_t row, const int32_t* block_tables, int64_t bt_stride,
-                                   const int32_t* bt_row, const int64_t* positions, int32_t T_, int32_t heads,
-                                   int32_t rank, int32_t rot_dim, float scale, int32_t window, int32_t part_min,
-                                   int32_t nparts, const float* sinks, const void* gate, int64_t gate_stride, void* out,
-                                   void* workspace, int32_t dtype, void* stream) {
+namespace {
+
+int latent_attend(const void* qa, const void* q_rot, int64_t q_stride, int64_t q_head, const void* cache, int32_t row,
+                  const int32_t* block_tables, int64_t bt_stride, const int32_t* bt_row, const int64_t* positions, int32_t T_,
+                  int32_t heads, int32_t rank, int32_t rot_dim, float scale, int32_t window, int32_t part_min, int32_t nparts,
+                  const float* sinks, const void* gate, int64_t gate_stride, void* out, void* workspace, int32_t dtype,
+                  const RowsProduct* up, void* stream) {
     SKYRL_REQUIRE_T(dtype, "latent_attend");
     SKYRL_REQUIRE(!gate || gate_stride >= heads, "latent_attend: gate_stride");
     SKYRL_REQUIRE(T_ >= 0 && T_ <= 65535 && heads > 0 && rank > 0 && rank <= 2048 && rot_dim >= 0,
@@ -881,9 +1183,56 @@ extern "C" int skyrl_latent_attend(const void* qa, const void* q_rot, int64_t q_
     }
     int rc = check_launch("latent_attend_mfma_kernel");
     if (rc != SKYRL_OK || nparts == 1) return rc;
+    if (up) {
+        hipLaunchKernelGGL(latent_merge_up_kernel, dim3((up->N + 15) / 16, 1, heads), dim3(2 * kFormers), 0, s, *up,
+                           Merge{ws_o, ws_ml, positions, T_, heads, rank, window, part_min, nparts, end_, o_});
+        return check_launch("latent_merge_up_kernel");
+    }
     hipLaunchKernelGGL(latent_merge_kernel, dim3(heads, T_), dim3(kWave * 2), 0, s, ws_o, ws_ml, positions, T_, heads, rank,
                        window, part_min, nparts, end_, o_);
     return check_launch("latent_merge_kernel");
+}
+
+}  // namespace
+
+extern "C" int skyrl_latent_attend(const void* qa, const void* q_rot, int64_t q_stride, int64_t q_head,
+                                   const void* cache, int32_t row, const int32_t* block_tables, int64_t bt_stride,
+                                   const int32_t* bt_row, const int64_t* positions, int32_t T_, int32_t heads,
+                                   int32_t rank, int32_t rot_dim, float scale, int32_t window, int32_t part_min,
+                                   int32_t nparts, const float* sinks, const void* gate, int64_t gate_stride, void* out,
+                                   void* workspace, int32_t dtype, void* stream) {
+    return latent_attend(qa, q_rot, q_stride, q_head, cache, row, block_tables, bt_stride, bt_row, positions, T_, heads, rank, rot_dim,
+                         scale, window, part_min, nparts, sinks, gate, gate_stride, out, workspace, dtype, nullptr, stream);
+}
+
+extern "C" int32_t skyrl_latent_attend_up_fits(int32_t T_, int32_t rank, int32_t rot_dim, int32_t row, int32_t nparts) {
+    return T_ > 0 && T_ <= kMergeRows && nparts > 1 && nparts <= kMergeParts && rank % 8 == 0 && rank <= kMergeRank &&
+           skyrl_latent_attend_mfma(rank, rot_dim, row, SKYRL_BF16);
+}
+
+extern "C" int skyrl_latent_attend_up(const void* qa, const void* q_rot, int64_t q_stride, int64_t q_head,
+                                      const void* cache, int32_t row, const int32_t* block_tables, int64_t bt_stride,
+                                      const int32_t* bt_row, const int64_t* positions, int32_t T_, int32_t heads,
+                                      int32_t rank, int32_t rot_dim, float scale, int32_t window, int32_t part_min,
+                                      int32_t nparts, const float* sinks, const void* gate, int64_t gate_stride, void* out,
+                                      void* workspace, const void* up, int32_t vdim, void* y, int64_t y_token, int64_t y_head,
+                                      void* stream) {
+    SKYRL_REQUIRE(skyrl_latent_attend_up_fits(T_, rank, rot_dim, row, nparts), "latent_attend_up: sizes that it does not take");
+    SKYRL_REQUIRE(up && y && vdim > 0 && aligned16(up) && (reinterpret_cast<uintptr_t>(y) & 1) == 0,
+                  "latent_attend_up: rows must be 16-byte aligned");
+    RowsProduct p{};
+    p.n = T_;
+    p.K = rank;
+    p.w = reinterpret_cast<const uint16_t*>(up);
+    p.ldw = rank;
+    p.N = vdim;
+    p.out = y;
+    p.ldo = y_token;
+    p.row_blocks = 1;
+    p.w_batch = (int64_t)vdim * rank;
+    p.out_batch = y_head;
+    return latent_attend(qa, q_rot, q_stride, q_head, cache, row, block_tables, bt_stride, bt_row, positions, T_, heads, rank, rot_dim,
+                         scale, window, part_min, nparts, sinks, gate, gate_stride, out, workspace, SKYRL_BF16, &p, stream);
 }
 
 extern "C" int skyrl_latent_gather(const void* cache, int32_t row, const int32_t* block_tables, int64_t bt_stride,

@@ -8,45 +8,14 @@
 // Measured, us in a step's profile, both launches before and the one now (2048 deep): 3648 rows 4.4 + 5.0, 6.8; 12352 rows 4.3 +
 // 10.8, 10.9; gated 12288 rows 4.3 + 11.0, 11.3; two shares of 2112 rows 4.7 + 5.5, 6.2; behind 8 experts' rows, 12352 rows
 // 6.1 + 11.8, 11.9. Eight pieces of 16 rows (four of 64) under way: all of 2048 (half of it).
-#include "rows.h"
+#include "normed.h"
 
 namespace skyrl {
 namespace {
 
-constexpr int kNT = 256;  // threads that form the row; as many stream
+constexpr int kNT = kFormers;
 constexpr int kLongest = 4096;  // of a row
 constexpr int kShares = 4, kRows = 8;  // of a product, of a token, that are summed: all are loaded ahead of the weights
-
-// LDS by hand, since the barriers are.
-__device__ __forceinline__ uint32_t lds_at(const void* p) { return (uint32_t)(uintptr_t)(lds_void*)p; }
-__device__ __forceinline__ void lds_put(uint32_t at, float v) { asm volatile("ds_write_b32 %0, %1" ::"v"(at), "v"(v) : "memory"); }
-__device__ __forceinline__ float lds_get(uint32_t at) {
-    float v;
-    asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=v"(v) : "v"(at) : "memory");
-    return v;
-}
-__device__ __forceinline__ f32x4 lds_get4(uint32_t at) {
-    f32x4 v;
-    asm volatile("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=v"(v) : "v"(at) : "memory");
-    return v;
-}
-__device__ __forceinline__ void lds_put2(uint32_t at, uint2 v) {
-    const uint64_t w = (uint64_t)v.y << 32 | v.x;
-    asm volatile("ds_write_b64 %0, %1" ::"v"(at), "v"(w) : "memory");
-}
-__device__ __forceinline__ void lds_barrier() {
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
-// Sum over the block, in every thread; red: four floats of LDS, free again after the next barrier.
-__device__ __forceinline__ float total(float v, uint32_t red) {
-    v = wave_total(v);
-    if ((threadIdx.x & 63) == 0) lds_put(red + (threadIdx.x % kNT >> 6) * 4, v);
-    lds_barrier();
-    const f32x4 s = lds_get4(red);
-    return ((0.f + s[0]) + s[1]) + s[2] + s[3];
-}
 
 __device__ __forceinline__ float4 four(uint2 v) {
     return make_float4(__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16),
@@ -114,7 +83,7 @@ struct AddNorm {
         }
         static __device__ __forceinline__ int barriers(const AddNorm& p) { return p.kind == SKYRL_NORM_LAYER ? 2 : 1; }  // of form
         // the normed row into LDS at x
-        __device__ __forceinline__ void form(const AddNorm& p, uint32_t x, uint32_t red) {
+        __device__ __forceinline__ void form(const AddNorm& p, uint32_t x, int, uint32_t red) {
             const int nv = p.H / 4;
             float sum = 0.f, ss = 0.f;
 #pragma unroll
@@ -257,7 +226,7 @@ struct GateNorm {
         static __device__ __forceinline__ int barriers(const GateNorm& p) {
             return p.groups == 1 || p.H / 8 / p.groups > p.L ? 2 : 0;
         }
-        __device__ __forceinline__ void form(const GateNorm& p, uint32_t x, uint32_t red) {
+        __device__ __forceinline__ void form(const GateNorm& p, uint32_t x, int, uint32_t red) {
             const int nv = p.H / 8;
 #pragma unroll
             for (int k = 0; k < MAXK; ++k) {
@@ -328,47 +297,13 @@ struct GateNorm {
     using RowOf = Row<H_ / 8 / kNT>;
 };
 
+constexpr int kRed = 2 * kLongest / 8;
+
 // As rows_product_kernel with four waves, the row in all 16 places. LONG: rows up to this length.
 template <int MODE, int NT, int S, int LONG, class Pre>
 __global__ __launch_bounds__(2 * kNT) void normed_product_kernel(RowsProduct p, Pre pre) {
-    constexpr int WK = kNT / kWave;
-    using St = Stream<NT, 1, WK, S, true>;
-    using Row = typename Pre::template RowOf<LONG>;
-    constexpr int OC = out_cols<MODE, NT>(), kRed = 2 * kLongest / 8;
-    __shared__ __attribute__((aligned(16))) uint16_t smem[St::kLds + LONG + 2 * kRed];
-    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int n0 = blockIdx.x * OC;
-    const uint32_t x = lds_at(smem + St::kLds);
-    if (wave >= WK) {
-        __builtin_amdgcn_s_setprio(2);
-        Row row;
-        row.load(pre);
-        row.form(pre, x, x + LONG * 2);
-        const int end = tid - kNT;  // the last piece's end
-        if (end < (64 - p.K % 64) % 64 / 4) lds_put2(x + p.K * 2 + end * 8, make_uint2(0u, 0u));
-        lds_barrier();
-        __builtin_amdgcn_s_setprio(0);
-        if (blockIdx.x == 0 && blockIdx.y == 0) row.leave(pre);
-        __syncthreads();  // those of St::store
-        __syncthreads();
-    } else {
-        const int steps = (p.K + 63) / 64, shares = gridDim.y * WK, share = blockIdx.y * WK + wave;
-        const int s0 = (int)((int64_t)steps * share / shares), nk = (int)((int64_t)steps * (share + 1) / shares) - s0;
-        f32x4 acc[1][NT];
-        St::run(
-            smem, p.K, s0, nk,
-            [&](int r) {
-                const int at = MODE == kGated && r >= OC ? p.N + min(n0 + r - OC, p.N - 1) : min(n0 + r, p.N - 1);
-                return p.w + at * p.ldw;
-            },
-            [&](int) { return (const uint16_t*)nullptr; }, acc,
-            [&]() {
-                for (int i = Row::barriers(pre); i >= 0; --i) lds_barrier();
-                return x;
-            });
-        St::store(smem, acc);
-    }
-    put_rows<MODE, St, 2 * WK>(smem, p, n0, 0, 0);
+    __shared__ __attribute__((aligned(16))) uint16_t smem[formed_lds<NT, S, LONG, 1, kRed>()];
+    formed_product<MODE, NT, S, LONG, 1, kRed>(p, pre, smem, 0, blockIdx.x == 0 && blockIdx.y == 0);
 }
 
 constexpr int kWideCols = 8192;  // as in rows_product.hip

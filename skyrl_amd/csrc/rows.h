@@ -77,4 +77,26 @@ __device__ __forceinline__ void put_rows(const uint16_t* smem, const RowsProduct
     }
 }
 
+// NT 16-row weight tiles (kGated: half of each matrix) and MT 16-row tiles of x per workgroup, the depth in `splits` * WK shares;
+// blocks of MT tiles and products of a batch along z.
+template <int MODE, int NT, int MT, int WK, int S>
+__device__ __forceinline__ void rows_block(const RowsProduct& p, uint16_t* smem, int bx, int by, int bz, int splits) {
+    using St = Stream<NT, MT, WK, S>;
+    constexpr int BM = St::BM, OC = out_cols<MODE, NT>();
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n0 = bx * OC, batch = bz / p.row_blocks, m0 = bz % p.row_blocks * BM;
+    const int steps = (p.K + 63) / 64, shares = splits * WK, share = by * WK + wave;
+    const int s0 = (int)((int64_t)steps * share / shares), nk = (int)((int64_t)steps * (share + 1) / shares) - s0;
+    f32x4 acc[MT][NT];
+    St::run(
+        smem, p.K, s0, nk,
+        [&](int r) {  // rows past the last: the last
+            const int row = MODE == kGated && r >= OC ? p.N + min(n0 + r - OC, p.N - 1) : min(n0 + r, p.N - 1);
+            return p.w + batch * p.w_batch + row * p.ldw;
+        },
+        [&](int r) { return p.x + batch * p.x_batch + min(m0 + r, p.n - 1) * p.ldx; }, acc);
+    St::store(smem, acc);
+    put_rows<MODE, St, WK>(smem, p, n0, m0, batch);
+}
+
 }  // namespace skyrl

@@ -23,27 +23,10 @@
 namespace skyrl {
 namespace {
 
-// NT 16-row weight tiles (kGated: half of each matrix) and MT 16-row tiles of x per workgroup, the depth in gridDim.y * WK shares;
-// blocks of MT tiles and products of a batch along z.
 template <int MODE, int NT, int MT, int WK, int S>
 __global__ __launch_bounds__(WK* kWave) void rows_product_kernel(RowsProduct p) {
-    using St = Stream<NT, MT, WK, S>;
-    constexpr int BM = St::BM, OC = out_cols<MODE, NT>();
-    __shared__ __attribute__((aligned(16))) uint16_t smem[St::kLds];
-    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int n0 = blockIdx.x * OC, batch = blockIdx.z / p.row_blocks, m0 = blockIdx.z % p.row_blocks * BM;
-    const int steps = (p.K + 63) / 64, shares = gridDim.y * WK, share = blockIdx.y * WK + wave;
-    const int s0 = (int)((int64_t)steps * share / shares), nk = (int)((int64_t)steps * (share + 1) / shares) - s0;
-    f32x4 acc[MT][NT];
-    St::run(
-        smem, p.K, s0, nk,
-        [&](int r) {  // rows past the last: the last
-            const int row = MODE == kGated && r >= OC ? p.N + min(n0 + r - OC, p.N - 1) : min(n0 + r, p.N - 1);
-            return p.w + batch * p.w_batch + row * p.ldw;
-        },
-        [&](int r) { return p.x + batch * p.x_batch + min(m0 + r, p.n - 1) * p.ldx; }, acc);
-    St::store(smem, acc);
-    put_rows<MODE, St, WK>(smem, p, n0, m0, batch);
+    __shared__ __attribute__((aligned(16))) uint16_t smem[Stream<NT, MT, WK, S>::kLds];
+    rows_block<MODE, NT, MT, WK, S>(p, smem, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.y);
 }
 
 constexpr int kWide = 8192;       // output columns from which wider tiles still fill the chip and read x less often

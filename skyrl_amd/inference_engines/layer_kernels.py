@@ -527,15 +527,69 @@ def latent_write(proj, rot_dim, positions, slots, cos_sin, cache, eps, heads: in
     width = at + (rank + rot_dim if rank else 0)
     if (heads and q_rank) or proj.dim() != 2 or proj.shape[1] < width or proj.stride(1) != 1:
         raise ValueError(f"proj must be [T, >= {width}] with unit column stride, queries or their latent first")
+    _check_write(proj, rot_dim, positions, slots, cos_sin, cache, q_norm, q_rank, rank, norm_weight)
+    _ffi.call("skyrl_latent_write", _ptr(proj), proj.stride(0), T, heads, dim, rot_dim, int(halves), q_rank, _ptr(q_norm),
+              rank, at, _ptr(norm_weight), float(eps), _ptr(positions), _ptr(slots), _ptr(cos_sin), _ptr(cache),
+              cache.shape[2] if rank else 0, _code(proj), _stream(dev))
+
+
+def _check_write(proj, rot_dim, positions, slots, cos_sin, cache, q_norm, q_rank: int, rank: int, norm_weight):
+    T = proj.shape[0]
     _check_rotation(positions, cos_sin, rot_dim, T)
     _check(q_norm, "q_norm", proj.dtype, (q_rank,))
     if rank:
         _check(norm_weight, "norm_weight", proj.dtype, (rank,))
         _check(slots, "slots", torch.int64, (T,))
         _check_cache(cache, rank, rot_dim, proj.dtype)
-    _ffi.call("skyrl_latent_write", _ptr(proj), proj.stride(0), T, heads, dim, rot_dim, int(halves), q_rank, _ptr(q_norm),
-              rank, at, _ptr(norm_weight), float(eps), _ptr(positions), _ptr(slots), _ptr(cos_sin), _ptr(cache),
-              cache.shape[2] if rank else 0, _code(proj), _stream(dev))
+
+
+def _bf16_rows(*tensors) -> bool:
+    """16-byte aligned bf16 on the GPU, rows a multiple of 16 bytes apart."""
+    return all(t.dtype == torch.bfloat16 and t.is_cuda and t.stride(-1) == 1 and t.data_ptr() % 16 == 0
+               and all(s % 8 == 0 for s in t.stride()[:-1]) for t in tensors)
+
+
+LIFT_ROWS, LIFT_DIM, QUERY_RANK = 64, 256, 2048  # what skyrl_latent_lift and skyrl_latent_query take at most
+
+
+def latent_lift(proj, rot_dim, positions, slots, cos_sin, cache, eps, up, heads: int, dim: int, rank: int = 0, norm_weight=None,
+                halves: bool = False) -> Optional[torch.Tensor]:
+    """latent_write with queries and, in the same launch, rows_batch of their unrotated parts with up [heads, R, dim]: returns qa
+    [heads, T, R]; None (nothing done) for sizes and types that take two launches."""
+    T, R = proj.shape[0], up.shape[1]
+    if (not 0 < T <= LIFT_ROWS or not 0 < dim <= LIFT_DIM or dim % 8 or (dim + rot_dim) % 8 or proj.dim() != 2
+            or not _bf16_rows(proj, up) or not up.is_contiguous()):
+        return None
+    dev = _require_gpu(proj, norm_weight, positions, slots, cos_sin, cache, up)
+    width = heads * (dim + rot_dim) + (rank + rot_dim if rank else 0)
+    if proj.shape[1] < width or up.shape != (heads, R, dim):
+        raise ValueError(f"proj must be [T, >= {width}], queries first, and up [{heads}, any, {dim}]")
+    _check_write(proj, rot_dim, positions, slots, cos_sin, cache, None, 0, rank, norm_weight)
+    qa = torch.empty((heads, T, R), dtype=proj.dtype, device=dev)
+    _ffi.call("skyrl_latent_lift", _ptr(proj), proj.stride(0), T, heads, dim, rot_dim, int(halves), rank, _ptr(norm_weight),
+              float(eps), _ptr(positions), _ptr(slots), _ptr(cos_sin), _ptr(cache), cache.shape[2] if rank else 0, _ptr(up), R,
+              _ptr(qa), _stream(dev))
+    return qa
+
+
+def latent_query(proj, rot_dim, positions, slots, cos_sin, cache, eps, w, q_norm, rank: int = 0, norm_weight=None,
+                 halves: bool = False) -> Optional[torch.Tensor]:
+    """latent_write with a query latent and linear of it with w [N, q_rank], in one launch, for one token; the latent itself is not
+    stored. None (nothing done) for sizes and types that take two launches."""
+    q_rank, N = q_norm.shape[0], w.shape[0]
+    if (proj.dim() != 2 or proj.shape[0] != 1 or q_rank > QUERY_RANK or q_rank % 8 or not _bf16_rows(w) or not w.is_contiguous()
+            or proj.dtype != torch.bfloat16 or proj.stride(1) != 1):
+        return None
+    dev = _require_gpu(proj, q_norm, norm_weight, positions, slots, cos_sin, cache, w)
+    width = q_rank + (rank + rot_dim if rank else 0)
+    if proj.shape[1] < width or w.shape[1] != q_rank:
+        raise ValueError(f"proj must be [1, >= {width}], the query latent first, and w [any, {q_rank}]")
+    _check_write(proj, rot_dim, positions, slots, cos_sin, cache, q_norm, q_rank, rank, norm_weight)
+    q = torch.empty((1, N), dtype=proj.dtype, device=dev)
+    _ffi.call("skyrl_latent_query", _ptr(proj), max(proj.stride(0), width), rot_dim, int(halves), q_rank, _ptr(q_norm), rank,
+              _ptr(norm_weight), float(eps), _ptr(positions), _ptr(slots), _ptr(cos_sin), _ptr(cache),
+              cache.shape[2] if rank else 0, _ptr(w), N, _ptr(q), _stream(dev))
+    return q
 
 
 def _check_end(sinks, gate, heads, T, dtype):
@@ -546,10 +600,11 @@ def _check_end(sinks, gate, heads, T, dtype):
 
 
 def latent_attend(qa, q_rot, cache, rank, rot_dim, block_tables, bt_row, positions, scale, window, nparts=1,
-                  part_min=64, workspace=None, sinks=None, gate=None) -> torch.Tensor:
+                  part_min=64, workspace=None, sinks=None, gate=None, up=None) -> Optional[torch.Tensor]:
     """Latent-space attention, one query row per token. qa [heads, T, rank]; q_rot [T, heads, rot_dim]
     (any token and head stride); returns [heads, T, rank]. sinks f32 [heads]: exp(sink) joins the denominators; gate
-    [T, heads]: outputs times its sigmoid."""
+    [T, heads]: outputs times its sigmoid. up (w [heads, vdim, rank], y [heads, T, vdim] of any strides but the last): a few
+    tokens whose contexts are merged leave their up-projected rows in y in the merge's launch, and None is returned."""
     dev = _require_gpu(qa, q_rot, cache, block_tables, bt_row, positions, sinks, gate)
     heads, T, R = qa.shape
     _check(qa, "qa", cache.dtype, (heads, T, rank))
@@ -565,6 +620,17 @@ def latent_attend(qa, q_rot, cache, rank, rot_dim, block_tables, bt_row, positio
         ws = workspace.get(need) if workspace is not None else torch.empty(need, dtype=torch.uint8, device=dev)
     else:
         nparts = 1
+    if up is not None and qa.dtype == torch.bfloat16 and _ffi.query("skyrl_latent_attend_up_fits", T, rank, rot_dim, cache.shape[2], nparts):
+        w, y = up
+        if w.dim() == 3 and w.is_contiguous() and _bf16_rows(w) and y.dtype == torch.bfloat16 and y.stride(2) == 1:
+            if w.shape[0] != heads or w.shape[2] != rank or y.shape != (heads, T, w.shape[1]):
+                raise ValueError(f"up must be [{heads}, vdim, {rank}] and y [{heads}, {T}, vdim]")
+            _require_gpu(qa, w, y)
+            _ffi.call("skyrl_latent_attend_up", _ptr(qa), _ptr(q_rot), q_rot.stride(0), q_rot.stride(1), _ptr(cache),
+                      cache.shape[2], _ptr(block_tables), block_tables.stride(0), _ptr(bt_row), _ptr(positions), T, heads,
+                      rank, rot_dim, float(scale), int(window or 0), part_min, nparts, _ptr(sinks), _ptr(gate), gate_stride,
+                      _ptr(out), _ptr(ws), _ptr(w), w.shape[1], _ptr(y), y.stride(1), y.stride(0), _stream(dev))
+            return None
     _ffi.call("skyrl_latent_attend", _ptr(qa), _ptr(q_rot), q_rot.stride(0), q_rot.stride(1), _ptr(cache),
               cache.shape[2], _ptr(block_tables), block_tables.stride(0), _ptr(bt_row), _ptr(positions), T, heads,
               rank, rot_dim, float(scale), int(window or 0), part_min, nparts, _ptr(sinks), _ptr(gate), gate_stride,

@@ -391,8 +391,8 @@ class LatentAttention:
         return int(_ffi.query("skyrl_latent_attend_workspace_bytes", tokens, self.heads, self.rank, n)) if n > 1 else 0
 
     # ---- step
-    def _attend_rows(self, q, gate, out, inp, a: int, b: int, cache, workspace):
-        """Tokens [a, b) in the decode form. More than lk.ORDERED_ROWS of them in a step of more than lk.MAX_ROWS tokens, whose
+    def _attend_rows(self, q, gate, out, inp, a: int, b: int, cache, workspace, qa=None):
+        """Tokens [a, b) in the decode form (qa: their up-projected queries where these are there already). More than lk.ORDERED_ROWS of them in a step of more than lk.MAX_ROWS tokens, whose
         products are all the library's, have its bits in their up-projections too, and beside portions the shares that fill a
         round: such a row is what it was whatever is the faster form of fewer rows (shares that fit: 19 us less a layer for 48
         rows beside prompts, of a step of 2100 us)."""
@@ -400,33 +400,40 @@ class LatentAttention:
         n = b - a
         many = q.shape[0] > lk.MAX_ROWS and n > lk.ORDERED_ROWS
         q3 = q[a:b].view(n, H, D + self.rot_dim)
-        qa = torch.empty((H, n, R), dtype=q.dtype, device=q.device)
-        if not lk.rows_batch(q3[:, :, :D].transpose(0, 1), self.wuk_t, qa, in_order=many):
-            qa = torch.bmm(q3[:, :, :D].transpose(0, 1), self.wuk.view(H, D, R))
+        if qa is None:
+            qa = torch.empty((H, n, R), dtype=q.dtype, device=q.device)
+            if not lk.rows_batch(q3[:, :, :D].transpose(0, 1), self.wuk_t, qa, in_order=many):
+                qa = torch.bmm(q3[:, :, :D].transpose(0, 1), self.wuk.view(H, D, R))
+        to = out[a:b].view(n, H, self.vdim).transpose(0, 1)
         o = lk.latent_attend(qa, q3[:, :, D:], cache, R, self.rot_dim, inp.block_tables, inp.bt_row[a:b],
                              inp.positions[a:b], self.scale, self.window,
                              nparts=self.nparts(n, inp.max_ctx, up=many and not inp.one_token),
                              part_min=kernels.MIN_PARTITION, workspace=workspace, sinks=self.sinks,
-                             gate=None if gate is None else gate[a:b])
-        to = out[a:b].view(n, H, self.vdim).transpose(0, 1)
-        if not lk.rows_batch(o, self.wuv.view(H, self.vdim, R), to, in_order=many):
+                             gate=None if gate is None else gate[a:b], up=(self.wuv.view(H, self.vdim, R), to))
+        if o is not None and not lk.rows_batch(o, self.wuv.view(H, self.vdim, R), to, in_order=many):
             to.copy_(torch.bmm(o, self.wuv_t))
 
     def inner(self, proj: torch.Tensor, out: torch.Tensor, inp, cache: torch.Tensor, workspace) -> None:
         H, T, qr = self.heads, proj.shape[0], self.q_rank
         where = (self.rot_dim, inp.positions, inp.slots, self.cos_sin, cache, self.eps)
         own = {} if self.kv_from is not None else {"rank": self.rank, "norm_weight": self.dkv_norm}
-        first = {"q_norm": self.dq_norm} if qr else {"heads": H, "dim": self.dim}
-        lk.latent_write(proj, *where, halves=self.halves, **first, **own)
-        q = proj[:, :self.q_rows]
-        if qr:
-            q = lk.linear(q, self.wuq)
-            lk.latent_write(q, *where, heads=H, dim=self.dim, halves=self.halves)
-        gate = None if self.gate_at is None else proj[:, self.gate_at:]
+        own["halves"] = self.halves
         prompt = inp.plan is not None and self.window in inp.plan and lk.prefill_fits(self.dim, self.rot_dim, self.vdim, self.dtype)
         ts = inp.short_tokens if prompt else T
+        q, heads = proj, {"heads": H, "dim": self.dim}
+        if qr:
+            q = lk.latent_query(proj, *where, self.wuq, self.dq_norm, **own)
+            if q is None:
+                lk.latent_write(proj, *where, q_norm=self.dq_norm, **own)
+                q = lk.linear(proj[:, :self.q_rows], self.wuq)
+            own = {"halves": self.halves}
+        qa = lk.latent_lift(q, *where, self.wuk_t, **heads, **own) if ts == T else None
+        if qa is None:
+            lk.latent_write(q, *where, **heads, **own)
+        q = q[:, :H * (self.dim + self.rot_dim)]
+        gate = None if self.gate_at is None else proj[:, self.gate_at:]
         for a in range(0, ts, 32768):  # the decode form's grid limit
-            self._attend_rows(q, gate, out, inp, a, min(ts, a + 32768), cache, workspace)
+            self._attend_rows(q, gate, out, inp, a, min(ts, a + 32768), cache, workspace, qa)
         if ts < T:
             seg, tiles, rows, longest = inp.plan[self.window]
             latent, k_rot = lk.latent_gather(cache, self.rank, self.rot_dim, inp.block_tables, seg, rows, longest)

@@ -111,6 +111,76 @@ def test_latent_attend(heads, rank, rot, window, dtype):
         close(out, want, dtype)
 
 
+def _write_case(n, width, rot, rank, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    rand = lambda *s: torch.randn(*s, device=DEV, generator=g)  # noqa: E731
+    proj = rand(n, (width + rank + rot + 7) // 8 * 8 + 8).bfloat16()
+    pos = torch.randint(0, 90, (n,), device=DEV, generator=g)
+    slots = torch.randperm(n + 16, device=DEV, generator=g)[:n]
+    slots[n // 2] = -1 if n > 1 else slots[0]
+    cache = torch.zeros((n // 16 + 2, 16, (rank + rot + 31) // 32 * 32), device=DEV, dtype=torch.bfloat16)
+    r = {"base": 1000.0, "dims": rot}
+    return rand, proj, (rot, pos, slots, mixers.rotary_table(r, 100).to(DEV)), cache
+
+
+@pytest.mark.parametrize("n", (1, 2, 16, 17, 33, 64))
+@pytest.mark.parametrize("heads,dim,rot,rank,up", [(2, 8, 8, 16, 24), (3, 72, 24, 40, 40), (16, 128, 64, 512, 512), (2, 256, 64, 0, 64)])
+def test_writes_beside_an_up_projection(n, heads, dim, rot, rank, up):
+    """One launch for what two did: the same rows, cache and products."""
+    rand, proj, where, cache = _write_case(n, heads * (dim + rot), rot, rank, n + heads)
+    w, nw = rand(heads, up, dim).bfloat16(), rand(rank).bfloat16() if rank else None
+    args = dict(heads=heads, dim=dim, rank=rank, norm_weight=nw, halves=bool(heads % 2))
+    p2, c2 = proj.clone(), cache.clone()
+    lk.latent_write(p2, *where, c2, 1e-4, **args)
+    want = torch.empty(heads, n, up, device=DEV, dtype=torch.bfloat16)
+    q = p2[:, :heads * (dim + rot)].view(n, heads, dim + rot)[:, :, :dim].transpose(0, 1)
+    assert lk.rows_batch(q, w, want)
+    qa = lk.latent_lift(proj, *where, cache, 1e-4, w, **args)
+    assert torch.equal(proj, p2) and torch.equal(qa, want)
+    if rank:  # sums of 128 threads instead of 256: a bf16 step where they round apart
+        d = (cache.float() - c2.float()).abs()
+        assert float((d - 2.0 ** -7 * c2.float().abs()).max()) <= 0 and int((d > 0).sum()) <= 0.01 * d.numel()
+    assert lk.latent_lift(torch.cat([proj] * 65)[:65], *where, cache, 1e-4, w, **args) is None
+
+
+@pytest.mark.parametrize("q_rank,N,rank,rot", [(8, 16, 16, 8), (200, 72, 40, 24), (768, 3072, 512, 64), (2048, 40, 0, 64), (1536, 24, 512, 64)])
+def test_query_latent_ahead_of_its_product(q_rank, N, rank, rot):
+    rand, proj, where, cache = _write_case(1, q_rank, rot, rank, q_rank)
+    w, qn, nw = rand(N, q_rank).bfloat16(), rand(q_rank).bfloat16(), rand(rank).bfloat16() if rank else None
+    p2, c2, before = proj.clone(), cache.clone(), proj.clone()
+    lk.latent_write(p2, *where, c2, 1e-4, q_norm=qn, rank=rank, norm_weight=nw)
+    want = lk.linear(p2[:, :q_rank], w)
+    q = lk.latent_query(proj, *where, cache, 1e-4, w, qn, rank=rank, norm_weight=nw)
+    assert torch.equal(proj, before)
+    ref = p2[:, :q_rank].double() @ w.double().t()
+    assert float((q.double() - ref).norm()) <= 2.0 ** -8 * float(ref.norm()) and q.shape == want.shape
+    if rank:
+        assert float((cache.float() - c2.float()).abs().max()) <= 2.0 ** -7 * float(c2.float().abs().max())
+    assert lk.latent_query(torch.cat([proj] * 2), *where, cache, 1e-4, w, qn) is None
+
+
+@pytest.mark.parametrize("T,heads,rank,rot,vdim", [(1, 16, 512, 64, 128), (2, 3, 40, 24, 24), (3, 16, 512, 64, 128), (4, 32, 256, 64, 40)])
+@pytest.mark.parametrize("ends", (False, True))
+def test_merge_ahead_of_the_up_projection(T, heads, rank, rot, vdim, ends):
+    g = torch.Generator().manual_seed(rank + T)
+    pos = [333, 5, 200, 64][:T]
+    cache, tables, _ = paged_latents(g, [p + 1 for p in pos], rank, rot, torch.bfloat16)
+    q = rnd(g, T, heads, rank + rot, dtype=torch.bfloat16).to(DEV)
+    qa = q[:, :, :rank].transpose(0, 1).contiguous()
+    w = rnd(g, heads, vdim, rank, dtype=torch.bfloat16).to(DEV)
+    iota = torch.arange(T, dtype=torch.int32, device=DEV)
+    ended = dict(sinks=rnd(g, heads, dtype=torch.float32).to(DEV), gate=rnd(g, T, heads, dtype=torch.bfloat16).to(DEV)) if ends else {}
+    for nparts, part_min, window in ((3, 16, None), (40, 16, 100), (40, 64, None)):
+        args = (qa, q[:, :, rank:], cache.to(DEV), rank, rot, tables.to(DEV), iota, torch.tensor(pos, device=DEV),
+                1.0 / math.sqrt(rank + rot), window)
+        o = lk.latent_attend(*args, nparts=nparts, part_min=part_min, **ended)
+        y = torch.full((T, heads, vdim + 8), float("nan"), device=DEV, dtype=torch.bfloat16)[:, :, :vdim].transpose(0, 1)
+        assert lk.latent_attend(*args, nparts=nparts, part_min=part_min, up=(w, y), **ended) is None
+        ref = torch.stack([o[h].cpu().double() @ w[h].cpu().double().t() for h in range(heads)])
+        assert float((y.cpu().double() - ref).norm()) <= 2.0 ** -8 * float(ref.norm())
+    assert lk.latent_attend(*args, up=(w, y)) is not None  # one share: no merge
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("heads,dim,rot,rank", [(3, 20, 12, 40), (16, 128, 64, 512), (1, 7, 2, 9)])
 def test_latent_write(heads, dim, rot, rank, dtype):
