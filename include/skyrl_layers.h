@@ -455,6 +455,9 @@ int skyrl_gdelta_out(const skyrl_gdelta_shape* shape, const int32_t* chunk, int3
  *   skyrl_moe_route    idx i32 [n, top], weight f32 [n, top] (the scores s of the chosen).
  *   skyrl_moe_choose   the same from logits f32 that are the sum of `shares` rows share_stride apart, row_stride between
  *                      tokens (at most 64 experts), and, with order, skyrl_moe_sort of them (at most 128 pairs).
+ *   skyrl_moe_one      one token in bf16: skyrl_moe_choose and skyrl_moe_gate_up of its pairs in one launch, in tiles of 16
+ *                      rows, tile k of choice k: idx, weight [top], order [top, 16], tile_expert [top + 1], act [16 top, ff] (of a
+ *                      tile its first row) for skyrl_moe_down.
  *   skyrl_moe_tiles    the most tiles of tm rows that npairs pairs can fill.
  *   skyrl_moe_sort     pairs by expert: order i32 [ntiles, tm] (pair, or -1), tile_expert i32 [ntiles + 1] (-1: unused; the
  *                      last: tiles in use). counts: scratch of skyrl_moe_counts(experts, npairs) i32 (0: NULL).
@@ -469,6 +472,9 @@ int skyrl_moe_route(const skyrl_moe_shape* shape, const void* x, int32_t n, cons
 int skyrl_moe_choose(const skyrl_moe_shape* shape, const float* logits, int32_t shares, int64_t share_stride,
                      int64_t row_stride, int32_t n, const float* correction, int32_t* idx, float* weight, int32_t tm,
                      int32_t ntiles, int32_t* order, int32_t* tile_expert, void* stream);
+int skyrl_moe_one(const skyrl_moe_shape* shape, const float* logits, int32_t shares, int64_t share_stride,
+                  const float* correction, const void* x, const void* w, int32_t* idx, float* weight, int32_t* order,
+                  int32_t* tile_expert, void* act, void* stream);
 int32_t skyrl_moe_tiles(int32_t experts, int32_t npairs, int32_t tm);
 int32_t skyrl_moe_counts(int32_t experts, int32_t npairs);
 int skyrl_moe_sort(const int32_t* idx, int32_t npairs, int32_t experts, int32_t tm, int32_t ntiles, int32_t* counts,

@@ -1318,6 +1318,31 @@ def moe_choose(sh, logits, column: int, correction, tm: int):
     return idx, weight, order, tile_expert
 
 
+def moe_one(sh, logits, column: int, correction, x, gate_up, down) -> Optional[torch.Tensor]:
+    """moe_choose and moe_experts of one token, the choice in the experts' first launch; None for sizes that take their own."""
+    if x.shape[0] != 1 or x.dtype != torch.bfloat16 or sh.experts > CHOOSE_EXPERTS or sh.width % 8 or sh.ff % 8 or not _bf16_rows(x, gate_up, down):
+        return None
+    dev = _require_gpu(logits, correction, x, gate_up, down)
+    shares, n, N = logits.shape
+    _check(logits, "logits", torch.float32, (shares, 1, N))
+    _check(correction, "correction", torch.float32, (sh.experts,))
+    _check(x, "x", torch.bfloat16, (1, sh.width))
+    _check(gate_up, "gate_up", x.dtype, (sh.experts, 2, sh.ff, sh.width))
+    _check(down, "down", x.dtype, (sh.experts, sh.width, sh.ff))
+    if not 0 <= column <= N - sh.experts:
+        raise ValueError("moe_one: the router's logits are columns of the product")
+    idx, order = (torch.empty(s, dtype=torch.int32, device=dev) for s in ((sh.top,), (sh.top, 16)))
+    tile_expert, weight = torch.empty(sh.top + 1, dtype=torch.int32, device=dev), torch.empty(sh.top, dtype=torch.float32, device=dev)
+    act = torch.empty((sh.top * 16, sh.ff), dtype=x.dtype, device=dev)
+    out = torch.empty((sh.top, sh.width), dtype=x.dtype, device=dev)
+    ref, st = ctypes.byref(sh), _stream(dev)
+    _ffi.call("skyrl_moe_one", ref, ctypes.c_void_p(logits.data_ptr() + 4 * column), shares, N, _ptr(correction), _ptr(x),
+              _ptr(gate_up), _ptr(idx), _ptr(weight), _ptr(order), _ptr(tile_expert), _ptr(act), st)
+    _ffi.call("skyrl_moe_down", ref, _ptr(act), _ptr(down), _ptr(order), _ptr(tile_expert), 16, sh.top, _ptr(weight), _ptr(out),
+              _code(x), st)
+    return out
+
+
 def moe_tile(sh, n: int) -> int:
     """Rows per tile of the experts' products for n tokens."""
     mean = n * sh.top / sh.experts

@@ -1101,6 +1101,9 @@ class RoutedExperts:
     def forward(self, x: torch.Tensor, inp, state, workspace, logits=None) -> torch.Tensor:
         """logits: (layer_kernels.linear's parts that hold the router's, their first column)."""
         if logits is not None:
+            y = lk.moe_one(self.shape, *logits, self.correction, x, self.gate_up, self.down)
+            if y is not None:
+                return y
             tm = lk.moe_rows(self.shape, x.shape[0])
             idx, weight, *tiles = lk.moe_choose(self.shape, *logits, self.correction, tm)
             return lk.moe_experts(self.shape, x, idx, weight, self.gate_up, self.down, tm, tiles)

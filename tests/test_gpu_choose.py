@@ -75,3 +75,25 @@ def test_joint_product_chooses_as_the_router(dev, n):
     pick = lambda i: (at + corr.double()).gather(1, i.long())  # noqa: E731
     torch.testing.assert_close(pick(idx), pick(other), atol=1e-5, rtol=0)
     torch.testing.assert_close(weight.double(), at.gather(1, idx.long()), atol=1e-5, rtol=0)
+
+
+@pytest.mark.parametrize("experts,groups,keep,top,width,ff", [(64, 8, 4, 8, 512, 96), (60, 12, 5, 7, 72, 40), (33, 3, 2, 22, 64, 8),
+                                                              (8, 2, 2, 8, 2048, 768), (1, 1, 1, 1, 8, 24)])
+@pytest.mark.parametrize("shares", (1, 3))
+def test_choice_in_the_first_product(dev, experts, groups, keep, top, width, ff, shares):
+    """One token: the experts and weights of moe_choose and, bit for bit, the rows of its products."""
+    g = torch.Generator(device=dev).manual_seed(experts + shares)
+    sh = lk.moe_shape(width, ff, experts, top, groups, keep)
+    logits = torch.randn(shares, 1, 24 + experts, device=dev, generator=g)
+    corr = torch.randn(experts, device=dev, generator=g) * 0.3
+    rand = lambda *s: (torch.randn(*s, device=dev, generator=g) * 0.1).bfloat16()  # noqa: E731
+    x, gate_up, down = rand(1, width), rand(experts, 2, ff, width), rand(experts, width, ff)
+    for z in (logits, torch.full_like(logits, float("nan"))):
+        idx, weight, order, tile_expert = lk.moe_choose(sh, z, 24, corr, 16)
+        want = lk.moe_experts(sh, x, idx, weight, gate_up, down, 16, (order, tile_expert))
+        got = lk.moe_one(sh, z, 24, corr, x, gate_up, down)
+        if z is logits:
+            assert torch.equal(got, want) and got.shape == (top, width)
+        else:
+            assert bool(got.isnan().all())
+    assert lk.moe_one(sh, logits, 24, corr, torch.cat([x, x]), gate_up, down) is None
