@@ -532,34 +532,148 @@ __global__ __launch_bounds__(kNT) void delta_chunk_kernel(Dims d, const int32_t*
 
 // One workgroup per (sequence, head, 16 columns of S). NS: 16-wide steps of dim (EXACT: dim = 16 NS); DT
 // 16-row tiles of S per wave; SETS: register sets of operands. With two (dim up to 128) a chunk's operands are under way for
-// the whole chunk before: they come from HBM, and a chunk's f32 products take 1.7 us. Only U = U0 - W S and the update of S
-// are a chain; the products that end in the output stand where the others' results go through LDS. Bound: the f32 matrix
-// rate (178 us for 8192 tokens of 32 heads of 128 x 128). Measured there: 712 us with operands in rows, loaded half a chunk
-// ahead, and products in the order of the equations; 412 us this way, of which 300 with operands that are in L2 (three
-// sets spill, and a touch of the lines two chunks ahead is waited for itself: loads return in order).
+// the whole chunk before. Only U = U0 - W S and the update of S are a chain, which four waves walk; four others, one beside each
+// on its SIMD, form the outputs, so that the matrix unit has work while a chain's wave waits for LDS or for the others.
+// Operands come from HBM and each is read by all slices of S: a slice's threads touch their share of the lines two chunks ahead,
+// else all of them ask for a line that is still on its way (418 us against 370 below).
+// Bound: the f32 matrix rate (178 us for 8192 tokens of 32 heads of 128 x 128). Measured there: 712 us with operands in rows,
+// loaded half a chunk ahead, and products in the order of the equations; 418 us with one set of waves for both, products that end
+// in the output where the others' results go through LDS; 328 us this way, 298 with operands that are in L2.
 template <int NS, bool EXACT, int SETS>
-__global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(1))) void delta_chain_kernel(
+__global__ __launch_bounds__(2 * kNT) __attribute__((amdgpu_waves_per_eu(2))) void delta_chain_kernel(
     Dims d, SeqRef sq, const int32_t* __restrict__ seq_chunks, int seq0, int nseq, const float* __restrict__ qk,
     const float* __restrict__ kt, const float* __restrict__ W, const float* __restrict__ U, const float* __restrict__ P,
     const float* __restrict__ G, float* __restrict__ state, float* __restrict__ o) {
     constexpr int LS = NS * 16 + 4, LU = kC + 4, DT = (NS + 3) / 4;
     __shared__ __attribute__((aligned(16))) float s_s[2][16 * LS];   // S^T slice, by turns
-    __shared__ __attribute__((aligned(16))) float s_u[2][16 * LU];   // U^T and its decayed copy
+    __shared__ __attribute__((aligned(16))) float s_u[2][16 * LU];   // U^T, by turns
+    __shared__ __attribute__((aligned(16))) float s_d[16 * LU];      // decayed
     const int V16 = d.v16(), D16 = EXACT ? NS * 16 : d.d16(), VP = d.vpad(), nt = V16 / 16;
-    // the slices of one (sequence, head) read the same W, Q, K and P: consecutive on one XCD
-    const int xcd = blockIdx.x % 8, slot = blockIdx.x / 8, grp = slot / nt * 8 + xcd;
+    // the slices of one (sequence, head) read the same W, Q, K and P, neighbouring heads the same Q and K: on one XCD
+    const int xcd = blockIdx.x % 8, slot = blockIdx.x / 8, grp = xcd * ((nseq * d.H + 7) / 8) + slot / nt;
     if (grp >= nseq * d.H) return;
     const int vt = slot % nt, h = grp % d.H, si = grp / d.H;
     const int seq = seq0 + si, row = sq.rows[seq];
     if (row < 0) return;
     const int64_t pos0 = sq.positions[sq.cu[seq]];
     const int kh = h / (d.H / d.K);
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tid = threadIdx.x % kNT, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const bool outputs = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) != 0;
     const int c = lane & 15, g = lane >> 4;
     const int ns = EXACT ? NS : D16 / 16;
+    const int c0 = seq_chunks[si], c1 = seq_chunks[si + 1];
+    if (c0 >= c1) return;
+    const int vcol = 16 * vt + c, goff = 16 * wave + 4 * g, woff = wave * ns * kTile + 4 * lane;
+    // What is the same in every lane stays a vector load, which is waited for a step later with the others: a scalar one is waited
+    // for with the next LDS read, and a value that the compiler knows to be uniform is moved to a scalar at once.
+    int zero;
+    asm("v_mov_b32 %0, 0" : "=v"(zero));
+    auto read_s = [&](int B, float4 (&b)[NS]) {
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+            if (EXACT || s < ns) b[s] = ld4(&s_s[B][c * LS + 16 * s + 4 * g]);
+    };
+    // The loop has both turns or none: with a way from the first to itself past the second, even one that is never taken, it would
+    // wait for all its loads at once, as nothing is known to be behind them. The last chunk's loads are its own again: loads
+    // without a branch.
+    auto walk = [&](auto step) {
+        int ci = c0;
+        for (; ci + 1 < c1; ci += 2) {
+            step(std::integral_constant<int, 0>{}, ci);
+            step(std::integral_constant<int, 1>{}, ci + 1);
+        }
+        if (ci < c1) step(std::integral_constant<int, 0>{}, ci);
+    };
+    if (outputs) {
+        struct Operands {
+            float4 q[NS], eg;
+        } in[SETS];
+        float4 p[4], ul[4];
+        int t0 = 0, n = 0, t1, n1;  // first token, tokens (any chunk may be short): of the outputs under way, of p's chunk
+        // Lines of 128 bytes of a chunk's W, q and k transposed (ns * 4 KB, ns * 32 lines each) and P (16 KB).
+        const int per = ns * 32, line = vt * kNT + tid, sec = line / per;
+        const char* ahead = sec == 0   ? reinterpret_cast<const char*>(W + (int64_t)h * 4 * ns * kTile) + line * 128
+                            : sec == 1 ? reinterpret_cast<const char*>(qk + (int64_t)kh * 8 * ns * kTile) + (line - per) * 128
+                            : sec == 2 ? reinterpret_cast<const char*>(kt + (int64_t)kh * 4 * ns * kTile) + (line - 2 * per) * 128
+                                       : reinterpret_cast<const char*>(P + (int64_t)h * 16 * kTile) + min(line - 3 * per, 127) * 128;
+        const int64_t ahead_step = (int64_t)(sec == 0 ? d.H * 4 * ns : sec == 1 ? d.K * 8 * ns : sec == 2 ? d.K * 4 * ns : d.H * 16) * kTile * 4;
+        int touched = 0;
+        const int ostep = d.H * d.V;
+        auto load_q = [&](Operands& x, int ci, int s) {
+            if (EXACT || s < ns) x.q[s] = ld4(qk + ((int64_t)ci * d.K + kh) * 8 * ns * kTile + woff + s * kTile);
+        };
+        auto load_eg = [&](Operands& x, int ci) { x.eg = ld4(G + ((int64_t)ci * d.H + h) * 2 * kC + goff); };
+        auto load_p = [&](int ci) {
+            const int64_t ch = (int64_t)ci * d.H + h;
+#pragma unroll
+            for (int s = 0; s < 4; ++s)  // lower triangular: the blocks above are loaded, not used
+                p[s] = ld4(P + ((ch * 4 + wave) * 4 + s) * kTile + 4 * lane);
+            const int2 at = *reinterpret_cast<const int2*>(sq.chunk + 4 * ci + zero);
+            t1 = at.x;
+            n1 = at.y;
+        };
+        // A chunk's outputs are a phase behind the chain: diag(e^G) Q S while it updates S, mostly, and P U while it forms the
+        // next U. What is read of LDS is read a phase ahead.
+        f32x4 ao = {0.f, 0.f, 0.f, 0.f};
+        auto finish = [&]() {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {  // the blocks above the diagonal as zeros: behind a branch their loads would be, too
+                const bool in = s <= wave;
+                ao = mma4(make_float4(in ? p[s].x : 0.f, in ? p[s].y : 0.f, in ? p[s].z : 0.f, in ? p[s].w : 0.f), ul[s], ao);
+            }
+            t0 = t1, n = n1;
+            float* op = o + ((int64_t)t0 * d.H + h) * d.V;
+            if (vcol < d.V) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (goff + i < n) op[(goff + i) * ostep + vcol] = ao[i];
+            }
+        };
+        load_eg(in[0], c0);
+#pragma unroll
+        for (int s = 0; s < NS; ++s) load_q(in[0], c0, s);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) p[s] = ul[s] = make_float4(0.f, 0.f, 0.f, 0.f);
+        t1 = n1 = 0;
+        walk([&](auto turn, int ci) {
+            constexpr int B = decltype(turn)::value, EARLY = NS / 4;
+            Operands &x = in[B % SETS], &next = in[(B + 1) % SETS];
+            const int cn = min(ci + 1, c1 - 1);
+            __syncthreads();  // S^T of the chunk before is in LDS
+            float4 b[NS];
+            read_s(B, b);
+            finish();  // the chunk before; at the first, nothing
+            load_p(ci);
+            if (SETS > 1) load_eg(next, cn);
+            asm volatile("" ::"v"(touched));
+            touched = *reinterpret_cast<const int*>(ahead + min(ci + 2, c1 - 1) * ahead_step);
+            ao = f32x4{0.f, 0.f, 0.f, 0.f};
+            auto product = [&](int s) {  // a load a product: a burst of them would hold the products up
+                if (EXACT || s < ns) ao = mma4(x.q[s], b[s], ao);
+                if (SETS > 1) load_q(next, cn, s);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+#pragma unroll
+            for (int s = 0; s < EARLY; ++s) product(s);
+            __syncthreads();  // U^T is
+#pragma unroll
+            for (int s = 0; s < 4; ++s) ul[s] = ld4(&s_u[B][c * LU + 16 * s + 4 * g]);
+#pragma unroll
+            for (int s = EARLY; s < NS; ++s) product(s);
+            ao[0] *= x.eg.x;
+            ao[1] *= x.eg.y;
+            ao[2] *= x.eg.z;
+            ao[3] *= x.eg.w;
+            if constexpr (SETS == 1) {
+                load_eg(next, cn);
+#pragma unroll
+                for (int s = 0; s < NS; ++s) load_q(next, cn, s);
+            }
+        });
+        finish();
+        return;
+    }
     float* st_ = state + ((int64_t)row * d.H + h) * d.D * VP;
-    const int vcol = 16 * vt + c;
-
     // this wave's rows of S: tiles wave, wave + 4, ...; element i: dim 16 tile + 4 g + i, column c
     f32x4 S[DT];
 #pragma unroll
@@ -572,118 +686,80 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(1))) void d
         }
         if (EXACT || tile < ns) *reinterpret_cast<f32x4*>(&s_s[0][c * LS + 16 * tile + 4 * g]) = S[k];
     }
-    const int c0 = seq_chunks[si], c1 = seq_chunks[si + 1];
-    if (c0 >= c1) return;
-    const int goff = 16 * wave + 4 * g, ostep = d.H * d.V, woff = wave * ns * kTile + 4 * lane;
     struct Operands {
-        float4 w[NS], q[NS], p[4], kk[DT][4], u0, eg, er;
+        float4 w[NS], kk[DT][4], u0, er;
         float decay;
-        int t0, n;  // first token, tokens: any chunk may be short
     } in[SETS];
-    // the parts of a chunk's operands that a step of 16 dims, or of 16 tokens, needs
+    auto load_w = [&](Operands& x, int ci, int s) {
+        if (EXACT || s < ns) x.w[s] = ld4(W + ((int64_t)ci * d.H + h) * 4 * ns * kTile + woff + s * kTile);
+    };
     auto load_ends = [&](Operands& x, int ci) {
         const int64_t ch = (int64_t)ci * d.H + h;
         x.u0 = ld4(U + ((ch * nt + vt) * 4 + wave) * kTile + 4 * lane);
-        x.eg = ld4(G + ch * 2 * kC + goff);
         x.er = ld4(G + ch * 2 * kC + kC + goff);
-        x.decay = G[ch * 2 * kC + kC - 1];
-        x.t0 = sq.chunk[4 * ci];
-        x.n = sq.chunk[4 * ci + 1];
+        x.decay = G[ch * 2 * kC + kC - 1 + zero];
     };
-    auto load_dims = [&](Operands& x, int ci, int s) {
-        if (!EXACT && s >= ns) return;
-        x.w[s] = ld4(W + ((int64_t)ci * d.H + h) * 4 * ns * kTile + woff + s * kTile);
-        x.q[s] = ld4(qk + ((int64_t)ci * d.K + kh) * 8 * ns * kTile + woff + s * kTile);
-    };
-    auto load_tokens = [&](Operands& x, int ci, int s) {
+    auto load_k = [&](Operands& x, int ci, int s) {
 #pragma unroll
         for (int k = 0; k < DT; ++k)
             if (EXACT || wave + 4 * k < ns)
                 x.kk[k][s] = ld4(kt + (((int64_t)ci * d.K + kh) * ns + wave + 4 * k) * 4 * kTile + s * kTile + 4 * lane);
-        if (SETS > 1 || s <= wave)  // P is lower triangular: the blocks above are loaded, not used
-            x.p[s] = ld4(P + ((((int64_t)ci * d.H + h) * 4 + wave) * 4 + s) * kTile + 4 * lane);
     };
-    auto step = [&](auto turn, int ci) {
+    load_ends(in[0], c0);
+#pragma unroll
+    for (int s = 0; s < NS; ++s) load_w(in[0], c0, s);
+    if constexpr (SETS > 1) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) load_k(in[0], c0, s);
+    }
+    __builtin_amdgcn_s_setprio(1);  // ahead of the outputs' waves
+    walk([&](auto turn, int ci) {
         constexpr int B = decltype(turn)::value;
         Operands &x = in[B % SETS], &next = in[(B + 1) % SETS];
-        const int cn = min(ci + 1, c1 - 1);  // the last chunk's again: loads without a branch are waited for one by one
+        const int cn = min(ci + 1, c1 - 1);
         if constexpr (SETS == 1) {
 #pragma unroll
-            for (int s = 0; s < 4; ++s) load_tokens(x, ci, s);
+            for (int s = 0; s < 4; ++s) load_k(x, ci, s);
         }
-        __syncthreads();  // S^T of the previous chunk is in LDS
+        __syncthreads();  // S^T of the chunk before is in LDS
         float4 b[NS];
-#pragma unroll
-        for (int s = 0; s < NS; ++s)
-            if (EXACT || s < ns) b[s] = ld4(&s_s[B][c * LS + 16 * s + 4 * g]);
-        const float4 eg = x.eg;  // with one set the next chunk's take their place
-        const float decay = x.decay;
-        const int t0 = x.t0, n = x.n;
-        f32x4 aw = {0.f, 0.f, 0.f, 0.f}, ao = aw;
-        // A load a product or two: a burst of them would hold the products up.
+        read_s(B, b);
+        const float decay = x.decay;  // with one set the next chunk's takes its place
+        f32x4 aw = {0.f, 0.f, 0.f, 0.f};
         if constexpr (SETS > 1) load_ends(next, cn);
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
             if (EXACT || s < ns) aw = mma4(x.w[s], b[s], aw);
-            if (SETS > 1) load_dims(next, cn, s);
+            if (SETS > 1) load_w(next, cn, s);
             __builtin_amdgcn_sched_barrier(0);
         }
         const float4 u = make_float4(x.u0.x - aw[0], x.u0.y - aw[1], x.u0.z - aw[2], x.u0.w - aw[3]);
-        st4(&s_u[0][c * LU + goff], u);
-        st4(&s_u[1][c * LU + goff], make_float4(u.x * x.er.x, u.y * x.er.y, u.z * x.er.z, u.w * x.er.w));
-#pragma unroll
-        for (int s = 0; s < NS; ++s) {
-            if (EXACT || s < ns) ao = mma4(x.q[s], b[s], ao);
-            if (SETS > 1 && s < 4) load_tokens(next, cn, s);
-            __builtin_amdgcn_sched_barrier(0);
-        }
+        st4(&s_u[B][c * LU + goff], u);
+        st4(&s_d[c * LU + goff], make_float4(u.x * x.er.x, u.y * x.er.y, u.z * x.er.z, u.w * x.er.w));
 #pragma unroll
         for (int k = 0; k < DT; ++k) S[k] = S[k] * decay;
-        __syncthreads();
-        float4 ud[4], ul[4];
+        __syncthreads();  // U^T is
+        float4 ud[4];
 #pragma unroll
-        for (int s = 0; s < 4; ++s) ud[s] = ld4(&s_u[1][c * LU + 16 * s + 4 * g]);
+        for (int s = 0; s < 4; ++s) ud[s] = ld4(&s_d[c * LU + 16 * s + 4 * g]);
 #pragma unroll
-        for (int s = 0; s < 4; ++s) ul[s] = ld4(&s_u[0][c * LU + 16 * s + 4 * g]);
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
+        for (int s = 0; s < 4; ++s) {
 #pragma unroll
             for (int k = 0; k < DT; ++k)
                 if (EXACT || wave + 4 * k < ns) S[k] = mma4(x.kk[k][s], ud[s], S[k]);
+            if (SETS > 1) load_k(next, cn, s);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         if constexpr (SETS == 1) {
             load_ends(next, cn);
 #pragma unroll
-            for (int s = 0; s < NS; ++s) load_dims(next, cn, s);
+            for (int s = 0; s < NS; ++s) load_w(next, cn, s);
         }
 #pragma unroll
         for (int k = 0; k < DT; ++k)
             if (EXACT || wave + 4 * k < ns)
                 *reinterpret_cast<f32x4*>(&s_s[1 - B][c * LS + 16 * (wave + 4 * k) + 4 * g]) = S[k];
-        ao[0] *= eg.x;
-        ao[1] *= eg.y;
-        ao[2] *= eg.z;
-        ao[3] *= eg.w;
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-            if (s <= wave) ao = mma4(x.p[s], ul[s], ao);
-        float* op = o + ((int64_t)t0 * d.H + h) * d.V;
-        if (vcol < d.V) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                if (goff + i < n) op[(goff + i) * ostep + vcol] = ao[i];
-        }
-    };
-    load_ends(in[0], c0);
-#pragma unroll
-    for (int s = 0; s < NS; ++s) load_dims(in[0], c0, s);
-    if constexpr (SETS > 1) {
-#pragma unroll
-        for (int s = 0; s < 4; ++s) load_tokens(in[0], c0, s);
-    }
-    for (int ci = c0; ci < c1; ci += 2) {
-        step(std::integral_constant<int, 0>{}, ci);
-        if (ci + 1 < c1) step(std::integral_constant<int, 1>{}, ci + 1);
-    }
+    });
 #pragma unroll
     for (int k = 0; k < DT; ++k)
 #pragma unroll
@@ -847,7 +923,7 @@ extern "C" int skyrl_delta_chunk(const skyrl_delta_shape* shape, const int32_t* 
 
 #define LAUNCH_CHAIN(NS, EXACT, SETS)                                                                           \
     hipLaunchKernelGGL((delta_chain_kernel<NS, EXACT, SETS>),                                                           \
-                       dim3((unsigned)(nseq * d.H + 7) / 8 * 8 * (d.v16() / 16)), dim3(kNT), 0, as_stream(stream), \
+                       dim3((unsigned)(nseq * d.H + 7) / 8 * 8 * (d.v16() / 16)), dim3(2 * kNT), 0, as_stream(stream), \
                        d, SeqRef{chunk, cu, rows, positions}, seq_chunks, seq0, nseq, qk, kt, W, U, P, G, state, o)
 
 extern "C" int skyrl_delta_chain(const skyrl_delta_shape* shape, const int32_t* chunk, const int32_t* seq_chunks,

@@ -445,6 +445,21 @@ def test_delta_chunks_of_any_length(shape, monkeypatch):
     close(c.S[1][..., :c.sh.vdim], Sb, torch.float32)
 
 
+@pytest.mark.parametrize("shape,n", [((9, 3, 128, 128, 4), 64), ((9, 3, 128, 128, 4), 65), ((1, 1, 128, 16, 1), 1101),
+                                     ((4, 2, 64, 128, 4), 1217), ((2, 1, 16, 256, 2), 700), ((3, 1, 240, 32, 4), 450)])
+def test_delta_walks_of_odd_and_even_turns(shape, n):
+    """One chunk, two, many; few slices of the state and many; heads that do not fill the XCDs evenly."""
+    c = DeltaCase(*shape, torch.float32, seed=n)
+    a = c.inputs(n)
+    want, S = c.oracle(a)
+    for row, part in ((1, n), (3, n - 64 if n > 100 else n)):  # whole, and continued by a second step
+        out = [c.step([(row, 0, a[:part])], 0)[0]]
+        if part < n:
+            out.append(c.step([(row, part, a[part:])], 0)[0])
+        close(torch.cat(out), want, torch.float32)
+        close(c.S[row][..., :c.sh.vdim], S, torch.float32, f32=1e-4)
+
+
 # ---------------------------------------------------------------- the model through the engine's steps
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name", sorted(CONFIGS))
