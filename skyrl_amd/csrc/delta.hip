@@ -378,7 +378,9 @@ __device__ __forceinline__ float4 as_float4(const f32x4& v) { return make_float4
 // diagonal block by substitution, the blocks below follow diagonal by diagonal from
 // T_rb = -T_rr sum_k A_rk T_kb, and T then multiplies both right-hand sides. A 16 x 16 result's registers
 // (rows 4 g + i, column c) are the next product's right operand as they are, and a transposed product's are its operand order.
-__global__ __launch_bounds__(kNT) void delta_chunk_kernel(Dims d, const int32_t* __restrict__ chunk,
+// Bound: 600 MB of HBM and the f32 products, about as long (8192 tokens of 32 heads of 128 x 128: 75 us each); the next slab and
+// the next right-hand side are loaded while one is worked on: 158 us, where each was loaded when it was due 176.
+__global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(4))) void delta_chunk_kernel(Dims d, const int32_t* __restrict__ chunk,
                                                           const float* __restrict__ qk, const float* __restrict__ kt,
                                                           const float* __restrict__ vt, const float* __restrict__ lg, const float* __restrict__ beta,
                                                           float* __restrict__ W, float* __restrict__ U,
@@ -421,16 +423,28 @@ __global__ __launch_bounds__(kNT) void delta_chunk_kernel(Dims d, const int32_t*
     }
     const int nd = D16 / 16;
     const float* qp = qk + ((int64_t)ci * d.K + kh) * 2 * 4 * nd * kTile;
+    float4 slab[2][4];  // of q and k: four dim tiles of every token tile, the next ones while these are worked on
+    auto load_slab = [&](int d0) {
+        const int w = min(4, nd - d0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {  // token tile i; tiles past the last: the last again
+            const int x = min(tid, w * kWave - 1);
+            const float* src = qp + (i * nd + d0) * kTile + x * 4;
+            slab[0][i] = ld4(src);
+            slab[1][i] = ld4(src + 4 * nd * kTile);
+        }
+    };
+    static_assert(kNT == 4 * kWave, "a token tile's four dim tiles by one pass of the threads");
+    load_slab(0);
     for (int d0 = 0; d0 < nd; d0 += 4) {
         const int w = min(4, nd - d0);
         __syncthreads();
-        for (int e = tid; e < 4 * 4 * kWave; e += kNT) {  // four dim tiles of every token tile
-            const int i = e >> 8, x = e & 255;
-            if (x >> 6 >= w) continue;
-            const float* src = qp + (i * nd + d0) * kTile + x * 4;
-            st4(&s_q[e * 4], ld4(src));
-            st4(&s_k[e * 4], ld4(src + 4 * nd * kTile));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            st4(&s_q[(i * kNT + tid) * 4], slab[0][i]);
+            st4(&s_k[(i * kNT + tid) * 4], slab[1][i]);
         }
+        if (d0 + 4 < nd) load_slab(d0 + 4);
         __syncthreads();
         for (int s = 0; s < w; ++s) {
 #pragma unroll
@@ -443,6 +457,18 @@ __global__ __launch_bounds__(kNT) void delta_chunk_kernel(Dims d, const int32_t*
         }
     }
     __syncthreads();
+    // the right-hand sides, a tile ahead of their use
+    const int nv = V16 / 16;
+    float4 ahead[4];
+    auto load_x = [&](int tile) {  // past the last: the last again
+        tile = min(tile, nd + nv - 1);
+        const bool isw = tile < nd;
+        const int vtile = tile - nd;
+        const float* src = (isw ? kt + (((int64_t)ci * d.K + kh) * nd + tile) * 4 * kTile : vt + (ch * nv + vtile) * 4 * kTile) + lane * 4;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) ahead[s] = ld4(src + s * kTile);
+    };
+    load_x(wave);
     float *s_a = s_k, *s_t = s_q;
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
@@ -502,15 +528,14 @@ __global__ __launch_bounds__(kNT) void delta_chunk_kernel(Dims d, const int32_t*
     }
     __syncthreads();
     // T times [diag(beta e^G) K | diag(beta) V], 16 columns at a time; the first transposed
-    const int nv = V16 / 16;
     for (int tile = wave; tile < nd + nv; tile += 4) {
         const bool isw = tile < nd;
         const int vtile = tile - nd;
-        const float* src = (isw ? kt + (((int64_t)ci * d.K + kh) * nd + tile) * 4 * kTile : vt + (ch * nv + vtile) * 4 * kTile) + lane * 4;
         const bool on = isw || 16 * vtile + c < d.V;  // columns past vdim hold nothing
         float4 x[4];
 #pragma unroll
-        for (int s = 0; s < 4; ++s) x[s] = on ? ld4(src + s * kTile) : make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int s = 0; s < 4; ++s) x[s] = on ? ahead[s] : make_float4(0.f, 0.f, 0.f, 0.f);
+        load_x(tile + 4);
         f32x4 o[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) o[r] = f32x4{0.f, 0.f, 0.f, 0.f};
