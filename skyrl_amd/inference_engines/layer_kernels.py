@@ -1344,9 +1344,15 @@ def moe_one(sh, logits, column: int, correction, x, gate_up, down) -> Optional[t
 
 
 def moe_tile(sh, n: int) -> int:
-    """Rows per tile of the experts' products for n tokens."""
-    mean = n * sh.top / sh.experts
-    return 256 if mean >= 112 else 128 if mean >= 48 else 64 if mean >= 12 else 16
+    """Rows per tile of the experts' products for n tokens. Tiles of 64 rather than 128 up to 60 rows an expert where the gated ones
+    have the narrow form (up to 2048 wide; 64 experts, 8 a token, both products, us: 768 x 2048, 384 tokens 138 against 165, 448
+    150 / 165, 512 170 / 167; 1536 x 4096, 384 tokens 466 / 494 and, unevenly loaded, 531 / 500, 448 528 / 489). 128 rather than
+    256 up to 200 where a quarter of the wide form's columns would be none and 256 rows are staged (576 x 1536: 800 tokens 113 /
+    134, 1200 146 / 141, 2000 168 / 164; 768 x 2048, 896 tokens 194 / 186). Widths below 1024, whose products are launches, as the
+    widest."""
+    mean, real = n * sh.top / sh.experts, sh.width >= 1024
+    return (256 if mean >= (200 if real and sh.ff % 128 else 112) else 128 if mean >= (60 if real and sh.width <= 2048 else 48)
+            else 64 if mean >= 12 else 16)
 
 
 def moe_rows(sh, n: int) -> int:
