@@ -59,7 +59,9 @@ extern "C" {
  *   skyrl_add_norm_product, skyrl_gate_norm_product  one row of a model in bf16: the norm of skyrl_add_norm_parts (parts 0: no
  *                   sum) or skyrl_gate_norm_add_parts and skyrl_rows_product of the normed row, in one launch. The residual is
  *                   read from h and leaves in h_out, another buffer; x_out (may be NULL): the normed row. turn0, turn1 as
- *                   skyrl_rows_product_tanh's columns (equal: none; not with splits or act). skyrl_normed_product_fits: whether a
+ *                   skyrl_rows_product_tanh's columns (equal: none; not with splits or act). With tokens the row begins at
+ *                   row tokens[0] of table bf16 [*, K]: add_norm's residual is that times scale (h is not read), and
+ *                   gate_norm's `a` is that, without a gate, the residual 0 before (a, gate, gate_bias and h are not read). skyrl_normed_product_fits: whether a
  *                   row of K with that many shares (of the sum or of the gate's logits) and rows to be summed is taken.
  *   skyrl_gated_product  many rows: the gated product (act of skyrl_gate_mul) of x bf16 [n, K] (row stride ldx) and w bf16
  *                   [N gate rows, N up rows] (row stride ldw), rows 16-byte aligned, as bf16 [n, N] contiguous: summed and
@@ -114,6 +116,9 @@ typedef struct {
     void* out;
     int32_t K, N, act, splits, turn0, turn1;
     float alpha, limit;
+    const int64_t* tokens;
+    const void* table;
+    float scale;
 } skyrl_normed_product;
 int32_t skyrl_normed_product_fits(int32_t K, int32_t shares, int32_t rows);
 int skyrl_add_norm_product(const skyrl_normed_product* product, const float* delta, int32_t parts, const void* step,

@@ -276,7 +276,7 @@ class NormedProduct(ctypes.Structure):
 
     _fields_ = [("h", _P), ("h_out", _P), ("x_out", _P), ("w", _P), ("ldw", _I64), ("bias", _P), ("out", _P)] + [
         (n, ctypes.c_int32) for n in ("K", "N", "act", "splits", "turn0", "turn1")] + [
-        (n, ctypes.c_float) for n in ("alpha", "limit")]
+        (n, ctypes.c_float) for n in ("alpha", "limit")] + [("tokens", _P), ("table", _P), ("scale", ctypes.c_float)]
 
 
 # the exported surface of include/skyrl_layers.h, in libraries of its own (LAYER_LIBS)

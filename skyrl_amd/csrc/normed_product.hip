@@ -5,6 +5,7 @@
 // forms the row for itself, from 24 to 60 KB of which its L2 has most, while its first pieces of the weights are on their way: four
 // waves stream, four form the row (a wave that did both would wait for its weights with its row). Sums are in the order of add_norm_kernel and gate_norm_add_kernel, the same bits. The first workgroup leaves the new residual,
 // in another buffer, since the rest still read the old one, and the normed row where a later launch reads it too.
+// The first row of a step is read from the embedding's table in the same way (a step of one row 5.5 us less).
 // Measured, us in a step's profile, both launches before and the one now (2048 deep): 3648 rows 4.4 + 5.0, 6.8; 12352 rows 4.3 +
 // 10.8, 10.9; gated 12288 rows 4.3 + 11.0, 11.3; two shares of 2112 rows 4.7 + 5.5, 6.2; behind 8 experts' rows, 12352 rows
 // 6.1 + 11.8, 11.9. Eight pieces of 16 rows (four of 64) under way: all of 2048 (half of it).
@@ -58,17 +59,23 @@ struct AddNorm {
     int kind;
     float* h_out;
     uint16_t* out;
+    const int64_t* tokens;  // the residual is a row of table times scale (NULL: h)
+    const uint16_t* table;
+    float scale;
 
     template <int MAXK>  // groups of four a thread
     struct Row {
         float4 h[MAXK], d[kShares][MAXK], kept[MAXK];
-        uint2 s[MAXK], w[MAXK], y[MAXK];
+        uint2 s[MAXK], w[MAXK], y[MAXK], e[MAXK];
         __device__ __forceinline__ void load(const AddNorm& p) {
             const int nv = p.H / 4;
 #pragma unroll
             for (int k = 0; k < MAXK; ++k) {
                 const int v = min((int)threadIdx.x % kNT + k * kNT, nv - 1);
-                h[k] = ld4(p.h + 4 * v);
+                h[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+                e[k] = make_uint2(0u, 0u);
+                if (p.tokens) e[k] = *reinterpret_cast<const uint2*>(p.table + p.tokens[0] * p.H + 4 * v);
+                else h[k] = ld4(p.h + 4 * v);
                 w[k] = *reinterpret_cast<const uint2*>(p.w + 4 * v);
                 s[k] = make_uint2(0u, 0u);
                 if (p.step) s[k] = *reinterpret_cast<const uint2*>(p.step + 4 * v);
@@ -90,6 +97,10 @@ struct AddNorm {
             for (int k = 0; k < MAXK; ++k) {
                 const int v = threadIdx.x % kNT + k * kNT;
                 if (v >= nv) continue;
+                if (p.tokens) {
+                    const float4 x = four(e[k]);
+                    h[k] = make_float4(x.x * p.scale, x.y * p.scale, x.z * p.scale, x.w * p.scale);
+                }
 #pragma unroll
                 for (int i = 1; i < kShares; ++i) {
                     d[0][k].x += d[i][k].x; d[0][k].y += d[i][k].y; d[0][k].z += d[i][k].z; d[0][k].w += d[i][k].w;
@@ -153,6 +164,7 @@ struct GateNorm {
     int H;
     float* h_out;
     uint16_t* out;
+    const int64_t* tokens;  // the row of a, with no gate and a residual that starts at 0 (NULL: neither)
 
     template <int MAXK>  // groups of eight a thread
     struct Row {
@@ -167,8 +179,11 @@ struct GateNorm {
 #pragma unroll
             for (int k = 0; k < MAXK; ++k) {
                 const int v = 8 * min((int)threadIdx.x % kNT + k * kNT, nv - 1);
-                hh[k].load(p.h + v);
-                b[k].load(p.zb + v);
+                hh[k] = Eight<float>{};
+                if (!p.tokens) {
+                    hh[k].load(p.h + v);
+                    b[k].load(p.zb + v);
+                }
                 w[k].load(p.w + v);
                 wn[k].load(p.wn + v);
 #pragma unroll
@@ -179,7 +194,7 @@ struct GateNorm {
 #pragma unroll
                 for (int i = 0; i < NA; ++i) {
                     a[i][k] = Eight<A>{};
-                    if (i < p.parts) a[i][k].load(p.a + i * p.H + v);
+                    if (i < p.parts) a[i][k].load(p.a + (p.tokens ? p.tokens[0] + i : i) * p.H + v);
                 }
             }
         }
@@ -248,12 +263,13 @@ struct GateNorm {
 #pragma unroll
                     for (int j = 0; j < 8; ++j) zz[j] += x[j];
                 }
-                b[k].get(x);
+                if (!p.tokens) {
+                    b[k].get(x);
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    y[k][j] *= sigmoid_<uint16_t>(zz[j] + x[j]);
-                    r[k] += y[k][j] * y[k][j];
+                    for (int j = 0; j < 8; ++j) y[k][j] *= sigmoid_<uint16_t>(zz[j] + x[j]);
                 }
+#pragma unroll
+                for (int j = 0; j < 8; ++j) r[k] += y[k][j] * y[k][j];
             }
             scales(p, red);
 #pragma unroll
@@ -335,7 +351,7 @@ bool aligned(const void* p) { return !p || aligned16(p); }
 
 // The product's operands; an error's text, or NULL.
 const char* bad_product(const skyrl_normed_product* q) {
-    if (!q || !q->w || !q->out || !q->h || !q->h_out) return "normed_product: null pointer";
+    if (!q || !q->w || !q->out || !q->h_out || (q->tokens ? !q->table : !q->h)) return "normed_product: null pointer";
     if (q->K <= 0 || q->K > kLongest || q->K % 8 != 0 || q->N <= 0 || q->ldw < q->K || q->ldw % 8 != 0)
         return "normed_product: bad sizes";
     if (q->h == q->h_out) return "normed_product: the residual must leave in another buffer";
@@ -344,7 +360,7 @@ const char* bad_product(const skyrl_normed_product* q) {
         return "normed_product: a gated product has an activation, no bias and no splits";
     if (q->splits && q->splits != skyrl_rows_product_splits(1, q->K, q->N))
         return "normed_product: splits are skyrl_rows_product_splits'";
-    if (!aligned16(q->w) || !aligned16(q->h) || !aligned16(q->h_out) || !aligned(q->x_out) ||
+    if (!aligned16(q->w) || !aligned(q->h) || !aligned(q->table) || !aligned16(q->h_out) || !aligned(q->x_out) ||
         (reinterpret_cast<uintptr_t>(q->out) & (q->splits ? 3 : 1)))
         return "normed_product: rows must be 16-byte aligned";
     return nullptr;
@@ -384,7 +400,8 @@ extern "C" int skyrl_add_norm_product(const skyrl_normed_product* q, const float
     SKYRL_REQUIRE(weight && parts >= 0 && parts <= kShares && (parts == 0 || delta), "add_norm_product: null pointer, or more shares than are taken");
     SKYRL_REQUIRE(aligned(delta) && aligned(step) && aligned16(weight), "add_norm_product: rows must be 16-byte aligned");
     const AddNorm pre{delta, parts, q->h, reinterpret_cast<const uint16_t*>(step), reinterpret_cast<const uint16_t*>(weight), w_base,
-                      q->K, eps, kind, q->h_out, reinterpret_cast<uint16_t*>(q->x_out)};
+                      q->K, eps, kind, q->h_out, reinterpret_cast<uint16_t*>(q->x_out), q->tokens,
+                      reinterpret_cast<const uint16_t*>(q->table), q->scale};
     return run(product(q), pre, q->act >= 0, q->splits, as_stream(stream));
 }
 
@@ -393,13 +410,17 @@ extern "C" int skyrl_gate_norm_product(const skyrl_normed_product* q, const void
                                        int32_t groups, float eps, float mult, const void* next, void* stream) {
     const char* bad = bad_product(q);
     SKYRL_REQUIRE(!bad, bad);
-    SKYRL_REQUIRE(a && gate && gate_bias && weight && next, "gate_norm_product: null pointer");
+    if (q->tokens) {
+        a = q->table;
+        a_shares = 0, parts = 1, gate = gate_bias = nullptr, gate_shares = 1, gate_stride = q->K;
+    }
+    SKYRL_REQUIRE(a && weight && next && (q->tokens || (gate && gate_bias)), "gate_norm_product: null pointer");
     SKYRL_REQUIRE(groups > 0 && q->K % groups == 0 && q->K / groups % 8 == 0, "gate_norm_product: groups must be multiples of 8");
     SKYRL_REQUIRE((a_shares > 0) != (gate_shares > 0) && parts > 0 && (a_shares == 0 || parts == 1) &&
                       a_shares <= kShares && gate_shares <= kShares && parts <= kRows && (gate_shares == 0 || gate_stride >= q->K) &&
                       gate_stride % 4 == 0,
                   "gate_norm_product: either the rows or the gate's logits are a product's shares");
-    SKYRL_REQUIRE(aligned16(a) && aligned16(gate) && aligned16(gate_bias) && aligned16(weight) && aligned16(next),
+    SKYRL_REQUIRE(aligned16(a) && aligned(gate) && aligned(gate_bias) && aligned16(weight) && aligned16(next),
                   "gate_norm_product: rows must be 16-byte aligned");
     int L = 1;
     while (L < kWave && q->K / 8 / groups % (2 * L) == 0) L <<= 1;
@@ -407,8 +428,8 @@ extern "C" int skyrl_gate_norm_product(const skyrl_normed_product* q, const void
     uint16_t* x = reinterpret_cast<uint16_t*>(q->x_out);
     if (a_shares)
         return run(product(q), GateNorm<float, uint16_t>{reinterpret_cast<const float*>(a), a_shares, reinterpret_cast<const uint16_t*>(gate),
-                   1, 0, gate_bias, w, groups, L, eps, mult, q->h, wn, q->K, q->h_out, x}, q->act >= 0, q->splits, as_stream(stream));
+                   1, 0, gate_bias, w, groups, L, eps, mult, q->h, wn, q->K, q->h_out, x, nullptr}, q->act >= 0, q->splits, as_stream(stream));
     return run(product(q), GateNorm<uint16_t, float>{reinterpret_cast<const uint16_t*>(a), parts, reinterpret_cast<const float*>(gate),
-               gate_shares, gate_stride, gate_bias, w, groups, L, eps, mult, q->h, wn, q->K, q->h_out, x}, q->act >= 0, q->splits,
+               q->tokens ? 0 : gate_shares, gate_stride, gate_bias, w, groups, L, eps, mult, q->h, wn, q->K, q->h_out, x, q->tokens}, q->act >= 0, q->splits,
                as_stream(stream));
 }

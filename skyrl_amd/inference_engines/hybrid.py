@@ -328,15 +328,23 @@ class HybridDecoder:
         if s.design.sandwich:
             return self._run_sandwich(inp, cache, want, trail)
         norm = dict(eps=s.norm_eps, kind=s.design.norm, base=s.design.norm_base)
-        h = lk.embed(inp.tokens, self.embed, s.embed_scale)
-        x = torch.empty(h.shape, dtype=self.dtype, device=self.device)
+        n = inp.tokens.shape[0]
+        one = trail is None and n == 1  # a row whose norms are formed in the products behind them
+        h = None if one else lk.embed(inp.tokens, self.embed, s.embed_scale)
+        x = torch.empty((n, s.hidden_size), dtype=self.dtype, device=self.device)
         delta = None
-        form = lk.normed if trail is None else lk.add_norm
+        form = lk.normed if one else lk.add_norm
         ws = self.workspace if inp.one_token else self.portion_workspace
         for r, state in zip(s.runs, cache.runs):
             step = None if r.step is None else self.loop_step[r.step]
             for weight, sub in self.layers[r.layer]["subs"]:
-                rows = form(delta, h, weight, step=step, out=x, **norm)
+                rows = None
+                if h is None:
+                    rows = lk.normed_embedding(inp.tokens, self.embed, s.embed_scale, weight, step=step, **norm)
+                    if rows is None:
+                        h = lk.embed(inp.tokens, self.embed, s.embed_scale)
+                if rows is None:
+                    rows = form(delta, h, weight, step=step, out=x, **norm)
                 delta, step = sub.forward(rows, inp, state, ws, parts=True), None
                 h = lk.residual(rows, h)
             if trail is not None:
@@ -377,8 +385,12 @@ class HybridDecoder:
         steps = [(state, *sub) for r, state in zip(s.runs, cache.runs) for sub in self.layers[r.layer]["subs"]]
         ends = {sum(len(self.layers[q.layer]["subs"]) for q in s.runs[:k + 1]) - 1 for k in range(len(s.runs))}
         before = [st[1] for st in steps] + [self.norm]  # the norm ahead of every sublayer, then the final one
-        h = torch.empty((inp.tokens.shape[0], s.hidden_size), dtype=torch.float32, device=self.device)
-        x = lk.gate_norm_add(self.embed, h, self.embed_norm, before[0], rows=inp.tokens, fresh=True, **norm)
+        h, x = None, None
+        if trail is None and inp.tokens.shape[0] == 1:
+            x = lk.gate_normed_embedding(inp.tokens, self.embed, self.embed_norm, before[0], **norm)
+        if x is None:
+            h = torch.empty((inp.tokens.shape[0], s.hidden_size), dtype=torch.float32, device=self.device)
+            x = lk.gate_norm_add(self.embed, h, self.embed_norm, before[0], rows=inp.tokens, fresh=True, **norm)
         ws = self.workspace if inp.one_token else self.portion_workspace
         for k, (state, _, sub, after) in enumerate(steps):
             y, gate = sub.forward(x, inp, state, ws)

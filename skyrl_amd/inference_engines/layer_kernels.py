@@ -65,16 +65,16 @@ def embed(tokens: torch.Tensor, table: torch.Tensor, scale: float, positions: Op
 # ---------------------------------------------------------------- the norm ahead of a product
 class NormedRow:
     """A row [1, H] whose norm is formed by the first product of it (skyrl_add_norm_product, skyrl_gate_norm_product), or by a
-    launch of its own when something else asks for the rows. `hidden` is the residual, of before or, afterwards, of behind the
-    norm."""
+    launch of its own when something else asks for the rows. `hidden` is the residual, of before (None: an embedding's, which is
+    read with the row) or, afterwards, of behind the norm; `alone` returns that."""
 
-    def __init__(self, hidden: torch.Tensor, out: torch.Tensor, fused, alone):
+    def __init__(self, hidden: Optional[torch.Tensor], out: torch.Tensor, fused, alone):
         self.hidden, self.out, self.fused, self.alone = hidden, out, fused, alone
         self.shape, self.dtype, self.device = out.shape, out.dtype, out.device
 
     def rows(self) -> torch.Tensor:
         if self.alone is not None:
-            self.alone(self.out)
+            self.hidden = self.alone(self.out)
             self.fused = self.alone = None
         return self.out
 
@@ -92,8 +92,8 @@ class NormedRow:
         splits = int(_ffi.query("skyrl_rows_product_splits", 1, H, N)) if parts else 0
         y = (torch.empty((splits, 1, N), dtype=torch.float32, device=dev) if splits
              else torch.empty((1, N), dtype=torch.bfloat16, device=dev))
-        h = torch.empty_like(self.hidden)
-        q = _ffi.NormedProduct(self.hidden.data_ptr(), h.data_ptr(), self.out.data_ptr(), w.data_ptr(), w.stride(0),
+        h = torch.empty((1, H), dtype=torch.float32, device=dev)
+        q = _ffi.NormedProduct(None if self.hidden is None else self.hidden.data_ptr(), h.data_ptr(), self.out.data_ptr(), w.data_ptr(), w.stride(0),
                                None if bias is None else bias.data_ptr(), y.data_ptr(), H, N, ACTIVATIONS[act] if gated else -1,
                                splits, *(turn or (0, 0)), alpha, limit)
         if not self.fused(q, gated, splits):
@@ -132,10 +132,11 @@ def normed(delta: Optional[torch.Tensor], hidden: torch.Tensor, weight: torch.Te
     parts = delta.shape[0] if delta is not None and delta.dim() == 3 else 0
 
     def alone(to):
-        return add_norm(delta, hidden, weight, eps, kind, step, to, base)
+        add_norm(delta, hidden, weight, eps, kind, step, to, base)
+        return hidden
 
     if (delta is not None and not parts) or not _row_fits(hidden, weight, parts, 1, delta, step, out):
-        return alone(out)
+        return add_norm(delta, hidden, weight, eps, kind, step, out, base)
     _check(hidden, "hidden", torch.float32)
     _check(weight, "weight", torch.bfloat16, (H,))
     _check(delta, "delta", torch.float32, (parts, 1, H))
@@ -162,12 +163,13 @@ def gate_normed(a: torch.Tensor, hidden: torch.Tensor, weight: torch.Tensor, nex
     gate_shares = gate.shape[0] if gate is not None and gate.dim() == 3 else 0
 
     def alone(to):
-        return gate_norm_add(a, hidden, weight, next_weight, eps, groups, mult, parts, gate, gate_bias, out=to)
+        gate_norm_add(a, hidden, weight, next_weight, eps, groups, mult, parts, gate, gate_bias, out=to)
+        return hidden
 
     if (gate is None or gate_bias is None or bool(shares) == bool(gate_shares) or groups < 1 or H % groups or H // groups % 8
             or (shares and parts != 1) or (gate_shares and gate.shape[2] % 4)
             or not _row_fits(hidden, weight, max(shares, gate_shares), parts, a, next_weight, gate, gate_bias, out)):
-        return alone(out)
+        return gate_norm_add(a, hidden, weight, next_weight, eps, groups, mult, parts, gate, gate_bias, out=out)
     _check(hidden, "hidden", torch.float32)
     _check(a, "a", torch.float32 if shares else torch.bfloat16, (shares, 1, H) if shares else (parts, H))
     _check(weight, "weight", torch.bfloat16, (H,))
@@ -191,6 +193,68 @@ def gate_normed(a: torch.Tensor, hidden: torch.Tensor, weight: torch.Tensor, nex
         return True
 
     return NormedRow(hidden, torch.empty((1, H), dtype=torch.bfloat16, device=dev) if out is None else out, fused, alone)
+
+
+def _embedded_row(tokens, table, weight, *others) -> bool:
+    return (tokens.shape[0] == 1 and table.dtype == torch.bfloat16 and table.is_cuda and table.dim() == 2 and table.is_contiguous()
+            and weight.dtype == torch.bfloat16 and bool(_ffi.query("skyrl_normed_product_fits", table.shape[1], 1, 1))
+            and all(t is None or t.data_ptr() % 16 == 0 for t in (table, weight, *others)))
+
+
+def _embedding_of(q, tokens, table, scale: float = 1.0) -> None:
+    q.tokens, q.table, q.scale = tokens.data_ptr(), table.data_ptr(), scale
+
+
+def normed_embedding(tokens: torch.Tensor, table: torch.Tensor, scale: float, weight: torch.Tensor, eps: float, kind: str = "layer",
+                     step: Optional[torch.Tensor] = None, base: float = 0.0) -> Optional[NormedRow]:
+    """The norm of embed (and `step`) of one token as a NormedRow; None for sizes and types that take their own launches."""
+    if not _embedded_row(tokens, table, weight, step):
+        return None
+    dev, H = _require_gpu(tokens, table, weight, step), table.shape[1]
+    _check(tokens, "tokens", torch.int64, (1,))
+    _check(weight, "weight", torch.bfloat16, (H,))
+    _check(step, "step", torch.bfloat16, (H,))
+
+    def alone(to):
+        hidden = embed(tokens, table, scale)
+        add_norm(None, hidden, weight, eps, kind, step, to, base)
+        return hidden
+
+    def fused(q, gated, splits):
+        if splits:
+            return False
+        _embedding_of(q, tokens, table, float(scale))
+        _ffi.call("skyrl_add_norm_product", ctypes.byref(q), None, 0, _ptr(step), _ptr(weight), float(base), float(eps), NORMS[kind],
+                  _stream(dev))
+        return True
+
+    return NormedRow(None, torch.empty((1, H), dtype=torch.bfloat16, device=dev), fused, alone)
+
+
+def gate_normed_embedding(tokens: torch.Tensor, table: torch.Tensor, weight: torch.Tensor, next_weight: torch.Tensor, eps: float,
+                          groups: int = 1, mult: float = 1.0) -> Optional[NormedRow]:
+    """gate_norm_add of one token's row of table, `fresh` and without a gate, as a NormedRow; None as normed_embedding."""
+    if not _embedded_row(tokens, table, weight, next_weight) or groups < 1 or table.shape[1] % groups or table.shape[1] // groups % 8:
+        return None
+    dev, H = _require_gpu(tokens, table, weight, next_weight), table.shape[1]
+    _check(tokens, "tokens", torch.int64, (1,))
+    _check(weight, "weight", torch.bfloat16, (H,))
+    _check(next_weight, "next_weight", torch.bfloat16, (H,))
+
+    def alone(to):
+        hidden = torch.empty((1, H), dtype=torch.float32, device=dev)
+        gate_norm_add(table, hidden, weight, next_weight, eps, groups, mult, rows=tokens, fresh=True, out=to)
+        return hidden
+
+    def fused(q, gated, splits):
+        if gated or splits:
+            return False
+        _embedding_of(q, tokens, table)
+        _ffi.call("skyrl_gate_norm_product", ctypes.byref(q), None, 0, 1, None, 0, 0, None, _ptr(weight), groups, float(eps), float(mult),
+                  _ptr(next_weight), _stream(dev))
+        return True
+
+    return NormedRow(None, torch.empty((1, H), dtype=torch.bfloat16, device=dev), fused, alone)
 
 
 # ---------------------------------------------------------------- products of few rows

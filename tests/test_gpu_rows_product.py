@@ -307,3 +307,31 @@ def test_what_follows_a_product(dev, n, N, K):
         assert torch.equal(t[:, :first], plain[:, :first]) and torch.equal(t[:, last:], plain[:, last:])
         if last > first:
             assert torch.equal(t[:, first:last], lk.tanh(plain[:, first:last]))
+
+
+@pytest.mark.parametrize("H,N", [(8, 24), (264, 8200), (2048, 96), (4096, 40)])
+def test_embedding_ahead_of_a_product(dev, H, N):
+    g = torch.Generator(device=dev).manual_seed(H)
+    rand = lambda *s: torch.randn(*s, device=dev, generator=g).bfloat16()  # noqa: E731
+    table, w, weight, nxt, step = rand(50, H), rand(N, H), rand(H), rand(H), rand(H)
+    for token, st in ((0, None), (49, step)):
+        tok = torch.tensor([token], device=dev)
+        h = lk.embed(tok, table, 1.75)
+        want = lk.add_norm(None, h, weight, 1e-4, "layer", st)
+        row = lk.normed_embedding(tok, table, 1.75, weight, 1e-4, "layer", st)
+        y = lk.linear(row, w)
+        assert row.fused is None and torch.equal(lk.residual(row, None), h) and torch.equal(lk.rows_of(row), want)
+        assert _close(y, want, w)
+        alone = lk.normed_embedding(tok, table, 1.75, weight, 1e-4, "layer", st)
+        assert torch.equal(lk.rows_of(alone), want) and torch.equal(lk.residual(alone, None), h)
+        groups = 1 if H == 8 else 4 if H > 300 else 3
+        h = torch.empty(1, H, device=dev)
+        want = lk.gate_norm_add(table, h, weight, nxt, 1e-6, groups, 0.5, rows=tok, fresh=True)
+        for fuse in (True, False):
+            row = lk.gate_normed_embedding(tok, table, weight, nxt, 1e-6, groups, 0.5)
+            if fuse:
+                assert _close(lk.linear(row, w), want, w, want.double() @ w.double().t()) or H > 2048
+            got, hidden = lk.rows_of(row), lk.residual(row, None)
+            assert float((hidden - h).norm()) <= 1e-6 * float(h.norm())
+            assert float((got - want).float().norm()) <= 2.0 ** -9 * float(want.float().norm())
+    assert lk.normed_embedding(torch.tensor([1, 2], device=dev), table, 1.0, weight, 1e-4) is None

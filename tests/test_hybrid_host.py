@@ -525,6 +525,13 @@ def test_experts_tiles_follow_the_mean_load():
     assert [mixers.lk.moe_tile(sh, n) for n in (1, 64, 95, 96, 383, 384, 895, 896, 8192)] == [16, 16, 16, 64, 64, 128, 128, 256, 256]
 
 
+@pytest.mark.parametrize("width,ff,sizes", [(2048, 768, {479: 64, 480: 128, 895: 128, 896: 256}), (1536, 576, {479: 64, 1599: 128, 1600: 256}),
+                                            (4096, 1536, {383: 64, 384: 128, 896: 256}), (512, 192, {384: 128, 896: 256})])
+def test_experts_tiles_follow_the_faster_form(width, ff, sizes):
+    sh = mixers.lk.moe_shape(width, ff, 64, 8, 8, 4)
+    assert {n: mixers.lk.moe_tile(sh, n) for n in sizes} == sizes
+
+
 def test_oracle_grouped_norm_and_routing():
     x, w = torch.randn(3, 12, dtype=torch.float64), torch.randn(12, dtype=torch.float64)
     got = ref.grouped_rms_norm(x, w, 3, 1e-3)
