@@ -157,7 +157,7 @@ __global__ __launch_bounds__(NWV * kWave) void moe_route_kernel(Router ro, const
                                                                 int width, const uint16_t* __restrict__ w,
                                                                 const float* __restrict__ correction,
                                                                 int32_t* __restrict__ idx, float* __restrict__ weight) {
-    using St = Stream<NE, 1, NWV, S>;
+    using St = Stream<NE, 1, NWV, S, false, false>;  // every workgroup reads the router
     constexpr int E16 = NE * 16, LZ = St::LR, EP = (E16 + kWave - 1) / kWave;
     __shared__ __attribute__((aligned(16))) uint16_t smem[St::kLds];
     float(*s_z)[16 * LZ] = reinterpret_cast<float(*)[16 * LZ]>(smem);  // the shares' sums, where the pieces were

@@ -23,10 +23,10 @@
 namespace skyrl {
 namespace {
 
-template <int MODE, int NT, int MT, int WK, int S>
+template <int MODE, int NT, int MT, int WK, int S, bool ONCE>
 __global__ __launch_bounds__(WK* kWave) void rows_product_kernel(RowsProduct p) {
     __shared__ __attribute__((aligned(16))) uint16_t smem[Stream<NT, MT, WK, S>::kLds];
-    rows_block<MODE, NT, MT, WK, S>(p, smem, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.y);
+    rows_block<MODE, NT, MT, WK, S, ONCE>(p, smem, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.y);
 }
 
 constexpr int kWide = 8192;       // output columns from which wider tiles still fill the chip and read x less often
@@ -67,11 +67,11 @@ int splits_for(int n, int K, int N) {
     return s < 1 ? 1 : s > 8 ? 8 : s;
 }
 
-template <int MODE, int NT, int MT, int WK, int S>
+template <int MODE, int NT, int MT, int WK, int S, bool ONCE = true>
 void launch_rows(RowsProduct p, int splits, hipStream_t s, int batch = 1) {
     constexpr int OC = MODE == kGated ? 8 * NT : 16 * NT;
     p.row_blocks = (p.n + 16 * MT - 1) / (16 * MT);
-    hipLaunchKernelGGL((rows_product_kernel<MODE, NT, MT, WK, S>), dim3((p.N + OC - 1) / OC, splits, p.row_blocks * batch),
+    hipLaunchKernelGGL((rows_product_kernel<MODE, NT, MT, WK, S, ONCE>), dim3((p.N + OC - 1) / OC, splits, p.row_blocks * batch),
                        dim3(WK * kWave), 0, s, p);
 }
 
@@ -174,17 +174,18 @@ int rows_batch(const void* x, int64_t ldx, int64_t x_batch, int32_t n, int32_t K
     // A head's matrix is small: all its pieces are under way at once. Shallow ones (the queries' up-projection) take two
     // waves a workgroup and 32 columns, deep ones (the outputs') four waves and 16 columns. In order: one wave, which has the
     // whole depth (16 heads, 256 rows: 12.4 and 15.0 us, in shares 12.2 and 13.5, the library 22.8 and 35.6 with its copy).
+    // Past 64 rows the blocks of 64 share a head's matrix: the forms of more than 32 rows leave it in the caches.
     if (in_order) {
-        if (K <= 256) launch_rows<kRound, 2, 4, 1, 2>(p, 1, s, batch);
-        else launch_rows<kRound, 1, 4, 1, 3>(p, 1, s, batch);
+        if (K <= 256) launch_rows<kRound, 2, 4, 1, 2, false>(p, 1, s, batch);
+        else launch_rows<kRound, 1, 4, 1, 3, false>(p, 1, s, batch);
     } else if (K <= 256) {
         if (n <= 16) launch_rows<kRound, 2, 1, 2, 2>(p, 1, s, batch);
         else if (n <= 32) launch_rows<kRound, 2, 2, 2, 2>(p, 1, s, batch);
-        else launch_rows<kRound, 2, 4, 2, 1>(p, 1, s, batch);
+        else launch_rows<kRound, 2, 4, 2, 1, false>(p, 1, s, batch);
     } else {
         if (n <= 16) launch_rows<kRound, 1, 1, 4, 2>(p, 1, s, batch);
         else if (n <= 32) launch_rows<kRound, 1, 2, 4, 2>(p, 1, s, batch);
-        else launch_rows<kRound, 1, 4, 4, 2>(p, 1, s, batch);
+        else launch_rows<kRound, 1, 4, 4, 2, false>(p, 1, s, batch);
     }
     return check_launch("rows_product_kernel");
 }

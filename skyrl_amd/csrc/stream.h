@@ -13,9 +13,13 @@ typedef __attribute__((address_space(1))) void gbl_void;
 
 __device__ const uint4 kZero16 = {0u, 0u, 0u, 0u};
 
-// NT 16-row weight tiles, MT 16-row tiles of x, WK waves. HELD: the rows of x lie in LDS whole and are not streamed.
-template <int NT, int MT, int WK, int S, bool HELD = false>
+// NT 16-row weight tiles, MT 16-row tiles of x, WK waves. HELD: the rows of x lie in LDS whole and are not streamed. ONCE: no
+// other workgroup reads these weight rows, so they go past the caches (non-temporal): a step's weights, several times the
+// last-level cache, put out what is read again and wait for its lines to be put out (32768 x 2048: 1 row 24.8 -> 21.9 us, 64 rows
+// 31.4 -> 27.4; in a step's place, eight of 64 experts of 768 x 2048 for 64 rows 74.8 + 39.3 -> 59.7 + 34.3).
+template <int NT, int MT, int WK, int S, bool HELD = false, bool ONCE = true>
 struct Stream {
+    static constexpr int kPolicy = ONCE ? 2 : 0;  // the load's cache policy bits: 2 is nt
     static constexpr int BN = 16 * NT, BM = 16 * MT, WP = 2 * NT, XP = HELD ? 0 : 2 * MT, L = WP + XP;  // 1 KB pieces: 8 rows, 64 deep
     static constexpr int kStage = (BN + (HELD ? 0 : BM)) * 64;  // elements
     static constexpr int LR = BN + 4;              // a row of a share's sums
@@ -59,7 +63,7 @@ struct Stream {
 #pragma unroll
             for (int i = 0; i < WP; ++i) {
                 const void* src = in ? (const void*)(ws[i] + t * 64) : (const void*)&kZero16;
-                __builtin_amdgcn_global_load_lds((gbl_void*)src, (lds_void*)(dst + i * 512), 16, 0, 0);
+                __builtin_amdgcn_global_load_lds((gbl_void*)src, (lds_void*)(dst + i * 512), 16, 0, kPolicy);
             }
 #pragma unroll
             for (int i = 0; i < XP; ++i) {
