@@ -441,7 +441,9 @@ __global__ __launch_bounds__(WK* kWave) void moe_one_kernel(Router ro, const flo
 
 // A workgroup: one tile of TM rows and TN weight rows (GATED: half of each matrix, the same columns), WM x WN waves. S
 // stages of 64-deep pieces. Tiles of one expert share its weights and a tile's columns its rows: with several tiles per
-// expert (TM > 16) an XCD takes a run of tiles, a tile's columns together. The output leaves through LDS, whole rows.
+// expert (TM > 16) an XCD takes a run of tiles, a tile's columns together. The output leaves through LDS, whole rows. The weights
+// go past the caches (non-temporal): an expert mostly has one tile, and a step's experts are several times the last-level cache
+// (768 x 2048, 256 tokens, a step's place: gate_up 92 -> 74 us, down 44.5 -> 43).
 template <int TM, int TN, int WM, int WN, int S, bool GATED>
 __global__ __launch_bounds__(WM* WN* kWave) void moe_gemm_kernel(Product p, const uint16_t* __restrict__ x,
                                                                  const uint16_t* __restrict__ w,
@@ -515,7 +517,7 @@ __global__ __launch_bounds__(WM* WN* kWave) void moe_gemm_kernel(Product p, cons
         for (int i = 0; i < WL; ++i) {
             const int k = k0 + wk[i];
             const void* src = k < p.K ? (const void*)(ws[i] + k) : (const void*)&kZero16;
-            __builtin_amdgcn_global_load_lds((gbl_void*)src, (lds_void*)(dst + TM * BK + (wave * WL + i) * 512), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((gbl_void*)src, (lds_void*)(dst + TM * BK + (wave * WL + i) * 512), 16, 0, 2);  // nt
         }
     };
     const int wm = wave / WN, wn = wave % WN;
