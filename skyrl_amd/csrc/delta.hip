@@ -51,7 +51,9 @@ __device__ __forceinline__ float conv_silu(const T* __restrict__ proj, int64_t s
 // One workgroup per (sequence, head), the state in registers. A decode step is bound by the state, read and written once. The
 // first token is a copy of the loop's body of its own (AHEAD: at most kWin taps, a channel per thread), so that nothing but
 // the products waits for the state: 32 heads of 128 x 128, one token each: 64 rows 62.6 us (4.3 TB/s) against 79.8, 1 row 9.0
-// against 11.7.
+// against 11.7. The state goes past the caches both ways (non-temporal): left there it is put out before the next step by the
+// weights, and what is written is in their way (64 rows 59.4 -> 57.3 us; with the latent pages, which go the same way, four small
+// products of the step 27.5 -> 18.4 us).
 // A value as it is stored, in a register of its own: what is loaded ahead is converted, and waited for, where it is used.
 template <typename T>
 using Raw = std::conditional_t<sizeof(T) == 2, uint32_t, T>;
@@ -116,7 +118,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void de
     float S[RPT][4];
 #pragma unroll
     for (int i = 0; i < RPT; ++i) {
-        const float4 v = ld4(st_ + (int64_t)min(rg + i * RG, D - 1) * VP + 4 * cg);
+        const float4 v = ld4_once(st_ + (int64_t)min(rg + i * RG, D - 1) * VP + 4 * cg);
         S[i][0] = v.x; S[i][1] = v.y; S[i][2] = v.z; S[i][3] = v.w;
     }
     const float neg_rate = -expf(rate);
@@ -221,7 +223,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void de
 #pragma unroll
     for (int i = 0; i < RPT; ++i) {
         const int r = rg + i * RG;
-        if (act && r < D) st4(st_ + (int64_t)r * VP + 4 * cg, make_float4(S[i][0], S[i][1], S[i][2], S[i][3]));
+        if (act && r < D) st4_once(st_ + (int64_t)r * VP + 4 * cg, make_float4(S[i][0], S[i][1], S[i][2], S[i][3]));
     }
     if (save_conv) {  // one token: its slot is not among those the convolutions read
         const T* p = proj + (int64_t)t0 * stride;

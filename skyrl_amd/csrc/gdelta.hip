@@ -5,6 +5,7 @@
 // Token form (gdelta_scan): one workgroup per (sequence, head), the state in registers over the sequence's tokens. Both
 // products with the state read the old one, z = S^T u and y = S^T (w r), in one sweep:
 //   o = y - (r . a u) z + (r . k) v.
+// The state goes past the caches both ways (non-temporal), as delta_scan's; the launch itself takes what it took (256 rows 52 to 54 us).
 //
 // Prompt form (chunk, chain, out): chunks of 64 tokens. With G_t the summed log decays up to token t, per channel, and
 //   al_t = e^{G_(t-1)} u_t,  be_t = e^{-G_t} a_t u_t,  ka_t = e^{-G_t} k_t,  rh_t = e^{G_t} r_t
@@ -91,7 +92,7 @@ __global__ __launch_bounds__(NT) void gdelta_scan_kernel(Dims d, In<T> in, const
     for (int i = 0; i < RPT; ++i) {
         const int r = rg + i * RG;
         float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (act && r < D && !fresh) v = ld4(st_ + (int64_t)r * VP + 4 * cg);
+        if (act && r < D && !fresh) v = ld4_once(st_ + (int64_t)r * VP + 4 * cg);
         S[i][0] = v.x; S[i][1] = v.y; S[i][2] = v.z; S[i][3] = v.w;
     }
     const bool ch = tid < D;
@@ -201,7 +202,7 @@ __global__ __launch_bounds__(NT) void gdelta_scan_kernel(Dims d, In<T> in, const
 #pragma unroll
     for (int i = 0; i < RPT; ++i) {
         const int r = rg + i * RG;
-        if (act && r < D) st4(st_ + (int64_t)r * VP + 4 * cg, make_float4(S[i][0], S[i][1], S[i][2], S[i][3]));
+        if (act && r < D) st4_once(st_ + (int64_t)r * VP + 4 * cg, make_float4(S[i][0], S[i][1], S[i][2], S[i][3]));
     }
 }
 

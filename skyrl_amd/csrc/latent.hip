@@ -284,6 +284,8 @@ __global__ __launch_bounds__(kNT * HG) __attribute__((amdgpu_waves_per_eu(1, 2))
     const int np = min(sp.per, sp.np - part * sp.per);
     const int32_t* bt = tables + (int64_t)bt_row[t] * bt_stride + first;
     // Pages come in windows of 64, whose block ids a wave holds by lane (no table load ahead of a page's).
+    // Pages go past the caches (non-temporal): up to 32 heads a workgroup has them alone, and the step's weights put them out
+    // before the next step (in a step's place: 64 rows 29.5 -> 24.5 us, 256 rows 67 -> 58.5).
     // Loads are unconditional, the last page again past the end: a branch around them would turn every
     // wait into one for all loads in flight.
     const int rc = EXACT ? NK * 4 : nk * 4;  // pieces per row
@@ -303,13 +305,13 @@ __global__ __launch_bounds__(kNT * HG) __attribute__((amdgpu_waves_per_eu(1, 2))
     auto load_page = [&](int j) {
         const uint16_t* p = cache + (int64_t)__builtin_amdgcn_readlane(tbl, min(j, npw - 1)) * kBS * row;
 #pragma unroll
-        for (int k = 0; k < NL; ++k) st_[k] = *reinterpret_cast<const s16x8*>(p + piece(k) * 8);
+        for (int k = 0; k < NL; ++k) st_[k] = __builtin_nontemporal_load(reinterpret_cast<const s16x8*>(p + piece(k) * 8));
     };
     // The query rows of this head group, [latent | rotated | 0], through LDS into MFMA operands. Loads return in order: those of
     // whole 16-byte pieces go ahead of the pages', all at once, and land while the block table is read (16 heads, 512 + 64,
     // context 1024, us with the merge, against a loop of loads behind the first pages': 1 row 12.3 against 18.0, 64 rows 23.7
     // against 28.8, 256 rows 60.5 against 67.1, over and over on one cache, part of which stays on chip; in engine passes 64 rows
-    // take 30 to 35, 256 rows 68, the cache's 302 MB at 4.4 TB/s).
+    // take 24.5, 256 rows 58.5, the cache's 302 MB at 5.2 TB/s).
     constexpr int QP = HG * 16 * NK * 4, QL = (QP + NT - 1) / NT;
     const bool pieces = rank % 8 == 0 && rot % 8 == 0 && q_stride % 8 == 0 && q_head % 8 == 0 &&
                         (reinterpret_cast<uintptr_t>(q_rot) & 15) == 0;
