@@ -647,8 +647,9 @@ int launch_product(const Product& p, const void* x, const void* w, void* out, in
         // x 2048, both products, 256 tokens: 139.6 us against 143.5, streamed in shares 137; 1536 x 4096: 469 against 459).
         const bool once = ntiles <= 2 * experts;
         if (p.tm == 256 && wide_fits(p.K, p.N, GATED)) {
-            return launch_wide<GATED ? kGateUp : kDown>(Wide{x_, w_, o_, p.K, p.N, p.K, p.K, ntiles, p.order, p.tile_expert,
-                                                             p.row_div, p.weight, 0, Gate{}}, s);
+            constexpr int kind = GATED ? kGateUp : kDown;
+            const Wide wide{x_, w_, o_, p.K, p.N, p.K, p.K, ntiles, p.order, p.tile_expert, p.row_div, p.weight, 0, Gate{}};
+            return once ? launch_wide<kind, SKYRL_ACT_SILU, true>(wide, s) : launch_wide<kind>(wide, s);
         }
         if (p.tm == 256) LAUNCH_GEMM(256, 256, 2, 4, 2);
         else if (p.tm == 128) LAUNCH_GEMM(128, 128, 2, 2, 2);

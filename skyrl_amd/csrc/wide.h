@@ -73,7 +73,9 @@ __device__ __forceinline__ void product(f32x4& a, const s16x8& w, const s16x8& x
 // being at 1.75 to 1.9 GHz then. Measured, 64 experts of 768 x 2048, 8 per token, gate_up / down, us (before: eight waves, a
 // workgroup per tile and columns, two stages): 2048 tokens 153 / 85 (174 / 94), 5637 tokens 273 / 170 (305 / 189), 8192 tokens
 // 380 / 255 (434 / 275).
-template <int KIND, int ACT>
+// ONCE: an expert's weights go past the caches (non-temporal), for about one tile an expert: a step of 1563 tokens (195
+// pairs each) 2040 -> 1990 us. With several tiles, which read them from there, that is the slower way (700 pairs: 4498 -> 4628).
+template <int KIND, int ACT, bool ONCE>
 __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
     constexpr bool GATED = KIND != kDown, ROUTED = KIND != kGated, GATHER = KIND != kDown;
     const int ncols = p.N / (GATED ? 128 : 256);
@@ -133,7 +135,8 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
         const int64_t k0 = min(t, nk - 1) * BK;
         const int64_t row = (i % L) / 2 * 64 + (GATED && i >= L + L / 2 ? p.N - OC : 0);
         const uint16_t* src = i >= L ? ws[i % 2] + (k0 + row * p.ldw) : GATHER ? xs[i % L] + k0 : xs[i % 2] + (k0 + row * p.ldx);
-        __builtin_amdgcn_global_load_lds((gbl_void*)src, (lds_void*)dst, 16, 0, 0);
+        if (ONCE && i >= L) __builtin_amdgcn_global_load_lds((gbl_void*)src, (lds_void*)dst, 16, 0, 2);
+        else __builtin_amdgcn_global_load_lds((gbl_void*)src, (lds_void*)dst, 16, 0, 0);
     };
     int n0, q = 0;
     const double per_row = KIND == kGateUp ? 1.0 / p.row_div : 0.0;
@@ -331,12 +334,12 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
 // Items one each for up to three rounds of workgroups, which then go to the CUs as these get free; with more, a workgroup per
 // CU (gate_up as above, 2048 tokens: 161 us against 171; 8192: 395 against 380).
 inline bool wide_fits(int K, int N, bool gated) { return K > 0 && K % 64 == 0 && N % (gated ? 128 : 256) == 0; }
-template <int KIND, int ACT = SKYRL_ACT_SILU>
+template <int KIND, int ACT = SKYRL_ACT_SILU, bool ONCE = false>
 int launch_wide(const Wide& p, hipStream_t s) {
     const int64_t items = (int64_t)(p.N / (KIND == kDown ? 256 : 128)) * p.ntiles;
     SKYRL_REQUIRE(items < (1ll << 31) && p.ntiles < (1 << 23), "wide products: too many rows in one call");
     const unsigned grid = (unsigned)(items > 3 * kCUs ? kCUs : (items + 7) / 8 * 8);
-    hipLaunchKernelGGL((wide_kernel<KIND, ACT>), dim3(grid), dim3(256), 0, s, p);
+    hipLaunchKernelGGL((wide_kernel<KIND, ACT, ONCE>), dim3(grid), dim3(256), 0, s, p);
     return check_launch("wide_kernel");
 }
 

@@ -494,6 +494,18 @@ def test_tile_sizes_agree_bit_for_bit(width, ff, experts, top, n):
     assert all(torch.equal(outs[0], o) for o in outs[1:])
 
 
+@pytest.mark.parametrize("n", (1, 639, 640))
+def test_wide_tiles_agree_on_both_sides_of_a_tile_an_expert(n):
+    """Up to 639 tokens, 2 of 4 experts each, the wide form's weights go past the caches: the same rows as from tiles of 64."""
+    g = torch.Generator(device=DEV).manual_seed(n)
+    sh = lk.moe_shape(256, 256, 4, 2)
+    mk = lambda *s, scale=1.0: (torch.randn(s, generator=g, device=DEV) * scale).to(BF16)  # noqa: E731
+    x, wgu, wd = mk(n, 256), mk(4, 2, 256, 256, scale=0.1), mk(4, 256, 256, scale=0.1)
+    idx, weight = lk.moe_route(sh, x, mk(4, 256), torch.zeros(4, device=DEV))
+    wide, staged = (lk.moe_experts(sh, x, idx, weight, wgu, wd, tm=tm) for tm in (256, 64))
+    assert torch.equal(wide, staged)
+
+
 @pytest.mark.parametrize("experts,top,n,tm", [(64, 8, 4, 16), (64, 8, 95, 16), (64, 8, 128, 32), (16, 4, 60, 32)])
 def test_streamed_tiles_repeat_bit_for_bit(experts, top, n, tm):
     """The tiles that decode steps take, products of a real layer's size over and over: an operand that is overwritten while it
