@@ -100,10 +100,12 @@ __device__ __forceinline__ void write_row(const Write<T>& w, int t) {
     };
     const float* cs = w.cos_sin + w.positions[t] * rot;
     auto pair = [&](const T* x, int i) { return Turned{x[pr.first(i)], x[pr.second(i)], cs[i], cs[h2 + i]}; };
+    // Which of the two products is rounded is said here: left to the compiler it changes with the code around it, and one rotated
+    // bf16 value in some 200,000 with it.
     auto turn = [&](const Turned& e, T* to, int i) {
         const float u = ld(&e.u), v = ld(&e.v);
-        st(to + pr.first(i), u * e.c - v * e.s);
-        st(to + pr.second(i), v * e.c + u * e.s);
+        st(to + pr.first(i), fmaf(u, e.c, -(v * e.s)));
+        st(to + pr.second(i), sizeof(T) == 2 ? fmaf(u, e.s, v * e.c) : fmaf(v, e.c, u * e.s));
     };
     auto head = [&](int e) { return p + (int64_t)(e / h2) * qd + w.dim; };
     if (w.q_rank > 0) load(q, p, w.q_norm, w.q_rank);

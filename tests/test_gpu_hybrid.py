@@ -210,6 +210,30 @@ def test_latent_write(heads, dim, rot, rank, dtype):
     assert bool((got[~touched.to(DEV)] == 7.0).all()) and bool((got[:, rank + rot:] == 7.0).all())
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("halves", (False, True))
+def test_rotation_rounds_the_same_product(dtype, halves):
+    """Rotated parts, queries' and keys', bit for bit: one product rounded, the other and the sum in one rounding. A sum with the
+    products' parts exchanged differs in some of so many bf16 values."""
+    g = torch.Generator(device=DEV).manual_seed(3)
+    T, heads, dim, rot, rank = 1500, 16, 8, 64, 16
+    proj = torch.randn(T, heads * (dim + rot) + rank + rot, device=DEV, generator=g).to(dtype)
+    before, pos = proj.double(), torch.randint(0, 4000, (T,), device=DEV, generator=g)
+    table = mixers.rotary_table({"base": 10000.0, "dims": rot}, 4096).to(DEV)
+    cache = torch.zeros(T // BS + 1, BS, lk.latent_row(rank, rot), device=DEV, dtype=dtype)
+    lk.latent_write(proj, rot, pos, torch.arange(T, device=DEV), table, cache, 1e-4, heads=heads, dim=dim, rank=rank,
+                    norm_weight=torch.ones(rank, device=DEV, dtype=dtype), halves=halves)
+    c, s = table.double()[pos][:, None].chunk(2, -1)
+    pairs = (slice(0, rot // 2), slice(rot // 2, rot)) if halves else (slice(0, rot, 2), slice(1, rot, 2))
+    w = heads * (dim + rot)
+    for got, was in ((proj[:, :w].view(T, heads, -1)[..., dim:], before[:, :w].view(T, heads, -1)[..., dim:]),
+                     (cache.view(-1, cache.shape[2])[:T, None, rank:rank + rot], before[:, None, w + rank:])):
+        u, v = was[..., pairs[0]], was[..., pairs[1]]
+        second = u * s + (v * c).float() if dtype == torch.bfloat16 else v * c + (u * s).float()  # f64: exact up to its one rounding
+        assert torch.equal(got[..., pairs[0]], (u * c - (v * s).float()).float().to(dtype))
+        assert torch.equal(got[..., pairs[1]], second.float().to(dtype))
+
+
 PREFILL = [  # heads, dim, rot, vdim, rank, window, [(start, tokens)]
     (3, 20, 12, 28, 40, 37, [(0, 70), (5, 33)]),
     (6, 40, 24, 72, 48, 80, [(0, 130), (300, 64), (79, 40)]),
