@@ -47,7 +47,7 @@ __device__ __forceinline__ float total(float v, uint32_t red) {
 template <int MODE, int NT, int S, int LONG, int ROWS, int kRed, class Pre>
 __device__ __forceinline__ void formed_product(const RowsProduct& p, const Pre& pre, uint16_t* smem, int batch, bool first) {
     constexpr int WK = kFormers / kWave, kPitch = LONG * 2 + (ROWS > 1 ? 16 : 0);  // bytes
-    using St = Stream<NT, 1, WK, S, true>;
+    using St = Stream<NT, 1, WK, S, true, true, MODE == kParts>;
     using Row = typename Pre::template RowOf<LONG>;
     constexpr int OC = out_cols<MODE, NT>();
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);

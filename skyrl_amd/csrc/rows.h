@@ -79,9 +79,9 @@ __device__ __forceinline__ void put_rows(const uint16_t* smem, const RowsProduct
 
 // NT 16-row weight tiles (kGated: half of each matrix) and MT 16-row tiles of x per workgroup, the depth in `splits` * WK shares;
 // blocks of MT tiles and products of a batch along z.
-template <int MODE, int NT, int MT, int WK, int S, bool ONCE = true>
+template <int MODE, int NT, int MT, int WK, int S, bool ONCE = true, bool EXACT = false>
 __device__ __forceinline__ void rows_block(const RowsProduct& p, uint16_t* smem, int bx, int by, int bz, int splits) {
-    using St = Stream<NT, MT, WK, S, false, ONCE>;
+    using St = Stream<NT, MT, WK, S, false, ONCE, EXACT>;
     constexpr int BM = St::BM, OC = out_cols<MODE, NT>();
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n0 = bx * OC, batch = bz / p.row_blocks, m0 = bz % p.row_blocks * BM;

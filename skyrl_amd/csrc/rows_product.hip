@@ -23,10 +23,10 @@
 namespace skyrl {
 namespace {
 
-template <int MODE, int NT, int MT, int WK, int S, bool ONCE>
+template <int MODE, int NT, int MT, int WK, int S, bool ONCE, bool EXACT>
 __global__ __launch_bounds__(WK* kWave) void rows_product_kernel(RowsProduct p) {
     __shared__ __attribute__((aligned(16))) uint16_t smem[Stream<NT, MT, WK, S>::kLds];
-    rows_block<MODE, NT, MT, WK, S, ONCE>(p, smem, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.y);
+    rows_block<MODE, NT, MT, WK, S, ONCE, EXACT>(p, smem, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.y);
 }
 
 constexpr int kWide = 8192;       // output columns from which wider tiles still fill the chip and read x less often
@@ -67,11 +67,11 @@ int splits_for(int n, int K, int N) {
     return s < 1 ? 1 : s > 8 ? 8 : s;
 }
 
-template <int MODE, int NT, int MT, int WK, int S, bool ONCE = true>
+template <int MODE, int NT, int MT, int WK, int S, bool ONCE = true, bool EXACT = false>
 void launch_rows(RowsProduct p, int splits, hipStream_t s, int batch = 1) {
     constexpr int OC = MODE == kGated ? 8 * NT : 16 * NT;
     p.row_blocks = (p.n + 16 * MT - 1) / (16 * MT);
-    hipLaunchKernelGGL((rows_product_kernel<MODE, NT, MT, WK, S, ONCE>), dim3((p.N + OC - 1) / OC, splits, p.row_blocks * batch),
+    hipLaunchKernelGGL((rows_product_kernel<MODE, NT, MT, WK, S, ONCE, EXACT>), dim3((p.N + OC - 1) / OC, splits, p.row_blocks * batch),
                        dim3(WK * kWave), 0, s, p);
 }
 
@@ -126,7 +126,8 @@ int rows_product(const void* x, int64_t ldx, int32_t n, int32_t K, const void* w
         else if (n <= 32) launch_rows<kGated, 4, 2, 4, 2>(p, 1, s);
         else launch_rows<kGated, 4, 4, 4, 2>(p, 1, s);
     } else if (splits) {
-        if (n <= 16) launch_rows<kParts, 1, 1, 4, 4>(p, splits, s);
+        if (n == 1) launch_rows<kParts, 1, 1, 4, 4, true, true>(p, splits, s);
+        else if (n <= 16) launch_rows<kParts, 1, 1, 4, 4>(p, splits, s);
         else if (n <= 32) launch_rows<kParts, 2, 2, 4, 2>(p, splits, s);
         else if (n <= 64) launch_rows<kParts, 2, 4, 4, 2>(p, splits, s);
         else launch_rows<kParts, 2, 8, 4, 1>(p, splits, s);

@@ -17,7 +17,10 @@ __device__ const uint4 kZero16 = {0u, 0u, 0u, 0u};
 // other workgroup reads these weight rows, so they go past the caches (non-temporal): a step's weights, several times the
 // last-level cache, put out what is read again and wait for its lines to be put out (32768 x 2048: 1 row 24.8 -> 21.9 us, 64 rows
 // 31.4 -> 27.4; in a step's place, eight of 64 experts of 768 x 2048 for 64 rows 74.8 + 39.3 -> 59.7 + 34.3).
-template <int NT, int MT, int WK, int S, bool HELD = false, bool ONCE = true>
+// EXACT: the pieces' sums are added in 64 bits, for one row whose results leave in f32. One chain of f32 sums a wave rounds more than
+// the lanes of a wave per weight row did: error / result against 64 bits 0.95e-7, 1.90e-7, 1.65e-7 at 2048, 4096, 6144 deep (2048,
+// 4096, 2048 columns), where those had 0.75e-7, 0.85e-7, 0.91e-7, and this has 0.64e-7 at all (3.9, 8.1, 6.8 us; 4.0, 8.2, 6.9).
+template <int NT, int MT, int WK, int S, bool HELD = false, bool ONCE = true, bool EXACT = false>
 struct Stream {
     static constexpr int kPolicy = ONCE ? 2 : 0;  // the load's cache policy bits: 2 is nt
     static constexpr int BN = 16 * NT, BM = 16 * MT, WP = 2 * NT, XP = HELD ? 0 : 2 * MT, L = WP + XP;  // 1 KB pieces: 8 rows, 64 deep
@@ -78,6 +81,7 @@ struct Stream {
 #pragma unroll
         for (int t = 0; t < S; ++t)
             if (t < nk) fetch(t);
+        double sums[EXACT ? MT : 1][EXACT ? NT : 1][4] = {};
         const uint32_t base = (uint32_t)(uintptr_t)(lds_void*)own + c * 128;
         const uint32_t held = HELD ? between() + s0 * 128 + g * 16 : 0;
         for (int t = 0; t < nk; ++t) {
@@ -120,6 +124,24 @@ struct Stream {
 #pragma unroll
                     for (int n = 0; n < NT; ++n)
                         acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[h][n], xf[h][m], acc[m][n], 0, 0, 0);
+            if constexpr (EXACT) {
+#pragma unroll
+                for (int m = 0; m < MT; ++m)
+#pragma unroll
+                    for (int n = 0; n < NT; ++n) {
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) sums[m][n][j] += (double)acc[m][n][j];
+                        acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    }
+            }
+        }
+        if constexpr (EXACT) {
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int n = 0; n < NT; ++n)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) acc[m][n][j] = (float)sums[m][n][j];
         }
     }
 

@@ -218,6 +218,24 @@ def _close(y, x, w, want=None):
     return bool(((y - want).abs() <= 2.0 ** -8 * want.abs() + 2 * off).all())
 
 
+@pytest.mark.parametrize("N,K", [(2048, 2048), (1536, 4608), (4096, 4096), (2048, 6144), (4096, 6144), (24, 2056)])
+def test_shares_of_one_row_keep_their_bits(dev, N, K):
+    """f32 shares of one row against 64 bits: within two roundings of the result (2^-23 in the 2-norm), at any depth; f32 sums along a
+    wave's share of 1024 are off by three."""
+    x, w, _ = _data(dev, 1, N, K, N + K)
+    y = lk.linear(x, w, parts=True)
+    ref = x.double() @ w.double().t()
+    assert y.dim() == 3 and float((y.double().sum(0) - ref).norm()) <= 2.0 ** -23 * float(ref.norm())
+    if K <= 4096:
+        g = torch.Generator(device=dev).manual_seed(K)
+        r = lambda *s: torch.randn(*s, device=dev, generator=g)  # noqa: E731
+        row = lk.gate_normed(r(2, 1, K), r(1, K), r(K).bfloat16(), r(K).bfloat16(), 1e-6, gate=r(1, K).bfloat16(), gate_bias=r(K))
+        y = lk.linear(row, w, parts=True)
+        ref = lk.rows_of(row).double() @ w.double().t()
+        assert row.alone is None and y.dim() == 3
+        assert float((y.double().sum(0) - ref).norm()) <= 2.0 ** -23 * float(ref.norm())
+
+
 # rows of one group of four, of a remainder of the last piece, of both register forms; wide and narrow products
 @pytest.mark.parametrize("H,N", [(8, 16), (72, 203), (264, 8200), (1536, 96), (2048, 8192), (2056, 40), (4096, 12296), (4096, 24)])
 @pytest.mark.parametrize("parts", (0, 1, 2, 4))
