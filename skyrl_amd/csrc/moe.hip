@@ -293,7 +293,11 @@ struct Product {
     int row_div;              // row of x: pair / row_div (the token), or 0: the sorted place itself
     const float* weight;      // of the pair, NULL: 1
     int out_pairs;            // rows of the output: the pair's, or the sorted place
+    bool past;                // weights that one tile reads go past the caches
 };
+// Experts' matrices from this size on do: several layers' smaller ones stay in the last-level cache (256 MB) from one step to the
+// next (64 experts, three layers in turn, both products, us, cached / past: 192 x 512, 479 tokens 17 / 20; 384 x 1024, 64 tokens 35 / 32).
+constexpr int64_t kPast = 32 << 20;
 
 // GATED: two weight matrices of N rows per expert, out = silu(gate) * up.
 template <typename T, bool GATED>
@@ -351,11 +355,12 @@ __global__ __launch_bounds__(kNT) void moe_plain_kernel(Product p, const T* __re
 // waves stream a share of the depth each (stream.h). Bound: the experts' weights, each read once. Measured, 64 experts of 768 x
 // 2048, 8 per token, gate_up / down, us (TB/s of weights) against moe_gemm_kernel's, whose stages hold two workgroups a CU, in
 // step: 4 tokens 32.1 / 16.9 (5.3 / 5.0) against 41.5 / 17.7, 64 tokens 69.8 / 38.8 (5.8 / 5.2) against 83.0 / 39.4,
-// 128 tokens in tiles of 32 72.8 / 42.3 against 86.8 / 41.3.
+// 128 tokens in tiles of 32 72.8 / 42.3 against 86.8 / 41.3. Weights go past the caches or not as moe_gemm_kernel's (both products, all
+// cached / all past: 64 tokens 95.6 (108 / 95), unevenly loaded 54 (55 / 56), 160 in tiles of 32 71 (72 / 79)).
 template <int NT, int MT, int WK, int S, bool GATED>
 __global__ __launch_bounds__(WK* kWave) void moe_stream_kernel(Product p, const uint16_t* __restrict__ x,
                                                                const uint16_t* __restrict__ w, uint16_t* __restrict__ out,
-                                                               int ncols) {
+                                                               int ncols, int ntiles) {
     using St = Stream<NT, MT, WK, S>;
     constexpr int OC = GATED ? St::BN / 2 : St::BN;
     __shared__ __attribute__((aligned(16))) uint16_t smem[St::kLds];
@@ -367,14 +372,13 @@ __global__ __launch_bounds__(WK* kWave) void moe_stream_kernel(Product p, const 
     const uint16_t* we = w + (int64_t)e * (GATED ? 2 : 1) * p.N * p.K;
     const int steps = (p.K + 63) / 64, s0 = steps * wave / WK, nk = steps * (wave + 1) / WK - s0;
     f32x4 acc[MT][NT];
-    St::run(
-        smem, p.K, s0, nk,
-        [&](int r) { return we + (int64_t)((GATED && r >= OC ? p.N : 0) + min(n0 + (GATED ? r % OC : r), p.N - 1)) * p.K; },
-        [&](int r) {  // places without a pair: row 0, not stored
-            const int pair = p.order[place0 + r];
-            return x + (pair < 0 ? 0 : p.row_div ? pair / p.row_div : place0 + r) * p.K;
-        },
-        acc);
+    auto wrow = [&](int r) { return we + (int64_t)((GATED && r >= OC ? p.N : 0) + min(n0 + (GATED ? r % OC : r), p.N - 1)) * p.K; };
+    auto xrow = [&](int r) {  // places without a pair: row 0, not stored
+        const int pair = p.order[place0 + r];
+        return x + (pair < 0 ? 0 : p.row_div ? pair / p.row_div : place0 + r) * p.K;
+    };
+    if (p.past && one_tile(p.tile_expert, tile, ntiles, e)) St::run(smem, p.K, s0, nk, wrow, xrow, acc);
+    else Stream<NT, MT, WK, S, false, false>::run(smem, p.K, s0, nk, wrow, xrow, acc);
     St::store(smem, acc);
     for (int i = tid; i < St::BM * (OC / 4); i += WK * kWave) {
         const int r = i / (OC / 4), n = i % (OC / 4) * 4, col = n0 + n, pair = p.order[place0 + r];
@@ -441,9 +445,11 @@ __global__ __launch_bounds__(WK* kWave) void moe_one_kernel(Router ro, const flo
 
 // A workgroup: one tile of TM rows and TN weight rows (GATED: half of each matrix, the same columns), WM x WN waves. S
 // stages of 64-deep pieces. Tiles of one expert share its weights and a tile's columns its rows: with several tiles per
-// expert (TM > 16) an XCD takes a run of tiles, a tile's columns together. The output leaves through LDS, whole rows. The weights
-// go past the caches (non-temporal): an expert mostly has one tile, and a step's experts are several times the last-level cache
-// (768 x 2048, 256 tokens, a step's place: gate_up 92 -> 74 us, down 44.5 -> 43).
+// expert (TM > 16) an XCD takes a run of tiles, a tile's columns together. The output leaves through LDS, whole rows. Weights of an
+// expert with one tile go past the caches (non-temporal), as a step's experts are several times the last-level cache; with several
+// tiles, which all read them, they stay: a loop for each, since a branch at every load costs 3 to 10 %. 64 experts, both products, us
+// (all cached / all past): 768 x 2048, 256 tokens 118 (128 / 118); unevenly loaded 111 (115 / 116); 576 x 1536, 1200 tokens in tiles of 128
+// 142 (141 / 164), 8000 in tiles of 64 664 (659 / 1097).
 template <int TM, int TN, int WM, int WN, int S, bool GATED>
 __global__ __launch_bounds__(WM* WN* kWave) void moe_gemm_kernel(Product p, const uint16_t* __restrict__ x,
                                                                  const uint16_t* __restrict__ w,
@@ -504,7 +510,7 @@ __global__ __launch_bounds__(WM* WN* kWave) void moe_gemm_kernel(Product p, cons
         wk[i] = (lane % CH ^ swz(r)) * 8;
         ws[i] = we + row * p.K;
     }
-    auto fetch = [&](int t) {  // piece t (the last again past the end) into stage t % S
+    auto fetch = [&](auto nt, int t) {  // piece t (the last again past the end) into stage t % S
         uint16_t* dst = smem + (t % S) * kStage;
         const int k0 = min(t, nk - 1) * BK;
 #pragma unroll
@@ -517,7 +523,9 @@ __global__ __launch_bounds__(WM* WN* kWave) void moe_gemm_kernel(Product p, cons
         for (int i = 0; i < WL; ++i) {
             const int k = k0 + wk[i];
             const void* src = k < p.K ? (const void*)(ws[i] + k) : (const void*)&kZero16;
-            __builtin_amdgcn_global_load_lds((gbl_void*)src, (lds_void*)(dst + TM * BK + (wave * WL + i) * 512), 16, 0, 2);  // nt
+            lds_void* to = (lds_void*)(dst + TM * BK + (wave * WL + i) * 512);
+            if (nt.value) __builtin_amdgcn_global_load_lds((gbl_void*)src, to, 16, 0, 2);
+            else __builtin_amdgcn_global_load_lds((gbl_void*)src, to, 16, 0, 0);
         }
     };
     const int wm = wave / WN, wn = wave % WN;
@@ -563,26 +571,30 @@ __global__ __launch_bounds__(WM* WN* kWave) void moe_gemm_kernel(Product p, cons
                 acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[ks][n], xf[ks][m], acc[m][n], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
     };
+    auto sums = [&](auto nt) {
 #pragma unroll
-    for (int t = 0; t < S; ++t) fetch(t);
-    wait_loads<(S - 1) * (XL + WL)>();
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    operands(0, 0);
-    for (int t = 0; t < nk; ++t) {
-        operands(t, 1);
-        ready(0);
-        products(0);
-        wait_loads<(S - 2) * (XL + WL)>();  // this wave's loads of piece t + 1 have landed, its reads of piece t too
-        __builtin_amdgcn_s_barrier();       // and everyone's
+        for (int t = 0; t < S; ++t) fetch(nt, t);
+        wait_loads<(S - 1) * (XL + WL)>();
+        __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        fetch(t + S);
-        operands(t + 1, 0);
-        ready(1);
-        products(1);
-    }
-    wait_loads<0>();  // nothing is under way, into LDS or into the registers of the last reads
-    hold(0);
+        operands(0, 0);
+        for (int t = 0; t < nk; ++t) {
+            operands(t, 1);
+            ready(0);
+            products(0);
+            wait_loads<(S - 2) * (XL + WL)>();  // this wave's loads of piece t + 1 have landed, its reads of piece t too
+            __builtin_amdgcn_s_barrier();       // and everyone's
+            asm volatile("" ::: "memory");
+            fetch(nt, t + S);
+            operands(t + 1, 0);
+            ready(1);
+            products(1);
+        }
+        wait_loads<0>();  // nothing is under way, into LDS or into the registers of the last reads
+        hold(0);
+    };
+    if (p.past && one_tile(p.tile_expert, tile, ntiles, e)) sums(std::true_type{});
+    else sums(std::false_type{});
     __syncthreads();
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
@@ -615,7 +627,7 @@ bool fast_form(int K, int N, int tm, int dtype, const void* x, const void* w, co
 }
 
 template <bool GATED>
-int launch_product(const Product& p, const void* x, const void* w, void* out, int ntiles, int experts, int dtype, hipStream_t s) {
+int launch_product(Product p, const void* x, const void* w, void* out, int ntiles, int experts, int dtype, hipStream_t s) {
     if (fast_form(p.K, p.N, p.tm, dtype, x, w, out)) {
         const uint16_t* x_ = reinterpret_cast<const uint16_t*>(x);
         const uint16_t* w_ = reinterpret_cast<const uint16_t*>(w);
@@ -635,7 +647,7 @@ int launch_product(const Product& p, const void* x, const void* w, void* out, in
         const int64_t ncols = (p.N + kCols - 1) / kCols;                                                              \
         SKYRL_REQUIRE(ncols * ntiles < (1ll << 31), "moe: grid too large");                                           \
         hipLaunchKernelGGL((moe_stream_kernel<NT, MT, WK, S, GATED>), dim3((unsigned)(ncols * ntiles)), dim3(WK * kWave), 0, s, \
-                           p, x_, w_, o_, (int)ncols);                                                                \
+                           p, x_, w_, o_, (int)ncols, ntiles);                                                                \
     } while (0)
         // Streamed where an expert has about one tile, so that its weights are read once: tiles of 16 below 16 pairs per
         // expert (ntiles is npairs / tm + experts), and of 32. A streamed row is the sum of its waves' shares of the depth. Tiles
@@ -646,10 +658,11 @@ int launch_product(const Product& p, const void* x, const void* w, void* out, in
         // a CU, and 64 tiles of 768 columns are three rounds of the narrow ones, one and a half of the others (64 experts of 768
         // x 2048, both products, 256 tokens: 139.6 us against 143.5, streamed in shares 137; 1536 x 4096: 469 against 459).
         const bool once = ntiles <= 2 * experts;
+        p.past = (int64_t)experts * (GATED ? 4 : 2) * p.N * p.K >= kPast;
         if (p.tm == 256 && wide_fits(p.K, p.N, GATED)) {
             constexpr int kind = GATED ? kGateUp : kDown;
             const Wide wide{x_, w_, o_, p.K, p.N, p.K, p.K, ntiles, p.order, p.tile_expert, p.row_div, p.weight, 0, Gate{}};
-            return once ? launch_wide<kind, SKYRL_ACT_SILU, true>(wide, s) : launch_wide<kind>(wide, s);
+            return once && p.past ? launch_wide<kind, SKYRL_ACT_SILU, true>(wide, s) : launch_wide<kind>(wide, s);
         }
         if (p.tm == 256) LAUNCH_GEMM(256, 256, 2, 4, 2);
         else if (p.tm == 128) LAUNCH_GEMM(128, 128, 2, 2, 2);
@@ -794,7 +807,7 @@ extern "C" int skyrl_moe_gate_up(const skyrl_moe_shape* shape, const void* x, co
     SKYRL_REQUIRE(tm > 0 && ntiles >= 0, "moe_gate_up: bad sizes");
     if (ntiles == 0) return SKYRL_OK;
     SKYRL_REQUIRE(x && w && order && tile_expert && act, "moe_gate_up: null pointer");
-    const Product p{shape->width, shape->ff, order, tile_expert, tm, shape->top, nullptr, 0};
+    const Product p{shape->width, shape->ff, order, tile_expert, tm, shape->top, nullptr, 0, false};
     return launch_product<true>(p, x, w, act, ntiles, shape->experts, dtype, as_stream(stream));
 }
 
@@ -807,6 +820,6 @@ extern "C" int skyrl_moe_down(const skyrl_moe_shape* shape, const void* act, con
     SKYRL_REQUIRE(tm > 0 && ntiles >= 0, "moe_down: bad sizes");
     if (ntiles == 0) return SKYRL_OK;
     SKYRL_REQUIRE(act && w && order && tile_expert && weight && out, "moe_down: null pointer");
-    const Product p{shape->ff, shape->width, order, tile_expert, tm, 0, weight, 1};
+    const Product p{shape->ff, shape->width, order, tile_expert, tm, 0, weight, 1, false};
     return launch_product<false>(p, act, w, out, ntiles, shape->experts, dtype, as_stream(stream));
 }

@@ -56,6 +56,11 @@ __device__ __forceinline__ void product(f32x4& a, const s16x8& w, const s16x8& x
     asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(a) : "v"(w), "v"(x));
 }
 
+// Whether an expert's tiles, which follow each other, are this one alone.
+__device__ __forceinline__ bool one_tile(const int32_t* tile_expert, int tile, int ntiles, int e) {
+    return (tile == 0 || tile_expert[tile - 1] != e) && (tile + 1 == ntiles || tile_expert[tile + 1] != e);
+}
+
 // Tiles of 256 rows (prompts): 256 weight rows per workgroup of four waves, 128 x 128 results and a SIMD each. A wave has nobody
 // to hide behind, so its reads of the next operands and the loads of later stages are placed between the products, one every
 // few. With 128 x 64 a wave (eight of them) the operands' reads alone took as many LDS cycles as the products took matrix cycles.
@@ -73,8 +78,9 @@ __device__ __forceinline__ void product(f32x4& a, const s16x8& w, const s16x8& x
 // being at 1.75 to 1.9 GHz then. Measured, 64 experts of 768 x 2048, 8 per token, gate_up / down, us (before: eight waves, a
 // workgroup per tile and columns, two stages): 2048 tokens 153 / 85 (174 / 94), 5637 tokens 273 / 170 (305 / 189), 8192 tokens
 // 380 / 255 (434 / 275).
-// ONCE: an expert's weights go past the caches (non-temporal), for about one tile an expert: a step of 1563 tokens (195
-// pairs each) 2040 -> 1990 us. With several tiles, which read them from there, that is the slower way (700 pairs: 4498 -> 4628).
+// ONCE: weights of an expert with one tile go past the caches (non-temporal), those of an expert with several, which read them from
+// there, do not: 64 experts of 768 x 2048, both products, us (all cached / all past): 1563 tokens 185 (195 / 186), unevenly loaded 192
+// (196 / 202), 2048 tokens 260 (259 / 275). The loops for both are one inlined body each: as calls they kept their captures in scratch.
 template <int KIND, int ACT, bool ONCE>
 __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
     constexpr bool GATED = KIND != kDown, ROUTED = KIND != kGated, GATHER = KIND != kDown;
@@ -113,12 +119,14 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
     };
     // the item after this one: its rows' pairs are read an item ahead
     int next_e = 0, next_pair = 0, next_rows[L];
-    auto peek = [&](int it) {
+    bool next_once = false, once = false;  // the item's
+    auto peek = [&](int it) __attribute__((always_inline)) {
         if constexpr (ROUTED) {
             int tile, col;
             place(it, tile, col);
             const int32_t* order = p.order + (int64_t)tile * TM;
             next_e = p.tile_expert[tile];
+            if constexpr (ONCE) next_once = one_tile(p.tile_expert, tile, p.ntiles, next_e);
             next_pair = order[tid];
             if constexpr (GATHER)
 #pragma unroll
@@ -130,17 +138,17 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
     const int chunk[2] = {(lane % 8 ^ lane / 16) * 8, (lane % 8 ^ (lane / 16 + 4)) * 8};  // even, odd piece
     const uint16_t *xs[GATHER ? L : 2], *ws[2];
     auto wrap = [](int slot) { return slot >= RING ? slot - RING : slot; };
-    auto fetch = [&](int t, int base, int i) {  // load i of stage t (the last again past the end), whose first slot is base
+    auto fetch = [&](auto nt, int t, int base, int i) __attribute__((always_inline)) {  // load i of stage t (the last again past the end), whose first slot is base
         uint16_t* dst = smem + wrap(base + i / 2) * kSlot + (wave * 2 + i % 2) * 512;
         const int64_t k0 = min(t, nk - 1) * BK;
         const int64_t row = (i % L) / 2 * 64 + (GATED && i >= L + L / 2 ? p.N - OC : 0);
         const uint16_t* src = i >= L ? ws[i % 2] + (k0 + row * p.ldw) : GATHER ? xs[i % L] + k0 : xs[i % 2] + (k0 + row * p.ldx);
-        if (ONCE && i >= L) __builtin_amdgcn_global_load_lds((gbl_void*)src, (lds_void*)dst, 16, 0, 2);
+        if (nt.value && i >= L) __builtin_amdgcn_global_load_lds((gbl_void*)src, (lds_void*)dst, 16, 0, 2);
         else __builtin_amdgcn_global_load_lds((gbl_void*)src, (lds_void*)dst, 16, 0, 0);
     };
     int n0, q = 0;
     const double per_row = KIND == kGateUp ? 1.0 / p.row_div : 0.0;
-    auto open = [&](int it) {  // start on the item that was peeked at
+    auto open = [&](int it) __attribute__((always_inline)) {  // start on the item that was peeked at
         const int r0 = wave * 16 + lane / 8;
         int tile, nb;
         place(it, tile, nb);
@@ -163,10 +171,15 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
             const uint16_t* xt = p.x + (tile * TM + r0) * p.ldx;
             xs[0] = xt + chunk[0], xs[1] = xt + 8 * p.ldx + chunk[1];
         }
+        auto first = [&](auto nt) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < 2 * L; ++i) fetch(0, 0, i);
+            for (int i = 0; i < 2 * L; ++i) fetch(nt, 0, 0, i);
 #pragma unroll
-        for (int i = 0; i < E1 + E2 + F3; ++i) fetch(1, 8, i);
+            for (int i = 0; i < E1 + E2 + F3; ++i) fetch(nt, 1, 8, i);
+        };
+        once = next_once;
+        if (ONCE && once) first(std::true_type{});
+        else first(std::false_type{});
         if constexpr (KIND == kGated) next_pair = tile * TM + tid < p.n ? tile * TM + tid : -1;
         s_row[q][tid] = GATED && next_pair >= 0 ? tile * TM + tid : next_pair;
         if constexpr (!GATED) s_wt[q][tid] = p.weight && next_pair >= 0 ? p.weight[next_pair] : 1.f;
@@ -184,7 +197,7 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
     const uint32_t oat = lds0 + (16 * kSlot + wave * 16 * LO) * 2;
 
     // A step's products in four groups: half of the depth ks, half h of the 2 MH tiles of rows that are in use.
-    auto run = [&](auto mh_, bool more) {
+    auto run = [&](auto mh_, auto nt, bool more) __attribute__((always_inline)) {
         constexpr int MH = mh_, M = MH * NT;
         f32x4 acc[2 * MH][NT];
 #pragma unroll
@@ -212,7 +225,7 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
             }
         };
         // the products of (ks, h) with `jobs` calls of job spread between them
-        auto group = [&](auto ks_, auto h_, auto jobs_, auto job) {
+        auto group = [&](auto ks_, auto h_, auto jobs_, auto job) __attribute__((always_inline)) {
             constexpr int ks = ks_, h = h_, J = jobs_;
 #pragma unroll
             for (int i = 0; i < M; ++i) {
@@ -236,16 +249,16 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
             const int b1 = wrap(b0 + 8), b2 = wrap(b1 + 8);  // of the next stages
             group(I0{}, I0{}, std::integral_constant<int, MH + 2 * L - E1 - E2 - F3>{}, [&](int j) {
                 if (j < MH) read_x(b0, 0, 1, j);
-                else fetch(t + 1, b1, E1 + E2 + F3 + j - MH);
+                else fetch(nt, t + 1, b1, E1 + E2 + F3 + j - MH);
             });
             group(I0{}, I1{}, std::integral_constant<int, NT + MH + E1>{}, [&](int j) {
                 if (j < NT) read_w(b0, 1, j);
                 else if (j < NT + MH) read_x(b0, 1, 0, j - NT);
-                else fetch(t + 2, b2, j - NT - MH);
+                else fetch(nt, t + 2, b2, j - NT - MH);
             });
             group(I1{}, I0{}, std::integral_constant<int, MH + E2>{}, [&](int j) {
                 if (j < MH) read_x(b0, 1, 1, j);
-                else fetch(t + 2, b2, E1 + j - MH);
+                else fetch(nt, t + 2, b2, E1 + j - MH);
             });
             wait_loads<E1 + E2>();         // this wave's loads of stage t + 1 have landed, its reads of stage t too
             __builtin_amdgcn_s_barrier();  // and everyone's
@@ -253,7 +266,7 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
             group(I1{}, I1{}, std::integral_constant<int, NT + MH + F3>{}, [&](int j) {
                 if (j < NT) read_w(b1, 0, j);
                 else if (j < NT + MH) read_x(b1, 0, 0, j - NT);
-                else fetch(t + 2, b2, E1 + E2 + j - NT - MH);
+                else fetch(nt, t + 2, b2, E1 + E2 + j - NT - MH);
             });
             b0 = b1;
         }
@@ -271,7 +284,7 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
             open(item + stride);
         }
         uint4 v[2][SI];
-        auto gather = [&](int m, uint4 (&y)[SI]) {
+        auto gather = [&](int m, uint4 (&y)[SI]) __attribute__((always_inline)) {
 #pragma unroll
             for (int n = 0; n < NT; ++n) asm volatile("" : "+a"(acc[m][n]));  // in the accumulators' registers until here
 #pragma unroll
@@ -296,7 +309,7 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
                 y[k] = *reinterpret_cast<const uint4*>(&b[k]);
             }
         };
-        auto leave = [&](int m, const uint4 (&y)[SI]) {
+        auto leave = [&](int m, const uint4 (&y)[SI]) __attribute__((always_inline)) {
             int row[SI];
 #pragma unroll
             for (int k = 0; k < SI; ++k) row[k] = s_row[o][(2 * m + wm) * 16 + k * (64 / LR) + lane / LR];
@@ -324,10 +337,14 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
         const int rows = max(max(sr[0], sr[1]), max(sr[2], sr[3]));
         const bool more = item + stride < end;
         if (more) peek(item + stride);
-        if (rows > 192) run(std::integral_constant<int, 4>{}, more);
-        else if (rows > 128) run(std::integral_constant<int, 3>{}, more);
-        else if (rows > 64) run(std::integral_constant<int, 2>{}, more);
-        else run(std::integral_constant<int, 1>{}, more);
+        auto all = [&](auto nt) __attribute__((always_inline)) {
+            if (rows > 192) run(std::integral_constant<int, 4>{}, nt, more);
+            else if (rows > 128) run(std::integral_constant<int, 3>{}, nt, more);
+            else if (rows > 64) run(std::integral_constant<int, 2>{}, nt, more);
+            else run(std::integral_constant<int, 1>{}, nt, more);
+        };
+        if (ONCE && once) all(std::bool_constant<ONCE>{});
+        else all(std::false_type{});
     }
 }
 

@@ -506,6 +506,34 @@ def test_wide_tiles_agree_on_both_sides_of_a_tile_an_expert(n):
     assert torch.equal(wide, staged)
 
 
+@pytest.mark.parametrize("n", (64, 200, 700))
+def test_experts_with_one_tile_beside_such_with_several(n):
+    """Matrices of 67 and 34 MB, whose weights go past the caches where an expert has one tile: loads from nothing to all tokens an
+    expert, so that every tile size has both. Tiles of 64 and more agree bit for bit, streamed ones sum in shares."""
+    g = torch.Generator(device=DEV).manual_seed(n)
+    sh = lk.moe_shape(1024, 256, 64, 4)
+    mk = lambda *s, scale=1.0: (torch.randn(s, generator=g, device=DEV) * scale).to(BF16)  # noqa: E731
+    x, wgu, wd = mk(n, 1024), mk(64, 2, 256, 1024, scale=0.05), mk(64, 1024, 256, scale=0.1)
+    score = torch.rand(n, 64, generator=g, device=DEV) + 3 * torch.rand(64, generator=g, device=DEV)
+    score[:, 7] += 9  # an expert that every token chooses
+    weight, idx = (score - score.min()).topk(4, -1)
+    idx, weight = idx.to(torch.int32), weight.contiguous()
+    loads = torch.bincount(idx.flatten().long(), minlength=64)
+    assert int(loads.max()) == n and int(((loads > 0) & (loads <= 16)).sum()) > 0
+    rows = {tm: lk.moe_experts(sh, x, idx, weight, wgu, wd, tm=tm) for tm in (16, 32, 64, 128, 256)}
+    for tm in (128, 256):
+        assert torch.equal(rows[tm], rows[64])
+    e, xr = idx.flatten().long(), x.double().repeat_interleave(4, 0)
+    want = torch.empty(4 * n, 1024, dtype=torch.float64, device=DEV)
+    for k in range(64):
+        at = (e == k).nonzero()[:, 0]
+        z = xr[at] @ wgu[k].double().transpose(1, 2)
+        act = (torch.nn.functional.silu(z[0]) * z[1]).to(BF16).double()  # as it is stored between the products
+        want[at] = act @ wd[k].double().t() * weight.flatten()[at, None].double()
+    for tm in rows:
+        assert float((rows[tm].double() - want).norm()) <= 2.0 ** -8 * float(want.norm())
+
+
 @pytest.mark.parametrize("experts,top,n,tm", [(64, 8, 4, 16), (64, 8, 95, 16), (64, 8, 128, 32), (16, 4, 60, 32)])
 def test_streamed_tiles_repeat_bit_for_bit(experts, top, n, tm):
     """The tiles that decode steps take, products of a real layer's size over and over: an operand that is overwritten while it
