@@ -1408,14 +1408,16 @@ def moe_one(sh, logits, column: int, correction, x, gate_up, down) -> Optional[t
 
 
 def moe_tile(sh, n: int) -> int:
-    """Rows per tile of the experts' products for n tokens. Tiles of 64 rather than 128 up to 60 rows an expert where the gated ones
-    have the narrow form (up to 2048 wide; 64 experts, 8 a token, both products, us: 768 x 2048, 384 tokens 138 against 165, 448
-    150 / 165, 512 170 / 167; 1536 x 4096, 384 tokens 466 / 494 and, unevenly loaded, 531 / 500, 448 528 / 489). 128 rather than
-    256 up to 200 where a quarter of the wide form's columns would be none and 256 rows are staged (576 x 1536: 800 tokens 113 /
-    134, 1200 146 / 141, 2000 168 / 164; 768 x 2048, 896 tokens 194 / 186). Widths below 1024, whose products are launches, as the
-    widest."""
-    mean, real = n * sh.top / sh.experts, sh.width >= 1024
-    return (256 if mean >= (200 if real and sh.ff % 128 else 112) else 128 if mean >= (60 if real and sh.width <= 2048 else 48)
+    """Rows per tile of the experts' products for n tokens: 64 from 12 rows an expert, 128 from 48, 256 from 112. Both products of 64
+    experts, 8 a token, us, loads even / a third / two thirds apart:
+    128 from 60 at widths of 1536 to 2048 (tiles of 64 against 128: 768 x 2048, 448 tokens 143 / 161 / 140 against 160 / 163 / 137, 512
+    169 / 169 / 155, 163 / 167 / 152; but 384 x 1024, 384 tokens 44 / 50 / 46, 43 / 43 / 42; 1536 x 4096 441 / 511 / 464, 485 / 486 / 445).
+    256 from 136 below 2048 where a quarter of the wide form's columns would be none and 256 rows are staged (128 against 256: 576 x
+    1536, 1024 tokens 126 / 122 / 117, 135 / 136 / 132, 1200 tokens 146 / 142 / 120, 137 / 137 / 133; but 704 x 2048, 1024 tokens
+    192 / 200 / 187, 174 / 189 / 186; 1472 x 4096, 896 tokens 584 / 647 / 582, 574 / 575 / 572)."""
+    mean = n * sh.top / sh.experts
+    staged = 1536 <= sh.width < 2048 and sh.ff % 128
+    return (256 if mean >= (136 if staged else 112) else 128 if mean >= (60 if 1536 <= sh.width <= 2048 else 48)
             else 64 if mean >= 12 else 16)
 
 

@@ -525,7 +525,10 @@ def test_experts_tiles_follow_the_mean_load():
     assert [mixers.lk.moe_tile(sh, n) for n in (1, 64, 95, 96, 383, 384, 895, 896, 8192)] == [16, 16, 16, 64, 64, 128, 128, 256, 256]
 
 
-@pytest.mark.parametrize("width,ff,sizes", [(2048, 768, {479: 64, 480: 128, 895: 128, 896: 256}), (1536, 576, {479: 64, 1599: 128, 1600: 256}),
+@pytest.mark.parametrize("width,ff,sizes", [(2048, 768, {479: 64, 480: 128, 895: 128, 896: 256}),
+                                            (1536, 576, {479: 64, 480: 128, 1087: 128, 1088: 256, 1200: 256}),
+                                            (2048, 704, {895: 128, 896: 256}), (4096, 1472, {384: 128, 896: 256, 1400: 256}),
+                                            (1024, 384, {383: 64, 384: 128, 895: 128, 896: 256}),
                                             (4096, 1536, {383: 64, 384: 128, 896: 256}), (512, 192, {384: 128, 896: 256})])
 def test_experts_tiles_follow_the_faster_form(width, ff, sizes):
     sh = mixers.lk.moe_shape(width, ff, 64, 8, 8, 4)
