@@ -1637,8 +1637,7 @@ constexpr int kPTieCap = 1024;  // elements at a split cut key
 constexpr int kPTieRes = 64;    // pass 1 ranks at most this many cut-key records (else pass 2)
 constexpr int kPCandCap = 2048; // pass 1's exactly scored elements (seeds + bound survivors)
 constexpr int32_t kRowPending = -4;  // RowFilter.ik between the two top_p kernels: pass 2 to run
-constexpr int kP2Splits = 8;         // pieces per left row in sample_topp_pass2_kernel
-constexpr int kP2Rows = 32;          // rows side by side in its grid: a workgroup per CU
+constexpr int kP2Splits = 8;         // workgroups per left row in sample_topp_pass2_kernel
 struct ToppPending {  // a row pass 1 did not decide, for sample_topp_pass2_kernel
     float xlo, xc, lse, mx;  // admissibility bound, the cut key's value, the raw lse, the raw max
     float e_s;               // e*: pass 1's best admissible record (score, index)
@@ -2754,9 +2753,10 @@ __global__ __launch_bounds__(kPNT) __attribute__((amdgpu_waves_per_eu(4))) void 
 }
 
 // Pass 2 of the rows sample_topp_kernel left pending (RowFilter.ik = kRowPending), each row cut into
-// kP2Splits pieces of contiguous vectors (a fixed partition: the split-mode sampler's pattern). Mostly no row is left, so a
-// workgroup looks at every kP2Rows-th row: 512 rows take 2.9 us to find that there are none, with a workgroup for each row and
-// piece 3.7 (64 rows 2.1 and 1.9, one row 2.3 and 3.6; the next launch's own minimum is 1.7).
+// kP2Splits workgroups of contiguous vectors (a fixed partition: the split-mode sampler's pattern). The other rows' workgroups
+// exit: 512 rows take 3.7 us to find that none is left. With 32 rows side by side in the grid, whose workgroups walk every 32nd row,
+// that is 2.9, but left rows wait for each other and the walk's loop costs each of them 8 us: all rows left, both passes, us, here / so:
+// 1 row 55 / 62, 64 rows 70 / 100, 512 rows 126 / 411.
 // (Measured and dropped: a (slots x 8) grid over the left rows only, 25.6 vs 24 us; pass 2
 // inside pass 1's launch with the left rows' pieces claimed by the workgroups that finished -- a
 // CAS-claimed queue head ~1.4 ms, a row-by-row walk ~120 us, tickets ~88-91 vs 80-82 us a launch:
@@ -2764,29 +2764,22 @@ __global__ __launch_bounds__(kPNT) __attribute__((amdgpu_waves_per_eu(4))) void 
 // MODE 2 over the admissible elements x >= xlo of the piece, bar and best starting from e*; the
 // split cut key's indices appended to the row's tie list (one agent-scope add per lane). The last
 // arriving piece (arrive_last) merges the pieces' bests, ranks the ties by index (the first c are
-// admissible, scored exactly) and writes token, logprob and cut.
+// admissible, scored exactly) and writes token, logprob and cut. The other rows' workgroups exit.
 template <typename T, bool TOPP>
 __global__ __launch_bounds__(kPNT) void sample_topp_pass2_kernel(
     const T* __restrict__ logits, int64_t ld, int V, float inv_t, uint64_t seed, const int64_t* __restrict__ seq_ids,
     int64_t step, int32_t* __restrict__ tokens, float* __restrict__ logp_out, RowFilter* __restrict__ filt,
     const ToppPending* __restrict__ pend, unsigned* __restrict__ pend_nt, int32_t* __restrict__ ties,
-    Best* __restrict__ parts, int nseq) {
+    Best* __restrict__ parts) {
     constexpr int NT = kPNT, NW = NT / kWave, VEC = 8, kPer = 8;  // up to kPer vectors per lane
+    const int row_i = blockIdx.x, piece = blockIdx.y;
+    if (filt[row_i].ik != kRowPending) return;  // (workgroup-uniform)
     __shared__ float s_bar, s_bs[NW];
     __shared__ int32_t s_bi[NW];
     __shared__ int s_last, s_icut;
     __shared__ int32_t s_tidx[kPTieCap];
-    const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
-    // of the rows r0, r0 + gridDim.x, .. the left ones (no row of them is done before this workgroup's piece is: every wave reads
-    // the same)
-    auto left = [&](int r0) {
-        const int r = r0 + lane * (int)gridDim.x;
-        return __builtin_amdgcn_ballot_w64(r < nseq && filt[r].ik == kRowPending);
-    };
-    unsigned long long m = left(blockIdx.x);
-    if (m == 0 && nseq <= kWave * (int)gridDim.x) return;
-    auto run = [&](int row_i, int piece) {
     const ToppPending st = pend[row_i];
+    const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
     const T* row = logits + (int64_t)row_i * ld;
     const uint4* rv = reinterpret_cast<const uint4*>(row);
     const int nvec = V / VEC;
@@ -3003,16 +2996,6 @@ __global__ __launch_bounds__(kPNT) void sample_topp_pass2_kernel(
         filt[row_i] = RowFilter{st.mx, 0u, kRowDone, st.kc, icut};
 #endif
     }
-    };
-    for (int r0 = blockIdx.x;;) {
-        for (; m; m &= m - 1) {
-            run(r0 + (__ffsll((long long)m) - 1) * (int)gridDim.x, blockIdx.y);
-            __syncthreads();  // the shared words are the next row's
-        }
-        r0 += kWave * gridDim.x;
-        if (r0 >= nseq) return;
-        m = left(r0);
-    }
 }
 
 constexpr int kMaxSplits = 64;
@@ -3118,8 +3101,8 @@ int launch_sample(const void* logits, int64_t ld, int nseq, int V, float tempera
                                    probe);
             int rc = check_launch("sample_topp_kernel");
             if (rc || !use_topp || (probe >= 1 && probe <= 4) || probe == 11) return rc;  // (probes 1-4, 11)
-            hipLaunchKernelGGL((sample_topp_pass2_kernel<T, true>), dim3(nseq < kP2Rows ? nseq : kP2Rows, kP2Splits), dim3(kPNT), 0, stream, lg, ld,
-                               V, inv_t, seed, seq_ids, step, tokens, logp, filt, pend, pend_nt, pties, pparts, nseq);
+            hipLaunchKernelGGL((sample_topp_pass2_kernel<T, true>), dim3(nseq, kP2Splits), dim3(kPNT), 0, stream, lg, ld,
+                               V, inv_t, seed, seq_ids, step, tokens, logp, filt, pend, pend_nt, pties, pparts);
             return check_launch("sample_topp_pass2_kernel");
         }
     }

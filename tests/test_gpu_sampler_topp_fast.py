@@ -126,9 +126,8 @@ def test_topp_fast_ranks_cut_key_ties_in_pass1(dev):
 
 @pytest.mark.parametrize("n", [31, 32, 33, 100, 2100])
 @pytest.mark.parametrize("temp,p", [(1.0, 0.9), (0.05, 0.95), (8.0, 0.5)])
-def test_pass2_workgroups_take_several_rows(dev, n, temp, p):
-    """Pass 2's grid has 32 rows side by side, whose workgroups take every 32nd, 64 of them at a look: all rows through pass 2
-    and the ordinary run, at temperatures whose masses end far above and far below the row's values."""
+def test_pass2_of_all_rows_equals_the_ordinary_run(dev, n, temp, p):
+    """All rows through pass 2 and the ordinary run, at temperatures whose masses end far above and far below the row's values."""
     V = 2056
     g = torch.Generator().manual_seed(n)
     x = (torch.randn(n, V, generator=g) * 3).to(torch.bfloat16).to(dev)
