@@ -269,6 +269,7 @@ __global__ __launch_bounds__(kNT * HG) __attribute__((amdgpu_waves_per_eu(1, 2))
     __shared__ __attribute__((aligned(16))) uint16_t s_c[64 * LDR];  // first the query, then the tile
     __shared__ __attribute__((aligned(16))) float s_scores[HG * 16 * LDS_];  // scores [head][key of the tile]
     const int t = blockIdx.z;
+    const int near_row = bt_row[min(max(t - 1 + min((int)threadIdx.x & 63, 2), 0), ntok - 1)];
     const int pos = (int)positions[t];
     const int lo = window > 0 ? max(0, pos - window + 1) : 0;
     const PageSplit sp = page_split(lo, pos, part_min, nparts);
@@ -286,10 +287,13 @@ __global__ __launch_bounds__(kNT * HG) __attribute__((amdgpu_waves_per_eu(1, 2))
     const int np = min(sp.per, sp.np - part * sp.per);
     const int32_t* bt = tables + (int64_t)bt_row[t] * bt_stride + first;
     // Pages come in windows of 64, whose block ids a wave holds by lane (no table load ahead of a page's).
-    // Pages go past the caches (non-temporal): up to 32 heads a workgroup has them alone, and the step's weights put them out
-    // before the next step (in a step's place: 64 rows 29.5 -> 24.5 us, 256 rows 67 -> 58.5).
+    // Pages that a workgroup has alone go past the caches (non-temporal), since the step's weights put them out before the next step:
+    // up to 32 heads, and where the neighbouring tokens' page in the place of its first is another one, which it is not for tokens
+    // of one sequence or for sequences that share a prompt. 512 + 64, 16 / 32 heads, us with the caches swept before each launch (all
+    // cached; all past): 64 rows 41.5 / 34 (52 / 46; 41.5 / 34), 256 rows 80 / 66 (112 / 105; 80 / 65), 256 rows on 32 prompts 71 / 59
+    // (72 / 60; 73 / 66), 64 sequences of 4 tokens 73 / 61 (74 / 61; 83 / 64); 48 heads, 64 sequences of 4 tokens 111 (110; 127).
     // Loads are unconditional, the last page again past the end: a branch around them would turn every
-    // wait into one for all loads in flight.
+    // wait into one for all loads in flight. Both ways of the one in load_page issue the same number.
     const int rc = EXACT ? NK * 4 : nk * 4;  // pieces per row
     auto piece = [&](int k) { return min(lane + 64 * (hg + HG * k), 16 * rc - 1); };
     int lds_at[NL];
@@ -304,10 +308,23 @@ __global__ __launch_bounds__(kNT * HG) __attribute__((amdgpu_waves_per_eu(1, 2))
         npw = min(64, np - w0);
         tbl = bt[w0 + min(lane, npw - 1)];
     };
+    window_at(0);
+    const int near = tables[(int64_t)near_row * bt_stride + first];  // by lane: the first page here of tokens t - 1, t, t + 1
+    bool alone = false;
     auto load_page = [&](int j) {
         const uint16_t* p = cache + (int64_t)__builtin_amdgcn_readlane(tbl, min(j, npw - 1)) * kBS * row;
+        auto load = [&](auto once) {
+            asm volatile("; pages %0" ::"n"(once.value));  // else the compiler takes both ways' loads for the same, ordinary ones
 #pragma unroll
-        for (int k = 0; k < NL; ++k) st_[k] = __builtin_nontemporal_load(reinterpret_cast<const s16x8*>(p + piece(k) * 8));
+            for (int k = 0; k < NL; ++k) {
+                const s16x8* src = reinterpret_cast<const s16x8*>(p + piece(k) * 8);
+                if constexpr (once.value) st_[k] = __builtin_nontemporal_load(src);
+                else st_[k] = *src;
+            }
+            asm volatile("; pages %0" ::"n"(once.value));
+        };
+        if (alone) load(std::true_type{});
+        else load(std::false_type{});
     };
     // The query rows of this head group, [latent | rotated | 0], through LDS into MFMA operands. Loads return in order: those of
     // whole 16-byte pieces go ahead of the pages', all at once, and land while the block table is read (16 heads, 512 + 64,
@@ -336,7 +353,9 @@ __global__ __launch_bounds__(kNT * HG) __attribute__((amdgpu_waves_per_eu(1, 2))
             q_[i] = *reinterpret_cast<const s16x8*>((latent ? qa : q_rot) + at);
         }
     }
-    window_at(0);
+    const int mine = __builtin_amdgcn_readlane(near, 1);
+    alone = gridDim.y == 1 && (t == 0 || __builtin_amdgcn_readlane(near, 0) != mine) &&
+            (t == ntok - 1 || __builtin_amdgcn_readlane(near, 2) != mine);
     load_page(wave);
     if (pieces) {
 #pragma unroll

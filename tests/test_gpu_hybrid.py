@@ -111,6 +111,30 @@ def test_latent_attend(heads, rank, rot, window, dtype):
         close(out, want, dtype)
 
 
+@pytest.mark.parametrize("heads,rank,rot", [(3, 40, 24), (16, 512, 64), (32, 512, 64), (40, 256, 64), (20, 512, 96)])
+@pytest.mark.parametrize("window", (None, 100))
+def test_pages_of_one_token_and_of_several(heads, rank, rot, window):
+    """Tokens beside others of their sequence, beside a sequence that shares its first pages and beside strangers: each has the bits
+    that it has in a launch of its own, where its pages are nobody else's."""
+    g = torch.Generator().manual_seed(heads)
+    lens = [300, 90, 333, 333, 310]
+    cache, tables, _ = paged_latents(g, lens, rank, rot, torch.bfloat16)
+    tables[3, :10], tables[4, :20] = tables[2, :10], tables[3, :20]
+    rows = [0, 0, 0, 1, 2, 3, 4, 4, 1]
+    pos = [297, 298, 299, 89, 332, 332, 308, 309, 5]
+    T = len(rows)
+    q = rnd(g, T, heads, rank + rot, dtype=torch.bfloat16).to(DEV)
+    qa = q[:, :, :rank].transpose(0, 1).contiguous()
+    cache, tables = cache.to(DEV), tables.to(DEV)
+    rows, pos = torch.tensor(rows, dtype=torch.int32, device=DEV), torch.tensor(pos, device=DEV)
+    for nparts in (1, 3, 17):
+        run = lambda a, b: lk.latent_attend(qa[:, a:b].contiguous(), q[a:b, :, rank:], cache, rank, rot, tables, rows[a:b],  # noqa: E731
+                                            pos[a:b], 0.1, window, nparts=nparts, part_min=16)
+        both = run(0, T)
+        for t in range(T):
+            assert torch.equal(both[:, t], run(t, t + 1)[:, 0])
+
+
 def _write_case(n, width, rot, rank, seed):
     g = torch.Generator(device=DEV).manual_seed(seed)
     rand = lambda *s: torch.randn(*s, device=DEV, generator=g)  # noqa: E731
