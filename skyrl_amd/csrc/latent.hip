@@ -771,10 +771,12 @@ __device__ __forceinline__ s16x8 key_chunk(const uint16_t* nope, const uint16_t*
         else if (d < dim + rot) f = *reinterpret_cast<const s16x8*>(rotp + (d - dim));
         return f;
     }
+    const uint16_t* none = dim > 0 ? nope : rotp;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < 8; ++j) {  // loads without a branch
         const int dd = d + j;
-        f[j] = (short)(dd < dim ? nope[dd] : dd < dim + rot ? rotp[dd - dim] : (uint16_t)0);
+        const uint16_t x = *(dd < dim ? nope + dd : dd < dim + rot ? rotp + (dd - dim) : none);
+        f[j] = (short)(dd < dim + rot ? x : 0);
     }
     return f;
 }
@@ -861,15 +863,18 @@ __global__ __launch_bounds__(512 / QT) __attribute__((amdgpu_waves_per_eu(2))) v
     const int r8 = lane >> 3;
     auto key_swizzle = [](int r) { return ((r & 3) >> 1) | ((r >> 3 & 3) << 1); };
     auto piece = [&](int i) { return wave + NW * i; };  // the wave's i-th: of keys 8-row group % 8, column group / 8
-    auto kcol = [&](int i) { return 64 * (piece(i) / 8) + 8 * ((lane & 7) ^ key_swizzle(piece(i) % 8 * 8 + r8)); };
     s16x8 kr[VEC ? 1 : KPW];
     auto fetch = [&](int j) {
         char* dst = smem + (j - j0 & 1) * BUF;
         const int64_t r0 = seg_row + (int64_t)j * kKT;
+        int own = lane;
+        // else the addresses and limits of all unaligned pieces' elements stay in registers from tile to tile, and most of them in
+        // memory: 164 and 408 bytes a lane at dk of 128 and 192, now none and 12
+        if (!VEC) asm volatile("" : "+v"(own));
 #pragma unroll
         for (int i = 0; i < KPW; ++i) {
-            const int64_t row = r0 + piece(i) % 8 * 8 + r8;
-            const int d = kcol(i);
+            const int at = piece(i) % 8 * 8 + (own >> 3), d = 64 * (piece(i) / 8) + 8 * ((own & 7) ^ key_swizzle(at));
+            const int64_t row = r0 + at;
             const uint16_t *kp = k_nope + row * k_stride + (int64_t)h * dim, *rp = k_rot + row * rot;
             if constexpr (VEC) {
                 const void* src = d < dim ? (const void*)(kp + d) : d < dk ? (const void*)(rp + (d - dim)) : (const void*)&kNoKey;
