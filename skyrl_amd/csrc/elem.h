@@ -91,6 +91,19 @@ __device__ __forceinline__ float sigmoidf_(float x) { return 1.f / (1.f + expf(-
 __device__ __forceinline__ float siluf_(float x) { return x / (1.f + expf(-x)); }
 __device__ __forceinline__ float softplusf_(float x) { return fmaxf(x, 0.f) + log1pf(expf(-fabsf(x))); }
 
+// Sum of squares, in one order wherever a row's norm is formed: left to the compiler, either of the first two is the rounded one.
+template <int N>
+__device__ __forceinline__ float squares(const float (&y)[N]) {
+    if constexpr (N == 1) {
+        return y[0] * y[0];
+    } else {
+        float s = fmaf(y[0], y[0], y[1] * y[1]);
+#pragma unroll
+        for (int j = 2; j < N; ++j) s = fmaf(y[j], y[j], s);
+        return s;
+    }
+}
+
 // Sum over a block of NT threads, in every thread; lds holds NT / 64 floats and is free again on return.
 template <int NT>
 __device__ __forceinline__ float block_total(float v, float* lds) {

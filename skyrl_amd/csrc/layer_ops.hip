@@ -528,8 +528,7 @@ __global__ __launch_bounds__(NT) void gate_norm_add_kernel(GateNormAdd<T, A, Z> 
 #pragma unroll
                 for (int j = 0; j < VEC; ++j) y[k][j] *= sigmoid_<T>(z[j] + b[j]);
             }
-#pragma unroll
-            for (int j = 0; j < VEC; ++j) r[k] += y[k][j] * y[k][j];
+            r[k] = squares(y[k]);
         }
     }
     scales();
@@ -540,10 +539,8 @@ __global__ __launch_bounds__(NT) void gate_norm_add_kernel(GateNormAdd<T, A, Z> 
         r[k] = 0.f;
         if (v < nv) {
 #pragma unroll
-            for (int j = 0; j < VEC; ++j) {
-                h[k][j] += p.mult * (y[k][j] * rk * ld(&ws[k].v[j]));
-                r[k] += h[k][j] * h[k][j];
-            }
+            for (int j = 0; j < VEC; ++j) h[k][j] += p.mult * (y[k][j] * rk * ld(&ws[k].v[j]));
+            r[k] = squares(h[k]);
             stv(p.h + base + VEC * v, h[k]);
         }
     }

@@ -3,8 +3,9 @@
 // Bound: the weights' bytes, as in rows_product.hip. A step of one row is a chain of launches of a few us each, and every second
 // one was the norm of a single row (4 to 5.5 us, one workgroup on the chip): now each of the product's workgroups (about 200)
 // forms the row for itself, from 24 to 60 KB of which its L2 has most, while its first pieces of the weights are on their way: four
-// waves stream, four form the row (a wave that did both would wait for its weights with its row). Sums are in the order of add_norm_kernel and gate_norm_add_kernel, the same bits. The first workgroup leaves the new residual,
-// in another buffer, since the rest still read the old one, and the normed row where a later launch reads it too.
+// waves stream, four form the row (a wave that did both would wait for its weights with its row). Sums are in the order and the
+// roundings of add_norm_kernel and gate_norm_add_kernel: the same bits. The first workgroup leaves the new residual, in another
+// buffer, since the rest still read the old one, and the normed row where a later launch reads it too.
 // The first row of a step is read from the embedding's table in the same way (a step of one row 5.5 us less).
 // Measured, us in a step's profile, both launches before and the one now (2048 deep): 3648 rows 4.4 + 5.0, 6.8; 12352 rows 4.3 +
 // 10.8, 10.9; gated 12288 rows 4.3 + 11.0, 11.3; two shares of 2112 rows 4.7 + 5.5, 6.2; behind 8 experts' rows, 12352 rows
@@ -201,11 +202,21 @@ struct GateNorm {
         __device__ __forceinline__ void scales(const GateNorm& p, uint32_t red) {
             const int nv = p.H / 8, per = nv / p.groups, sums = per / p.L;
             const float len = (float)(p.H / p.groups);
-            if (p.groups == 1) {
+            if (p.groups == 1) {  // a wave's 64 groups of eight at a time, as that kernel has them
+#pragma unroll
+                for (int k = 0; k < MAXK; ++k) {
+                    const float t = wave_total(r[k]);
+                    if ((threadIdx.x & 63) == 0) lds_put(red + (k * kNT / kWave + (threadIdx.x % kNT >> 6)) * 4, t);
+                }
+                lds_barrier();
                 float one = 0.f;
 #pragma unroll
-                for (int k = 0; k < MAXK; ++k) one += r[k];
-                one = 1.f / sqrtf(total(one, red) / len + p.eps);
+                for (int k = 0; k < MAXK; ++k) {
+                    const f32x4 t = lds_get4(red + k * kNT / kWave * 4);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) one += t[i];
+                }
+                one = 1.f / sqrtf(one / len + p.eps);
 #pragma unroll
                 for (int k = 0; k < MAXK; ++k) r[k] = one;
                 return;
@@ -268,8 +279,7 @@ struct GateNorm {
 #pragma unroll
                     for (int j = 0; j < 8; ++j) y[k][j] *= sigmoid_<uint16_t>(zz[j] + x[j]);
                 }
-#pragma unroll
-                for (int j = 0; j < 8; ++j) r[k] += y[k][j] * y[k][j];
+                r[k] = squares(y[k]);
             }
             scales(p, red);
 #pragma unroll
@@ -281,10 +291,8 @@ struct GateNorm {
                 float x[8];
                 w[k].get(x);
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    h[k][j] += p.mult * (y[k][j] * rk * x[j]);
-                    r[k] += h[k][j] * h[k][j];
-                }
+                for (int j = 0; j < 8; ++j) h[k][j] += p.mult * (y[k][j] * rk * x[j]);
+                r[k] = squares(h[k]);
             }
             scales(p, red + kLongest / 8 * 4);
 #pragma unroll
