@@ -611,7 +611,10 @@ struct LatentNorm {
 constexpr int kQueryRank = 2048;
 __global__ __launch_bounds__(2 * kFormers) void latent_query_kernel(Write<uint16_t> w, RowsProduct p, LatentNorm pre) {
     __shared__ __attribute__((aligned(16))) uint16_t smem[formed_lds<1, 4, kQueryRank, 1, 8>()];
-    if (blockIdx.x == gridDim.x - 1) return write_row<uint16_t, 2 * kFormers>(w, 0);
+    if (blockIdx.x == gridDim.x - 1) {  // as latent_write: its 256 threads' sums (barriers are not waited for by waves that have ended)
+        if (threadIdx.x < kNT) write_row<uint16_t, kNT>(w, 0);
+        return;
+    }
     formed_product<kRound, 1, 4, kQueryRank, 1, 8>(p, pre, smem, 0, false);
 }
 

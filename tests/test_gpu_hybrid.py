@@ -161,9 +161,7 @@ def test_writes_beside_an_up_projection(n, heads, dim, rot, rank, up):
     assert lk.rows_batch(q, w, want)
     qa = lk.latent_lift(proj, *where, cache, 1e-4, w, **args)
     assert torch.equal(proj, p2) and torch.equal(qa, want)
-    if rank:  # sums of 128 threads instead of 256: a bf16 step where they round apart
-        d = (cache.float() - c2.float()).abs()
-        assert float((d - 2.0 ** -7 * c2.float().abs()).max()) <= 0 and int((d > 0).sum()) <= 0.01 * d.numel()
+    assert torch.equal(cache, c2)
     assert lk.latent_lift(torch.cat([proj] * 65)[:65], *where, cache, 1e-4, w, **args) is None
 
 
@@ -179,8 +177,20 @@ def test_query_latent_ahead_of_its_product(q_rank, N, rank, rot):
     ref = p2[:, :q_rank].double() @ w.double().t()
     assert float((q.double() - ref).norm()) <= 2.0 ** -8 * float(ref.norm()) and q.shape == want.shape
     if rank:
-        assert float((cache.float() - c2.float()).abs().max()) <= 2.0 ** -7 * float(c2.float().abs().max())
+        assert torch.equal(cache, c2)
     assert lk.latent_query(torch.cat([proj] * 2), *where, cache, 1e-4, w, qn) is None
+
+
+def test_query_latent_writes_the_cache_of_other_steps():
+    """1500 tokens one by one and in one write: a sum in another order moves some of so many bf16 values."""
+    n, q_rank, rank, rot = 1500, 8, 512, 64
+    rand, proj, (_, pos, slots, table), cache = _write_case(n, q_rank, rot, rank, 9)
+    w, qn, nw = rand(16, q_rank).bfloat16(), rand(q_rank).bfloat16(), rand(rank).bfloat16()
+    one = cache.clone()
+    for t in range(n):
+        lk.latent_query(proj[t:t + 1], rot, pos[t:t + 1], slots[t:t + 1], table, one, 1e-4, w, qn, rank=rank, norm_weight=nw)
+    lk.latent_write(proj, rot, pos, slots, table, cache, 1e-4, q_norm=qn, rank=rank, norm_weight=nw)
+    assert torch.equal(one, cache)
 
 
 @pytest.mark.parametrize("T,heads,rank,rot,vdim", [(1, 16, 512, 64, 128), (2, 3, 40, 24, 24), (3, 16, 512, 64, 128), (4, 32, 256, 64, 40)])
