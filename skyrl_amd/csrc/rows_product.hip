@@ -30,7 +30,7 @@ __global__ __launch_bounds__(WK* kWave) void rows_product_kernel(RowsProduct p) 
 }
 
 constexpr int kWide = 8192;       // output columns from which wider tiles still fill the chip and read x less often
-constexpr int kFill = 256;        // workgroups that a split product is cut into
+constexpr int kFill = 256;        // one workgroup a CU: what a split product is cut into
 constexpr int kManyRowsCols = 4096;
 
 enum Form { kFormRound, kFormGated, kFormParts };
@@ -75,16 +75,48 @@ void launch_rows(RowsProduct p, int splits, hipStream_t s, int batch = 1) {
                        dim3(WK * kWave), 0, s, p);
 }
 
+// Up to 16 rows of x, 16 rows of weights a workgroup up to 512 workgroups of these, 64 up to one workgroup a CU, then 32; us at
+// 1 / 16 rows of x with 16, 32 and 64 rows of weights:
+//   8192 x 2048    7.5 / 8.4     7.7 / 8.0     8.7 / 9.6
+//   8192 x 4096    13.3 / 14.9   13.8 / 14.3   16.9 / 19.2
+//   10240 x 2048   9.9 / 11.2    10.1 / 11.5   9.5 / 10.2
+//   16640 x 2048   15.6 / 16.1   15.6 / 16.0   17.5 / 18.3
+//   24576 x 4096   34.1 / 38.1   34.2 / 35.0   37.1 / 40.0
 template <int MODE>
 void launch_rounded(const RowsProduct& p, hipStream_t s) {
-    if (p.N >= kWide) {
-        if (p.n <= 16) launch_rows<MODE, 4, 1, 4, 2>(p, 1, s);
-        else if (p.n <= 32) launch_rows<MODE, 4, 2, 4, 2>(p, 1, s);
+    if (p.n <= 16) {
+        if (p.N <= kWide) launch_rows<MODE, 1, 1, 4, 4>(p, 1, s);
+        else if (p.N <= 2 * kWide) launch_rows<MODE, 4, 1, 4, 2>(p, 1, s);
+        else launch_rows<MODE, 2, 1, 4, 2>(p, 1, s);
+    } else if (p.N >= kWide) {
+        if (p.n <= 32) launch_rows<MODE, 4, 2, 4, 2>(p, 1, s);
         else launch_rows<MODE, 4, 4, 2, 2>(p, 1, s);
     } else {
-        if (p.n <= 16) launch_rows<MODE, 1, 1, 4, 4>(p, 1, s);
-        else if (p.n <= 32) launch_rows<MODE, 1, 2, 4, 3>(p, 1, s);
+        if (p.n <= 32) launch_rows<MODE, 1, 2, 4, 3>(p, 1, s);
         else launch_rows<MODE, 1, 4, 4, 2>(p, 1, s);
+    }
+}
+
+// Gated, a pair of rows is two rows of weights. Up to 16 rows of x, 32 rows of weights, but 64 where 32 were more than one workgroup
+// a CU and 64 are not, unless the depth makes up for it; us at 1 / 16 rows of x with 32 and 64 rows of weights:
+//   2048 pairs x 2048    6.1 / 7.0     9.5 / 9.9
+//   4096 pairs x 2048    8.7 / 8.3     11.1 / 10.2
+//   6144 pairs x 2048    12.2 / 12.3   11.7 / 11.1
+//   6144 pairs x 4096    20.4 / 23.3   24.7 / 25.1
+//   12288 pairs x 2048   19.4 / 20.0   20.6 / 21.4
+// At 33 to 64 rows of x two waves, two workgroups a CU, where these are one round and four waves would be two; us at 64 rows with two
+// and four waves: 6144 x 2048 17.9, 15.7; 8448 x 2048 25.0, 27.4; 16384 x 2048 30.0, 33.0; 24576 x 2048 53.2, 47.7.
+void launch_gated(const RowsProduct& p, hipStream_t s) {
+    const int tiles = (p.N + 31) / 32;  // of 64 rows
+    if (p.n <= 16) {
+        if (tiles > kFill / 2 && tiles <= kFill && p.K <= 3072) launch_rows<kGated, 4, 1, 2, 4>(p, 1, s);
+        else launch_rows<kGated, 2, 1, 4, 3>(p, 1, s);
+    } else if (p.n <= 32) {
+        launch_rows<kGated, 4, 2, 4, 2>(p, 1, s);
+    } else if (tiles > kFill && tiles <= 2 * kFill) {
+        launch_rows<kGated, 4, 4, 2, 2>(p, 1, s);
+    } else {
+        launch_rows<kGated, 4, 4, 4, 2>(p, 1, s);
     }
 }
 
@@ -118,13 +150,9 @@ int rows_product(const void* x, int64_t ldx, int32_t n, int32_t K, const void* w
                         reinterpret_cast<const uint16_t*>(bias), Gate{act, alpha, limit}, turn0, turn1, cap, out, ldo, (int64_t)n * ldo, 1, 0, 0, 0};
     hipStream_t s = as_stream(stream);
     // Wide tiles where there are columns enough, since every workgroup reads x again; else 16 rows of weights, so that
-    // the chip is full (3648 x 2048 at 64 rows: 8.5 us with 16, 9.4 with 32). Up to 16 rows 64 rows of weights for the wide ones
-    // (12352 x 2048: 12.0 us, with 32 13.8; gated 11.8 with two waves of four slots, 12.4 with four of two). Gated, 64 rows: four
-    // waves 16.4 us, two 18.3.
+    // the chip is full (3648 x 2048 at 64 rows: 8.5 us with 16, 9.4 with 32).
     if (gate) {
-        if (n <= 16) launch_rows<kGated, 4, 1, 2, 4>(p, 1, s);
-        else if (n <= 32) launch_rows<kGated, 4, 2, 4, 2>(p, 1, s);
-        else launch_rows<kGated, 4, 4, 4, 2>(p, 1, s);
+        launch_gated(p, s);
     } else if (splits) {
         if (n == 1) launch_rows<kParts, 1, 1, 4, 4, true, true>(p, splits, s);
         else if (n <= 16) launch_rows<kParts, 1, 1, 4, 4>(p, splits, s);

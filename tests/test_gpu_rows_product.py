@@ -175,9 +175,12 @@ def test_batch_in_order(dev, n, N, K):
 
 # n, columns, depth; what the form has: waves along the depth, slots of each wave's ring
 DEEP = {"rounded": [(16, 3650, 2056, 4, 4), (20, 3650, 2056, 4, 3), (64, 3650, 2056, 4, 2),
-                    (16, 8200, 2056, 4, 2), (32, 8200, 2040, 4, 2), (50, 8200, 2040, 2, 2), (1, 3650, 2056, 4, 4), (1, 8200, 2056, 4, 2)],
+                    (16, 8200, 2056, 4, 2), (32, 8200, 2040, 4, 2), (50, 8200, 2040, 2, 2), (1, 3650, 2056, 4, 4), (1, 8200, 2056, 4, 2),
+                    (16, 8192, 2056, 4, 4), (16, 16392, 2056, 4, 2), (1, 16392, 2056, 4, 2)],
         "parts": [(16, 4104, 2056, 4, 4), (11, 2048, 6152, 4, 4), (32, 2050, 6152, 4, 2), (64, 2056, 6152, 4, 2), (100, 2056, 6152, 4, 1), (1, 2056, 6152, 4, 4)],
-        "gated": [(16, 2056, 2040, 4, 2), (32, 2056, 2040, 4, 2), (64, 2056, 2040, 2, 2), (1, 2056, 2040, 2, 4), (64, 2056, 2040, 4, 2)],
+        "gated": [(16, 2056, 2040, 4, 2), (32, 2056, 2040, 4, 2), (64, 2056, 2040, 2, 2), (1, 2056, 2040, 2, 4), (64, 2056, 2040, 4, 2),
+                  (16, 2056, 2040, 4, 3), (16, 4104, 2040, 2, 4), (1, 8192, 2040, 2, 4), (5, 8200, 2040, 4, 3), (9, 4104, 3080, 4, 3),
+                  (40, 8200, 2040, 2, 2), (64, 16392, 2040, 4, 2)],
         "batch": [(16, 40, 1096, 4, 2), (32, 72, 1096, 4, 2), (100, 24, 1096, 4, 2)]}
 
 
