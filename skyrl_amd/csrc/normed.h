@@ -43,7 +43,8 @@ __device__ __forceinline__ float total(float v, uint32_t red) {
 
 // Pre: RowOf<LONG> with load(pre), form(pre, x, pitch, red): the rows into LDS at x, `pitch` bytes apart, red: kRed floats of
 // scratch; barriers(pre): lds_barrier calls of form; leave(pre): what else becomes of the rows, called in the first workgroup.
-// At most ROWS rows of up to LONG, each in 16 / n of the places; four shares of the depth a workgroup, of its gridDim.y-th.
+// n rows, at most ROWS, of up to LONG: one each in the first places, the last one in the others of 16; four shares of the depth a
+// workgroup, of its gridDim.y-th.
 template <int MODE, int NT, int S, int LONG, int ROWS, int kRed, class Pre>
 __device__ __forceinline__ void formed_product(const RowsProduct& p, const Pre& pre, uint16_t* smem, int batch, bool first) {
     constexpr int WK = kFormers / kWave, kPitch = LONG * 2 + (ROWS > 1 ? 16 : 0);  // bytes

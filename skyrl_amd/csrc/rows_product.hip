@@ -6,14 +6,14 @@
 // with f32 sums of its own that the next norm adds. One row takes the same form, with that row in all 16 places: a wave per
 // weight row, lanes along the depth, took 5.6, 11.6, 6.2, 12.8 and 27.0 us for the five matrices below (its sums start when the
 // whole row is there).
-// Measured on one MI355X, weights from HBM, us (GB/s of weights) against the library's:
+// Measured on one MI355X, weights from HBM and past the caches (stream.h), us, here / the library's:
 //   N, K            1 row            16 rows          32 rows          64 rows
-//   2048, 2048      4.1 / 11.0       4.3 / 11.1       4.6 / 11.3       5.6 / 11.8
-//   2048, 6144      6.8 / 11.0       7.5 / 11.2       8.0 / 16.8       9.9 / 19.7
-//   3648, 2048      5.1 / 11.8       5.6 / 11.8       6.6 / 11.8       8.5 / 12.2   (no splits)
-//   12288, 2048     11.5 / 14.9      11.9 / 14.9      13.4 / 16.8      16.8 / 18.3  (no splits; 4.4 TB/s at one row)
-//   12288, 2048     11.6             11.8             13.4             16.4         (gated)
-//   32768, 2048     25.5 / 31.8      26.0 / 31.9      28.3 / 36.8      28.7 / 37.1  (no splits; 5.3 TB/s at one row)
+//   2048, 2048      3.9 / 10.9       4.1 / 11.0       4.4 / 11.2       5.5 / 11.7
+//   2048, 6144      6.9 / 11.1       7.2 / 11.2       7.5 / 16.5       9.6 / 19.4
+//   3648, 2048      4.8 / 11.8       5.5 / 11.7       6.5 / 11.6       8.4 / 12.1   (no splits)
+//   12288, 2048     11.5 / 16.6      10.9 / 15.2      12.3 / 15.2      16.7 / 16.3  (no splits; 4.4 TB/s at one row)
+//   24576, 2048     20.6 / 40.0      21.7 / 40.1      23.6 / 29.3      29.7 / 30.2  (gated: 12288 pairs of rows)
+//   32768, 2048     24.1 / 35.1      24.6 / 32.9      27.5 / 35.3      27.9 / 35.7  (no splits; 5.6 TB/s at one row)
 // At 64 rows a workgroup's x is as many bytes as its weights, over the same 64 bytes a clock into LDS: 12288 x 2048 gated takes
 // 16.4 us, 13.4 without x, 7.3 without the weights, 5.3 without either; leaving out the products changes it by 0.4.
 // Batches (a head's up-projections of latent attention, 512 x 128 and 128 x 512): 16 heads, 1 / 64 rows, both products with the
@@ -40,16 +40,16 @@ bool rows_take(int n, int K, int N, int form) {
     return n > 0 && K > 0 && N > 0 && K % 8 == 0 && (n <= 64 || (n <= 128 && N <= kManyRowsCols && form == kFormParts));
 }
 
-// Where they are the faster form; us, here / the library's. Above 64 rows its tiles are as fast on wide matrices (128 rows, 12288
-// x 2048: 21.0 / 20.7) and slower on narrow ones only against parts (2048 x 2048 6.9 / 11.5, 2048 x 6144 14.2 / 17.8; rounded
-// 29.3). Depths above 2048 give them more to pipeline:
-//   up to 16 rows  until a matrix is both deep and large: 4096 x 4096 8.5 / 15.5, 30720 x 4096 44.7 / 59.8, 4096 x 6144 in parts
-//                  12.4 / 22.6 (one row: 11.0 / 22.5), 2048 x 8192 8.7 / 13.2 (8.1 / 12.6), but 4096 x 8192 16.7 / 15.9 (16.6 / 15.5).
-//   more rows      in parts, up to 8192 columns (32 rows: 4096 x 12288 24.1 / 27.2, 8192 x 4096 16.0 / 17.1; 64 rows: 27.3 /
-//                  36.0, 18.2 / 18.9); rounded or gated, narrow ones (64 rows, 4096 x 4096 14.3 / 15.6, but 6144 x 4096 23.4 /
-//                  17.8) and up to 32 rows of wide ones 4096 deep (32768 x 4096 53.5 / 65.6, gated 24576 x 4096 43.8 / 49.8;
-//                  64 rows: 67.8 / 61.8, 55.0 / 50.7).
-//   past 16384     at any number of rows (4096 x 18432: 26.9 / 46.7, 42.4 / 122.3, 54.9 / 130.8 at 1, 32, 64 rows).
+// Where they are the faster form; us, here / the library's. Above 64 rows its tiles are as fast on wide matrices and slower on narrow
+// ones only against parts (128 rows, 2048 x 2048 7.2 / 11.1, 2048 x 6144 12.9 / 17.6). Depths above 2048 give them more to pipeline:
+//   up to 16 rows  until a matrix is both deep and large: 4096 x 4096 8.4 / 15.5, 30720 x 4096 43.3 / 59.3, 4096 x 6144 in parts
+//                  12.9 / 23.0 (one row: 11.0 / 22.9), 2048 x 8192 8.5 / 13.1 (7.6 / 12.7); 4096 x 8192 16.1 / 16.2 (15.5 / 15.8), and
+//                  past it little between them (4096 x 12288 20.9 / 22.1): the line is where they were equal with cached weights.
+//   more rows      in parts, up to 8192 columns (32 rows: 4096 x 12288 21.7 / 26.9, 8192 x 4096 14.3 / 16.9; 64 rows: 27.6 /
+//                  37.4, 17.7 / 19.3); rounded or gated, narrow ones (64 rows, 4096 x 4096 13.7 / 15.0, but 6144 x 4096 23.7 /
+//                  18.0) and up to 32 rows of wide ones 4096 deep (32768 x 4096 50.2 / 66.7, gated 24576 x 4096 44.5 / 54.0;
+//                  64 rows: 68.2 / 64.9, 52.3 / 54.4).
+//   past 16384     at any number of rows (4096 x 18432: 26.9 / 51.6, 42.2 / 123.0, 53.6 / 131.8 at 1, 32, 64 rows).
 bool rows_fit(int n, int K, int N, int form) {
     if (!rows_take(n, K, N, form)) return false;
     if (n > 64 || K <= 2048 || K > (1 << 14)) return true;

@@ -2417,8 +2417,8 @@ __global__ __launch_bounds__(kPNT) __attribute__((amdgpu_waves_per_eu(4))) void 
     }
     if constexpr (TOPP) {
         // top_p: a row pass 1 did not decide goes to sample_topp_pass2_kernel (launched next), cut
-        // into kP2Splits workgroups: few rows are left (~5 %), and one alone on this workgroup's CU
-        // spends ~20 us in the visits' VALU. min_p alone leaves most rows (~70 %): the in-row pass 2
+        // into kP2Splits workgroups: few rows are left (SKYRL_TP_RBAR), and one alone on this workgroup's
+        // CU spends ~20 us in the visits' VALU. min_p alone leaves most rows (~70 %): the in-row pass 2
         // below, at full occupancy, is the better form there.
         if (probe < 3 || probe > 4) {
             if (threadIdx.x == 0) {

@@ -14,9 +14,10 @@ typedef __attribute__((address_space(1))) void gbl_void;
 __device__ const uint4 kZero16 = {0u, 0u, 0u, 0u};
 
 // NT 16-row weight tiles, MT 16-row tiles of x, WK waves. HELD: the rows of x lie in LDS whole and are not streamed. ONCE: no
-// other workgroup reads these weight rows, so they go past the caches (non-temporal): a step's weights, several times the
-// last-level cache, put out what is read again and wait for its lines to be put out (32768 x 2048: 1 row 24.8 -> 21.9 us, 64 rows
-// 31.4 -> 27.4; in a step's place, eight of 64 experts of 768 x 2048 for 64 rows 74.8 + 39.3 -> 59.7 + 34.3).
+// other workgroup reads these weight rows (moe_stream_kernel has both, by tile), so they go past the caches (non-temporal): a
+// step's weights, several times the last-level cache, put out what is read again and wait for its lines to be put out (32768 x
+// 2048: 16 rows 28.0 -> 24.6 us, 64 rows 30.1 -> 27.9; in a step's place, eight of 64 experts of 768 x 2048 for 64 rows 74.8 + 39.3
+// -> 59.7 + 34.3).
 // EXACT: the pieces' sums are added in 64 bits, for one row whose results leave in f32. One chain of f32 sums a wave rounds more than
 // the lanes of a wave per weight row did: error / result against 64 bits 0.95e-7, 1.90e-7, 1.65e-7 at 2048, 4096, 6144 deep (2048,
 // 4096, 2048 columns), where those had 0.75e-7, 0.85e-7, 0.91e-7, and this has 0.64e-7 at all (3.9, 8.1, 6.8 us; 4.0, 8.2, 6.9).
@@ -40,8 +41,8 @@ struct Stream {
 
     // acc[m][n]: lane (c, g) has x row 16 m + c, weight rows 16 n + 4 g .. + 3. wrow(r), xrow(r): start of the tile's row r, valid
     // for every r (rows past the last: any row, not stored). K a multiple of 8, the wave's pieces s0 .. s0 + nk - 1 of 64.
-    // HELD: between(), called when the first pieces are under way, returns the LDS address of the one row there is, readable up to
-    // a multiple of 64 with numbers in it; xrow is not called.
+    // HELD: between(), called when the first pieces are under way, returns the LDS address of the row in this lane's place, readable
+    // up to a multiple of 64 with numbers in it; xrow is not called.
     struct Streamed {
         __device__ uint32_t operator()() const { return 0; }
     };
