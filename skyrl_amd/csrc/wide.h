@@ -15,6 +15,27 @@ __device__ __forceinline__ void wait_loads() {
 __device__ __forceinline__ void lds_read(s16x8& v, uint32_t at, int offset) {
     asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(at), "n"(offset));
 }
+__device__ __forceinline__ void lds_read(uint32_t& v, uint32_t at, int offset) {
+    asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(v) : "v"(at), "n"(offset));
+}
+__device__ __forceinline__ void lds_write(uint32_t at, uint32_t v) {
+    asm volatile("ds_write_b32 %0, %1" ::"v"(at), "v"(v) : "memory");
+}
+__device__ __forceinline__ void lds_write(uint32_t at, uint2 v) {
+    asm volatile("ds_write_b64 %0, %1" ::"v"(at), "v"(v) : "memory");
+}
+// 16 bytes from the lanes whose row is not negative, without a way round the store.
+__device__ __forceinline__ void store_row(uint16_t* to, s16x8 v, int row) {
+    uint64_t all;
+    asm volatile(
+        "v_cmp_lt_i32 vcc, -1, %3\n\t"
+        "s_and_saveexec_b64 %0, vcc\n\t"
+        "global_store_dwordx4 %1, %2, off\n\t"
+        "s_mov_b64 exec, %0"
+        : "=&s"(all)
+        : "v"(to), "v"(v), "v"(row)
+        : "vcc", "scc", "memory");
+}
 
 // The gated product of one pair of f32 sums where it is rounded to 16 bits at once: gated()'s forms with the bare exponential and
 // reciprocal, whose error (1e-6 at arguments of 20) is lost in that rounding. Against 64 bits, relative 2-norm, depths 1536 to
@@ -43,17 +64,37 @@ struct Wide {
     int ntiles;  // routed: at most, those in use in tile_expert[ntiles]
     // routed
     const int32_t *order, *tile_expert;
-    int row_div;          // kGateUp: row of x of a pair: pair / row_div
+    int row_div;          // kGateUp: row of x of a pair: pair / row_div, by div_mul and div_shift
+    uint32_t div_mul;
+    int div_shift;
     const float* weight;  // kDown: of the pair, NULL: 1
     // kGated
     int n;
     Gate gate;
 };
 
+// n / d for 0 <= n < 2^31, 1 < d <= 2^31: the upper half of n ceil(2^(32 + s) / d), shifted by s = ceil(log2 d) - 1. The multiplier
+// is less than d <= 2^(s + 1) parts of 2^(32 + s) / d too large, n times which is less than one part of d.
+inline void set_division(Wide& p) {
+    int s = 0;
+    while ((2ll << s) < p.row_div) ++s;
+    p.div_shift = s;
+    p.div_mul = p.row_div > 1 ? (uint32_t)(((1ull << (32 + s)) + p.row_div - 1) / p.row_div) : 0;
+}
+
 // a += w x on 16 x 16 x 32, in the accumulator's own registers (the compiler's form may take others and copy them back on
 // every turn of a loop). Before anything but a product reads them, the caller lets 16 cycles pass.
 __device__ __forceinline__ void product(f32x4& a, const s16x8& w, const s16x8& x) {
     asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(a) : "v"(w), "v"(x));
+}
+
+__device__ __forceinline__ void first_product(f32x4& a, const s16x8& w, const s16x8& x) {
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(a) : "v"(w), "v"(x));
+}
+
+// A uniform value that no store of this launch changes, by a scalar load.
+__device__ __forceinline__ int32_t uniform(const int32_t* p) {
+    return *reinterpret_cast<const __attribute__((address_space(4))) int32_t*>(reinterpret_cast<uintptr_t>(p));
 }
 
 // Whether an expert's tiles, which follow each other, are this one alone.
@@ -67,43 +108,56 @@ __device__ __forceinline__ bool one_tile(const int32_t* tile_expert, int tile, i
 // Stages of 64 deep go round a ring of LDS slots of 64 rows, 19 for two stages of 8 and the first three of a third: with two
 // stages alone a stage's loads started when the one before was released and either met all at once (64 bytes a cycle and CU)
 // or had too little time to land.
-// A workgroup per CU goes through its XCD's run of items (a tile and 256 weight rows): the next one's first stages are loaded
-// while the results leave, 16 rows at a time through a piece of LDS of the wave's own.
+// A workgroup per CU goes through its XCD's run of items (a tile and 256 weight rows). The ring does not stop between them: an
+// item's last two steps load the next one's first two stages, which land while the results leave, 16 rows at a time through a piece
+// of LDS of the wave's own. The next item's rows and weights of pairs go to LDS by direct loads, too, since a load into a register
+// would be waited for with everything under way. The first step of an item does not wait for the stores ahead of it, and starts the sums.
+// What is left over behind the whole rounds is cut into halves of the columns where there are workgroups for both (1500 x 2048,
+// 6144 gated: 288 items, 93 us in two whole rounds, 74 in one and a half). Cut by rows, both halves would read the weights.
 // A tile's rows are spread over the two rows of waves by sixteens, and products past its last 64 used rows are left out (700
 // pairs per expert: a sixth of the rows is padding). The depth is a multiple of 64, the columns of the item's.
 //   kGateUp, kDown  routed experts (moe.hip): rows by the pairs' order. kGateUp takes a row of x per token and leaves one per
 //                   place, silu(gate) up; kDown takes one per place and leaves one per pair, weighted.
 //   kGated          one matrix of N gate and N up rows, x and the output row by row, any activation (gated_product.hip).
-// Bound: the products; in the loop they run at 1.5 PFLOP/s over all CUs, the rate of a large product of the library, the clock
-// being at 1.75 to 1.9 GHz then. Measured, 64 experts of 768 x 2048, 8 per token, gate_up / down, us (before: eight waves, a
-// workgroup per tile and columns, two stages): 2048 tokens 153 / 85 (174 / 94), 5637 tokens 273 / 170 (305 / 189), 8192 tokens
-// 380 / 255 (434 / 275).
+// Bound: the products at the power limit (weights of zeros: 8192 x 2048, 6144 gated in 226 us, random ones in 297, 1.39 PFLOP/s, the
+// clock at 1.8 to 1.9 GHz); kDown: its loads, 12 stages an item and 128 KB of results. Measured, 64 experts of 768 x 2048, 8 per
+// token, gate_up / down, us (before: an item's loads start when the one before has left, addresses in the ring by compare and
+// select): 1000 tokens 96 / 53 (111 / 58), 1563 tokens 103 / 58 (119 / 65), 3000 tokens 154 / 98 (162 / 106), 5637 tokens 247 / 152
+// (265 / 166), 8192 tokens 356 / 230 (379 / 260); gated: 8192 x 2048, 6144 297 (321), 4000 x 2048, 6144 150 (161).
+// Where the loads of an item's last steps were cases in the loop's body, its branches took more than all this gave (324).
 // ONCE: weights of an expert with one tile go past the caches (non-temporal), those of an expert with several, which read them from
-// there, do not: 64 experts of 768 x 2048, both products, us (all cached / all past): 1563 tokens 185 (195 / 186), unevenly loaded 192
-// (196 / 202), 2048 tokens 260 (259 / 275). The loops for both are one inlined body each: as calls they kept their captures in scratch.
+// there, do not: both products, us (all cached / all past), before: 1563 tokens 185 (195 / 186), unevenly loaded 192 (196 / 202), 2048
+// tokens 260 (259 / 275). The loops for both are one inlined body each: as calls they kept their captures in scratch.
 template <int KIND, int ACT, bool ONCE>
 __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
     constexpr bool GATED = KIND != kDown, ROUTED = KIND != kGated, GATHER = KIND != kDown;
     const int ncols = p.N / (GATED ? 128 : 256);
-    constexpr int TM = 256, BK = 64, NT = 8, L = 8;       // results: NT 16-wide tiles of columns a wave; L loads each of x, w
-    constexpr int kSlot = 64 * BK, RING = 19;              // 64 rows; slots of a stage: four of x, four of w
-    constexpr int OC = GATED ? 128 : 256, WC = OC / 2;     // output columns, a wave's
-    constexpr int LR = WC / 8, SI = LR / 4, LO = WC + 8;   // lanes per row as it leaves, stores of 16 rows, row in LDS
-    constexpr int E1 = 3, E2 = 3, F3 = 5;                  // a stage's loads in the groups of products: early, from the release on
-    __shared__ __attribute__((aligned(16))) uint16_t smem[RING * kSlot];
-    uint16_t* const s_out = smem + 16 * kSlot;             // free between items, as the first stages go to slots 0 .. 13
-    static_assert(4 * 16 * LO <= 3 * kSlot && E1 + E2 == 6, "ring");
-    __shared__ int s_row[2][TM], s_rows[2][4];  // of the output, or -1; the last in use
-    __shared__ float s_wt[2][TM];
+    constexpr int TM = 256, BK = 64, L = 8;               // L loads each of x, w
+    // 64 rows, bytes. Slots of a stage: four of x, four of w, those ahead that are loaded ahead: weights that come from HBM, which
+    // have the longer way (1563 tokens 103 / 58 us, behind the rows 106 / 60), else the rows (5637 tokens 247 / 152, 250 / 153).
+    constexpr uint32_t SLOT = 64 * BK * 2, RING = 19;
+    constexpr bool WF = ONCE;
+    constexpr int OC = GATED ? 128 : 256;                  // output columns
+    constexpr int REST = 5;                                // of a stage's loads, the last ones
+    constexpr int kOut = 5;                                // of a stage's slots, the first where results pass through LDS
+    __shared__ __attribute__((aligned(16))) uint16_t smem[RING * SLOT / 2];
+    __shared__ int s_rows[2][4];  // of 64 rows each: the last in use; kAll: all are
+    constexpr uint32_t kAll = 1 << 16;
+    __shared__ int s_row[ROUTED ? 2 : 1][TM];        // the pairs of this item's and the next one's rows, or -1
+    __shared__ float s_wt[KIND == kDown ? 2 : 1][TM];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c = lane & 15, g = lane >> 4, wm = wave >> 1, wn = wave & 1;
-    const int ntiles = ROUTED ? p.tile_expert[p.ntiles] : p.ntiles;
+    const int ntiles = ROUTED ? uniform(p.tile_expert + p.ntiles) : p.ntiles;
     const int64_t items = (int64_t)ntiles * ncols;
-    const int xcd = blockIdx.x % 8, stride = gridDim.x / 8;
-    const int end = (int)(items * (xcd + 1) / 8);
-    int item = (int)(items * xcd / 8) + blockIdx.x / 8;
-    if (item >= end) return;
+    const int xcd = blockIdx.x % 8, stride = gridDim.x / 8, at = blockIdx.x / 8;
+    const int first = (int)(items * xcd / 8), left = (int)(items * (xcd + 1) / 8) - first, rounds = left / stride, over = left % stride;
+    const bool halve = 2 * over <= stride;
+    const int mine = rounds + (at < (halve ? 2 * over : over));  // items of this workgroup
+    if (mine == 0) return;
     const int nk = p.K / BK;
+    // The i-th of them, and whether it is one half of its columns or the other (1, 2).
+    auto nth = [&](int i) { return first + i * stride + (halve && i == rounds ? at / 2 : at); };
+    auto half_of = [&](int i) { return halve && i == rounds ? 1 + at % 2 : 0; };
 
     // An XCD's workgroups read few tiles' rows and few columns' weights at a time. Routed: a tile's columns follow each other
     // (an expert has about as many tiles as its weights have columns here). kGated: blocks of four tiles, column by column.
@@ -117,102 +171,153 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
             tile = 4 * block + in - col * high;
         }
     };
-    // the item after this one: its rows' pairs are read an item ahead
-    int next_e = 0, next_pair = 0, next_rows[L];
-    bool next_once = false, once = false;  // the item's
-    auto peek = [&](int it) __attribute__((always_inline)) {
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_void*)smem, rows_at = (uint32_t)(uintptr_t)(lds_void*)&s_rows[0][0],
+                   row_at = (uint32_t)(uintptr_t)(lds_void*)&s_row[0][0], wt_at = (uint32_t)(uintptr_t)(lds_void*)&s_wt[0][0];
+    // The item after this one: what it needs of its tile is on its way an item ahead.
+    int next_tile = 0, next_n0 = 0, next_half = 0, next_e = 0, e_before = 0, e_after = 0;
+    auto peek = [&](int i, int qn) __attribute__((always_inline)) {
+        int col;
+        place(nth(i), next_tile, col);
+        next_half = half_of(i);
+        next_n0 = col * OC;
         if constexpr (ROUTED) {
-            int tile, col;
-            place(it, tile, col);
-            const int32_t* order = p.order + (int64_t)tile * TM;
-            next_e = p.tile_expert[tile];
-            if constexpr (ONCE) next_once = one_tile(p.tile_expert, tile, p.ntiles, next_e);
-            next_pair = order[tid];
-            if constexpr (GATHER)
-#pragma unroll
-                for (int i = 0; i < L; ++i) next_rows[i] = order[i / 2 * 64 + wave * 16 + i % 2 * 8 + lane / 8];
+            __builtin_amdgcn_global_load_lds((gbl_void*)(p.order + ((int64_t)next_tile * TM + tid)), (lds_void*)&s_row[qn][wave * kWave], 4, 0, 0);
+            next_e = uniform(p.tile_expert + next_tile);
+            if constexpr (ONCE) {
+                e_before = next_tile > 0 ? uniform(p.tile_expert + next_tile - 1) : -1;
+                e_after = next_tile + 1 < p.ntiles ? uniform(p.tile_expert + next_tile + 1) : -1;
+            }
         }
     };
     // A slot is loaded by all waves, two pieces of 8 rows each. Global sources of this lane's 16 bytes: chunk (lane % 8) ^ (row
     // / 2 % 8), so that the 16 rows a matrix operand reads at a time lie in different banks. Rows of w follow each other.
     const int chunk[2] = {(lane % 8 ^ lane / 16) * 8, (lane % 8 ^ (lane / 16 + 4)) * 8};  // even, odd piece
     const uint16_t *xs[GATHER ? L : 2], *ws[2];
-    auto wrap = [](int slot) { return slot >= RING ? slot - RING : slot; };
-    auto fetch = [&](auto nt, int t, int base, int i) __attribute__((always_inline)) {  // load i of stage t (the last again past the end), whose first slot is base
-        uint16_t* dst = smem + wrap(base + i / 2) * kSlot + (wave * 2 + i % 2) * 512;
-        const int64_t k0 = min(t, nk - 1) * BK;
-        const int64_t row = (i % L) / 2 * 64 + (GATED && i >= L + L / 2 ? p.N - OC : 0);
-        const uint16_t* src = i >= L ? ws[i % 2] + (k0 + row * p.ldw) : GATHER ? xs[i % L] + k0 : xs[i % 2] + (k0 + row * p.ldx);
-        if (nt.value && i >= L) __builtin_amdgcn_global_load_lds((gbl_void*)src, (lds_void*)dst, 16, 0, 2);
-        else __builtin_amdgcn_global_load_lds((gbl_void*)src, (lds_void*)dst, 16, 0, 0);
+    int64_t wslot[4] = {};  // what a slot's rows of w are past the item's first; those of a half are the first slots'
+    auto wrap = [](uint32_t at) { return min(at, at - RING * SLOT); };  // of less than two rings
+    auto fetch = [&](auto nt, int k0, uint32_t base, int i) __attribute__((always_inline)) {  // load i at depth k0 of the stage at base
+        const bool is_w = (i < L) == WF;
+        const int u = i % L;
+        const uint16_t* src = is_w     ? ws[u % 2] + (k0 + wslot[u / 2])
+                              : GATHER ? xs[u] + k0
+                                       : xs[u % 2] + (k0 + u / 2 * 64 * p.ldx);
+        lds_void* dst = (lds_void*)(uintptr_t)(lds0 + wrap(base + i / 2 * SLOT + wave * (SLOT / 4)) + u % 2 * (SLOT / 8));
+        if (nt.value && is_w) __builtin_amdgcn_global_load_lds((gbl_void*)src, dst, 16, 0, 2);
+        else __builtin_amdgcn_global_load_lds((gbl_void*)src, dst, 16, 0, 0);
     };
-    int n0, q = 0;
-    const double per_row = KIND == kGateUp ? 1.0 / p.row_div : 0.0;
-    auto open = [&](int it) __attribute__((always_inline)) {  // start on the item that was peeked at
+    int n0 = 0, q = 0, tile = 0, half = 0;  // the item's
+    bool once = false;
+    // Turn to the item that was peeked at: from here on its stages are loaded. What is written to LDS and read of it is not the
+    // compiler's, which would wait for every load into LDS under way.
+    auto turn = [&](int qn) __attribute__((always_inline)) {
         const int r0 = wave * 16 + lane / 8;
-        int tile, nb;
-        place(it, tile, nb);
-        n0 = nb * OC;
+        uint32_t pair = 0, rows[L] = {};
+        if constexpr (ROUTED) lds_read(pair, row_at + (qn * TM + tid) * 4, 0);
+        if constexpr (KIND == kGateUp)
+#pragma unroll
+            for (int i = 0; i < L; ++i) lds_read(rows[i], row_at + (qn * TM + r0) * 4, (i / 2 * 64 + i % 2 * 8) * 4);
         const uint16_t* we = p.w + (ROUTED ? (int64_t)max(next_e, 0) * (GATED ? 2 : 1) * p.N * p.ldw : 0);
-        we += (n0 + r0) * p.ldw;
+        we += (next_n0 + r0) * p.ldw;
         ws[0] = we + chunk[0], ws[1] = we + 8 * p.ldw + chunk[1];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            wslot[j] = ((j * 64 ^ (next_half == 2 ? OC / 2 : 0)) + (GATED && j >= 2 ? p.N - OC : 0)) * p.ldw;
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        asm volatile("" : "+v"(pair));
         if constexpr (KIND == kGated) {
 #pragma unroll
             for (int i = 0; i < L; ++i)  // rows past the last: the last one, not stored
-                xs[i] = p.x + min(tile * TM + i / 2 * 64 + i % 2 * 8 + r0, p.n - 1) * p.ldx + chunk[i % 2];
+                xs[i] = p.x + min(next_tile * TM + i / 2 * 64 + i % 2 * 8 + r0, p.n - 1) * p.ldx + chunk[i % 2];
+            pair = next_tile * TM + tid < p.n ? 0 : -1;
         } else if constexpr (KIND == kGateUp) {
 #pragma unroll
             for (int i = 0; i < L; ++i) {
-                const int pair = max(next_rows[i], 0);  // places without a pair: row 0, not stored
-                const int d = (int)(pair * per_row), rest = pair - d * p.row_div;  // pair / row_div, one off at most
-                xs[i] = p.x + (d + (rest >= p.row_div) - (rest < 0)) * p.ldx + chunk[i % 2];
+                asm volatile("" : "+v"(rows[i]));
+                const uint32_t row = max((int)rows[i], 0);  // places without a pair: row 0, not stored
+                xs[i] = p.x + (p.row_div > 1 ? __umulhi(row, p.div_mul) >> p.div_shift : row) * p.ldx + chunk[i % 2];
             }
         } else {
-            const uint16_t* xt = p.x + (tile * TM + r0) * p.ldx;
+            const uint16_t* xt = p.x + (next_tile * TM + r0) * p.ldx;
             xs[0] = xt + chunk[0], xs[1] = xt + 8 * p.ldx + chunk[1];
+            if (p.weight) __builtin_amdgcn_global_load_lds((gbl_void*)(p.weight + max((int)pair, 0)), (lds_void*)&s_wt[qn][wave * kWave], 4, 0, 0);
+            else lds_write(wt_at + (qn * TM + tid) * 4, __float_as_uint(1.f));
         }
-        auto first = [&](auto nt) __attribute__((always_inline)) {
-#pragma unroll
-            for (int i = 0; i < 2 * L; ++i) fetch(nt, 0, 0, i);
-#pragma unroll
-            for (int i = 0; i < E1 + E2 + F3; ++i) fetch(nt, 1, 8, i);
-        };
-        once = next_once;
-        if (ONCE && once) first(std::true_type{});
-        else first(std::false_type{});
-        if constexpr (KIND == kGated) next_pair = tile * TM + tid < p.n ? tile * TM + tid : -1;
-        s_row[q][tid] = GATED && next_pair >= 0 ? tile * TM + tid : next_pair;
-        if constexpr (!GATED) s_wt[q][tid] = p.weight && next_pair >= 0 ? p.weight[next_pair] : 1.f;
-        const uint64_t in = __ballot(next_pair >= 0);
-        if (lane == 0) s_rows[q][wave] = in ? 64 * wave + 64 - __builtin_clzll(in) : 0;
+        const uint64_t in = __ballot((int)pair >= 0);
+        if (lane == 0)
+            lds_write(rows_at + (qn * 4 + wave) * 4, (uint32_t)(in ? 64 * wave + 64 - __builtin_clzll(in) : 0) | (~in ? 0u : kAll));
     };
-    const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_void*)smem;
+    auto turned = [&]() __attribute__((always_inline)) {  // the item's output and tile
+        tile = next_tile, half = next_half;
+        n0 = next_n0 + (half == 2 ? OC / 2 : 0);
+        once = ONCE && e_before != next_e && e_after != next_e;
+    };
+    const bool chain = nk > 2;  // an item's last steps load the next one's first stages
+    uint32_t b0 = 0;            // where the next stage starts in the ring
+    auto prime = [&](int i) __attribute__((always_inline)) {
+        peek(i, q);
+        wait_loads<0>();
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        turn(q);
+        turned();
+#pragma unroll
+        for (int i = 0; i < 2 * L; ++i) fetch(std::false_type{}, 0, b0, i);
+#pragma unroll
+        for (int i = 0; i < 2 * L; ++i) fetch(std::false_type{}, nk > 1 ? BK : 0, wrap(b0 + 8 * SLOT), i);
+        wait_loads<0>();
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
     uint32_t xat[2], wat[2];  // of the lane in a slot, by half of the depth
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
         wat[ks] = lds0 + c * BK * 2 + ((ks * 4 + g) ^ (c / 2)) * 16;
         xat[ks] = wat[ks] + wm * 16 * BK * 2;
     }
-    const int w0 = 4 + (GATED ? wn : 2 * wn), w1 = GATED ? w0 + 2 : w0 + 1;  // the wave's slots of w
-    const uint32_t oat = lds0 + (16 * kSlot + wave * 16 * LO) * 2;
+    bool whole = false;  // the last item had all rows: its stores are counted
 
     // A step's products in four groups: half of the depth ks, half h of the 2 MH tiles of rows that are in use.
-    auto run = [&](auto mh_, auto nt, bool more) __attribute__((always_inline)) {
-        constexpr int MH = mh_, M = MH * NT;
-        f32x4 acc[2 * MH][NT];
-#pragma unroll
-        for (int m = 0; m < 2 * MH; ++m)
-#pragma unroll
-            for (int n = 0; n < NT; ++n) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
-        s16x8 wf[2][NT], xf[2][MH];
-        // The operands' reads are not the compiler's: it would wait for every load into LDS under way before one. Their
-        // registers are tied past the wait that ends the group they are in.
-        auto read_w = [&](int base, int ks, int n) {
-            lds_read(wf[ks][n], wat[ks] + wrap(base + (n < NT / 2 ? w0 : w1)) * (kSlot * 2), n % (NT / 2) * 16 * BK * 2);
+    // HALF: of one half of the item's columns, a workgroup's last.
+    auto run = [&](auto mh_, auto half_, auto nt, int rows, bool all_rows, bool more) __attribute__((always_inline)) {
+        constexpr bool HALF = half_;
+        constexpr int MH = mh_, NT = HALF ? 4 : 8, M = MH * NT;     // NT 16-wide tiles of columns a wave
+        constexpr int WC = OC / (HALF ? 4 : 2);                   // output columns a wave
+        constexpr int LR = WC / 8, SI = LR / 4;                   // lanes per row as it leaves, stores of 16 rows
+        constexpr int LW = HALF ? L / 2 : L;                      // loads of w a stage
+        constexpr int E1 = HALF ? 2 : 3, E2 = E1, F3 = 5, F1 = LW + L - E1 - E2 - F3;  // a stage's loads in the groups of products:
+                                                                                        // early, from the release on, in the next step
+        static_assert(4 * 16 * WC * 2 <= 2 * SLOT && (HALF || F1 == REST), "ring");
+        const bool chained = !HALF && more && chain;
+        // load i of the run's: half of the columns is two slots' rows of w, with GATED the gate's and the other matrix' first
+        auto stage = [&](int k0, uint32_t base, int i) __attribute__((always_inline)) {
+            const int before = WF ? 0 : L, u = i - before;  // of w's loads
+            const bool is_w = u >= 0 && u < LW;
+            fetch(nt, k0, base, is_w ? before + (HALF && GATED && u >= 2 ? u + 2 : u) : WF ? i - LW + L : i);
         };
-        auto read_x = [&](int base, int ks, int h, int i) {
+        // the wave's slots of w and its rows in them
+        const uint32_t w0 = ((WF ? 0 : 4) + (GATED ? (HALF ? 0 : wn) : HALF ? wn : 2 * wn)) * SLOT, w1 = w0 + (GATED ? 2 : HALF ? 0 : 1) * SLOT;
+        constexpr int WT = GATED || !HALF ? NT / 2 : NT;          // tiles of a slot
+        const uint32_t wrow = GATED && HALF ? wn * 32 * BK * 2 : 0;
+        // Results pass through LDS, 16 rows of WC columns a wave, 16-byte chunks xor-swizzled by the row.
+        auto mix = [](int row) { return row / (16 / LR); };
+        uint32_t put_at[WC / 16], get_at[SI];
+#pragma unroll
+        for (int n = 0; n < WC / 16; ++n)
+            put_at[n] = (wave % 2 * 16 * WC + c * WC) * 2 + ((2 * n + g / 2) ^ mix(c)) * 16 + g % 2 * 8;
+#pragma unroll
+        for (int k = 0; k < SI; ++k) {
+            const int row = k * (64 / LR) + lane / LR;
+            get_at[k] = (wave % 2 * 16 * WC + row * WC) * 2 + ((lane % LR) ^ mix(row)) * 16;
+        }
+        f32x4 acc[2 * MH][NT];
+        s16x8 wf[2][NT], xf[2][MH];
+        // The operands' reads are not the compiler's either. Their registers are tied past the wait that ends the group they are in.
+        auto read_w = [&](uint32_t base, int ks, int n) {
+            lds_read(wf[ks][n], wat[ks] + wrow + wrap(base + (n < WT ? w0 : w1)), n % WT * 16 * BK * 2);
+        };
+        auto read_x = [&](uint32_t base, int ks, int h, int i) {
             const int m = h * MH + i;
-            lds_read(xf[h][i], xat[ks] + wrap(base + m / 2) * (kSlot * 2), m % 2 * 32 * BK * 2);
+            lds_read(xf[h][i], xat[ks] + wrap(base + ((WF ? 4 : 0) + m / 2) * SLOT), m % 2 * 32 * BK * 2);
         };
         auto landed = [&]() {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -225,12 +330,13 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
             }
         };
         // the products of (ks, h) with `jobs` calls of job spread between them
-        auto group = [&](auto ks_, auto h_, auto jobs_, auto job) __attribute__((always_inline)) {
+        auto group = [&](auto first, auto ks_, auto h_, auto jobs_, auto job) __attribute__((always_inline)) {
             constexpr int ks = ks_, h = h_, J = jobs_;
 #pragma unroll
             for (int i = 0; i < M; ++i) {
                 const int m = i / NT, n = i % NT;
-                product(acc[h * MH + m][n], wf[ks][n], xf[h][m]);
+                if constexpr (first.value) first_product(acc[h * MH + m][n], wf[ks][n], xf[h][m]);
+                else product(acc[h * MH + m][n], wf[ks][n], xf[h][m]);
 #pragma unroll
                 for (int j = 0; j < J; ++j)
                     if (j * M / J == i) job(j);
@@ -240,122 +346,179 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
         };
         using I0 = std::integral_constant<int, 0>;
         using I1 = std::integral_constant<int, 1>;
-#pragma unroll
-        for (int n = 0; n < NT; ++n) read_w(0, 0, n), read_w(0, 1, n);
-#pragma unroll
-        for (int i = 0; i < MH; ++i) read_x(0, 0, 0, i), read_x(0, 0, 1, i);
-        landed();
-        for (int t = 0, b0 = 0; t < nk; ++t) {
-            const int b1 = wrap(b0 + 8), b2 = wrap(b1 + 8);  // of the next stages
-            group(I0{}, I0{}, std::integral_constant<int, MH + 2 * L - E1 - E2 - F3>{}, [&](int j) {
+        using Later = std::false_type;
+        int k2 = 0;  // depth of the loads under way
+        // A step, whose loads are two stages ahead, at depth k; with `turning`, the next item's from here on.
+        auto step = [&](auto first, auto turning, int k) __attribute__((always_inline)) {
+            const uint32_t b1 = wrap(b0 + 8 * SLOT), b2 = wrap(b1 + 8 * SLOT);  // of the next stages
+            constexpr int G1 = first.value ? 0 : F1;        // the first step's stand ahead of the last item's stores
+            group(first, I0{}, I0{}, std::integral_constant<int, MH + G1>{}, [&](int j) {
                 if (j < MH) read_x(b0, 0, 1, j);
-                else fetch(nt, t + 1, b1, E1 + E2 + F3 + j - MH);
+                else stage(k2, b1, E1 + E2 + F3 + j - MH);
             });
-            group(I0{}, I1{}, std::integral_constant<int, NT + MH + E1>{}, [&](int j) {
+            k2 = k;
+            if constexpr (turning.value)
+                if (chained) turn(q ^ 1);
+            group(first, I0{}, I1{}, std::integral_constant<int, NT + MH + E1>{}, [&](int j) {
                 if (j < NT) read_w(b0, 1, j);
                 else if (j < NT + MH) read_x(b0, 1, 0, j - NT);
-                else fetch(nt, t + 2, b2, j - NT - MH);
+                else stage(k2, b2, j - NT - MH);
             });
-            group(I1{}, I0{}, std::integral_constant<int, MH + E2>{}, [&](int j) {
+            group(Later{}, I1{}, I0{}, std::integral_constant<int, MH + E2>{}, [&](int j) {
                 if (j < MH) read_x(b0, 1, 1, j);
-                else fetch(nt, t + 2, b2, E1 + j - MH);
+                else stage(k2, b2, E1 + j - MH);
             });
-            wait_loads<E1 + E2>();         // this wave's loads of stage t + 1 have landed, its reads of stage t too
+            // this wave's loads of stage t + 1 have landed, its reads of stage t too
+            if (first.value && whole) wait_loads<E1 + E2 + OC / 8>();
+            else wait_loads<E1 + E2>();
             __builtin_amdgcn_s_barrier();  // and everyone's
             asm volatile("" ::: "memory");
-            group(I1{}, I1{}, std::integral_constant<int, NT + MH + F3>{}, [&](int j) {
+            group(Later{}, I1{}, I1{}, std::integral_constant<int, NT + MH + F3>{}, [&](int j) {
                 if (j < NT) read_w(b1, 0, j);
                 else if (j < NT + MH) read_x(b1, 0, 0, j - NT);
-                else fetch(nt, t + 2, b2, E1 + E2 + j - NT - MH);
+                else stage(k2, b2, E1 + E2 + j - NT - MH);
             });
             b0 = b1;
+        };
+#pragma unroll
+        for (int n = 0; n < NT; ++n) read_w(b0, 0, n);
+#pragma unroll
+        for (int i = 0; i < MH; ++i) read_x(b0, 0, 0, i);
+        landed();
+        // Past the item's last stage the loads are the next item's, or the last stage's again. The steps around that are copies of
+        // their own: as cases of the loop's body they cost it 7 %.
+        const int last = (nk - 1) * BK;
+        step(std::true_type{}, Later{}, min(2 * BK, last));
+        if constexpr (HALF) {
+            for (int t = 1; t < nk; ++t) step(Later{}, Later{}, min((t + 2) * BK, last));
+        } else {
+            for (int t = 1; t < nk - 2; ++t) step(Later{}, Later{}, (t + 2) * BK);
+            if (nk > 2) step(Later{}, std::true_type{}, chained ? 0 : last);
+            if (nk > 1) step(Later{}, Later{}, chained ? BK : last);
+            if (chained)
+#pragma unroll
+                for (int i = 2 * L - REST; i < 2 * L; ++i) fetch(nt, k2, wrap(b0 + 8 * SLOT), i);  // what remains of the next item's
         }
-        wait_loads<0>();
-        asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last products are in their registers
-        __syncthreads();
-        const int o = q;
-        uint16_t* to = p.out + n0 + wn * WC + lane % LR * 8;
-        float scale[2 * MH];
+        uint16_t* const to = p.out + n0 + wn * WC + lane % LR * 8;
+        const int own = tile * TM;
+        // The last products are in their registers 16 cycles on. The item's last stage is read: two of its slots, the ones that
+        // nothing is loaded into before the next barrier, are the results' way.
+        uint32_t scale[2 * MH];
+        if constexpr (!GATED) {
+#pragma unroll
+            for (int m = 0; m < 2 * MH; ++m) lds_read(scale[m], wt_at + q * TM * 4 + (wm * 16 + c) * 4, m * 128);
+        }
+        if (chained) turned();
+        asm volatile("s_nop 15\n\ts_nop 15\n\ts_waitcnt lgkmcnt(0)" ::: "memory");
         if constexpr (!GATED)
 #pragma unroll
-            for (int m = 0; m < 2 * MH; ++m) scale[m] = s_wt[o][(2 * m + wm) * 16 + c];
-        if (more) {
-            q ^= 1;
-            open(item + stride);
-        }
-        uint4 v[2][SI];
-        auto gather = [&](int m, uint4 (&y)[SI]) __attribute__((always_inline)) {
+            for (int m = 0; m < 2 * MH; ++m) asm volatile("" : "+v"(scale[m]));
+        const uint32_t out_at = lds0 + wrap(wrap(b0 + (RING - 8) * SLOT) + (kOut + wave / 2) * SLOT);
+        auto put = [&](int m) __attribute__((always_inline)) {
 #pragma unroll
             for (int n = 0; n < NT; ++n) asm volatile("" : "+a"(acc[m][n]));  // in the accumulators' registers until here
 #pragma unroll
-            for (int n = 0; n < (GATED ? NT / 2 : NT); ++n) {
+            for (int n = 0; n < WC / 16; ++n) {
                 float z[4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     if constexpr (GATED) z[i] = gated16<ACT>(acc[m][n][i], acc[m][n + NT / 2][i], p.gate);
-                    else z[i] = acc[m][n][i] * scale[m];
+                    else z[i] = acc[m][n][i] * __uint_as_float(scale[m]);
                 }
-                *reinterpret_cast<uint2*>(&s_out[wave * 16 * LO + c * LO + n * 16 + 4 * g]) =
-                    make_uint2(pack_bf16x2(z[0], z[1]), pack_bf16x2(z[2], z[3]));
+                lds_write(out_at + put_at[n], make_uint2(pack_bf16x2(z[0], z[1]), pack_bf16x2(z[2], z[3])));
             }
-            asm volatile("" ::: "memory");
-            s16x8 b[SI];
-#pragma unroll
-            for (int k = 0; k < SI; ++k) lds_read(b[k], oat + (lane / LR * LO + lane % LR * 8) * 2, k * (64 / LR) * LO * 2);
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        };
+        s16x8 y[2][SI];
+        uint32_t row[2][SI];
+        // A wave's LDS accesses are in order: the reads of 16 rows follow their writes and go ahead of the next ones'.
+        auto get = [&](int m) __attribute__((always_inline)) {
 #pragma unroll
             for (int k = 0; k < SI; ++k) {
-                asm volatile("" : "+v"(b[k]));
-                y[k] = *reinterpret_cast<const uint4*>(&b[k]);
+                if constexpr (KIND == kDown)
+                    lds_read(row[m & 1][k], row_at + q * TM * 4 + (wm * 16 + lane / LR) * 4, (m * 32 + k * (64 / LR)) * 4);
+                lds_read(y[m & 1][k], out_at + get_at[k], 0);
             }
         };
-        auto leave = [&](int m, const uint4 (&y)[SI]) __attribute__((always_inline)) {
-            int row[SI];
+        auto leave = [&](int m) __attribute__((always_inline)) {
 #pragma unroll
-            for (int k = 0; k < SI; ++k) row[k] = s_row[o][(2 * m + wm) * 16 + k * (64 / LR) + lane / LR];
-#pragma unroll
-            for (int k = 0; k < SI; ++k)
-                if (row[k] >= 0) *reinterpret_cast<uint4*>(to + (int64_t)row[k] * p.N) = y[k];
+            for (int k = 0; k < SI; ++k) {
+                asm volatile("" : "+v"(y[m & 1][k]));
+                int64_t to_row;
+                int on;
+                if constexpr (KIND == kDown) {
+                    asm volatile("" : "+v"(row[m & 1][k]));
+                    on = (int)row[m & 1][k];
+                    to_row = row[m & 1][k];
+                } else {
+                    const int r = (2 * m + wm) * 16 + k * (64 / LR) + lane / LR;
+                    on = rows - 1 - r;
+                    to_row = own + r;
+                }
+                store_row(to + to_row * p.N, y[m & 1][k], on);
+            }
         };
-        gather(0, v[0]);
-        gather(1, v[1]);
-        wait_loads<0>();  // the next item's first stages, before stores are under way too
-        leave(0, v[0]);
-        leave(1, v[1]);
+        put(0);
+        get(0);
 #pragma unroll
-        for (int m = 2; m < 2 * MH; ++m) {
-            gather(m, v[m & 1]);
-            leave(m, v[m & 1]);
+        for (int m = 0; m < 2 * MH; ++m) {
+            if (m + 1 < 2 * MH) {
+                put(m + 1);
+                asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(WC / 16) : "memory");
+                get(m + 1);
+            } else {
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            }
+            leave(m);
         }
+        whole = MH == 4 && all_rows && nk > 3;  // with fewer stages the next item's rows are needed right behind the first step
     };
-    peek(item);
-    open(item);
-    wait_loads<0>();
-    for (; item < end; item += stride) {
-        __syncthreads();
-        const int* sr = s_rows[q];
-        const int rows = max(max(sr[0], sr[1]), max(sr[2], sr[3]));
-        const bool more = item + stride < end;
-        if (more) peek(item + stride);
-        auto all = [&](auto nt) __attribute__((always_inline)) {
-            if (rows > 192) run(std::integral_constant<int, 4>{}, nt, more);
-            else if (rows > 128) run(std::integral_constant<int, 3>{}, nt, more);
-            else if (rows > 64) run(std::integral_constant<int, 2>{}, nt, more);
-            else run(std::integral_constant<int, 1>{}, nt, more);
+    prime(0);
+    for (int i = 0;; ++i) {
+        uint32_t r4[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) lds_read(r4[j], rows_at + q * 16, j * 4);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int j = 0; j < 4; ++j) asm volatile("" : "+v"(r4[j]));
+        int rows = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) rows = max(rows, (int)(r4[j] & (kAll - 1)));
+        rows = __builtin_amdgcn_readfirstlane(rows);
+        const bool all_rows = __builtin_amdgcn_readfirstlane(r4[0] & r4[1] & r4[2] & r4[3]) & kAll, more = i + 1 < mine;
+        if (more && chain) peek(i + 1, q ^ 1);
+        auto all = [&](auto half_, auto nt) __attribute__((always_inline)) {
+            if (rows > 192) run(std::integral_constant<int, 4>{}, half_, nt, rows, all_rows, more);
+            else if (rows > 128) run(std::integral_constant<int, 3>{}, half_, nt, rows, all_rows, more);
+            else if (rows > 64) run(std::integral_constant<int, 2>{}, half_, nt, rows, all_rows, more);
+            else run(std::integral_constant<int, 1>{}, half_, nt, rows, all_rows, more);
         };
-        if (ONCE && once) all(std::bool_constant<ONCE>{});
-        else all(std::false_type{});
+        if (half) {
+            if (ONCE && once) all(std::true_type{}, std::bool_constant<ONCE>{});
+            else all(std::true_type{}, std::false_type{});
+        } else {
+            if (ONCE && once) all(std::false_type{}, std::bool_constant<ONCE>{});
+            else all(std::false_type{}, std::false_type{});
+        }
+        if (!more) break;
+        q ^= 1;
+        __builtin_amdgcn_s_barrier();  // everyone's results have left LDS
+        asm volatile("" ::: "memory");
+        if (!chain) {
+            wait_loads<0>();
+            prime(i + 1);
+        }
     }
+    wait_loads<0>();  // into LDS that is another workgroup's next
 }
 
-// Items one each for up to three rounds of workgroups, which then go to the CUs as these get free; with more, a workgroup per
-// CU (gate_up as above, 2048 tokens: 161 us against 171; 8192: 395 against 380).
+// A workgroup per CU, or two for every item where these are fewer (each a half of its columns).
 inline bool wide_fits(int K, int N, bool gated) { return K > 0 && K % 64 == 0 && N % (gated ? 128 : 256) == 0; }
 template <int KIND, int ACT = SKYRL_ACT_SILU, bool ONCE = false>
-int launch_wide(const Wide& p, hipStream_t s) {
+int launch_wide(Wide p, hipStream_t s) {
+    set_division(p);
     const int64_t items = (int64_t)(p.N / (KIND == kDown ? 256 : 128)) * p.ntiles;
     SKYRL_REQUIRE(items < (1ll << 31) && p.ntiles < (1 << 23), "wide products: too many rows in one call");
-    const unsigned grid = (unsigned)(items > 3 * kCUs ? kCUs : (items + 7) / 8 * 8);
+    const unsigned grid = (unsigned)(items > kCUs / 2 ? kCUs : (2 * items + 7) / 8 * 8);
     hipLaunchKernelGGL((wide_kernel<KIND, ACT, ONCE>), dim3(grid), dim3(256), 0, s, p);
     return check_launch("wide_kernel");
 }

@@ -506,6 +506,22 @@ def test_wide_tiles_agree_on_both_sides_of_a_tile_an_expert(n):
     assert torch.equal(wide, staged)
 
 
+@pytest.mark.parametrize("width,ff,experts,n", [(256, 128, 300, 9000), (512, 192, 250, 4000), (768, 384, 110, 9000), (512, 640, 64, 9000)])
+def test_wide_tiles_in_rounds(width, ff, experts, n):
+    """Several items a workgroup, whole ones and halves, tiles of all heights behind each other, depths of two stages (each item on its
+    own), three and more: the rows that tiles of 64 give, every time."""
+    g = torch.Generator(device=DEV).manual_seed(n + ff)
+    sh = lk.moe_shape(width, ff, experts, 1)
+    mk = lambda *s, scale=1.0: (torch.randn(s, generator=g, device=DEV) * scale).to(BF16)  # noqa: E731
+    x, wgu, wd = mk(n, width), mk(experts, 2, ff, width, scale=0.05), mk(experts, width, ff, scale=0.05)
+    loads = torch.rand(experts, generator=g, device=DEV) ** 3 + 1e-3
+    idx = torch.multinomial(loads, n, replacement=True, generator=g).int().view(n, 1)
+    weight = torch.rand(n, 1, generator=g, device=DEV) + 0.2
+    want = lk.moe_experts(sh, x, idx, weight, wgu, wd, tm=64)
+    for _ in range(3):
+        assert torch.equal(lk.moe_experts(sh, x, idx, weight, wgu, wd, tm=256), want)
+
+
 @pytest.mark.parametrize("n", (64, 200, 700))
 def test_experts_with_one_tile_beside_such_with_several(n):
     """Matrices of 67 and 34 MB, whose weights go past the caches where an expert has one tile: loads from nothing to all tokens an

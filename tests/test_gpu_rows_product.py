@@ -64,6 +64,12 @@ def test_gated(dev, n, N, K, act):
     assert bool(((y.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2 * slack + 1e-5 * (g * u).abs() + 1e-6).all())
 
 
+@pytest.mark.parametrize("n,N,K", [(2113, 4096, 64), (2300, 6400, 128), (2113, 4096, 192), (2300, 6400, 256), (4161, 3968, 320)])
+def test_gated_in_rounds(dev, n, N, K):
+    """One to five stages an item, a second round of whole items and one of halves, a last tile of 65, 252 and 65 rows."""
+    test_gated(dev, n, N, K, "silu")
+
+
 def test_what_the_library_takes(dev):
     x, w, _ = _data(dev, 129, 64, 64, 0)
     assert not lk._rows_fit(x, w)                                  # too many rows
