@@ -67,6 +67,9 @@ extern "C" {
  *                   [N gate rows, N up rows] (row stride ldw), rows 16-byte aligned, as bf16 [n, N] contiguous: summed and
  *                   gated in f32, rounded once. K a multiple of 64, N of 128. skyrl_gated_product_fits: whether it takes the
  *                   sizes and is the faster form.
+ *   skyrl_dense_product  many rows: x w^T of x bf16 [n, K] (row stride ldx) and w bf16 [N, K] (row stride ldw), rows 16-byte
+ *                   aligned, operands of less than 4 GB, as bf16 [n, N] contiguous: summed in f32 along the depth, rounded
+ *                   once. K a multiple of 64, N of 8. skyrl_dense_product_fits: whether it takes the sizes and is the faster form.
  *   skyrl_rows_batch  `batch` such products without bias, x, w and out bf16 x_batch, w_batch and out_batch apart.
  *                   skyrl_rows_batch_in_order: each sum in the order of the depth, not in shares of it.
  *   skyrl_add_norm_parts, skyrl_gate_norm_add_parts  of a model in bf16, the sublayer's output being such a sum of
@@ -97,6 +100,9 @@ int skyrl_gate_norm_add(const void* a, const int64_t* rows, int32_t parts, const
 int32_t skyrl_gated_product_fits(int32_t n, int32_t K, int32_t N);
 int skyrl_gated_product(const void* x, int64_t ldx, int32_t n, int32_t K, const void* w, int64_t ldw, int32_t N, int32_t act,
                         float alpha, float limit, void* out, void* stream);
+int32_t skyrl_dense_product_fits(int32_t n, int32_t K, int32_t N);
+int skyrl_dense_product(const void* x, int64_t ldx, int32_t n, int32_t K, const void* w, int64_t ldw, int32_t N, void* out,
+                        void* stream);
 int32_t skyrl_rows_product_fits(int32_t n, int32_t K, int32_t N, int32_t form);
 int32_t skyrl_rows_product_splits(int32_t n, int32_t K, int32_t N);
 int skyrl_rows_product(const void* x, int64_t ldx, int32_t n, int32_t K, const void* w, int64_t ldw, int32_t N,

@@ -296,6 +296,8 @@ LAYERS_SIGNATURES = {
     "skyrl_conv_save": (_INT, [_P, _I64, _I32, _I32, _P, _P, _P, _I32, _P, _I32, _P]),
     "skyrl_softcap": (_INT, [_P, _P, _I64, _F, _I32, _P]),
     "skyrl_gate_norm_add": (_INT, [_P, _P, _I32, _P, _I64, _P, _P, _I32, _F, _F, _P, _I32, _P, _I32, _I32, _P, _I32, _P]),
+    "skyrl_dense_product_fits": (_I32, [_I32, _I32, _I32]),
+    "skyrl_dense_product": (_INT, [_P, _I64, _I32, _I32, _P, _I64, _I32, _P, _P]),
     "skyrl_gated_product_fits": (_I32, [_I32, _I32, _I32]),
     "skyrl_gated_product": (_INT, [_P, _I64, _I32, _I32, _P, _I64, _I32, _I32, _F, _F, _P, _P]),
     "skyrl_rows_product_fits": (_I32, [_I32, _I32, _I32, _I32]),

@@ -19,7 +19,7 @@ extern "C" int skyrl_gated_product(const void* x, int64_t ldx, int32_t n, int32_
     SKYRL_REQUIRE(aligned16(x) && aligned16(w) && aligned16(out) && ldx % 8 == 0 && ldw % 8 == 0 && ldw >= K && (n == 1 || ldx >= K),
                   "gated_product: rows must be 16-byte aligned");
     const Wide p{reinterpret_cast<const uint16_t*>(x), reinterpret_cast<const uint16_t*>(w), reinterpret_cast<uint16_t*>(out), K, N,
-                 ldx, ldw, (n + 255) / 256, nullptr, nullptr, 1, 0, 0, nullptr, n, Gate{act, alpha, limit}};
+                 ldx, ldw, (n + 255) / 256, nullptr, nullptr, 1, 0, 0, nullptr, n, 256, Gate{act, alpha, limit}};
     if (act == SKYRL_ACT_SILU) return launch_wide<kGated, SKYRL_ACT_SILU>(p, as_stream(stream));
     if (act == SKYRL_ACT_CLAMPED) return launch_wide<kGated, SKYRL_ACT_CLAMPED>(p, as_stream(stream));
     return launch_wide<kGated, SKYRL_ACT_GELU_TANH>(p, as_stream(stream));

@@ -661,7 +661,7 @@ int launch_product(Product p, const void* x, const void* w, void* out, int ntile
         p.past = (int64_t)experts * (GATED ? 4 : 2) * p.N * p.K >= kPast;
         if (p.tm == 256 && wide_fits(p.K, p.N, GATED)) {
             constexpr int kind = GATED ? kGateUp : kDown;
-            const Wide wide{x_, w_, o_, p.K, p.N, p.K, p.K, ntiles, p.order, p.tile_expert, p.row_div, 0, 0, p.weight, 0, Gate{}};
+            const Wide wide{x_, w_, o_, p.K, p.N, p.K, p.K, ntiles, p.order, p.tile_expert, p.row_div, 0, 0, p.weight, 0, 0, Gate{}};
             return once && p.past ? launch_wide<kind, SKYRL_ACT_SILU, true>(wide, s) : launch_wide<kind>(wide, s);
         }
         if (p.tm == 256) LAUNCH_GEMM(256, 256, 2, 4, 2);

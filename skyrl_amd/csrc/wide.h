@@ -24,6 +24,14 @@ __device__ __forceinline__ void lds_write(uint32_t at, uint32_t v) {
 __device__ __forceinline__ void lds_write(uint32_t at, uint2 v) {
     asm volatile("ds_write_b64 %0, %1" ::"v"(at), "v"(v) : "memory");
 }
+// 16 bytes a lane into LDS from `offset` bytes past what `all` begins with and the lane's own. Operands of less than 4 GB: a uniform
+// step of the depth costs no vector instruction, and an address one register.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t whole_buffer(const void* p) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, 0xffffffff, 0x00027000);
+}
+__device__ __forceinline__ void buffer_to_lds(__amdgpu_buffer_rsrc_t all, uint32_t own, int offset, uint32_t to) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(all, (lds_void*)(uintptr_t)to, 16, own, offset, 0, 0);
+}
 // 16 bytes from the lanes whose row is not negative, without a way round the store.
 __device__ __forceinline__ void store_row(uint16_t* to, s16x8 v, int row) {
     uint64_t all;
@@ -54,7 +62,7 @@ __device__ __forceinline__ float gated16(float g, float u, const Gate& f) {
     return gelu_tanh_<uint16_t>(g) * u;
 }
 
-enum WideKind { kGateUp, kDown, kGated };
+enum WideKind { kGateUp, kDown, kGated, kDense };
 constexpr int kCUs = 256;  // a multiple of the 8 XCDs
 struct Wide {
     const uint16_t *x, *w;
@@ -68,8 +76,8 @@ struct Wide {
     uint32_t div_mul;
     int div_shift;
     const float* weight;  // kDown: of the pair, NULL: 1
-    // kGated
-    int n;
+    // kGated, kDense
+    int n, tile_rows;  // rows of a tile: 64 to 256 by 64
     Gate gate;
 };
 
@@ -118,7 +126,8 @@ __device__ __forceinline__ bool one_tile(const int32_t* tile_expert, int tile, i
 // pairs per expert: a sixth of the rows is padding). The depth is a multiple of 64, the columns of the item's.
 //   kGateUp, kDown  routed experts (moe.hip): rows by the pairs' order. kGateUp takes a row of x per token and leaves one per
 //                   place, silu(gate) up; kDown takes one per place and leaves one per pair, weighted.
-//   kGated          one matrix of N gate and N up rows, x and the output row by row, any activation (gated_product.hip).
+//   kGated, kDense  one matrix, x and the output row by row in tiles of tile_rows (gated_product.hip): of N gate and N up rows,
+//                   any activation; of N rows, a multiple of 8, as they are.
 // Bound: the products at the power limit (weights of zeros: 8192 x 2048, 6144 gated in 226 us, random ones in 297, 1.39 PFLOP/s, the
 // clock at 1.8 to 1.9 GHz); kDown: its loads, 12 stages an item and 128 KB of results. Measured, 64 experts of 768 x 2048, 8 per
 // token, gate_up / down, us (before: an item's loads start when the one before has left, addresses in the ring by compare and
@@ -130,8 +139,8 @@ __device__ __forceinline__ bool one_tile(const int32_t* tile_expert, int tile, i
 // tokens 260 (259 / 275). The loops for both are one inlined body each: as calls they kept their captures in scratch.
 template <int KIND, int ACT, bool ONCE>
 __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
-    constexpr bool GATED = KIND != kDown, ROUTED = KIND != kGated, GATHER = KIND != kDown;
-    const int ncols = p.N / (GATED ? 128 : 256);
+    constexpr bool GATED = KIND == kGateUp || KIND == kGated, ROUTED = KIND == kGateUp || KIND == kDown, GATHER = KIND != kDown;
+    const int ncols = KIND == kDense ? (p.N + 255) / 256 : p.N / (GATED ? 128 : 256);
     constexpr int TM = 256, BK = 64, L = 8;               // L loads each of x, w
     // 64 rows, bytes. Slots of a stage: four of x, four of w, those ahead that are loaded ahead: weights that come from HBM, which
     // have the longer way (1563 tokens 103 / 58 us, behind the rows 106 / 60), else the rows (5637 tokens 247 / 152, 250 / 153).
@@ -193,17 +202,22 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
     // / 2 % 8), so that the 16 rows a matrix operand reads at a time lie in different banks. Rows of w follow each other.
     const int chunk[2] = {(lane % 8 ^ lane / 16) * 8, (lane % 8 ^ (lane / 16 + 4)) * 8};  // even, odd piece
     const uint16_t *xs[GATHER ? L : 2], *ws[2];
+    uint32_t xo[L] = {}, wo[L] = {};  // kDense: in bytes from the first row
+    const __amdgpu_buffer_rsrc_t x_all = whole_buffer(p.x), w_all = whole_buffer(p.w);
     int64_t wslot[4] = {};  // what a slot's rows of w are past the item's first; those of a half are the first slots'
     auto wrap = [](uint32_t at) { return min(at, at - RING * SLOT); };  // of less than two rings
     auto fetch = [&](auto nt, int k0, uint32_t base, int i) __attribute__((always_inline)) {  // load i at depth k0 of the stage at base
         const bool is_w = (i < L) == WF;
         const int u = i % L;
-        const uint16_t* src = is_w     ? ws[u % 2] + (k0 + wslot[u / 2])
-                              : GATHER ? xs[u] + k0
-                                       : xs[u % 2] + (k0 + u / 2 * 64 * p.ldx);
-        lds_void* dst = (lds_void*)(uintptr_t)(lds0 + wrap(base + i / 2 * SLOT + wave * (SLOT / 4)) + u % 2 * (SLOT / 8));
-        if (nt.value && is_w) __builtin_amdgcn_global_load_lds((gbl_void*)src, dst, 16, 0, 2);
-        else __builtin_amdgcn_global_load_lds((gbl_void*)src, dst, 16, 0, 0);
+        const uint32_t to = lds0 + wrap(base + i / 2 * SLOT + wave * (SLOT / 4)) + u % 2 * (SLOT / 8);
+        lds_void* dst = (lds_void*)(uintptr_t)to;
+        if constexpr (KIND == kDense) {
+            buffer_to_lds(is_w ? w_all : x_all, is_w ? wo[u] : xo[u], k0 * 2, to);
+        } else {
+            const uint16_t* src = is_w ? ws[u % 2] + (k0 + wslot[u / 2]) : GATHER ? xs[u] + k0 : xs[u % 2] + (k0 + u / 2 * 64 * p.ldx);
+            if (nt.value && is_w) __builtin_amdgcn_global_load_lds((gbl_void*)src, dst, 16, 0, 2);
+            else __builtin_amdgcn_global_load_lds((gbl_void*)src, dst, 16, 0, 0);
+        }
     };
     int n0 = 0, q = 0, tile = 0, half = 0;  // the item's
     bool once = false;
@@ -216,19 +230,29 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
         if constexpr (KIND == kGateUp)
 #pragma unroll
             for (int i = 0; i < L; ++i) lds_read(rows[i], row_at + (qn * TM + r0) * 4, (i / 2 * 64 + i % 2 * 8) * 4);
-        const uint16_t* we = p.w + (ROUTED ? (int64_t)max(next_e, 0) * (GATED ? 2 : 1) * p.N * p.ldw : 0);
-        we += (next_n0 + r0) * p.ldw;
-        ws[0] = we + chunk[0], ws[1] = we + 8 * p.ldw + chunk[1];
+        const int flip = next_half == 2 ? OC / 2 : 0;
+        if constexpr (KIND == kDense) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-            wslot[j] = ((j * 64 ^ (next_half == 2 ? OC / 2 : 0)) + (GATED && j >= 2 ? p.N - OC : 0)) * p.ldw;
+            for (int i = 0; i < L; ++i)  // rows past the last: the last one, its columns not stored
+                wo[i] = (min(next_n0 + (i / 2 * 64 ^ flip) + i % 2 * 8 + r0, p.N - 1) * (uint32_t)p.ldw + chunk[i % 2]) * 2;
+        } else {
+            const uint16_t* we = p.w + (ROUTED ? (int64_t)max(next_e, 0) * (GATED ? 2 : 1) * p.N * p.ldw : 0);
+            we += (next_n0 + r0) * p.ldw;
+            ws[0] = we + chunk[0], ws[1] = we + 8 * p.ldw + chunk[1];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) wslot[j] = ((j * 64 ^ flip) + (GATED && j >= 2 ? p.N - OC : 0)) * p.ldw;
+        }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         asm volatile("" : "+v"(pair));
-        if constexpr (KIND == kGated) {
+        if constexpr (!ROUTED) {
+            const int row0 = next_tile * p.tile_rows;
 #pragma unroll
-            for (int i = 0; i < L; ++i)  // rows past the last: the last one, not stored
-                xs[i] = p.x + min(next_tile * TM + i / 2 * 64 + i % 2 * 8 + r0, p.n - 1) * p.ldx + chunk[i % 2];
-            pair = next_tile * TM + tid < p.n ? 0 : -1;
+            for (int i = 0; i < L; ++i) {  // rows past the last: the last one, not stored
+                const int row = min(row0 + i / 2 * 64 + i % 2 * 8 + r0, p.n - 1);
+                if constexpr (KIND == kDense) xo[i] = (row * (uint32_t)p.ldx + chunk[i % 2]) * 2;
+                else xs[i] = p.x + row * p.ldx + chunk[i % 2];
+            }
+            pair = tid < p.tile_rows && row0 + tid < p.n ? 0 : -1;
         } else if constexpr (KIND == kGateUp) {
 #pragma unroll
             for (int i = 0; i < L; ++i) {
@@ -300,15 +324,6 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
         const uint32_t wrow = GATED && HALF ? wn * 32 * BK * 2 : 0;
         // Results pass through LDS, 16 rows of WC columns a wave, 16-byte chunks xor-swizzled by the row.
         auto mix = [](int row) { return row / (16 / LR); };
-        uint32_t put_at[WC / 16], get_at[SI];
-#pragma unroll
-        for (int n = 0; n < WC / 16; ++n)
-            put_at[n] = (wave % 2 * 16 * WC + c * WC) * 2 + ((2 * n + g / 2) ^ mix(c)) * 16 + g % 2 * 8;
-#pragma unroll
-        for (int k = 0; k < SI; ++k) {
-            const int row = k * (64 / LR) + lane / LR;
-            get_at[k] = (wave % 2 * 16 * WC + row * WC) * 2 + ((lane % LR) ^ mix(row)) * 16;
-        }
         f32x4 acc[2 * MH][NT];
         s16x8 wf[2][NT], xf[2][MH];
         // The operands' reads are not the compiler's either. Their registers are tied past the wait that ends the group they are in.
@@ -400,20 +415,32 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
                 for (int i = 2 * L - REST; i < 2 * L; ++i) fetch(nt, k2, wrap(b0 + 8 * SLOT), i);  // what remains of the next item's
         }
         uint16_t* const to = p.out + n0 + wn * WC + lane % LR * 8;
-        const int own = tile * TM;
+        const int own = tile * (ROUTED ? TM : p.tile_rows);
+        const bool in = KIND != kDense || n0 + wn * WC + lane % LR * 8 < p.N;  // this lane's columns
         // The last products are in their registers 16 cycles on. The item's last stage is read: two of its slots, the ones that
         // nothing is loaded into before the next barrier, are the results' way.
         uint32_t scale[2 * MH];
-        if constexpr (!GATED) {
+        if constexpr (KIND == kDown) {
 #pragma unroll
             for (int m = 0; m < 2 * MH; ++m) lds_read(scale[m], wt_at + q * TM * 4 + (wm * 16 + c) * 4, m * 128);
         }
         if (chained) turned();
         asm volatile("s_nop 15\n\ts_nop 15\n\ts_waitcnt lgkmcnt(0)" ::: "memory");
-        if constexpr (!GATED)
+        if constexpr (KIND == kDown)
 #pragma unroll
             for (int m = 0; m < 2 * MH; ++m) asm volatile("" : "+v"(scale[m]));
         const uint32_t out_at = lds0 + wrap(wrap(b0 + (RING - 8) * SLOT) + (kOut + wave / 2) * SLOT);
+        uint32_t put_at[WC / 16], get_at[SI];
+        int l = lane;
+        asm volatile("" : "+v"(l));  // formed here: as values of the whole launch they were put out to memory
+#pragma unroll
+        for (int n = 0; n < WC / 16; ++n)
+            put_at[n] = out_at + (wave % 2 * 16 * WC + l % 16 * WC) * 2 + ((2 * n + l / 32) ^ mix(l % 16)) * 16 + l / 16 % 2 * 8;
+#pragma unroll
+        for (int k = 0; k < SI; ++k) {
+            const int row = k * (64 / LR) + l / LR;
+            get_at[k] = out_at + (wave % 2 * 16 * WC + row * WC) * 2 + ((l % LR) ^ mix(row)) * 16;
+        }
         auto put = [&](int m) __attribute__((always_inline)) {
 #pragma unroll
             for (int n = 0; n < NT; ++n) asm volatile("" : "+a"(acc[m][n]));  // in the accumulators' registers until here
@@ -423,9 +450,10 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     if constexpr (GATED) z[i] = gated16<ACT>(acc[m][n][i], acc[m][n + NT / 2][i], p.gate);
-                    else z[i] = acc[m][n][i] * __uint_as_float(scale[m]);
+                    else if constexpr (KIND == kDown) z[i] = acc[m][n][i] * __uint_as_float(scale[m]);
+                    else z[i] = acc[m][n][i];
                 }
-                lds_write(out_at + put_at[n], make_uint2(pack_bf16x2(z[0], z[1]), pack_bf16x2(z[2], z[3])));
+                lds_write(put_at[n], make_uint2(pack_bf16x2(z[0], z[1]), pack_bf16x2(z[2], z[3])));
             }
         };
         s16x8 y[2][SI];
@@ -436,7 +464,7 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
             for (int k = 0; k < SI; ++k) {
                 if constexpr (KIND == kDown)
                     lds_read(row[m & 1][k], row_at + q * TM * 4 + (wm * 16 + lane / LR) * 4, (m * 32 + k * (64 / LR)) * 4);
-                lds_read(y[m & 1][k], out_at + get_at[k], 0);
+                lds_read(y[m & 1][k], get_at[k], 0);
             }
         };
         auto leave = [&](int m) __attribute__((always_inline)) {
@@ -451,7 +479,7 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
                     to_row = row[m & 1][k];
                 } else {
                     const int r = (2 * m + wm) * 16 + k * (64 / LR) + lane / LR;
-                    on = rows - 1 - r;
+                    on = in ? rows - 1 - r : -1;
                     to_row = own + r;
                 }
                 store_row(to + to_row * p.N, y[m & 1][k], on);
@@ -516,7 +544,7 @@ inline bool wide_fits(int K, int N, bool gated) { return K > 0 && K % 64 == 0 &&
 template <int KIND, int ACT = SKYRL_ACT_SILU, bool ONCE = false>
 int launch_wide(Wide p, hipStream_t s) {
     set_division(p);
-    const int64_t items = (int64_t)(p.N / (KIND == kDown ? 256 : 128)) * p.ntiles;
+    const int64_t items = (int64_t)(KIND == kDense ? (p.N + 255) / 256 : p.N / (KIND == kDown ? 256 : 128)) * p.ntiles;
     SKYRL_REQUIRE(items < (1ll << 31) && p.ntiles < (1 << 23), "wide products: too many rows in one call");
     const unsigned grid = (unsigned)(items > kCUs / 2 ? kCUs : (2 * items + 7) / 8 * 8);
     hipLaunchKernelGGL((wide_kernel<KIND, ACT, ONCE>), dim3(grid), dim3(256), 0, s, p);

@@ -259,6 +259,7 @@ def gate_normed_embedding(tokens: torch.Tensor, table: torch.Tensor, weight: tor
 
 # ---------------------------------------------------------------- products of few rows
 MAX_ROWS = 128  # that skyrl_rows_product takes at most
+ROUNDED_ROWS = 64  # of a rounded result
 
 
 def _rows_fit(x: torch.Tensor, w: torch.Tensor, gated: bool = False, parts: bool = False) -> bool:
@@ -270,6 +271,22 @@ def _rows_fit(x: torch.Tensor, w: torch.Tensor, gated: bool = False, parts: bool
     N = w.shape[0] // 2 if gated else w.shape[0]
     return (x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.is_cuda
             and bool(_ffi.query("skyrl_rows_product_fits", n, K, N, 1 if gated else 2 if parts else 0)) and _rows_aligned(x, w))
+
+
+def _dense_fit(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether skyrl_dense_product takes x [n, K] (a column range) and w [N, K] and is the faster form."""
+    (n, K), N = x.shape, w.shape[0]
+    return (n > ROUNDED_ROWS and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.is_cuda and w.shape[1] == K
+            and bool(_ffi.query("skyrl_dense_product_fits", n, K, N)) and n * x.stride(0) < 1 << 31 and N * w.stride(0) < 1 << 31
+            and _rows_aligned(x, w))
+
+
+def _dense(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    dev = _require_gpu(x, w)
+    (n, K), N = x.shape, w.shape[0]
+    out = torch.empty((n, N), dtype=torch.bfloat16, device=dev)
+    _ffi.call("skyrl_dense_product", _ptr(x), x.stride(0), n, K, _ptr(w), w.stride(0), N, _ptr(out), _stream(dev))
+    return out
 
 
 def gives_parts(x: torch.Tensor, w: torch.Tensor) -> bool:
@@ -289,7 +306,8 @@ def _rows_aligned(x: torch.Tensor, w: torch.Tensor) -> bool:
 
 
 def linear(x, w: torch.Tensor, bias: Optional[torch.Tensor] = None, parts: bool = False, turn=None) -> torch.Tensor:
-    """x w^T + bias. Few bf16 rows take skyrl_rows_product, everything else the library. With `parts` the result of
+    """x w^T + bias. Few bf16 rows take skyrl_rows_product, many without a bias skyrl_dense_product where it is the faster one,
+    everything else the library. With `parts` the result of
     few rows may be f32 [splits, n, N], to be summed over the first index where it is read (add_norm, gate_norm_add,
     joined). turn (first, last): these columns go through tanh, where `turns` says so. x: rows, or a NormedRow."""
     if isinstance(x, NormedRow):
@@ -300,7 +318,7 @@ def linear(x, w: torch.Tensor, bias: Optional[torch.Tensor] = None, parts: bool 
     if not _rows_fit(x, w, parts=parts):
         if turn is not None:
             raise ValueError("a library's product turns no columns")
-        return F.linear(x, w, bias)
+        return F.linear(x, w, bias) if bias is not None or not _dense_fit(x, w) else _dense(x, w)
     dev = _require_gpu(x, w, bias)
     (n, K), N = x.shape, w.shape[0]
     if w.shape[1] != K:

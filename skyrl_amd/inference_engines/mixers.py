@@ -437,8 +437,8 @@ class LatentAttention:
         if ts < T:
             seg, tiles, rows, longest = inp.plan[self.window]
             latent, k_rot = lk.latent_gather(cache, self.rank, self.rot_dim, inp.block_tables, seg, rows, longest)
-            k = F.linear(latent, self.wuk)
-            v_t = torch.mm(self.wuv, latent.t())
+            k = lk.linear(latent, self.wuk)
+            v_t = lk.linear(self.wuv, latent)
             lk.latent_prefill(q, k, k_rot, v_t, tiles, H, self.dim, self.rot_dim, self.vdim, self.scale, self.window,
                               out, sinks=self.sinks, gate=gate)
 

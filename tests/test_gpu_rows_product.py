@@ -70,6 +70,38 @@ def test_gated_in_rounds(dev, n, N, K):
     test_gated(dev, n, N, K, "silu")
 
 
+@pytest.mark.parametrize("n,N,K", [(65, 40, 64), (129, 1000, 192), (200, 2040, 1088),            # tiles of 64 x 32
+                                   (65, 8000, 64), (130, 5000, 320),                             # 64 x 64
+                                   (300, 5000, 64), (700, 3400, 256), (65, 16384, 128),          # 64 x 128
+                                   (300, 9000, 64), (1000, 4104, 192),                           # 128 x 128
+                                   (2100, 520, 64), (1537, 5000, 640), (3000, 5000, 128), (3073, 6152, 192), (8200, 1032, 320)])  # 192, 256 rows
+@pytest.mark.parametrize("pad", (0, 24))
+def test_dense(dev, n, N, K, pad):
+    """Many rows: one stage and several, more stages than are under way, the last tile's rows and columns."""
+    x, w, _ = _data(dev, n, N, K, n + N, pad)
+    ref, off = _bounds(x, w)
+    for _ in range(2):
+        y = lk._dense(x, w)
+        assert y.shape == (n, N) and bool(((y.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2 * off).all())
+
+
+def test_many_rows_take_the_faster_form(dev):
+    for n, N, K, own in ((65, 2048, 2048, True), (256, 2048, 2048, True), (256, 3408, 2048, True), (1024, 12352, 2048, True), (5637, 12352, 2048, True),
+                         (5637, 3072, 768, True), (2048, 5824, 512, True), (1563, 2048, 2048, False), (8192, 2048, 2048, False),
+                         (8192, 2048, 6144, False), (256, 32768, 2048, False), (300, 4096, 12288, False), (300, 2044, 2048, False),
+                         (300, 2048, 2056, False)):
+        x, w, b = _data(dev, n, N, K, 0)
+        assert lk._dense_fit(x, w) == own, (n, N, K)
+        assert not lk._dense_fit(x[:64], w) and not lk._dense_fit(x.float(), w.float())
+        ref = torch.nn.functional.linear(x, w)
+        y = lk.linear(x, w)
+        assert float((y.float() - ref.float()).norm()) <= 1e-3 * float(ref.float().norm())  # the same rounding but where a sum's order differs
+        assert torch.equal(lk.linear(x, w, b), torch.nn.functional.linear(x, w, b))
+    x, w, _ = _data(dev, 256, 2048, 2048, 0, 4)
+    assert not lk._dense_fit(x, w)  # row strides of 2052
+    assert torch.equal(lk.linear(x, w), torch.nn.functional.linear(x, w))
+
+
 def test_what_the_library_takes(dev):
     x, w, _ = _data(dev, 129, 64, 64, 0)
     assert not lk._rows_fit(x, w)                                  # too many rows
