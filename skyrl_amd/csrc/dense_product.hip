@@ -160,7 +160,9 @@ int64_t wide_rounds(int n, int N, int rows) {
 // The form, and whether it is the faster one beside the library's. Up to some 1000 rows the smallest tiles that are one round
 // of workgroups (64 x 32 to 64 x 64 fit a CU twice, and 64 x 128 do, so that half a round more costs little): a CU's loads bound
 // them, 80 to 90 GB/s, and the library's tiles leave CUs idle. Above, the wide form where its items fill 70 % of their rounds
-// and the library's columns are no multiple of its own 256, which costs it 10 to 25 %. Shallow products are launches and latency.
+// and the columns are no multiple of the library's own 256, which costs it 10 to 25 %, or the rows none, where the two are within 2 %
+// alone and this is the faster one among a step's other launches: eight layers' 5637 rows of 2048 x 2048 39 us each beside 46, 1563 rows
+// in tiles of 128 x 128 22 beside 25. Shallow products are launches and latency.
 // us, here / the library's, weights from HBM, both in a captured graph:
 //   N, K            256 rows       512            1024           1563           3000          5637          8192
 //   2048, 2048      8.2 / 10.8     10.0 / 12.3    14.3 / 16.3    -              -             -             -
@@ -169,7 +171,7 @@ int64_t wide_rounds(int n, int N, int rows) {
 //   3072, 768       6.1 / 8.6      8.1 / 10.5     -              -              -             31 / 47       38 / 46
 //   2048, 512       4.7 / 6.8      5.5 / 8.6      7.0 / 9.7      9.3 / 11.4     12.8 / 14.2   17.5 / 27.9   21.5 / 23.2
 //   24640, 4096     -              -              -              267 / 374      456 / 515     837 / 929     1149 / 1218
-// Where the library stays, us, the same: 1563 x 2048, 3408 28.7 / 30.4 and 2048 28.1 / 20.9; 3000 x 2048, 2048 29.1 / 27.9; 8192 x
+// Where the library stays, us, the same: 1563 x 2048, 3408 28.7 / 30.4; 3000 x 2048, 2048 29.1 / 27.9; 8192 x
 // 2048, 2048 53 / 51; 1300 x 6144, 2048 50.6 / 39.0; 512 x 2048, 12352 40.7 / 35.4; 2048 x 2048, 32768 216 / 200.
 Form form_of(int n, int K, int N, bool& faster) {
     faster = true;
@@ -183,7 +185,8 @@ Form form_of(int n, int K, int N, bool& faster) {
     const int64_t r256 = wide_rounds(n, N, 256), r192 = wide_rounds(n, N, 192), rounds = r192 < r256 ? r192 : r256;
     const bool full = (int64_t)n * N * 100 >= 70 * rounds * 256 * 256 * kCUs / 100;
     if (K <= 512 && n <= 2048) return tiles_of(n, N, 64, 128) <= 2 * kCUs ? k64x128 : k128x128;
-    faster = K <= 512 || (full && ((n >= 800 && N % 256 != 0) || (n >= 5000 && K <= 1024)));
+    if (n <= 2048 && K <= 2048 && tiles_of(n, N, 128, 128) <= kCUs) return k128x128;
+    faster = K <= 512 || (full && ((n >= 800 && N % 256 != 0) || (n >= 4096 && n % 256 != 0) || (n >= 5000 && K <= 1024)));
     return r192 < r256 ? kWide192 : kWide256;
 }
 

@@ -87,7 +87,7 @@ def test_dense(dev, n, N, K, pad):
 
 def test_many_rows_take_the_faster_form(dev):
     for n, N, K, own in ((65, 2048, 2048, True), (256, 2048, 2048, True), (256, 3408, 2048, True), (1024, 12352, 2048, True), (5637, 12352, 2048, True),
-                         (5637, 3072, 768, True), (2048, 5824, 512, True), (1563, 2048, 2048, False), (8192, 2048, 2048, False),
+                         (5637, 3072, 768, True), (2048, 5824, 512, True), (1563, 2048, 2048, True), (3000, 2048, 2048, False), (8192, 2048, 2048, False),
                          (8192, 2048, 6144, False), (256, 32768, 2048, False), (300, 4096, 12288, False), (300, 2044, 2048, False),
                          (300, 2048, 2056, False)):
         x, w, b = _data(dev, n, N, K, 0)
