@@ -1647,16 +1647,30 @@ struct ToppPending {  // a row pass 1 did not decide, for sample_topp_pass2_kern
     long long c;             // the split cut key's kept tie ranks
 };
 
+// Few rows: a row's pieces are workgroups of their own (SPLIT), which leave these; the last to arrive has the row's counts, the
+// records that reached a piece's bar and the largest of the bars, and goes on as if it had streamed the row. An element that a
+// piece skipped scored below that piece's bar, so below the largest: the certificate holds as it stands, and at least as often.
+constexpr int kTPieces = 8, kTPub = 64;
+struct alignas(16) ToppPart {
+    uint64_t hist[kPHalf / 2];   // four bins a word (a piece has less than 65536 elements)
+    uint32_t slow[kPSlowCap];
+    float cs[kTPub];             // records at or above the bar: score, index, bits
+    int32_t ci[kTPub];
+    uint32_t ck[kTPub];
+    float vmax, bar;
+    uint32_t nslow, bad, zero[2], nrec, more;  // more: there were others
+};
+
 // uniform (scalar) copy of a wave-uniform float, so the hot loops keep it in an SGPR
 __device__ __forceinline__ float uni(float x) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x))); }
 
-template <typename T, bool TOPP>
+template <typename T, bool TOPP, bool SPLIT = false>
 __global__ __launch_bounds__(kPNT) __attribute__((amdgpu_waves_per_eu(4))) void sample_topp_kernel(
     const T* __restrict__ logits, int64_t ld, int V, float inv_t, int use_minp, float ln_min_p, float top_p,
     uint64_t seed, const int64_t* __restrict__ seq_ids, int64_t step, int32_t* __restrict__ tokens,
     float* __restrict__ logp_out, RowFilter* __restrict__ filt, ToppPending* __restrict__ pend,
-    unsigned* __restrict__ pend_nt, int probe) {
-    static_assert(sizeof(T) == 2, "bf16 rows");
+    unsigned* __restrict__ pend_nt, int probe, ToppPart* __restrict__ tparts, unsigned* __restrict__ counters) {
+    static_assert(sizeof(T) == 2 && (TOPP || !SPLIT), "bf16 rows");
     constexpr int NT = kPNT, NW = NT / kWave, VEC = 8;
     constexpr int kDummy = 2 * kPHalf;  // 64 words taking the out-of-window elements' increments (no branch)
     __shared__ __attribute__((aligned(16))) uint32_t s_hist[2 * kPHalf + kWave];
@@ -1692,12 +1706,22 @@ __global__ __launch_bounds__(kPNT) __attribute__((amdgpu_waves_per_eu(4))) void 
     const int nvec = V / VEC;
     constexpr int kStep = 4 * NT;
     const uint64_t t_start = __builtin_amdgcn_s_memrealtime();  // (probes 5 / 6: per-row phase times)
-    const int nfull = (nvec / kStep) * kStep;
+    // this workgroup's vectors of the row: all of them, or its piece's
+    const int piece = SPLIT ? (int)blockIdx.y : 0, pieces = SPLIT ? (int)gridDim.y : 1;
+    const int v_lo = SPLIT ? (int)((int64_t)nvec * piece / pieces) : 0;
+    const int v_n = SPLIT ? (int)((int64_t)nvec * (piece + 1) / pieces) - v_lo : nvec;
+    const uint4* pv = rv + v_lo;
+    const int e_lo = v_lo * VEC;
+    const bool last_piece = !SPLIT || piece == pieces - 1;  // has the ragged tail
+    const int nfull = (v_n / kStep) * kStep;
     uint4 cur[4], nxt[4];
-    if (nfull > 0) {
+    // a step's vectors of this lane; past the last one it reads that again. The vectors after the last whole step are loaded with
+    // it, all at once: a load each, waited for, was 2 us of a call (512 rows of 151936: 54.8 -> 52.8 us).
+    auto load4 = [&](uint4 (&to)[4], int base) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) cur[u] = rv[u * NT + threadIdx.x];
-    }
+        for (int u = 0; u < 4; ++u) to[u] = pv[min(base + u * NT + (int)threadIdx.x, v_n - 1)];
+    };
+    if (v_n > 0) load4(cur, 0);
     if (threadIdx.x == 0) {
         s_nslow = 0u;
         s_bad = 0u;
@@ -1938,7 +1962,7 @@ __global__ __launch_bounds__(kPNT) __attribute__((amdgpu_waves_per_eu(4))) void 
                 kb = xk > xb ? k : kb;
                 xb = fmaxf(xb, xk);
             }
-            const int vb = (int)threadIdx.x * VEC + kb;
+            const int vb = e_lo + (int)threadIdx.x * VEC + kb;
             const uint32_t h = ehash(key, keyb, (uint32_t)vb >> 3);
             const float sc = noise_score(xb, inv_t, vb, h, group_min_e(h), key2);
             uint16_t bb = raw[0];
@@ -1954,20 +1978,17 @@ __global__ __launch_bounds__(kPNT) __attribute__((amdgpu_waves_per_eu(4))) void 
             }
         }
         for (int base = 0; base < nfull; base += kStep) {
-            const bool more = base + kStep < nfull;
+            const bool more = base + kStep < v_n;
             switch (((nfull - base) * 4 - 1) / nfull) {  // progress priority, as the row-mode sampler
                 case 3: __builtin_amdgcn_s_setprio(3); break;
                 case 2: __builtin_amdgcn_s_setprio(2); break;
                 case 1: __builtin_amdgcn_s_setprio(1); break;
                 default: __builtin_amdgcn_s_setprio(0); break;
             }
-            if (more) {
-#pragma unroll
-                for (int u = 0; u < 4; ++u) nxt[u] = rv[base + kStep + u * NT + threadIdx.x];
-            }
+            if (more) load4(nxt, base + kStep);
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                visit1(cur[u], (base + u * NT + (int)threadIdx.x) * VEC);
+                visit1(cur[u], e_lo + (base + u * NT + (int)threadIdx.x) * VEC);
                 __builtin_amdgcn_sched_barrier(0);
             }
             if (more) {
@@ -1993,10 +2014,13 @@ __global__ __launch_bounds__(kPNT) __attribute__((amdgpu_waves_per_eu(4))) void 
             thr_run = uni(s_runmax) * inv_t + ln_min_p;
         }
     }
-    for (int i0 = nfull; i0 < nvec; i0 += NT) {  // same trip count in every thread (wave ballots inside)
+    for (int i0 = nfull; i0 < v_n; i0 += NT) {  // same trip count in every thread (wave ballots inside)
         const int i = i0 + (int)threadIdx.x;
-        if (i < nvec) {
-            visit1(rv[i], i * VEC);
+        const uint4 pk = cur[0];
+#pragma unroll
+        for (int u = 0; u < 3; ++u) cur[u] = cur[u + 1];
+        if (i < v_n) {
+            visit1(pk, e_lo + i * VEC);
         } else {  // an idle lane joins the ballots with nothing to score
             const uint16_t nb[VEC] = {0xff80u, 0xff80u, 0xff80u, 0xff80u, 0xff80u, 0xff80u, 0xff80u, 0xff80u};
             const float nx[VEC] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY, -INFINITY, -INFINITY, -INFINITY, -INFINITY};
@@ -2004,7 +2028,7 @@ __global__ __launch_bounds__(kPNT) __attribute__((amdgpu_waves_per_eu(4))) void 
             else gumbel(nx, nb, -INFINITY, 0, 0);
         }
     }
-    if (nvec * VEC < V) {  // the ragged tail: one partial group, lanes 0 .. cnt-1 one element each
+    if (last_piece && nvec * VEC < V) {  // the ragged tail: one partial group, lanes 0 .. cnt-1 one element each
         const int t0 = nvec * VEC, cnt = V - t0;
         uint16_t tb[VEC];
         float tx[VEC];
@@ -2019,7 +2043,7 @@ __global__ __launch_bounds__(kPNT) __attribute__((amdgpu_waves_per_eu(4))) void 
         if constexpr (kList) collect(tx, tm, t0, threadIdx.x == 0 ? cnt : 0);
         else gumbel(tx, tb, tm, t0, threadIdx.x == 0 ? cnt : 0);
     }
-    for (int i = nvec * VEC + threadIdx.x; i < V; i += NT) {  // ragged tail, one element per thread
+    for (int i = last_piece ? nvec * VEC + (int)threadIdx.x : V; i < V; i += NT) {  // ragged tail, one element per thread
         const uint16_t b = row[i];
         const float x = bf16_to_f32(b);
         vmx = fmaxf(vmx, x);
@@ -2031,6 +2055,103 @@ __global__ __launch_bounds__(kPNT) __attribute__((amdgpu_waves_per_eu(4))) void 
     if (bad) s_bad = 1u;
     if (lane == 0) s_vmax[w] = vmx;
     __syncthreads();
+    bool whole = true;  // every record is there
+    if constexpr (SPLIT) {
+        __shared__ uint32_t s_nrec, s_head[kTPieces][8];
+        __shared__ int s_last;
+        ToppPart* const part = tparts + ((int64_t)row_i * pieces + piece);
+        const float own_bar = rbar();
+        if (threadIdx.x == 0) s_nrec = 0u;
+        __syncthreads();
+        for (int i = threadIdx.x; i < (int)min(s_nc, (uint32_t)kPCandCap); i += NT)
+            if (s_cs[i] >= own_bar) {
+                const uint32_t r = atomicAdd(&s_nrec, 1u);
+                if (r < (uint32_t)kTPub) {
+                    st_wt(&part->cs[r], s_cs[i]);
+                    st_wt(&part->ci[r], s_ci[i]);
+                    st_wt(&part->ck[r], (uint32_t)s_ck[i]);
+                }
+            }
+#pragma unroll
+        for (int k = 0; k < kPHalf / (2 * NT); ++k) {
+            const int j = threadIdx.x + NT * k;
+            const uint4 n = *reinterpret_cast<const uint4*>(&s_hist[4 * j]);
+            st_wt(&part->hist[j], (uint64_t)(n.x | n.y << 16) | (uint64_t)(n.z | n.w << 16) << 32);
+        }
+        for (int i = threadIdx.x; i < (int)min(s_nslow, (uint32_t)kPSlowCap); i += NT) st_wt(&part->slow[i], (uint32_t)s_slow[i]);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every wave's, ahead of the ticket
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            float m = s_vmax[0];
+            for (int j = 1; j < NW; ++j) m = fmaxf(m, s_vmax[j]);
+            st_wt(&part->vmax, m);
+            st_wt(&part->bar, own_bar);
+            st_wt(&part->nslow, s_nslow);
+            st_wt(&part->bad, s_bad);
+            st_wt(&part->zero[0], s_zero[0]);
+            st_wt(&part->zero[1], s_zero[1]);
+            st_wt(&part->nrec, min(s_nrec, (uint32_t)kTPub));
+            st_wt(&part->more, s_nc > (uint32_t)kPCandCap || s_nrec > (uint32_t)kTPub ? 1u : 0u);
+        }
+        if (!arrive_last(counters + row_i, (unsigned)pieces, &s_last)) return;
+        rearm(counters + row_i);
+        const ToppPart* const all = tparts + (int64_t)row_i * pieces;
+        auto word = [&](const void* q) { return __hip_atomic_load(reinterpret_cast<const uint32_t*>(q), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+        if ((int)threadIdx.x < pieces * 8) s_head[threadIdx.x / 8][threadIdx.x % 8] = word(reinterpret_cast<const uint32_t*>(&all[threadIdx.x / 8].vmax) + threadIdx.x % 8);
+        // The counts, four bins a word. All loads ahead of the sums (pieces that are none: the last one's, not added).
+        constexpr int kWords = kPHalf / (2 * NT);
+        uint64_t four[kTPieces][kWords];
+#pragma unroll
+        for (int q = 0; q < kTPieces; ++q)
+#pragma unroll
+            for (int k = 0; k < kWords; ++k)
+                four[q][k] = __hip_atomic_load(&all[min(q, pieces - 1)].hist[threadIdx.x + NT * k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        float m = -INFINITY, bar = -INFINITY;
+        uint32_t nslow = 0u, bads = 0u, z0 = 0u, z1 = 0u, nrec = 0u;
+        const int own_q = threadIdx.x / kTPub, own_r = threadIdx.x % kTPub;  // the record this thread carries
+        static_assert(kTPieces * kTPub == NT, "a thread a record");
+        int to = -1;
+        for (int q = 0; q < pieces; ++q) {
+            const uint32_t* h = s_head[q];
+            m = fmaxf(m, __uint_as_float(h[0]));
+            bar = fmaxf(bar, __uint_as_float(h[1]));
+            for (uint32_t i = threadIdx.x; i < min(h[2], (uint32_t)kPSlowCap); i += NT)
+                if (nslow + i < (uint32_t)kPSlowCap) s_slow[nslow + i] = (uint16_t)word(&all[q].slow[i]);
+            if (q == own_q && own_r < (int)h[6]) to = (int)nrec + own_r;
+            whole &= h[7] == 0u;
+            nslow += h[2], bads |= h[3], z0 += h[4], z1 += h[5], nrec += h[6];
+        }
+        if (to >= 0) {
+            const uint32_t sc = word(&all[own_q].cs[own_r]), id = word(&all[own_q].ci[own_r]), bits = word(&all[own_q].ck[own_r]);
+            s_cs[to] = __uint_as_float(sc);
+            s_ci[to] = (int32_t)id;
+            s_ck[to] = (uint16_t)bits;
+        }
+#pragma unroll
+        for (int k = 0; k < kWords; ++k) {
+            uint32_t n[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+            for (int q = 0; q < kTPieces; ++q) {
+                const uint64_t x = q < pieces ? four[q][k] : 0ull;
+#pragma unroll
+                for (int b = 0; b < 4; ++b) n[b] += (uint32_t)(x >> 16 * b) & 0xffffu;
+            }
+            *reinterpret_cast<uint4*>(&s_hist[4 * (threadIdx.x + NT * k)]) = make_uint4(n[0], n[1], n[2], n[3]);
+        }
+        if (threadIdx.x < NW) {
+            s_vmax[threadIdx.x] = m;
+            s_wbest[threadIdx.x] = bar;  // rbar() is the largest of the pieces' from here on
+        }
+        if (threadIdx.x == 0) {
+            s_nslow = nslow;
+            s_bad = bads;
+            s_zero[0] = z0;
+            s_zero[1] = z1;
+            s_nc = nrec;
+        }
+        __syncthreads();
+    }
     float mx = s_vmax[0];
 #pragma unroll
     for (int j = 1; j < NW; ++j) mx = fmaxf(mx, s_vmax[j]);
@@ -2265,7 +2386,7 @@ __global__ __launch_bounds__(kPNT) __attribute__((amdgpu_waves_per_eu(4))) void 
         }
     } else {
         const int nc = (int)min(s_nc, (uint32_t)kPCandCap);
-        const bool complete = s_nc <= (uint32_t)kPCandCap;
+        const bool complete = s_nc <= (uint32_t)kPCandCap && whole;
         auto cls = [&](int i) -> int {  // 1 admissible, 0 inadmissible, 2 an element of the split cut key
             const uint32_t kk = okey_bf16(s_ck[i]);
             if constexpr (TOPP) {
@@ -3019,6 +3140,23 @@ size_t ws_align(size_t b) { return (b + 255) / 256 * 256; }
 // allocated once stays valid under every variant
 size_t parts_bytes(int nseq) { return ws_align((size_t)nseq * kMaxSplits * sizeof(Part)); }
 
+// Pieces of a row with top_p. A workgroup streams its row at about 10 GB/s (its LDS adds), whatever else is idle: one row took the 35 us
+// that 256 take. Up to eight pieces of at least one streaming step (16384 elements): two more hand-offs (publish, ticket and merge:
+// 6 us) pay from four pieces on, and with more workgroups than CUs (over 64 rows) from six steps on. A u16 count holds a piece.
+// us a call, whole rows -> pieces: V 151936: 1 row 35.1 -> 24.0, 64 37.3 -> 27.9, 96 38.4 -> 36.5, 128 39.2 -> 33.3; V 262144:
+// 1 row 49.3 -> 26.8, 96 55.9 -> 40.3; V 102400: 1 row 27.8 -> 23.2, 128 31.1 -> 30.2; V 65536: 64 rows 24.9 -> 22.7, but 128
+// 24.7 -> 27.0; two pieces at V 32768 18.5 -> 20.9, three at 170 rows of 102400 31.7 -> 34.0.
+constexpr int kTParts = 512;
+int topp_pieces(int nseq, int V) {
+    const int steps = V / 8 / (4 * kPNT), fit = nseq > 0 ? kTParts / nseq : 1;
+    int pieces = steps < kTPieces ? steps : kTPieces;
+    if (pieces > fit) pieces = fit;
+    if (pieces < 4 || (nseq > kTParts / kTPieces && steps < 6)) return 1;
+    return ((V / 8 + pieces - 1) / pieces + 1) * 8 > 65535 ? 1 : pieces;
+}
+// enough for any number of rows up to this one
+size_t topp_parts_bytes(int nseq) { return (size_t)(nseq < kTParts / kTPieces ? nseq * kTPieces : kTParts) * sizeof(ToppPart); }
+
 template <typename T, int MODE>
 void launch_mode(dim3 grid, bool row_mode, hipStream_t stream, const T* lg, int64_t ld, int V, int chunk, float inv_t,
                  int use_topk, int use_minp, float ln_min_p, uint64_t seed, const int64_t* seq_ids, int64_t step,
@@ -3091,14 +3229,21 @@ int launch_sample(const void* logits, int64_t ld, int nseq, int V, float tempera
             Best* pparts = reinterpret_cast<Best*>(pw);
             pw += ws_align((size_t)nseq * kP2Splits * sizeof(Best));
             int32_t* pties = reinterpret_cast<int32_t*>(pw);
-            if (use_topp)
+            pw += ws_align((size_t)nseq * kPTieCap * sizeof(int32_t));
+            ToppPart* tparts = reinterpret_cast<ToppPart*>(pw);
+            const int pieces = probe ? 1 : topp_pieces(nseq, V);
+            if (use_topp && pieces > 1)
+                hipLaunchKernelGGL((sample_topp_kernel<T, true, true>), dim3(nseq, pieces), dim3(kPNT), 0, stream, lg, ld, V, inv_t,
+                                   use_minp, ln_min_p, top_p, seed, seq_ids, step, tokens, logp, filt, pend, pend_nt,
+                                   probe, tparts, counters);
+            else if (use_topp)
                 hipLaunchKernelGGL((sample_topp_kernel<T, true>), dim3(nseq), dim3(kPNT), 0, stream, lg, ld, V, inv_t,
                                    use_minp, ln_min_p, top_p, seed, seq_ids, step, tokens, logp, filt, pend, pend_nt,
-                                   probe);
+                                   probe, tparts, counters);
             else
                 hipLaunchKernelGGL((sample_topp_kernel<T, false>), dim3(nseq), dim3(kPNT), 0, stream, lg, ld, V, inv_t,
                                    use_minp, ln_min_p, 1.0f, seed, seq_ids, step, tokens, logp, filt, pend, pend_nt,
-                                   probe);
+                                   probe, tparts, counters);
             int rc = check_launch("sample_topp_kernel");
             if (rc || !use_topp || (probe >= 1 && probe <= 4) || probe == 11) return rc;  // (probes 1-4, 11)
             hipLaunchKernelGGL((sample_topp_pass2_kernel<T, true>), dim3(nseq, kP2Splits), dim3(kPNT), 0, stream, lg, ld,
@@ -3138,7 +3283,7 @@ extern "C" size_t skyrl_sample_workspace_bytes(int32_t nseq, int32_t V) {
     return kCounterBytes + ws_align((size_t)nseq * sizeof(RowFilter)) +
            parts_bytes(nseq) + ws_align((size_t)nseq * sizeof(ToppPending)) +
            ws_align((size_t)nseq * 2 * sizeof(unsigned)) + ws_align((size_t)nseq * kP2Splits * sizeof(Best)) +
-           (size_t)nseq * kPTieCap * sizeof(int32_t) + 256;
+           ws_align((size_t)nseq * kPTieCap * sizeof(int32_t)) + topp_parts_bytes(nseq) + 256;
 }
 
 extern "C" int skyrl_sample(const void* logits, int dtype, int64_t ld, int32_t nseq, int32_t V, float temperature,

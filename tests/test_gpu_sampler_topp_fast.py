@@ -280,3 +280,34 @@ def test_pass2_state_across_batch_sizes(dev):
         ts, ls, _ = _run(x[:n], False, temperature=1.0, top_p=0.9, seed=8, seq_ids=ids[:n], step=k)
         assert torch.equal(tf, ts), (n, probe, int((tf != ts).sum()))
         assert bool((ff[:, 2] == _ROW_DONE).all()), (n, probe)
+
+
+@pytest.mark.parametrize("V", [16391, 65536, 65543, 151936, 262144])
+@pytest.mark.parametrize("n", [1, 5, 64, 65, 128, 171])
+def test_rows_in_pieces(dev, n, V):
+    """Few rows of enough elements are streamed in four to eight pieces: the two-kernel path's tokens, cuts and logprobs for rows
+    whose winner, ties or oddities lie in one piece or in all, call after call (the pieces' arrival counters are re-armed)."""
+    g = torch.Generator(device=dev).manual_seed(V + n)
+    x = torch.empty(n, -(-V // 8) * 8, device=dev, dtype=torch.bfloat16)[:, :V]
+    x.normal_(0.0, 2.5, generator=g)
+    odd = [lambda r: r.fill_(1.5),                                              # one value: a tie group of the whole row
+           lambda r: r.copy_((r.float() * 4).round() / 4),                       # a coarse grid: the cut splits a tie group
+           lambda r: r[V // 3:].fill_(float("-inf")),                            # pieces without a weight
+           lambda r: r[-200:].fill_(20.0),                                       # more equal best ones than a piece leaves
+           lambda r: r[::40].fill_(1e-6),                                        # more values below 2^-16 than are listed
+           lambda r: r[V - 1:].fill_(30.0),                                      # the ragged tail's
+           lambda r: r[7:8].fill_(float("inf")),
+           lambda r: r.mul_(0.01)]                                               # nearly flat: a cut far down
+    for i, f in enumerate(odd):
+        if n > 1 and i < n - 1:
+            f(x[i + 1])
+    ids = torch.arange(n, dtype=torch.int64, device=dev) * 3 + 7
+    for step, (temp, p) in enumerate(((0.6, 0.95), (1.0, 0.9), (1.3, 0.3))):
+        _ab(x, 0, temperature=temp, top_p=p, seed=5, seq_ids=ids, step=step)
+    one = [ops.sample(x, temperature=1.0, top_p=0.95, seed=9, seq_ids=ids, step=s) for s in range(3)]
+    whole = torch.cat([x, x.new_full((512, x.shape[1]), 0.0)[:, :V]]) if V % 8 == 0 else None
+    if whole is not None:  # among more rows a row is one workgroup's: the same bits
+        wide = torch.cat([ids, ids.new_zeros(512)])
+        for s, (t, l) in enumerate(one):
+            tw, lw = ops.sample(whole, temperature=1.0, top_p=0.95, seed=9, seq_ids=wide, step=s)
+            assert torch.equal(t, tw[:n]) and torch.equal(l.nan_to_num(), lw[:n].nan_to_num())
