@@ -481,7 +481,7 @@ __global__ __launch_bounds__(WM* WN* kWave) void moe_gemm_kernel(Product p, cons
     const int n0 = nb * OC;
     const uint16_t* we = w + (int64_t)e * (GATED ? 2 : 1) * p.N * p.K;
     const int64_t place0 = (int64_t)tile * TM;
-    const int nk = (p.K + BK - 1) / BK;
+    const int nk = (p.K + BK - 1) / BK, start = depth_start(e, p.K);
 
     if (tid < TM) {  // what the end needs of the rows
         const int pair = p.order[place0 + tid];
@@ -512,7 +512,9 @@ __global__ __launch_bounds__(WM* WN* kWave) void moe_gemm_kernel(Product p, cons
     }
     auto fetch = [&](auto nt, int t) {  // piece t (the last again past the end) into stage t % S
         uint16_t* dst = smem + (t % S) * kStage;
-        const int k0 = min(t, nk - 1) * BK;
+        int step = min(t, nk - 1) + start;
+        step = step >= nk ? step - nk : step;
+        const int k0 = step * BK;
 #pragma unroll
         for (int i = 0; i < XL; ++i) {
             const int k = k0 + xk[i], piece = min(wave * XL + i, XP - 1);
@@ -654,15 +656,24 @@ int launch_product(Product p, const void* x, const void* w, void* out, int ntile
         // of 64 and more, and of 16 at other loads, sum a row in one order, so that a step's rows do not depend on which of
         // them its load takes. The package itself asks for 16 below 12 pairs per expert, streamed; a caller who asks for them at
         // larger loads has the bits of larger tiles (both products, 300 tokens: 202 us, streamed 183, in tiles of 64 146).
-        // Tiles of 64, gated: up to 2048 deep 64 weight rows in four stages in place of 128 in three. Two workgroups of either fit
-        // a CU, and 64 tiles of 768 columns are three rounds of the narrow ones, one and a half of the others (64 experts of 768
-        // x 2048, both products, 256 tokens: 139.6 us against 143.5, streamed in shares 137; 1536 x 4096: 469 against 459).
+        // Tiles of 64 and more by wide.h, where the depth and columns are multiples of its own: the ring of a CU does not stop
+        // between items, which costs two workgroups a CU a tenth (64 experts of 768 x 2048, gate_up / down, us, against
+        // moe_gemm_kernel: 256 tokens in tiles of 64 63 / 39 (72 / 42), 500 in tiles of 128 71 / 44 (88 / 50); 1536 x 4096, 500 tokens 260 /
+        // 160 (311 / 182, all experts from depth 0)). Not tiles of 64 of a depth of less than 512, whose items are a few steps: 384 x 1024, down,
+        // 256 tokens 13.2 us, by wide.h 14.7.
+        // Else, tiles of 64, gated: up to 2048 deep 64 weight rows in four stages in place of 128 in three. Two workgroups of either fit
+        // a CU, and 64 tiles of 768 columns are three rounds of the narrow ones, one and a half of the others.
         const bool once = ntiles <= 2 * experts;
         p.past = (int64_t)experts * (GATED ? 4 : 2) * p.N * p.K >= kPast;
-        if (p.tm == 256 && wide_fits(p.K, p.N, GATED)) {
+        if (p.tm >= 64 && wide_fits(p.K, p.N, GATED) && (GATED || p.tm > 64 || p.K >= 512)) {
             constexpr int kind = GATED ? kGateUp : kDown;
             const Wide wide{x_, w_, o_, p.K, p.N, p.K, p.K, ntiles, p.order, p.tile_expert, p.row_div, 0, 0, p.weight, 0, 0, Gate{}};
-            return once && p.past ? launch_wide<kind, SKYRL_ACT_SILU, true>(wide, s) : launch_wide<kind>(wide, s);
+            auto launch = [&](auto tm) {
+                return once && p.past ? launch_wide<kind, SKYRL_ACT_SILU, true, tm>(wide, s) : launch_wide<kind, SKYRL_ACT_SILU, false, tm>(wide, s);
+            };
+            if (p.tm == 64) return launch(std::integral_constant<int, 64>{});
+            if (p.tm == 128) return launch(std::integral_constant<int, 128>{});
+            return launch(std::integral_constant<int, 256>{});
         }
         if (p.tm == 256) LAUNCH_GEMM(256, 256, 2, 4, 2);
         else if (p.tm == 128) LAUNCH_GEMM(128, 128, 2, 2, 2);

@@ -105,17 +105,26 @@ __device__ __forceinline__ int32_t uniform(const int32_t* p) {
     return *reinterpret_cast<const __attribute__((address_space(4))) int32_t*>(reinterpret_cast<uintptr_t>(p));
 }
 
+// The step of the depth that an expert's products begin with; past the last one they go on at the first. Workgroups run about in
+// step, and at a row stride of 4 KB the same depth of all rows lies in the same few of the memory's channels: weights from HBM
+// came at 5.2 TB/s where all experts began at 0, at 6.2 where each begins elsewhere (64 experts of 768 x 2048, gate_up, us: 256 tokens
+// 79 -> 63, 700 tokens in tiles of 128 90 -> 75; down, rows of 1536 bytes, 40.7 -> 39.4). One start for an expert: its tiles, and
+// a tile's columns, share what they read (a start for each column: 5637 tokens 265 us, 243 with this).
+__device__ __forceinline__ int depth_start(int e, int K) {
+    return K % 256 == 0 ? (int)__umulhi((uint32_t)e * 0x9E3779B9u, (uint32_t)K / 64) : 0;
+}
+
 // Whether an expert's tiles, which follow each other, are this one alone.
 __device__ __forceinline__ bool one_tile(const int32_t* tile_expert, int tile, int ntiles, int e) {
     return (tile == 0 || tile_expert[tile - 1] != e) && (tile + 1 == ntiles || tile_expert[tile + 1] != e);
 }
 
-// Tiles of 256 rows (prompts): 256 weight rows per workgroup of four waves, 128 x 128 results and a SIMD each. A wave has nobody
+// Tiles of TM rows, 256 (prompts) or, routed, 64 and 128: 256 weight rows per workgroup of four waves, 128 x 128 results and a SIMD each. A wave has nobody
 // to hide behind, so its reads of the next operands and the loads of later stages are placed between the products, one every
 // few. With 128 x 64 a wave (eight of them) the operands' reads alone took as many LDS cycles as the products took matrix cycles.
 // Stages of 64 deep go round a ring of LDS slots of 64 rows, 19 for two stages of 8 and the first three of a third: with two
 // stages alone a stage's loads started when the one before was released and either met all at once (64 bytes a cycle and CU)
-// or had too little time to land.
+// or had too little time to land. With tiles of 64 a stage is five slots, three stages are ahead.
 // A workgroup per CU goes through its XCD's run of items (a tile and 256 weight rows). The ring does not stop between them: an
 // item's last two steps load the next one's first two stages, which land while the results leave, 16 rows at a time through a piece
 // of LDS of the wave's own. The next item's rows and weights of pairs go to LDS by direct loads, too, since a load into a register
@@ -123,7 +132,7 @@ __device__ __forceinline__ bool one_tile(const int32_t* tile_expert, int tile, i
 // What is left over behind the whole rounds is cut into halves of the columns where there are workgroups for both (1500 x 2048,
 // 6144 gated: 288 items, 93 us in two whole rounds, 74 in one and a half). Cut by rows, both halves would read the weights.
 // A tile's rows are spread over the two rows of waves by sixteens, and products past its last 64 used rows are left out (700
-// pairs per expert: a sixth of the rows is padding). The depth is a multiple of 64, the columns of the item's.
+// pairs per expert: a sixth of the rows is padding), their loads are not: tiles of 64 and 128 where most experts have no more. The depth is a multiple of 64, the columns of the item's.
 //   kGateUp, kDown  routed experts (moe.hip): rows by the pairs' order. kGateUp takes a row of x per token and leaves one per
 //                   place, silu(gate) up; kDown takes one per place and leaves one per pair, weighted.
 //   kGated, kDense  one matrix, x and the output row by row in tiles of tile_rows (gated_product.hip): of N gate and N up rows,
@@ -137,18 +146,21 @@ __device__ __forceinline__ bool one_tile(const int32_t* tile_expert, int tile, i
 // ONCE: weights of an expert with one tile go past the caches (non-temporal), those of an expert with several, which read them from
 // there, do not: both products, us (all cached / all past), before: 1563 tokens 185 (195 / 186), unevenly loaded 192 (196 / 202), 2048
 // tokens 260 (259 / 275). The loops for both are one inlined body each: as calls they kept their captures in scratch.
-template <int KIND, int ACT, bool ONCE>
+template <int KIND, int ACT, bool ONCE, int TM>
 __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
     constexpr bool GATED = KIND == kGateUp || KIND == kGated, ROUTED = KIND == kGateUp || KIND == kDown, GATHER = KIND != kDown;
     const int ncols = KIND == kDense ? (p.N + 255) / 256 : p.N / (GATED ? 128 : 256);
-    constexpr int TM = 256, BK = 64, L = 8;               // L loads each of x, w
+    constexpr int BK = 64, XS = TM / 64;                   // slots of x
+    constexpr int LW = 8, LX = 2 * XS, L = LX + LW;        // loads of w, of x, of a stage
+    constexpr int SS = 4 + XS;                             // slots of a stage
+    constexpr int AHEAD = XS == 1 ? 3 : 2;                 // stages under way
     // 64 rows, bytes. Slots of a stage: four of x, four of w, those ahead that are loaded ahead: weights that come from HBM, which
     // have the longer way (1563 tokens 103 / 58 us, behind the rows 106 / 60), else the rows (5637 tokens 247 / 152, 250 / 153).
     constexpr uint32_t SLOT = 64 * BK * 2, RING = 19;
     constexpr bool WF = ONCE;
     constexpr int OC = GATED ? 128 : 256;                  // output columns
-    constexpr int REST = 5;                                // of a stage's loads, the last ones
-    constexpr int kOut = 5;                                // of a stage's slots, the first where results pass through LDS
+    constexpr int REST = XS == 4 ? 5 : 0;                  // of a stage's loads, the last ones
+    constexpr int kOut = XS == 4 ? 5 : 2;                  // of a stage's slots, the first where results pass through LDS
     __shared__ __attribute__((aligned(16))) uint16_t smem[RING * SLOT / 2];
     __shared__ int s_rows[2][4];  // of 64 rows each: the last in use; kAll: all are
     constexpr uint32_t kAll = 1 << 16;
@@ -190,7 +202,8 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
         next_half = half_of(i);
         next_n0 = col * OC;
         if constexpr (ROUTED) {
-            __builtin_amdgcn_global_load_lds((gbl_void*)(p.order + ((int64_t)next_tile * TM + tid)), (lds_void*)&s_row[qn][wave * kWave], 4, 0, 0);
+            if (XS == 4 || wave < XS)
+                __builtin_amdgcn_global_load_lds((gbl_void*)(p.order + ((int64_t)next_tile * TM + tid)), (lds_void*)&s_row[qn][wave * kWave], 4, 0, 0);
             next_e = uniform(p.tile_expert + next_tile);
             if constexpr (ONCE) {
                 e_before = next_tile > 0 ? uniform(p.tile_expert + next_tile - 1) : -1;
@@ -201,14 +214,16 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
     // A slot is loaded by all waves, two pieces of 8 rows each. Global sources of this lane's 16 bytes: chunk (lane % 8) ^ (row
     // / 2 % 8), so that the 16 rows a matrix operand reads at a time lie in different banks. Rows of w follow each other.
     const int chunk[2] = {(lane % 8 ^ lane / 16) * 8, (lane % 8 ^ (lane / 16 + 4)) * 8};  // even, odd piece
-    const uint16_t *xs[GATHER ? L : 2], *ws[2];
-    uint32_t xo[L] = {}, wo[L] = {};  // kDense: in bytes from the first row
+    const uint16_t *xs[GATHER ? LX : 2], *ws[2];
+    uint32_t xo[LX] = {}, wo[LW] = {};  // kDense: in bytes from the first row
     const __amdgpu_buffer_rsrc_t x_all = whole_buffer(p.x), w_all = whole_buffer(p.w);
     int64_t wslot[4] = {};  // what a slot's rows of w are past the item's first; those of a half are the first slots'
     auto wrap = [](uint32_t at) { return min(at, at - RING * SLOT); };  // of less than two rings
+    int k_start = 0;        // of the item whose loads are under way
+    auto depth = [&](int k) { return ROUTED && k + k_start >= p.K ? k + k_start - p.K : k + k_start; };
     auto fetch = [&](auto nt, int k0, uint32_t base, int i) __attribute__((always_inline)) {  // load i at depth k0 of the stage at base
-        const bool is_w = (i < L) == WF;
-        const int u = i % L;
+        const bool is_w = WF ? i < LW : i >= LX;
+        const int u = WF ? (is_w ? i : i - LW) : is_w ? i - LX : i;
         const uint32_t to = lds0 + wrap(base + i / 2 * SLOT + wave * (SLOT / 4)) + u % 2 * (SLOT / 8);
         lds_void* dst = (lds_void*)(uintptr_t)to;
         if constexpr (KIND == kDense) {
@@ -225,15 +240,15 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
     // compiler's, which would wait for every load into LDS under way.
     auto turn = [&](int qn) __attribute__((always_inline)) {
         const int r0 = wave * 16 + lane / 8;
-        uint32_t pair = 0, rows[L] = {};
-        if constexpr (ROUTED) lds_read(pair, row_at + (qn * TM + tid) * 4, 0);
+        uint32_t pair = 0, rows[LX] = {};
+        if constexpr (ROUTED) lds_read(pair, row_at + (qn * TM + tid % TM) * 4, 0);
         if constexpr (KIND == kGateUp)
 #pragma unroll
-            for (int i = 0; i < L; ++i) lds_read(rows[i], row_at + (qn * TM + r0) * 4, (i / 2 * 64 + i % 2 * 8) * 4);
+            for (int i = 0; i < LX; ++i) lds_read(rows[i], row_at + (qn * TM + r0) * 4, (i / 2 * 64 + i % 2 * 8) * 4);
         const int flip = next_half == 2 ? OC / 2 : 0;
         if constexpr (KIND == kDense) {
 #pragma unroll
-            for (int i = 0; i < L; ++i)  // rows past the last: the last one, its columns not stored
+            for (int i = 0; i < LW; ++i)  // rows past the last: the last one, its columns not stored
                 wo[i] = (min(next_n0 + (i / 2 * 64 ^ flip) + i % 2 * 8 + r0, p.N - 1) * (uint32_t)p.ldw + chunk[i % 2]) * 2;
         } else {
             const uint16_t* we = p.w + (ROUTED ? (int64_t)max(next_e, 0) * (GATED ? 2 : 1) * p.N * p.ldw : 0);
@@ -242,12 +257,13 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) wslot[j] = ((j * 64 ^ flip) + (GATED && j >= 2 ? p.N - OC : 0)) * p.ldw;
         }
+        if constexpr (ROUTED) k_start = depth_start(next_e, p.K) * BK;
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         asm volatile("" : "+v"(pair));
         if constexpr (!ROUTED) {
             const int row0 = next_tile * p.tile_rows;
 #pragma unroll
-            for (int i = 0; i < L; ++i) {  // rows past the last: the last one, not stored
+            for (int i = 0; i < LX; ++i) {  // rows past the last: the last one, not stored
                 const int row = min(row0 + i / 2 * 64 + i % 2 * 8 + r0, p.n - 1);
                 if constexpr (KIND == kDense) xo[i] = (row * (uint32_t)p.ldx + chunk[i % 2]) * 2;
                 else xs[i] = p.x + row * p.ldx + chunk[i % 2];
@@ -255,7 +271,7 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
             pair = tid < p.tile_rows && row0 + tid < p.n ? 0 : -1;
         } else if constexpr (KIND == kGateUp) {
 #pragma unroll
-            for (int i = 0; i < L; ++i) {
+            for (int i = 0; i < LX; ++i) {
                 asm volatile("" : "+v"(rows[i]));
                 const uint32_t row = max((int)rows[i], 0);  // places without a pair: row 0, not stored
                 xs[i] = p.x + (p.row_div > 1 ? __umulhi(row, p.div_mul) >> p.div_shift : row) * p.ldx + chunk[i % 2];
@@ -263,9 +279,12 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
         } else {
             const uint16_t* xt = p.x + (next_tile * TM + r0) * p.ldx;
             xs[0] = xt + chunk[0], xs[1] = xt + 8 * p.ldx + chunk[1];
-            if (p.weight) __builtin_amdgcn_global_load_lds((gbl_void*)(p.weight + max((int)pair, 0)), (lds_void*)&s_wt[qn][wave * kWave], 4, 0, 0);
-            else lds_write(wt_at + (qn * TM + tid) * 4, __float_as_uint(1.f));
+            if (XS == 4 || wave < XS) {
+                if (p.weight) __builtin_amdgcn_global_load_lds((gbl_void*)(p.weight + max((int)pair, 0)), (lds_void*)&s_wt[qn][wave * kWave], 4, 0, 0);
+                else lds_write(wt_at + (qn * TM + tid) * 4, __float_as_uint(1.f));
+            }
         }
+        if (XS < 4 && wave >= XS) pair = -1;
         const uint64_t in = __ballot((int)pair >= 0);
         if (lane == 0)
             lds_write(rows_at + (qn * 4 + wave) * 4, (uint32_t)(in ? 64 * wave + 64 - __builtin_clzll(in) : 0) | (~in ? 0u : kAll));
@@ -275,7 +294,7 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
         n0 = next_n0 + (half == 2 ? OC / 2 : 0);
         once = ONCE && e_before != next_e && e_after != next_e;
     };
-    const bool chain = nk > 2;  // an item's last steps load the next one's first stages
+    const bool chain = nk > 2 * AHEAD - 2;  // an item's last steps load the next one's first stages; its rows have landed then
     uint32_t b0 = 0;            // where the next stage starts in the ring
     auto prime = [&](int i) __attribute__((always_inline)) {
         peek(i, q);
@@ -285,9 +304,9 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
         turn(q);
         turned();
 #pragma unroll
-        for (int i = 0; i < 2 * L; ++i) fetch(std::false_type{}, 0, b0, i);
+        for (int j = 0; j < AHEAD; ++j)
 #pragma unroll
-        for (int i = 0; i < 2 * L; ++i) fetch(std::false_type{}, nk > 1 ? BK : 0, wrap(b0 + 8 * SLOT), i);
+            for (int i = 0; i < L; ++i) fetch(std::false_type{}, depth(min(j, nk - 1) * BK), wrap(b0 + j * SS * SLOT), i);
         wait_loads<0>();
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
@@ -307,19 +326,19 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
         constexpr int MH = mh_, NT = HALF ? 4 : 8, M = MH * NT;     // NT 16-wide tiles of columns a wave
         constexpr int WC = OC / (HALF ? 4 : 2);                   // output columns a wave
         constexpr int LR = WC / 8, SI = LR / 4;                   // lanes per row as it leaves, stores of 16 rows
-        constexpr int LW = HALF ? L / 2 : L;                      // loads of w a stage
-        constexpr int E1 = HALF ? 2 : 3, E2 = E1, F3 = 5, F1 = LW + L - E1 - E2 - F3;  // a stage's loads in the groups of products:
-                                                                                        // early, from the release on, in the next step
-        static_assert(4 * 16 * WC * 2 <= 2 * SLOT && (HALF || F1 == REST), "ring");
+        constexpr int HW = HALF ? LW / 2 : LW;                    // loads of w a stage
+        // A stage's loads in the groups of products: early, from the release on, in the next step.
+        constexpr int E1 = XS == 4 ? (HALF ? 2 : 3) : HW / 2, E2 = E1, F3 = XS == 4 ? 5 : LX, F1 = HW + LX - E1 - E2 - F3;
+        static_assert(4 * 16 * WC * 2 <= 2 * SLOT && (HALF || F1 == REST) && AHEAD * SS + (E1 + E2) / 2 <= (int)RING, "ring");
         const bool chained = !HALF && more && chain;
         // load i of the run's: half of the columns is two slots' rows of w, with GATED the gate's and the other matrix' first
         auto stage = [&](int k0, uint32_t base, int i) __attribute__((always_inline)) {
-            const int before = WF ? 0 : L, u = i - before;  // of w's loads
-            const bool is_w = u >= 0 && u < LW;
-            fetch(nt, k0, base, is_w ? before + (HALF && GATED && u >= 2 ? u + 2 : u) : WF ? i - LW + L : i);
+            const int before = WF ? 0 : LX, u = i - before;  // of w's loads
+            const bool is_w = u >= 0 && u < HW;
+            fetch(nt, k0, base, is_w ? before + (HALF && GATED && u >= 2 ? u + 2 : u) : WF ? i - HW + LW : i);
         };
         // the wave's slots of w and its rows in them
-        const uint32_t w0 = ((WF ? 0 : 4) + (GATED ? (HALF ? 0 : wn) : HALF ? wn : 2 * wn)) * SLOT, w1 = w0 + (GATED ? 2 : HALF ? 0 : 1) * SLOT;
+        const uint32_t w0 = ((WF ? 0 : XS) + (GATED ? (HALF ? 0 : wn) : HALF ? wn : 2 * wn)) * SLOT, w1 = w0 + (GATED ? 2 : HALF ? 0 : 1) * SLOT;
         constexpr int WT = GATED || !HALF ? NT / 2 : NT;          // tiles of a slot
         const uint32_t wrow = GATED && HALF ? wn * 32 * BK * 2 : 0;
         // Results pass through LDS, 16 rows of WC columns a wave, 16-byte chunks xor-swizzled by the row.
@@ -365,15 +384,16 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
         int k2 = 0;  // depth of the loads under way
         // A step, whose loads are two stages ahead, at depth k; with `turning`, the next item's from here on.
         auto step = [&](auto first, auto turning, int k) __attribute__((always_inline)) {
-            const uint32_t b1 = wrap(b0 + 8 * SLOT), b2 = wrap(b1 + 8 * SLOT);  // of the next stages
+            // of the next stage, of the one to load and the one before that
+            const uint32_t b1 = wrap(b0 + SS * SLOT), bl = wrap(b0 + (AHEAD - 1) * SS * SLOT), b2 = wrap(bl + SS * SLOT);
             constexpr int G1 = first.value ? 0 : F1;        // the first step's stand ahead of the last item's stores
             group(first, I0{}, I0{}, std::integral_constant<int, MH + G1>{}, [&](int j) {
                 if (j < MH) read_x(b0, 0, 1, j);
-                else stage(k2, b1, E1 + E2 + F3 + j - MH);
+                else stage(k2, bl, E1 + E2 + F3 + j - MH);
             });
-            k2 = k;
             if constexpr (turning.value)
                 if (chained) turn(q ^ 1);
+            k2 = depth(k);
             group(first, I0{}, I1{}, std::integral_constant<int, NT + MH + E1>{}, [&](int j) {
                 if (j < NT) read_w(b0, 1, j);
                 else if (j < NT + MH) read_x(b0, 1, 0, j - NT);
@@ -384,8 +404,9 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
                 else stage(k2, b2, E1 + j - MH);
             });
             // this wave's loads of stage t + 1 have landed, its reads of stage t too
-            if (first.value && whole) wait_loads<E1 + E2 + OC / 8>();
-            else wait_loads<E1 + E2>();
+            constexpr int LATER = (AHEAD - 2) * (HW + LX) + E1 + E2;
+            if (first.value && whole) wait_loads<LATER + OC / 8>();
+            else wait_loads<LATER>();
             __builtin_amdgcn_s_barrier();  // and everyone's
             asm volatile("" ::: "memory");
             group(Later{}, I1{}, I1{}, std::integral_constant<int, NT + MH + F3>{}, [&](int j) {
@@ -403,16 +424,18 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
         // Past the item's last stage the loads are the next item's, or the last stage's again. The steps around that are copies of
         // their own: as cases of the loop's body they cost it 7 %.
         const int last = (nk - 1) * BK;
-        step(std::true_type{}, Later{}, min(2 * BK, last));
+        step(std::true_type{}, Later{}, min(AHEAD * BK, last));
         if constexpr (HALF) {
-            for (int t = 1; t < nk; ++t) step(Later{}, Later{}, min((t + 2) * BK, last));
+            for (int t = 1; t < nk; ++t) step(Later{}, Later{}, min((t + AHEAD) * BK, last));
         } else {
-            for (int t = 1; t < nk - 2; ++t) step(Later{}, Later{}, (t + 2) * BK);
-            if (nk > 2) step(Later{}, std::true_type{}, chained ? 0 : last);
-            if (nk > 1) step(Later{}, Later{}, chained ? BK : last);
+            for (int t = 1; t < nk - AHEAD; ++t) step(Later{}, Later{}, (t + AHEAD) * BK);
+            if (nk > AHEAD) step(Later{}, std::true_type{}, chained ? 0 : last);
+#pragma unroll
+            for (int j = 1; j < AHEAD; ++j)
+                if (nk > AHEAD - j) step(Later{}, Later{}, chained ? j * BK : last);
             if (chained)
 #pragma unroll
-                for (int i = 2 * L - REST; i < 2 * L; ++i) fetch(nt, k2, wrap(b0 + 8 * SLOT), i);  // what remains of the next item's
+                for (int i = L - REST; i < L; ++i) fetch(nt, k2, wrap(b0 + (AHEAD - 1) * SS * SLOT), i);  // what remains of the next item's
         }
         uint16_t* const to = p.out + n0 + wn * WC + lane % LR * 8;
         const int own = tile * (ROUTED ? TM : p.tile_rows);
@@ -429,7 +452,7 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
         if constexpr (KIND == kDown)
 #pragma unroll
             for (int m = 0; m < 2 * MH; ++m) asm volatile("" : "+v"(scale[m]));
-        const uint32_t out_at = lds0 + wrap(wrap(b0 + (RING - 8) * SLOT) + (kOut + wave / 2) * SLOT);
+        const uint32_t out_at = lds0 + wrap(wrap(b0 + (RING - SS) * SLOT) + (kOut + wave / 2) * SLOT);
         uint32_t put_at[WC / 16], get_at[SI];
         int l = lane;
         asm volatile("" : "+v"(l));  // formed here: as values of the whole launch they were put out to memory
@@ -498,7 +521,7 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
             }
             leave(m);
         }
-        whole = MH == 4 && all_rows && nk > 3;  // with fewer stages the next item's rows are needed right behind the first step
+        whole = MH == 4 && all_rows && nk > AHEAD + 1;  // with fewer stages the next item's rows are needed right behind the first step
     };
     prime(0);
     for (int i = 0;; ++i) {
@@ -515,10 +538,14 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
         const bool all_rows = __builtin_amdgcn_readfirstlane(r4[0] & r4[1] & r4[2] & r4[3]) & kAll, more = i + 1 < mine;
         if (more && chain) peek(i + 1, q ^ 1);
         auto all = [&](auto half_, auto nt) __attribute__((always_inline)) {
-            if (rows > 192) run(std::integral_constant<int, 4>{}, half_, nt, rows, all_rows, more);
-            else if (rows > 128) run(std::integral_constant<int, 3>{}, half_, nt, rows, all_rows, more);
-            else if (rows > 64) run(std::integral_constant<int, 2>{}, half_, nt, rows, all_rows, more);
-            else run(std::integral_constant<int, 1>{}, half_, nt, rows, all_rows, more);
+            const auto of = [&](auto mh) __attribute__((always_inline)) { run(mh, half_, nt, rows, all_rows, more); };
+            if constexpr (XS == 4)
+                if (rows > 192) return of(std::integral_constant<int, 4>{});
+            if constexpr (XS == 4)
+                if (rows > 128) return of(std::integral_constant<int, 3>{});
+            if constexpr (XS >= 2)
+                if (rows > 64) return of(std::integral_constant<int, 2>{});
+            of(std::integral_constant<int, 1>{});
         };
         if (half) {
             if (ONCE && once) all(std::true_type{}, std::bool_constant<ONCE>{});
@@ -541,13 +568,13 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
 
 // A workgroup per CU, or two for every item where these are fewer (each a half of its columns).
 inline bool wide_fits(int K, int N, bool gated) { return K > 0 && K % 64 == 0 && N % (gated ? 128 : 256) == 0; }
-template <int KIND, int ACT = SKYRL_ACT_SILU, bool ONCE = false>
+template <int KIND, int ACT = SKYRL_ACT_SILU, bool ONCE = false, int TM = 256>
 int launch_wide(Wide p, hipStream_t s) {
     set_division(p);
     const int64_t items = (int64_t)(KIND == kDense ? (p.N + 255) / 256 : p.N / (KIND == kDown ? 256 : 128)) * p.ntiles;
     SKYRL_REQUIRE(items < (1ll << 31) && p.ntiles < (1 << 23), "wide products: too many rows in one call");
     const unsigned grid = (unsigned)(items > kCUs / 2 ? kCUs : (2 * items + 7) / 8 * 8);
-    hipLaunchKernelGGL((wide_kernel<KIND, ACT, ONCE>), dim3(grid), dim3(256), 0, s, p);
+    hipLaunchKernelGGL((wide_kernel<KIND, ACT, ONCE, TM>), dim3(grid), dim3(256), 0, s, p);
     return check_launch("wide_kernel");
 }
 

@@ -1440,9 +1440,15 @@ def moe_tile(sh, n: int) -> int:
 
 
 def moe_rows(sh, n: int) -> int:
-    """moe_tile, but 32 where an expert has about one tile of that: its weights are then streamed once, which tiles of 64 half
-    filled do more slowly (128 tokens, 8 of 64 experts of 768 x 2048: 115 against 128 us)."""
-    return 32 if 12 * sh.experts <= n * sh.top < 24 * sh.experts else moe_tile(sh, n)
+    """moe_tile, but 32 from 12 to 24 rows an expert, where it has about one tile of that and its weights are streamed once. Where the
+    wide form takes both products, to 18 at widths from 2048, and 128 already from 48 rows. 8 of 64 experts, both products, us, tiles of 32 /
+    64: 768 x 2048, 128 tokens 102 / 99, 160 tokens 107 / 100; 1536 x 4096, 160 tokens 387 / 386; 384 x 1024 33.1 / 34.5; of 64 / 128:
+    768 x 2048, 350 tokens 106 / 108, 400 tokens 118 / 110; 1536 x 4096, 450 tokens 429 / 415; 384 x 1024 39.4 / 36.4."""
+    wide = sh.ff % 128 == 0 and sh.width % 256 == 0
+    mean = n * sh.top / sh.experts
+    if 12 <= mean < (18 if wide and sh.width >= 2048 else 24):
+        return 32
+    return 128 if wide and 48 <= mean < 60 else moe_tile(sh, n)
 
 
 def moe_sort(sh, idx, tm: int):

@@ -522,6 +522,23 @@ def test_wide_tiles_in_rounds(width, ff, experts, n):
         assert torch.equal(lk.moe_experts(sh, x, idx, weight, wgu, wd, tm=256), want)
 
 
+@pytest.mark.parametrize("width", [64, 128, 192, 256, 320, 384, 512, 768])
+def test_small_wide_tiles(width):
+    """Tiles of 64 and 128 in the wide form, depths from one stage to more than the ring holds (an item on its own, the shortest that
+    are chained), several items a workgroup, experts of no row to many: the rows that the staged form's tiles of 16 give, every time."""
+    g = torch.Generator(device=DEV).manual_seed(width)
+    experts, ff, n = 48, 640, 6500
+    sh = lk.moe_shape(width, ff, experts, 1)
+    mk = lambda *s, scale=1.0: (torch.randn(s, generator=g, device=DEV) * scale).to(BF16)  # noqa: E731
+    x, wgu, wd = mk(n, width), mk(experts, 2, ff, width, scale=0.05), mk(experts, width, ff, scale=0.05)
+    loads = torch.rand(experts, generator=g, device=DEV) ** 3
+    idx = torch.multinomial(loads, n, replacement=True, generator=g).int().view(n, 1)
+    weight = torch.rand(n, 1, generator=g, device=DEV) + 0.2
+    want = lk.moe_experts(sh, x, idx, weight, wgu, wd, tm=16)
+    for tm in (64, 128, 64, 128):
+        assert torch.equal(lk.moe_experts(sh, x, idx, weight, wgu, wd, tm=tm), want)
+
+
 @pytest.mark.parametrize("n", (64, 200, 700))
 def test_experts_with_one_tile_beside_such_with_several(n):
     """Matrices of 67 and 34 MB, whose weights go past the caches where an expert has one tile: loads from nothing to all tokens an
