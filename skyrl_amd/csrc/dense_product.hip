@@ -146,7 +146,7 @@ void launch_dense(const Dense& p, hipStream_t s) {
     hipLaunchKernelGGL((dense_kernel<TM, TN, S>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(256), 0, s, p);
 }
 
-enum Form { k64x32, k64x64, k64x128, k128x128, kWide192, kWide256 };
+enum Form { kOnce, k64x32, k64x64, k64x128, k128x128, kWide192, kWide256 };
 int64_t tiles_of(int n, int N, int tm, int tn) { return (int64_t)((n + tm - 1) / tm) * ((N + tn - 1) / tn); }
 
 // Rounds of whole tiles of 256 that the wide form with tiles of `rows` takes, in hundredths: a tile of 192 is 82 of them, half of
@@ -171,10 +171,19 @@ int64_t wide_rounds(int n, int N, int rows) {
 //   3072, 768       6.1 / 8.6      8.1 / 10.5     -              -              -             31 / 47       38 / 46
 //   2048, 512       4.7 / 6.8      5.5 / 8.6      7.0 / 9.7      9.3 / 11.4     12.8 / 14.2   17.5 / 27.9   21.5 / 23.2
 //   24640, 4096     -              -              -              267 / 374      456 / 515     837 / 929     1149 / 1218
+// One tile of 128 or 256 rows and columns for the whole chip (logits): the wide form, in which weights go past the caches and neighbouring
+// columns begin at another depth (wide.h's depth_start; with several tiles of rows they would read x at as many depths):
+//   N, K            65 rows       128           256
+//   32768, 2048     28.2 / 37.6   30.4 / 40.5   42.3 / 46.2
+//   28672, 2048     -             28.7 / 34.2   42.0 / 45.3   (192 pieces of 128 columns of 4096 deep: 60.0 / 57.4, 84.8 / 72.0)
+//   40000, 2048     -             40.6 / 51.2   54.5 / 59.5
+//   65536, 4096     -             -             121 / 162
+//   151936, 2048    -             124 / 175     161 / 219
 // Where the library stays, us, the same: 1563 x 2048, 3408 28.7 / 30.4; 3000 x 2048, 2048 29.1 / 27.9; 8192 x
 // 2048, 2048 53 / 51; 1300 x 6144, 2048 50.6 / 39.0; 512 x 2048, 12352 40.7 / 35.4; 2048 x 2048, 32768 216 / 200.
 Form form_of(int n, int K, int N, bool& faster) {
     faster = true;
+    if (n > 64 && n <= 256 && N >= 28672) return kOnce;
     if (n <= 1400 && K <= 6144 && (n <= 1024 || K <= 2048)) {
         if (tiles_of(n, N, 64, 32) <= kCUs) return k64x32;
         if (tiles_of(n, N, 64, 64) <= kCUs) return k64x64;
@@ -215,6 +224,8 @@ extern "C" int skyrl_dense_product(const void* x, int64_t ldx, int32_t n, int32_
     bool faster;
     const Form form = form_of(n, K, N, faster);
     SKYRL_REQUIRE(tiles_of(n, N, 64, 32) < (1ll << 30), "dense_product: too many rows in one call");
+    const Wide one{x_, w_, o_, K, N, ldx, ldw, 1, nullptr, nullptr, 1, 0, 0, nullptr, n, n <= 128 ? 128 : 256, Gate{}};
+    if (form == kOnce) return n <= 128 ? launch_wide<kDense, SKYRL_ACT_SILU, true, 128>(one, s) : launch_wide<kDense, SKYRL_ACT_SILU, true>(one, s);
     if (form == k64x32) launch_dense<64, 32, 6>(d, s);
     else if (form == k64x64) launch_dense<64, 64, 4>(d, s);
     else if (form == k64x128) launch_dense<64, 128, 3>(d, s);

@@ -29,8 +29,9 @@ __device__ __forceinline__ void lds_write(uint32_t at, uint2 v) {
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t whole_buffer(const void* p) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, 0xffffffff, 0x00027000);
 }
+template <int POLICY = 0>
 __device__ __forceinline__ void buffer_to_lds(__amdgpu_buffer_rsrc_t all, uint32_t own, int offset, uint32_t to) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(all, (lds_void*)(uintptr_t)to, 16, own, offset, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(all, (lds_void*)(uintptr_t)to, 16, own, offset, 0, POLICY);
 }
 // 16 bytes from the lanes whose row is not negative, without a way round the store. NT: past the caches, with the weights (64 experts
 // of 768 x 2048, gate_up / down, us: 800 tokens 76 / 48 -> 70 / 45, 1563 tokens 93 / 58 -> 91 / 55; with weights that stay, 5637 tokens 239 /
@@ -122,7 +123,8 @@ __device__ __forceinline__ int32_t uniform(const int32_t* p) {
 // step, and at a row stride of 4 KB the same depth of all rows lies in the same few of the memory's channels: weights from HBM
 // came at 5.2 TB/s where all experts began at 0, at 6.2 where each begins elsewhere (64 experts of 768 x 2048, gate_up, us: 256 tokens
 // 79 -> 63, 700 tokens in tiles of 128 90 -> 75; down, rows of 1536 bytes, 40.7 -> 39.4). One start for an expert: its tiles, and
-// a tile's columns, share what they read (a start for each column: 5637 tokens 265 us, 243 with this).
+// a tile's columns, share what they read (a start for each column: 5637 tokens 265 us, 243 with this). kDense with ONCE, where all
+// columns read the same few rows: a start for each 128 columns.
 __device__ __forceinline__ int depth_start(int e, int K) {
     return K % 256 == 0 ? (int)__umulhi((uint32_t)e * 0x9E3779B9u, (uint32_t)K / 64) : 0;
 }
@@ -148,6 +150,7 @@ __device__ __forceinline__ bool one_tile(const int32_t* tile_expert, int tile, i
 // pairs per expert: a sixth of the rows is padding), their loads are not: tiles of 64 and 128 where most experts have no more. The depth is a multiple of 64, the columns of the item's.
 //   kGateUp, kDown  routed experts (moe.hip): rows by the pairs' order. kGateUp takes a row of x per token and leaves one per
 //                   place, silu(gate) up; kDown takes one per place and leaves one per pair, weighted.
+// kDense with ONCE: the weights of one tile of rows, all past the caches.
 //   kGated, kDense  one matrix, x and the output row by row in tiles of tile_rows (gated_product.hip): of N gate and N up rows,
 //                   any activation; of N rows, a multiple of 8, as they are.
 // Bound: the products at the power limit (weights of zeros: 8192 x 2048, 6144 gated in 226 us, random ones in 297, 1.39 PFLOP/s, the
@@ -233,14 +236,15 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
     int64_t wslot[4] = {};  // what a slot's rows of w are past the item's first; those of a half are the first slots'
     auto wrap = [](uint32_t at) { return min(at, at - RING * SLOT); };  // of less than two rings
     int k_start = 0;        // of the item whose loads are under way
-    auto depth = [&](int k) { return ROUTED && k + k_start >= p.K ? k + k_start - p.K : k + k_start; };
+    auto depth = [&](int k) { return (ROUTED || ONCE) && k + k_start >= p.K ? k + k_start - p.K : k + k_start; };
     auto fetch = [&](auto nt, int k0, uint32_t base, int i) __attribute__((always_inline)) {  // load i at depth k0 of the stage at base
         const bool is_w = WF ? i < LW : i >= LX;
         const int u = WF ? (is_w ? i : i - LW) : is_w ? i - LX : i;
         const uint32_t to = lds0 + wrap(base + i / 2 * SLOT + wave * (SLOT / 4)) + u % 2 * (SLOT / 8);
         lds_void* dst = (lds_void*)(uintptr_t)to;
         if constexpr (KIND == kDense) {
-            buffer_to_lds(is_w ? w_all : x_all, is_w ? wo[u] : xo[u], k0 * 2, to);
+            if (nt.value && is_w) buffer_to_lds<2>(w_all, wo[u], k0 * 2, to);
+            else buffer_to_lds(is_w ? w_all : x_all, is_w ? wo[u] : xo[u], k0 * 2, to);
         } else {
             const uint16_t* src = is_w ? ws[u % 2] + (k0 + wslot[u / 2]) : GATHER ? xs[u] + k0 : xs[u % 2] + (k0 + u / 2 * 64 * p.ldx);
             if (nt.value && is_w) __builtin_amdgcn_global_load_lds((gbl_void*)src, dst, 16, 0, 2);
@@ -270,7 +274,7 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) wslot[j] = ((j * 64 ^ flip) + (GATED && j >= 2 ? p.N - OC : 0)) * p.ldw;
         }
-        if constexpr (ROUTED) k_start = depth_start(next_e, p.K) * BK;
+        if constexpr (ROUTED || ONCE) k_start = depth_start(ROUTED ? next_e : next_n0 / (OC / 2) + (next_half == 2), p.K) * BK;
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         asm volatile("" : "+v"(pair));
         if constexpr (!ROUTED) {
@@ -305,7 +309,7 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
     auto turned = [&]() __attribute__((always_inline)) {  // the item's output and tile
         tile = next_tile, half = next_half;
         n0 = next_n0 + (half == 2 ? OC / 2 : 0);
-        once = ONCE && e_before != next_e && e_after != next_e;
+        once = ONCE && (!ROUTED || (e_before != next_e && e_after != next_e));
     };
     const bool chain = nk > 2 * AHEAD - 2;  // an item's last steps load the next one's first stages; its rows have landed then
     uint32_t b0 = 0;            // where the next stage starts in the ring
@@ -518,7 +522,7 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
                     on = in ? rows - 1 - r : -1;
                     to_row = own + r;
                 }
-                store_row<ONCE>(to + to_row * p.N, y[m & 1][k], on);
+                store_row<ONCE && ROUTED>(to + to_row * p.N, y[m & 1][k], on);
             }
         };
         put(0);

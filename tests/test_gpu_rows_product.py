@@ -85,10 +85,18 @@ def test_dense(dev, n, N, K, pad):
         assert y.shape == (n, N) and bool(((y.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2 * off).all())
 
 
+@pytest.mark.parametrize("n,N,K", [(65, 28672, 64), (100, 28680, 320), (128, 30000, 256), (129, 28672, 512), (256, 66056, 128), (200, 28680, 768)])
+def test_dense_one_tile_of_rows(dev, n, N, K):
+    """One tile of 128 or 256 rows, halves of items and whole ones, depths with a start for each column and without."""
+    test_dense(dev, n, N, K, 24)
+    x, w, _ = _data(dev, n, N, K, n)
+    assert lk._dense_fit(x, w) and torch.equal(lk._dense(x, w), lk._dense(x, w))
+
+
 def test_many_rows_take_the_faster_form(dev):
     for n, N, K, own in ((65, 2048, 2048, True), (256, 2048, 2048, True), (256, 3408, 2048, True), (1024, 12352, 2048, True), (5637, 12352, 2048, True),
                          (5637, 3072, 768, True), (2048, 5824, 512, True), (1563, 2048, 2048, True), (3000, 2048, 2048, False), (8192, 2048, 2048, False),
-                         (8192, 2048, 6144, False), (256, 32768, 2048, False), (300, 4096, 12288, False), (300, 2044, 2048, False),
+                         (8192, 2048, 6144, False), (256, 32768, 2048, True), (300, 4096, 12288, False), (300, 2044, 2048, False),
                          (300, 2048, 2056, False)):
         x, w, b = _data(dev, n, N, K, 0)
         assert lk._dense_fit(x, w) == own, (n, N, K)
