@@ -4,11 +4,18 @@
 
 using namespace skyrl;
 
-// Where it is the faster one: from three quarters of a round of workgroups on. Against the library's product and gate_mul, us,
-// n x K rows and N: 8192 x 2048, 6144: 321 against 366; 6000: 255, 345; 4096: 166, 189; 1024: 51, 59; 512 (96 items): 49, 39.
-// 3000 x 4096, 12288: 469, 614; 512: 87, 96; 384: 83, 81. 4096 x 1536, 8960: 204, 231; 512: 37, 45.
+// Where it is the faster one. From 512 rows, by tiles of 256, from three quarters of a round of workgroups on. Against the library's
+// product and gate_mul, us, n x K rows and N: 8192 x 2048, 6144: 297 against 366; 1024: 51, 59; 512 (96 items): 49, 39. 3000 x 4096, 12288:
+// 469, 614; 512: 87, 96; 384: 83, 81. 4096 x 1536, 8960: 204, 231; 512: 37, 45.
+// Below, by tiles of 64 in one round, against dense_product's and gate_mul, weights from HBM: 128 x 2048, 6144: 21.6 against 25.2; 128, 256, 400, 511 x
+// 1536, 4608: 13, 18, 20, 27 against 15, 22, 29, 30; 256 x 1536, 8960: 34, 37. Not 192 x 2048, 6144: 28.7, 27.9; 256 x 2048, 2048:
+// 14.6, 13.6; 128 x 4096, 12288: 65, 61.
+static bool few_rows(int32_t n, int32_t K, int32_t N) {
+    return n > 64 && n < 512 && K <= (n <= 128 ? 2048 : 1536) && N >= 4096 && (int64_t)((n + 63) / 64) * (N / 128) <= kCUs * 9 / 8;
+}
 extern "C" int32_t skyrl_gated_product_fits(int32_t n, int32_t K, int32_t N) {
-    return n >= 512 && N > 0 && wide_fits(K, N, true) && (int64_t)((n + 255) / 256) * (N / 128) >= kCUs * 3 / 4;
+    if (N <= 0 || !wide_fits(K, N, true)) return 0;
+    return few_rows(n, K, N) || (n >= 512 && (int64_t)((n + 255) / 256) * (N / 128) >= kCUs * 3 / 4);
 }
 
 extern "C" int skyrl_gated_product(const void* x, int64_t ldx, int32_t n, int32_t K, const void* w, int64_t ldw, int32_t N,
@@ -18,9 +25,14 @@ extern "C" int skyrl_gated_product(const void* x, int64_t ldx, int32_t n, int32_
     SKYRL_REQUIRE(act == SKYRL_ACT_SILU || act == SKYRL_ACT_GELU_TANH || act == SKYRL_ACT_CLAMPED, "gated_product: act");
     SKYRL_REQUIRE(aligned16(x) && aligned16(w) && aligned16(out) && ldx % 8 == 0 && ldw % 8 == 0 && ldw >= K && (n == 1 || ldx >= K),
                   "gated_product: rows must be 16-byte aligned");
+    const int rows = few_rows(n, K, N) ? 64 : 256;
     const Wide p{reinterpret_cast<const uint16_t*>(x), reinterpret_cast<const uint16_t*>(w), reinterpret_cast<uint16_t*>(out), K, N,
-                 ldx, ldw, (n + 255) / 256, nullptr, nullptr, 1, 0, 0, nullptr, n, 256, Gate{act, alpha, limit}};
-    if (act == SKYRL_ACT_SILU) return launch_wide<kGated, SKYRL_ACT_SILU>(p, as_stream(stream));
-    if (act == SKYRL_ACT_CLAMPED) return launch_wide<kGated, SKYRL_ACT_CLAMPED>(p, as_stream(stream));
-    return launch_wide<kGated, SKYRL_ACT_GELU_TANH>(p, as_stream(stream));
+                 ldx, ldw, (n + rows - 1) / rows, nullptr, nullptr, 1, 0, 0, nullptr, n, rows, Gate{act, alpha, limit}};
+    auto launch = [&](auto a) {
+        if (rows == 64) return launch_wide<kGated, a, false, 64>(p, as_stream(stream));
+        return launch_wide<kGated, a>(p, as_stream(stream));
+    };
+    if (act == SKYRL_ACT_SILU) return launch(std::integral_constant<int, SKYRL_ACT_SILU>{});
+    if (act == SKYRL_ACT_CLAMPED) return launch(std::integral_constant<int, SKYRL_ACT_CLAMPED>{});
+    return launch(std::integral_constant<int, SKYRL_ACT_GELU_TANH>{});
 }

@@ -379,7 +379,7 @@ def gated_linear(x: torch.Tensor, w: torch.Tensor, act: str, alpha: float = 1.0,
             return y
         x = x.rows()
     (n, K), N = x.shape, w.shape[0] // 2
-    many = (n > MAX_ROWS and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.is_cuda
+    many = (n > ROUNDED_ROWS and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.is_cuda
             and bool(_ffi.query("skyrl_gated_product_fits", n, K, N)) and _rows_aligned(x, w))
     if w.shape[0] % 2 or not (many or _rows_fit(x, w, True)):
         return None

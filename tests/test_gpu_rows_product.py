@@ -64,6 +64,14 @@ def test_gated(dev, n, N, K, act):
     assert bool(((y.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2 * slack + 1e-5 * (g * u).abs() + 1e-6).all())
 
 
+@pytest.mark.parametrize("n,N,K", [(65, 4096, 64), (128, 6144, 2048), (129, 4096, 256), (256, 8960, 320), (511, 4608, 384), (448, 4608, 1536)])
+def test_gated_small_tiles(dev, n, N, K):
+    """Tiles of 64 rows: one stage an item, fewer than are under way and more, items on their own and several a workgroup."""
+    assert lk._ffi.query("skyrl_gated_product_fits", n, K, N)
+    test_gated(dev, n, N, K, "silu")
+    test_gated(dev, n, N, K, "gelu_tanh")
+
+
 @pytest.mark.parametrize("n,N,K", [(2113, 4096, 64), (2300, 6400, 128), (2113, 4096, 192), (2300, 6400, 256), (4161, 3968, 320)])
 def test_gated_in_rounds(dev, n, N, K):
     """One to five stages an item, a second round of whole items and one of halves, a last tile of 65, 252 and 65 rows."""
