@@ -50,7 +50,7 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kMaxSplitRows = 1024;  // split mode is never used at or above this many rows
-// Workspace: a fixed-size region of per-row arrival counters first (only split mode uses them),
+// Workspace: a fixed-size region of per-row arrival counters first (split mode and top_p rows in pieces use them),
 // so that the counters sit at the same place for every batch size and never overlap another
 // call's row filters or partials in a reused workspace (a split-mode call after one with fewer
 // rows would otherwise read that call's partials as counters): every counter is zero at

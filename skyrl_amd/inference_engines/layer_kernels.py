@@ -1427,9 +1427,11 @@ def moe_one(sh, logits, column: int, correction, x, gate_up, down) -> Optional[t
 
 def moe_tile(sh, n: int) -> int:
     """Rows per tile of the experts' products for n tokens: 64 from 12 rows an expert, 128 from 48, 256 from 112. Both products of 64
-    experts, 8 a token, us, loads even / a third / two thirds apart:
-    128 from 60 at widths of 1536 to 2048 (tiles of 64 against 128: 768 x 2048, 448 tokens 143 / 161 / 140 against 160 / 163 / 137, 512
-    169 / 169 / 155, 163 / 167 / 152; but 384 x 1024, 384 tokens 44 / 50 / 46, 43 / 43 / 42; 1536 x 4096 441 / 511 / 464, 485 / 486 / 445).
+    experts, 8 a token, us:
+    Where the wide form takes both, tiles of 128 against 256: 768 x 2048, 700 tokens 128 / 137, 900 132 / 133, 1000 143 / 135; 1536 x 4096, 700
+    tokens 435 / 467, 900 475 / 463; 384 x 1024 41 / 45, 44 / 45, 1100 tokens 54 / 46. moe_rows has the line between 64 and 128.
+    Where it takes the second alone: 128 from 60 at widths of 1536 to 2048 (loads even / a third / two thirds apart, staged tiles of 64 against
+    128: 448 tokens 143 / 161 / 140 against 160 / 163 / 137, 512 169 / 169 / 155, 163 / 167 / 152).
     256 from 136 below 2048 where a quarter of the wide form's columns would be none and 256 rows are staged (128 against 256: 576 x
     1536, 1024 tokens 126 / 122 / 117, 135 / 136 / 132, 1200 tokens 146 / 142 / 120, 137 / 137 / 133; but 704 x 2048, 1024 tokens
     192 / 200 / 187, 174 / 189 / 186; 1472 x 4096, 896 tokens 584 / 647 / 582, 574 / 575 / 572)."""
