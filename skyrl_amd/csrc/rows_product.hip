@@ -11,11 +11,12 @@
 //   2048, 2048      3.9 / 10.9       4.1 / 11.0       4.4 / 11.2       5.5 / 11.7
 //   2048, 6144      6.9 / 11.1       7.2 / 11.2       7.5 / 16.5       9.6 / 19.4
 //   3648, 2048      4.8 / 11.8       5.5 / 11.7       6.5 / 11.6       8.4 / 12.1   (no splits)
-//   12288, 2048     11.5 / 16.6      10.9 / 15.2      12.3 / 15.2      16.7 / 16.3  (no splits; 4.4 TB/s at one row)
+//   12288, 2048     11.5 / 16.6      11.8 / 15.2      12.7 / 15.2      15.5 / 16.3  (no splits; 4.4 TB/s at one row)
 //   24576, 2048     20.6 / 40.0      21.7 / 40.1      23.6 / 29.3      29.7 / 30.2  (gated: 12288 pairs of rows)
 //   32768, 2048     24.1 / 35.1      24.6 / 32.9      27.5 / 35.3      27.9 / 35.7  (no splits; 5.6 TB/s at one row)
-// At 64 rows a workgroup's x is as many bytes as its weights, over the same 64 bytes a clock into LDS: 12288 x 2048 gated takes
-// 16.4 us, 13.4 without x, 7.3 without the weights, 5.3 without either; leaving out the products changes it by 0.4.
+// At 64 rows a workgroup's x is as many bytes as its weights, over the same 64 bytes a clock into LDS: 12288 x 2048 gated took,
+// in 192 workgroups of 64 rows of weights, 16.4 us, 13.4 without x, 7.3 without the weights, 5.3 without either; leaving out the products
+// changed it by 0.4. In 256 of 48 it takes 15.0.
 // Batches (a head's up-projections of latent attention, 512 x 128 and 128 x 512): 16 heads, 1 / 64 rows, both products with the
 // copy that the library's needed: 15.4 / 17.1 us, here 5.9 / 7.6 us.
 #include "rows.h"
@@ -75,44 +76,72 @@ void launch_rows(RowsProduct p, int splits, hipStream_t s, int batch = 1) {
                        dim3(WK * kWave), 0, s, p);
 }
 
-// Up to 16 rows of x, 16 rows of weights a workgroup up to 512 workgroups of these, 64 up to one workgroup a CU, then 32; us at
+// From 17 rows of x on, the fewest rows of weights a workgroup of which one a CU holds all: 16 (rounded ones), 32 (with gated ones both
+// matrices'), 48, else 64. With more, CUs stood idle: 6144 pairs are 192 workgroups of 64 and 256 of 48. us at 32 / 64 rows of x with 64 rows of weights, 48, 32:
+//   768 pairs x 2048     10.2 / 13.3   9.1 / 11.9    8.3 / 9.6
+//   4096 pairs x 2048    12.7 / 15.9   11.8 / 14.8   10.5 / 12.4
+//   6144 pairs x 2048    14.1 / 16.3   12.9 / 15.0   15.4 / 19.7
+//   6144 pairs x 4096    23.8 / 29.4   21.5 / 26.3   26.7 / -
+//   8192 x 2048          12.7 / 16.6   11.6 / 14.7   9.9 / 13.3
+//   12288 x 2048         14.4 / 17.6   12.8 / 16.7   15.1 / 19.8
+//   12352 x 2048         14.2 / 18.0   16.6 / 19.4   15.2 / -   (64 rows of x with four waves for two, up to one workgroup a CU: 15.6)
+// with 16 rows of weights and 32: 2048 x 2048 64 rows 8.4, 9.6; 4608 x 2048 10.4 / 13.7, 9.2 / 10.4; 8184 x 2048 64 rows 15.2, 12.4.
+// Four waves share the depth, two where 64 rows of x take several rounds of 64 rows of weights.
+int weight_tiles(int rows) { return rows <= 16 * kFill ? 1 : rows <= 32 * kFill ? 2 : rows <= 48 * kFill ? 3 : 4; }
+
+// Up to 16 rows of x, 16 rows of weights a workgroup up to 512 workgroups of these, 48 or 64 up to one workgroup a CU, then 32; us at
 // 1 / 16 rows of x with 16, 32 and 64 rows of weights:
 //   8192 x 2048    7.5 / 8.4     7.7 / 8.0     8.7 / 9.6
 //   8192 x 4096    13.3 / 14.9   13.8 / 14.3   16.9 / 19.2
 //   10240 x 2048   9.9 / 11.2    10.1 / 11.5   9.5 / 10.2
+//   12288 x 2048   -             -             11.8 / 12.4  (48 rows: 11.4 / 11.8)
 //   16640 x 2048   15.6 / 16.1   15.6 / 16.0   17.5 / 18.3
 //   24576 x 4096   34.1 / 38.1   34.2 / 35.0   37.1 / 40.0
 template <int MODE>
 void launch_rounded(const RowsProduct& p, hipStream_t s) {
+    const int nt = weight_tiles(p.N);
     if (p.n <= 16) {
         if (p.N <= kWide) launch_rows<MODE, 1, 1, 4, 4>(p, 1, s);
+        else if (nt == 3) launch_rows<MODE, 3, 1, 4, 2>(p, 1, s);
         else if (p.N <= 2 * kWide) launch_rows<MODE, 4, 1, 4, 2>(p, 1, s);
         else launch_rows<MODE, 2, 1, 4, 2>(p, 1, s);
-    } else if (p.N >= kWide) {
-        if (p.n <= 32) launch_rows<MODE, 4, 2, 4, 2>(p, 1, s);
-        else launch_rows<MODE, 4, 4, 2, 2>(p, 1, s);
+    } else if (p.n <= 32) {
+        if (nt == 1) launch_rows<MODE, 1, 2, 4, 3>(p, 1, s);
+        else if (nt == 2) launch_rows<MODE, 2, 2, 4, 2>(p, 1, s);
+        else if (nt == 3) launch_rows<MODE, 3, 2, 4, 2>(p, 1, s);
+        else launch_rows<MODE, 4, 2, 4, 2>(p, 1, s);
     } else {
-        if (p.n <= 32) launch_rows<MODE, 1, 2, 4, 3>(p, 1, s);
-        else launch_rows<MODE, 1, 4, 4, 2>(p, 1, s);
+        if (nt == 1) launch_rows<MODE, 1, 4, 4, 2>(p, 1, s);
+        else if (nt == 2) launch_rows<MODE, 2, 4, 4, 2>(p, 1, s);
+        else if (nt == 3) launch_rows<MODE, 3, 4, 4, 2>(p, 1, s);
+        else if (p.N <= 64 * kFill) launch_rows<MODE, 4, 4, 4, 2>(p, 1, s);
+        else launch_rows<MODE, 4, 4, 2, 2>(p, 1, s);
     }
 }
 
 // Gated, a pair of rows is two rows of weights. Up to 16 rows of x, 32 rows of weights, but 64 where 32 were more than one workgroup
-// a CU and 64 are not, unless the depth makes up for it; us at 1 / 16 rows of x with 32 and 64 rows of weights:
+// a CU and 64 are not, unless the depth makes up for it, or 48 where these are (4608 pairs x 1536, one row: 9.4 -> 8.6); us at 1 / 16 rows of x with 32 and 64 rows of weights:
 //   2048 pairs x 2048    6.1 / 7.0     9.5 / 9.9
 //   4096 pairs x 2048    8.7 / 8.3     11.1 / 10.2
 //   6144 pairs x 2048    12.2 / 12.3   11.7 / 11.1
 //   6144 pairs x 4096    20.4 / 23.3   24.7 / 25.1
 //   12288 pairs x 2048   19.4 / 20.0   20.6 / 21.4
-// At 33 to 64 rows of x two waves, two workgroups a CU, where these are one round and four waves would be two; us at 64 rows with two
+// Above, weight_tiles. At 33 to 64 rows of x and 64 rows of weights two waves, two workgroups a CU, where these are one round and four waves would be two; us at 64 rows with two
 // and four waves: 6144 x 2048 17.9, 15.7; 8448 x 2048 25.0, 27.4; 16384 x 2048 30.0, 33.0; 24576 x 2048 53.2, 47.7.
 void launch_gated(const RowsProduct& p, hipStream_t s) {
-    const int tiles = (p.N + 31) / 32;  // of 64 rows
+    const int tiles = (p.N + 31) / 32, nt = weight_tiles(2 * p.N);  // of 64 rows
     if (p.n <= 16) {
-        if (tiles > kFill / 2 && tiles <= kFill && p.K <= 3072) launch_rows<kGated, 4, 1, 2, 4>(p, 1, s);
+        if (nt == 3 && p.K <= 3072) launch_rows<kGated, 3, 1, 4, 3>(p, 1, s);
+        else if (tiles > kFill / 2 && tiles <= kFill && p.K <= 3072) launch_rows<kGated, 4, 1, 2, 4>(p, 1, s);
         else launch_rows<kGated, 2, 1, 4, 3>(p, 1, s);
     } else if (p.n <= 32) {
-        launch_rows<kGated, 4, 2, 4, 2>(p, 1, s);
+        if (nt <= 2) launch_rows<kGated, 2, 2, 4, 2>(p, 1, s);
+        else if (nt == 3) launch_rows<kGated, 3, 2, 4, 2>(p, 1, s);
+        else launch_rows<kGated, 4, 2, 4, 2>(p, 1, s);
+    } else if (nt <= 2) {
+        launch_rows<kGated, 2, 4, 4, 2>(p, 1, s);
+    } else if (nt == 3) {
+        launch_rows<kGated, 3, 4, 4, 2>(p, 1, s);
     } else if (tiles > kFill && tiles <= 2 * kFill) {
         launch_rows<kGated, 4, 4, 2, 2>(p, 1, s);
     } else {

@@ -72,6 +72,17 @@ def test_gated_small_tiles(dev, n, N, K):
     test_gated(dev, n, N, K, "gelu_tanh")
 
 
+@pytest.mark.parametrize("N", [4096, 4100, 8192, 8196, 12288, 12292, 16384, 16388])
+@pytest.mark.parametrize("n,K", [(16, 264), (17, 136), (32, 520), (33, 264), (64, 1032)])
+def test_rows_of_weights_a_workgroup(dev, n, N, K):
+    """Both sides of each number of weight rows a workgroup, 16 to 64: rounded, capped, and gated pairs of as many rows."""
+    test_products(dev, n, N, K, 24)
+    test_gated(dev, n, N // 2, K, "silu")
+    x, w, _ = _data(dev, n, N, K, n, 24)
+    y = lk.linear(x, w).float()
+    assert torch.allclose(lk.capped_linear(x, w, 3.0), 3.0 * torch.tanh(y / 3.0), rtol=2e-6, atol=1e-6)  # of the rounded product, in f32
+
+
 @pytest.mark.parametrize("n,N,K", [(2113, 4096, 64), (2300, 6400, 128), (2113, 4096, 192), (2300, 6400, 256), (4161, 3968, 320)])
 def test_gated_in_rounds(dev, n, N, K):
     """One to five stages an item, a second round of whole items and one of halves, a last tile of 65, 252 and 65 rows."""
