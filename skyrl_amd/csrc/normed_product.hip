@@ -331,6 +331,9 @@ __global__ __launch_bounds__(2 * kNT) void normed_product_kernel(RowsProduct p, 
 }
 
 constexpr int kWideCols = 8192;  // as in rows_product.hip
+// Pairs up to which 48 rows of weights a workgroup are at most one a CU: 64 leave CUs idle (6144 x 2048, of a step of one row 214.9 ->
+// 213.9 us with four such products; rounded ones of 8192 to 12288 columns: no change).
+constexpr int kPairs = 24 * 256;
 
 template <int LONG, class Pre>
 void launch(const RowsProduct& p, const Pre& pre, bool gate, int splits, hipStream_t s) {
@@ -338,7 +341,10 @@ void launch(const RowsProduct& p, const Pre& pre, bool gate, int splits, hipStre
     hipLaunchKernelGGL((normed_product_kernel<MODE, NT, S, LONG, Pre>), dim3((p.N + out_cols<MODE, NT>() - 1) / out_cols<MODE, NT>(), \
                        splits ? splits : 1), dim3(2 * kNT), 0, s, p, pre)
     if (gate) {
-        if constexpr (Pre::kBeforeGated) LAUNCH(kGated, 4, 4);
+        if constexpr (Pre::kBeforeGated) {
+            if (p.N <= kPairs) LAUNCH(kGated, 3, 5);
+            else LAUNCH(kGated, 4, 4);
+        }
     } else if (splits) {
         if constexpr (Pre::kBeforeParts) LAUNCH(kParts, 1, 4);
     } else if (p.N >= kWideCols) LAUNCH(kRound, 4, 4);

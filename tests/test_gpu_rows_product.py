@@ -279,6 +279,30 @@ def test_rings_are_refilled(dev, form, n, N, K, waves, slots):
         assert bool(((y - z).abs() <= 2.0 ** -8 * z.abs() + 2 * off + 1e-5).all())
 
 
+@pytest.mark.parametrize("form,n,N", [("rounded", 33, 5000), ("rounded", 50, 8200), ("rounded", 64, 12296), ("rounded", 32, 8200), ("rounded", 17, 5000),
+                                      ("rounded", 9, 12288), ("gated", 33, 4096), ("gated", 64, 6144), ("gated", 20, 2056), ("gated", 32, 6144),
+                                      ("gated", 16, 6144)])
+def test_rings_of_other_widths_are_refilled(dev, form, n, N):
+    test_rings_are_refilled(dev, form, n, N, 2040, 4, 3 if form == "gated" and n <= 16 else 2)
+
+
+@pytest.mark.parametrize("pairs", [100, 6144, 6148])
+def test_gated_of_a_normed_row(dev, pairs):
+    """Both sides of the number of weight rows a workgroup: the product of the norm's row, launched alone."""
+    g = torch.Generator(device=dev).manual_seed(pairs)
+    r = lambda *s: torch.randn(*s, device=dev, generator=g)  # noqa: E731
+    w = (r(2 * pairs, 2048) * 0.02).bfloat16()
+    delta, h, weight = r(4, 1, 2048), r(1, 2048), r(2048).bfloat16()
+    rows = [lk.normed(delta, h, weight, 1e-5) for _ in range(3)]  # h is read: the residual leaves in another buffer
+    y = [lk.gated_linear(row, w, "silu") for row in rows]
+    row = rows[0]
+    x = lk.rows_of(row)
+    z, off = _bounds(x, w)
+    a, u = z[:, :pairs], z[:, pairs:]
+    slack = 1.2 * off[:, :pairs] * (u.abs() + 1) + (a.abs() + 1) * off[:, pairs:]
+    assert all(torch.equal(y[0], t) for t in y) and bool(((y[0].double() - a * torch.sigmoid(a) * u).abs() <= 2.0 ** -8 * (a * u).abs() + 2 * slack + 1e-5).all())
+
+
 def _close(y, x, w, want=None):
     ref, off = _bounds(x, w)
     want = ref if want is None else want
