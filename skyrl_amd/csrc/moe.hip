@@ -448,7 +448,7 @@ __global__ __launch_bounds__(WK* kWave) void moe_one_kernel(Router ro, const flo
 // expert (TM > 16) an XCD takes a run of tiles, a tile's columns together. The output leaves through LDS, whole rows. Weights of an
 // expert with one tile go past the caches (non-temporal), as a step's experts are several times the last-level cache; with several
 // tiles, which all read them, they stay: a loop for each, since a branch at every load costs 3 to 10 %. 64 experts, both products, us
-// (all cached / all past): 768 x 2048, 256 tokens 118 (128 / 118); unevenly loaded 111 (115 / 116); 576 x 1536, 1200 tokens in tiles of 128
+// (all cached / all past; 768 x 2048 while it took this form): 768 x 2048, 256 tokens 118 (128 / 118); unevenly loaded 111 (115 / 116); 576 x 1536, 1200 tokens in tiles of 128
 // 142 (141 / 164), 8000 in tiles of 64 664 (659 / 1097).
 template <int TM, int TN, int WM, int WN, int S, bool GATED>
 __global__ __launch_bounds__(WM* WN* kWave) void moe_gemm_kernel(Product p, const uint16_t* __restrict__ x,
