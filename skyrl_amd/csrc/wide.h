@@ -124,8 +124,9 @@ __device__ __forceinline__ int32_t uniform(const int32_t* p) {
 // came at 5.2 TB/s where all experts began at 0, at 6.2 where each begins elsewhere (64 experts of 768 x 2048, gate_up, us: 256 tokens
 // 79 -> 63, 700 tokens in tiles of 128 90 -> 75; down, rows of 1536 bytes, 40.7 -> 39.4). One start for an expert: its tiles, and
 // a tile's columns, share what they read (a start for each column: 5637 tokens 265 us, 243 with this). kDense with ONCE, where all
-// columns read the same few rows, and kGated with tiles of 64: a start for each half of an item's columns (128 x 2048, 6144 gated 22.0 ->
-// 21.6 us).
+// columns read the same few rows: a start for each half of an item's columns. Which items are halved follows from the columns alone there,
+// so a row's sums do not depend on its place. kGated has one call's items of a column whole and halved: all from 0, as its tiles of 256
+// (128 x 2048, 6144 gated 22.1 us, 21.1 with a start for each half, by which equal rows of different tiles had different bits).
 __device__ __forceinline__ int depth_start(int e, int K) {
     return K % 256 == 0 ? (int)__umulhi((uint32_t)e * 0x9E3779B9u, (uint32_t)K / 64) : 0;
 }
@@ -237,7 +238,7 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
     int64_t wslot[4] = {};  // what a slot's rows of w are past the item's first; those of a half are the first slots'
     auto wrap = [](uint32_t at) { return min(at, at - RING * SLOT); };  // of less than two rings
     int k_start = 0;        // of the item whose loads are under way
-    constexpr bool TURNED = ROUTED || ONCE || XS == 1;
+    constexpr bool TURNED = ROUTED || ONCE;
     auto depth = [&](int k) { return TURNED && k + k_start >= p.K ? k + k_start - p.K : k + k_start; };
     auto fetch = [&](auto nt, int k0, uint32_t base, int i) __attribute__((always_inline)) {  // load i at depth k0 of the stage at base
         const bool is_w = WF ? i < LW : i >= LX;

@@ -72,6 +72,15 @@ def test_gated_small_tiles(dev, n, N, K):
     test_gated(dev, n, N, K, "gelu_tanh")
 
 
+@pytest.mark.parametrize("n,N,K", [(128, 6144, 2048), (192, 4608, 1536), (256, 8960, 768), (448, 4608, 1536)])
+def test_gated_rows_of_equal_tiles(dev, n, N, K):
+    """A row has the same bits in every tile of 64 of its call, whichever of the tiles' items are halved."""
+    x, w, _ = _data(dev, 64, 2 * N, K, n)
+    assert lk._ffi.query("skyrl_gated_product_fits", n, K, N)
+    y = lk.gated_linear(x.repeat(n // 64, 1), w, "silu").view(n // 64, 64, N)
+    assert bool((y == y[0]).all())
+
+
 @pytest.mark.parametrize("N", [4096, 4100, 8192, 8196, 12288, 12292, 16384, 16388])
 @pytest.mark.parametrize("n,K", [(16, 264), (17, 136), (32, 520), (33, 264), (64, 1032)])
 def test_rows_of_weights_a_workgroup(dev, n, N, K):
