@@ -337,7 +337,9 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
         wat[ks] = lds0 + c * BK * 2 + ((ks * 4 + g) ^ (c / 2)) * 16;
         xat[ks] = wat[ks] + wm * 16 * BK * 2;
     }
-    bool whole = false;  // the last item had all rows: its stores are counted
+    // The last item had all rows and, in this wave, columns: every store had a lane and is counted. Whether one without any is, nothing
+    // here depends on.
+    bool whole = false;
 
     // A step's products in four groups: half of the depth ks, half h of the 2 MH tiles of rows that are in use.
     // HALF: of one half of the item's columns, a workgroup's last.
@@ -459,7 +461,7 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
         }
         uint16_t* const to = p.out + n0 + wn * WC + lane % LR * 8;
         const int own = tile * (ROUTED ? TM : p.tile_rows);
-        const bool in = KIND != kDense || n0 + wn * WC + lane % LR * 8 < p.N;  // this lane's columns
+        const bool in = KIND != kDense || n0 + wn * WC + lane % LR * 8 < p.N, any = KIND != kDense || n0 + wn * WC < p.N;  // this lane's columns, some lane's
         // The last products are in their registers 16 cycles on. The item's last stage is read: two of its slots, the ones that
         // nothing is loaded into before the next barrier, are the results' way.
         uint32_t scale[2 * MH];
@@ -541,7 +543,7 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
             }
             leave(m);
         }
-        whole = MH == 4 && all_rows && nk > AHEAD + 1;  // with fewer stages the next item's rows are needed right behind the first step
+        whole = MH == 4 && all_rows && any && nk > AHEAD + 1;  // with fewer stages the next item's rows are needed right behind the first step
     };
     prime(0);
     for (int i = 0;; ++i) {

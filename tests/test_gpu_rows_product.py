@@ -113,6 +113,16 @@ def test_dense(dev, n, N, K, pad):
         assert y.shape == (n, N) and bool(((y.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2 * off).all())
 
 
+@pytest.mark.parametrize("n,N,K", [(2560, 12352, 320), (4096, 6272, 512), (3072, 9224, 256)])
+def test_dense_items_past_the_last_column(dev, n, N, K):
+    """Full tiles of 256 rows in several rounds, whose last columns leave waves of an item without a store: the same bits every time."""
+    x, w, _ = _data(dev, n, N, K, n + N)
+    ref, off = _bounds(x, w)
+    y = lk._dense(x, w)
+    assert bool(((y.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2 * off).all())
+    assert all(torch.equal(lk._dense(x, w), y) for _ in range(3))
+
+
 @pytest.mark.parametrize("n,N,K", [(65, 28672, 64), (100, 28680, 320), (128, 30000, 256), (129, 28672, 512), (256, 66056, 128), (200, 28680, 768)])
 def test_dense_one_tile_of_rows(dev, n, N, K):
     """One tile of 128 or 256 rows, halves of items and whole ones, depths with a start for each column and without."""
