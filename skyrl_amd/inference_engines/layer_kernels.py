@@ -305,17 +305,19 @@ def _rows_aligned(x: torch.Tensor, w: torch.Tensor) -> bool:
             and (n == 1 or x.stride(0) >= K) and w.stride(0) >= K and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
-def linear(x, w: torch.Tensor, bias: Optional[torch.Tensor] = None, parts: bool = False, turn=None) -> torch.Tensor:
+def linear(x, w: torch.Tensor, bias: Optional[torch.Tensor] = None, parts: bool = False, turn=None,
+           in_order: bool = False) -> torch.Tensor:
     """x w^T + bias. Few bf16 rows take skyrl_rows_product, many without a bias skyrl_dense_product where it is the faster one,
     everything else the library. With `parts` the result of
     few rows may be f32 [splits, n, N], to be summed over the first index where it is read (add_norm, gate_norm_add,
-    joined). turn (first, last): these columns go through tanh, where `turns` says so. x: rows, or a NormedRow."""
+    joined). turn (first, last): these columns go through tanh, where `turns` says so. in_order: no form of few rows, which cut the
+    depth. x: rows, or a NormedRow."""
     if isinstance(x, NormedRow):
         y = x.product(w, bias, parts=parts, turn=turn)
         if y is not None:
             return y
         x = x.rows()
-    if not _rows_fit(x, w, parts=parts):
+    if in_order or not _rows_fit(x, w, parts=parts):
         if turn is not None:
             raise ValueError("a library's product turns no columns")
         return F.linear(x, w, bias) if bias is not None or not _dense_fit(x, w) else _dense(x, w)

@@ -437,8 +437,9 @@ class LatentAttention:
         if ts < T:
             seg, tiles, rows, longest = inp.plan[self.window]
             latent, k_rot = lk.latent_gather(cache, self.rank, self.rot_dim, inp.block_tables, seg, rows, longest)
-            k = lk.linear(latent, self.wuk)
-            v_t = lk.linear(self.wuv, latent)
+            many = T > lk.MAX_ROWS  # as in _attend_rows: also the keys of a portion that sees no more than 64
+            k = lk.linear(latent, self.wuk, in_order=many)
+            v_t = lk.linear(self.wuv, latent, in_order=many)
             lk.latent_prefill(q, k, k_rot, v_t, tiles, H, self.dim, self.rot_dim, self.vdim, self.scale, self.window,
                               out, sinks=self.sinks, gate=gate)
 

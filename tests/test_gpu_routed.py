@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 import torch
 
-from hybrid_cases import SANDWICH, general, low_rank, make_sandwich_weights, routed, sandwich_config
+from hybrid_cases import SANDWICH, config, general, latent, low_rank, make_sandwich_weights, routed, sandwich_config
 from hybrid_gpu import DEV, DTYPES, build, close, feed, generate, greedy, model_close, rms, rnd, tokens_of
 from oracle import hybrid_ref as ref
 from skyrl_amd.inference_engines import layer_kernels as lk
@@ -201,6 +201,37 @@ def test_decode_rows_of_many_tokens_take_the_librarys_products(heads, T, n, alon
     else:
         o.copy_(torch.bmm(mid, mix.wuv_t).transpose(0, 1))
     assert bool(o.isfinite().all()) and torch.equal(out[:n].view(n, heads, V), o)
+
+
+@pytest.mark.parametrize("short,keys", [(130, 40), (100, 64), (97, 32), (96, 32), (130, 65)])
+def test_keys_of_a_short_portion(monkeypatch, short, keys):
+    """A portion with up to 64 keys: in a step of more than 128 tokens its keys and values sum along the depth, as those of a longer one."""
+    heads, C = 4, 512
+    mix = build(config([latent(heads=heads, dim=128, rot_dim=32, vdim=64, kv_rank=C, window=None)], width=256), BF16)[0].layers[0]["mixer"]
+    g = torch.Generator(device=DEV).manual_seed(short + keys)
+    mk = lambda *s: torch.randn(s, generator=g, device=DEV).to(BF16)  # noqa: E731
+    T, blocks = short + keys, 8
+    cache = mk((short + 1) * blocks, BS, lk.latent_row(C, 32))
+    lens, starts = [1] * short + [keys], [50] * short + [0]
+    plan = mixers.prompt_plan(lens, starts, short, short, None)
+    pos = torch.tensor(starts[:short] + list(range(keys)), device=DEV)
+    row = torch.tensor(list(range(short)) + [short] * keys, device=DEV)
+    tables = torch.arange((short + 1) * blocks, dtype=torch.int32, device=DEV).view(short + 1, blocks)
+    inp = SimpleNamespace(block_tables=tables, bt_row=row.int(), positions=pos, slots=tables[row, pos // BS].long() * BS + pos % BS, max_ctx=max(51, keys),
+                          one_token=False, short_tokens=short, plan={None: tuple(dev(torch.from_numpy(t)) for t in plan[:2]) + plan[2:]})
+    seen = {}
+    gather, prefill = lk.latent_gather, lk.latent_prefill
+    monkeypatch.setattr(lk, "latent_gather", lambda *a: seen.setdefault("latent", gather(*a)))
+    monkeypatch.setattr(lk, "latent_prefill", lambda q, k, k_rot, v_t, *a, **kw: seen.update(k=k, v_t=v_t) or prefill(q, k, k_rot, v_t, *a, **kw))
+    mix.inner(mk(T, mix.in_rows), torch.zeros(T, heads * 64, dtype=BF16, device=DEV), inp, cache, None)
+    at = seen["latent"][0]
+    k, v_t = torch.nn.functional.linear(at, mix.wuk), torch.mm(mix.wuv, at.t())
+    assert at.shape[0] == plan[2] == (keys + 63) // 64 * 64
+    for got, want in ((seen["k"], k), (seen["v_t"], v_t)):
+        if T > lk.MAX_ROWS:
+            assert torch.equal(got, want)
+        else:
+            close(got, want.double().cpu(), BF16)
 
 
 
