@@ -274,11 +274,12 @@ def _rows_fit(x: torch.Tensor, w: torch.Tensor, gated: bool = False, parts: bool
 
 
 def _dense_fit(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether skyrl_dense_product takes x [n, K] (a column range) and w [N, K] and is the faster form."""
+    """Whether skyrl_dense_product takes x [n, K] (a column range) and w [N, K] and is the faster form. It has no backward: products that
+    are differentiated stay the library's."""
     (n, K), N = x.shape, w.shape[0]
     return (n > ROUNDED_ROWS and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.is_cuda and w.shape[1] == K
             and bool(_ffi.query("skyrl_dense_product_fits", n, K, N)) and n * x.stride(0) < 1 << 31 and N * w.stride(0) < 1 << 31
-            and _rows_aligned(x, w))
+            and _rows_aligned(x, w) and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)))
 
 
 def _dense(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:

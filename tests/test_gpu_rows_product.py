@@ -148,6 +148,24 @@ def test_many_rows_take_the_faster_form(dev):
     assert torch.equal(lk.linear(x, w), torch.nn.functional.linear(x, w))
 
 
+@pytest.mark.parametrize("n,N,K", [(65, 2048, 512), (300, 2048, 2048), (5637, 3072, 768)])
+def test_many_rows_that_need_gradients(dev, n, N, K):
+    """The library's product, which has them, also where ours is the faster one."""
+    x, w, _ = _data(dev, n, N, K, n)
+    assert lk._dense_fit(x, w)
+    dy = torch.randn(n, N, device=dev).bfloat16()
+    for of_x, of_w in ((True, False), (False, True), (True, True)):
+        got, want = [], []
+        for f, to in ((lk.linear, got), (torch.nn.functional.linear, want)):
+            a, b = x.clone().requires_grad_(of_x), w.clone().requires_grad_(of_w)
+            y = f(a, b)
+            y.backward(dy)
+            to += [y, a.grad, b.grad]
+        assert all((a is None and b is None) or torch.equal(a, b) for a, b in zip(got, want))
+        with torch.no_grad():
+            assert not lk.linear(x.clone().requires_grad_(of_x), w.clone().requires_grad_(of_w)).requires_grad
+
+
 def test_what_the_library_takes(dev):
     x, w, _ = _data(dev, 129, 64, 64, 0)
     assert not lk._rows_fit(x, w)                                  # too many rows
