@@ -10,6 +10,7 @@ from typing import Optional
 
 import torch
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 from .. import _ffi
 from ..ops import _ptr, _require_gpu, _stream
@@ -273,13 +274,18 @@ def _rows_fit(x: torch.Tensor, w: torch.Tensor, gated: bool = False, parts: bool
             and bool(_ffi.query("skyrl_rows_product_fits", n, K, N, 1 if gated else 2 if parts else 0)) and _rows_aligned(x, w))
 
 
+def _transformed(*tensors: torch.Tensor) -> bool:
+    """Whether a product of these is differentiated either way, mapped or traced: such products are the library's."""
+    return (any(torch._C._functorch.is_functorch_wrapped_tensor(t) for t in tensors) or forward_ad._current_level >= 0
+            or torch.jit.is_tracing() or (torch.is_grad_enabled() and any(t.requires_grad for t in tensors)))
+
+
 def _dense_fit(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether skyrl_dense_product takes x [n, K] (a column range) and w [N, K] and is the faster form. It has no backward: products that
-    are differentiated stay the library's."""
+    """Whether skyrl_dense_product takes x [n, K] (a column range) and w [N, K] and is the faster form."""
     (n, K), N = x.shape, w.shape[0]
     return (n > ROUNDED_ROWS and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.is_cuda and w.shape[1] == K
             and bool(_ffi.query("skyrl_dense_product_fits", n, K, N)) and n * x.stride(0) < 1 << 31 and N * w.stride(0) < 1 << 31
-            and _rows_aligned(x, w) and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)))
+            and not _transformed(x, w) and _rows_aligned(x, w))
 
 
 def _dense(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:

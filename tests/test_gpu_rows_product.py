@@ -166,6 +166,23 @@ def test_many_rows_that_need_gradients(dev, n, N, K):
             assert not lk.linear(x.clone().requires_grad_(of_x), w.clone().requires_grad_(of_w)).requires_grad
 
 
+@pytest.mark.filterwarnings("ignore::DeprecationWarning")
+def test_many_rows_that_are_transformed(dev):
+    """Mapped, forward-differentiated and traced products are the library's too."""
+    x, w, _ = _data(dev, 300, 2048, 512, 0)
+    assert lk._dense_fit(x, w)
+    taken = []
+    for f in (torch.func.vmap, lambda f: lambda a: torch.func.jvp(f, (a,), (a,)), torch.func.grad):
+        f(lambda a: taken.append(lk._dense_fit(a[0] if a.dim() == 3 else a, w)) or a.float().sum())(x.expand(2, 300, 512).contiguous())
+    assert taken == [False] * 3
+    with torch.autograd.forward_ad.dual_level():
+        y = torch.autograd.forward_ad.unpack_dual(lk.linear(torch.autograd.forward_ad.make_dual(x, 2 * x), w))
+    want = torch.nn.functional.linear(x, w)
+    assert torch.equal(y.primal, want) and torch.equal(y.tangent, 2 * want)
+    f = torch.jit.trace(lambda a: lk.linear(a, w), x)
+    assert torch.equal(f(2 * x), 2 * want)
+
+
 def test_what_the_library_takes(dev):
     x, w, _ = _data(dev, 129, 64, 64, 0)
     assert not lk._rows_fit(x, w)                                  # too many rows
