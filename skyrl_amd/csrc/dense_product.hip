@@ -159,10 +159,7 @@ int64_t wide_rounds(int n, int N, int rows) {
 
 // The form, and whether it is the faster one beside the library's. Up to some 1000 rows the smallest tiles that are one round
 // of workgroups (64 x 32 to 64 x 64 fit a CU twice, and 64 x 128 do, so that half a round more costs little): a CU's loads bound
-// them, 80 to 90 GB/s, and the library's tiles leave CUs idle. Above, the wide form where its items fill 70 % of their rounds
-// and the columns are no multiple of the library's own 256, which costs it 10 to 25 %, or the rows none, where the two are within 2 %
-// alone and this is the faster one among a step's other launches: eight layers' 5637 rows of 2048 x 2048 39 us each beside 46, 1563 rows
-// in tiles of 128 x 128 22 beside 25. Shallow products are launches and latency.
+// them, 80 to 90 GB/s, and the library's tiles leave CUs idle. Above, the wide form, beside the library's tiles of 256 x 256.
 // us, here / the library's, weights from HBM, both in a captured graph:
 //   N, K            256 rows       512            1024           1563           3000          5637          8192
 //   2048, 2048      8.2 / 10.8     10.0 / 12.3    14.3 / 16.3    -              -             -             -
@@ -179,23 +176,61 @@ int64_t wide_rounds(int n, int N, int rows) {
 //   40000, 2048     -             40.6 / 51.2   54.5 / 59.5
 //   65536, 4096     -             -             121 / 162
 //   151936, 2048    -             124 / 175     161 / 219
-// Where the library stays, us, the same: 1563 x 2048, 3408 28.7 / 30.4; 3000 x 2048, 2048 29.1 / 27.9; 8192 x
-// 2048, 2048 53 / 51; 1300 x 6144, 2048 50.6 / 39.0; 512 x 2048, 12352 40.7 / 35.4; 2048 x 2048, 32768 216 / 200.
+// Where a line lies: of 2500 sizes (65 to 8192 rows, 8 to 152000 columns, 64 to 12288 deep) those that it takes are 1.29 times as fast as
+// the library's (geometric mean; one in a hundred is more than 3 % slower, the worst, 273 x 1280, 10880, 10 %), those that it leaves 0.93
+// times. Left, rows x K, N:
+//   64 x 32, few of them along a long depth, which the library cuts: 256 x 6144, 24 15.0 / 7.8; 65 x 2048, 512 7.4 / 6.3; 512 x 4096,
+//     512 12.0 / 11.4; 65 x 4096, 2560 11.9 / 11.1. With more than half of the CUs, 256 x 4096, 1264 1.20 times as fast. As 64 x 64: 65 x
+//     4096, 5120 19.7 / 17.7, and past 4096 deep where rows fill its tiles (256 x 6144, 3072 31.1 / 28.7; 192 x 6144, 4096 is 1.5 times as fast).
+//   64 x 128: 384 x 6144, 3072 46 / 36, 512 x 4096, 2560 22.4 / 21.6 (240 of 256 tiles: 1.07); 1400 x 2048, 2048 21.3 / 19.2, whose 352 tiles are 1 3/8 rounds.
+//   128 x 128 with up to 192 of the CUs: 1500 x 2048, 1024 20.1 / 14.3, 1563 x 1536, 1536 17.1 / 16.0 (1563 x 2048, 2048, 208 tiles: 20.8 / 20.6
+//     alone, and in a step between other launches 22 / 25); 768 x 1536, 4096 17.4 / 16.4, 384 x 1536, 8192 17.8 / 16.2; shallow
+//     ones of several rounds where the library's tiles fit: 1024 x 512, 16384 29.5 / 22.7 (1024 x 512, 9280 is even, 1400 x 384, 3408 1.3 times as fast).
+//   Shallow and narrow, from 2049 rows: 3000 x 256, 512 7.5 / 6.4, 2049 x 512, 1536 12.5 / 10.1 (4096 x 512, 1536 1.16 times as fast).
+//   Columns a multiple of 256, as many rounds as the library: 7091 x 1536, 2048 41 / 38, 6270 x 3072, 2560 81 / 72; past 2048 deep also where
+//     a third less: 5637 x 6144, 2048 127 / 113, 6405 x 3072, 7680 0.91 times (5432 x 3072, 3072, 1.33 rounds for 2: 96 / 111). Other columns
+//     past 6144 deep: 2844 x 10048, 12160 0.85 times.
 Form form_of(int n, int K, int N, bool& faster) {
     faster = true;
     if (n > 64 && n <= 256 && N >= 28672) return kOnce;
+    const bool columns = N % 256 != 0;  // that the library's tiles do not fit
     if (n <= 1400 && K <= 6144 && (n <= 1024 || K <= 2048)) {
-        if (tiles_of(n, N, 64, 32) <= kCUs) return k64x32;
-        if (tiles_of(n, N, 64, 64) <= kCUs) return k64x64;
-        const int64_t t = tiles_of(n, N, 64, 128);
-        if ((K <= 2048 || N < 4096) && (t <= kCUs || (K <= 2048 && n > 512 && t <= kCUs * 11 / 8))) return k64x128;
-        if (K <= 2048 && tiles_of(n, N, 128, 128) <= kCUs) return k128x128;
+        const int64_t least = K <= 3072 || n > 96 ? kCUs / 2 : kCUs * 5 / 8;
+        int64_t t = tiles_of(n, N, 64, 32);
+        if (t <= kCUs) {
+            faster = K <= 1024 || t > (K <= 2048 ? kCUs / 8 : least);
+            return k64x32;
+        }
+        if ((t = tiles_of(n, N, 64, 64)) <= kCUs) {
+            faster = (K <= 2048 || t > least) && (K <= 4096 || (n > 96 && n <= 192));
+            return k64x64;
+        }
+        t = tiles_of(n, N, 64, 128);
+        if ((K <= 2048 || N < 4096) && (t <= kCUs || (K <= 2048 && n > 512 && t <= kCUs * (K <= 1024 ? 22 : 21) / 16))) {
+            faster = K <= 3072 || (K <= 4096 && t > kCUs * 3 / 4);
+            return k64x128;
+        }
+        if (K <= 2048 && (t = tiles_of(n, N, 128, 128)) <= kCUs) {
+            faster = n <= 256 || columns || K < 1024 || t > kCUs * 7 / 8;
+            return k128x128;
+        }
+    }
+    if (K <= 512 && n <= 2048) {
+        const bool one = tiles_of(n, N, 64, 128) <= 2 * kCUs;
+        faster = one ? N > 32 : columns;
+        return one ? k64x128 : k128x128;
+    }
+    if (n <= 2048 && K <= 2048 && tiles_of(n, N, 128, 128) <= kCUs) {
+        faster = tiles_of(n, N, 128, 128) > kCUs * 3 / 4;
+        return k128x128;
     }
     const int64_t r256 = wide_rounds(n, N, 256), r192 = wide_rounds(n, N, 192), rounds = r192 < r256 ? r192 : r256;
-    const bool full = (int64_t)n * N * 100 >= 70 * rounds * 256 * 256 * kCUs / 100;
-    if (K <= 512 && n <= 2048) return tiles_of(n, N, 64, 128) <= 2 * kCUs ? k64x128 : k128x128;
-    if (n <= 2048 && K <= 2048 && tiles_of(n, N, 128, 128) <= kCUs) return k128x128;
-    faster = K <= 512 || (full && ((n >= 800 && N % 256 != 0) || (n >= 4096 && n % 256 != 0) || (n >= 5000 && K <= 1024)));
+    const int64_t whole = (tiles_of(n, N, 256, 256) + kCUs - 1) / kCUs * 100;  // the library's
+    if (K <= 512) faster = N >= 2048 || (N >= 1536 && (columns || n >= 4096));
+    else if ((int64_t)n * N * 100 < 70 * rounds * 256 * 256 * kCUs / 100) faster = false;
+    else if (columns) faster = n >= 800 && K <= 6144;
+    else if (n < 4096 || (n % 256 == 0 && (n < 5000 || K > 1024))) faster = false;
+    else faster = K <= 1024 ? rounds < whole || whole > 100 : K <= 2048 ? rounds < whole : K <= 3072 && 3 * rounds <= 2 * whole;
     return r192 < r256 ? kWide192 : kWide256;
 }
 

@@ -299,3 +299,18 @@ def test_variant_applies_to_its_call_only():
             assert _ffi.query("skyrl_policy_train_supports", V, 1, 1.0) == 1
         assert _ffi.query("skyrl_policy_train_supports", V, 1, 1.0) == 0
     assert _ffi.query("skyrl_policy_train_supports", V, 1, 1.0) == 1 and _ffi.current_variant() is None
+
+
+@pytest.mark.parametrize("n,N,K,takes", [
+    (65, 512, 2048, 0), (65, 520, 1024, 1), (256, 2048, 2048, 1), (65, 2560, 4096, 0), (128, 2560, 4096, 1), (256, 24, 6144, 0),     # 64 x 32
+    (512, 512, 4096, 0), (256, 1264, 4096, 1), (65, 5120, 4096, 0), (192, 4096, 6144, 1), (256, 3072, 6144, 0),                       # to 64 x 64
+    (384, 3072, 6144, 0), (512, 2560, 4096, 0), (1400, 2048, 2048, 0), (1400, 2048, 1024, 1), (1300, 2048, 2048, 1),                  # 64 x 128
+    (768, 4096, 1536, 0), (768, 4104, 1536, 1), (256, 12288, 2048, 1), (1500, 1024, 2048, 0), (1563, 1536, 1536, 0),                  # 128 x 128
+    (1563, 2048, 2048, 1), (1024, 16384, 512, 0), (1400, 3408, 384, 1), (2048, 8, 512, 0),
+    (2049, 8, 512, 0), (3000, 512, 256, 0), (2049, 1536, 512, 0), (4096, 1536, 512, 1), (3000, 1600, 512, 1),                         # wide
+    (5637, 2048, 2048, 1), (7091, 2048, 1536, 0), (6270, 2560, 3072, 0), (5432, 3072, 3072, 1), (5637, 2048, 6144, 0),
+    (5637, 4096, 12288, 0), (4096, 12352, 2048, 1), (2844, 12160, 10048, 0), (8192, 3072, 768, 1), (8192, 2048, 2048, 0),
+    (65, 28672, 4096, 1), (256, 151936, 2048, 1), (300, 2044, 2048, 0), (300, 2048, 2056, 0), (0, 2048, 2048, 0)])
+def test_dense_products_that_the_library_is_slower_at(n, N, K, takes):
+    """Both sides of each line of the rule: the sizes that skyrl_dense_product leaves were up to twice as slow by it."""
+    assert bool(_ffi.query("skyrl_dense_product_fits", n, K, N)) == bool(takes)
