@@ -314,3 +314,10 @@ def test_variant_applies_to_its_call_only():
 def test_dense_products_that_the_library_is_slower_at(n, N, K, takes):
     """Both sides of each line of the rule: the sizes that skyrl_dense_product leaves were up to twice as slow by it."""
     assert bool(_ffi.query("skyrl_dense_product_fits", n, K, N)) == bool(takes)
+
+
+@pytest.mark.parametrize("n,N,K,takes", [(128, 6144, 2048, 1), (129, 6144, 2048, 0), (511, 4608, 768, 1), (450, 4608, 1536, 0), (448, 4608, 1536, 1),
+                                         (289, 7168, 1024, 0), (289, 7168, 768, 1), (400, 6144, 512, 0), (1024, 6144, 2048, 1)])
+def test_gated_products_of_many_rows(n, N, K, takes):
+    """One round of tiles of 64, an eighth more of shallow ones; from 512 rows three quarters of a round of tiles of 256."""
+    assert bool(_ffi.query("skyrl_gated_product_fits", n, K, N)) == bool(takes)
