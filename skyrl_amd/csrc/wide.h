@@ -131,6 +131,25 @@ __device__ __forceinline__ int depth_start(int e, int K) {
     return K % 256 == 0 ? (int)__umulhi((uint32_t)e * 0x9E3779B9u, (uint32_t)K / 64) : 0;
 }
 
+// A workgroup's items: of an XCD's run, one in `stride`, and of what is left over behind the whole rounds halves of the columns where
+// there are workgroups for both.
+struct Share {
+    int first, stride, at, rounds, mine;
+    bool halve;
+    __host__ __device__ Share(int64_t items, int grid, int block) : stride(grid / 8), at(block / 8) {
+        const int xcd = block % 8;
+        first = (int)(items * xcd / 8);
+        const int left = (int)(items * (xcd + 1) / 8) - first, over = left % stride;
+        rounds = left / stride, halve = 2 * over <= stride;
+        mine = rounds + (at < (halve ? 2 * over : over));
+    }
+    // The i-th of them, and whether it is one half of its columns or the other (1, 2).
+    __host__ __device__ int nth(int i) const { return first + i * stride + (halve && i == rounds ? at / 2 : at); }
+    __host__ __device__ int half_of(int i) const { return halve && i == rounds ? 1 + at % 2 : 0; }
+};
+// A workgroup per CU, or as many as every XCD needs to halve all of its items.
+inline int wide_grid(int64_t items) { return (int)(items > kCUs / 2 ? kCUs : (items + 7) / 8 * 16); }
+
 // Whether an expert's tiles, which follow each other, are this one alone.
 __device__ __forceinline__ bool one_tile(const int32_t* tile_expert, int tile, int ntiles, int e) {
     return (tile == 0 || tile_expert[tile - 1] != e) && (tile + 1 == ntiles || tile_expert[tile + 1] != e);
@@ -187,16 +206,10 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c = lane & 15, g = lane >> 4, wm = wave >> 1, wn = wave & 1;
     const int ntiles = ROUTED ? uniform(p.tile_expert + p.ntiles) : p.ntiles;
-    const int64_t items = (int64_t)ntiles * ncols;
-    const int xcd = blockIdx.x % 8, stride = gridDim.x / 8, at = blockIdx.x / 8;
-    const int first = (int)(items * xcd / 8), left = (int)(items * (xcd + 1) / 8) - first, rounds = left / stride, over = left % stride;
-    const bool halve = 2 * over <= stride;
-    const int mine = rounds + (at < (halve ? 2 * over : over));  // items of this workgroup
+    const Share share((int64_t)ntiles * ncols, gridDim.x, blockIdx.x);
+    const int mine = share.mine;
     if (mine == 0) return;
     const int nk = p.K / BK;
-    // The i-th of them, and whether it is one half of its columns or the other (1, 2).
-    auto nth = [&](int i) { return first + i * stride + (halve && i == rounds ? at / 2 : at); };
-    auto half_of = [&](int i) { return halve && i == rounds ? 1 + at % 2 : 0; };
 
     // An XCD's workgroups read few tiles' rows and few columns' weights at a time. Routed: a tile's columns follow each other
     // (an expert has about as many tiles as its weights have columns here). kGated: blocks of four tiles, column by column.
@@ -216,8 +229,8 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
     int next_tile = 0, next_n0 = 0, next_half = 0, next_e = 0, e_before = 0, e_after = 0;
     auto peek = [&](int i, int qn) __attribute__((always_inline)) {
         int col;
-        place(nth(i), next_tile, col);
-        next_half = half_of(i);
+        place(share.nth(i), next_tile, col);
+        next_half = share.half_of(i);
         next_n0 = col * OC;
         if constexpr (ROUTED) {
             if (XS == 4 || wave < XS)
@@ -588,15 +601,13 @@ __global__ __launch_bounds__(256) void wide_kernel(Wide p) {
     wait_loads<0>();  // into LDS that is another workgroup's next
 }
 
-// A workgroup per CU, or two for every item where these are fewer (each a half of its columns).
 inline bool wide_fits(int K, int N, bool gated) { return K > 0 && K % 64 == 0 && N % (gated ? 128 : 256) == 0; }
 template <int KIND, int ACT = SKYRL_ACT_SILU, bool ONCE = false, int TM = 256>
 int launch_wide(Wide p, hipStream_t s) {
     set_division(p);
     const int64_t items = (int64_t)(KIND == kDense ? (p.N + 255) / 256 : p.N / (KIND == kDown ? 256 : 128)) * p.ntiles;
     SKYRL_REQUIRE(items < (1ll << 31) && p.ntiles < (1 << 23), "wide products: too many rows in one call");
-    const unsigned grid = (unsigned)(items > kCUs / 2 ? kCUs : (2 * items + 7) / 8 * 8);
-    hipLaunchKernelGGL((wide_kernel<KIND, ACT, ONCE, TM>), dim3(grid), dim3(256), 0, s, p);
+    hipLaunchKernelGGL((wide_kernel<KIND, ACT, ONCE, TM>), dim3((unsigned)wide_grid(items)), dim3(256), 0, s, p);
     return check_launch("wide_kernel");
 }
 
