@@ -527,20 +527,29 @@ def test_tile_sizes_agree_bit_for_bit(width, ff, experts, top, n):
 
 @pytest.mark.parametrize("n", (1, 639, 640))
 def test_wide_tiles_agree_on_both_sides_of_a_tile_an_expert(n):
-    """Up to 639 tokens, 2 of 4 experts each, the wide form's weights go past the caches: the same rows as from tiles of 64."""
+    """Up to 639 tokens, 2 of 4 experts each, the wide form's weights go past the caches: in tiles of 256 and 64 the rows that the staged
+    form's tiles of 16 give; of one token, which those stream in shares of the depth, the exact ones."""
     g = torch.Generator(device=DEV).manual_seed(n)
     sh = lk.moe_shape(256, 256, 4, 2)
     mk = lambda *s, scale=1.0: (torch.randn(s, generator=g, device=DEV) * scale).to(BF16)  # noqa: E731
     x, wgu, wd = mk(n, 256), mk(4, 2, 256, 256, scale=0.1), mk(4, 256, 256, scale=0.1)
     idx, weight = lk.moe_route(sh, x, mk(4, 256), torch.zeros(4, device=DEV))
-    wide, staged = (lk.moe_experts(sh, x, idx, weight, wgu, wd, tm=tm) for tm in (256, 64))
-    assert torch.equal(wide, staged)
+    tiles, small, staged = (lk.moe_experts(sh, x, idx, weight, wgu, wd, tm=tm) for tm in (256, 64, 16))
+    assert torch.equal(tiles, small)
+    if n > 1:
+        assert lk._ffi.query("skyrl_moe_tiles", 4, 2 * n, 16) > 8  # not streamed
+        assert torch.equal(tiles, staged)
+    else:
+        e, h = idx[0].long(), x[0].double()
+        act = (torch.nn.functional.silu(wgu[e, 0].double() @ h) * (wgu[e, 1].double() @ h)).to(BF16).double()
+        close(tiles, ((wd[e].double() @ act[:, :, None])[:, :, 0] * weight[0, :, None].double()).cpu(), BF16, bf16=8e-3)
 
 
-@pytest.mark.parametrize("width,ff,experts,n", [(256, 128, 300, 9000), (512, 192, 250, 4000), (768, 384, 110, 9000), (512, 640, 64, 9000)])
+@pytest.mark.parametrize("width,ff,experts,n", [(256, 128, 300, 9000), (512, 192, 250, 4400), (768, 384, 110, 9000), (512, 640, 64, 9000),
+                                                 (64, 256, 300, 9000), (192, 256, 300, 9000)])
 def test_wide_tiles_in_rounds(width, ff, experts, n):
-    """Several items a workgroup, whole ones and halves, tiles of all heights behind each other, depths of two stages (each item on its
-    own), three and more: the rows that tiles of 64 give, every time."""
+    """Several items a workgroup, whole ones and halves, tiles of all heights behind each other, depths of one and two stages (each item
+    on its own), three and more: the rows that the staged form's tiles of 16 give, every time."""
     g = torch.Generator(device=DEV).manual_seed(n + ff)
     sh = lk.moe_shape(width, ff, experts, 1)
     mk = lambda *s, scale=1.0: (torch.randn(s, generator=g, device=DEV) * scale).to(BF16)  # noqa: E731
@@ -548,7 +557,8 @@ def test_wide_tiles_in_rounds(width, ff, experts, n):
     loads = torch.rand(experts, generator=g, device=DEV) ** 3 + 1e-3
     idx = torch.multinomial(loads, n, replacement=True, generator=g).int().view(n, 1)
     weight = torch.rand(n, 1, generator=g, device=DEV) + 0.2
-    want = lk.moe_experts(sh, x, idx, weight, wgu, wd, tm=64)
+    assert lk._ffi.query("skyrl_moe_tiles", experts, n, 16) > 2 * experts  # not streamed
+    want = lk.moe_experts(sh, x, idx, weight, wgu, wd, tm=16)
     for _ in range(3):
         assert torch.equal(lk.moe_experts(sh, x, idx, weight, wgu, wd, tm=256), want)
 
