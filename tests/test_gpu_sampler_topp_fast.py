@@ -311,3 +311,22 @@ def test_rows_in_pieces(dev, n, V):
         for s, (t, l) in enumerate(one):
             tw, lw = ops.sample(whole, temperature=1.0, top_p=0.95, seed=9, seq_ids=wide, step=s)
             assert torch.equal(t, tw[:n]) and torch.equal(l.nan_to_num(), lw[:n].nan_to_num())
+
+
+@pytest.mark.parametrize("n,V", [(1, 65536), (7, 65543), (64, 151936), (65, 98304), (128, 151941)])
+def test_rows_in_pieces_with_min_p(dev, n, V):
+    """Both filters where a row is several workgroups': every row decided without a second look, the two-kernel path's tokens, cuts and
+    logprobs, and the oracle's; floors above and below the top_p cut, a maximum in one piece that cuts all the others' elements."""
+    from oracle import sampler as osamp
+
+    g = torch.Generator().manual_seed(V + n)
+    x = (torch.randn(n, -(-V // 8) * 8, generator=g) * 2.5).to(torch.bfloat16)[:, :V]
+    x[n // 2, V - 3] = 40.0
+    ids = torch.arange(n, dtype=torch.int64) * 3 + 7
+    xd = x.contiguous().to(dev) if V % 8 == 0 else torch.empty(n, -(-V // 8) * 8, device=dev, dtype=torch.bfloat16)[:, :V].copy_(x)
+    for step, (temp, p, mp) in enumerate(((1.0, 0.95, 0.02), (0.7, 0.9, 0.2), (1.3, 0.5, 0.3), (1.0, 0.999, 1e-4), (0.6, 0.95, 0.99))):
+        kw = dict(temperature=temp, top_p=p, min_p=mp, seed=5, step=step)
+        tok, lp, _ = _ab(xd, n, seq_ids=ids.to(dev), **kw)
+        etok, elp = osamp.sample(x, temp, -1, p, mp, 5, ids, step)
+        assert torch.equal(tok, etok), (kw, int((tok != etok).sum()))
+        torch.testing.assert_close(lp, elp, atol=1e-4, rtol=1e-4)
