@@ -68,7 +68,8 @@ extern "C" {
  *                   gated in f32, rounded once. K a multiple of 64, N of 128. skyrl_gated_product_fits: whether it takes the
  *                   sizes and is the faster form.
  *   skyrl_dense_product  many rows: x w^T of x bf16 [n, K] (row stride ldx) and w bf16 [N, K] (row stride ldw), rows 16-byte
- *                   aligned, operands of less than 4 GB, as bf16 [n, N] contiguous: summed in f32 along the depth, rounded
+ *                   aligned, operands of less than 4 GB, as bf16 [n, N] contiguous: summed in f32 in one chain along the
+ *                   depth, from 0 or, n up to 256 and N from 28672 on, from a depth of the columns' own and round, rounded
  *                   once. K a multiple of 64, N of 8. skyrl_dense_product_fits: whether it takes the sizes and is the faster form.
  *   skyrl_rows_batch  `batch` such products without bias, x, w and out bf16 x_batch, w_batch and out_batch apart.
  *                   skyrl_rows_batch_in_order: each sum in the order of the depth, not in shares of it.

@@ -1,5 +1,6 @@
 // Products of many bf16 rows, y[n, N] = x[n, K] w[N, K]^T rounded once (skyrl_dense_product): the tiles of 256 of wide.h, and smaller
-// ones where those would leave the chip partly idle. Either form sums a result along the depth in one chain of 32-deep products.
+// ones where those would leave the chip partly idle. Each form sums a result in one chain of 32-deep products along the depth, from 0 but
+// for kOnce, which begins at a depth of the columns' own and goes round.
 #include "wide.h"
 
 namespace skyrl {

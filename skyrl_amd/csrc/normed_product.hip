@@ -331,8 +331,9 @@ __global__ __launch_bounds__(2 * kNT) void normed_product_kernel(RowsProduct p, 
 }
 
 constexpr int kWideCols = 8192;  // as in rows_product.hip
-// Pairs up to which 48 rows of weights a workgroup are at most one a CU: 64 leave CUs idle (6144 x 2048, of a step of one row 214.9 ->
-// 213.9 us with four such products; rounded ones of 8192 to 12288 columns: no change).
+// Pairs up to which 48 rows of weights a workgroup are at most one a CU: 64 leave CUs idle (us a launch, 64 / 48: 6144 x 2048 10.95 / 10.68,
+// 4608 x 1536 9.12 / 8.50, 4096 x 2048 10.06 / 9.46; in a step of one row with four such products within its noise; rounded ones of
+// 8192 to 12288 columns: no change).
 constexpr int kPairs = 24 * 256;
 
 template <int LONG, class Pre>

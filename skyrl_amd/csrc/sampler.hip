@@ -1716,7 +1716,7 @@ __global__ __launch_bounds__(kPNT) __attribute__((amdgpu_waves_per_eu(4))) void 
     const int nfull = (v_n / kStep) * kStep;
     uint4 cur[4], nxt[4];
     // a step's vectors of this lane; past the last one it reads that again. The vectors after the last whole step are loaded with
-    // it, all at once: a load each, waited for, was 2 us of a call (512 rows of 151936: 54.8 -> 52.8 us).
+    // it, all at once: a load each, waited for, was 3 us of a call (512 rows of 151936, top_p 0.95 at T = 0.6: 57.0 -> 53.9 us).
     auto load4 = [&](uint4 (&to)[4], int base) {
 #pragma unroll
         for (int u = 0; u < 4; ++u) to[u] = pv[min(base + u * NT + (int)threadIdx.x, v_n - 1)];
@@ -3154,7 +3154,8 @@ int topp_pieces(int nseq, int V) {
     if (pieces < 4 || (nseq > kTParts / kTPieces && steps < 6)) return 1;
     return ((V / 8 + pieces - 1) / pieces + 1) * 8 > 65535 ? 1 : pieces;
 }
-// enough for any number of rows up to this one
+// Enough for any number of rows up to this one: 19 KB a piece, 9.8 MB from 64 rows on. Of any vocabulary and type, also those that take no
+// pieces, since a workspace is sized for its rows.
 size_t topp_parts_bytes(int nseq) { return (size_t)(nseq < kTParts / kTPieces ? nseq * kTPieces : kTParts) * sizeof(ToppPart); }
 
 template <typename T, int MODE>

@@ -175,10 +175,11 @@ __device__ __forceinline__ bool one_tile(const int32_t* tile_expert, int tile, i
 //   kGated, kDense  one matrix, x and the output row by row in tiles of tile_rows (gated_product.hip): of N gate and N up rows,
 //                   any activation; of N rows, a multiple of 8, as they are.
 // Bound: the products at the power limit (weights of zeros: 8192 x 2048, 6144 gated in 226 us, random ones in 297, 1.39 PFLOP/s, the
-// clock at 1.8 to 1.9 GHz); kDown: its loads, 12 stages an item and 128 KB of results. Measured, 64 experts of 768 x 2048, 8 per
-// token, gate_up / down, us (before: an item's loads start when the one before has left, addresses in the ring by compare and
-// select): 1000 tokens 96 / 53 (111 / 58), 1563 tokens 103 / 58 (119 / 65), 3000 tokens 154 / 98 (162 / 106), 5637 tokens 247 / 152
-// (265 / 166), 8192 tokens 356 / 230 (379 / 260); gated: 8192 x 2048, 6144 297 (321), 4000 x 2048, 6144 150 (161).
+// clock at 1.8 to 1.9 GHz); kDown: its loads, 12 stages an item and 128 KB of results. What the ring and the direct loads gave alone, all
+// experts from depth 0 (before: an item's loads start when the one before has left, addresses in the ring by compare and select; 64 experts of
+// 768 x 2048, 8 per token, gate_up / down, us): 1000 tokens 96 / 53 (111 / 58), 1563 tokens 103 / 58 (119 / 65), 3000 tokens 154 / 98
+// (162 / 106), 5637 tokens 247 / 152 (265 / 166), 8192 tokens 356 / 230 (379 / 260); with depth_start and store_row as they are 1563 tokens take
+// 91 / 55, 5637 239 / 150. gated: 8192 x 2048, 6144 297 (321), 4000 x 2048, 6144 150 (161).
 // Where the loads of an item's last steps were cases in the loop's body, its branches took more than all this gave (324).
 // ONCE: weights of an expert with one tile go past the caches (non-temporal), those of an expert with several, which read them from
 // there, do not: both products, us (all cached / all past), before: 1563 tokens 185 (195 / 186), unevenly loaded 192 (196 / 202), 2048

@@ -1454,7 +1454,9 @@ def moe_rows(sh, n: int) -> int:
     """moe_tile, but 32 from 12 to 24 rows an expert, where it has about one tile of that and its weights are streamed once. Where the
     wide form takes both products, to 18 at widths from 2048, and 128 already from 48 rows. 8 of 64 experts, both products, us, tiles of 32 /
     64: 768 x 2048, 128 tokens 102 / 99, 160 tokens 107 / 100; 1536 x 4096, 160 tokens 387 / 386; 384 x 1024 33.1 / 34.5; of 64 / 128:
-    768 x 2048, 350 tokens 106 / 108, 400 tokens 118 / 110; 1536 x 4096, 450 tokens 429 / 415; 384 x 1024 39.4 / 36.4."""
+    768 x 2048, 350 tokens 106 / 108, 400 tokens 118 / 110; 1536 x 4096, 450 tokens 429 / 415; 384 x 1024 39.4 / 36.4. 20 rows an expert,
+    tiles of 32 / 64, loads even, a third apart, and so uneven that a third has none: 64 of 768 x 2048 107 / 103, 100 / 99, 79 / 86; 128 of these
+    212 / 197, 175 / 151, 142 / 126; 32 of 1536 x 4096 199 / 195, 215 / 194, 175 / 171."""
     wide = sh.ff % 128 == 0 and sh.width % 256 == 0
     mean = n * sh.top / sh.experts
     if 12 <= mean < (18 if wide and sh.width >= 2048 else 24):

@@ -392,10 +392,10 @@ class LatentAttention:
 
     # ---- step
     def _attend_rows(self, q, gate, out, inp, a: int, b: int, cache, workspace, qa=None):
-        """Tokens [a, b) in the decode form (qa: their up-projected queries where these are there already). More than lk.ORDERED_ROWS of them in a step of more than lk.MAX_ROWS tokens, whose
-        products all sum along the depth in one chain, do so in their up-projections too, and beside portions the shares that fill a
-        round: such a row is what it was whatever is the faster form of fewer rows (shares that fit: 19 us less a layer for 48
-        rows beside prompts, of a step of 2100 us)."""
+        """Tokens [a, b) in the decode form (qa: their up-projected queries where these are there already). More than lk.ORDERED_ROWS of
+        them in a step of more than lk.MAX_ROWS tokens sum their up-projections along the depth, as the other products of such a step
+        do, and take beside portions the shares that fill a round: such a row does not depend on the faster form of fewer rows (shares
+        that fit: 19 us less a layer for 48 rows beside prompts, of a step of 2100 us)."""
         H, D, R = self.heads, self.dim, self.rank
         n = b - a
         many = q.shape[0] > lk.MAX_ROWS and n > lk.ORDERED_ROWS
